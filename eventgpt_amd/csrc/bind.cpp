@@ -1177,6 +1177,32 @@ std::tuple<Tensor, Tensor> event_voxel_ranges(const Tensor& x, const Tensor& y, 
   return {hist, vox};
 }
 
+// whether event_voxel_sorted takes this image and these bins
+bool event_voxel_sorted_ok(int64_t bins, int64_t H, int64_t W) {
+  if (bins < 1 || bins > 65535 || H < 1 || W < 1 || bins * 2 * H * W >= (1ll << 31)) return false;
+  return evgpt::event_voxel_plan(1, (int)bins, (int)H, (int)W).log_rows >= 0;
+}
+
+// The same outputs for a stream in any order; t is read only when binning by time.
+std::tuple<Tensor, Tensor> event_voxel_sorted(const Tensor& x, const Tensor& y, const Tensor& p, const Tensor& t, int64_t bins,
+                                              int64_t H, int64_t W, bool signed_mode, bool by_count) {
+  check_i32(x, "x"); check_i32(y, "y"); check_i32(p, "p");
+  const int64_t n = x.numel();
+  TORCH_CHECK(n > 0 && n < (1ll << 31) - 65536 && y.numel() == n && p.numel() == n);
+  TORCH_CHECK(by_count || (t.is_cuda() && t.scalar_type() == at::kLong && t.is_contiguous() && t.numel() == n));
+  TORCH_CHECK(event_voxel_sorted_ok(bins, H, W), "event_voxel_sorted: image too wide or too many bins");
+  const evgpt::EventVoxelPlan plan = evgpt::event_voxel_plan((int)n, (int)bins, (int)H, (int)W);
+  Tensor work = at::empty({(int64_t)(plan.rec_bytes + plan.span_bytes + plan.range_bytes + plan.off_bytes)},
+                          x.options().dtype(at::kByte));
+  Tensor hist = at::empty({bins, 2, H, W}, x.options());
+  Tensor vox = at::empty({bins, H, W}, x.options().dtype(at::kFloat));
+  evgpt::launch_event_voxel_sorted(x.data_ptr<int>(), y.data_ptr<int>(), p.data_ptr<int>(),
+                                   by_count ? nullptr : reinterpret_cast<const long long*>(t.data_ptr<int64_t>()), (int)n, (int)bins,
+                                   (int)H, (int)W, plan, work.data_ptr<uint8_t>(), hist.data_ptr<int>(), vox.data_ptr<float>(),
+                                   signed_mode ? 1 : 0, by_count ? 1 : 0, cur_stream());
+  return {hist, vox};
+}
+
 // img uint8 [T,H,W,3] -> bf16 [T,3,S,S]; tables are int32 GPU tensors
 Tensor clip_preprocess(const Tensor& img, const Tensor& hstart, const Tensor& hcount,
                        const Tensor& hweight, const Tensor& vstart, const Tensor& vcount,
@@ -1401,6 +1427,8 @@ TORCH_LIBRARY(evgpt, m) {
   m.def("event_raster(Tensor x, Tensor y, Tensor p, int n_slices, int H, int W, int mode) -> Tensor", &event_raster);
   m.def("event_voxel(Tensor x, Tensor y, Tensor p, Tensor t, int t0, int span, int bins, int H, int W, bool signed_mode, bool by_count) -> (Tensor, Tensor)", &event_voxel);
   m.def("event_voxel_ranges(Tensor x, Tensor y, Tensor p, Tensor bounds, int H, int W, bool signed_mode, int chunks=0) -> (Tensor, Tensor)", &event_voxel_ranges);
+  m.def("event_voxel_sorted_ok(int bins, int H, int W) -> bool", &event_voxel_sorted_ok);
+  m.def("event_voxel_sorted(Tensor x, Tensor y, Tensor p, Tensor t, int bins, int H, int W, bool signed_mode, bool by_count) -> (Tensor, Tensor)", &event_voxel_sorted);
   m.def("clip_preprocess(Tensor img, Tensor hstart, Tensor hcount, Tensor hweight, Tensor vstart, Tensor vcount, Tensor vweight, int S, int resize_h, int resize_w, int top, int left, float[] mean, float[] stdv) -> Tensor", &clip_preprocess);
   m.def("gemm_force_config(int cfg) -> ()", &gemm_force_config);
   m.def("gemm_enable_256(bool on) -> ()", &gemm_enable_256);

@@ -125,6 +125,12 @@ void gemm_force_splitk(int sk);         // 0 = automatic; for tuning runs
 // ---- event_ops.hip
 void launch_event_raster(const int* x, const int* y, const int* p, int n_events, int n_slices,
                          int H, int W, int* keys, unsigned char* img, int mode, hipStream_t st);
+// how an event stream is counted by sorting (log_rows < 0: not), and the bytes of its scratch memory
+struct EventVoxelPlan { int log_rows, bands, chunks; size_t rec_bytes, span_bytes, range_bytes, off_bytes; };
+EventVoxelPlan event_voxel_plan(int n, int bins, int H, int W);
+void launch_event_voxel_sorted(const int* x, const int* y, const int* p, const long long* t, int n, int bins, int H, int W,
+                               const EventVoxelPlan& plan, unsigned char* work, int* out_hist, float* out_vox, int signed_mode,
+                               int by_count, hipStream_t st);
 int event_voxel_band_rows(int H, int W);
 void launch_event_voxel_ranges(const int* x, const int* y, const int* p, const int* bounds, int n_events,
                                int bins, int H, int W, int* out_hist, float* out_vox, int signed_mode,

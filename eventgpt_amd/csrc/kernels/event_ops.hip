@@ -194,6 +194,271 @@ void launch_event_voxel_ranges(const int* x, const int* y, const int* p, const i
                      rows, out_hist, out_vox, signed_mode);
 }
 
+// Counting without global atomics (what calls run on from 4 096 events: ops/event_ops.py), for streams in any order.  Three launches, no host round trip:
+//   span   one pass over t: extent and whether it is sorted (binning by time only)
+//   sort   a block orders its chunk of 8 192 events by (bin, band of `rows` image rows) in LDS and writes one 16-bit
+//          record per event -- polarity and place within the band -- plus where each key's run starts
+//   count  a block owns one (bin, band): it adds the runs of all chunks in LDS counters and writes both outputs whole
+// The chunk of a sorted stream lies in one or two bins, so the sort reads t at its two ends only; the unsorted one
+// reads it for every event.  Bound by memory: 12 B in, 2 B out, 2 B in per event (and 8 B for the span) plus 12 B out per
+// pixel and bin.  1e7 clustered events, 480 x 640, 5 bins by time on a sorted stream: span 16 us, sort 34, count 24; the
+// whole call 86 us (218 MB it cannot do without: 2.5 TB/s), 766 with voxel_lds_kernel below, which scans y once a band
+// (506 us) behind host round trips for the extent and the order of t.
+constexpr int VS_THREADS = 512, VS_PER = 16, VS_CHUNK = VS_THREADS * VS_PER, VS_KEYS = 4096, VS_SPANS = 256;
+constexpr int VC_THREADS = 1024;
+
+struct VoxelSpan { long long lo, hi; long long unsorted; };
+
+struct VoxelArgs {
+  const int *x, *y, *p;
+  const long long* t;
+  const VoxelSpan* span;         // [VS_SPANS] partial extents
+  unsigned short* rec;           // [chunks][VS_CHUNK]
+  unsigned short* off;           // [chunks][keys + 1]
+  int2* range;                   // [chunks] first and last bin
+  int n, bins, H, W, log_rows, bands, keys, chunks, by_count;
+};
+
+__global__ __launch_bounds__(1024) void voxel_span_kernel(const long long* __restrict__ t, int n, VoxelSpan* __restrict__ out) {
+  constexpr int DEPTH = 8;
+  __shared__ long long lo_s[16], hi_s[16];
+  __shared__ int bad_s;
+  if (threadIdx.x == 0) bad_s = 0;
+  const int per = (static_cast<int>((static_cast<long long>(n) + VS_SPANS - 1) / VS_SPANS) + 1023) & ~1023;
+  const long long first = static_cast<long long>(blockIdx.x) * per;
+  const long long last = min(first + per, static_cast<long long>(n));
+  long long lo = t[0], hi = lo;
+  bool bad = false;
+  for (long long i0 = first; i0 < last; i0 += 1024 * DEPTH) {
+    long long v[DEPTH], w[DEPTH];
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      const long long i = min(i0 + d * 1024 + threadIdx.x, last - 1);
+      v[d] = t[i];
+      w[d] = (threadIdx.x & 63) == 63 ? t[min(i + 1, static_cast<long long>(n) - 1)] : 0;
+    }
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      const long long next = __shfl_down(v[d], 1, 64);
+      lo = min(lo, v[d]);
+      hi = max(hi, v[d]);
+      bad |= v[d] > ((threadIdx.x & 63) == 63 ? w[d] : next);
+    }
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    lo = min(lo, static_cast<long long>(__shfl_xor(lo, off, 64)));
+    hi = max(hi, static_cast<long long>(__shfl_xor(hi, off, 64)));
+  }
+  __syncthreads();
+  if (bad) bad_s = 1;
+  if ((threadIdx.x & 63) == 0) { lo_s[threadIdx.x >> 6] = lo; hi_s[threadIdx.x >> 6] = hi; }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int i = 1; i < 16; ++i) { lo = min(lo, lo_s[i]); hi = max(hi, hi_s[i]); }
+    out[blockIdx.x] = {lo, hi, bad_s};
+  }
+}
+
+__global__ __launch_bounds__(VS_THREADS) void voxel_sort_kernel(VoxelArgs a) {
+  __shared__ int cnt[VS_KEYS];
+  __shared__ __attribute__((aligned(16))) unsigned short rec[VS_CHUNK];
+  __shared__ int wave_total[VS_THREADS / 64];
+  __shared__ long long ends[2][VS_SPANS / 64];
+  __shared__ int unsorted_s;
+  const int c0 = blockIdx.x * VS_CHUNK, tid = threadIdx.x;
+  const int in_chunk = min(VS_CHUNK, a.n - c0);
+  int xv[VS_PER], yv[VS_PER], pv[VS_PER];
+#pragma unroll
+  for (int e = 0; e < VS_PER; ++e) {
+    const int i = c0 + min(e * VS_THREADS + tid, in_chunk - 1);
+    xv[e] = a.x[i]; yv[e] = a.y[i]; pv[e] = a.p[i];
+  }
+  long long t0 = 0;
+  double span = 1.0;
+  const auto bin_of = [&](int i) {
+    const int b = a.by_count ? static_cast<int>(static_cast<long long>(i) * a.bins / a.n)
+                             : static_cast<int>(static_cast<double>(a.t[i] - t0) / span * a.bins);
+    return b < 0 ? 0 : (b >= a.bins ? a.bins - 1 : b);
+  };
+  bool unsorted = false;
+  if (!a.by_count) {
+    if (tid == 0) unsorted_s = 0;
+    __syncthreads();
+    if (tid < VS_SPANS) {
+      const VoxelSpan s = a.span[tid];
+      long long lo = s.lo, hi = s.hi;
+      if (s.unsorted) unsorted_s = 1;
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) {
+        lo = min(lo, static_cast<long long>(__shfl_xor(lo, off, 64)));
+        hi = max(hi, static_cast<long long>(__shfl_xor(hi, off, 64)));
+      }
+      if ((tid & 63) == 0) { ends[0][tid >> 6] = lo; ends[1][tid >> 6] = hi; }
+    }
+    __syncthreads();
+    long long t1 = ends[1][0];
+    t0 = ends[0][0];
+    for (int i = 1; i < VS_SPANS / 64; ++i) { t0 = min(t0, ends[0][i]); t1 = max(t1, ends[1][i]); }
+    span = static_cast<double>(t1 > t0 ? t1 - t0 : 1);
+    unsorted = unsorted_s != 0;
+  }
+  const int b0 = unsorted ? 0 : bin_of(c0), b1 = unsorted ? a.bins - 1 : bin_of(c0 + in_chunk - 1);
+  const int keys = (b1 - b0 + 1) * a.bands, rows = 1 << a.log_rows;
+  for (int k = tid; k < keys; k += VS_THREADS) cnt[k] = 0;
+  __syncthreads();
+  unsigned int item[VS_PER];                       // key << 16 | place; all ones: outside the image
+  unsigned short rank[VS_PER];
+#pragma unroll
+  for (int e = 0; e < VS_PER; ++e) {
+    const int j = e * VS_THREADS + tid;
+    item[e] = 0xffffffffu;
+    rank[e] = 0;
+    if (j >= in_chunk || xv[e] < 0 || xv[e] >= a.W || yv[e] < 0 || yv[e] >= a.H) continue;
+    const int key = (b0 == b1 ? 0 : bin_of(c0 + j) - b0) * a.bands + (yv[e] >> a.log_rows);
+    const int place = ((pv[e] != 0 ? rows : 0) + (yv[e] & (rows - 1))) * a.W + xv[e];
+    item[e] = static_cast<unsigned int>(key) << 16 | place;
+    rank[e] = static_cast<unsigned short>(atomicAdd(&cnt[key], 1));
+  }
+  __syncthreads();
+  // exclusive scan of the counts, VS_KEYS / VS_THREADS of them a thread
+  constexpr int KT = VS_KEYS / VS_THREADS;
+  int mine[KT], sum = 0;
+#pragma unroll
+  for (int k = 0; k < KT; ++k) {
+    mine[k] = sum;
+    sum += tid * KT + k < keys ? cnt[tid * KT + k] : 0;
+  }
+  int scan = sum;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int v = __shfl_up(scan, off, 64);
+    if ((tid & 63) >= off) scan += v;
+  }
+  if ((tid & 63) == 63) wave_total[tid >> 6] = scan;
+  __syncthreads();
+  int before = scan - sum;
+  for (int w = 0; w < (tid >> 6); ++w) before += wave_total[w];
+  int total = 0;
+  for (int w = 0; w < VS_THREADS / 64; ++w) total += wave_total[w];
+  unsigned short* off = a.off + static_cast<size_t>(blockIdx.x) * (a.keys + 1);
+#pragma unroll
+  for (int k = 0; k < KT; ++k)
+    if (tid * KT + k < keys) {
+      cnt[tid * KT + k] = before + mine[k];
+      off[tid * KT + k] = static_cast<unsigned short>(before + mine[k]);
+    }
+  if (tid == 0) {
+    off[keys] = static_cast<unsigned short>(total);
+    a.range[blockIdx.x] = make_int2(b0, b1);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < VS_PER; ++e)
+    if (item[e] != 0xffffffffu) rec[cnt[item[e] >> 16] + rank[e]] = static_cast<unsigned short>(item[e]);
+  __syncthreads();
+  u32x4_t* dst = reinterpret_cast<u32x4_t*>(a.rec + static_cast<size_t>(blockIdx.x) * VS_CHUNK);
+  const u32x4_t* src = reinterpret_cast<const u32x4_t*>(rec);
+  for (int i = tid; i * 8 < total; i += VS_THREADS) dst[i] = src[i];      // (the tail past `total` is never read)
+}
+
+__global__ __launch_bounds__(VC_THREADS) void voxel_count_kernel(VoxelArgs a, int* __restrict__ out_hist, float* __restrict__ out_vox,
+                                                                 int signed_mode) {
+  extern __shared__ int cnt[];                     // [2][rows][W]
+  __shared__ int2 runs[VC_THREADS];                // first record and length
+  __shared__ int n_runs;
+  const int band = blockIdx.x, b = blockIdx.y, rows = 1 << a.log_rows, tid = threadIdx.x;
+  const int half = rows * a.W;
+  for (int i = tid; i < 2 * half; i += VC_THREADS) cnt[i] = 0;
+  const int lane = tid & 63;
+  for (int base = 0; base < a.chunks; base += VC_THREADS) {
+    if (tid == 0) n_runs = 0;
+    __syncthreads();
+    const int c = base + tid;
+    if (c < a.chunks) {
+      const int2 r = a.range[c];
+      if (r.x <= b && b <= r.y) {
+        const unsigned short* off = a.off + static_cast<size_t>(c) * (a.keys + 1) + (b - r.x) * a.bands + band;
+        const int s = off[0], len = off[1] - s;
+        if (len > 0) runs[atomicAdd(&n_runs, 1)] = make_int2(c * VS_CHUNK + s, len);
+      }
+    }
+    __syncthreads();
+    const int n = n_runs;
+    for (int j = tid >> 6; j < n; j += VC_THREADS / 64) {
+      const int2 r = runs[j];
+      const unsigned short* rec = a.rec + r.x;
+      for (int i = lane; i < r.y; i += 256) {      // four loads of a run in flight
+        int v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = i + u * 64 < r.y ? rec[i + u * 64] : -1;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (v[u] >= 0) atomicAdd(&cnt[v[u]], 1);
+      }
+    }
+    __syncthreads();
+  }
+  const int y0 = band << a.log_rows, cells = min(rows, a.H - y0) * a.W;
+  const size_t plane = static_cast<size_t>(a.H) * a.W, at = static_cast<size_t>(y0) * a.W;
+  int* hist = out_hist + static_cast<size_t>(b) * 2 * plane + at;
+  float* vox = out_vox + static_cast<size_t>(b) * plane + at;
+  for (int i = tid; i < cells; i += VC_THREADS) {
+    const int neg = cnt[i], pos = cnt[half + i];
+    hist[i] = neg;
+    hist[plane + i] = pos;
+    vox[i] = static_cast<float>(signed_mode ? pos - neg : pos + neg);
+  }
+}
+
+// log2 of the rows of a band: as many as fill 48 KB of counters, fewer while there are not two blocks per CU; -1 where
+// the image is too wide for a 16-bit place or the keys too many for the sort's counters
+int event_voxel_log_rows(int bins, int H, int W) {
+  if (W > 19200) return -1;
+  int l = 0;
+  while ((2ll << l) < H && (2ll << (l + 1)) * W * 4 <= 48 * 1024) ++l;
+  const auto blocks = [&](int k) { return static_cast<long long>(bins) * ((H + (1 << k) - 1) >> k); };
+  while (l > 0 && blocks(l) < 512 && blocks(l - 1) <= VS_KEYS) --l;
+  return blocks(l) <= VS_KEYS ? l : -1;
+}
+
+EventVoxelPlan event_voxel_plan(int n, int bins, int H, int W) {
+  EventVoxelPlan plan;
+  plan.log_rows = event_voxel_log_rows(bins, H, W);
+  plan.bands = plan.log_rows < 0 ? 0 : (H + (1 << plan.log_rows) - 1) >> plan.log_rows;
+  plan.chunks = static_cast<int>((static_cast<long long>(n) + VS_CHUNK - 1) / VS_CHUNK);
+  plan.off_bytes = 0;
+  plan.range_bytes = static_cast<size_t>(plan.chunks) * sizeof(int2);
+  plan.span_bytes = VS_SPANS * sizeof(VoxelSpan);
+  plan.rec_bytes = static_cast<size_t>(plan.chunks) * VS_CHUNK * 2;
+  plan.off_bytes = static_cast<size_t>(plan.chunks) * (bins * plan.bands + 1) * 2;
+  return plan;
+}
+
+void launch_event_voxel_sorted(const int* x, const int* y, const int* p, const long long* t, int n, int bins, int H, int W,
+                               const EventVoxelPlan& plan, unsigned char* work, int* out_hist, float* out_vox, int signed_mode,
+                               int by_count, hipStream_t st) {
+  VoxelArgs a;
+  a.x = x; a.y = y; a.p = p; a.t = t;
+  // records first: every chunk of them starts on 16 bytes
+  a.rec = reinterpret_cast<unsigned short*>(work);
+  VoxelSpan* span = reinterpret_cast<VoxelSpan*>(work + plan.rec_bytes);
+  a.span = span;
+  a.range = reinterpret_cast<int2*>(work + plan.rec_bytes + plan.span_bytes);
+  a.off = reinterpret_cast<unsigned short*>(work + plan.rec_bytes + plan.span_bytes + plan.range_bytes);
+  a.n = n; a.bins = bins; a.H = H; a.W = W; a.log_rows = plan.log_rows; a.bands = plan.bands; a.keys = bins * plan.bands;
+  a.chunks = plan.chunks; a.by_count = by_count;
+  if (!by_count) hipLaunchKernelGGL(voxel_span_kernel, dim3(VS_SPANS), dim3(1024), 0, st, t, n, span);
+  hipLaunchKernelGGL(voxel_sort_kernel, dim3(plan.chunks), dim3(VS_THREADS), 0, st, a);
+  const size_t smem = static_cast<size_t>(2) * (1 << plan.log_rows) * W * sizeof(int);
+  static bool attr_set = false;
+  if (!attr_set) {
+    hipFuncSetAttribute(reinterpret_cast<const void*>(&voxel_count_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024);  // (W = 19 200; the runs take 8 KB)
+    attr_set = true;
+  }
+  hipLaunchKernelGGL(voxel_count_kernel, dim3(plan.bands, bins), dim3(VC_THREADS), smem, st, a, out_hist, out_vox, signed_mode);
+}
+
 // --------------------------------------------------------- CLIP preprocessing
 // img: [T][H][W][3] uint8.  Two-pass fixed-point resample identical to PIL's
 // (horizontal pass with uint8 rounding, then vertical), restricted to the
