@@ -212,23 +212,92 @@ Tensor linear_t(const Tensor& a, const Tensor& w, bool a_t, bool w_t, const c10:
 // t [.., R] = alpha * x [.., K] · w [R, K]^T for a low-rank adapter's R <= 16 rows: one launch, no split-K pass.
 // x: contiguous, or 2-D with strided rows.  drop_p > 0: x is masked while it is loaded (keep mask of
 // (seed, element index), 1 / (1 - p) folded into alpha); lowrank_mask reproduces m (.) x for the backward.
-Tensor lowrank_out(const Tensor& x, const Tensor& w, double alpha, double drop_p, int64_t seed) {
-  check_bf16(w, "w");
-  TORCH_CHECK(w.dim() == 2 && x.dim() >= 1, "lowrank_out: w is [R, K]");
+// Several adapters that read the same x: one pass over it.
+std::vector<Tensor> lowrank_out_set(const Tensor& x, const std::vector<Tensor>& w, double alpha, double drop_p,
+                                    const std::vector<int64_t>& seeds) {
+  TORCH_CHECK(w.size() >= 1 && w.size() <= 3 && seeds.size() == w.size(), "lowrank_out: one to three adapters");
   const bool strided = x.dim() == 2 && !x.is_contiguous();
   if (strided) check_rows(x, "x"); else check_bf16(x, "x");
-  const int64_t K = x.size(-1), R = w.size(0), M = K ? x.numel() / K : 0;
-  TORCH_CHECK(w.size(1) == K && K % 8 == 0 && K >= 8, "lowrank_out: K mismatch or K % 8 != 0");
+  TORCH_CHECK(w[0].dim() == 2 && x.dim() >= 1, "lowrank_out: w is [R, K]");
+  const int64_t K = x.size(-1), R = w[0].size(0), M = K ? x.numel() / K : 0;
+  TORCH_CHECK(K % 8 == 0 && K >= 8, "lowrank_out: K mismatch or K % 8 != 0");
   TORCH_CHECK(R >= 1 && R <= 16, "lowrank_out: 1 <= R <= 16");
   TORCH_CHECK(M < (1ll << 31) / 16 && x.numel() < (1ll << 40), "lowrank_out: too many rows");
   TORCH_CHECK(drop_p >= 0 && drop_p < 1, "lowrank_out: 0 <= drop_p < 1");
   auto sizes = x.sizes().vec();
   sizes.back() = R;
-  Tensor y = at::empty(sizes, x.options());
+  std::vector<Tensor> out;
+  evgpt::LowrankSet set{};
+  set.n = (int)w.size();
+  for (int i = 0; i < set.n; ++i) {
+    check_bf16(w[i], "w");
+    TORCH_CHECK(w[i].dim() == 2 && w[i].size(0) == R && w[i].size(1) == K, "lowrank_out: K mismatch or K % 8 != 0");
+    out.push_back(at::empty(sizes, x.options()));
+    set.b[i] = bptr(w[i]);
+    set.out[i] = bptr_mut(out.back());
+    set.seed[i] = (unsigned long long)seeds[i];
+  }
   if (M > 0)
-    evgpt::launch_lowrank_out(bptr(x), bptr(w), bptr_mut(y), (int)M, (int)R, (int)K, strided ? x.stride(0) : K,
-                              (float)alpha, (float)drop_p, (unsigned long long)seed, cur_stream());
-  return y;
+    evgpt::launch_lowrank_out(bptr(x), set, (int)M, (int)R, (int)K, strided ? x.stride(0) : K, (float)alpha, (float)drop_p, cur_stream());
+  return out;
+}
+Tensor lowrank_out(const Tensor& x, const Tensor& w, double alpha, double drop_p, int64_t seed) {
+  return lowrank_out_set(x, {w}, alpha, drop_p, {seed})[0];
+}
+
+// the rank-r intermediates of a set of adapters over M rows
+static evgpt::LowrankSet lowrank_inputs(const std::vector<Tensor>& t, const std::vector<int64_t>& seeds, int64_t M, const char* what) {
+  evgpt::LowrankSet set{};
+  TORCH_CHECK(t.size() >= 1 && t.size() <= 3 && (seeds.empty() || seeds.size() == t.size()), what, ": one to three adapters");
+  set.n = (int)t.size();
+  const int64_t R = t[0].size(-1);
+  TORCH_CHECK(R == 8 || R == 16, what, ": rank 8 or 16");
+  for (int i = 0; i < set.n; ++i) {
+    check_bf16(t[i], "t");
+    TORCH_CHECK(t[i].size(-1) == R && t[i].numel() == M * R, what, ": t is [rows, rank]");
+    set.t[i] = bptr(t[i]);
+    set.seed[i] = seeds.empty() ? 0ull : (unsigned long long)seeds[i];
+  }
+  return set;
+}
+
+// y [M, N] (rows may be strided) += sum of m_i (.) (t_i [M, R] · b_i^T) in place; b_i [N, R], or [R, N] when transposed (only
+// then masks and several adapters).
+void lowrank_add_(const std::vector<Tensor>& t, const std::vector<Tensor>& b, bool transposed, const Tensor& y, double drop_p,
+                  const std::vector<int64_t>& seeds) {
+  check_rows(y, "y");
+  const int64_t M = y.size(0), N = y.size(1);
+  evgpt::LowrankSet set = lowrank_inputs(t, seeds, M, "lowrank_add_");
+  const int64_t R = t[0].size(-1);
+  TORCH_CHECK(b.size() == t.size() && N % 8 == 0 && drop_p >= 0 && drop_p < 1, "lowrank_add_: shapes");
+  TORCH_CHECK(transposed || (set.n == 1 && drop_p == 0), "lowrank_add_: masks and several adapters take b as [R, N]");
+  TORCH_CHECK(drop_p == 0 || (y.is_contiguous() && !seeds.empty()), "lowrank_add_: masks belong to a contiguous y");
+  for (int i = 0; i < set.n; ++i) {
+    check_bf16(b[i], "b");
+    TORCH_CHECK(b[i].dim() == 2 && b[i].size(0) == (transposed ? R : N) && b[i].size(1) == (transposed ? N : R), "lowrank_add_: b");
+    set.b[i] = bptr(b[i]);
+  }
+  TORCH_CHECK((M + 63) / 64 <= 65535, "lowrank_add_: too many rows");
+  evgpt::launch_lowrank_add(set, bptr_mut(y), (int)M, (int)N, (int)R, y.stride(0), transposed, (float)drop_p, cur_stream());
+}
+
+// out_i = t_i [M, R]^T · (m_i (.) g [M, C]), written [R, C], or [C, R] when transposed; g's rows may be strided
+void lowrank_wgrad_(const Tensor& g, const std::vector<Tensor>& t, const std::vector<Tensor>& out, bool transposed, double drop_p,
+                    const std::vector<int64_t>& seeds) {
+  check_rows(g, "g");
+  const int64_t M = g.size(0), C = g.size(1);
+  evgpt::LowrankSet set = lowrank_inputs(t, seeds, M, "lowrank_wgrad_");
+  const int64_t R = t[0].size(-1);
+  TORCH_CHECK(out.size() == t.size() && M >= 1 && C % 8 == 0 && drop_p >= 0 && drop_p < 1, "lowrank_wgrad_: shapes");
+  TORCH_CHECK(drop_p == 0 || (g.is_contiguous() && !seeds.empty()), "lowrank_wgrad_: masks belong to a contiguous g");
+  for (int i = 0; i < set.n; ++i) {
+    TORCH_CHECK(out[i].is_cuda() && out[i].is_contiguous() && out[i].scalar_type() == at::kBFloat16 && out[i].dim() == 2 &&
+                out[i].size(0) == (transposed ? C : R) && out[i].size(1) == (transposed ? R : C), "lowrank_wgrad_: out");
+    set.out[i] = reinterpret_cast<evgpt::bf16_t*>(out[i].data_ptr());
+  }
+  Tensor part = at::empty({evgpt::lowrank_wgrad_slabs((int)M, (int)C), set.n, R, C}, g.options().dtype(at::kFloat));
+  evgpt::launch_lowrank_wgrad(bptr(g), set, part.data_ptr<float>(), (int)M, (int)C, (int)R, g.stride(0), transposed, (float)drop_p,
+                              cur_stream());
 }
 
 // m (.) x with lowrank_out's keep mask (no rescaling); contiguous, a multiple of 8 elements
@@ -1373,6 +1442,9 @@ TORCH_LIBRARY(evgpt, m) {
   m.def("linear_swiglu(Tensor x, Tensor w_gate_up) -> Tensor", &linear_swiglu);
   m.def("linear_partial(Tensor x, Tensor w, int max_split=0) -> Tensor", &linear_partial);
   m.def("lowrank_out(Tensor x, Tensor w, float alpha, float drop_p=0.0, int seed=0) -> Tensor", &lowrank_out);
+  m.def("lowrank_out_set(Tensor x, Tensor[] w, float alpha, float drop_p, int[] seeds) -> Tensor[]", &lowrank_out_set);
+  m.def("lowrank_add_(Tensor[] t, Tensor[] b, bool transposed, Tensor(a!) y, float drop_p, int[] seeds) -> ()", &lowrank_add_);
+  m.def("lowrank_wgrad_(Tensor g, Tensor[] t, Tensor(a!)[] out, bool transposed, float drop_p, int[] seeds) -> ()", &lowrank_wgrad_);
   m.def("lowrank_mask(Tensor x, float drop_p, int seed) -> Tensor", &lowrank_mask);
   m.def("lowrank_mask_add_(Tensor(a!) acc, Tensor x, float drop_p, int seed) -> ()", &lowrank_mask_add_);
   m.def("linear_rows_(Tensor x, Tensor w, Tensor(a!) out, bool accumulate) -> ()", &linear_rows_);

@@ -175,9 +175,15 @@ void launch_layernorm(const bf16_t* x, const bf16_t* w, const bf16_t* b, bf16_t*
 void launch_rope_kv_prefill(const bf16_t* qkv, bf16_t* q_out, bf16_t* k_cache, bf16_t* v_cache,
                             const float* cos_tab, const float* sin_tab, const int* pos0, int B,
                             int S, int Hq, int Hkv, int D, int l_max, hipStream_t st);
-// C [M, R] = alpha * A [M, K] · W [R, K]^T for R <= 16 and K % 8 == 0 (rank-r projection of a low-rank adapter)
-void launch_lowrank_out(const bf16_t* A, const bf16_t* W, bf16_t* C, int M, int R, int K, long long lda, float alpha,
-                        float drop_p, unsigned long long seed, hipStream_t st);
+// up to three low-rank adapters of one projection: rank-r intermediates t, matrices b, outputs, mask seeds
+struct LowrankSet { const bf16_t* t[3]; const bf16_t* b[3]; bf16_t* out[3]; unsigned long long seed[3]; int n; };
+// out_i [M, R] = alpha * A [M, K] · b_i [R, K]^T for R <= 16 and K % 8 == 0 (rank-r projections of low-rank adapters)
+void launch_lowrank_out(const bf16_t* A, const LowrankSet& set, int M, int R, int K, long long lda, float alpha, float drop_p,
+                        hipStream_t st);
+void launch_lowrank_add(const LowrankSet& set, bf16_t* Y, int M, int N, int R, long long ldy, bool trans, float drop_p, hipStream_t st);
+int lowrank_wgrad_slabs(int M, int C);      // fp32 slabs [n, R, C] the call below wants in `part`
+void launch_lowrank_wgrad(const bf16_t* G, const LowrankSet& set, float* part, int M, int C, int R, long long ldg, bool transposed,
+                          float drop_p, hipStream_t st);
 void launch_lowrank_mask(const bf16_t* x, bf16_t* y, long long n, float drop_p, unsigned long long seed, bool add,
                          hipStream_t st);
 void launch_rope_qkv(const bf16_t* packed_in, bf16_t* packed_out, bf16_t* q, bf16_t* k, bf16_t* v,

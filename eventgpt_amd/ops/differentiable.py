@@ -566,15 +566,24 @@ def _lora_projection_forward(x, weight, residual, scale, drop_p, offsets, ab):
     x2 = xc.view(-1, k)
     y = hip.linear(xc, weight, None, None, residual)
     y2 = y.view(-1, y.shape[-1])
-    ts, seeds = [], []
-    for i, off in enumerate(offsets):
-        a, b = ab[2 * i], ab[2 * i + 1]
-        seed = next_seed() if drop_p > 0 else 0
-        t = raw.lowrank_out(x2, a, scale, drop_p, seed)                  # [M, r], scale / (1 - p) applied
-        raw.linear_rows_(t, b, y2[:, off:off + b.shape[0]], True)
-        ts.append(t)
-        seeds.append(seed)
+    seeds = [next_seed() if drop_p > 0 else 0 for _ in offsets]
+    ts = []
+    for group in _adapter_groups(ab):                                    # one pass over x for adapters of one rank
+        ts += raw.lowrank_out_set(x2, [ab[2 * i] for i in group], scale, drop_p, [seeds[i] for i in group])
+    for off, t, b in zip(offsets, ts, ab[1::2]):                         # t [M, r], scale / (1 - p) applied
+        raw.lowrank_add_([t], [b], False, y2[:, off:off + b.shape[0]], 0.0, [])
     return y, x2, ts, seeds
+
+
+def _adapter_groups(ab):
+    """Adapters ``ab = [A0, B0, A1, B1, ..]`` in runs of up to three of one rank: what one launch takes."""
+    groups = []
+    for i in range(len(ab) // 2):
+        if groups and len(groups[-1]) < 3 and ab[2 * groups[-1][0]].shape[0] == ab[2 * i].shape[0]:
+            groups[-1].append(i)
+        else:
+            groups.append([i])
+    return groups
 
 
 class _LoRAProjection(torch.autograd.Function):
@@ -584,11 +593,11 @@ class _LoRAProjection(torch.autograd.Function):
     keep mask.  One node instead of a dropout, a rank-r node, a strided add and their backward copies per
     adapter:
 
-    * forward: base GEMM (residual in its epilogue), then per adapter the rank-r kernel with the mask applied
-      while ``x`` is loaded and a GEMM that accumulates ``t_i B_i^T`` in place onto its column block;
+    * forward: base GEMM (residual in its epilogue), then one pass over ``x`` for the rank-r intermediates of all
+      adapters, the masks applied while it is loaded, and per adapter a pass that adds ``t_i B_i^T`` onto its columns;
     * backward: the base input gradient, then per adapter ``dt_i`` and ``dB_i`` read the incoming gradient's
-      column block where it is (row-strided operands), ``dA_i`` contracts with ``m_i (.) x`` recomputed from
-      the seed, and ``m_i (.) (dt_i A_i)`` is accumulated onto the input gradient in place.
+      column block where it is (row-strided operands); one pass over ``x`` gives every ``dA_i`` (masks recomputed
+      from the seeds while it is loaded) and one pass adds every ``m_i (.) (dt_i A_i)`` onto the input gradient.
 
     Saved per node: ``x`` once and the ``[rows, r]`` intermediates -- not one dropped copy of ``x`` per adapter."""
 
@@ -619,30 +628,26 @@ class _LoRAProjection(torch.autograd.Function):
                 dx2 = hip.linear(g2, wt)
             else:
                 dx2 = linear_dgrad(g2, weight.contiguous())
-        grads = []
         s_eff = scale / (1.0 - p)
-        kpad = _round64(g2.shape[0])
+        grads, dts = [None] * (2 * n_ad), [None] * n_ad
         for i, off in enumerate(offsets):
             a, b, t = ab[2 * i], ab[2 * i + 1], ts[i]
             gi = g2[:, off:off + b.shape[0]]                                  # a view: rows strided by ntot
-            need_a, need_b = ctx.needs_input_grad[6 + 2 * i], ctx.needs_input_grad[7 + 2 * i]
-            da = db = None
-            dt = None
-            if need_a or dx2 is not None:
-                dt = raw.lowrank_out(gi, b.detach().t().contiguous(), s_eff, 0.0, 0)      # s / (1 - p) * dY_i B_i
-            if need_b:
-                sink = _free_sink(b, gi)
-                db = raw.linear_t(gi, t, True, True, None, None, 0, False, kpad, sink)
-                db = db.view_as(b)
-            if need_a:
-                xm = raw.lowrank_mask(x2, p, seeds[i]) if p > 0 else x2
-                da = _wgrad_to_sink(a, dt, xm)
+            if ctx.needs_input_grad[6 + 2 * i] or dx2 is not None:
+                dts[i] = raw.lowrank_out(gi, b.detach().t().contiguous(), s_eff, 0.0, 0)  # s / (1 - p) * dY_i B_i
+            if ctx.needs_input_grad[7 + 2 * i]:
+                db = _free_sink(b, gi)
+                db = grads[2 * i + 1] = torch.empty_like(b) if db is None else db.view_as(b)
+                raw.lowrank_wgrad_(gi, [t], [db], True, 0.0, [])
+        for group in _adapter_groups(ab):
+            need = [i for i in group if ctx.needs_input_grad[6 + 2 * i]]
+            if need:
+                for i in need:
+                    da = _free_sink(ab[2 * i], g2)
+                    grads[2 * i] = torch.empty_like(ab[2 * i]) if da is None else da.view_as(ab[2 * i])
+                raw.lowrank_wgrad_(x2, [dts[i] for i in need], [grads[2 * i] for i in need], False, p, [seeds[i] for i in need])
             if dx2 is not None:
-                if p > 0:
-                    raw.lowrank_mask_add_(dx2, linear_dgrad(dt, a.detach().contiguous()), p, seeds[i])
-                else:
-                    raw.linear_t(dt, a.detach().contiguous(), False, True, None, dx2, 0, False, _round64(a.shape[0]), dx2)
-            grads += [da, db]
+                raw.lowrank_add_([dts[i] for i in group], [ab[2 * i].detach() for i in group], True, dx2, p, [seeds[i] for i in group])
         dx = None if dx2 is None else dx2.view(*gy.shape[:-1], x2.shape[1])
         return (dx, None, (gy if ctx.needs_input_grad[2] else None), None, None, None, *grads)
 

@@ -455,6 +455,42 @@ def test_lora_input_mask_statistics_and_fused_load(dev):
     assert torch.equal(acc, want)
 
 
+@pytest.mark.parametrize("M,C,R,n,p", [(1, 8, 8, 1, 0.0), (33, 136, 16, 2, 0.1), (257, 520, 8, 3, 0.2), (64, 256, 16, 1, 0.0),
+                                       (1030, 4096, 16, 3, 0.0), (700, 1032, 16, 1, 0.1)])
+def test_rank_r_update_and_weight_gradient_at_their_edges(dev, M, C, R, n, p):
+    """``y += sum m_i (.) t_i b_i^T`` in place and ``t_i^T (m_i (.) g)``: row and column remainders, rank 8 (half of an
+    MFMA's contraction is zeros), one to three adapters, masks, row-strided operands.  fp32 sums against double: the
+    result's own bf16 rounding (2^-8 of it) and 1e-5 of the sum of magnitudes."""
+    from eventgpt_amd.ops import hip
+    raw, seeds = hip.raw, [5 + i for i in range(n)]
+    t = [_rand(M, R, dev=dev, seed=i) for i in range(n)]
+    a = [_rand(R, C, dev=dev, seed=10 + i) for i in range(n)]
+    wide = _rand(M, C + 24, dev=dev, seed=30)
+    ones = torch.ones(M, C, dtype=torch.bfloat16, device=dev)
+    mask = [(raw.lowrank_mask(ones, p, s) if p > 0 else ones).double() for s in seeds]
+
+    def close(got, want, size):
+        assert bool(((got.double() - want).abs() <= want.abs() * 2 ** -8 + 1e-5 * size + 1e-30).all())
+    y = wide[:, 8:8 + C].contiguous()
+    want = y.double() + sum(m * (ti.double() @ ai.double()) for m, ti, ai in zip(mask, t, a))
+    size = y.double().abs() + sum(ti.double().abs() @ ai.double().abs() for ti, ai in zip(t, a))
+    raw.lowrank_add_(t, a, True, y, p, seeds)
+    close(y, want, size)
+    y = wide.clone()
+    raw.lowrank_add_(t[:1], [a[0].t().contiguous()], False, y[:, 8:8 + C], 0.0, [])
+    close(y[:, 8:8 + C], wide[:, 8:8 + C].double() + t[0].double() @ a[0].double(), wide[:, 8:8 + C].double().abs()
+          + t[0].double().abs() @ a[0].double().abs())
+    assert torch.equal(y[:, :8], wide[:, :8]) and torch.equal(y[:, 8 + C:], wide[:, 8 + C:])
+    g = wide[:, 8:8 + C] if p == 0 else wide[:, 8:8 + C].contiguous()
+    out = [torch.empty(R, C, dtype=torch.bfloat16, device=dev) for _ in range(n)]
+    raw.lowrank_wgrad_(g, t, out, False, p, seeds)
+    for o, ti, m in zip(out, t, mask):
+        close(o, ti.double().t() @ (g.double() * m), ti.double().abs().t() @ g.double().abs())
+    out_t = [torch.empty(C, R, dtype=torch.bfloat16, device=dev) for _ in range(n)]
+    raw.lowrank_wgrad_(g, t, out_t, True, p, seeds)
+    assert all(torch.equal(o.t(), ot) for o, ot in zip(out, out_t))
+
+
 @pytest.mark.parametrize("p,single", [(0.0, False), (0.1, False), (0.1, True), (0.0, True)])
 def test_lora_projection_node_against_fp32(dev, p, single):
     """Frozen projection + low-rank adapters on column ranges as one autograd node: output, input gradient,
