@@ -294,6 +294,10 @@ void launch_attn_decode(const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_
                         int Hkv, int D, int l_max, int nsplit, float scale, hipStream_t st, int ring = 0);
 
 // ---- attn_prefill.hip
+// causal attention inside chunks, one block per entry of items [n][4] and head: first query row, rows (<= 64), key row of the
+// chunk, position of the first row in it; two-part softmax weights; head size 64 or 128, rows of q and o Hq * D apart
+void launch_attn_items(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf16_t* o, const int* items, int n_items, int Hq, int Hkv,
+                       int D, long long kld, float scale, const bf16_t* gate, int gate_ld, hipStream_t st);
 void launch_attn_prefill(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf16_t* o,
                          const long long* strides, const int* kv_len, int B, int Sq, int Sk,
                          int Hq, int Hkv, int D, int causal, int q_offset, int q_offset_from_len,

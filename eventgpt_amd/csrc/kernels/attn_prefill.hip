@@ -48,9 +48,10 @@ struct AttnParams {
                                 // scaled-log2 domain (max + log2(sum)); the backward recomputes P from it
   const bf16_t* gate;           // optional [B * Sq][gate_ld]: head h's output is multiplied by sigmoid of column h
   int gate_ld;
+  const int* items;             // ITEMS: [blocks][4] first query row, rows (<= 64), key row of the chunk, position in it
 };
-__device__ __forceinline__ float head_gate(const AttnParams& p, int b, int qi, int h) {
-  return 1.f / (1.f + __expf(-bf16_to_f32(p.gate[(static_cast<long long>(b) * p.Sq + qi) * p.gate_ld + h])));
+__device__ __forceinline__ float head_gate(const AttnParams& p, long long row, int h) {
+  return 1.f / (1.f + __expf(-bf16_to_f32(p.gate[row * p.gate_ld + h])));
 }
 
 // GROUPS = 2: the block is two such groups of 4 waves over the SAME 64 query rows; group 0 takes the
@@ -59,7 +60,10 @@ __device__ __forceinline__ float head_gate(const AttnParams& p, int b, int qi, i
 // few hundred query rows of a few heads are fewer blocks than CUs, each a serial chain over its key
 // tiles; two groups halve the chain and double the waves (used for the ViT, see launch_attn_prefill).
 // WP: the softmax weights enter the second product as two bf16 parts (16 mantissa bits) instead of one.
-template <int D, bool CAUSAL, bool SPLIT = false, int GROUPS = 1, bool WP = false>
+// ITEMS: block x takes the query rows, keys and position of an entry of `items`, so runs of any lengths and sequences share
+// a launch.  Eight prompts of 342 to 682 tokens, 32 heads of 128: one launch a prompt 170 us a layer, one for all 80; 32 prompts of
+// 200, 16 heads: 52 (148 with the 64-column blocks of attn_chunk.hip).
+template <int D, bool CAUSAL, bool SPLIT = false, int GROUPS = 1, bool WP = false, bool ITEMS = false>
 __global__ __launch_bounds__(256 * GROUPS) void attn_prefill_kernel(AttnParams p) {
   constexpr int CPR = D / 8;                  // 16-byte chunks per row
   constexpr int TILE_BYTES = TK * D * 2;
@@ -80,8 +84,18 @@ __global__ __launch_bounds__(256 * GROUPS) void attn_prefill_kernel(AttnParams p
   // a device-side key count can never address past the buffer capacity p.Sk
   int Sk = p.kv_len ? p.kv_len[b] : p.Sk;
   Sk = Sk > p.Sk ? p.Sk : (Sk < 0 ? 0 : Sk);
-  const int q_off = p.q_offset_from_len ? (Sk - p.Sq) : p.q_offset;
-  const int qb0 = SPLIT ? 0 : blockIdx.x * 64;  // first query row of the block
+  int q_off = p.q_offset_from_len ? (Sk - p.Sq) : p.q_offset;
+  long long row0 = static_cast<long long>(b) * p.Sq;      // the block's rows in the gate
+  if constexpr (ITEMS) {                       // (p is this thread's copy)
+    const int* it = p.items + (gridDim.x - 1 - blockIdx.x) * 4;      // a sequence's last rows see the most keys: first
+    row0 = it[0];
+    q_off = it[3];
+    p.Sq = min(it[1], 64);
+    Sk = q_off + p.Sq;
+    p.q += row0 * p.q_ss; p.o += row0 * p.o_ss;
+    p.k += static_cast<long long>(it[2]) * p.k_ss; p.v += static_cast<long long>(it[2]) * p.v_ss;
+  }
+  const int qb0 = SPLIT || ITEMS ? 0 : blockIdx.x * 64;  // first query row of the block
   const int qi = qb0 + wid * 16 + fr;        // this lane's query row
   const int qi_c = qi < p.Sq ? qi : p.Sq - 1;
 
@@ -295,7 +309,7 @@ __global__ __launch_bounds__(256 * GROUPS) void attn_prefill_kernel(AttnParams p
     return;
   }
   float inv = l > 0.f ? 1.f / l : 0.f;
-  if (p.gate && qi < p.Sq) inv *= head_gate(p, b, qi, h);
+  if (p.gate && qi < p.Sq) inv *= head_gate(p, row0 + qi, h);
   if (p.lse && g == 0 && qi < p.Sq)
     p.lse[(static_cast<long long>(b) * p.Hq + h) * p.Sq + qi] = l > 0.f ? m * p.scale_log2e + log2f(l) : INFINITY;
   if (qi < p.Sq) {
@@ -556,7 +570,7 @@ __global__ __launch_bounds__(AW_WAVES * 64) void attn_prefill_wide_kernel(AttnPa
     lt += __shfl_xor(lt, 32, 64);
     float inv = lt > 0.f ? 1.f / lt : 0.f;
     if (qi[qt] >= p.Sq) continue;
-    if (p.gate) inv *= head_gate(p, b, qi[qt], h);
+    if (p.gate) inv *= head_gate(p, static_cast<long long>(b) * p.Sq + qi[qt], h);
     if (p.lse && g == 0)
       p.lse[(static_cast<long long>(b) * p.Hq + h) * p.Sq + qi[qt]] = lt > 0.f ? m[qt] * p.scale_log2e + log2f(lt) : INFINITY;
     bf16_t* op = p.o + b * p.o_sb + static_cast<long long>(qi[qt]) * p.o_ss + h * p.o_sh;
@@ -601,6 +615,20 @@ __global__ __launch_bounds__(D) void attn_split_combine_kernel(AttnParams p) {
   }
   bf16_t* op = p.o + b * p.o_sb + static_cast<long long>(qi) * p.o_ss + h * p.o_sh;
   op[d] = f32_to_bf16(l > 0.f ? acc / l : 0.f);
+}
+
+void launch_attn_items(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf16_t* o, const int* items, int n_items, int Hq, int Hkv,
+                       int D, long long kld, float scale, const bf16_t* gate, int gate_ld, hipStream_t st) {
+  AttnParams p{};
+  p.q = q; p.k = k; p.v = v; p.o = o;
+  p.q_ss = p.o_ss = static_cast<long long>(Hq) * D;
+  p.k_ss = p.v_ss = kld;
+  p.q_sh = p.k_sh = p.v_sh = p.o_sh = D;
+  p.Hq = Hq; p.Hkv = Hkv; p.items = items; p.gate = gate; p.gate_ld = gate_ld;
+  p.scale_log2e = scale * 1.4426950408889634f;
+  const dim3 grid(n_items, Hq), block(256);
+  if (D == 128) hipLaunchKernelGGL((attn_prefill_kernel<128, true, false, 1, true, true>), grid, block, 0, st, p);
+  else hipLaunchKernelGGL((attn_prefill_kernel<64, true, false, 1, true, true>), grid, block, 0, st, p);
 }
 
 static int g_attn_groups = 0;  // key-tile groups per 64-row block: 0 = by shape, 1 / 2 = forced (tests, tuning)

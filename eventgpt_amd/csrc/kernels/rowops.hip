@@ -420,6 +420,37 @@ void launch_commit_rows(const float* logits, long long ld_logits, int* sampled, 
                        vocab, active);
 }
 
+// Given tokens enter a decode step in one launch: the slots' tokens, and the mask of who advances.
+__global__ __launch_bounds__(256) void feed_rows_kernel(RowList r, const int* __restrict__ tok, int* __restrict__ sampled,
+                                                        int* __restrict__ active, int clear, int B) {
+  if (active && clear) {
+    for (int b = threadIdx.x; b < B; b += 256) active[b] = 0;
+    __syncthreads();
+  }
+  if (static_cast<int>(threadIdx.x) >= r.n) return;
+  const int s = r.row[threadIdx.x];
+  sampled[s] = tok ? tok[threadIdx.x] : r.value[threadIdx.x];
+  if (active) active[s] = 1;
+}
+void launch_feed_rows(const RowList& r, const int* tok, int* sampled, int* active, bool clear, int B, hipStream_t st) {
+  hipLaunchKernelGGL(feed_rows_kernel, dim3(1), dim3(256), 0, st, r, tok, sampled, active, clear ? 1 : 0, B);
+}
+
+__global__ __launch_bounds__(256) void take_rows_kernel(const float* __restrict__ x, RowList r, float* __restrict__ y, long long N) {
+  const float* src = x + r.row[blockIdx.y] * N;
+  float* dst = y + blockIdx.y * N;
+  if ((N & 3) == 0) {                    // (both bases are 16-byte aligned: whole rows are)
+    for (long long c = (blockIdx.x * 256ll + threadIdx.x) * 4; c < N; c += gridDim.x * 1024ll)
+      *reinterpret_cast<f32x4_t*>(dst + c) = *reinterpret_cast<const f32x4_t*>(src + c);
+  } else {
+    for (long long c = blockIdx.x * 256ll + threadIdx.x; c < N; c += gridDim.x * 256ll) dst[c] = src[c];
+  }
+}
+void launch_take_rows(const float* x, const RowList& r, float* y, long long N, hipStream_t st) {
+  const long long blocks = (N + 1023) / 1024;
+  hipLaunchKernelGGL(take_rows_kernel, dim3(blocks > 64 ? 64 : static_cast<int>(blocks), r.n), dim3(256), 0, st, x, r, y, N);
+}
+
 // Attention inputs of one row.  The q and k sections are read once, into LDS (STAGED; rows too wide for it are read
 // again instead), where an element finds the one it is rotated with.
 template <typename T, bool STAGED>

@@ -249,6 +249,41 @@ void commit_rows_(const OptTensor& logits, const Tensor& sampled, const Tensor& 
                             done.data_ptr<int>(), cur.data_ptr<int>(), (int)eos, (int)B, (int)x.size(1),
                             (int)embed.size(0), iptr(active), cur_stream());
 }
+// Per-slot buffers written from host lists without a copy to the device: the lists travel as kernel arguments.
+// sampled[slots[i]] = tokens[i] (or the device's tok[i]); with `active`, it becomes one at the slots and zero elsewhere
+void feed_rows_(const Tensor& sampled, const OptTensor& active, at::IntArrayRef slots, at::IntArrayRef tokens, const OptTensor& tok) {
+  check_i(sampled, "sampled");
+  const int64_t n = slots.size(), B = sampled.numel();
+  if (active.has_value()) { check_i(*active, "active"); TORCH_CHECK(active->numel() == B, "feed_rows: active"); }
+  if (tok.has_value()) { check_i(*tok, "tok"); TORCH_CHECK(tok->numel() == n && tokens.empty(), "feed_rows: one token per slot"); }
+  else TORCH_CHECK((int64_t)tokens.size() == n, "feed_rows: one token per slot");
+  for (int64_t s : slots) TORCH_CHECK(s >= 0 && s < B, "feed_rows: slot ", s, " of ", B);
+  evgpt::RowList r;
+  for (int64_t i = 0; i == 0 || i < n; i += evgpt::ROW_LIST) {
+    r.n = (int)std::min<int64_t>(n - i, evgpt::ROW_LIST);
+    for (int j = 0; j < r.n; ++j) {
+      r.row[j] = (int)slots[i + j];
+      r.value[j] = tok.has_value() ? 0 : (int)tokens[i + j];
+    }
+    evgpt::launch_feed_rows(r, tok.has_value() ? tok->data_ptr<int>() + i : nullptr, sampled.data_ptr<int>(),
+                            active.has_value() ? active->data_ptr<int>() : nullptr, i == 0, (int)B, cur_stream());
+  }
+}
+// rows of x [B, N] fp32 (row stride a multiple of four) in order
+Tensor take_rows(const Tensor& x, at::IntArrayRef rows) {
+  check_f(x, "x");
+  TORCH_CHECK(x.dim() == 2, "take_rows: x [B, N]");
+  const int64_t n = rows.size(), B = x.size(0), N = x.size(1);
+  Tensor y = at::empty({n, N}, x.options());
+  for (int64_t s : rows) TORCH_CHECK(s >= 0 && s < B, "take_rows: row ", s, " of ", B);
+  evgpt::RowList r;
+  for (int64_t i = 0; i < n && N > 0; i += evgpt::ROW_LIST) {
+    r.n = (int)std::min<int64_t>(n - i, evgpt::ROW_LIST);
+    for (int j = 0; j < r.n; ++j) r.row[j] = (int)rows[i + j];
+    evgpt::launch_take_rows(x.data_ptr<float>(), r, y.data_ptr<float>() + i * N, N, cur_stream());
+  }
+  return y;
+}
 void sample_top_p(const Tensor& logits, const Tensor& out, double temperature, double top_p, int64_t seed,
                   const Tensor& step, int64_t top_k) {
   check_f(logits, "logits"); check_i(out, "out"); check_i(step, "step");
@@ -354,7 +389,11 @@ Tensor attn_chunk(const Tensor& q, const Tensor& k, const Tensor& v, const Tenso
   int64_t gld;
   const void* g = head_gates(gate, gcol, q, &gld);
   Tensor o = at::empty_like(q);
-  if (items.size(0) > 0)
+  if (items.size(0) > 0 && !is_f32(q) && (q.size(2) == 64 || q.size(2) == 128))
+    evgpt::launch_attn_items(bptr(q), bptr(k), bptr(v), bptr_mut(o), items.data_ptr<int>(), (int)items.size(0), (int)q.size(1),
+                             (int)k.size(1), (int)q.size(2), k.stride(0), (float)scale, static_cast<const evgpt::bf16_t*>(g), (int)gld,
+                             cur_stream());
+  else if (items.size(0) > 0)
     evgpt::launch_attn_chunk(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), items.data_ptr<int>(), (int)items.size(0),
                              is_f32(q), (int)q.size(1), (int)k.size(1), (int)q.size(2), k.stride(0), (float)scale, g, (int)gld,
                              cur_stream());
@@ -969,6 +1008,8 @@ TORCH_LIBRARY(evlay, m) {
   m.def("glu_rows(Tensor src, int act, bool f32) -> Tensor", &glu_rows);
   m.def("group_norm_rows(Tensor y, Tensor? gate, int gcol, int gate_mode, Tensor w, int heads, int v, int vp, int parts, int ld_out, float eps, bool f32) -> Tensor", &group_norm_rows);
   m.def("commit_rows_(Tensor? logits, Tensor(g!) sampled, Tensor embed, float scale, Tensor(a!) x, Tensor(b!) out_tokens, Tensor(c!) step, Tensor(d!) pos, Tensor(e!) done, Tensor(f!) cur_token, int eos, Tensor? active) -> ()", &commit_rows_);
+  m.def("feed_rows_(Tensor(a!) sampled, Tensor(b!)? active, int[] slots, int[] tokens, Tensor? tok=None) -> ()", &feed_rows_);
+  m.def("take_rows(Tensor x, int[] rows) -> Tensor", &take_rows);
   m.def("sample_top_p(Tensor logits, Tensor(a!) out, float temperature, float top_p, int seed, Tensor step, int top_k=0) -> ()", &sample_top_p);
   m.def("attn_prep_(Tensor src, int q_col, int k_col, int v_col, Tensor? qw, Tensor? kw, int Hq, int Hkv, int D, int nq, int nk, float eps, Tensor cos, Tensor sin, Tensor? row_slot, Tensor row_pos, Tensor? row_kv, Tensor? row_keep, Tensor(a!)? k_buf, Tensor(b!)? v_buf, Tensor(c!) k_cache, Tensor(d!) v_cache) -> Tensor", &attn_prep_);
   m.def("chunk_keys_copy_(Tensor k_cache, Tensor v_cache, Tensor(a!) k_buf, Tensor(b!) v_buf, Tensor copies) -> ()", &chunk_keys_copy_);

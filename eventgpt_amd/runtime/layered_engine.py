@@ -188,8 +188,8 @@ class LayeredEngine(DecodeEngine):
 
     @torch.no_grad()
     def _feed(self, slots, ids, starts, want=None):
-        """Append ``ids[i]`` to the sequences; returns the last residual row of each and the logits at the
-        wanted places (``want[i]``: places in ``ids[i]``) in order."""
+        """Append ``ids[i]`` to the sequences; returns the last residual row of each (without ``want``) and the logits at
+        the wanted places (``want[i]``: places in ``ids[i]``) in order."""
         ids = [t.reshape(-1) for t in ids]
         if any(t.numel() == 0 for t in ids):
             raise ValueError("an empty prompt has no last token to continue from")
@@ -199,7 +199,7 @@ class LayeredEngine(DecodeEngine):
             x, row0 = self._pack(p_slots, p_ids, p_starts)
             sel, keys = [], []
             for i, off, t, r in zip(idx, offs, p_ids, row0):
-                if off + t.numel() == ids[i].numel():
+                if want is None and off + t.numel() == ids[i].numel():
                     last[i] = x[r + t.numel() - 1].clone()
                 for w in (want[i] if want is not None else ()):
                     if off <= w < off + t.numel():
@@ -251,19 +251,22 @@ class LayeredEngine(DecodeEngine):
             self._fed[s] += int(t.numel())
         if not step:
             _, logits = self._feed(slots, tokens, starts, want)
-            for s in slots:
-                self.pos[s] = self._fed[s] - 1
+            self.raw.feed_rows_(self.pos, None, list(slots), [self._fed[s] - 1 for s in slots])
             self._pos_hi = max([self._pos_hi] + [self._fed[s] for s in slots])
             return logits
         if max(self._fed) > self.l_max:
             raise ValueError(f"sequence exceeds max_len ({self.l_max})")
-        self.active.zero_()
-        self.active[list(slots)] = 1
-        self.sampled[list(slots)] = torch.cat([t.reshape(-1) for t in tokens]).to(self.device, torch.int32)
+        # slots and host tokens travel as kernel arguments: nothing here waits for the device, so steps queue up behind each
+        # other (1b-size Nusitar, one stream: 500 us a token with index tensors and copies around the graph, 400 now)
+        if all(t.is_cuda for t in tokens):
+            tok = torch.cat([t.reshape(-1) for t in tokens]).to(torch.int32)
+            self.raw.feed_rows_(self.sampled, self.active, list(slots), [], tok.to(self.device))
+        else:
+            self.raw.feed_rows_(self.sampled, self.active, list(slots), [int(t) for t in tokens])
         self._commit_sampled()
         self.decode_step(greedy=False)
         rows = [s for s, w in zip(slots, want) for _ in w]
-        return self.logits[rows].clone() if rows else None
+        return self.raw.take_rows(self.logits, rows) if rows else None
 
     def release(self, slots: Sequence[int]) -> None:
         """Give the slots of finished sequences back."""

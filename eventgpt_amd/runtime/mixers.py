@@ -27,6 +27,14 @@ from ..models.layered import (AttentionSpec, DenseMLPSpec, LatentAttentionSpec, 
                               ParallelSpec)
 
 ATTN_TILE = 64           # query rows per work item of the chunk attention
+
+
+def long_run(rows: int, reps: int) -> bool:
+    """Runs of query rows that get a launch of their own: the 256-row blocks of the flash kernel want 1 400 rows, or several
+    runs of 512 (``attn_prefill.hip``); shorter runs of a pack share one launch of 64-row blocks."""
+    return rows >= 1400 or (reps > 1 and rows >= 512)
+
+
 GATE_NONE, GATE_SILU_BEFORE, GATE_SIGMOID_AFTER = 0, 1, 2      # group_norm_rows
 
 
@@ -111,13 +119,13 @@ class RowBatch:
         return flat.split([len(l) for l in lists])
 
     def chunk_tables(self, size: int):
-        """For a chunk mask of ``size``: ``(runs, items, row_kv, row_keep, copies, kv_rows)``.  Keys live in a buffer
-        with the rows of every sequence in order, preceded by the cached keys of the chunk it continues."""
+        """For a chunk mask of ``size``: ``(runs, items, row_kv, row_keep, copies, kv_rows)``, the items of ``long_run`` runs
+        last.  Keys live in a buffer with the rows of every sequence in order, preceded by the cached keys of the chunk it continues."""
         t = self._tables.get(size)
         if t is not None:
             return t
         runs: List[Tuple[int, int, int, int, int]] = []     # q row, rows, key row of the chunk, position in it, repeats
-        items: List[int] = []
+        items: Tuple[List[int], List[int]] = ([], [])       # of the short runs, of the long ones
         row_kv: List[int] = []
         keep: List[int] = []
         copies: List[int] = []
@@ -139,10 +147,10 @@ class RowBatch:
                 runs.append((s.row0 + done, n, key0, off, reps))
                 for r in range(reps):
                     for a in range(0, n, ATTN_TILE):
-                        items += [s.row0 + done + r * n + a, min(ATTN_TILE, n - a), key0 + r * n, off + a]
+                        items[long_run(n, reps)].extend((s.row0 + done + r * n + a, min(ATTN_TILE, n - a), key0 + r * n, off + a))
                 done += n * reps
             kv = base + s.rows
-        items_d, row_kv_d, keep_d, copies_d = self._upload(items, row_kv, keep, copies)
+        items_d, row_kv_d, keep_d, copies_d = self._upload(items[0] + items[1], row_kv, keep, copies)
         t = (runs, items_d.view(-1, 4), row_kv_d, keep_d, copies_d.view(-1, 4) if copies else None, kv)
         self._tables[size] = t
         return t
@@ -153,16 +161,16 @@ class RowBatch:
         t = self._tables.get("causal")
         if t is None:
             runs: List[Tuple[int, int, int, int, int]] = []
-            items: List[int] = []
+            items: Tuple[List[int], List[int]] = ([], [])
             copies: List[int] = []
             kv = 0
             for s in self.seqs:
                 runs.append((s.row0, s.rows, kv, s.start, 1))
                 for a in range(0, s.rows, ATTN_TILE):
-                    items += [s.row0 + a, min(ATTN_TILE, s.rows - a), kv, s.start + a]
+                    items[long_run(s.rows, 1)].extend((s.row0 + a, min(ATTN_TILE, s.rows - a), kv, s.start + a))
                 copies += [s.slot, 0, kv, s.start + s.rows]
                 kv += s.start + s.rows
-            items_d, copies_d = self._upload(items, copies)
+            items_d, copies_d = self._upload(items[0] + items[1], copies)
             t = self._tables["causal"] = (runs, items_d.view(-1, 4), copies_d.view(-1, 4), kv)
         return t
 
@@ -287,6 +295,18 @@ class Mixer:
         return stream.few and stream.x.shape[0] * k + 4096 <= self._lds
 
 
+def attend_runs(raw, q, k, v, runs, items, scale: float, flash: bool, *gate) -> torch.Tensor:
+    """Causal attention of a pack's runs, ``[rows, H * D]``: a launch of the flash kernel for each long run if it takes the
+    heads, one launch for all others (``RowBatch.chunk_tables``)."""
+    short = sum(-(-n // ATTN_TILE) * reps for _, n, _, _, reps in runs if not long_run(n, reps)) if flash else len(items)
+    o = raw.attn_chunk(q, k, v, items[:short], scale, *gate)
+    if flash:
+        for q0, n, key0, off, reps in runs:
+            if long_run(n, reps):
+                raw.attn_runs_(q, k, v, o, q0, n, key0, off, reps, scale, *gate)
+    return o.view(o.shape[0], -1)
+
+
 class AttentionBranch(Mixer):
     def __init__(self, engine, spec: AttentionSpec, t):
         """``t(name)``: the layer's tensor of that name."""
@@ -326,14 +346,7 @@ class AttentionBranch(Mixer):
         lq, lk, lv, H, G, D, nq, nk = self.dims(col)
         q = raw.attn_prep_(src, lq, lk, lv, self.qw, self.kw, H, G, D, nq, nk, self.eps, self.cos, self.sin, rows.slot,
                            rows.pos, row_kv, keep, k, v, self.k_cache, self.v_cache)
-        # few long runs: the flash kernel, one launch each; many short ones: one launch for all
-        if not self.f32 and D <= 128 and len(runs) <= 4 * len(rows.seqs) and max(r[1] for r in runs) > 256:
-            o = torch.empty_like(q)
-            for q0, n, key0, off, reps in runs:
-                raw.attn_runs_(q, k, v, o, q0, n, key0, off, reps, s.scale)
-        else:
-            o = raw.attn_chunk(q, k, v, items, s.scale)
-        return o.view(o.shape[0], -1)
+        return attend_runs(raw, q, k, v, runs, items, s.scale, not self.f32 and D <= 128)
 
 
 class MatrixMemoryBranch(Mixer):
@@ -515,14 +528,7 @@ class LatentAttentionMixer(Mixer):
         runs, items, _, kv_rows = rows.causal_tables()
         kv = raw.linear(rows.latents(self.owner.cache, raw.latent_gather), self.w_ukv, False)
         q, k, v = q.view(-1, H, D), kv[:, :H * D].unflatten(1, (H, D)), kv[:, H * D:].unflatten(1, (H, D))
-        gate = (src, self.proj.col["g"])
-        if not self.f32 and D <= 128 and max(r[1] for r in runs) > 256:
-            o = torch.empty_like(q)
-            for q0, n, key0, off, reps in runs:
-                raw.attn_runs_(q, k, v, o, q0, n, key0, off, reps, s.scale, *gate)
-        else:
-            o = raw.attn_chunk(q, k, v, items, s.scale, *gate)
-        return o.view(o.shape[0], -1)
+        return attend_runs(raw, q, k, v, runs, items, s.scale, not self.f32 and D <= 128, src, self.proj.col["g"])
 
     def forward(self, rows: RowBatch, stream: Stream, norm: torch.Tensor) -> None:
         raw, s, col = self.raw, self.spec, self.proj.col

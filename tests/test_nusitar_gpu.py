@@ -529,6 +529,49 @@ def test_chunk_attention(raw, dev, dtype, H, G, D, size):
         assert N.rel_err(o.view(len(lens), -1), want[last.cpu()]) < tol
 
 
+def test_packs_of_long_and_short_runs_share_the_item_launch(raw, dev):
+    """Runs that take the wide blocks get a launch each, the others one launch over their items (remainders of one row
+    to a full tile, gated heads): the same rows as the wide and 64-row kernels give run by run.  Both kernels carry the
+    weights as two bf16 parts and round the output once; row maxima are taken in another order: 2^-8 of a row's size."""
+    from eventgpt_amd.runtime import mixers
+    H, G, D, scale = 8, 2, 128, 128 ** -0.5
+    lens = [1, 1500, 63, 64, 65, 700, 128]
+    T = sum(lens)
+    q, k, v = (typed(rnd(T, n, D, seed=i), torch.bfloat16, dev)[0] for i, n in enumerate((H, G, G)))
+    gate = typed(rnd(T, 16, seed=4), torch.bfloat16, dev)[0]
+    for size in (4096, 600):                              # plain causal runs; chunks with repeats
+        runs, items, *_ = RowBatch(dev, False, seqs=pack(lens)).chunk_tables(size)
+        assert any(mixers.long_run(n, reps) for _, n, _, _, reps in runs)
+        want = torch.zeros_like(q)
+        for q0, n, key0, off, reps in runs:
+            raw.attn_runs_(q, k, v, want, q0, n, key0, off, reps, scale, gate, 8)
+        got = mixers.attend_runs(raw, q, k, v, runs, items, scale, True, gate, 8).view(T, H, D)
+        err = (got.float() - want.float()).norm(dim=-1) / want.float().norm(dim=-1)
+        assert float(err.max()) < 2 ** -8
+
+
+@pytest.mark.parametrize("B,n", [(1, 1), (5, 3), (130, 129)])
+def test_given_tokens_and_rows_travel_as_arguments(raw, dev, B, n):
+    """Slots in any order, more of them than one launch carries, tokens of the host and of the device."""
+    slots = torch.randperm(B, generator=torch.Generator().manual_seed(B))[:n].tolist()
+    for dev_tokens in (False, True):
+        sampled = torch.full((B,), -7, dtype=torch.int32, device=dev)
+        active = torch.full((B,), 3, dtype=torch.int32, device=dev)
+        tok = torch.arange(100, 100 + n, dtype=torch.int32)
+        raw.feed_rows_(sampled, active, slots, [] if dev_tokens else tok.tolist(), tok.to(dev) if dev_tokens else None)
+        want, on = torch.full((B,), -7, dtype=torch.int32), torch.zeros(B, dtype=torch.int32)
+        want[slots], on[slots] = tok, 1
+        assert torch.equal(sampled.cpu(), want) and torch.equal(active.cpu(), on)
+    for N in (7, 64, 5000):
+        x = rnd(B, N).float().to(dev)
+        rows = slots + slots[:1]
+        assert torch.equal(raw.take_rows(x, rows), x[rows])
+    with pytest.raises(RuntimeError):
+        raw.take_rows(x, [B])
+    with pytest.raises(RuntimeError):
+        raw.feed_rows_(sampled, None, [0], [1, 2])
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("size", [16, 64, 130, 400])
 def test_attention_sees_exactly_its_chunk(raw, dev, dtype, size):
