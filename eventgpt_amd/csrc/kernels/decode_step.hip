@@ -10,23 +10,46 @@
 
 namespace evgpt {
 
-// rows of S (of one head) from v0 on, vb of them: S = decay S + add v k^T, y = S q
+// The state rows a wave updates first (row wid * 4 + lane / 16 of the block, up to 256 columns): requested before the
+// position, gates and small vectors they are combined with have arrived.  The kernels are a chain of such round trips on a
+// few MB: one stream of 64 heads of 64 x 128 took 8.0 us with the rows requested behind the chain, 5.6 now
+// (the convolution's operands are requested together as well); 4 heads of 512 x 256 with 20 attention heads 7.9, now 6.8.
+constexpr int STATE_PRE = 4;
+struct StateRows { f32x4_t v[STATE_PRE]; };
+__device__ __forceinline__ StateRows request_state(const float* S, int N, int v0, int vb) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, i = wid * 4 + (lane >> 4);
+  StateRows r;
+  const float* Sr = S + static_cast<long long>(v0 + min(i, vb - 1)) * N;
+#pragma unroll
+  for (int u = 0; u < STATE_PRE; ++u) r.v[u] = load4(Sr + min((lane & 15) * 4 + u * 64, N - 4));
+  return r;
+}
+
+// rows of S (of one head) from v0 on, vb of them, by the block's first four waves: S = decay S + add v k^T, y = S q
 template <typename Y>
 __device__ __forceinline__ void stream_state(float* __restrict__ S, int N, int v0, int vb, bool fresh, float decay,
-                                             const float* qs, const float* ks, const float* avs, Y&& put) {
+                                             const float* qs, const float* ks, const float* avs, const StateRows& first, Y&& put) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, l16 = lane & 15, rg = lane >> 4;
+  if (wid >= 4) return;
   for (int i = wid * 4 + rg; i < vb; i += 16) {
     float* Sr = S + static_cast<long long>(v0 + i) * N;
     const float av = avs[i];
     float y = 0.f;
-    for (int e = l16 * 4; e < N; e += 64) {
+    const auto step = [&](int e, f32x4_t old) {
       const f32x4_t kk = *reinterpret_cast<const f32x4_t*>(ks + e), qq = *reinterpret_cast<const f32x4_t*>(qs + e);
       f32x4_t s = kk * av;
-      if (!fresh) s += load4(Sr + e) * decay;
+      if (!fresh) s += old * decay;
       *reinterpret_cast<f32x4_t*>(Sr + e) = s;
 #pragma unroll
       for (int j = 0; j < 4; ++j) y += s[j] * qq[j];
-    }
+    };
+    f32x4_t old[STATE_PRE];
+#pragma unroll
+    for (int u = 0; u < STATE_PRE; ++u) old[u] = i < 16 ? first.v[u] : load4(Sr + min(l16 * 4 + u * 64, N - 4));
+#pragma unroll
+    for (int u = 0; u < STATE_PRE; ++u)
+      if (l16 * 4 + u * 64 < N) step(l16 * 4 + u * 64, old[u]);
+    for (int e = l16 * 4 + STATE_PRE * 64; e < N; e += 64) step(e, load4(Sr + e));
     y = group_sum<16>(y);
     if (l16 == 0) put(i, y);
   }
@@ -90,11 +113,15 @@ __global__ __launch_bounds__(256) void parallel_step_kernel(StepHeads sh, StepMe
     for (int i = threadIdx.x; i < vb; i += 256) m.out[static_cast<long long>(gi) * m.V + v0 + i] = 0.f;
     return;
   }
+  float* S = m.S + static_cast<long long>(gi) * m.V * m.N;
+  const StateRows rows = request_state(S, m.N, v0, vb);
   const bool fresh = p <= 0;
   float *qs = lds, *ks = lds + m.N, *avs = ks + m.N;
   const long long from = (static_cast<long long>(p & 1) * m.slots + b) * m.H + h;
   const long long to = (static_cast<long long>((p + 1) & 1) * m.slots + b) * m.H + h;
-  if (threadIdx.x == 0) {
+  const float m_old = m.m[from];
+  const float n_old = m.n[from * m.N + min(static_cast<int>(threadIdx.x), m.N - 1)];
+  if (threadIdx.x == 255) {
     gates[0] = m.cap * tanhf((src1(m.src, b, m.i_col + h) + m.ib[h]) / m.cap);
     gates[1] = -softplus_f(-m.cap * tanhf((src1(m.src, b, m.f_col + h) + m.fb[h]) / m.cap));
   }
@@ -103,13 +130,13 @@ __global__ __launch_bounds__(256) void parallel_step_kernel(StepHeads sh, StepMe
     ks[e] = src_t<T>(m.src, b, m.k_col + h * m.N + e);
   }
   __syncthreads();
-  const float m0 = fresh ? 0.f : m.m[from];
+  const float m0 = fresh ? 0.f : m_old;
   const float li = gates[0], lf = gates[1], m1 = fmaxf(lf + m0, li);
   const float decay = expf(lf + m0 - m1), add = expf(li - m1);
   for (int i = threadIdx.x; i < vb; i += 256) avs[i] = add * src_t<T>(m.src, b, m.v_col + h * m.V + v0 + i);
   float dot = 0.f;
   for (int e = threadIdx.x; e < m.N; e += 256) {
-    const float n1 = (fresh ? 0.f : m.n[from * m.N + e] * decay) + add * ks[e];
+    const float n1 = (fresh ? 0.f : (e < 256 ? n_old : m.n[from * m.N + e]) * decay) + add * ks[e];
     if (v0 == 0) m.n[to * m.N + e] = n1;
     dot += n1 * qs[e];
   }
@@ -117,42 +144,56 @@ __global__ __launch_bounds__(256) void parallel_step_kernel(StepHeads sh, StepMe
   if (v0 == 0 && threadIdx.x == 0) m.m[to] = m1;
   const float inv = 1.f / (fmaxf(fabsf(dot), expf(-m1)) + 1e-6f);
   float* out = m.out + static_cast<long long>(gi) * m.V + v0;
-  stream_state(m.S + static_cast<long long>(gi) * m.V * m.N, m.N, v0, vb, fresh, decay, qs, ks, avs,
-               [&](int i, float y) { out[i] = y * inv; });
+  stream_state(S, m.N, v0, vb, fresh, decay, qs, ks, avs, rows, [&](int i, float y) { out[i] = y * inv; });
 }
 
+// threads: one per convolution channel of the block where that is at most 512 (the state takes four waves)
 template <typename T>
-__global__ __launch_bounds__(256) void ssd_step_kernel(StepSsd a, const int* __restrict__ pos, const int* __restrict__ live,
+__global__ __launch_bounds__(512) void ssd_step_kernel(StepSsd a, const int* __restrict__ pos, const int* __restrict__ live,
                                                        int vb) {
-  extern __shared__ __attribute__((aligned(16))) float lds[];      // [N] C, [N] B, [vb] weighted x, [vb] x
+  extern __shared__ __attribute__((aligned(16))) float lds[];      // [N] C, [N] B, [vb] weighted x, [vb] x, [vb] silu(z)
   __shared__ float gates[2];
   const int b = blockIdx.z, h = blockIdx.y, v0 = blockIdx.x * vb, p = pos[b];
-  const int gi = b * a.H + h, per_group = a.H / a.G, g = h / per_group;
+  const int gi = b * a.H + h, per_group = a.H / a.G, g = h / per_group, nt = blockDim.x;
   float* out = a.out + static_cast<long long>(gi) * a.V + v0;
   if (live && !live[b]) {
-    for (int i = threadIdx.x; i < vb; i += 256) out[i] = 0.f;
+    for (int i = threadIdx.x; i < vb; i += nt) out[i] = 0.f;
     return;
   }
+  float* S = a.S + static_cast<long long>(gi) * a.V * a.N;
+  const StateRows rows = request_state(S, a.N, v0, vb);
   const bool fresh = p <= 0;
-  float *cs = lds, *bs = lds + a.N, *avs = bs + a.N, *xs = avs + vb;
+  float *cs = lds, *bs = lds + a.N, *avs = bs + a.N, *xs = avs + vb, *zs = xs + vb;
   const int C = a.H * a.V + 2 * a.G * a.N;
-  if (threadIdx.x == 0) {
+  if (static_cast<int>(threadIdx.x) == nt - 1) {
     const float dt = softplus_f(src1(a.src, b, a.dt_col + h) + a.dt_bias[h]);
     gates[0] = expf(-expf(a.a_log[h]) * dt);
     gates[1] = dt;
   }
   T* ring = static_cast<T*>(a.ring) + static_cast<long long>(b) * a.taps * C;
-  for (int i = threadIdx.x; i < 2 * a.N + vb; i += 256) {
+  for (int i = threadIdx.x; i < 2 * a.N + vb; i += nt) {
     const bool is_x = i >= 2 * a.N;
     const int c = is_x ? h * a.V + v0 + i - 2 * a.N
                        : a.H * a.V + (i < a.N ? g * a.N + i : (a.G + g) * a.N + i - a.N);     // B, then C
-    const T cur = from_f32<T>(src1(a.src, b, a.x_col + c));
-    float acc = a.conv_b[c];
     const float* w = a.conv_w + static_cast<long long>(c) * a.taps;
-    for (int j = 0; j < a.taps; ++j) {
-      const int d = a.taps - 1 - j;
-      if (p - d < 0) continue;
-      acc += w[j] * (d == 0 ? to_f32(cur) : to_f32(ring[static_cast<long long>((p - d) % a.taps) * C + c]));
+    float acc = a.conv_b[c];
+    T cur;
+    if (a.taps == 4) {                  // (all operands on their way before the first product)
+      const f32x4_t w4 = load4(w);
+      T old[3];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) old[j] = ring[static_cast<long long>(max(p + j - 3, 0) & 3) * C + c];
+      cur = from_f32<T>(src1(a.src, b, a.x_col + c));
+#pragma unroll
+      for (int j = 0; j < 3; ++j) acc = fmaf(w4[j], p + j - 3 < 0 ? 0.f : to_f32(old[j]), acc);
+      acc = fmaf(w4[3], p < 0 ? 0.f : to_f32(cur), acc);
+    } else {
+      cur = from_f32<T>(src1(a.src, b, a.x_col + c));
+      for (int j = 0; j < a.taps; ++j) {
+        const int d = a.taps - 1 - j;
+        if (p - d < 0) continue;
+        acc = fmaf(w[j], d == 0 ? to_f32(cur) : to_f32(ring[static_cast<long long>((p - d) % a.taps) * C + c]), acc);
+      }
     }
     const float v = to_f32(from_f32<T>(acc * sigmoid_f(acc)));
     if (is_x) xs[i - 2 * a.N] = v;
@@ -163,13 +204,14 @@ __global__ __launch_bounds__(256) void ssd_step_kernel(StepSsd a, const int* __r
   }
   __syncthreads();
   const float decay = gates[0], dt = gates[1];
-  for (int i = threadIdx.x; i < vb; i += 256) avs[i] = dt * xs[i];
+  for (int i = threadIdx.x; i < vb; i += nt) {
+    avs[i] = dt * xs[i];
+    const float z = src_t<T>(a.src, b, a.z_col + h * a.V + v0 + i);
+    zs[i] = z * sigmoid_f(z);
+  }
   __syncthreads();
   const float skip = a.skip[h];
-  stream_state(a.S + static_cast<long long>(gi) * a.V * a.N, a.N, v0, vb, fresh, decay, cs, bs, avs, [&](int i, float y) {
-    const float z = src_t<T>(a.src, b, a.z_col + h * a.V + v0 + i);
-    out[i] = (y + skip * xs[i]) * z * sigmoid_f(z);
-  });
+  stream_state(S, a.N, v0, vb, fresh, decay, cs, bs, avs, rows, [&](int i, float y) { out[i] = (y + skip * xs[i]) * zs[i]; });
 }
 
 // state rows per block: sixteen keep a single stream's launch wide, more amortise the head's small vectors
@@ -190,9 +232,10 @@ void launch_parallel_step(const StepHeads& h, const StepMemory& m, const int* po
 void launch_ssd_step(const StepSsd& a, const int* pos, const int* live, bool f32, int B, hipStream_t st) {
   const int vb = rows_per_block(a.H, a.V, B);
   const dim3 grid(a.V / vb, a.H, B);
-  const size_t lds = (2 * a.N + 2 * vb) * 4;
-  if (f32) hipLaunchKernelGGL(ssd_step_kernel<float>, grid, dim3(256), lds, st, a, pos, live, vb);
-  else hipLaunchKernelGGL(ssd_step_kernel<bf16_t>, grid, dim3(256), lds, st, a, pos, live, vb);
+  const size_t lds = (2 * a.N + 3 * vb) * 4;
+  const int threads = min(512, max(256, (2 * a.N + vb + 63) / 64 * 64));
+  if (f32) hipLaunchKernelGGL(ssd_step_kernel<float>, grid, dim3(threads), lds, st, a, pos, live, vb);
+  else hipLaunchKernelGGL(ssd_step_kernel<bf16_t>, grid, dim3(threads), lds, st, a, pos, live, vb);
 }
 
 }  // namespace evgpt

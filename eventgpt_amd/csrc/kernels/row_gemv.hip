@@ -114,58 +114,119 @@ __device__ void store_latents(const LatentStore& s, int B) {
   }
 }
 
+// (every operand of the kept chunks is requested before the first sum; the two branches' sums meet behind one barrier)
 template <typename T>
 __device__ void prepare_merge(const GemvInput& in, int b, int K, T* xs, float* red, bool lead) {
   const long long o = static_cast<long long>(b) * K;
   const float* x = static_cast<const float*>(in.x) + o;
+  float xk[GV_KEEP][8], ak[GV_KEEP][8], bk[GV_KEEP][8], pk[GV_KEEP][8], qk[GV_KEEP][8], wk[GV_KEEP][8];
+  kept_chunks(K, [&](int k, int c) {
+    load8(in.a + o + c, ak[k]); load8(in.b + o + c, bk[k]); load8(x + c, xk[k]);
+    load8(in.wa + c, pk[k]); load8(in.wb + c, qk[k]); load8(in.w + c, wk[k]);
+  });
   float sa = 0.f, sb = 0.f;
-  for (int c = threadIdx.x * 8; c < K; c += 2048) {
+  kept_chunks(K, [&](int k, int) { sa += sumsq8(ak[k]); sb += sumsq8(bk[k]); });
+  for (int c = (threadIdx.x + GV_KEEP * 256) * 8; c < K; c += 2048) {
     float v[8];
     load8(in.a + o + c, v);
     sa += sumsq8(v);
     load8(in.b + o + c, v);
     sb += sumsq8(v);
   }
+  sa = wave_sum(sa);
+  sb = wave_sum(sb);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) { red[threadIdx.x >> 6] = sa; red[4 + (threadIdx.x >> 6)] = sb; }
+  __syncthreads();
   const float inv_n = 1.f / static_cast<float>(in.n);
-  const float ra = 0.5f * rsqrtf(block_sum(sa, red) * inv_n + in.eps);
-  const float rb = 0.5f * rsqrtf(block_sum(sb, red) * inv_n + in.eps);
+  const float ra = 0.5f * rsqrtf((red[0] + red[1] + red[2] + red[3]) * inv_n + in.eps);
+  const float rb = 0.5f * rsqrtf((red[4] + red[5] + red[6] + red[7]) * inv_n + in.eps);
   float ss = 0.f;
-  auto value = [&](int c, float (&v)[8]) {
-    float p[8], q[8];
-    load8(x + c, v);
-    load8(in.a + o + c, p);
-    load8(in.wa + c, q);
+  auto merged = [&](float (&v)[8], const float (&a)[8], const float (&p)[8], const float (&bb)[8], const float (&q)[8]) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] += p[i] * ra * q[i];
-    load8(in.b + o + c, p);
-    load8(in.wb + c, q);
+    for (int i = 0; i < 8; ++i) v[i] += a[i] * ra * p[i];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] += p[i] * rb * q[i];
+    for (int i = 0; i < 8; ++i) v[i] += bb[i] * rb * q[i];
   };
-  for (int c = threadIdx.x * 8; c < K; c += 2048) {
+  auto value = [&](int c, float (&v)[8]) {
+    float p[8], q[8], t[8], u[8];
+    load8(x + c, v);
+    load8(in.a + o + c, t);
+    load8(in.wa + c, p);
+    load8(in.b + o + c, u);
+    load8(in.wb + c, q);
+    merged(v, t, p, u, q);
+  };
+  kept_chunks(K, [&](int k, int c) {
+    merged(xk[k], ak[k], pk[k], bk[k], qk[k]);
+    ss += sumsq8(xk[k]);
+    if (lead) store8(in.x_out + o + c, xk[k]);
+  });
+  for (int c = (threadIdx.x + GV_KEEP * 256) * 8; c < K; c += 2048) {
     float v[8];
     value(c, v);
     ss += sumsq8(v);
     if (lead) store8(in.x_out + o + c, v);
   }
   const float r = rsqrtf(block_sum(ss, red) * inv_n + in.eps);
-  for (int c = threadIdx.x * 8; c < K; c += 2048) {
+  auto put = [&](int c, const float (&v)[8], float (&w)[8]) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) w[i] *= v[i] * r;
+    store8(xs + c, w);
+  };
+  kept_chunks(K, [&](int k, int c) { put(c, xk[k], wk[k]); });
+  for (int c = (threadIdx.x + GV_KEEP * 256) * 8; c < K; c += 2048) {
     float v[8], w[8];
     value(c, v);
     load8(in.w + c, w);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] *= r * w[i];
-    store8(xs + c, v);
+    put(c, v, w);
   }
 }
 
+// inv: a factor per part; sums (behind it): a sum of squares per chunk of eight.  Heads without padding whose parts are whole
+// chunks, up to GV_KEEP chunks a thread: every operand is requested once, at the start; otherwise the parts' sums come
+// first and the rows are read again.
 template <typename T>
 __device__ void prepare_group(const GemvInput& in, int b, int K, T* xs, float* inv) {
   const int slots = in.heads * in.vp, plen = in.heads * in.v / in.parts;
   const float* y = in.y + static_cast<long long>(b) * slots;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const bool gated = in.gate_mode == GATE_SIGMOID_AFTER;
   __syncthreads();                      // inv of the row before
   const bool dense = in.v == in.vp && (plen & 7) == 0;
+  if (dense && K <= GV_KEEP * 2048) {
+    float* sums = inv + in.parts;
+    float a[GV_KEEP][8], w[GV_KEEP][8], t[GV_KEEP][8];
+    kept_chunks(K, [&](int k, int c) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) a[k][i] = t[k][i] = w[k][i] = 0.f;
+      if (c >= slots) return;
+      load8(y + c, a[k]);
+      load8(in.w + c, w[k]);
+      if (gated) src8(in.gate, b, in.gcol + c, t[k]);
+    });
+    kept_chunks(K, [&](int k, int c) { sums[c >> 3] = sumsq8(a[k]); });
+    __syncthreads();
+    for (int p = wid; p < in.parts; p += 4) {
+      float s = 0.f;
+      for (int i = lane; i < plen >> 3; i += 64) s += sums[p * (plen >> 3) + i];
+      s = wave_sum(s);
+      if (lane == 0) inv[p] = rsqrtf(s / static_cast<float>(plen) + in.eps);
+    }
+    __syncthreads();
+    kept_chunks(K, [&](int k, int c) {
+      if (c < slots) {
+        const float f = inv[c / plen];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) a[k][i] *= f * w[k][i];
+        if (gated)
+#pragma unroll
+          for (int i = 0; i < 8; ++i) a[k][i] *= sigmoid_f(t[k][i]);
+      }
+      store8(xs + c, a[k]);
+    });
+    return;
+  }
   for (int p = wid; p < in.parts; p += 4) {
     float s = 0.f;
     if (dense) {
@@ -195,7 +256,7 @@ __device__ void prepare_group(const GemvInput& in, int b, int K, T* xs, float* i
       const int part0 = min(c0 / plen, in.parts - 1), next = (part0 + 1) * plen;
 #pragma unroll
       for (int i = 0; i < 8; ++i) a[i] *= inv[c0 + i < next ? part0 : min((c0 + i) / plen, in.parts - 1)] * w[i];
-      if (in.gate_mode == GATE_SIGMOID_AFTER) {
+      if (gated) {
         float t[8];
         src8(in.gate, b, in.gcol + c, t);
 #pragma unroll
@@ -228,12 +289,13 @@ __global__ __launch_bounds__(256) void row_gemv_kernel(GemvCall call, int blocks
   const int blk = second ? blockIdx.x - blocks0 : blockIdx.x;
   const int nblk = call.count == 2 ? (second ? gridDim.x - blocks0 : blocks0) : blocks0;
   const int K = p.K, nchunk = K / CE, nit = (nchunk + 255) / 256;
-  const int units = EPI == GV_GLU ? p.N / 4 : p.N / GV_R;
+  const int units = p.N / GV_R;
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const T* W = static_cast<const T*>(p.W);
   T* xs = reinterpret_cast<T*>(smem);
-  auto row_of = [&](int u, int r) {       // GLU: two gate rows, then the matching up rows
-    return EPI == GV_GLU ? (r < 2 ? u * 2 + r : p.N / 2 + u * 2 + r - 2) : u * GV_R + r;
+  constexpr int HR = GV_R / 2;
+  auto row_of = [&](int u, int r) {       // GLU: the unit's gate rows, then the matching up rows
+    return EPI == GV_GLU ? (r < HR ? u * HR + r : p.N / 2 + u * HR + r - HR) : u * GV_R + r;
   };
   u32x4_t cur[GV_NI][GV_R], nxt[GV_NI][GV_R];
   auto fetch = [&](u32x4_t (&w)[GV_NI][GV_R], int u, int it) {
@@ -302,10 +364,10 @@ __global__ __launch_bounds__(256) void row_gemv_kernel(GemvCall call, int blocks
     __syncthreads();
     auto total = [&](int i) { return part[flip][0][i] + part[flip][1][i] + part[flip][2][i] + part[flip][3][i]; };
     if constexpr (EPI == GV_GLU) {
-      if (tid < 2 * B) {
+      if (tid < HR * B) {
         const int r = tid / B, b = tid % B;
-        const float g = total(r * B + b), v = total((r + 2) * B + b);
-        static_cast<T*>(call.h)[static_cast<long long>(b) * (p.N / 2) + u * 2 + r] =
+        const float g = total(r * B + b), v = total((r + HR) * B + b);
+        static_cast<T*>(call.h)[static_cast<long long>(b) * (p.N / 2) + u * HR + r] =
             from_f32<T>((call.act == GLU_SILU ? g * sigmoid_f(g) : gelu_tanh_f(g)) * v);
       }
     } else {
@@ -332,19 +394,23 @@ size_t row_gemv_lds(const GemvCall& c, bool f32, int B) {
   for (int i = 0; i < c.count; ++i) {
     const GemvInput& in = c.p[i].in;
     if (in.kind == GV_PLAIN && c.count == 1) continue;
-    const size_t need = static_cast<size_t>(B) * c.p[i].K * (f32 ? 4 : 2) + (in.kind == GV_GROUP ? in.parts * 4 : 0);
+    const size_t need = static_cast<size_t>(B) * c.p[i].K * (f32 ? 4 : 2) +
+                        (in.kind == GV_GROUP ? in.parts * 4 + (c.p[i].K <= GV_KEEP * 2048 ? c.p[i].K / 2 : 0) : 0);
     most = need > most ? need : most;
   }
   return most;
 }
 template <typename T, int B>
 static void launch_b(const GemvCall& c, size_t lds, hipStream_t st) {
-  // two or three blocks per CU: enough waves to stream, few enough that the inputs are not prepared too often.  Width 4096,
-  // us at 256 / 512 / 768 / 1280 / 2048 blocks: one row, norm + 18560 rows 38.5 / 26.5 / 26.8 / 28.9 / 29.9, merge + gate/up
-  // 45.8 / 33.4 / 35.4 / 40.2 / 42.0, two output projections 19.8 / 18.3 / 15.9 / 18.0 / 21.3; four rows, norm + 18560 rows
-  // 58.9 / 38.8 / 34.6 / 41.6 / 47.4
+  // two or three blocks per CU: enough waves to stream, few enough that the inputs are not prepared too often.  us at 384 /
+  // 512 / 640 / 768 / 1024 blocks, one row: width 4096, norm + 18560 rows 28.3 / 25.8 / 27.5 / 26.5 / 28.9, merge + gate/up
+  // 32.3 / 30.5 / 32.9 / 31.4 / 34.7, two output projections 15.3 / 14.7 / 14.8 / 13.5 / 17.5; width 2048 (a thread has one
+  // chunk of a row, so half the loads of a batch are in flight), norm + 9280 rows 12.6 / 11.3 / 10.4 / 10.2 / 12.4, merge +
+  // gate/up 14.5 / 12.6 / 12.2 / 11.6 / 14.7, head 32.4 / 26.8 / 25.5 / 22.8 / 28.3.  Four rows, width 4096, norm + 18560
+  // rows at 256 / 512 / 768 / 1280: 58.9 / 38.8 / 34.6 / 41.6.  (Eight rows a unit: level at width 2048, 5 % behind at 4096.)
   const int kind = c.p[0].in.kind;
-  const int budget = g_blocks ? g_blocks : (B == 1 && c.count == 1 && (kind == GV_NORM || kind == GV_MERGE || kind == GV_POST) ? 512 : 768);
+  const bool one_chunk = c.p[0].K * sizeof(T) <= 256 * 16;
+  const int budget = g_blocks ? g_blocks : (B == 1 && c.count == 1 && !one_chunk && (kind == GV_NORM || kind == GV_MERGE || kind == GV_POST) ? 512 : 768);
   const int b0 = blocks_of(c.p[0], c.count == 2 ? budget / 2 : budget), b1 = c.count == 2 ? blocks_of(c.p[1], budget / 2) : 0;
   const dim3 grid(b0 + b1 + (c.latent.cache ? 1 : 0)), block(256);
   const bool plain = c.count == 1 && kind == GV_PLAIN;

@@ -432,6 +432,32 @@ def test_few_row_products(raw, dev, dtype, B, width, ff, heads, v, vp):
     assert N.rel_err(two[0, :, :width], (hr @ Dr.T)[:, :width]) < tol and N.rel_err(two[1, :, :width], (padded(full, kp) @ Gr.T)[:, :width]) < tol
 
 
+@pytest.mark.parametrize("B,width,ff,heads,v,vp", [(1, 4360, 320, 36, 128, 128), (2, 4104, 64, 17, 256, 256), (1, 2048, 64, 8, 504, 512)])
+def test_few_row_products_past_the_kept_chunks(raw, dev, B, width, ff, heads, v, vp):
+    """Rows of more columns than a thread keeps in registers (4 096), and a group norm at exactly that many."""
+    test_few_row_products(raw, dev, torch.bfloat16, B, width, ff, heads, v, vp)
+
+
+@pytest.mark.parametrize("H,G,Nn,V,B", [(2, 1, 320, 64, 1), (64, 4, 128, 64, 40), (1, 1, 32, 32, 3)])
+def test_ssd_step_of_four_taps_is_the_general_one(raw, dev, H, G, Nn, V, B):
+    """Four taps are read as vectors: the same numbers as five taps whose first weight is zero, over more state columns than
+    are requested ahead, blocks of sixteen and of more rows, from the first token on."""
+    C, inner = H * V + 2 * G * Nn, H * V
+    f = dict(dtype=torch.float32, device=dev)
+    rows = torch.randn(7, B, 2 * inner + 2 * G * Nn + H + (-H) % 8, generator=torch.Generator().manual_seed(H)).to(dev)
+    w4, bias, dt_bias, a_log, skip = (rnd(*s, seed=i).float().to(dev) for i, s in enumerate([(C, 4), (C,), (H,), (H,), (H,)]))
+    outs = []
+    for taps in (4, 5):
+        w = torch.cat([torch.zeros(C, taps - 4, **f), w4], 1).contiguous()
+        S, ring = torch.full((B, H, V, Nn), 9.0, **f), torch.full((B, taps, C), 9.0, dtype=torch.bfloat16, device=dev)
+        out = []
+        for t in range(7):
+            pos = torch.full((B,), t, dtype=torch.int32, device=dev)
+            out.append(raw.ssd_step_(rows[t], [0, inner, inner + C, H, G, Nn, V], w, bias, ring, dt_bias, a_log, skip, S, pos, None))
+        outs.append((torch.stack(out), S))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_matrix_memory_extreme_gates(raw, dev, dtype):
     """A key written with a huge input gate long ago, forget gates at the cap: the maximum runs far from zero."""
