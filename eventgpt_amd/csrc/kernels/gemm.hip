@@ -436,7 +436,7 @@ __device__ __forceinline__ void gemm_rope_epilogue(const GemmParams& p, f32x4_t 
 
 template <int BM, int BN, int WGM, int WGN, int STAGES, bool AT = false, bool BT = false, bool KT = false,
           bool ROPE = false, bool GRP = false>
-__global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmParams p) {
+__global__ __launch_bounds__(WGM * WGN * 64) void gemm_bf16_kernel(GemmParams p) {
   static_assert(!GRP || (!AT && !BT && !KT && !ROPE), "grouped products are plain ones");
   static_assert(!AT || BM == 64 || BM == 128, "K-strided A needs a 64- or 128-row tile");
   static_assert(!BT || BN == 64 || BN == 128, "K-strided W needs a 64- or 128-column tile");
@@ -444,7 +444,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmParams p) {
   constexpr int TM = WM / 16, TN = WN / 16;    // 16x16 tiles per wave
   constexpr int A_BYTES = BM * BK * 2, B_BYTES = BN * BK * 2;
   constexpr int STAGE = A_BYTES + B_BYTES;
-  static_assert(WGM * WGN == 4, "4 waves");
+  constexpr int NW = WGM * WGN;                // waves
+  static_assert((NW == 4 || NW == 8) && BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "waves stage whole groups of eight rows");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
@@ -487,10 +488,10 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmParams p) {
   // length, so edge tiles need no clamping.
   const int srow = lane >> 3, schunk = lane & 7;
   const int wid_u = __builtin_amdgcn_readfirstlane(wid);
-  int voff_a[BM / 32], voff_w[BN / 32];
+  int voff_a[BM / (8 * NW)], voff_w[BN / (8 * NW)];
 #pragma unroll
-  for (int i = 0; i < BM / 32; ++i) {
-    const int rg = wid_u * (BM / 32) + i;
+  for (int i = 0; i < BM / (8 * NW); ++i) {
+    const int rg = wid_u * (BM / (8 * NW)) + i;
     if constexpr (AT) {
       constexpr int CPR = BM / 8;
       const int lin = rg * 64 + lane;                 // 16-byte chunk index in the image
@@ -508,8 +509,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmParams p) {
     }
   }
 #pragma unroll
-  for (int i = 0; i < BN / 32; ++i) {
-    const int rg = wid_u * (BN / 32) + i;
+  for (int i = 0; i < BN / (8 * NW); ++i) {
+    const int rg = wid_u * (BN / (8 * NW)) + i;
     if constexpr (BT) {
       constexpr int CPR = BN / 8;
       const int lin = rg * 64 + lane;
@@ -540,8 +541,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmParams p) {
       // branch): chunks at or past k_cols get an offset outside the descriptor's range
       constexpr int kOut = 0x7ffffff0;
 #pragma unroll
-      for (int i = 0; i < BM / 32; ++i) {
-        const int rg = wid_u * (BM / 32) + i;
+      for (int i = 0; i < BM / (8 * NW); ++i) {
+        const int rg = wid_u * (BM / (8 * NW)) + i;
         int vo = voff_a[i];
         if constexpr (!AT) {
           const int row = rg * 8 + srow;
@@ -550,8 +551,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmParams p) {
         buffer_to_lds16(src_a, lim_a, base + rg * 1024, vo);
       }
 #pragma unroll
-      for (int i = 0; i < BN / 32; ++i) {
-        const int rg = wid_u * (BN / 32) + i;
+      for (int i = 0; i < BN / (8 * NW); ++i) {
+        const int rg = wid_u * (BN / (8 * NW)) + i;
         int vo = voff_w[i];
         if constexpr (!BT) {
           const int row = rg * 8 + srow;
@@ -562,13 +563,13 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmParams p) {
       return;
     }
 #pragma unroll
-    for (int i = 0; i < BM / 32; ++i) {  // BM/8 row-groups over 4 waves
-      const int rg = wid_u * (BM / 32) + i;
+    for (int i = 0; i < BM / (8 * NW); ++i) {  // BM/8 row-groups over the waves
+      const int rg = wid_u * (BM / (8 * NW)) + i;
       buffer_to_lds16(src_a, lim_a, base + rg * 1024, voff_a[i]);
     }
 #pragma unroll
-    for (int i = 0; i < BN / 32; ++i) {
-      const int rg = wid_u * (BN / 32) + i;
+    for (int i = 0; i < BN / (8 * NW); ++i) {
+      const int rg = wid_u * (BN / (8 * NW)) + i;
       buffer_to_lds16(src_w, lim_w, base + A_BYTES + rg * 1024, voff_w[i]);
     }
   };
@@ -588,7 +589,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmParams p) {
   // younger tiles' loads outstanding, followed by a raw s_barrier (a
   // __syncthreads() would drain them all).  After the barrier every wave has
   // finished reading the buffer of tile kt-1, which is the one re-staged next.
-  constexpr int G = (BM + BN) / 32;  // direct-to-LDS instructions per wave per stage
+  constexpr int G = (BM + BN) / (8 * NW);  // direct-to-LDS instructions per wave per stage
 #pragma unroll
   for (int s = 0; s < STAGES - 1; ++s)
     if (s < nk) stage(s, s);
@@ -1117,8 +1118,8 @@ static void launch_cfg(const GemmParams& p, hipStream_t st) {
   GemmParams q = p;
   q.group_m = g_group_m;
   q.split_major = (g_split_major && p.splitk > 1 && p.M > 32) ? 1 : 0;
-  hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, WGM, WGN, STAGES, AT, BT, KT, ROPE>), dim3(tiles), dim3(256), smem,
-                     st, q);
+  hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, WGM, WGN, STAGES, AT, BT, KT, ROPE>), dim3(tiles), dim3(WGM * WGN * 64),
+                     smem, st, q);
 }
 
 // Tile choice: the largest tile that still puts >= ~1.5 blocks on each of the 256
@@ -1126,7 +1127,7 @@ static void launch_cfg(const GemmParams& p, hipStream_t st) {
 // 4096-wide matrix, verify batches) take smaller tiles with a deeper ring, since
 // a grid below one block per CU is bound by the latency of its own K loop.
 enum GemmCfg { CFG_128x128 = 0, CFG_64x128 = 1, CFG_64x64 = 2, CFG_32x64 = 3, CFG_32x128 = 4, CFG_256x256 = 5,
-               CFG_128x256 = 6 };
+               CFG_128x256 = 6, CFG_64x128_W8 = 7 };
 
 static int g_forced_cfg = -1;
 void gemm_force_config(int cfg) { g_forced_cfg = cfg; }
@@ -1152,6 +1153,25 @@ static bool use_256(int M, int N, int K = 0) {
   // once the tiles come near one round (836 x 12288 x 4096: 914 vs 833 TFLOP/s; K-strided W,
   // 836 x 11008 x 4096: 686 vs 582), behind for 64 tiles (836 x 4096: 338 vs 700)
   return g_use_256 && ((M >= 1024 && t >= 128) || (M >= 768 && t >= 160));
+}
+
+// Short contractions (the ViT's 1024-wide layers: 16 K-tiles) are bound by the round trip of each K-tile, which waves of
+// other workgroups have to cover: eight waves on the 64 x 128 tile with two stages (48 KB: three workgroups, 24 waves a
+// CU), or with three where the tiles are fewer than three for every two CUs.  us against the best of the other tiles, weights
+// in the die-level cache: 1154 x 4096 x 1024 22.5 vs 32.8, 1154 x 3072 16.1 vs 16.7, 2885 x 4096 45.1 vs 54.2 (8-wave
+// 256 x 256, 192 tiles), 2885 x 3072 34.4 vs 37.5; 577 x 4096 from memory 18.7 vs 20.5 (two stages 22.2).  Whole vision path,
+// ms at 1 / 2 / 3 / 4 / 5 frames: 2.11 / 3.24 / 3.82 / 4.80 / 4.95 -> 2.04 / 2.90 / 3.61 / 4.29 / 4.71.  Behind where the
+// tiles leave CUs idle (577 x 3072, 240 tiles: 13.6 vs 11.9), over longer contractions (636 x 12288 x 4096: 116 vs 74; 600 x
+// 9280 x 2048 39 vs 36), for 1024 columns (2885 rows 15.5 vs 14.2) and towards a whole round of 256 x 256 tiles (with the
+// 3462 and 4039 rows of six and seven frames into 3072 columns, 168 and 192 of them: 5.40 -> 5.47 and 5.86 -> 6.02 ms).
+static bool use_64x128_w8(int M, int N, int K) {
+  const long long t = static_cast<long long>((M + 63) / 64) * ((N + 127) / 128);
+  return K > 0 && K <= 1024 && N >= 2048 && t >= 300 &&
+         static_cast<long long>((M + 255) / 256) * ((N + 255) / 256) < (N >= 4096 ? 200 : 160);
+}
+static void launch_64x128_w8(const GemmParams& p, hipStream_t st) {
+  if (static_cast<long long>((p.M + 63) / 64) * ((p.N + 127) / 128) < 400) launch_cfg<64, 128, 2, 4, 3>(p, st);
+  else launch_cfg<64, 128, 2, 4, 2>(p, st);
 }
 
 static int g_forced_splitk = 0;
@@ -1183,6 +1203,7 @@ static GemmCfg pick_cfg(int M, int N, int K = 0, int k_real = 0) {
   };
   // thresholds from benchmarks/bench_gemm.py on MI355X
   if (M <= 32) return tiles(32, 128) >= 256 ? CFG_32x128 : CFG_32x64;
+  if (use_64x128_w8(M, N, k_real)) return CFG_64x128_W8;
   if (use_256(M, N, k_real)) return CFG_256x256;
   if (K && narrow_256_splits(M, N, K) >= 2) return CFG_256x256;
   // Narrow outputs over a long contraction (a few hundred rows into 4096 columns over 11008, the
@@ -1193,17 +1214,22 @@ static GemmCfg pick_cfg(int M, int N, int K = 0, int k_real = 0) {
     // (a caller that consumes the fp32 slabs itself -- g_for_slabs -- pays no reduction pass, and the same
     // choice wins from K = 4096 on: 636 x 4096 x 4096 as 160 tiles x 3 splits 28 us, 64 x 128 unsplit 36.7;
     // with the reduction pass it loses there, 519 vs 571 TFLOP/s)
-    if (K >= (g_for_slabs ? 4096 : 8192) && tiles(128, 128) >= 96 && tiles(128, 128) < 256) return CFG_128x128;
+    // (256 tiles are one a CU: 900 x 4096 x 4096 in two splits 38.7 us, unsplit 58.0)
+    if (K >= (g_for_slabs ? 4096 : 8192) && tiles(128, 128) >= 96 && tiles(128, 128) < (g_for_slabs ? 257 : 256)) return CFG_128x128;
     if (K >= 4096 && tiles(64, 128) >= 48 && tiles(64, 128) < 128) return CFG_64x128;
   }
-  if (tiles(128, 128) >= 384) return CFG_128x128;
+  // (more rows, slabs summed by the caller: 1154 x 1024 x 4096 in three splits 19.4 us, 2885 rows in two 33.2; unsplit
+  // 64 x 128 tiles 26.4 and 38.4)
+  if (g_for_slabs && g_forced_splitk == 0 && M > 1024 && K >= 4096 && tiles(128, 128) >= 64 && tiles(128, 128) < 256) return CFG_128x128;
+  // 600 x 9280 x 2048, 365 tiles: 35.6 us, 64 x 128 tiles 42.5; 300 x 12288 x 4096, 288 tiles: 63.5 vs 53.8
+  if (tiles(128, 128) >= 336) return CFG_128x128;
   if (tiles(64, 128) >= 300) return CFG_64x128;
   if (tiles(64, 64) >= 300) return CFG_64x64;
   return CFG_32x64;
 }
 
 static long long cfg_tiles(GemmCfg c, int M, int N) {
-  static const int bm[] = {128, 64, 64, 32, 32, 256, 128}, bn[] = {128, 128, 64, 64, 128, 256, 256};
+  static const int bm[] = {128, 64, 64, 32, 32, 256, 128, 64}, bn[] = {128, 128, 64, 64, 128, 256, 256, 128};
   return static_cast<long long>((M + bm[c] - 1) / bm[c]) * ((N + bn[c] - 1) / bn[c]);
 }
 
@@ -1231,6 +1257,10 @@ int gemm_splitk(int M, int N, int K) {
           }
         }
       }
+      if (g_for_slabs && K >= 4096 && !use_256(M, N, K) && pick_cfg(M, N, K) == CFG_128x128) {
+        const long long tl = cfg_tiles(CFG_128x128, M, N);
+        return tl < 256 ? static_cast<int>(tl <= 128 ? 3 : 2) : 1;
+      }
       return 1;
     }
     if (!use_256(M, N, K) && narrow_256_splits(M, N, K) >= 2) return narrow_256_splits(M, N, K);
@@ -1245,7 +1275,7 @@ int gemm_splitk(int M, int N, int K) {
       s = static_cast<int>(want < most ? want : most);
       return s < 1 ? 1 : (s > 16 ? 16 : s);
     }
-    if (cfg == CFG_128x128 && K >= (g_for_slabs ? 4096 : 8192) && tl >= 96 && tl < 256) s = static_cast<int>(512 / tl);
+    if (cfg == CFG_128x128 && K >= (g_for_slabs ? 4096 : 8192) && tl >= 96 && tl < (g_for_slabs ? 257 : 256)) s = static_cast<int>(512 / tl);
     else if (cfg == CFG_64x128 && K >= 4096 && tl >= 48 && tl < 128) s = static_cast<int>(256 / tl);
     return s < 1 ? 1 : (s > 4 ? 4 : s);
   }
@@ -1374,6 +1404,7 @@ void launch_gemm_bf16(const bf16_t* A, const bf16_t* W, bf16_t* C, float* Cf, co
   switch (cfg) {
     case CFG_128x128: launch_cfg<128, 128, 2, 2, 2>(p, st); break;
     case CFG_64x128: launch_cfg<64, 128, 2, 2, 3>(p, st); break;
+    case CFG_64x128_W8: launch_64x128_w8(p, st); break;
     case CFG_64x64: launch_cfg<64, 64, 2, 2, 4>(p, st); break;
     case CFG_32x64: launch_cfg<32, 64, 1, 4, 4>(p, st); break;
     case CFG_256x256: launch_256<false, false>(p, st); break;
@@ -1577,6 +1608,7 @@ int launch_gemm_partial(const bf16_t* A, const bf16_t* W, float* partial, int M,
   switch (cfg) {
     case CFG_128x128: launch_cfg<128, 128, 2, 2, 2>(p, st); break;
     case CFG_64x128: launch_cfg<64, 128, 2, 2, 3>(p, st); break;
+    case CFG_64x128_W8: launch_64x128_w8(p, st); break;
     case CFG_64x64: launch_cfg<64, 64, 2, 2, 4>(p, st); break;
     case CFG_32x64: launch_cfg<32, 64, 1, 4, 4>(p, st); break;
     case CFG_256x256: launch_256<false, false>(p, st); break;

@@ -264,3 +264,37 @@ def test_persistent_256_with_k_split_glu_and_kstrided_operands(dev, force256):
     gy, w2, x2 = _rand(5000, 4608, dev=dev, scale=0.5), _rand(4608, 4352, dev=dev, seed=1, scale=0.05), _rand(5000, 4352, dev=dev, seed=2)
     _check(diff.linear_dgrad(gy, w2), gy.float() @ w2.float(), 4608)
     _check(diff.linear_wgrad(gy, x2), gy.float().t() @ x2.float(), 5000)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (65, 136, 128), (577, 4096, 1024), (700, 2056, 320), (64, 128, 1024)])
+def test_eight_waves_on_the_64_row_tile(dev, M, N, K):
+    """The 64 x 128 tile of eight waves, forced: row and column remainders, one K-tile and a contraction that is no multiple
+    of the two stages, bias, activation and residual, argmax partials; and as the rule takes it.  Repeats are equal."""
+    from eventgpt_amd.ops import hip
+    x, w = _rand(M, K, dev=dev), _rand(N, K, dev=dev, seed=1, scale=0.05)
+    bias, res = _rand(N, dev=dev, seed=2), _rand(M, N, dev=dev, seed=3)
+    lin = x.float() @ w.float().t() + bias.float()
+    want = torch.nn.functional.gelu(lin).to(torch.bfloat16).float() + res.float()
+    try:
+        hip.raw.gemm_force_config(7)
+        y = hip.raw.linear(x, w, bias, res, 1, False)
+        _check(y, want, K)
+        for _ in range(3):
+            assert torch.equal(hip.raw.linear(x, w, bias, res, 1, False), y)
+        _check(hip.raw.linear(x, w, bias, None, 0, True), lin, K)
+        pv, pi = hip.raw.linear_argmax_partials(x, w, bias)
+        got = pi.gather(1, pv.argmax(1, keepdim=True))[:, 0].long()
+        assert torch.equal(lin.gather(1, got[:, None]).to(torch.bfloat16), lin.max(1, keepdim=True).values.to(torch.bfloat16))
+    finally:
+        hip.raw.gemm_force_config(-1)
+    _check(hip.raw.linear(x, w, bias, res, 1, False), want, K)
+
+
+@pytest.mark.parametrize("M,N,K,slabs", [(1154, 1024, 4096, 3), (2885, 1024, 4096, 2), (900, 4096, 4096, 2), (1025, 1024, 4160, 3)])
+def test_slabs_of_about_a_round_of_tiles(dev, M, N, K, slabs):
+    """Products whose caller sums the slabs, split where 128 x 128 tiles are at most one a CU: the slabs add up."""
+    from eventgpt_amd.ops import hip
+    x, w = _rand(M, K, dev=dev), _rand(N, K, dev=dev, seed=1, scale=0.05)
+    part = hip.raw.linear_partial(x, w)
+    assert part.shape == (slabs, M, N)
+    _check(part.sum(0), x.float() @ w.float().t(), K)
