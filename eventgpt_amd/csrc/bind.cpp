@@ -1272,14 +1272,10 @@ std::tuple<Tensor, Tensor> event_voxel_sorted(const Tensor& x, const Tensor& y, 
   return {hist, vox};
 }
 
-// img uint8 [T,H,W,3] -> bf16 [T,3,S,S]; tables are int32 GPU tensors
-Tensor clip_preprocess(const Tensor& img, const Tensor& hstart, const Tensor& hcount,
-                       const Tensor& hweight, const Tensor& vstart, const Tensor& vcount,
-                       const Tensor& vweight, int64_t S, int64_t resize_h, int64_t resize_w,
-                       int64_t top, int64_t left, std::vector<double> mean,
-                       std::vector<double> stdv) {
-  TORCH_CHECK(img.is_cuda() && img.scalar_type() == at::kByte && img.is_contiguous() &&
-              img.dim() == 4 && img.size(3) == 3, "clip_preprocess: uint8 [T,H,W,3] expected");
+// img uint8 [T,H,W,3] -> bf16 [T,3,S,S]; tables are int32 GPU tensors.  codes: img is [T,H,W], one code a pixel
+static Tensor clip_pixels(const Tensor& img, bool codes, const Tensor& hstart, const Tensor& hcount, const Tensor& hweight,
+                          const Tensor& vstart, const Tensor& vcount, const Tensor& vweight, int64_t S, int64_t resize_h,
+                          int64_t resize_w, int64_t top, int64_t left, const std::vector<double>& mean, const std::vector<double>& stdv) {
   for (const Tensor* tb : {&hstart, &hcount, &hweight, &vstart, &vcount, &vweight}) check_i32(*tb, "table");
   const int64_t T = img.size(0), H = img.size(1), W = img.size(2);
   TORCH_CHECK(mean.size() == 3 && stdv.size() == 3);
@@ -1289,17 +1285,100 @@ Tensor clip_preprocess(const Tensor& img, const Tensor& hstart, const Tensor& hc
                           hweight.dim() == 2 && hweight.size(0) == resize_w));
   TORCH_CHECK(!need_v || (vstart.numel() == resize_h && vcount.numel() == resize_h &&
                           vweight.dim() == 2 && vweight.size(0) == resize_h));
+  const int ksh = need_h ? (int)hweight.size(1) : 1, ksv = need_v ? (int)vweight.size(1) : 1;
+  TORCH_CHECK(!codes || evgpt::clip_preproc_tiles_ok((int)T, (int)H, (int)resize_h, ksv), "clip: codes resized by too much");
   Tensor out = at::empty({T, 3, S, S}, img.options().dtype(at::kBFloat16));
   float m[3] = {(float)mean[0], (float)mean[1], (float)mean[2]};
   float sd[3] = {(float)stdv[0], (float)stdv[1], (float)stdv[2]};
-  evgpt::launch_clip_preproc(img.data_ptr<uint8_t>(), bptr_mut(out), hstart.data_ptr<int>(),
-                             hcount.data_ptr<int>(), hweight.data_ptr<int>(),
-                             vstart.data_ptr<int>(), vcount.data_ptr<int>(),
-                             vweight.data_ptr<int>(), (int)T, (int)H, (int)W, (int)S,
-                             (int)resize_h, (int)resize_w, (int)top, (int)left,
-                             need_h ? (int)hweight.size(1) : 1, need_v ? (int)vweight.size(1) : 1,
-                             m, sd, cur_stream());
+  if (T > 0 && S > 0)
+    evgpt::launch_clip_preproc(img.data_ptr<uint8_t>(), bptr_mut(out), hstart.data_ptr<int>(), hcount.data_ptr<int>(),
+                               hweight.data_ptr<int>(), vstart.data_ptr<int>(), vcount.data_ptr<int>(), vweight.data_ptr<int>(),
+                               (int)T, (int)H, (int)W, (int)S, (int)resize_h, (int)resize_w, (int)top, (int)left, ksh, ksv, m, sd,
+                               codes, cur_stream());
   return out;
+}
+Tensor clip_preprocess(const Tensor& img, const Tensor& hstart, const Tensor& hcount,
+                       const Tensor& hweight, const Tensor& vstart, const Tensor& vcount,
+                       const Tensor& vweight, int64_t S, int64_t resize_h, int64_t resize_w,
+                       int64_t top, int64_t left, std::vector<double> mean,
+                       std::vector<double> stdv) {
+  TORCH_CHECK(img.is_cuda() && img.scalar_type() == at::kByte && img.is_contiguous() &&
+              img.dim() == 4 && img.size(3) == 3, "clip_preprocess: uint8 [T,H,W,3] expected");
+  return clip_pixels(img, false, hstart, hcount, hweight, vstart, vcount, vweight, S, resize_h, resize_w, top, left, mean, stdv);
+}
+
+// A host event stream as one word an event (x | y << 15 | (p != 0) << 30) in pinned memory, and the image it needs: {words,
+// int64 [height, width]}.  An empty list where it does not fit: empty, other than integers, coordinates below zero or from 2^15 on.
+template <typename X, typename P>
+static bool pack_words(const X* x, const X* y, const P* p, int64_t n, int* out, int64_t* hw) {
+  int most_x = 0, most_y = 0;
+  unsigned int any = 0;
+  for (int64_t i = 0; i < n; ++i) {
+    const int xi = static_cast<int>(x[i]), yi = static_cast<int>(y[i]);
+    any |= static_cast<unsigned int>(xi) | static_cast<unsigned int>(yi);       // a sign or a high bit shows here
+    most_x = xi > most_x ? xi : most_x;
+    most_y = yi > most_y ? yi : most_y;
+    out[i] = xi | yi << 15 | (static_cast<int>(p[i]) != 0) << 30;
+  }
+  hw[0] = most_y + 1;
+  hw[1] = most_x + 1;
+  return any < 32768u;
+}
+std::vector<Tensor> pack_events(const Tensor& x, const Tensor& y, const Tensor& p) {
+  const int64_t n = x.numel();
+  for (const Tensor* t : {&x, &y, &p}) TORCH_CHECK(t->is_cpu() && t->is_contiguous(), "pack_events: contiguous host tensors");
+  TORCH_CHECK(y.numel() == n && p.numel() == n, "pack_events: x, y and p differ in length");
+  if (n == 0 || n >= (1ll << 30) || x.scalar_type() != y.scalar_type()) return {};
+  Tensor words = at::empty({n}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+  Tensor hw = at::empty({2}, at::TensorOptions().dtype(at::kLong));
+  bool ok = false;
+  const auto polarity = [&](auto xt) {
+    using X = decltype(xt);
+    const X *px = static_cast<const X*>(x.data_ptr()), *py = static_cast<const X*>(y.data_ptr());
+    int* out = words.data_ptr<int>();
+    int64_t* size = hw.data_ptr<int64_t>();
+    switch (p.scalar_type()) {
+      case at::kByte: case at::kBool: ok = pack_words(px, py, static_cast<const uint8_t*>(p.data_ptr()), n, out, size); break;
+      case at::kChar: ok = pack_words(px, py, static_cast<const int8_t*>(p.data_ptr()), n, out, size); break;
+      case at::kShort: ok = pack_words(px, py, static_cast<const int16_t*>(p.data_ptr()), n, out, size); break;
+      case at::kInt: ok = pack_words(px, py, static_cast<const int32_t*>(p.data_ptr()), n, out, size); break;
+      case at::kLong: ok = pack_words(px, py, static_cast<const int64_t*>(p.data_ptr()), n, out, size); break;
+      default: break;
+    }
+  };
+  switch (x.scalar_type()) {
+    case at::kByte: polarity(uint8_t{}); break;
+    case at::kShort: polarity(int16_t{}); break;
+    case at::kUInt16: polarity(uint16_t{}); break;
+    case at::kInt: polarity(int32_t{}); break;
+    case at::kLong:                      // (values past 32 bits would be cut: leave them to the general path)
+      if (x.max().item<int64_t>() < 32768 && y.max().item<int64_t>() < 32768 && x.min().item<int64_t>() >= 0 && y.min().item<int64_t>() >= 0)
+        polarity(int64_t{});
+      break;
+    default: break;
+  }
+  if (!ok) return {};
+  return {words, hw};
+}
+
+// whether event_clip_frames takes the stream's image
+bool event_codes_ok(int64_t n, int64_t n_slices, int64_t H, int64_t W, int64_t resize_h, int64_t ksv) {
+  return n_slices >= 1 && n_slices <= 65535 && evgpt::event_codes_ok(n, (int)n_slices, (int)H, (int)W) &&
+         evgpt::clip_preproc_tiles_ok((int)n_slices, (int)H, (int)resize_h, (int)ksv);
+}
+
+// packed words -> rasters of n_slices equal-count slices -> CLIP pixels bf16 [n_slices, 3, S, S]; mode as event_raster
+Tensor event_clip_frames(const Tensor& words, int64_t n_slices, int64_t H, int64_t W, int64_t mode, const Tensor& hstart,
+                         const Tensor& hcount, const Tensor& hweight, const Tensor& vstart, const Tensor& vcount, const Tensor& vweight,
+                         int64_t S, int64_t resize_h, int64_t resize_w, int64_t top, int64_t left, std::vector<double> mean,
+                         std::vector<double> stdv) {
+  check_i32(words, "words");
+  const int64_t n = words.numel();
+  TORCH_CHECK(n < (1ll << 30) && event_codes_ok(n, n_slices, H, W, resize_h, resize_h != H ? vweight.size(-1) : 1), "event_clip_frames: image");
+  Tensor codes = at::empty({n_slices, H, W}, words.options().dtype(at::kByte));
+  evgpt::launch_event_codes(reinterpret_cast<const unsigned int*>(words.data_ptr<int>()), (int)n, (int)n_slices, (int)H, (int)W,
+                            codes.data_ptr<uint8_t>(), (int)mode, cur_stream());
+  return clip_pixels(codes, true, hstart, hcount, hweight, vstart, vcount, vweight, S, resize_h, resize_w, top, left, mean, stdv);
 }
 
 // pixels [T,C,S,S] -> patch rows [T*G*G, Kp] (zero padded to a multiple of 64)
@@ -1502,6 +1581,9 @@ TORCH_LIBRARY(evgpt, m) {
   m.def("event_voxel_sorted_ok(int bins, int H, int W) -> bool", &event_voxel_sorted_ok);
   m.def("event_voxel_sorted(Tensor x, Tensor y, Tensor p, Tensor t, int bins, int H, int W, bool signed_mode, bool by_count) -> (Tensor, Tensor)", &event_voxel_sorted);
   m.def("clip_preprocess(Tensor img, Tensor hstart, Tensor hcount, Tensor hweight, Tensor vstart, Tensor vcount, Tensor vweight, int S, int resize_h, int resize_w, int top, int left, float[] mean, float[] stdv) -> Tensor", &clip_preprocess);
+  m.def("pack_events(Tensor x, Tensor y, Tensor p) -> Tensor[]", &pack_events);
+  m.def("event_codes_ok(int n, int n_slices, int H, int W, int resize_h, int ksv) -> bool", &event_codes_ok);
+  m.def("event_clip_frames(Tensor words, int n_slices, int H, int W, int mode, Tensor hstart, Tensor hcount, Tensor hweight, Tensor vstart, Tensor vcount, Tensor vweight, int S, int resize_h, int resize_w, int top, int left, float[] mean, float[] stdv) -> Tensor", &event_clip_frames);
   m.def("gemm_force_config(int cfg) -> ()", &gemm_force_config);
   m.def("gemm_enable_256(bool on) -> ()", &gemm_enable_256);
   m.def("gemm_persist_256(bool on) -> ()", &gemm_persist_256);

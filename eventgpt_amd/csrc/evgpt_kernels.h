@@ -138,11 +138,15 @@ void launch_event_voxel_ranges(const int* x, const int* y, const int* p, const i
 void launch_event_voxel(const int* x, const int* y, const int* p, const long long* t, int n_events,
                         long long t0, long long span, int bins, int H, int W, int* out_hist,
                         float* out_vox, int signed_mode, int by_count, hipStream_t st);
+// one code a pixel from a packed stream; what the preprocessing below takes for frames with `codes`
+bool event_codes_ok(long long n_events, int n_slices, int H, int W);
+void launch_event_codes(const unsigned int* ev, int n_events, int n_slices, int H, int W, unsigned char* codes, int mode, hipStream_t st);
+bool clip_preproc_tiles_ok(int T, int H, int resize_h, int ksv);
 void launch_clip_preproc(const unsigned char* img, bf16_t* out, const int* hstart,
                          const int* hcount, const int* hweight, const int* vstart,
                          const int* vcount, const int* vweight, int T, int H, int W, int S,
                          int resize_h, int resize_w, int top, int left, int ksh, int ksv,
-                         const float* mean, const float* stdv, hipStream_t st);
+                         const float* mean, const float* stdv, bool codes, hipStream_t st);
 
 // ---- adapter_ops.hip (device-resident speculative-decoding draft head)
 void launch_gather_rows_dev(const bf16_t* src, const int* index, int offset, const int* n_valid_dev,

@@ -60,6 +60,63 @@ void launch_event_raster(const int* x, const int* y, const int* p, int n_events,
   hipLaunchKernelGGL(raster_colorize_kernel, dim3(cb), dim3(256), 0, st, keys, img, n_pix, mode);
 }
 
+// Frames of a packed stream (x | y << 15 | positive << 30, one word an event) as one code a pixel: 0 untouched, 1 positive, 2
+// negative.  A block owns some rows of one slice in LDS and scans the slice's events, so nothing is filled beforehand, no
+// atomic leaves the CU and what the preprocessing reads is a third of an RGB frame.  Bound by the passes over LDS and the scan's
+// round trips.  Five slices: 20 000 events on 160 x 120 4.4 us, 12.3 as a fill, a scatter of global atomics and a colour pass;
+// 200 000 on 640 x 480 12.8 and 24.9; 2 500 000 there 101 and 108: from there on the atomics are as good.
+__global__ __launch_bounds__(1024) void event_codes_kernel(const unsigned int* __restrict__ ev, int n_events, int n_slices, int H, int W,
+                                                           int rows, unsigned char* __restrict__ codes, int mode) {
+  extern __shared__ int cell[];        // [rows][W]: last (index << 1 | positive) or the mask of polarities seen
+  const int s = blockIdx.y, y0 = blockIdx.x * rows, band = min(rows, H - y0), cells = band * W;
+  for (int i = threadIdx.x; i < cells; i += 1024) cell[i] = mode == 0 ? -1 : 0;
+  __syncthreads();
+  const int per = n_events / n_slices;
+  const int lo = s * per, hi = s + 1 < n_slices ? lo + per : n_events;      // the last slice takes the remainder
+  for (int i0 = lo + threadIdx.x; i0 < hi; i0 += 4096) {
+    unsigned int e[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) e[u] = ev[min(i0 + u * 1024, hi - 1)];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = i0 + u * 1024, x = e[u] & 0x7fff, r = static_cast<int>(e[u] >> 15 & 0x7fff) - y0, pol = e[u] >> 30;
+      if (i >= hi || r < 0 || r >= band || x >= W) continue;
+      if (mode == 0) atomicMax(&cell[r * W + x], (i - lo) << 1 | pol);
+      else atomicOr(&cell[r * W + x], pol ? 1 : 2);
+    }
+  }
+  __syncthreads();
+  unsigned char* out = codes + (static_cast<size_t>(s) * H + y0) * W;
+  for (int i = threadIdx.x; i < cells; i += 1024) {
+    const int k = cell[i];
+    out[i] = mode == 0 ? (k < 0 ? 0 : (k & 1 ? 1 : 2)) : (k & 2 ? 2 : (k & 1));
+  }
+}
+
+// image rows of a block: about 160 blocks, at most 144 KB of cells (0: the image is too wide)
+static int event_codes_rows(int n_slices, int H, int W) {
+  const int most = 144 * 1024 / 4 / W;
+  const int bands = (160 + n_slices - 1) / n_slices, rows = (H + bands - 1) / bands;
+  return rows < most ? rows : most;
+}
+// every block of a slice scans all its events: worth it up to the 500 000 events a slice measured above (fewer events
+// than slices are all of slice 0, which only the atomic kernel knows)
+bool event_codes_ok(long long n_events, int n_slices, int H, int W) {
+  if (n_slices < 1 || n_events < n_slices || n_slices > 65535 || H < 1 || W < 1 || H > 32768 || W > 32768) return false;
+  const int rows = event_codes_rows(n_slices, H, W);
+  return rows >= 1 && n_events / n_slices <= 500000 && (H + rows - 1) / rows * n_slices <= 1024;
+}
+void launch_event_codes(const unsigned int* ev, int n_events, int n_slices, int H, int W, unsigned char* codes, int mode, hipStream_t st) {
+  const int rows = event_codes_rows(n_slices, H, W);
+  static bool attr_set = false;
+  if (!attr_set) {
+    hipFuncSetAttribute(reinterpret_cast<const void*>(&event_codes_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 144 * 1024);
+    attr_set = true;
+  }
+  hipLaunchKernelGGL(event_codes_kernel, dim3((H + rows - 1) / rows, n_slices), dim3(1024), static_cast<size_t>(rows) * W * 4, st, ev,
+                     n_events, n_slices, H, W, rows, codes, mode);
+}
+
 // ------------------------------------------------------------ voxel / histogram
 // Time-binned accumulation.  t is int64 microseconds; bin = floor((t - t0) * bins / span)
 // clamped to bins-1.  out_hist: [bins][2][H][W] int32 counts (may be null);
@@ -524,17 +581,110 @@ __global__ __launch_bounds__(256) void clip_preproc_kernel(PreprocParams p) {
   }
 }
 
+// The same pixels in two passes over a tile of CP_ROWS x CP_COLS outputs: the source rows it needs are resized horizontally
+// into LDS (one word a pixel), then vertically.  A pixel costs its horizontal taps once instead of once per vertical tap, and
+// the sums fit 32 bits: weights of 22 fractional bits sum to one with magnitudes below 1.5, times 255.  Bound by that integer
+// work: five frames of 160 x 120 to 336 x 336 9.9 us, 17.7 one pixel at a time in 64 bits; of
+// 640 x 480 20.0 and 39.3.  Tiles of four rows where eight would leave CUs idle: one frame of 640 x 480 9.7, with eight 13.4, by
+// pixels 11.1.
+// CODES: the source is one code a pixel (event_codes_kernel) instead of three bytes.
+constexpr int CP_COLS = 112, CP_SRC = 48;
+
+__device__ __forceinline__ int clip8_fix32(int acc) { return min(max(acc >> 22, 0), 255); }
+
+template <bool CODES, int CP_ROWS>
+__global__ __launch_bounds__(256) void clip_preproc_tile_kernel(PreprocParams p) {
+  __shared__ unsigned int mid[CP_SRC][CP_COLS];
+  const int ox0 = blockIdx.x * CP_COLS, oy0 = blockIdx.y * CP_ROWS, t = blockIdx.z;
+  const int cols = min(CP_COLS, p.S - ox0), rows = min(CP_ROWS, p.S - oy0);
+  const bool need_h = p.resize_w != p.W, need_v = p.resize_h != p.H;
+  const int first = oy0 + p.top, last = first + rows - 1;      // rows of the resized image
+  const int r0 = need_v ? p.vstart[first] : first;
+  const int n_src = min((need_v ? p.vstart[last] + p.vcount[last] : last + 1) - r0, CP_SRC);
+  const unsigned char* frame = p.img + static_cast<size_t>(t) * p.H * p.W * (CODES ? 1 : 3);
+  constexpr int half = 1 << 21;
+  for (int i = threadIdx.x; i < n_src * CP_COLS; i += 256) {
+    const int r = i / CP_COLS, c = i % CP_COLS;
+    if (c >= cols) continue;
+    const int rx = ox0 + c + p.left, hs = need_h ? p.hstart[rx] : rx, hc = need_h ? p.hcount[rx] : 1;
+    const unsigned char* src = frame + (static_cast<size_t>(r0 + r) * p.W + hs) * (CODES ? 1 : 3);
+    int v[3] = {half, half, half};
+    const int* w = p.hweight + rx * p.ksh;
+    for (int k = 0; k < hc; ++k) {
+      int px[3];
+      if constexpr (CODES) {
+        const int code = src[k];                   // white, red or blue
+        px[0] = code == 2 ? 0 : 255; px[1] = code ? 0 : 255; px[2] = code == 1 ? 0 : 255;
+      } else {
+        px[0] = src[k * 3]; px[1] = src[k * 3 + 1]; px[2] = src[k * 3 + 2];
+      }
+      const int wk = need_h ? w[k] : 0;
+#pragma unroll
+      for (int ch = 0; ch < 3; ++ch) v[ch] = need_h ? v[ch] + wk * px[ch] : px[ch];
+    }
+#pragma unroll
+    for (int ch = 0; ch < 3; ++ch) v[ch] = need_h ? clip8_fix32(v[ch]) : v[ch];
+    mid[r][c] = v[0] | v[1] << 8 | v[2] << 16;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < rows * CP_COLS; i += 256) {
+    const int r = i / CP_COLS, c = i % CP_COLS;
+    if (c >= cols) continue;
+    const int ry = first + r, vs = (need_v ? p.vstart[ry] : ry) - r0;
+    int px[3];
+    if (need_v) {
+      const int vc = p.vcount[ry];
+      const int* w = p.vweight + ry * p.ksv;
+      int v[3] = {half, half, half};
+      for (int k = 0; k < vc; ++k) {
+        const unsigned int m = mid[vs + k][c];
+        const int wk = w[k];
+        v[0] += wk * static_cast<int>(m & 255); v[1] += wk * static_cast<int>(m >> 8 & 255); v[2] += wk * static_cast<int>(m >> 16);
+      }
+#pragma unroll
+      for (int ch = 0; ch < 3; ++ch) px[ch] = clip8_fix32(v[ch]);
+    } else {
+      const unsigned int m = mid[vs][c];
+      px[0] = m & 255; px[1] = m >> 8 & 255; px[2] = m >> 16;
+    }
+#pragma unroll
+    for (int ch = 0; ch < 3; ++ch) {
+      const float v = (static_cast<float>(px[ch]) * (1.f / 255.f) - p.mean[ch]) * p.inv_std[ch];
+      p.out[((static_cast<size_t>(t) * 3 + ch) * p.S + oy0 + r) * p.S + ox0 + c] = f32_to_bf16(v);
+    }
+  }
+}
+
+// source rows of a tile fit its LDS (a resize by less than about four)
+bool clip_preproc_tiles_ok(int T, int H, int resize_h, int ksv) {
+  const long long src = (7ll * H + resize_h - 1) / resize_h + ksv + 1;
+  return src <= CP_SRC && T <= 65535;
+}
+
 void launch_clip_preproc(const unsigned char* img, bf16_t* out, const int* hstart,
                          const int* hcount, const int* hweight, const int* vstart,
                          const int* vcount, const int* vweight, int T, int H, int W, int S,
                          int resize_h, int resize_w, int top, int left, int ksh, int ksv,
-                         const float* mean, const float* stdv, hipStream_t st) {
+                         const float* mean, const float* stdv, bool codes, hipStream_t st) {
   PreprocParams p;
   p.img = img; p.out = out; p.hstart = hstart; p.hcount = hcount; p.hweight = hweight;
   p.vstart = vstart; p.vcount = vcount; p.vweight = vweight;
   p.T = T; p.H = H; p.W = W; p.S = S; p.top = top; p.left = left; p.ksh = ksh; p.ksv = ksv;
   p.resize_h = resize_h; p.resize_w = resize_w;
   for (int c = 0; c < 3; ++c) { p.mean[c] = mean[c]; p.inv_std[c] = 1.f / stdv[c]; }
+  if (clip_preproc_tiles_ok(T, H, resize_h, ksv)) {
+    const int cols = (S + CP_COLS - 1) / CP_COLS;
+    if (cols * ((S + 7) / 8) * T >= 256) {
+      const dim3 grid(cols, (S + 7) / 8, T);
+      if (codes) hipLaunchKernelGGL((clip_preproc_tile_kernel<true, 8>), grid, dim3(256), 0, st, p);
+      else hipLaunchKernelGGL((clip_preproc_tile_kernel<false, 8>), grid, dim3(256), 0, st, p);
+    } else {
+      const dim3 grid(cols, (S + 3) / 4, T);
+      if (codes) hipLaunchKernelGGL((clip_preproc_tile_kernel<true, 4>), grid, dim3(256), 0, st, p);
+      else hipLaunchKernelGGL((clip_preproc_tile_kernel<false, 4>), grid, dim3(256), 0, st, p);
+    }
+    return;
+  }
   const long long total = static_cast<long long>(T) * S * S;
   int blocks = static_cast<int>((total + 255) / 256);
   if (blocks > 8192) blocks = 8192;

@@ -2,8 +2,9 @@
 
 Replaces the reference's host pipeline (python loop over every event to paint
 the raster, PIL resize, numpy normalise — common/common.py:17-37,64-74,110-129)
-with three launches on device-resident event arrays:
+with launches on device-resident event arrays:
 
+    event_clip_frames  one packed upload -> one code a pixel -> CLIP pixels: two launches for integer host streams
     event_raster    one atomic per event (last-wins / negative-wins), all T slices
     clip_preprocess PIL-exact two-pass bicubic + crop + normalise, all T frames
     (event_voxel    time-binned polarity histogram / signed voxel grid; LDS-privatised per band)
@@ -174,10 +175,42 @@ def preprocess_frames(frames, device, size: int = CLIP_IMAGE_SIZE, dtype=torch.b
     return torch.stack(px).to(device, dtype)
 
 
+def _packed(events: dict):
+    """``(pinned int32 words, (H, W))`` of a host event stream, or None where its values do not fit a word."""
+    from . import hip
+    cols = [np.asarray(events[k]) for k in ("x", "y", "p")]
+    t = np.asarray(events["t"])
+    if any(c.ndim != 1 or c.size != t.size or c.dtype.kind not in "iub" for c in cols) or t.ndim != 1 or t.dtype.kind not in "iuf":
+        return None
+    try:
+        out = hip.raw.pack_events(*(torch.from_numpy(np.require(c, requirements="CAW")) for c in cols))
+    except (TypeError, ValueError):   # a dtype or byte order torch does not have
+        return None
+    return (out[0], tuple(out[1].tolist())) if out else None
+
+
 def event_frames_gpu(events: dict, device, n_frames: int = 5, size: int = CLIP_IMAGE_SIZE,
                      conflict: str = "last") -> Tuple[list, torch.Tensor]:
-    """Host event dict -> ``([H, W], bf16 [T,3,size,size])`` entirely on the GPU."""
+    """Host event dict -> ``([H, W], bf16 [T,3,size,size])`` on the GPU.  Integer streams go up as one word an event from
+    pinned memory (polarity and coordinates; timestamps play no part in equal-count slices) and nothing waits for the
+    device; other streams, images and sizes, and a stream under capture, take the general ops."""
+    dev = torch.device(device)
+    packed = _packed(events) if dev.type == "cuda" and not torch.cuda.is_current_stream_capturing() else None
+    if packed is not None:
+        from . import hip
+        words, (h, w) = packed
+        rh, rw = cp.resized_shape(h, w, size)
+        ksv = cp.resample_table(h, rh).weight.shape[1] if rh != h else 1
+        if rh >= size and rw >= size and hip.raw.event_codes_ok(words.numel(), n_frames, h, w, rh, ksv):
+            words = words.to(dev, non_blocking=True)
+            return [h, w], hip.raw.event_clip_frames(words, n_frames, h, w, {"last": 0, "negative": 1}[conflict],
+                                                     *_with_crop(h, w, size, words.device))
     ev = events_to_device(events, device)
     hw = canvas_size(np.asarray(events["x"]), np.asarray(events["y"]))
     img = rasterize_gpu(ev, n_frames, hw, conflict)
     return list(hw), clip_preprocess_gpu(img, size)
+
+
+def _with_crop(h: int, w: int, size: int, device) -> tuple:
+    tables = _tables(h, w, size, device)
+    return (*tables[:6], size, *tables[6:], list(CLIP_MEAN), list(CLIP_STD))

@@ -140,3 +140,45 @@ def test_preprocess_frames_device_dispatch(dev):
     host = proc("USER: <video>\nwhat? ASSISTANT:", frames)
     assert out["pixel_values_videos"].shape == (1, 4, 3, S, S) and out["pixel_values_videos"].is_cuda
     assert torch.equal(out["pixel_values_videos"].float().cpu(), host["pixel_values_videos"].to(torch.bfloat16).float())
+
+
+def _host_stream(n, h, w, dtype, p_dtype, seed=3):
+    rng = np.random.default_rng(seed)
+    x, y = rng.integers(0, w, n), rng.integers(0, h, n)
+    x[0], y[0] = w - 1, h - 1
+    return {"x": x.astype(dtype), "y": y.astype(dtype), "p": rng.integers(0, 2, n).astype(p_dtype),
+            "t": np.sort(rng.integers(0, 50_000, n))}
+
+
+# bands with a short last one, rows that need no resize, a resize near the tiles' limit and one past it, one slice (short tiles),
+# slices with a remainder, as many events as slices and fewer; every integer type that is packed and some that are not
+@pytest.mark.parametrize("n,h,w,slices,dtype,p_dtype", [
+    (20_003, 120, 160, 5, np.int16, np.int8), (7_001, 481, 640, 3, np.uint16, np.uint8), (5_000, 336, 336, 5, np.int32, np.bool_),
+    (4_099, 97, 53, 7, np.int64, np.int64), (3_000, 1300, 1281, 2, np.int32, np.int32), (3_000, 1700, 1501, 2, np.int32, np.int32), (901, 60, 80, 1, np.int16, np.int8),
+    (5, 40, 40, 5, np.uint8, np.uint8),
+    (3, 40, 40, 5, np.int32, np.int16), (901, 60, 80, 1, np.float32, np.int8), (901, 60, 80, 4, ">i4", np.int8)])
+@pytest.mark.parametrize("conflict", ["last", "negative"])
+def test_packed_frames_equal_the_general_ops(dev, n, h, w, slices, dtype, p_dtype, conflict):
+    from eventgpt_amd.ops import event_ops as eo
+    ev = _host_stream(n, h, w, dtype, p_dtype)
+    size, px = eo.event_frames_gpu(ev, dev, slices, conflict=conflict)
+    img = eo.rasterize_gpu(eo.events_to_device(ev, dev), slices, (h, w), conflict)
+    want = np.stack([cp.preprocess_image(f) for f in img.cpu().numpy()])
+    assert size == [h, w] and torch.equal(px, eo.clip_preprocess_gpu(img))
+    # the same bytes, normalised in another order: rounding to 8 significant bits is off by half of 2^(e-7), at most 2^-8 of a
+    # value of 2^e or more; the float32 forms differ by a few 2^-24 of terms below 4
+    np.testing.assert_allclose(px.float().cpu().numpy(), want, rtol=2.0 ** -8, atol=1e-5)
+
+
+def test_streams_that_do_not_pack_stay_on_the_general_ops(dev):
+    from eventgpt_amd.ops import event_ops as eo
+    good = _host_stream(50, 40, 40, np.int64, np.int8)
+    assert eo._packed(good) is not None
+    for key, value in (("x", np.where(np.arange(50) == 9, 1 << 33, good["x"])), ("y", np.where(np.arange(50) == 9, -1, good["y"])),
+                       ("x", np.where(np.arange(50) == 9, 32768, good["x"])), ("p", good["p"][:-1]), ("p", good["p"].astype(np.float32))):
+        assert eo._packed({**good, key: value}) is None
+    assert eo._packed({k: v[:0] for k, v in good.items()}) is None
+    locked = {k: v.copy() for k, v in good.items()}
+    for v in locked.values():
+        v.flags.writeable = False
+    assert torch.equal(eo._packed(locked)[0], eo._packed(good)[0])
