@@ -530,4 +530,78 @@ void launch_layernorm_bwd(const bf16_t* x, const bf16_t* w, const bf16_t* g, bf1
   hipLaunchKernelGGL(layernorm_bwd_kernel, dim3(blocks), dim3(256), 0, st, x, w, g, dx, dw, db, rows, H, eps, rpb);
 }
 
+// ----------------------------------------------------------------------------- column sums (bias gradients)
+// out[c] = sum over rows of G[r][c] in float32, without atomics: a block sums a slab of rows for 512 columns (a lane owns eight,
+// four waves take every fourth row with CS_DEPTH rows in flight), the second launch adds the slabs.  Bound by reading G once.
+// 3 200 x 4 096: 14.2 us, 42.1 as a cast to float32 and a reduction of that; 40 000 x 512: 47.6 and 56.5, x 128: 39.7 and 36.6 (half
+// the lanes and more idle), so callers keep rows shorter than 512 off it.
+constexpr int CS_DEPTH = 4;
+
+__global__ __launch_bounds__(256) void column_sum_slab_kernel(const bf16_t* __restrict__ G, float* __restrict__ part, int M, int N,
+                                                              int rows_per_slab) {
+  __shared__ __attribute__((aligned(16))) float red[3][512];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, c = blockIdx.x * 512 + lane * 8;
+  const int row0 = blockIdx.y * rows_per_slab, row1 = min(M, row0 + rows_per_slab);
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (c < N)
+    for (int r = row0 + w; r < row1; r += 4 * CS_DEPTH) {
+      u32x4_t v[CS_DEPTH];
+#pragma unroll
+      for (int d = 0; d < CS_DEPTH; ++d)
+        v[d] = r + 4 * d < row1 ? *reinterpret_cast<const u32x4_t*>(G + static_cast<size_t>(r + 4 * d) * N + c) : u32x4_t{0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int d = 0; d < CS_DEPTH; ++d)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] += bf16_to_f32(static_cast<bf16_t>(v[d][e >> 1] >> (16 * (e & 1))));
+    }
+  if (w > 0)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) red[w - 1][lane * 8 + e] = acc[e];
+  __syncthreads();
+  if (w == 0 && c < N) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] += red[0][lane * 8 + e] + red[1][lane * 8 + e] + red[2][lane * 8 + e];
+    float* dst = part + static_cast<size_t>(blockIdx.y) * N + c;
+    *reinterpret_cast<f32x4_t*>(dst) = f32x4_t{acc[0], acc[1], acc[2], acc[3]};
+    *reinterpret_cast<f32x4_t*>(dst + 4) = f32x4_t{acc[4], acc[5], acc[6], acc[7]};
+  }
+}
+
+// sums of [slabs][N] float32 rows; blockIdx.y picks one of two sources (the weight's and the bias's partials of a LayerNorm)
+template <typename OUT>
+__global__ __launch_bounds__(256) void column_sum_final_kernel(const float* __restrict__ part0, const float* __restrict__ part1,
+                                                               OUT* __restrict__ out0, OUT* __restrict__ out1, int slabs, int N) {
+  __shared__ float red[4][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, c = blockIdx.x * 64 + lane;
+  const float* part = blockIdx.y ? part1 : part0;
+  OUT* out = blockIdx.y ? out1 : out0;
+  float a[4] = {0.f, 0.f, 0.f, 0.f};
+  if (c < N)
+    for (int s = w; s < slabs; s += 16)
+#pragma unroll
+      for (int d = 0; d < 4; ++d)
+        if (s + 4 * d < slabs) a[d] += part[static_cast<size_t>(s + 4 * d) * N + c];
+  red[w][lane] = (a[0] + a[1]) + (a[2] + a[3]);
+  __syncthreads();
+  if (w == 0 && c < N) {
+    const float v = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
+    if constexpr (sizeof(OUT) == 2) out[c] = f32_to_bf16(v);
+    else out[c] = v;
+  }
+}
+
+// about two blocks a CU, and sixteen rows (one trip of the four waves) at least
+int column_sum_slabs(int M, int N) {
+  const int cols = (N + 511) / 512, most = (M + 15) / 16, want = (512 + cols - 1) / cols;
+  return want < most ? want : most;
+}
+void launch_column_sum(const bf16_t* G, float* part, bf16_t* out, int M, int N, hipStream_t st) {
+  const int slabs = column_sum_slabs(M, N);
+  hipLaunchKernelGGL(column_sum_slab_kernel, dim3((N + 511) / 512, slabs), dim3(256), 0, st, G, part, M, N, (M + slabs - 1) / slabs);
+  hipLaunchKernelGGL((column_sum_final_kernel<bf16_t>), dim3((N + 63) / 64, 1), dim3(256), 0, st, part, part, out, out, slabs, N);
+}
+void launch_column_sum_pair(const float* p0, const float* p1, float* out0, float* out1, int slabs, int N, hipStream_t st) {
+  hipLaunchKernelGGL((column_sum_final_kernel<float>), dim3((N + 63) / 64, 2), dim3(256), 0, st, p0, p1, out0, out1, slabs, N);
+}
+
 }  // namespace evgpt

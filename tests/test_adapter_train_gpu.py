@@ -301,3 +301,18 @@ def test_padded_batch_step_equals_single_sample_steps(dev):
             continue
         ga, gb = pa.grad.float(), pb.grad.float()
         assert (ga - gb).abs().max() < 6e-2 * gb.abs().max() + 1e-4, (n, float((ga - gb).abs().max()), float(gb.abs().max()))
+
+
+# one row, a slab's remainder, columns past a block of 512 and short of a wave, many rows over few columns
+@pytest.mark.parametrize("m,n", [(1, 8), (15, 520), (17, 4096), (3200, 4096), (203, 1000), (70001, 16)])
+def test_column_sum_at_its_edges(dev, m, n):
+    from eventgpt_amd.ops import hip
+    g = torch.randn(m, n, generator=torch.Generator().manual_seed(m)).to(torch.bfloat16)
+    want = g.double().sum(0)
+    got = hip.raw.column_sum(g.to(dev)).cpu()
+    # float32 chains of at most the row count: m 2^-24 of the sum of magnitudes, then half a step of bfloat16
+    bound = m * 2.0 ** -24 * g.double().abs().sum(0) + 2.0 ** -8 * want.abs()
+    assert bool(((got.double() - want).abs() <= bound).all())
+    g[m // 2, n - 1] = float("inf")
+    got = hip.raw.column_sum(g.to(dev)).cpu()
+    assert got[-1] == float("inf") and bool(torch.isfinite(got[:-1]).all())
