@@ -1324,7 +1324,7 @@ Tensor clip_preprocess(const Tensor& img, const Tensor& hstart, const Tensor& hc
   return clip_pixels(img, false, hstart, hcount, hweight, vstart, vcount, vweight, S, resize_h, resize_w, top, left, mean, stdv);
 }
 
-// A host event stream as one word an event (x | y << 15 | (p != 0) << 30) in pinned memory, and the image it needs: {words,
+// A host event stream as one word an event (x | y << 15 | (p != 0) << 30), and the image it needs: {words,
 // int64 [height, width]}.  An empty list where it does not fit: empty, other than integers, coordinates below zero or from 2^15 on.
 template <typename X, typename P>
 static bool pack_words(const X* x, const X* y, const P* p, int64_t n, int* out, int64_t* hw) {
@@ -1346,7 +1346,7 @@ std::vector<Tensor> pack_events(const Tensor& x, const Tensor& y, const Tensor& 
   for (const Tensor* t : {&x, &y, &p}) TORCH_CHECK(t->is_cpu() && t->is_contiguous(), "pack_events: contiguous host tensors");
   TORCH_CHECK(y.numel() == n && p.numel() == n, "pack_events: x, y and p differ in length");
   if (n == 0 || n >= (1ll << 30) || x.scalar_type() != y.scalar_type()) return {};
-  Tensor words = at::empty({n}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+  Tensor words = at::empty({n}, at::TensorOptions().dtype(at::kInt));
   Tensor hw = at::empty({2}, at::TensorOptions().dtype(at::kLong));
   bool ok = false;
   const auto polarity = [&](auto xt) {
