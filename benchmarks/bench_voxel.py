@@ -34,7 +34,7 @@ def main():
             torch.cuda.synchronize()
             res[priv] = ((time.perf_counter() - t0) / 10 * 1e3, out)
         assert torch.equal(res[False][1][0], res[True][1][0])
-        print(f"{n:.0e} {name} events, by {by}: atomic-per-event {res[False][0]:.3f} ms, LDS bands {res[True][0]:.3f} ms "
+        print(f"{n:.0e} {name} events, by {by}: atomic-per-event {res[False][0]:.3f} ms, ordered in LDS {res[True][0]:.3f} ms "
               f"({n / res[True][0] / 1e6:.1f} G events/s), whole call incl. bounds + output zeroing", flush=True)
 
 
