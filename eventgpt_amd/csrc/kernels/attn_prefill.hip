@@ -39,7 +39,8 @@ struct AttnParams {
   int Sq, Sk, Hq, Hkv;
   int q_offset;                 // absolute position of query row 0 minus key 0 (causal)
   int q_offset_from_len;        // if set: q_offset = kv_len[b] - Sq
-  float scale_log2e;
+  float scale_log2e;            // positive: the softmax takes maxima of raw scores; see set_scale
+  unsigned int q_and, q_xor;    // applied to the words of Q
   // split-KV mode (few query rows against a long cache): block x = key split
   float* part_o;                // [B][Hq][nsplit][Sq][D] unnormalised fp32
   float* part_ml;               // [B][Hq][nsplit][Sq][2] (running max in log2 units, sum)
@@ -50,6 +51,18 @@ struct AttnParams {
   int gate_ld;
   const int* items;             // ITEMS: [blocks][4] first query row, rows (<= 64), key row of the chunk, position in it
 };
+// softmax(s Q K^T) with any s, by a positive scale: a negative s flips the signs of Q, zero clears Q (all scores are then equal)
+static void set_scale(AttnParams& p, float scale) {
+  p.q_and = scale == 0.f ? 0u : 0xffffffffu;
+  p.q_xor = scale < 0.f ? 0x80008000u : 0u;
+  p.scale_log2e = (scale == 0.f ? 1.f : (scale < 0.f ? -scale : scale)) * 1.4426950408889634f;
+}
+__device__ __forceinline__ bf16x8_t load_q(const AttnParams& p, const bf16_t* src) {
+  u32x4_t v = load16(src);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = (v[i] & p.q_and) ^ p.q_xor;
+  return __builtin_bit_cast(bf16x8_t, v);
+}
 __device__ __forceinline__ float head_gate(const AttnParams& p, long long row, int h) {
   return 1.f / (1.f + __expf(-bf16_to_f32(p.gate[row * p.gate_ld + h])));
 }
@@ -105,7 +118,7 @@ __global__ __launch_bounds__(256 * GROUPS) void attn_prefill_kernel(AttnParams p
     const bf16_t* qp = p.q + b * p.q_sb + static_cast<long long>(qi_c) * p.q_ss + h * p.q_sh;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
-      qf[ks] = *reinterpret_cast<const bf16x8_t*>(qp + ks * 32 + g * 8);
+      qf[ks] = load_q(p, qp + ks * 32 + g * 8);
   }
 
   const bf16_t* kbase = p.k + b * p.k_sb + hk * p.k_sh;
@@ -372,7 +385,7 @@ __global__ __launch_bounds__(AW_WAVES * 64) void attn_prefill_wide_kernel(AttnPa
     const int qc = qi[qt] < p.Sq ? qi[qt] : p.Sq - 1;
     const bf16_t* qp = p.q + b * p.q_sb + static_cast<long long>(qc) * p.q_ss + h * p.q_sh;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qf[qt][ks] = *reinterpret_cast<const bf16x8_t*>(qp + ks * 32 + g * 8);
+    for (int ks = 0; ks < KS; ++ks) qf[qt][ks] = load_q(p, qp + ks * 32 + g * 8);
   }
 
   const unsigned char* kbase = reinterpret_cast<const unsigned char*>(p.k + b * p.k_sb + hk * p.k_sh);
@@ -625,7 +638,7 @@ void launch_attn_items(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf16_t
   p.k_ss = p.v_ss = kld;
   p.q_sh = p.k_sh = p.v_sh = p.o_sh = D;
   p.Hq = Hq; p.Hkv = Hkv; p.items = items; p.gate = gate; p.gate_ld = gate_ld;
-  p.scale_log2e = scale * 1.4426950408889634f;
+  set_scale(p, scale);
   const dim3 grid(n_items, Hq), block(256);
   if (D == 128) hipLaunchKernelGGL((attn_prefill_kernel<128, true, false, 1, true, true>), grid, block, 0, st, p);
   else hipLaunchKernelGGL((attn_prefill_kernel<64, true, false, 1, true, true>), grid, block, 0, st, p);
@@ -653,7 +666,7 @@ void launch_attn_prefill(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf16
   p.o_sb = strides[9]; p.o_ss = strides[10]; p.o_sh = strides[11];
   p.kv_len = kv_len; p.Sq = Sq; p.Sk = Sk; p.Hq = Hq; p.Hkv = Hkv;
   p.q_offset = q_offset; p.q_offset_from_len = q_offset_from_len;
-  p.scale_log2e = scale * 1.4426950408889634f;
+  set_scale(p, scale);
   if (nsplit > 0) {
     // few query rows (Sq <= 64), causal, long cache: split the keys over blocks
     dim3 sgrid(nsplit, Hq, B), cgrid(Sq, Hq, B);

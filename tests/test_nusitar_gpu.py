@@ -555,6 +555,32 @@ def test_chunk_attention(raw, dev, dtype, H, G, D, size):
         assert N.rel_err(o.view(len(lens), -1), want[last.cpu()]) < tol
 
 
+@pytest.mark.parametrize("scale", [-0.2, 0.0])
+@pytest.mark.parametrize("H,G,D,lens", [(4, 2, 64, [1, 65, 130]), (2, 1, 128, [70, 300]), (2, 2, 64, [1500]), (2, 1, 128, [1500]), (64, 8, 64, [1030])])
+def test_scales_that_are_not_positive(raw, dev, H, G, D, lens, scale):
+    """Any scale is accepted, and the kernels that take row maxima before scaling serve it: items, 64-row blocks, wide blocks of
+    both sizes, tiles that cross the diagonal.  The output is rounded once (half of 2^-8 of a value), the weights add up to one and
+    have 16 bits each: 2^-16 of the largest of v besides."""
+    def close(got, want):
+        assert bool(((got.double().cpu().view_as(want) - want).abs() <= want.abs() * 2 ** -8 + vr.abs().max() * 2 ** -16).all())
+    T = sum(lens)
+    (q, qr), (k, kr), (v, vr) = (typed(rnd(T, n, D, seed=i), torch.bfloat16, dev) for i, n in enumerate((H, G, G)))
+    runs, items, *_ = RowBatch(dev, False, seqs=pack(lens)).chunk_tables(4096)
+    want, r0 = [], 0
+    for n in lens:
+        seen = torch.ones(n, n, dtype=torch.bool).tril()
+        w = [torch.softmax((qr[r0:r0 + n, h] @ kr[r0:r0 + n, h * G // H].T * scale).masked_fill(~seen, -torch.inf), 1) @ vr[r0:r0 + n, h * G // H]
+             for h in range(H)]
+        want.append(torch.stack(w, 1))
+        r0 += n
+    want = torch.cat(want).reshape(T, -1)
+    close(raw.attn_chunk(q, k, v, items, scale), want)
+    o = torch.zeros_like(q)
+    for q0, n, key0, off, reps in runs:
+        raw.attn_runs_(q, k, v, o, q0, n, key0, off, reps, scale)
+    close(o, want)
+
+
 def test_packs_of_long_and_short_runs_share_the_item_launch(raw, dev):
     """Runs that take the wide blocks get a launch each, the others one launch over their items (remainders of one row
     to a full tile, gated heads): the same rows as the wide and 64-row kernels give run by run.  Both kernels carry the

@@ -126,6 +126,15 @@ def test_attention(dev, D, H, Hkv, Sq, Sk, causal):
     _close(o, o_ref, 2e-2, 2e-2)
 
 
+@pytest.mark.parametrize("scale", [-0.15, 0.0])
+@pytest.mark.parametrize("D,Sq,Sk,causal", [(64, 577, 577, False), (128, 40, 300, True), (128, 1500, 1500, False)])
+def test_attention_scales_that_are_not_positive(dev, D, Sq, Sk, causal, scale):
+    """Two key groups a block, few rows against many keys, wide blocks without a mask; 2e-2 as above."""
+    q, k, v = (_rand(1, n, 4, D, dev=dev, seed=i) for i, n in enumerate((Sq, Sk, Sk)))
+    want = ref.attention(q.float() * (scale * D ** 0.5), k.float(), v.float(), causal, q_offset=Sk - Sq)
+    _close(_hip().attention(q, k, v, causal, scale, Sk - Sq), want, 2e-2, 2e-2)
+
+
 def test_attention_spike_rescale(dev):
     """A late key with a huge score forces the online-softmax rescale branch."""
     B, S, H, D = 1, 200, 2, 128
