@@ -29,10 +29,27 @@ from ..models.layered import (AttentionSpec, DenseMLPSpec, LatentAttentionSpec, 
 ATTN_TILE = 64           # query rows per work item of the chunk attention
 
 
-def long_run(rows: int, reps: int) -> bool:
-    """Runs of query rows that get a launch of their own: the 256-row blocks of the flash kernel want 1 400 rows, or several
-    runs of 512 (``attn_prefill.hip``); shorter runs of a pack share one launch of 64-row blocks."""
-    return rows >= 1400 or (reps > 1 and rows >= 512)
+def long_run(rows: int, reps: int, heads: int = 1, dim: int = 64, alone: bool = False) -> bool:
+    """Runs of query rows that get a launch of their own; the others of a pack share one launch of 64-row blocks.  The flash
+    kernel takes 256-row blocks of 1 400 rows, of several runs of 512, and from 512 rows on where the heads make 256 blocks
+    (``attn_prefill.hip``).  The last are worth it for a run that is ``alone``, from 1 024 rows, or that fills its blocks of 128-wide
+    heads; us of own launches / the shared one: 1 x 1024 rows, 64 heads of 128, 54 / 73; 4 x 1024 216 / 269; 8 x 512, 128 heads, 276 / 304;
+    behind with 520 + 60 + 60 rows, 96 heads (45 / 37), and 4 x 768, 96 heads of 64 (129 / 101)."""
+    if rows >= 1400 or (reps > 1 and rows >= 512):
+        return True
+    wide = rows >= 512 and -(-rows // 256) * heads >= 256
+    return wide and (alone or rows >= 1024 or (dim == 128 and rows % 256 == 0))
+
+
+def _run_items(runs, heads: int, dim: int) -> List[int]:
+    """Work items (first row, rows, key row of the chunk, position in it) of all runs, those of ``long_run`` runs last."""
+    items: Tuple[List[int], List[int]] = ([], [])
+    for q0, n, key0, off, reps in runs:
+        out = items[long_run(n, reps, heads, dim, len(runs) == 1)]
+        for r in range(reps):
+            for a in range(0, n, ATTN_TILE):
+                out.extend((q0 + r * n + a, min(ATTN_TILE, n - a), key0 + r * n, off + a))
+    return items[0] + items[1]
 
 
 GATE_NONE, GATE_SILU_BEFORE, GATE_SIGMOID_AFTER = 0, 1, 2      # group_norm_rows
@@ -118,14 +135,14 @@ class RowBatch:
         flat = torch.tensor([v for l in lists for v in l], dtype=torch.int32).to(self.device)
         return flat.split([len(l) for l in lists])
 
-    def chunk_tables(self, size: int):
+    def chunk_tables(self, size: int, heads: int = 1, dim: int = 64):
         """For a chunk mask of ``size``: ``(runs, items, row_kv, row_keep, copies, kv_rows)``, the items of ``long_run`` runs
-        last.  Keys live in a buffer with the rows of every sequence in order, preceded by the cached keys of the chunk it continues."""
-        t = self._tables.get(size)
+        of that many heads last.  Keys live in a buffer with the rows of every sequence in order, preceded by the cached keys of the chunk it continues."""
+        key = (size, heads, dim)
+        t = self._tables.get(key)
         if t is not None:
             return t
         runs: List[Tuple[int, int, int, int, int]] = []     # q row, rows, key row of the chunk, position in it, repeats
-        items: Tuple[List[int], List[int]] = ([], [])       # of the short runs, of the long ones
         row_kv: List[int] = []
         keep: List[int] = []
         copies: List[int] = []
@@ -145,33 +162,28 @@ class RowBatch:
                 reps = (s.rows - done) // size if off == 0 and n == size else 1
                 key0 = base + done - off
                 runs.append((s.row0 + done, n, key0, off, reps))
-                for r in range(reps):
-                    for a in range(0, n, ATTN_TILE):
-                        items[long_run(n, reps)].extend((s.row0 + done + r * n + a, min(ATTN_TILE, n - a), key0 + r * n, off + a))
                 done += n * reps
             kv = base + s.rows
-        items_d, row_kv_d, keep_d, copies_d = self._upload(items[0] + items[1], row_kv, keep, copies)
+        items_d, row_kv_d, keep_d, copies_d = self._upload(_run_items(runs, heads, dim), row_kv, keep, copies)
         t = (runs, items_d.view(-1, 4), row_kv_d, keep_d, copies_d.view(-1, 4) if copies else None, kv)
-        self._tables[size] = t
+        self._tables[key] = t
         return t
 
-    def causal_tables(self):
+    def causal_tables(self, heads: int = 1, dim: int = 64):
         """For plain causal attention: ``(runs, items, copies, kv_rows)`` of ``chunk_tables``, where a buffer holds
         every key of every sequence and ``copies`` brings all of them from the caches."""
-        t = self._tables.get("causal")
+        key = ("causal", heads, dim)
+        t = self._tables.get(key)
         if t is None:
             runs: List[Tuple[int, int, int, int, int]] = []
-            items: Tuple[List[int], List[int]] = ([], [])
             copies: List[int] = []
             kv = 0
             for s in self.seqs:
                 runs.append((s.row0, s.rows, kv, s.start, 1))
-                for a in range(0, s.rows, ATTN_TILE):
-                    items[long_run(s.rows, 1)].extend((s.row0 + a, min(ATTN_TILE, s.rows - a), kv, s.start + a))
                 copies += [s.slot, 0, kv, s.start + s.rows]
                 kv += s.start + s.rows
-            items_d, copies_d = self._upload(items[0] + items[1], copies)
-            t = self._tables["causal"] = (runs, items_d.view(-1, 4), copies_d.view(-1, 4), kv)
+            items_d, copies_d = self._upload(_run_items(runs, heads, dim), copies)
+            t = self._tables[key] = (runs, items_d.view(-1, 4), copies_d.view(-1, 4), kv)
         return t
 
     def latents(self, cache: torch.Tensor, gather) -> torch.Tensor:
@@ -180,7 +192,8 @@ class RowBatch:
         key = ("latents", cache.data_ptr())
         t = self._tables.get(key)
         if t is None:
-            _, _, copies, kv = self.causal_tables()
+            tables = (v for k, v in self._tables.items() if k[0] == "causal")    # (of any heads: the copies are the same)
+            _, _, copies, kv = next(tables, None) or self.causal_tables()
             one = self.seqs[0]
             t = cache[one.slot, :kv] if len(self.seqs) == 1 else gather(cache, copies, kv)
             self._tables[key] = t
@@ -297,13 +310,11 @@ class Mixer:
 
 def attend_runs(raw, q, k, v, runs, items, scale: float, flash: bool, *gate) -> torch.Tensor:
     """Causal attention of a pack's runs, ``[rows, H * D]``: a launch of the flash kernel for each long run if it takes the
-    heads, one launch for all others (``RowBatch.chunk_tables``)."""
-    short = sum(-(-n // ATTN_TILE) * reps for _, n, _, _, reps in runs if not long_run(n, reps)) if flash else len(items)
-    o = raw.attn_chunk(q, k, v, items[:short], scale, *gate)
-    if flash:
-        for q0, n, key0, off, reps in runs:
-            if long_run(n, reps):
-                raw.attn_runs_(q, k, v, o, q0, n, key0, off, reps, scale, *gate)
+    heads, one launch for all others (``RowBatch.chunk_tables`` for q's heads)."""
+    own = [run for run in runs if flash and long_run(run[1], run[4], *q.shape[1:], len(runs) == 1)]
+    o = raw.attn_chunk(q, k, v, items[:len(items) - sum(-(-n // ATTN_TILE) * reps for _, n, _, _, reps in own)], scale, *gate)
+    for q0, n, key0, off, reps in own:
+        raw.attn_runs_(q, k, v, o, q0, n, key0, off, reps, scale, *gate)
     return o.view(o.shape[0], -1)
 
 
@@ -338,7 +349,7 @@ class AttentionBranch(Mixer):
 
     def prompt(self, rows: RowBatch, src: torch.Tensor, col: Dict[str, int]) -> torch.Tensor:
         s, raw = self.spec, self.raw
-        runs, items, row_kv, keep, copies, kv_rows = rows.chunk_tables(self.size)
+        runs, items, row_kv, keep, copies, kv_rows = rows.chunk_tables(self.size, s.heads, self.D)
         k = torch.empty(kv_rows, s.kv_heads, self.D, dtype=self.dtype, device=self.device)
         v = torch.empty_like(k)
         if copies is not None:      # before the cache slots of the chunk are written over
@@ -525,7 +536,7 @@ class LatentAttentionMixer(Mixer):
     def prompt_attention(self, rows: RowBatch, q: torch.Tensor, src: torch.Tensor) -> torch.Tensor:
         raw, s, D = self.raw, self.spec, self.D
         H = s.heads
-        runs, items, _, kv_rows = rows.causal_tables()
+        runs, items, _, kv_rows = rows.causal_tables(H, D)
         kv = raw.linear(rows.latents(self.owner.cache, raw.latent_gather), self.w_ukv, False)
         q, k, v = q.view(-1, H, D), kv[:, :H * D].unflatten(1, (H, D)), kv[:, H * D:].unflatten(1, (H, D))
         return attend_runs(raw, q, k, v, runs, items, s.scale, not self.f32 and D <= 128, src, self.proj.col["g"])

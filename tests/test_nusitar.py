@@ -97,6 +97,30 @@ def test_padding_helpers():
     assert [mixers.pad_attn_head(n) for n in (1, 64, 65, 128, 129)] == [64, 64, 128, 128, 192]
 
 
+@pytest.mark.parametrize("heads,dim,lens,own", [
+    (64, 128, [1024], [1024]), (64, 64, [1100], [1100]), (63, 128, [1024], []), (64, 128, [30, 1024, 700], [1024]),
+    (128, 128, [512, 40], [512]), (128, 64, [512, 40], []), (128, 64, [512], [512]), (96, 128, [520, 60], []), (8, 64, [1400, 3], [1400])])
+def test_runs_that_fill_the_wide_blocks_get_their_own_launch(heads, dim, lens, own):
+    """By rows and heads; whatever the rule says, launches and items together cover every row once."""
+    row0 = [sum(lens[:i]) for i in range(len(lens))]
+    rb = RowBatch("cpu", False, seqs=[Sequence_(i, r, n, 0) for i, (r, n) in enumerate(zip(row0, lens))])
+
+    class Raw:
+        def attn_chunk(self, q, k, v, items, scale):
+            o = torch.zeros_like(q)
+            for r, n, _, _ in items.tolist():
+                o[r:r + n] += 1
+            return o
+
+        def attn_runs_(self, q, k, v, o, q0, rows, key0, off, reps, scale):
+            launches.append(rows)
+            o[q0:q0 + rows * reps] = 1
+    for tables in (rb.chunk_tables(4096, heads, dim), rb.causal_tables(heads, dim)):
+        launches = []
+        o = mixers.attend_runs(Raw(), torch.zeros(sum(lens), heads, dim), None, None, *tables[:2], 1.0, True)
+        assert launches == own and bool((o == 1).all())
+
+
 @pytest.mark.parametrize("size", [1, 2, 5, 7, 64, 100, 1000])
 def test_chunk_tables_cover_every_query_once(size):
     """Every query row is in one run and one work item, and its visible keys in the key buffer are the ones a chunk
