@@ -245,24 +245,28 @@ class LayeredEngine(DecodeEngine):
         """Feed given tokens (nothing is sampled): ``tokens[i]`` continues the sequence in ``slots[i]``.  Single
         tokens of running sequences go through the decode step, everything else through the packed prefill.
         Returns the logits ``[n, V]`` at the wanted places, in order, or None."""
-        starts = [self._fed[s] for s in slots]
+        slots = [range(self.B)[s] for s in slots]       # (from the end if negative; a call that raises feeds nothing)
+        starts, fed = [self._fed[s] for s in slots], list(self._fed)
         step = all(t.numel() == 1 and s > 0 for t, s in zip(tokens, starts))
         for s, t in zip(slots, tokens):
-            self._fed[s] += int(t.numel())
+            fed[s] += int(t.numel())
         if not step:
             _, logits = self._feed(slots, tokens, starts, want)
-            self.raw.feed_rows_(self.pos, None, list(slots), [self._fed[s] - 1 for s in slots])
-            self._pos_hi = max([self._pos_hi] + [self._fed[s] for s in slots])
+            self._fed = fed
+            self.raw.feed_rows_(self.pos, None, slots, [fed[s] - 1 for s in slots])
+            self._pos_hi = max([self._pos_hi] + [fed[s] for s in slots])
             return logits
-        if max(self._fed) > self.l_max:
+        if max(fed) > self.l_max:
             raise ValueError(f"sequence exceeds max_len ({self.l_max})")
         # slots and host tokens travel as kernel arguments: nothing here waits for the device, so steps queue up behind each
-        # other (1b-size Nusitar, one stream: 500 us a token with index tensors and copies around the graph, 400 now)
+        # other (1b-size Nusitar, one stream: 500 us a token with index tensors and copies around the graph, 400 without, 360 with
+        # the step kernels as they are)
         if all(t.is_cuda for t in tokens):
             tok = torch.cat([t.reshape(-1) for t in tokens]).to(torch.int32)
-            self.raw.feed_rows_(self.sampled, self.active, list(slots), [], tok.to(self.device))
+            self.raw.feed_rows_(self.sampled, self.active, slots, [], tok.to(self.device))
         else:
-            self.raw.feed_rows_(self.sampled, self.active, list(slots), [int(t) for t in tokens])
+            self.raw.feed_rows_(self.sampled, self.active, slots, [int(t) for t in tokens])
+        self._fed = fed
         self._commit_sampled()
         self.decode_step(greedy=False)
         rows = [s for s, w in zip(slots, want) for _ in w]

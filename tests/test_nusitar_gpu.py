@@ -779,6 +779,23 @@ def test_long_prompts_run_in_portions(mixed, mixed_want):
     assert N.rel_err(lg[151:], want[[99, 0]]) < tol
 
 
+def test_slots_from_the_end_and_calls_that_raise(dev):
+    """Slots count from the end if negative, in prompts and in steps; a call that raises feeds nothing."""
+    m = N.build(SMALL, torch.float32, dev, seed=6)
+    e = m.engine(max_len=40, max_batch=3)
+    a, b = N.prompt(20, 50, 8), N.prompt(17, 50, 9)
+    e.extend([0, 2], [a[:-2], b[:-2]], [[], []])
+    for slots, tokens, err in (([0, 3], [a[:1], b[:1]], IndexError), ([-4], [a[:1]], IndexError), ([0], [a[:0]], ValueError),
+                               ([0, -1], [a[:2], a.repeat(2)], ValueError)):
+        with pytest.raises(err):
+            e.extend(slots, tokens, [[]] * len(slots))
+    got = [e.extend([-1, 0], [b[i:i + 1] if i < -1 else b[i:], a[i:i + 1] if i < -1 else a[i:]], [[0], [0]]) for i in (-2, -1)]
+    for t, g in ((b, [g[0] for g in got]), (a, [g[1] for g in got])):
+        assert N.rel_err(torch.stack(g), N.oracle_logits(m, t)[-2:]) < MODEL_TOL[torch.float32]
+    e.reset()
+    assert N.rel_err(e.extend([-2], [a], [[19]]), N.oracle_logits(m, a)[-1:]) < MODEL_TOL[torch.float32]
+
+
 def test_long_decoding(dev):
     """Several hundred steps over many chunk borders, in 32 bit: nothing drifts."""
     m = N.build(SMALL, torch.float32, dev, seed=6)
