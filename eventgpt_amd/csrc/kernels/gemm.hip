@@ -1157,17 +1157,26 @@ static bool use_256(int M, int N, int K = 0) {
 
 // Short contractions (the ViT's 1024-wide layers: 16 K-tiles) are bound by the round trip of each K-tile, which waves of
 // other workgroups have to cover: eight waves on the 64 x 128 tile with two stages (48 KB: three workgroups, 24 waves a
-// CU), or with three where the tiles are fewer than three for every two CUs.  us against the best of the other tiles, weights
-// in the die-level cache: 1154 x 4096 x 1024 22.5 vs 32.8, 1154 x 3072 16.1 vs 16.7, 2885 x 4096 45.1 vs 54.2 (8-wave
-// 256 x 256, 192 tiles), 2885 x 3072 34.4 vs 37.5; 577 x 4096 from memory 18.7 vs 20.5 (two stages 22.2).  Whole vision path,
-// ms at 1 / 2 / 3 / 4 / 5 frames: 2.11 / 3.24 / 3.82 / 4.80 / 4.95 -> 2.04 / 2.90 / 3.61 / 4.29 / 4.71.  Behind where the
-// tiles leave CUs idle (577 x 3072, 240 tiles: 13.6 vs 11.9), over longer contractions (636 x 12288 x 4096: 116 vs 74; 600 x
-// 9280 x 2048 39 vs 36), for 1024 columns (2885 rows 15.5 vs 14.2) and towards a whole round of 256 x 256 tiles (with the
-// 3462 and 4039 rows of six and seven frames into 3072 columns, 168 and 192 of them: 5.40 -> 5.47 and 5.86 -> 6.02 ms).
-static bool use_64x128_w8(int M, int N, int K) {
-  const long long t = static_cast<long long>((M + 63) / 64) * ((N + 127) / 128);
-  return K > 0 && K <= 1024 && N >= 2048 && t >= 300 &&
-         static_cast<long long>((M + 255) / 256) * ((N + 255) / 256) < (N >= 4096 ? 200 : 160);
+// CU), or with three under 400 tiles (about three for every two CUs: 577 x 4096 x 1024 from memory 18.7 us, two stages
+// 22.2, four waves 20.5).  Behind where the tiles leave CUs idle (577 x 3072, 240 tiles: 13.6 vs 11.9), over longer
+// contractions (636 x 12288 x 4096: 116 vs 74; 600 x 9280 x 2048 39 vs 36) and for 1024 columns (2885 rows 15.5 vs 14.2).
+// Lines between, us with weights from memory, this tile vs the other choice:
+//  * one round of three workgroups a CU (768 tiles) is ahead: 750 tiles 1.09 to 1.47 times as fast
+//  * more than a round where the 128 x 128 tile takes one (512): ahead up to K = 320 (1.03 to 1.15; with 256 rows, whose few row
+//    tiles share a weight tile, 0.96), behind from there to 256 x 32000 x 1024 46.0 vs 33.0, 1000 x 8192 x 1024 40.0 vs 29.8, 2308 x
+//    3072 x 1024 32.0 vs 28.3; with an activation, whose epilogue more waves take, level at K = 640, behind from 768 (836 x 8192 0.87)
+//  * where that takes two: ahead (3300 x 2560 x 1024, 520 tiles of it, 1.33) unless the 8-wave kernel has more than 152 tiles
+//    of a round to itself: 140 to 152 of them 1.09 to 1.19, 172 to 192 0.84 to 1.0; with an activation 1.09 to 1.5 up to 199
+//  * a residual, which that kernel's epilogue reads in whole lines, keeps it ahead of this tile: 0.81 to 0.95
+static bool use_64x128_w8(int M, int N, int K, bool act, bool res) {
+  auto tiles = [&](int bm, int bn) {
+    return static_cast<long long>((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+  };
+  if (K <= 0 || K > 1024 || N < 2048 || tiles(64, 128) < 300 || tiles(256, 256) >= (N >= 4096 ? 200 : 160)) return false;
+  if (res && use_256(M, N, K)) return false;
+  if (tiles(64, 128) <= 768) return true;
+  if (tiles(128, 128) <= 512) return act ? K <= 640 : K <= 320 && M > 256;
+  return K <= 320 || act || !use_256(M, N, K) || tiles(256, 256) <= 152;
 }
 static void launch_64x128_w8(const GemmParams& p, hipStream_t st) {
   if (static_cast<long long>((p.M + 63) / 64) * ((p.N + 127) / 128) < 400) launch_cfg<64, 128, 2, 4, 3>(p, st);
@@ -1194,8 +1203,9 @@ static int narrow_256_splits(int M, int N, int K) {
 }
 
 // K = 0: the caller cannot split K (argmax partials, K-strided operands)
-// k_real: the contraction length when the caller knows it (the tile choice depends on it), also where K = 0
-static GemmCfg pick_cfg(int M, int N, int K = 0, int k_real = 0) {
+// k_real: the contraction length when the caller knows it (the tile choice depends on it), also where K = 0; act, res: the
+// epilogue applies an activation, adds a residual
+static GemmCfg pick_cfg(int M, int N, int K = 0, int k_real = 0, bool act = false, bool res = false) {
   if (k_real == 0) k_real = K;
   if (g_forced_cfg >= 0) return static_cast<GemmCfg>(g_forced_cfg);
   auto tiles = [&](int bm, int bn) {
@@ -1203,7 +1213,7 @@ static GemmCfg pick_cfg(int M, int N, int K = 0, int k_real = 0) {
   };
   // thresholds from benchmarks/bench_gemm.py on MI355X
   if (M <= 32) return tiles(32, 128) >= 256 ? CFG_32x128 : CFG_32x64;
-  if (use_64x128_w8(M, N, k_real)) return CFG_64x128_W8;
+  if (use_64x128_w8(M, N, k_real, act, res)) return CFG_64x128_W8;
   if (use_256(M, N, k_real)) return CFG_256x256;
   if (K && narrow_256_splits(M, N, K) >= 2) return CFG_256x256;
   // Narrow outputs over a long contraction (a few hundred rows into 4096 columns over 11008, the
@@ -1354,7 +1364,7 @@ void launch_gemm_bf16(const bf16_t* A, const bf16_t* W, bf16_t* C, float* Cf, co
     p.splitk = (K + p.k_per_split - 1) / p.k_per_split;  // drop empty trailing splits
     p.partial = splitk_ws;
   }
-  GemmCfg cfg = pick_cfg(M, N, (splitk_ws && !amax_val) ? K : 0, amax_val ? 0 : K);
+  GemmCfg cfg = pick_cfg(M, N, (splitk_ws && !amax_val) ? K : 0, amax_val ? 0 : K, act != ACT_NONE, res != nullptr);
   if (p.k_cols) {
     // short last K-tile: the two instances compiled with the masked staging path (these are the
     // low-rank products and other short contractions; the tile choice matters little for them)

@@ -290,6 +290,19 @@ def test_eight_waves_on_the_64_row_tile(dev, M, N, K):
     _check(hip.raw.linear(x, w, bias, res, 1, False), want, K)
 
 
+# either side of the lines between the tiles for short contractions: one and two rounds of 128 x 128 tiles, of 256 x 256 tiles
+@pytest.mark.parametrize("M,N,K", [(256, 32000, 1024), (836, 8192, 640), (836, 8192, 704), (2308, 3072, 320), (2308, 4096, 384), (3300, 2560, 1024),
+                                   (2885, 3072, 1024), (2885, 4096, 960)])
+def test_short_contractions_beside_the_lines_of_the_tile_choice(dev, M, N, K):
+    from eventgpt_amd.ops import hip
+    x, w = _rand(M, K, dev=dev), _rand(N, K, dev=dev, seed=1, scale=0.05)
+    bias, res = _rand(N, dev=dev, seed=2), _rand(M, N, dev=dev, seed=3)
+    lin = x.float() @ w.float().t() + bias.float()
+    _check(hip.raw.linear(x, w, bias, None, 0, True), lin, K)
+    _check(hip.raw.linear(x, w, bias, res, 0, False), lin.to(torch.bfloat16).float() + res.float(), K)
+    _check(hip.raw.linear(x, w, bias, None, 1, False), torch.nn.functional.gelu(lin), K)
+
+
 @pytest.mark.parametrize("M,N,K,slabs", [(1154, 1024, 4096, 3), (2885, 1024, 4096, 2), (900, 4096, 4096, 2), (1025, 1024, 4160, 3)])
 def test_slabs_of_about_a_round_of_tiles(dev, M, N, K, slabs):
     """Products whose caller sums the slabs, split where 128 x 128 tiles are at most one a CU: the slabs add up."""
