@@ -1231,8 +1231,10 @@ static GemmCfg pick_cfg(int M, int N, int K = 0, int k_real = 0, bool act = fals
   // (more rows, slabs summed by the caller: 1154 x 1024 x 4096 in three splits 19.4 us, 2885 rows in two 33.2; unsplit
   // 64 x 128 tiles 26.4 and 38.4)
   if (g_for_slabs && g_forced_splitk == 0 && M > 1024 && K >= 4096 && tiles(128, 128) >= 64 && tiles(128, 128) < 256) return CFG_128x128;
-  // 600 x 9280 x 2048, 365 tiles: 35.6 us, 64 x 128 tiles 42.5; 300 x 12288 x 4096, 288 tiles: 63.5 vs 53.8
-  if (tiles(128, 128) >= 336) return CFG_128x128;
+  // 600 x 9280 x 2048, 365 tiles: 35.6 us, 64 x 128 tiles 42.5; 300 x 12288 x 4096, 288 tiles: 63.5 vs 53.8.  Not where the 64 x 128
+  // tiles (72 KB: two workgroups a CU) are one round, rows that leave half of the larger ones empty: 156 x 21504 x 2048, 504 of
+  // them, 35.1 us, 128 x 128 tiles 44.9
+  if (tiles(128, 128) >= 384 || (tiles(128, 128) >= 336 && tiles(64, 128) > 512)) return CFG_128x128;
   if (tiles(64, 128) >= 300) return CFG_64x128;
   if (tiles(64, 64) >= 300) return CFG_64x64;
   return CFG_32x64;

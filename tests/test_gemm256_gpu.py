@@ -290,9 +290,10 @@ def test_eight_waves_on_the_64_row_tile(dev, M, N, K):
     _check(hip.raw.linear(x, w, bias, res, 1, False), want, K)
 
 
-# either side of the lines between the tiles for short contractions: one and two rounds of 128 x 128 tiles, of 256 x 256 tiles
+# either side of the lines between the tiles for short contractions: one and two rounds of 128 x 128 tiles, of 256 x 256 tiles; and
+# of the line at 336 tiles of 128 x 128 where rows leave some half empty
 @pytest.mark.parametrize("M,N,K", [(256, 32000, 1024), (836, 8192, 640), (836, 8192, 704), (2308, 3072, 320), (2308, 4096, 384), (3300, 2560, 1024),
-                                   (2885, 3072, 1024), (2885, 4096, 960)])
+                                   (2885, 3072, 1024), (2885, 4096, 960), (156, 21504, 2048), (156, 22016, 2048), (156, 21376, 2048)])
 def test_short_contractions_beside_the_lines_of_the_tile_choice(dev, M, N, K):
     from eventgpt_amd.ops import hip
     x, w = _rand(M, K, dev=dev), _rand(N, K, dev=dev, seed=1, scale=0.05)
