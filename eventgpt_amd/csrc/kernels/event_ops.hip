@@ -588,6 +588,8 @@ __global__ __launch_bounds__(256) void clip_preproc_kernel(PreprocParams p) {
 // 640 x 480 20.0 and 39.3.  Tiles of four rows where eight would leave CUs idle: one frame of 640 x 480 9.7, with eight 13.4, by
 // pixels 11.1.
 // CODES: the source is one code a pixel (event_codes_kernel) instead of three bytes.
+// Tables whose rows reach over more than CP_SRC source rows (no resize's do) are followed without the first pass: a block
+// then resizes each tap's row where it needs it.
 constexpr int CP_COLS = 112, CP_SRC = 48;
 
 __device__ __forceinline__ int clip8_fix32(int acc) { return min(max(acc >> 22, 0), 255); }
@@ -599,13 +601,25 @@ __global__ __launch_bounds__(256) void clip_preproc_tile_kernel(PreprocParams p)
   const int cols = min(CP_COLS, p.S - ox0), rows = min(CP_ROWS, p.S - oy0);
   const bool need_h = p.resize_w != p.W, need_v = p.resize_h != p.H;
   const int first = oy0 + p.top, last = first + rows - 1;      // rows of the resized image
-  const int r0 = need_v ? p.vstart[first] : first;
-  const int n_src = min((need_v ? p.vstart[last] + p.vcount[last] : last + 1) - r0, CP_SRC);
+  int r0 = first, r1 = last + 1;                               // source rows; a lane looks at one row of the tile
+  if (need_v) {
+    const int mine = first + min(static_cast<int>(threadIdx.x) & 7, rows - 1);
+    r0 = p.vstart[mine];
+    r1 = r0 + p.vcount[mine];
+#pragma unroll
+    for (int off = 1; off < 8; off <<= 1) {
+      r0 = min(r0, __shfl_xor(r0, off, 64));
+      r1 = max(r1, __shfl_xor(r1, off, 64));
+    }
+    r0 = __builtin_amdgcn_readfirstlane(r0);
+    r1 = __builtin_amdgcn_readfirstlane(r1);
+  }
+  const int n_src = r1 - r0;
+  const bool tall = n_src > CP_SRC;                            // (the same for the whole block)
   const unsigned char* frame = p.img + static_cast<size_t>(t) * p.H * p.W * (CODES ? 1 : 3);
   constexpr int half = 1 << 21;
-  for (int i = threadIdx.x; i < n_src * CP_COLS; i += 256) {
-    const int r = i / CP_COLS, c = i % CP_COLS;
-    if (c >= cols) continue;
+  // column c of source row r0 + r, resized horizontally: one byte a channel
+  const auto resized = [&](int r, int c) -> unsigned int {
     const int rx = ox0 + c + p.left, hs = need_h ? p.hstart[rx] : rx, hc = need_h ? p.hcount[rx] : 1;
     const unsigned char* src = frame + (static_cast<size_t>(r0 + r) * p.W + hs) * (CODES ? 1 : 3);
     int v[3] = {half, half, half};
@@ -624,35 +638,47 @@ __global__ __launch_bounds__(256) void clip_preproc_tile_kernel(PreprocParams p)
     }
 #pragma unroll
     for (int ch = 0; ch < 3; ++ch) v[ch] = need_h ? clip8_fix32(v[ch]) : v[ch];
-    mid[r][c] = v[0] | v[1] << 8 | v[2] << 16;
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < rows * CP_COLS; i += 256) {
-    const int r = i / CP_COLS, c = i % CP_COLS;
-    if (c >= cols) continue;
-    const int ry = first + r, vs = (need_v ? p.vstart[ry] : ry) - r0;
-    int px[3];
-    if (need_v) {
-      const int vc = p.vcount[ry];
-      const int* w = p.vweight + ry * p.ksv;
-      int v[3] = {half, half, half};
-      for (int k = 0; k < vc; ++k) {
-        const unsigned int m = mid[vs + k][c];
-        const int wk = w[k];
-        v[0] += wk * static_cast<int>(m & 255); v[1] += wk * static_cast<int>(m >> 8 & 255); v[2] += wk * static_cast<int>(m >> 16);
+    return v[0] | v[1] << 8 | v[2] << 16;
+  };
+  // the outputs, from rows that `row(r, c)` gives
+  const auto finish = [&](auto&& row) {
+    for (int i = threadIdx.x; i < rows * CP_COLS; i += 256) {
+      const int r = i / CP_COLS, c = i % CP_COLS;
+      if (c >= cols) continue;
+      const int ry = first + r, vs = (need_v ? p.vstart[ry] : ry) - r0;
+      int px[3];
+      if (need_v) {
+        const int vc = p.vcount[ry];
+        const int* w = p.vweight + ry * p.ksv;
+        int v[3] = {half, half, half};
+        for (int k = 0; k < vc; ++k) {
+          const unsigned int m = row(vs + k, c);
+          const int wk = w[k];
+          v[0] += wk * static_cast<int>(m & 255); v[1] += wk * static_cast<int>(m >> 8 & 255); v[2] += wk * static_cast<int>(m >> 16);
+        }
+#pragma unroll
+        for (int ch = 0; ch < 3; ++ch) px[ch] = clip8_fix32(v[ch]);
+      } else {
+        const unsigned int m = row(vs, c);
+        px[0] = m & 255; px[1] = m >> 8 & 255; px[2] = m >> 16;
       }
 #pragma unroll
-      for (int ch = 0; ch < 3; ++ch) px[ch] = clip8_fix32(v[ch]);
-    } else {
-      const unsigned int m = mid[vs][c];
-      px[0] = m & 255; px[1] = m >> 8 & 255; px[2] = m >> 16;
+      for (int ch = 0; ch < 3; ++ch) {
+        const float v = (static_cast<float>(px[ch]) * (1.f / 255.f) - p.mean[ch]) * p.inv_std[ch];
+        p.out[((static_cast<size_t>(t) * 3 + ch) * p.S + oy0 + r) * p.S + ox0 + c] = f32_to_bf16(v);
+      }
     }
-#pragma unroll
-    for (int ch = 0; ch < 3; ++ch) {
-      const float v = (static_cast<float>(px[ch]) * (1.f / 255.f) - p.mean[ch]) * p.inv_std[ch];
-      p.out[((static_cast<size_t>(t) * 3 + ch) * p.S + oy0 + r) * p.S + ox0 + c] = f32_to_bf16(v);
-    }
+  };
+  if (tall) {
+    finish(resized);
+    return;
   }
+  for (int i = threadIdx.x; i < n_src * CP_COLS; i += 256) {
+    const int r = i / CP_COLS, c = i % CP_COLS;
+    if (c < cols) mid[r][c] = resized(r, c);
+  }
+  __syncthreads();
+  finish([&](int r, int c) { return mid[r][c]; });
 }
 
 // source rows of a tile fit its LDS (a resize by less than about four)

@@ -116,6 +116,27 @@ def test_event_frames_gpu_end_to_end(dev):
         assert torch.equal(px.float().cpu(), want.to(torch.bfloat16).float())
 
 
+@pytest.mark.parametrize("order", ["reversed", "scattered"])
+def test_clip_preprocess_with_tables_of_any_order(dev, order):
+    """Rows that reach further over the source than a tile holds: what a host resize by the same tables gives."""
+    from eventgpt_amd.ops import hip
+    rng = np.random.default_rng(4)
+    H, S, taps = 300, 224, 3
+    img = rng.integers(0, 256, (2, H, S, 3)).astype(np.uint8)
+    start = np.linspace(0, H - taps, S).astype(np.int64)
+    start = start[::-1].copy() if order == "reversed" else rng.permutation(start)
+    weight = rng.dirichlet(np.ones(taps), S)
+    weight = np.round(weight * (1 << 22)).astype(np.int64)
+    rows = sum(weight[:, k][None, :, None, None] * img[:, start + k].astype(np.int64) for k in range(taps))
+    resized = np.ascontiguousarray(np.clip((rows + (1 << 21)) >> 22, 0, 255).astype(np.uint8))
+    table = [torch.from_numpy(a.astype(np.int32)).to(dev) for a in (start, np.full(S, taps), weight)]
+    none = [torch.zeros(1, dtype=torch.int32, device=dev)] * 2 + [torch.zeros(1, 1, dtype=torch.int32, device=dev)]
+    tail = (S, S, S, 0, 0, [0.48, 0.46, 0.41], [0.27, 0.26, 0.28])
+    got = hip.raw.clip_preprocess(torch.from_numpy(img).to(dev), *none, *table, *tail)
+    want = hip.raw.clip_preprocess(torch.from_numpy(resized).to(dev), *none, *none, *tail)
+    assert torch.equal(got, want)
+
+
 def test_preprocess_frames_device_dispatch(dev):
     """The frame preprocessing entry point gives the same pixels from the GPU kernel
     and from the host path, and the verifier's processor uses it when given a device."""
