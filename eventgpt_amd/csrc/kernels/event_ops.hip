@@ -698,9 +698,14 @@ void launch_clip_preproc(const unsigned char* img, bf16_t* out, const int* hstar
   p.T = T; p.H = H; p.W = W; p.S = S; p.top = top; p.left = left; p.ksh = ksh; p.ksv = ksv;
   p.resize_h = resize_h; p.resize_w = resize_w;
   for (int c = 0; c < 3; ++c) { p.mean[c] = mean[c]; p.inv_std[c] = 1.f / stdv[c]; }
-  if (clip_preproc_tiles_ok(T, H, resize_h, ksv)) {
+  // Outputs worth 160 full tiles of four rows take tiles, of eight rows from 256 full ones of those on; fewer pixels go one by one:
+  // us by tiles / pixels, 112 x 112 from 336 x 336, five frames 23.8 / 22.4, eight 24.2 / 35.7; one frame of 224 x 224 from 720 x
+  // 1280 27.0 / 24.7, two 27.3 / 40.3.  Thumbnails, of which a frame is a few blocks either way, share their taps' rows: 28 x 28 from
+  // 90 x 120 20.7 / 27.1, 56 x 56 11.2 / 10.2.  (Codes are always in tiles.)
+  const long long pixels = static_cast<long long>(T) * S * S;
+  if (clip_preproc_tiles_ok(T, H, resize_h, ksv) && (codes || S <= 32 || pixels >= 160 * 4 * CP_COLS)) {
     const int cols = (S + CP_COLS - 1) / CP_COLS;
-    if (cols * ((S + 7) / 8) * T >= 256) {
+    if (pixels >= 256 * 8 * CP_COLS) {
       const dim3 grid(cols, (S + 7) / 8, T);
       if (codes) hipLaunchKernelGGL((clip_preproc_tile_kernel<true, 8>), grid, dim3(256), 0, st, p);
       else hipLaunchKernelGGL((clip_preproc_tile_kernel<false, 8>), grid, dim3(256), 0, st, p);

@@ -116,6 +116,16 @@ def test_event_frames_gpu_end_to_end(dev):
         assert torch.equal(px.float().cpu(), want.to(torch.bfloat16).float())
 
 
+# pixels one by one, tiles of four and of eight rows: either side of both lines, remainders of a tile's columns and rows
+@pytest.mark.parametrize("T,S", [(1, 267), (1, 268), (5, 113), (6, 113), (3, 276), (3, 277), (35, 81), (2, 32), (2, 33)])
+def test_clip_preprocess_beside_the_lines_of_the_kernel_choice(dev, T, S):
+    from eventgpt_amd.ops import event_ops as eo
+    img = np.random.default_rng(S).integers(0, 256, (T, 200, 150, 3)).astype(np.uint8)
+    got = eo.clip_preprocess_gpu(torch.from_numpy(img).to(dev), S).float().cpu().numpy()
+    # as for the packed frames below: the same bytes, normalised in another order
+    np.testing.assert_allclose(got, np.stack([cp.preprocess_image(f, S) for f in img]), rtol=2.0 ** -8, atol=1e-5)
+
+
 @pytest.mark.parametrize("order", ["reversed", "scattered"])
 def test_clip_preprocess_with_tables_of_any_order(dev, order):
     """Rows that reach further over the source than a tile holds: what a host resize by the same tables gives."""
