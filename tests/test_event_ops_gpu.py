@@ -201,6 +201,18 @@ def test_packed_frames_equal_the_general_ops(dev, n, h, w, slices, dtype, p_dtyp
     np.testing.assert_allclose(px.float().cpu().numpy(), want, rtol=2.0 ** -8, atol=1e-5)
 
 
+@pytest.mark.parametrize("n,h,w,slices,packs", [(4, 40, 40, 5, False), (5, 40, 40, 5, True), (500_001, 40, 40, 1, False), (500_000, 40, 40, 1, True),
+                                                (1_000_001, 40, 40, 2, True), (200_000, 1500, 1700, 5, False), (199_999, 1500, 1700, 5, True)])
+def test_streams_whose_words_would_not_be_used_are_not_packed(dev, n, h, w, slices, packs, monkeypatch):
+    """By length, and for a long stream by its first events; the frames are the general ops' either way."""
+    from eventgpt_amd.ops import event_ops as eo
+    ev, seen = _host_stream(n, h, w, np.int32, np.int8), []
+    monkeypatch.setattr(eo, "_packed", lambda e, pack=eo._packed: seen.append(1) or pack(e))
+    size, px = eo.event_frames_gpu(ev, dev, slices)
+    assert size == [h, w] and bool(seen) == packs
+    assert torch.equal(px, eo.clip_preprocess_gpu(eo.rasterize_gpu(eo.events_to_device(ev, dev), slices, (h, w))))
+
+
 def test_streams_that_do_not_pack_stay_on_the_general_ops(dev):
     from eventgpt_amd.ops import event_ops as eo
     good = _host_stream(50, 40, 40, np.int64, np.int8)
