@@ -44,13 +44,13 @@ void check_f32(const Tensor& t, const char* name) {
               " must be a contiguous float32 GPU tensor");
 }
 
-// a [rows, cols] bf16 matrix whose rows may be strided (a column block of a wider matrix)
-void check_rows(const Tensor& t, const char* name) {
+// a [rows, cols] bf16 matrix whose rows may be strided (a column block of a wider matrix); wide: addressed with 64 bits
+void check_rows(const Tensor& t, const char* name, bool wide = false) {
   TORCH_CHECK(t.is_cuda() && t.scalar_type() == at::kBFloat16 && t.dim() == 2, name, ": 2-D bf16 GPU tensor");
   TORCH_CHECK(t.stride(1) == 1 && t.stride(0) >= t.size(1) && t.stride(0) % 8 == 0 &&
               (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0,
               name, ": unit column stride, row stride a multiple of 8, 16-byte aligned");
-  TORCH_CHECK(t.size(0) * t.stride(0) < (1ll << 30), name, ": addressed with 32-bit byte offsets (< 2 GiB)");
+  TORCH_CHECK(wide || t.size(0) * t.stride(0) < (1ll << 30), name, ": addressed with 32-bit byte offsets (< 2 GiB)");
 }
 
 // ------------------------------------------------------------------ norms
@@ -265,7 +265,7 @@ static evgpt::LowrankSet lowrank_inputs(const std::vector<Tensor>& t, const std:
 // then masks and several adapters).
 void lowrank_add_(const std::vector<Tensor>& t, const std::vector<Tensor>& b, bool transposed, const Tensor& y, double drop_p,
                   const std::vector<int64_t>& seeds) {
-  check_rows(y, "y");
+  check_rows(y, "y", true);
   const int64_t M = y.size(0), N = y.size(1);
   evgpt::LowrankSet set = lowrank_inputs(t, seeds, M, "lowrank_add_");
   const int64_t R = t[0].size(-1);
@@ -277,7 +277,7 @@ void lowrank_add_(const std::vector<Tensor>& t, const std::vector<Tensor>& b, bo
     TORCH_CHECK(b[i].dim() == 2 && b[i].size(0) == (transposed ? R : N) && b[i].size(1) == (transposed ? N : R), "lowrank_add_: b");
     set.b[i] = bptr(b[i]);
   }
-  TORCH_CHECK((M + 63) / 64 <= 65535, "lowrank_add_: too many rows");
+  TORCH_CHECK(M < (1ll << 30), "lowrank_add_: too many rows");
   evgpt::launch_lowrank_add(set, bptr_mut(y), (int)M, (int)N, (int)R, y.stride(0), transposed, (float)drop_p, cur_stream());
 }
 

@@ -145,8 +145,8 @@ template <int NA, bool TRANS, bool DROP>
 __global__ __launch_bounds__(256) void lowrank_add_kernel(LowrankSet set, bf16_t* __restrict__ Y, int M, int N, int R, long long ldy,
                                                           unsigned int thresh16) {
   const int lane = threadIdx.x & 63, frow = lane & 15, fq = lane >> 4;
-  const int c0 = blockIdx.x * 256 + (threadIdx.x >> 6) * 64, m0 = blockIdx.y * 64;
-  if (c0 >= N) return;
+  const int c0 = blockIdx.x * 256 + (threadIdx.x >> 6) * 64, m0 = (blockIdx.z * 65535 + blockIdx.y) * 64;
+  if (c0 >= N || m0 >= M) return;
   const u32x4_t z4 = {0u, 0u, 0u, 0u};
   const bool k_ok = fq * 8 < R;
   u32x4_t y[4][2];
@@ -226,7 +226,8 @@ __global__ __launch_bounds__(256) void lowrank_add_kernel(LowrankSet set, bf16_t
 void launch_lowrank_add(const LowrankSet& set, bf16_t* Y, int M, int N, int R, long long ldy, bool trans, float drop_p, hipStream_t st) {
   if (M <= 0) return;
   const unsigned int t16 = lowrank_thresh16(drop_p);
-  const dim3 grid((N + 255) / 256, (M + 63) / 64), block(256);
+  const int rows = (M + 63) / 64;                 // blocks of 64 rows, over two dimensions of the grid
+  const dim3 grid((N + 255) / 256, rows < 65535 ? rows : 65535, (rows + 65534) / 65535), block(256);
 #define LR_ADD(NA, TR, DR) hipLaunchKernelGGL((lowrank_add_kernel<NA, TR, DR>), grid, block, 0, st, set, Y, M, N, R, ldy, t16)
 #define LR_ADD_N(TR, DR)                          \
   if (set.n == 1) LR_ADD(1, TR, DR);              \

@@ -491,6 +491,24 @@ def test_rank_r_update_and_weight_gradient_at_their_edges(dev, M, C, R, n, p):
     assert all(torch.equal(o.t(), ot) for o, ot in zip(out, out_t))
 
 
+@pytest.mark.parametrize("M,N,p", [(65535 * 64 + 5, 8, 0.0), (65535 * 64 + 5, 8, 0.1), (70_000, 16384, 0.1)])
+def test_rank_r_update_of_very_many_rows(dev, M, N, p):
+    """More blocks of rows than one dimension of a grid has, and rows past 2 GiB: every row as a short update gives it."""
+    from eventgpt_amd.ops import hip
+    raw = hip.raw
+    t, a = _rand(M, 8, dev=dev), _rand(8, N, dev=dev, seed=1)
+    y = torch.zeros(M, N, dtype=torch.bfloat16, device=dev)
+    raw.lowrank_add_([t], [a], True, y, p, [7])
+    full = torch.zeros_like(y)
+    for r in range(0, M, 1 << 16):
+        full[r:r + (1 << 16)] = (t[r:r + (1 << 16)].float() @ a.float()).bfloat16()
+    keep = raw.lowrank_mask(torch.ones_like(y), p, 7) if p > 0 else torch.ones_like(y)
+    for r in range(0, M, 1 << 16):
+        d = (y[r:r + (1 << 16)].float() - full[r:r + (1 << 16)].float() * keep[r:r + (1 << 16)].float()).abs()
+        # (two roundings to bfloat16 of sums that differ in their order: one step of 2^-7 of a value, products of 8 around 1)
+        assert bool((d <= 2 ** -7 * full[r:r + (1 << 16)].float().abs() + 1e-5).all())
+
+
 @pytest.mark.parametrize("p,single", [(0.0, False), (0.1, False), (0.1, True), (0.0, True)])
 def test_lora_projection_node_against_fp32(dev, p, single):
     """Frozen projection + low-rank adapters on column ranges as one autograd node: output, input gradient,
