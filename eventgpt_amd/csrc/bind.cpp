@@ -295,8 +295,10 @@ void lowrank_wgrad_(const Tensor& g, const std::vector<Tensor>& t, const std::ve
                 out[i].size(0) == (transposed ? C : R) && out[i].size(1) == (transposed ? R : C), "lowrank_wgrad_: out");
     set.out[i] = reinterpret_cast<evgpt::bf16_t*>(out[i].data_ptr());
   }
-  Tensor part = at::empty({evgpt::lowrank_wgrad_slabs((int)M, (int)C), set.n, R, C}, g.options().dtype(at::kFloat));
-  evgpt::launch_lowrank_wgrad(bptr(g), set, part.data_ptr<float>(), (int)M, (int)C, (int)R, g.stride(0), transposed, (float)drop_p,
+  const int slabs = evgpt::lowrank_wgrad_slabs((int)M, (int)C);
+  Tensor part;
+  if (slabs > 1) part = at::empty({slabs, set.n, R, C}, g.options().dtype(at::kFloat));
+  evgpt::launch_lowrank_wgrad(bptr(g), set, slabs > 1 ? part.data_ptr<float>() : nullptr, (int)M, (int)C, (int)R, g.stride(0), transposed, (float)drop_p,
                               cur_stream());
 }
 

@@ -189,7 +189,7 @@ struct LowrankSet { const bf16_t* t[3]; const bf16_t* b[3]; bf16_t* out[3]; unsi
 void launch_lowrank_out(const bf16_t* A, const LowrankSet& set, int M, int R, int K, long long lda, float alpha, float drop_p,
                         hipStream_t st);
 void launch_lowrank_add(const LowrankSet& set, bf16_t* Y, int M, int N, int R, long long ldy, bool trans, float drop_p, hipStream_t st);
-int lowrank_wgrad_slabs(int M, int C);      // fp32 slabs [n, R, C] the call below wants in `part`
+int lowrank_wgrad_slabs(int M, int C);      // fp32 slabs [n, R, C] the call below wants in `part` if there are several
 void launch_lowrank_wgrad(const bf16_t* G, const LowrankSet& set, float* part, int M, int C, int R, long long ldg, bool transposed,
                           float drop_p, hipStream_t st);
 void launch_lowrank_mask(const bf16_t* x, bf16_t* y, long long n, float drop_p, unsigned long long seed, bool add,

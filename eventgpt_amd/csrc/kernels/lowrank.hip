@@ -248,12 +248,14 @@ void launch_lowrank_add(const LowrankSet& set, bf16_t* Y, int M, int N, int R, l
 // v_perm, column j of every lane's patch then being the operand of the j-th MFMA -- no trip of G through LDS.  T, a
 // thousandth of G, is turned through LDS once per block.  Rows are split over blocks into fp32 slabs [R, C] (about 512
 // blocks), which lowrank_wgrad_sum_kernel adds.  As a K-strided GEMM with a 16-wide tile side: 79 us at M = 6 688,
-// C = 4 096 (55 MB); here 14.6 and 5.0 for the slabs' sum, 21.6 for three adapters in one pass.
+// C = 4 096 (55 MB); here 14.6 and 5.0 for the slabs' sum, 21.6 for three adapters in one pass.  Up to LW_ROWS rows are one
+// slab, which the block writes as the result: one launch and no partials, as the GEMM had there (launch-bound).
 constexpr int LW_ROWS = 256;     // rows of T staged at a time
 
 template <int NA, bool DROP>
 __global__ __launch_bounds__(256) void lowrank_wgrad_kernel(const bf16_t* __restrict__ G, LowrankSet set, float* __restrict__ part, int M,
-                                                            int C, int R, long long ldg, int rows_per_block, unsigned int thresh16) {
+                                                            int C, int R, long long ldg, int rows_per_block, unsigned int thresh16,
+                                                            int transposed) {
   __shared__ __attribute__((aligned(16))) bf16_t tt[NA][16][LW_ROWS + 8];
   const int tid = threadIdx.x, lane = tid & 63, frow = lane & 15, fq = lane >> 4;
   const int c = (blockIdx.x * 4 + (tid >> 6)) * 128 + frow * 8;
@@ -315,6 +317,12 @@ __global__ __launch_bounds__(256) void lowrank_wgrad_kernel(const bf16_t* __rest
     for (int e = 0; e < 4; ++e) {
       const int r = 4 * fq + e;
       if (r >= R) continue;
+      if (gridDim.y == 1) {                      // one slab: there is nothing to add
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          set.out[a][transposed ? static_cast<size_t>(c + j) * R + r : static_cast<size_t>(r) * C + c + j] = f32_to_bf16(acc[a][j][e]);
+        continue;
+      }
       float* dst = part + ((static_cast<size_t>(blockIdx.y) * NA + a) * R + r) * C + c;
       *reinterpret_cast<f32x4_t*>(dst) = f32x4_t{acc[a][0][e], acc[a][1][e], acc[a][2][e], acc[a][3][e]};
       *reinterpret_cast<f32x4_t*>(dst + 4) = f32x4_t{acc[a][4][e], acc[a][5][e], acc[a][6][e], acc[a][7][e]};
@@ -350,13 +358,14 @@ void launch_lowrank_wgrad(const bf16_t* G, const LowrankSet& set, float* part, i
   const int slabs = lowrank_wgrad_slabs(M, C), rows = ((M + slabs - 1) / slabs + 31) / 32 * 32;
   const dim3 grid((C + 511) / 512, slabs), block(256);
 #define LR_WG(NA)                                                                                                                \
-  if (t16) hipLaunchKernelGGL((lowrank_wgrad_kernel<NA, true>), grid, block, 0, st, G, set, part, M, C, R, ldg, rows, t16);      \
-  else hipLaunchKernelGGL((lowrank_wgrad_kernel<NA, false>), grid, block, 0, st, G, set, part, M, C, R, ldg, rows, 0u)
+  if (t16) hipLaunchKernelGGL((lowrank_wgrad_kernel<NA, true>), grid, block, 0, st, G, set, part, M, C, R, ldg, rows, t16, transposed);      \
+  else hipLaunchKernelGGL((lowrank_wgrad_kernel<NA, false>), grid, block, 0, st, G, set, part, M, C, R, ldg, rows, 0u, transposed)
   if (set.n == 1) { LR_WG(1); }
   else if (set.n == 2) { LR_WG(2); }
   else { LR_WG(3); }
 #undef LR_WG
-  hipLaunchKernelGGL(lowrank_wgrad_sum_kernel, dim3((set.n * R * C / 4 + 255) / 256), block, 0, st, part, set, slabs, C, R, transposed);
+  if (slabs > 1)
+    hipLaunchKernelGGL(lowrank_wgrad_sum_kernel, dim3((set.n * R * C / 4 + 255) / 256), block, 0, st, part, set, slabs, C, R, transposed);
 }
 
 // y = m (.) x  (ADD = false)  or  y += m (.) x  (ADD = true) over contiguous [rows][K] tensors, m the keep mask

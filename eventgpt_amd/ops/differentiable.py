@@ -571,6 +571,9 @@ def _lora_projection_forward(x, weight, residual, scale, drop_p, offsets, ab):
     seeds = [next_seed() if drop_p > 0 else 0 for _ in offsets]
     ts = []
     for group in _adapter_groups(ab):                                    # one pass over x for adapters of one rank
+        if len(group) == 1:
+            ts.append(raw.lowrank_out(x2, ab[2 * group[0]], scale, drop_p, seeds[group[0]]))
+            continue
         ts += raw.lowrank_out_set(x2, [ab[2 * i] for i in group], scale, drop_p, [seeds[i] for i in group])
     for off, t, b in zip(offsets, ts, ab[1::2]):                         # t [M, r], scale / (1 - p) applied
         raw.lowrank_add_([t], [b], False, y2[:, off:off + b.shape[0]], 0.0, [])
