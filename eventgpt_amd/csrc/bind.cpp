@@ -211,7 +211,7 @@ Tensor linear_t(const Tensor& a, const Tensor& w, bool a_t, bool w_t, const c10:
 
 // t [.., R] = alpha * x [.., K] · w [R, K]^T for a low-rank adapter's R <= 16 rows: one launch, no split-K pass.
 // x: contiguous, or 2-D with strided rows.  drop_p > 0: x is masked while it is loaded (keep mask of
-// (seed, element index), 1 / (1 - p) folded into alpha); lowrank_mask reproduces m (.) x for the backward.
+// (seed, element index), 1 / (1 - p) folded into alpha); the backward's kernels apply the same mask from the seed.
 // Several adapters that read the same x: one pass over it.
 std::vector<Tensor> lowrank_out_set(const Tensor& x, const std::vector<Tensor>& w, double alpha, double drop_p,
                                     const std::vector<int64_t>& seeds) {
@@ -302,34 +302,14 @@ void lowrank_wgrad_(const Tensor& g, const std::vector<Tensor>& t, const std::ve
                               cur_stream());
 }
 
-// m (.) x with lowrank_out's keep mask (no rescaling); contiguous, a multiple of 8 elements
+// m (.) x with the keep mask that the kernels above apply while loading (no rescaling), for checking them; contiguous, a
+// multiple of 8 elements
 Tensor lowrank_mask(const Tensor& x, double drop_p, int64_t seed) {
   check_bf16(x, "x");
   TORCH_CHECK(x.numel() % 8 == 0 && drop_p >= 0 && drop_p < 1, "lowrank_mask: a multiple of 8 elements");
   Tensor y = at::empty_like(x);
-  evgpt::launch_lowrank_mask(bptr(x), bptr_mut(y), x.numel(), (float)drop_p, (unsigned long long)seed, false, cur_stream());
+  evgpt::launch_lowrank_mask(bptr(x), bptr_mut(y), x.numel(), (float)drop_p, (unsigned long long)seed, cur_stream());
   return y;
-}
-// acc += m (.) x in place
-void lowrank_mask_add_(const Tensor& acc, const Tensor& x, double drop_p, int64_t seed) {
-  check_bf16(x, "x"); check_bf16(acc, "acc");
-  TORCH_CHECK(x.numel() % 8 == 0 && acc.numel() == x.numel() && drop_p >= 0 && drop_p < 1, "lowrank_mask_add_: shapes");
-  evgpt::launch_lowrank_mask(bptr(x), bptr_mut(acc), x.numel(), (float)drop_p, (unsigned long long)seed, true, cur_stream());
-}
-
-// out [M, N] (rows may be strided: a column block of a wider matrix) = x [M, K] · w [N, K]^T (+ out when
-// accumulate); x's rows may be strided too.  The low-rank update written straight onto its columns of a
-// grouped projection.
-void linear_rows_(const Tensor& x, const Tensor& w, const Tensor& out, bool accumulate) {
-  check_rows(x, "x"); check_rows(out, "out"); check_bf16(w, "weight");
-  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
-  TORCH_CHECK(w.dim() == 2 && w.size(1) == K && K % 8 == 0 && out.size(0) == M && out.size(1) == N && N % 4 == 0 &&
-              out.stride(0) % 4 == 0, "linear_rows_: x [M, K], w [N, K], out [M, N], K % 8 == 0");
-  TORCH_CHECK(N * K < (1ll << 30), "linear_rows_: weight < 2 GiB");
-  if (M == 0) return;
-  evgpt::launch_gemm_bf16(bptr(x), bptr(w), bptr_mut(out), nullptr, nullptr, accumulate ? bptr(out) : nullptr, (int)M,
-                          (int)N, (int)K, (int)x.stride(0), (int)K, (int)out.stride(0), 0, nullptr, nullptr, nullptr, 1,
-                          cur_stream());
 }
 
 // ---- few-row projections: GEMM to fp32 split-K slabs + a fused consumer ----
@@ -1544,8 +1524,6 @@ TORCH_LIBRARY(evgpt, m) {
   m.def("lowrank_add_(Tensor[] t, Tensor[] b, bool transposed, Tensor(a!) y, float drop_p, int[] seeds) -> ()", &lowrank_add_);
   m.def("lowrank_wgrad_(Tensor g, Tensor[] t, Tensor(a!)[] out, bool transposed, float drop_p, int[] seeds) -> ()", &lowrank_wgrad_);
   m.def("lowrank_mask(Tensor x, float drop_p, int seed) -> Tensor", &lowrank_mask);
-  m.def("lowrank_mask_add_(Tensor(a!) acc, Tensor x, float drop_p, int seed) -> ()", &lowrank_mask_add_);
-  m.def("linear_rows_(Tensor x, Tensor w, Tensor(a!) out, bool accumulate) -> ()", &linear_rows_);
   m.def("linear_t(Tensor a, Tensor w, bool a_t, bool w_t, Tensor? bias, Tensor? res, int act, bool out_f32, int K, Tensor(a!)? out=None) -> Tensor", &linear_t);
   m.def("gemv_max_batch() -> int", []() -> int64_t { return evgpt::gemv_max_batch(); });
   m.def("reduce_residual_layernorm(Tensor partial, Tensor? bias, Tensor? res, Tensor? ln_w, Tensor? ln_b, float eps) -> (Tensor, Tensor)", &reduce_residual_layernorm);

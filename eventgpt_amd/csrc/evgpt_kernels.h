@@ -192,8 +192,7 @@ void launch_lowrank_add(const LowrankSet& set, bf16_t* Y, int M, int N, int R, l
 int lowrank_wgrad_slabs(int M, int C);      // fp32 slabs [n, R, C] the call below wants in `part` if there are several
 void launch_lowrank_wgrad(const bf16_t* G, const LowrankSet& set, float* part, int M, int C, int R, long long ldg, bool transposed,
                           float drop_p, hipStream_t st);
-void launch_lowrank_mask(const bf16_t* x, bf16_t* y, long long n, float drop_p, unsigned long long seed, bool add,
-                         hipStream_t st);
+void launch_lowrank_mask(const bf16_t* x, bf16_t* y, long long n, float drop_p, unsigned long long seed, hipStream_t st);
 void launch_rope_qkv(const bf16_t* packed_in, bf16_t* packed_out, bf16_t* q, bf16_t* k, bf16_t* v,
                      const long long* positions, const float* cos_tab, const float* sin_tab, long long tokens,
                      int Hq, int Hkv, int D, int max_pos, bool merge, hipStream_t st);

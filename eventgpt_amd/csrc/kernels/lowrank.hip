@@ -11,8 +11,8 @@
 // A may be a column block of a wider matrix (row stride lda), and the adapter's input dropout can be
 // applied while A is loaded (DROP): element (m, k) is zeroed unless its bit of lowrank_keep8(seed,
 // chunk (m K + k) / 8) is set -- the 1 / (1 - p) factor rides on alpha -- so the dropped copy of the
-// layer input is never written.  The backward recomputes the same mask from the seed
-// (lowrank_mask_kernel: m (.) x for the weight gradient of A, acc += m (.) g for the input gradient).
+// layer input is never written.  The backward's kernels recompute the same mask from the seed while they load x (weight
+// gradient of A) and store the input gradient.
 #include "common.h"
 #include "../evgpt_kernels.h"
 
@@ -368,31 +368,18 @@ void launch_lowrank_wgrad(const bf16_t* G, const LowrankSet& set, float* part, i
     hipLaunchKernelGGL(lowrank_wgrad_sum_kernel, dim3((set.n * R * C / 4 + 255) / 256), block, 0, st, part, set, slabs, C, R, transposed);
 }
 
-// y = m (.) x  (ADD = false)  or  y += m (.) x  (ADD = true) over contiguous [rows][K] tensors, m the keep mask
-// of lowrank_keep8 (no 1 / (1 - p) factor: the callers carry it on the rank-r intermediate)
-template <bool ADD>
-__global__ __launch_bounds__(256) void lowrank_mask_kernel(const bf16_t* __restrict__ x, bf16_t* __restrict__ y,
-                                                           long long n8, unsigned int thresh16,
-                                                           unsigned long long seed) {
-  for (long long i = blockIdx.x * 256ll + threadIdx.x; i < n8; i += gridDim.x * 256ll) {
-    u32x4_t v = lowrank_apply8(load16(x + i * 8), lowrank_keep8(seed, static_cast<unsigned long long>(i), thresh16));
-    if constexpr (ADD) {
-      const u32x4_t a = load16(y + i * 8);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        v[j] = pack_bf16x2(bf16lo(a[j]) + bf16lo(v[j]), bf16hi(a[j]) + bf16hi(v[j]));
-    }
-    *reinterpret_cast<u32x4_t*>(y + i * 8) = v;
-  }
+// y = m (.) x over contiguous [rows][K] tensors, m the keep mask of lowrank_keep8 (no 1 / (1 - p) factor), for checking the
+// kernels that apply it on the way
+__global__ __launch_bounds__(256) void lowrank_mask_kernel(const bf16_t* __restrict__ x, bf16_t* __restrict__ y, long long n8,
+                                                           unsigned int thresh16, unsigned long long seed) {
+  for (long long i = blockIdx.x * 256ll + threadIdx.x; i < n8; i += gridDim.x * 256ll)
+    *reinterpret_cast<u32x4_t*>(y + i * 8) = lowrank_apply8(load16(x + i * 8), lowrank_keep8(seed, static_cast<unsigned long long>(i), thresh16));
 }
-void launch_lowrank_mask(const bf16_t* x, bf16_t* y, long long n, float drop_p, unsigned long long seed, bool add,
-                         hipStream_t st) {
+void launch_lowrank_mask(const bf16_t* x, bf16_t* y, long long n, float drop_p, unsigned long long seed, hipStream_t st) {
   if (n <= 0) return;
   long long b = (n / 8 + 255) / 256;
   const unsigned blocks = static_cast<unsigned>(b > 8192 ? 8192 : (b < 1 ? 1 : b));
-  const unsigned int t16 = lowrank_thresh16(drop_p);
-  if (add) hipLaunchKernelGGL(lowrank_mask_kernel<true>, dim3(blocks), dim3(256), 0, st, x, y, n / 8, t16, seed);
-  else hipLaunchKernelGGL(lowrank_mask_kernel<false>, dim3(blocks), dim3(256), 0, st, x, y, n / 8, t16, seed);
+  hipLaunchKernelGGL(lowrank_mask_kernel, dim3(blocks), dim3(256), 0, st, x, y, n / 8, lowrank_thresh16(drop_p), seed);
 }
 
 }  // namespace evgpt

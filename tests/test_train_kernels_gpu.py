@@ -406,8 +406,8 @@ def test_decoder_layer_training_step_uses_only_intree_kernels(dev):
 
 
 def test_row_strided_operands_of_the_lora_products(dev):
-    """The products that read or write a column block of a wider matrix where it is: the rank-r kernel and
-    the K-strided GEMM on a row-strided gradient block, and the GEMM that accumulates onto a block in place."""
+    """The products that read a column block of a wider matrix where it is: the rank-r kernel and the K-strided GEMM on a
+    row-strided gradient block.  (The update of a block in place: the rank-r tests below.)"""
     from eventgpt_amd.ops import hip
     raw = hip.raw
     M, N, r = 300, 1024, 16
@@ -420,17 +420,6 @@ def test_row_strided_operands_of_the_lora_products(dev):
     want = raw.linear_t(blk.contiguous(), t, True, True, None, None, 0, False, 320)
     assert torch.equal(got, want)
     _close(got, blk.float().t() @ t.float(), 0.3, 2e-2)
-    bw = _rand(512, r, dev=dev, seed=3, scale=0.1)
-    y = wide.clone()
-    raw.linear_rows_(t, bw, y[:, 256:768], True)
-    ref_y = wide.float().clone()
-    ref_y[:, 256:768] += (t.float() @ bw.float().t()).bfloat16().float()
-    _close(y, ref_y, 2e-2, 1e-2)
-    assert torch.equal(y[:, :256], wide[:, :256]) and torch.equal(y[:, 768:], wide[:, 768:])
-    z = torch.zeros(M, N, dtype=torch.bfloat16, device=dev)
-    raw.linear_rows_(t, bw, z[:, 512:], False)
-    _close(z[:, 512:], t.float() @ bw.float().t(), 2e-2, 1e-2)
-    assert float(z[:, :512].abs().max()) == 0.0
 
 
 def test_lora_input_mask_statistics_and_fused_load(dev):
@@ -449,10 +438,6 @@ def test_lora_input_mask_statistics_and_fused_load(dev):
     fused = raw.lowrank_out(x, a, 2.0, p, 11)
     plain = raw.lowrank_out(raw.lowrank_mask(x, p, 11), a, 2.0 / (1 - p))
     assert torch.equal(fused, plain)
-    acc = _rand(M, K, dev=dev, seed=4)
-    want = (acc.float() + (x.float() * m1.float())).bfloat16()
-    raw.lowrank_mask_add_(acc, x, p, 11)
-    assert torch.equal(acc, want)
 
 
 @pytest.mark.parametrize("M,C,R,n,p", [(1, 8, 8, 1, 0.0), (33, 136, 16, 2, 0.1), (257, 520, 8, 3, 0.2), (64, 256, 16, 1, 0.0),
