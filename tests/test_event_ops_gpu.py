@@ -34,13 +34,14 @@ def test_voxel_and_histogram_match_numpy(dev):
 
 @pytest.mark.parametrize("n,hw,bins", [(200_000, (480, 640), 5), (70_001, (97, 130), 3), (5000, (48, 64), 7)])
 @pytest.mark.parametrize("by", ["time", "count"])
-def test_voxel_lds_bands_equal_atomic_kernel_and_numpy(dev, n, hw, bins, by):
-    """The per-band LDS histogram and the one-atomic-per-event kernel give identical counts;
-    both match the host implementation, with out-of-canvas events dropped."""
+@pytest.mark.parametrize("chunks", [0, 1, 37])
+def test_voxel_lds_bands_equal_atomic_kernel_and_numpy(dev, n, hw, bins, by, chunks):
+    """The kernel that orders events in LDS (``chunks`` 0), the per-band LDS histogram (one chunk and several) and the
+    one-atomic-per-event kernel give identical counts; all match the host implementation, with out-of-canvas events dropped."""
     from eventgpt_amd.ops import event_ops as eo
     ev = synthetic_events(n, hw[1] + 6, hw[0] + 4, seed=n % 97)      # some events fall outside the canvas
     d = eo.events_to_device(ev, dev)
-    h_lds, v_lds = eo.voxel_grid_gpu(d, bins, hw, by=by, privatised=True)
+    h_lds, v_lds = eo.voxel_grid_gpu(d, bins, hw, by=by, privatised=True, chunks=chunks)
     h_at, v_at = eo.voxel_grid_gpu(d, bins, hw, by=by, privatised=False)
     assert torch.equal(h_lds, h_at) and torch.equal(v_lds, v_at)
     inside = (ev["x"] < hw[1]) & (ev["y"] < hw[0])
@@ -54,14 +55,16 @@ def test_voxel_lds_bands_equal_atomic_kernel_and_numpy(dev, n, hw, bins, by):
         assert np.array_equal(h_lds.cpu().numpy(), want)
 
 
-def test_voxel_unsorted_stream_takes_the_atomic_kernel(dev):
+@pytest.mark.parametrize("chunks", [0, 1])
+def test_voxel_unsorted_stream(dev, chunks):
+    """Ordered in LDS, or, where index ranges are asked for (``chunks``) that it does not have, by the atomic kernel."""
     from eventgpt_amd.ops import event_ops as eo
     ev = synthetic_events(20_000, 64, 48, seed=5)
     perm = np.random.default_rng(0).permutation(20_000)
     shuffled = {k: v[perm] for k, v in ev.items()}
     d = eo.events_to_device(shuffled, dev)
     assert eo._bin_bounds(d, 5, "time", int(ev["t"].min()), int(ev["t"].max() - ev["t"].min())) is None
-    hist, _ = eo.voxel_grid_gpu(d, 5, (48, 64), privatised=True)
+    hist, _ = eo.voxel_grid_gpu(d, 5, (48, 64), privatised=True, chunks=chunks)
     assert np.array_equal(hist.cpu().numpy(), polarity_histogram(ev, 5, (48, 64)))
 
 
@@ -89,6 +92,20 @@ def test_voxel_sorting_kernels_equal_the_atomic_kernel(dev, n, hw, bins, by, ord
         h, v = eo.voxel_grid_gpu({**d, "t": d["t"].int()}, bins, hw, signed=False, by="time", privatised=True)
         h_at, v_at = eo.voxel_grid_gpu(d, bins, hw, signed=False, by="time", privatised=False)
         assert torch.equal(h, h_at) and torch.equal(v, v_at)
+
+
+@pytest.mark.parametrize("order", ["sorted", "shuffled"])
+def test_voxel_counts_over_more_chunks_than_one_pass_lists(dev, order):
+    """8 192 events a chunk, 1 024 chunks a pass of the counting kernel: its list of runs is filled twice."""
+    from eventgpt_amd.ops import event_ops as eo
+    n, hw, bins = 1024 * 8192 + 3, (97, 130), 3
+    g = torch.Generator().manual_seed(5)
+    t = torch.randint(0, 100_000, (n,), generator=g)
+    d = {"x": torch.randint(0, hw[1], (n,), generator=g, dtype=torch.int32), "y": torch.randint(0, hw[0], (n,), generator=g, dtype=torch.int32),
+         "p": torch.randint(0, 2, (n,), generator=g, dtype=torch.int32), "t": torch.sort(t).values if order == "sorted" else t}
+    d = {k: v.to(dev) for k, v in d.items()}
+    (h, v), (h_at, v_at) = (eo.voxel_grid_gpu(d, bins, hw, privatised=private) for private in (True, False))
+    assert int(h.sum()) == n and torch.equal(h, h_at) and torch.equal(v, v_at)
 
 
 @pytest.mark.parametrize("hw", [(480, 640), (120, 160), (336, 336), (400, 300)])

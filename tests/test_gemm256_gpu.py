@@ -266,10 +266,12 @@ def test_persistent_256_with_k_split_glu_and_kstrided_operands(dev, force256):
     _check(diff.linear_wgrad(gy, x2), gy.float().t() @ x2.float(), 5000)
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (65, 136, 128), (577, 4096, 1024), (700, 2056, 320), (64, 128, 1024)])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (65, 136, 128), (577, 4096, 1024), (700, 2056, 320), (64, 128, 1024),
+                                   (1154, 4096, 1024), (1155, 3080, 320), (1700, 2056, 64), (1601, 2048, 192)])
 def test_eight_waves_on_the_64_row_tile(dev, M, N, K):
-    """The 64 x 128 tile of eight waves, forced: row and column remainders, one K-tile and a contraction that is no multiple
-    of the two stages, bias, activation and residual, argmax partials; and as the rule takes it.  Repeats are equal."""
+    """The 64 x 128 tile of eight waves, forced: under 400 tiles with three stages, the last four with two; row and column
+    remainders, one K-tile and contractions that are no multiple of the stages, bias, activation and residual, argmax partials;
+    and as the rule takes it.  Repeats are equal."""
     from eventgpt_amd.ops import hip
     x, w = _rand(M, K, dev=dev), _rand(N, K, dev=dev, seed=1, scale=0.05)
     bias, res = _rand(N, dev=dev, seed=2), _rand(M, N, dev=dev, seed=3)

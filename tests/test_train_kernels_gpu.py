@@ -441,10 +441,11 @@ def test_lora_input_mask_statistics_and_fused_load(dev):
 
 
 @pytest.mark.parametrize("M,C,R,n,p", [(1, 8, 8, 1, 0.0), (33, 136, 16, 2, 0.1), (257, 520, 8, 3, 0.2), (64, 256, 16, 1, 0.0),
-                                       (1030, 4096, 16, 3, 0.0), (700, 1032, 16, 1, 0.1)])
+                                       (1030, 4096, 16, 3, 0.0), (700, 1032, 16, 1, 0.1), (600, 131072, 8, 1, 0.0), (600, 131072, 8, 2, 0.1)])
 def test_rank_r_update_and_weight_gradient_at_their_edges(dev, M, C, R, n, p):
     """``y += sum m_i (.) t_i b_i^T`` in place and ``t_i^T (m_i (.) g)``: row and column remainders, rank 8 (half of an
-    MFMA's contraction is zeros), one to three adapters, masks, row-strided operands.  fp32 sums against double: the
+    MFMA's contraction is zeros), one to three adapters, masks, row-strided operands, one slab and several, slabs of more rows
+    than are staged at a time (the last two: 320 of 256).  fp32 sums against double: the
     result's own bf16 rounding (2^-8 of it) and 1e-5 of the sum of magnitudes."""
     from eventgpt_amd.ops import hip
     raw, seeds = hip.raw, [5 + i for i in range(n)]
