@@ -1,5 +1,5 @@
 """Voxel / polarity-histogram kernels on a DSEC-size canvas (480x640, 5 bins): one global atomic
-per event vs per-band counting in LDS.  ``python benchmarks/bench_voxel.py [n_events]``."""
+per event vs events ordered by bin and band in LDS and counted there.  ``python benchmarks/bench_voxel.py [n_events]``."""
 import sys
 import time
 
@@ -35,7 +35,7 @@ def main():
             res[priv] = ((time.perf_counter() - t0) / 10 * 1e3, out)
         assert torch.equal(res[False][1][0], res[True][1][0])
         print(f"{n:.0e} {name} events, by {by}: atomic-per-event {res[False][0]:.3f} ms, ordered in LDS {res[True][0]:.3f} ms "
-              f"({n / res[True][0] / 1e6:.1f} G events/s), whole call incl. bounds + output zeroing", flush=True)
+              f"({n / res[True][0] / 1e6:.1f} G events/s), whole call (for the atomics: extent of the timestamps and zeroed outputs included)", flush=True)
 
 
 def sweep():

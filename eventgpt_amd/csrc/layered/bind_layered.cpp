@@ -269,7 +269,7 @@ void feed_rows_(const Tensor& sampled, const OptTensor& active, at::IntArrayRef 
                             active.has_value() ? active->data_ptr<int>() : nullptr, i == 0, (int)B, cur_stream());
   }
 }
-// rows of x [B, N] fp32 (row stride a multiple of four) in order
+// rows of contiguous x [B, N] fp32 in order
 Tensor take_rows(const Tensor& x, at::IntArrayRef rows) {
   check_f(x, "x");
   TORCH_CHECK(x.dim() == 2, "take_rows: x [B, N]");

@@ -59,13 +59,13 @@ void launch_glu_rows(const SrcRows& src, void* h, bool f32, int rows, int ip, in
 enum { GATE_NONE = 0, GATE_SILU_BEFORE = 1, GATE_SIGMOID_AFTER = 2 };
 void launch_group_norm_rows(const SrcRows& y, const SrcRows& gate, int gcol, int mode, const float* w, void* out, bool f32,
                             int rows, int heads, int v, int vp, int parts, int ld_out, float eps, hipStream_t st);
-// Commit of one token per sequence: the first maximum of its logits, or sampled[b] when logits is null.  `sampled`
-// receives the token either way.
-// a list of rows and a value for each, as a kernel argument
+// a list of rows and a value for each, as a kernel argument: slots that get a given token, and rows of x in order
 constexpr int ROW_LIST = 64;
 struct RowList { int n; int row[ROW_LIST]; int value[ROW_LIST]; };
 void launch_feed_rows(const RowList& r, const int* tok, int* sampled, int* active, bool clear, int B, hipStream_t st);
 void launch_take_rows(const float* x, const RowList& r, float* y, long long N, hipStream_t st);
+// Commit of one token per sequence: the first maximum of its logits, or sampled[b] when logits is null.  `sampled`
+// receives the token either way.
 void launch_commit_rows(const float* logits, long long ld_logits, int* sampled, const void* embed, bool f32, float scale, float* x, int* out_tokens,
                         int max_out, int* step, int* pos, int* done, int* cur_token, int eos, int B, int ld, int vocab,
                         const int* active, hipStream_t st);

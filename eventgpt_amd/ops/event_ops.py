@@ -7,7 +7,8 @@ with launches on device-resident event arrays:
     event_clip_frames  one packed upload -> one code a pixel -> CLIP pixels: two launches for integer host streams
     event_raster    one atomic per event (last-wins / negative-wins), all T slices
     clip_preprocess PIL-exact two-pass bicubic + crop + normalise, all T frames
-    (event_voxel    time-binned polarity histogram / signed voxel grid; LDS-privatised per band)
+    (event_voxel*   time- or count-binned polarity histogram / signed voxel grid: events ordered by bin and image band in
+                    LDS and counted there; per band, or by one atomic per event, where that does not take a stream)
 
 The resample tables are the ones ``data.clip_preprocess`` builds, so device and
 host produce bit-identical uint8 images.
