@@ -567,24 +567,35 @@ __global__ __launch_bounds__(256) void column_sum_slab_kernel(const bf16_t* __re
   }
 }
 
-// sums of [slabs][N] float32 rows; blockIdx.y picks one of two sources (the weight's and the bias's partials of a LayerNorm)
+// sums of [slabs][N] float32 rows; blockIdx.y picks one of two sources (the weight's and the bias's partials of a LayerNorm).  Bound
+// by round trips: the partials come from memory and a few columns are few blocks, so sixteen waves take every sixteenth
+// slab with CF_DEPTH of them requested before the first is added.  A LayerNorm's whole backward, 512 slabs, with sixteen waves /
+// four waves of chained trips / the library's two sums, us: 3 200 x 8 20 / 47 / 26, 3 200 x 128 20 / 47 / 42, 3 200 x 4 096 27 / 54 / 65,
+// 100 000 x 8 398 / 428 / 402.
+constexpr int CF_WAVES = 16, CF_DEPTH = 8;
+
 template <typename OUT>
-__global__ __launch_bounds__(256) void column_sum_final_kernel(const float* __restrict__ part0, const float* __restrict__ part1,
-                                                               OUT* __restrict__ out0, OUT* __restrict__ out1, int slabs, int N) {
-  __shared__ float red[4][64];
+__global__ __launch_bounds__(CF_WAVES * 64) void column_sum_final_kernel(const float* __restrict__ part0, const float* __restrict__ part1,
+                                                                         OUT* __restrict__ out0, OUT* __restrict__ out1, int slabs, int N) {
+  __shared__ float red[CF_WAVES][64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, c = blockIdx.x * 64 + lane;
   const float* part = blockIdx.y ? part1 : part0;
   OUT* out = blockIdx.y ? out1 : out0;
-  float a[4] = {0.f, 0.f, 0.f, 0.f};
+  float a[CF_DEPTH] = {};
   if (c < N)
-    for (int s = w; s < slabs; s += 16)
+    for (int s = w; s < slabs; s += CF_WAVES * CF_DEPTH) {
+      float v[CF_DEPTH];
 #pragma unroll
-      for (int d = 0; d < 4; ++d)
-        if (s + 4 * d < slabs) a[d] += part[static_cast<size_t>(s + 4 * d) * N + c];
-  red[w][lane] = (a[0] + a[1]) + (a[2] + a[3]);
+      for (int d = 0; d < CF_DEPTH; ++d) v[d] = s + CF_WAVES * d < slabs ? part[static_cast<size_t>(s + CF_WAVES * d) * N + c] : 0.f;
+#pragma unroll
+      for (int d = 0; d < CF_DEPTH; ++d) a[d] += v[d];
+    }
+  red[w][lane] = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
   __syncthreads();
   if (w == 0 && c < N) {
-    const float v = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
+    float v = 0.f;
+#pragma unroll
+    for (int i = 0; i < CF_WAVES; ++i) v += red[i][lane];
     if constexpr (sizeof(OUT) == 2) out[c] = f32_to_bf16(v);
     else out[c] = v;
   }
@@ -598,10 +609,10 @@ int column_sum_slabs(int M, int N) {
 void launch_column_sum(const bf16_t* G, float* part, bf16_t* out, int M, int N, hipStream_t st) {
   const int slabs = column_sum_slabs(M, N);
   hipLaunchKernelGGL(column_sum_slab_kernel, dim3((N + 511) / 512, slabs), dim3(256), 0, st, G, part, M, N, (M + slabs - 1) / slabs);
-  hipLaunchKernelGGL((column_sum_final_kernel<bf16_t>), dim3((N + 63) / 64, 1), dim3(256), 0, st, part, part, out, out, slabs, N);
+  hipLaunchKernelGGL((column_sum_final_kernel<bf16_t>), dim3((N + 63) / 64, 1), dim3(CF_WAVES * 64), 0, st, part, part, out, out, slabs, N);
 }
 void launch_column_sum_pair(const float* p0, const float* p1, float* out0, float* out1, int slabs, int N, hipStream_t st) {
-  hipLaunchKernelGGL((column_sum_final_kernel<float>), dim3((N + 63) / 64, 2), dim3(256), 0, st, p0, p1, out0, out1, slabs, N);
+  hipLaunchKernelGGL((column_sum_final_kernel<float>), dim3((N + 63) / 64, 2), dim3(CF_WAVES * 64), 0, st, p0, p1, out0, out1, slabs, N);
 }
 
 }  // namespace evgpt

@@ -316,3 +316,17 @@ def test_column_sum_at_its_edges(dev, m, n):
     g[m // 2, n - 1] = float("inf")
     got = hip.raw.column_sum(g.to(dev)).cpu()
     assert got[-1] == float("inf") and bool(torch.isfinite(got[:-1]).all())
+
+
+@pytest.mark.parametrize("rows,H", [(1, 8), (60, 72), (64, 8), (65, 136), (508, 64), (513, 1000), (2049, 8)])
+def test_layernorm_parameter_gradients_of_few_columns(dev, rows, H):
+    """Partial sums of 1 to 512 blocks of rows: fewer than the waves that add them, either side of what those hold in
+    flight, columns short of a wave."""
+    from eventgpt_amd.ops import hip
+    x, g, w = _rand(rows, H, dev=dev, seed=1), _rand(rows, H, dev=dev, seed=2), _rand(H, dev=dev, seed=3)
+    _, dw, db = hip.raw.layernorm_bwd(x, w, g, 1e-5)
+    xd, gd = x.double(), g.double()
+    xh = (xd - xd.mean(1, keepdim=True)) / torch.sqrt(xd.var(1, unbiased=False, keepdim=True) + 1e-5)
+    # float32 chains of at most the row count, and of the eight or fewer operations that make a row's term
+    for got, term in ((dw, gd * xh), (db, gd)):
+        assert bool(((got.double() - term.sum(0)).abs() <= (rows + H + 8) * 2.0 ** -23 * (term.abs().sum(0) + gd.abs().sum(0))).all())
