@@ -302,6 +302,19 @@ void lowrank_wgrad_(const Tensor& g, const std::vector<Tensor>& t, const std::ve
                               cur_stream());
 }
 
+// One adapter of its own: no lists to unpack, and the gradient is made here unless there is a place for it (a node of one
+// adapter over few rows is bound by the host: forward and backward of 1 to 100 rows 162-168 us, 169-192 by the calls above).
+void lowrank_add_one_(const Tensor& t, const Tensor& b, bool transposed, const Tensor& y, double drop_p, int64_t seed) {
+  lowrank_add_({t}, {b}, transposed, y, drop_p, {seed});
+}
+Tensor lowrank_wgrad(const Tensor& g, const Tensor& t, bool transposed, double drop_p, int64_t seed, const c10::optional<Tensor>& out) {
+  TORCH_CHECK(g.dim() == 2 && t.dim() == 2, "lowrank_wgrad: g [M, C], t [M, R]");
+  Tensor d = out.has_value() ? *out
+                             : transposed ? at::empty({g.size(1), t.size(1)}, g.options()) : at::empty({t.size(1), g.size(1)}, g.options());
+  lowrank_wgrad_(g, {t}, {d}, transposed, drop_p, {seed});
+  return d;
+}
+
 // m (.) x with the keep mask that the kernels above apply while loading (no rescaling), for checking them; contiguous, a
 // multiple of 8 elements
 Tensor lowrank_mask(const Tensor& x, double drop_p, int64_t seed) {
@@ -1523,6 +1536,8 @@ TORCH_LIBRARY(evgpt, m) {
   m.def("lowrank_out_set(Tensor x, Tensor[] w, float alpha, float drop_p, int[] seeds) -> Tensor[]", &lowrank_out_set);
   m.def("lowrank_add_(Tensor[] t, Tensor[] b, bool transposed, Tensor(a!) y, float drop_p, int[] seeds) -> ()", &lowrank_add_);
   m.def("lowrank_wgrad_(Tensor g, Tensor[] t, Tensor(a!)[] out, bool transposed, float drop_p, int[] seeds) -> ()", &lowrank_wgrad_);
+  m.def("lowrank_add_one_(Tensor t, Tensor b, bool transposed, Tensor(a!) y, float drop_p, int seed) -> ()", &lowrank_add_one_);
+  m.def("lowrank_wgrad(Tensor g, Tensor t, bool transposed, float drop_p, int seed, Tensor(a!)? out=None) -> Tensor", &lowrank_wgrad);
   m.def("lowrank_mask(Tensor x, float drop_p, int seed) -> Tensor", &lowrank_mask);
   m.def("linear_t(Tensor a, Tensor w, bool a_t, bool w_t, Tensor? bias, Tensor? res, int act, bool out_f32, int K, Tensor(a!)? out=None) -> Tensor", &linear_t);
   m.def("gemv_max_batch() -> int", []() -> int64_t { return evgpt::gemv_max_batch(); });

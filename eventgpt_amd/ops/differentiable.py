@@ -576,7 +576,7 @@ def _lora_projection_forward(x, weight, residual, scale, drop_p, offsets, ab):
             continue
         ts += raw.lowrank_out_set(x2, [ab[2 * i] for i in group], scale, drop_p, [seeds[i] for i in group])
     for off, t, b in zip(offsets, ts, ab[1::2]):                         # t [M, r], scale / (1 - p) applied
-        raw.lowrank_add_([t], [b], False, y2[:, off:off + b.shape[0]], 0.0, [])
+        raw.lowrank_add_one_(t, b, False, y2[:, off:off + b.shape[0]], 0.0, 0)
     return y, x2, ts, seeds
 
 
@@ -641,17 +641,20 @@ class _LoRAProjection(torch.autograd.Function):
             if ctx.needs_input_grad[6 + 2 * i] or dx2 is not None:
                 dts[i] = raw.lowrank_out(gi, b.detach().t().contiguous(), s_eff, 0.0, 0)  # s / (1 - p) * dY_i B_i
             if ctx.needs_input_grad[7 + 2 * i]:
-                db = _free_sink(b, gi)
-                db = grads[2 * i + 1] = torch.empty_like(b) if db is None else db.view_as(b)
-                raw.lowrank_wgrad_(gi, [t], [db], True, 0.0, [])
+                grads[2 * i + 1] = _lowrank_wgrad(b, gi, t, True)
         for group in _adapter_groups(ab):
             need = [i for i in group if ctx.needs_input_grad[6 + 2 * i]]
-            if need:
+            if len(need) == 1:
+                i = need[0]
+                grads[2 * i] = _lowrank_wgrad(ab[2 * i], x2, dts[i], False, p, seeds[i])
+            elif need:
                 for i in need:
                     da = _free_sink(ab[2 * i], g2)
                     grads[2 * i] = torch.empty_like(ab[2 * i]) if da is None else da.view_as(ab[2 * i])
                 raw.lowrank_wgrad_(x2, [dts[i] for i in need], [grads[2 * i] for i in need], False, p, [seeds[i] for i in need])
-            if dx2 is not None:
+            if dx2 is not None and len(group) == 1:
+                raw.lowrank_add_one_(dts[group[0]], ab[2 * group[0]].detach(), True, dx2, p, seeds[group[0]])
+            elif dx2 is not None:
                 raw.lowrank_add_([dts[i] for i in group], [ab[2 * i].detach() for i in group], True, dx2, p, [seeds[i] for i in group])
         dx = None if dx2 is None else dx2.view(*gy.shape[:-1], x2.shape[1])
         return (dx, None, (gy if ctx.needs_input_grad[2] else None), None, None, None, *grads)
@@ -665,6 +668,13 @@ def _free_sink(weight, g2):
         weight._grad_sink_used = True
         return sink
     return None
+
+
+def _lowrank_wgrad(weight, g, t, transposed, drop_p=0.0, seed=0):
+    """``t^T (m (.) g)`` (or its transpose) in the parameter's published gradient slot if that is still free."""
+    sink = _free_sink(weight, t)
+    dw = _raw().lowrank_wgrad(g, t, transposed, drop_p, seed, sink)
+    return dw if sink is None else dw.view_as(weight)
 
 
 def lora_projection_ok(x, weight, adapters, residual=None) -> bool:

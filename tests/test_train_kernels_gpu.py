@@ -477,6 +477,25 @@ def test_rank_r_update_and_weight_gradient_at_their_edges(dev, M, C, R, n, p):
     assert all(torch.equal(o.t(), ot) for o, ot in zip(out, out_t))
 
 
+@pytest.mark.parametrize("M,C,R,p", [(1, 8, 8, 0.0), (256, 136, 16, 0.1), (257, 520, 8, 0.1), (300, 1032, 16, 0.0)])
+def test_rank_r_calls_of_one_adapter(dev, M, C, R, p):
+    """The calls without lists are the ones with lists of one, with a place for the gradient and without."""
+    from eventgpt_amd.ops import hip
+    raw = hip.raw
+    g, t, b = _rand(M, C, dev=dev), _rand(M, R, dev=dev, seed=1), _rand(R, C, dev=dev, seed=2)
+    for transposed in (False, True):
+        want = torch.empty(*((C, R) if transposed else (R, C)), dtype=torch.bfloat16, device=dev)
+        raw.lowrank_wgrad_(g, [t], [want], transposed, p, [3])
+        place = torch.zeros_like(want)
+        assert torch.equal(raw.lowrank_wgrad(g, t, transposed, p, 3), want)
+        assert torch.equal(raw.lowrank_wgrad(g, t, transposed, p, 3, place), want) and torch.equal(place, want)
+    for args in ((b, True, p), (b.t().contiguous(), False, 0.0)):
+        y, z = g.clone(), g.clone()
+        raw.lowrank_add_([t], [args[0]], args[1], y, args[2], [3])
+        raw.lowrank_add_one_(t, args[0], args[1], z, args[2], 3)
+        assert torch.equal(y, z) and not torch.equal(y, g)
+
+
 @pytest.mark.parametrize("M,N,p", [(65535 * 64 + 5, 8, 0.0), (65535 * 64 + 5, 8, 0.1), (70_000, 16384, 0.1)])
 def test_rank_r_update_of_very_many_rows(dev, M, N, p):
     """More blocks of rows than one dimension of a grid has, and rows past 2 GiB: every row as a short update gives it."""
