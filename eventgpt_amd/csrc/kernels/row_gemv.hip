@@ -114,15 +114,19 @@ __device__ void store_latents(const LatentStore& s, int B) {
   }
 }
 
-// (every operand of the kept chunks is requested before the first sum; the two branches' sums meet behind one barrier)
-template <typename T>
+// (every operand of the kept chunks is requested before the first sum; the two branches' sums meet behind one barrier.  EARLY: the
+// weights of the last norm too.  With the accumulators of three and four rows that takes 179 registers, two blocks a CU where
+// the grid has three: a decode step of 3 / 4 streams, eight layers, 583 / 668 us at width 2048, 1124 / 1249 at 4096; with these weights
+// requested behind the merge 165 registers and 465 / 522, 929 / 1034.)
+template <typename T, bool EARLY>
 __device__ void prepare_merge(const GemvInput& in, int b, int K, T* xs, float* red, bool lead) {
   const long long o = static_cast<long long>(b) * K;
   const float* x = static_cast<const float*>(in.x) + o;
   float xk[GV_KEEP][8], ak[GV_KEEP][8], bk[GV_KEEP][8], pk[GV_KEEP][8], qk[GV_KEEP][8], wk[GV_KEEP][8];
   kept_chunks(K, [&](int k, int c) {
     load8(in.a + o + c, ak[k]); load8(in.b + o + c, bk[k]); load8(x + c, xk[k]);
-    load8(in.wa + c, pk[k]); load8(in.wb + c, qk[k]); load8(in.w + c, wk[k]);
+    load8(in.wa + c, pk[k]); load8(in.wb + c, qk[k]);
+    if constexpr (EARLY) load8(in.w + c, wk[k]);
   });
   float sa = 0.f, sb = 0.f;
   kept_chunks(K, [&](int k, int) { sa += sumsq8(ak[k]); sb += sumsq8(bk[k]); });
@@ -161,6 +165,7 @@ __device__ void prepare_merge(const GemvInput& in, int b, int K, T* xs, float* r
     merged(xk[k], ak[k], pk[k], bk[k], qk[k]);
     ss += sumsq8(xk[k]);
     if (lead) store8(in.x_out + o + c, xk[k]);
+    if constexpr (!EARLY) load8(in.w + c, wk[k]);
   });
   for (int c = (threadIdx.x + GV_KEEP * 256) * 8; c < K; c += 2048) {
     float v[8];
@@ -316,7 +321,7 @@ __global__ __launch_bounds__(256) void row_gemv_kernel(GemvCall call, int blocks
         if (p.in.kind == GV_POST) prepare_post(p.in, b, K, xb, red, blk == 0);
         else prepare_norm<T, true>(p.in, b, K, xb, red, blk == 0);
       } else if (p.in.kind == GV_NORM) prepare_norm<T, false>(p.in, b, K, xb, red, blk == 0);
-      else if (p.in.kind == GV_MERGE) prepare_merge(p.in, b, K, xb, red, blk == 0);
+      else if (p.in.kind == GV_MERGE) prepare_merge<T, (B <= 2)>(p.in, b, K, xb, red, blk == 0);
       else if (p.in.kind == GV_GROUP) prepare_group(p.in, b, K, xb, reinterpret_cast<float*>(smem + static_cast<long long>(B) * K * sizeof(T)));
       else
         for (int c = tid; c < nchunk; c += 256)
