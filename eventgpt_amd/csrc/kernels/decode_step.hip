@@ -25,31 +25,57 @@ __device__ __forceinline__ StateRows request_state(const float* S, int N, int v0
   return r;
 }
 
-// rows of S (of one head) from v0 on, vb of them, by the block's first four waves: S = decay S + add v k^T, y = S q
-template <typename Y>
+// rows of S (of one head) from v0 on, vb of them, by the block's first four waves: S = decay S + add v k^T, y = S q.
+// AHEAD: 256 columns of a row are requested while the ones before them are combined, for blocks of more than 16 rows, which have
+// several such groups a wave and nothing else to hide their loads.  32 streams of 6 heads of 256 x 512 beside 16 attention heads:
+// 46 us with a plain loop, 59 with only the first group requested early, 55 with the loads of a group together; a decode
+// step there 685, 723, 709 and 686 us this way, of 64 streams, 8 heads of 512 x 256, eight layers, 2 853, 2 770, 2 763 and 2 724.
+// Blocks of 16 rows do without its registers (80 and six blocks a CU, 64 and eight without; 16 streams of those
+// 6 heads 575 us a step with it, 552 without, 564 with the plain loop).
+template <bool AHEAD, typename Y>
 __device__ __forceinline__ void stream_state(float* __restrict__ S, int N, int v0, int vb, bool fresh, float decay,
                                              const float* qs, const float* ks, const float* avs, const StateRows& first, Y&& put) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, l16 = lane & 15, rg = lane >> 4;
   if (wid >= 4) return;
+  const auto request = [&](f32x4_t (&v)[STATE_PRE], int i, int e0) {
+#pragma unroll
+    for (int u = 0; u < STATE_PRE; ++u) v[u] = load4(S + static_cast<long long>(v0 + i) * N + min(e0 + l16 * 4 + u * 64, N - 4));
+  };
+  f32x4_t old[STATE_PRE], next[STATE_PRE];
+  if constexpr (AHEAD) {
+#pragma unroll
+    for (int u = 0; u < STATE_PRE; ++u) old[u] = first.v[u];
+  }
   for (int i = wid * 4 + rg; i < vb; i += 16) {
     float* Sr = S + static_cast<long long>(v0 + i) * N;
     const float av = avs[i];
     float y = 0.f;
-    const auto step = [&](int e, f32x4_t old) {
-      const f32x4_t kk = *reinterpret_cast<const f32x4_t*>(ks + e), qq = *reinterpret_cast<const f32x4_t*>(qs + e);
-      f32x4_t s = kk * av;
-      if (!fresh) s += old * decay;
-      *reinterpret_cast<f32x4_t*>(Sr + e) = s;
+    for (int e0 = 0; e0 < N; e0 += STATE_PRE * 64) {
+      if constexpr (AHEAD) {
+        if (e0 + STATE_PRE * 64 < N) request(next, i, e0 + STATE_PRE * 64);
+        else if (i + 16 < vb) request(next, i + 16, 0);
+      } else if (e0 == 0) {                        // (sixteen rows: the one a lane requested at the start)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) y += s[j] * qq[j];
-    };
-    f32x4_t old[STATE_PRE];
+        for (int u = 0; u < STATE_PRE; ++u) old[u] = first.v[u];
+      } else {
+        request(old, i, e0);
+      }
 #pragma unroll
-    for (int u = 0; u < STATE_PRE; ++u) old[u] = i < 16 ? first.v[u] : load4(Sr + min(l16 * 4 + u * 64, N - 4));
+      for (int u = 0; u < STATE_PRE; ++u) {
+        const int e = e0 + l16 * 4 + u * 64;
+        if (e >= N) continue;
+        const f32x4_t kk = *reinterpret_cast<const f32x4_t*>(ks + e), qq = *reinterpret_cast<const f32x4_t*>(qs + e);
+        f32x4_t s = kk * av;
+        if (!fresh) s += old[u] * decay;
+        *reinterpret_cast<f32x4_t*>(Sr + e) = s;
 #pragma unroll
-    for (int u = 0; u < STATE_PRE; ++u)
-      if (l16 * 4 + u * 64 < N) step(l16 * 4 + u * 64, old[u]);
-    for (int e = l16 * 4 + STATE_PRE * 64; e < N; e += 64) step(e, load4(Sr + e));
+        for (int j = 0; j < 4; ++j) y += s[j] * qq[j];
+      }
+      if constexpr (AHEAD) {
+#pragma unroll
+        for (int u = 0; u < STATE_PRE; ++u) old[u] = next[u];
+      }
+    }
     y = group_sum<16>(y);
     if (l16 == 0) put(i, y);
   }
@@ -95,7 +121,7 @@ __device__ void head_step(const AttnPrepArgs& a, int b, int head, int p, bool li
   }
 }
 
-template <typename T>
+template <typename T, bool AHEAD>
 __global__ __launch_bounds__(256) void parallel_step_kernel(StepHeads sh, StepMemory m, const int* __restrict__ pos,
                                                             const int* __restrict__ live, int vb) {
   extern __shared__ __attribute__((aligned(16))) float lds[];      // [N] query, [N] key, [vb] weighted values
@@ -144,11 +170,11 @@ __global__ __launch_bounds__(256) void parallel_step_kernel(StepHeads sh, StepMe
   if (v0 == 0 && threadIdx.x == 0) m.m[to] = m1;
   const float inv = 1.f / (fmaxf(fabsf(dot), expf(-m1)) + 1e-6f);
   float* out = m.out + static_cast<long long>(gi) * m.V + v0;
-  stream_state(S, m.N, v0, vb, fresh, decay, qs, ks, avs, rows, [&](int i, float y) { out[i] = y * inv; });
+  stream_state<AHEAD>(S, m.N, v0, vb, fresh, decay, qs, ks, avs, rows, [&](int i, float y) { out[i] = y * inv; });
 }
 
 // threads: one per convolution channel of the block where that is at most 512 (the state takes four waves)
-template <typename T>
+template <typename T, bool AHEAD>
 __global__ __launch_bounds__(512) void ssd_step_kernel(StepSsd a, const int* __restrict__ pos, const int* __restrict__ live,
                                                        int vb) {
   extern __shared__ __attribute__((aligned(16))) float lds[];      // [N] C, [N] B, [vb] weighted x, [vb] x, [vb] silu(z)
@@ -211,7 +237,7 @@ __global__ __launch_bounds__(512) void ssd_step_kernel(StepSsd a, const int* __r
   }
   __syncthreads();
   const float skip = a.skip[h];
-  stream_state(S, a.N, v0, vb, fresh, decay, cs, bs, avs, rows, [&](int i, float y) { out[i] = (y + skip * xs[i]) * zs[i]; });
+  stream_state<AHEAD>(S, a.N, v0, vb, fresh, decay, cs, bs, avs, rows, [&](int i, float y) { out[i] = (y + skip * xs[i]) * zs[i]; });
 }
 
 // state rows per block: sixteen keep a single stream's launch wide, more amortise the head's small vectors
@@ -226,16 +252,18 @@ void launch_parallel_step(const StepHeads& h, const StepMemory& m, const int* po
   const int vb = rows_per_block(m.H, m.V, B);
   const dim3 grid((h.on ? h.a.Hq + h.a.Hkv : 0) + m.H * (m.V / vb), B);
   const size_t lds = (2 * m.N + vb) * 4;
-  if (f32) hipLaunchKernelGGL(parallel_step_kernel<float>, grid, dim3(256), lds, st, h, m, pos, live, vb);
-  else hipLaunchKernelGGL(parallel_step_kernel<bf16_t>, grid, dim3(256), lds, st, h, m, pos, live, vb);
+  const auto kernel = vb > 16 ? (f32 ? &parallel_step_kernel<float, true> : &parallel_step_kernel<bf16_t, true>)
+                              : (f32 ? &parallel_step_kernel<float, false> : &parallel_step_kernel<bf16_t, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(256), lds, st, h, m, pos, live, vb);
 }
 void launch_ssd_step(const StepSsd& a, const int* pos, const int* live, bool f32, int B, hipStream_t st) {
   const int vb = rows_per_block(a.H, a.V, B);
   const dim3 grid(a.V / vb, a.H, B);
   const size_t lds = (2 * a.N + 3 * vb) * 4;
   const int threads = min(512, max(256, (2 * a.N + vb + 63) / 64 * 64));
-  if (f32) hipLaunchKernelGGL(ssd_step_kernel<float>, grid, dim3(threads), lds, st, a, pos, live, vb);
-  else hipLaunchKernelGGL(ssd_step_kernel<bf16_t>, grid, dim3(threads), lds, st, a, pos, live, vb);
+  const auto kernel = vb > 16 ? (f32 ? &ssd_step_kernel<float, true> : &ssd_step_kernel<bf16_t, true>)
+                              : (f32 ? &ssd_step_kernel<float, false> : &ssd_step_kernel<bf16_t, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, st, a, pos, live, vb);
 }
 
 }  // namespace evgpt

@@ -458,6 +458,46 @@ def test_ssd_step_of_four_taps_is_the_general_one(raw, dev, H, G, Nn, V, B):
     assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
 
 
+@pytest.mark.parametrize("H,Nn,V,B", [(6, 512, 256, 32), (6, 800, 256, 64), (16, 32, 128, 40), (12, 288, 192, 40), (64, 256, 64, 64)])
+def test_steps_of_many_sequences_are_the_ones_of_each(raw, dev, H, Nn, V, B):
+    """Blocks of 32 and 64 state rows against the blocks of 16 that a single sequence has: less than a group of 256 state
+    columns, exactly one, several, remainders; sequences that are parked; three steps on stale state."""
+    f = dict(dtype=torch.float32, device=dev)
+    g = torch.Generator().manual_seed(Nn)
+    pos = torch.tensor([b % 3 for b in range(B)], dtype=torch.int32, device=dev)
+    live = torch.tensor([int(b % 7 != 3) for b in range(B)], dtype=torch.int32, device=dev)
+
+    def close(a, b):                    # sums of Nn float32 products, in one order
+        assert bool(((a - b).abs() <= Nn * 2.0 ** -23 * b.abs().max()).all())
+    inner, C = H * V, H * V + 2 * Nn
+    conv, bias, dt_bias, a_log, skip = (rnd(*s, seed=i).float().to(dev) for i, s in enumerate([(C, 4), (C,), (H,), (H,), (H,)]))
+    S, ring = torch.randn(B, H, V, Nn, generator=g).to(dev), torch.randn(B, 4, C, generator=g).to(torch.bfloat16).to(dev)
+    one = [(S[b:b + 1].clone(), ring[b:b + 1].clone()) for b in range(B)]
+    for t in range(3):
+        rows = torch.randn(B, inner + C + H + (-H) % 8, generator=g).to(dev)
+        o = raw.ssd_step_(rows, [0, inner, inner + C, H, 1, Nn, V], conv, bias, ring, dt_bias, a_log, skip, S, pos + t, live)
+        for b, (s1, r1) in enumerate(one):
+            close(o[b:b + 1].float(), raw.ssd_step_(rows[b:b + 1], [0, inner, inner + C, H, 1, Nn, V], conv, bias, r1, dt_bias, a_log, skip, s1,
+                                                    pos[b:b + 1] + t, live[b:b + 1]).float())
+    close(S, torch.cat([s1 for s1, _ in one]))
+    D, at = 64, 3 * 64                  # one attention head beside the memories
+    m_dims = [at, at + H * Nn, at + 2 * H * Nn, at + 2 * H * Nn + H * V, at + 2 * H * Nn + H * V + H, H, Nn, V]
+    S, n = torch.randn(B, H, V, Nn, generator=g).to(dev), torch.randn(2, B, H, Nn, generator=g).to(dev)
+    m, cache = torch.randn(2, B, H, generator=g).to(dev), torch.zeros(2, B, 1, 8, D, dtype=torch.bfloat16, device=dev)
+    one = [(cache[:, b:b + 1].clone(), S[b:b + 1].clone(), n[:, b:b + 1].clone(), m[:, b:b + 1].clone()) for b in range(B)]
+    ones, trig, ib = torch.ones(D, **f), torch.ones(16, 4, **f), rnd(H, seed=6).float().to(dev)
+
+    def step(rows, cache, S, n, m, pos, live):
+        return raw.parallel_step_(rows, [0, D, 2 * D, 1, 1, D, D, D], ones, ones, 1e-3, trig, trig, cache[0], cache[1], m_dims, ib, ib, 5.0,
+                                  0.4, S, n, m, pos, live)[1].float()
+    for t in range(3):
+        rows = torch.randn(B, m_dims[4] + H + (-(m_dims[4] + H)) % 8, generator=g).to(dev)
+        o = step(rows, cache, S, n, m, pos + t, live)
+        for b, state in enumerate(one):
+            close(o[b:b + 1], step(rows[b:b + 1], *state, pos[b:b + 1] + t, live[b:b + 1]))
+    close(S, torch.cat([state[1] for state in one]))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_matrix_memory_extreme_gates(raw, dev, dtype):
     """A key written with a huge input gate long ago, forget gates at the cap: the maximum runs far from zero."""
