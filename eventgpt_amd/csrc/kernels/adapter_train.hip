@@ -533,8 +533,8 @@ void launch_layernorm_bwd(const bf16_t* x, const bf16_t* w, const bf16_t* g, bf1
 // ----------------------------------------------------------------------------- column sums (bias gradients)
 // out[c] = sum over rows of G[r][c] in float32, without atomics: a block sums a slab of rows for 512 columns (a lane owns eight,
 // four waves take every fourth row with CS_DEPTH rows in flight), the second launch adds the slabs.  Bound by reading G once.
-// 3 200 x 4 096: 14.2 us, 42.1 as a cast to float32 and a reduction of that; 40 000 x 512: 47.6 and 56.5, x 128: 39.7 and 36.6 (half
-// the lanes and more idle), so callers keep rows shorter than 512 off it.
+// 3 200 x 4 096: 8.8 us, 34.8 as a cast to float32 and a reduction of that; 40 000 x 512 11.6 and 48.7, x 128 9.0 and 31.7 (the callers'
+// line at 512 columns is from a second launch that took 30 us more there; below it they still reduce with the library).
 constexpr int CS_DEPTH = 4;
 
 __global__ __launch_bounds__(256) void column_sum_slab_kernel(const bf16_t* __restrict__ G, float* __restrict__ part, int M, int N,

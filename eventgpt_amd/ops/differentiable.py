@@ -381,7 +381,7 @@ class _Linear(torch.autograd.Function):
             # (cleared by its ``zero_grad``), never inferred from ``.grad`` alone.
             dw = _wgrad_to_sink(weight, g2, x2)
         if ctx.has_bias and ctx.needs_input_grad[2]:
-            # (one read of the gradient where a wave's 64 chunks of 16 bytes fit a row; narrower: the library's reduction)
+            # (one read of the gradient; rows of under 512 columns, where half of a wave's lanes idle, by the library's reduction)
             db = (_raw().column_sum(g2) if g2.dtype == torch.bfloat16 and n >= 512 and n % 8 == 0 and g2.numel() and g2.data_ptr() % 16 == 0
                   else g2.float().sum(0).to(gy.dtype))
         return dx, dw, db, (gy if ctx.needs_input_grad[3] else None)
