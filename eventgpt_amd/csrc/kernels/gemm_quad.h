@@ -1,0 +1,12 @@
+// The 4-wave kernel of 256 x 256 tiles (gemm_quad.hip).
+#pragma once
+#include "gemm_common.h"
+
+namespace evgpt {
+
+// What it takes: at least two K-tiles in every split, byte offsets of a tile's rows within 31 bits, and an output it stores in whole
+// 16-byte chunks (bf16, plain or gated) or fp32 slabs.
+bool gemm_quad_serves(const GemmParams& p);
+void launch_gemm_quad(const GemmParams& p, int grid, hipStream_t st);
+
+}  // namespace evgpt

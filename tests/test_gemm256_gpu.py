@@ -314,3 +314,25 @@ def test_slabs_of_about_a_round_of_tiles(dev, M, N, K, slabs):
     part = hip.raw.linear_partial(x, w)
     assert part.shape == (slabs, M, N)
     _check(part.sum(0), x.float() @ w.float().t(), K)
+
+
+@pytest.mark.parametrize("M,N,K,act", [(1, 8, 128, 0), (257, 264, 128, 2), (300, 520, 192, 1), (5000, 4104, 128, 0), (5000, 4104, 192, 2),
+                                       (9000, 2056, 320, 0)])
+def test_four_waves_on_the_256_tile(dev, force256, M, N, K, act):
+    """``gemm_quad.hip``: two and odd numbers of K-tiles, one and several output tiles a workgroup, ragged rows and columns, every
+    epilogue it has, against fp32 (``_check``'s bound: bf16 operands and outputs); the same bits from run to run."""
+    x, w = _rand(M, K, dev=dev), _rand(N, K, dev=dev, seed=1, scale=0.05)
+    bias, res = _rand(N, dev=dev, seed=2), _rand(M, N, dev=dev, seed=3)
+    lin = x.float() @ w.float().t() + bias.float()
+    want = (lin, torch.nn.functional.gelu(lin), lin * torch.sigmoid(1.702 * lin))[act].to(torch.bfloat16).float() + res.float()
+    first = force256.linear(x, w, bias, res, act, False)
+    _check(first, want, K)
+    for _ in range(3):
+        assert torch.equal(force256.linear(x, w, bias, res, act, False), first)
+    if N % 16 == 0 or act:
+        return
+    half = N // 2 // 8 * 8                                # gated: gate rows, then up rows
+    gu = x.float() @ w[:2 * half].float().t()
+    if half >= 16:
+        g, u = gu[:, :half].to(torch.bfloat16).float(), gu[:, half:].to(torch.bfloat16).float()
+        _check(force256.linear_swiglu(x, w[:2 * half].contiguous()), torch.nn.functional.silu(g) * u, K)
