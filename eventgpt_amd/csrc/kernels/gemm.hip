@@ -39,6 +39,7 @@
 #include <type_traits>
 
 #include "gemm_common.h"
+#include "gemm_grouped.h"
 #include "gemm_quad.h"
 
 namespace evgpt {
@@ -259,15 +260,6 @@ __device__ __forceinline__ void gemm_epilogue_rows(const GemmParams& p, f32x4_t 
     }
     asm volatile("" ::: "memory");
   }
-}
-
-// 16 bytes per lane from `src + voff` (range-checked against `bytes`: past it, zeros) straight
-// into LDS at `lds + 16 * lane`.  Kept out of the kernel template: the descriptor type exists
-// only in the device pass, and a template body the host pass cannot instantiate loses its
-// launch stub.
-__device__ __forceinline__ void buffer_to_lds16(const unsigned char* src, int bytes, unsigned char* lds, int voff) {
-  const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(src), 0, bytes, 0x00020000);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lptr_t)lds, 16, voff, 0, 0, 0);
 }
 
 // KT: a K-contiguous operand's rows end inside the last K-tile (GemmParams::k_cols > 0).  A template
@@ -1393,7 +1385,8 @@ void launch_gemm_grouped(const bf16_t* A, const bf16_t* W, bf16_t* C, const int*
   p.grp_start = start; p.grp_perm = perm; p.grp_top = top; p.grp_count = E;
   p.grp_wstride = static_cast<long long>(N) * K;
   const int per = rows / E;             // rows of an average group
-  if (per < 48) launch_grp<32, 128, 1, 4, 4>(p, rows, st);
+  if (gemm_grouped_few_serves(p, rows)) launch_gemm_grouped_few(p, rows, st);
+  else if (per < 48) launch_grp<32, 128, 1, 4, 4>(p, rows, st);
   else if (per < 192) launch_grp<64, 128, 2, 2, 3>(p, rows, st);
   else if (per < 768) launch_grp<128, 128, 2, 2, 2>(p, rows, st);
   else launch_256<false, false, 256, true>(p, st, rows);

@@ -82,6 +82,15 @@ template <int N> __device__ __forceinline__ void wait_vm() {
   else static_assert(N == 0, "add the literal");
 }
 
+// 16 bytes per lane from `src + voff` (range-checked against `bytes`: past it, zeros) straight
+// into LDS at `lds + 16 * lane`.  Kept out of the kernel template: the descriptor type exists
+// only in the device pass, and a template body the host pass cannot instantiate loses its
+// launch stub.
+__device__ __forceinline__ void buffer_to_lds16(const unsigned char* src, int bytes, unsigned char* lds, int voff) {
+  const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(src), 0, bytes, 0x00020000);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lptr_t)lds, 16, voff, 0, 0, 0);
+}
+
 // Tile index -> (row tile, column tile).  Consecutive tiles walk down a group of about `group_m` row tiles, then
 // move one column tile over, group after group (group_m <= 0 or few row tiles: whole columns).  The workgroups
 // of an XCD that run side by side then cover a near-square patch of the output and share its operand panels

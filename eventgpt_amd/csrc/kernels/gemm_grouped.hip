@@ -1,0 +1,153 @@
+// Grouped products (experts) of a few rows a group: a stream of the weights, as gemm_fewrow_kernel is for one matrix.
+//
+// A decode step of 32 rows gives each of 8 experts about 8 rows, and what counts is how fast the experts' matrices arrive.  The
+// 32 x 128 tile of the general kernel fetches 128 bytes of a weight row per K-tile and makes 352 workgroups of the gate / up product and
+// 128 of the down product.  Here a tile is 32 output columns: 32 gate and 32 up rows, or 32 rows whose K is divided between
+// two pairs of waves (704 and 512 workgroups), in K-tiles of 128, 256 contiguous bytes of a weight row each; rows that a group
+// does not have are neither fetched nor, past the first 16, multiplied.
+//
+// us, general tile -> this, weights from memory, 8 experts of 4096 x 5504 (two a row): gate / up 16 rows 149 -> 133, 32 rows 144 -> 132 (721 MB:
+// 5.5 TB/s), down 98 -> 73 and 94 -> 75; of 2048 x 2816: down 22.3 -> 21.1 and 22.8 -> 21.9, gate / up see the rule below.
+// Two stages: gate / up 155, down 94; four: down level.
+#include <type_traits>
+
+#include "gemm_common.h"
+
+namespace evgpt {
+
+namespace {
+
+constexpr int TK = 128, AM = 32, TN = 32, STAGES = 3;
+
+template <bool GLU>
+__global__ __launch_bounds__(256) void gemm_grouped_few_kernel(GemmParams p) {
+  constexpr int W_ROWS = GLU ? 2 * TN : TN, WI = W_ROWS / 16;      // staging instructions per wave: 4 rows x 256 bytes each
+  constexpr int A_BYTES = AM * TK * 2, STAGE = A_BYTES + W_ROWS * TK * 2;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tiles_n = p.N / TN;
+  int tile = xcd_remap(blockIdx.x, gridDim.x);
+  const int e = group_of_tile(p.grp_start, p.grp_count, AM, tiles_n, tile);
+  if (e < 0) return;
+  const int first = p.grp_start[e], all = p.grp_start[e + 1] - first;
+  const int tiles_m = (all + AM - 1) / AM;
+  const int m0 = tile % tiles_m * AM, n0 = tile / tiles_m * TN, rows = min(all - m0, AM);
+  const int nk = p.K / TK;
+
+  const int r4 = lane >> 4, slot = lane & 15;
+  auto run = [&](auto ai_c) {
+    constexpr int AI = decltype(ai_c)::value, G = WI + AI;         // 16-row blocks of x; staging instructions per wave and K-tile
+    int voff_a[AI], voff_w[WI];
+#pragma unroll
+    for (int i = 0; i < AI; ++i) {
+      const int row = (wid * AI + i) * 4 + r4, at = first + m0 + min(row, rows - 1);
+      const int src = p.grp_perm ? p.grp_perm[at] / p.grp_top : at;
+      voff_a[i] = row < rows ? (src * p.lda + ((slot ^ (row & 15)) * 8)) * 2 : 0x7fffff00;     // (past the range: zeros)
+    }
+#pragma unroll
+    for (int i = 0; i < WI; ++i) {
+      const int row = (wid * WI + i) * 4 + r4;
+      voff_w[i] = ((n0 + (row & (TN - 1)) + (row / TN) * p.glu_half) * p.ldw + ((slot ^ (row & 15)) * 8)) * 2;
+    }
+    const unsigned char* A = reinterpret_cast<const unsigned char*>(p.A);
+    const unsigned char* W = reinterpret_cast<const unsigned char*>(p.W + e * p.grp_wstride);
+    const int bytes_a = 2 * p.M * p.lda, bytes_w = 2 * (GLU ? 2 * p.glu_half : p.N) * p.ldw;
+    auto stage_w = [&](int buf, int kt) {
+#pragma unroll
+      for (int i = 0; i < WI; ++i)
+        buffer_to_lds16(W + kt * (2 * TK), bytes_w - kt * (2 * TK), smem + buf * STAGE + A_BYTES + (wid * WI + i) * 1024, voff_w[i]);
+    };
+    auto stage_a = [&](int buf, int kt) {
+#pragma unroll
+      for (int i = 0; i < AI; ++i)
+        buffer_to_lds16(A + kt * (2 * TK), bytes_a - kt * (2 * TK), smem + buf * STAGE + (wid * AI + i) * 1024, voff_a[i]);
+    };
+    f32x4_t acc[AI];
+#pragma unroll
+    for (int i = 0; i < AI; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const int frow = lane & 15, fq = lane >> 4, col = wid & 1, half = wid >> 1;
+#pragma unroll
+    for (int s = 0; s < STAGES - 1; ++s)
+      if (s < nk) {
+        stage_w(s, s);
+        stage_a(s, s);
+      }
+    int cur = 0;
+    for (int kt = 0; kt < nk; ++kt) {
+      const int ahead = min(STAGES - 2, nk - 1 - kt);              // younger K-tiles that may still be on their way
+      if (ahead <= 0) wait_vm<0>();
+      else if (ahead == 1) wait_vm<G>();
+      else wait_vm<2 * G>();
+      __builtin_amdgcn_s_barrier();
+      if (kt + STAGES - 1 < nk) {
+        int nb = cur + STAGES - 1;
+        if (nb >= STAGES) nb -= STAGES;
+        stage_w(nb, kt + STAGES - 1);
+        stage_a(nb, kt + STAGES - 1);
+      }
+      const unsigned char* a_img = smem + cur * STAGE + frow * 256;
+      const unsigned char* w_img = smem + cur * STAGE + A_BYTES + ((GLU ? half * TN : 0) + col * 16 + frow) * 256;
+#pragma unroll
+      for (int k = 0; k < (GLU ? 4 : 2); ++k) {
+        const int ks = GLU ? k : half * 2 + k, off = ((ks * 4 + fq) ^ frow) * 16;
+        const bf16x8_t wf = *reinterpret_cast<const bf16x8_t*>(w_img + off);
+#pragma unroll
+        for (int i = 0; i < AI; ++i) {
+          const bf16x8_t af = *reinterpret_cast<const bf16x8_t*>(a_img + i * 4096 + off);
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, af, acc[i], 0, 0, 0);
+        }
+      }
+      cur = cur + 1 == STAGES ? 0 : cur + 1;
+    }
+    // the second pair of waves (up rows, or the other half of K) hands its sums to the first
+    __syncthreads();
+    f32x4_t* pass = reinterpret_cast<f32x4_t*>(smem);
+    if (half) {
+#pragma unroll
+      for (int i = 0; i < AI; ++i) pass[(col * AI + i) * 64 + lane] = acc[i];
+    }
+    __syncthreads();
+    if (half) return;
+#pragma unroll
+    for (int i = 0; i < AI; ++i) {
+      const f32x4_t o = pass[(col * AI + i) * 64 + lane];
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        v[r] = GLU ? glu_gate(bf16_to_f32(f32_to_bf16(acc[i][r])), p.glu_act) * bf16_to_f32(f32_to_bf16(o[r])) : acc[i][r] + o[r];
+      if (i * 16 + frow < rows) {
+        const u32x2_t w = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+        *reinterpret_cast<u32x2_t*>(p.C + static_cast<size_t>(first + m0 + i * 16 + frow) * p.ldc + n0 + col * 16 + fq * 4) = w;
+      }
+    }
+  };
+  if (rows <= 16) run(std::integral_constant<int, 1>{});
+  else run(std::integral_constant<int, 2>{});
+}
+
+template <bool GLU>
+void launch(const GemmParams& p, int tiles, hipStream_t st) {
+  constexpr int smem = STAGES * (AM + (GLU ? 2 * TN : TN)) * TK * 2;
+  static const bool attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_grouped_few_kernel<GLU>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, smem) == hipSuccess;
+  (void)attr;
+  hipLaunchKernelGGL((gemm_grouped_few_kernel<GLU>), dim3(tiles), dim3(256), smem, st, p);
+}
+
+}  // namespace
+
+// Up to 16 rows an average group: 24 (96 rows, two experts each) down 25.4 vs 30.6 us.  The gated tiles come two to a CU, 512 a round: 704 of them
+// (2048 x 2816) are level with the 32 x 128 tile or up to 4 % behind from 16 rows on, 1376 (4096 x 5504) ahead by 9 %; with fewer than four
+// rows a group some groups are empty and they are ahead anyway (8 rows 39.7 -> 36.5, 5 rows 36.0 -> 32.6).
+bool gemm_grouped_few_serves(const GemmParams& p, int rows) {
+  if (p.K % TK || p.N % TN || p.ldc % 4 || rows > 16 * p.grp_count) return false;
+  return !p.glu_half || rows < 4 * p.grp_count || p.grp_count * (p.N / TN) > 1024;
+}
+
+void launch_gemm_grouped_few(const GemmParams& p, int rows, hipStream_t st) {
+  const int tiles = (rows / AM + p.grp_count) * (p.N / TN);       // at least as many as there can be
+  if (p.glu_half) launch<true>(p, tiles, st);
+  else launch<false>(p, tiles, st);
+}
+
+}  // namespace evgpt

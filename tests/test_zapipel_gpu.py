@@ -338,6 +338,14 @@ def test_grouped_products(raw, dev, dtype, counts, K, N):
     assert Z.rel_err(raw.moe_linear(full, w, st, None, 1, -1), grouped(fr)) < tol
 
 
+@pytest.mark.parametrize("counts,K,N", [([1, 0, 17, 33, 5, 0, 16, 32], 128, 64), ([3, 0, 1, 2], 384, 192), ([16] * 8, 2048, 8256),
+                                        ([0, 65, 0, 1], 256, 128), ([2], 640, 64)])
+def test_grouped_products_of_a_few_rows(raw, dev, counts, K, N):
+    """``gemm_grouped.hip``: groups of none, one, 16, 17, 32, 33 and 65 rows, one K-tile and more than its ring, both products.
+    Sums of K products in bf16 operands: what is stored is rounded once (2^-9), the gate's two factors before that."""
+    test_grouped_products(raw, dev, BF16, list(counts), K, N)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("E,top,K,ff,N", [(1, 1, 64, 64, 64), (5, 3, 128, 64, 192), (9, 2, 2112, 704, 2112), (70, 8, 64, 128, 64)])
 def test_experts_of_a_few_rows(raw, dev, dtype, E, top, K, ff, N):
