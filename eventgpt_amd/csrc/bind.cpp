@@ -821,14 +821,14 @@ std::tuple<Tensor, Tensor, Tensor> layernorm_bwd(const Tensor& x, const Tensor& 
 }
 
 // sum over the rows of bf16 [M, N] in float32, rounded once (bias gradients)
-Tensor column_sum(const Tensor& g) {
+Tensor column_sum(const Tensor& g, bool out_f32) {
   check_bf16(g, "g");
   TORCH_CHECK(g.dim() == 2 && g.size(0) >= 1 && g.size(0) < (1ll << 30) && g.size(1) >= 8 && g.size(1) < (1ll << 30) &&
                   g.size(1) % 8 == 0 && reinterpret_cast<uintptr_t>(g.data_ptr()) % 16 == 0,
               "column_sum: contiguous [M, N], N a multiple of 8, on 16 bytes");
   const int M = (int)g.size(0), N = (int)g.size(1);
-  Tensor part = at::empty({evgpt::column_sum_slabs(M, N), N}, g.options().dtype(at::kFloat)), out = at::empty({N}, g.options());
-  evgpt::launch_column_sum(bptr(g), part.data_ptr<float>(), bptr_mut(out), M, N, cur_stream());
+  Tensor part = at::empty({evgpt::column_sum_slabs(M, N), N}, g.options().dtype(at::kFloat)), out = at::empty({N}, g.options().dtype(out_f32 ? at::kFloat : at::kBFloat16));
+  evgpt::launch_column_sum(bptr(g), part.data_ptr<float>(), out.data_ptr(), out_f32, M, N, cur_stream());
   return out;
 }
 
@@ -1574,7 +1574,7 @@ TORCH_LIBRARY(evgpt, m) {
   m.def("gelu_bwd(Tensor x, Tensor grad) -> Tensor", &gelu_bwd);
   m.def("dropout_fwd(Tensor x, float p, int seed) -> Tensor", &dropout_fwd);
   m.def("layernorm_bwd(Tensor x, Tensor weight, Tensor grad, float eps, bool want_params=True) -> (Tensor, Tensor, Tensor)", &layernorm_bwd);
-  m.def("column_sum(Tensor g) -> Tensor", &column_sum);
+  m.def("column_sum(Tensor g, bool out_f32=False) -> Tensor", &column_sum);
   m.def("sumsq_accumulate(Tensor x, Tensor(a!) acc) -> ()", &sumsq_accumulate);
   m.def("fused_adamw(Tensor grad, Tensor(a!) master, Tensor(b!) exp_avg, Tensor(c!) exp_avg_sq, Tensor(d!) param_out, float lr, float beta1, float beta2, float eps, float weight_decay, int step, float clip, Tensor? clip_dev=None) -> ()", &fused_adamw);
   m.def("w4_dequant(Tensor packed, Tensor absmax, Tensor code, Tensor(a!)? out=None) -> Tensor", &w4_dequant);

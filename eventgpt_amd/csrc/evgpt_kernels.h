@@ -56,7 +56,8 @@ void launch_gelu_bwd(const bf16_t* x, const bf16_t* g, bf16_t* dx, long long n, 
 void launch_dropout(const bf16_t* x, bf16_t* y, long long n, float p, unsigned long long seed, hipStream_t st);
 // column sums: bf16 [M, N] (N a multiple of 8, rows on 16 bytes) with part float32 [slabs, N]; two sets of float32 [slabs, N] partials
 int column_sum_slabs(int M, int N);
-void launch_column_sum(const bf16_t* G, float* part, bf16_t* out, int M, int N, hipStream_t st);
+// out [N]: bf16 or fp32
+void launch_column_sum(const bf16_t* G, float* part, void* out, bool out_f32, int M, int N, hipStream_t st);
 void launch_column_sum_pair(const float* p0, const float* p1, float* out0, float* out1, int slabs, int N, hipStream_t st);
 int layernorm_bwd_blocks(int rows);    // rows of the [blocks][H] fp32 dw / db partial buffers
 void launch_layernorm_bwd(const bf16_t* x, const bf16_t* w, const bf16_t* g, bf16_t* dx, float* dw, float* db,

@@ -606,10 +606,17 @@ int column_sum_slabs(int M, int N) {
   const int cols = (N + 511) / 512, most = (M + 15) / 16, want = (512 + cols - 1) / cols;
   return want < most ? want : most;
 }
-void launch_column_sum(const bf16_t* G, float* part, bf16_t* out, int M, int N, hipStream_t st) {
+void launch_column_sum(const bf16_t* G, float* part, void* out, bool out_f32, int M, int N, hipStream_t st) {
   const int slabs = column_sum_slabs(M, N);
   hipLaunchKernelGGL(column_sum_slab_kernel, dim3((N + 511) / 512, slabs), dim3(256), 0, st, G, part, M, N, (M + slabs - 1) / slabs);
-  hipLaunchKernelGGL((column_sum_final_kernel<bf16_t>), dim3((N + 63) / 64, 1), dim3(CF_WAVES * 64), 0, st, part, part, out, out, slabs, N);
+  const dim3 grid((N + 63) / 64, 1), block(CF_WAVES * 64);
+  if (out_f32) {
+    float* o = static_cast<float*>(out);
+    hipLaunchKernelGGL((column_sum_final_kernel<float>), grid, block, 0, st, part, part, o, o, slabs, N);
+  } else {
+    bf16_t* o = static_cast<bf16_t*>(out);
+    hipLaunchKernelGGL((column_sum_final_kernel<bf16_t>), grid, block, 0, st, part, part, o, o, slabs, N);
+  }
 }
 void launch_column_sum_pair(const float* p0, const float* p1, float* out0, float* out1, int slabs, int N, hipStream_t st) {
   hipLaunchKernelGGL((column_sum_final_kernel<float>), dim3((N + 63) / 64, 2), dim3(CF_WAVES * 64), 0, st, p0, p1, out0, out1, slabs, N);

@@ -241,13 +241,13 @@ def linear_dgrad(gy: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     return _raw().linear_t(gy, weight, False, True, None, None, 0, False, _round64(n))
 
 
-def linear_wgrad(gy: torch.Tensor, x: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+def linear_wgrad(gy: torch.Tensor, x: torch.Tensor, out: Optional[torch.Tensor] = None, f32: bool = False) -> torch.Tensor:
     """``dW [N,K] = dY^T [N,M] @ X [M,K]``: both operands are strided in the token dimension.
-    ``out``: a contiguous bf16 ``[N,K]`` tensor the product is written into (an optimizer's
-    flat gradient buffer), instead of a new tensor."""
+    ``out``: a contiguous ``[N,K]`` tensor of the result's type the product is written into (an optimizer's
+    flat gradient buffer), instead of a new tensor.  ``f32``: the sums as they are, otherwise rounded to bf16."""
     # the contraction runs to the next multiple of 64; both operands are K-strided, whose staging
     # loads return zeros for the rows past the last token, so neither is padded
-    return _raw().linear_t(gy, x, True, True, None, None, 0, False, _round64(gy.shape[0]), out)
+    return _raw().linear_t(gy, x, True, True, None, None, 0, f32, _round64(gy.shape[0]), out)
 
 
 def enable_transposed_dgrad(module: torch.nn.Module, min_free_bytes: int = 32 << 30, group: bool = True) -> int:
@@ -333,14 +333,21 @@ def _transposed_for_dgrad(weight) -> Optional[torch.Tensor]:
     return wt
 
 
-def _wgrad_to_sink(weight, g2, x2):
-    """``dW = g2^T x2``, written into the parameter's published gradient slot if that is still free."""
+def _free_sink(weight, dtype):
+    """The parameter's published gradient slot, taken, if it is still free and of this type."""
     sink = getattr(weight, "_grad_sink", None)
     if (sink is not None and weight.grad is None and not getattr(weight, "_grad_sink_used", True)
-            and sink.dtype == g2.dtype and sink.shape == weight.shape and sink.is_contiguous()):
+            and sink.dtype == dtype and sink.shape == weight.shape and sink.is_contiguous()):
         weight._grad_sink_used = True
-        return linear_wgrad(g2, x2, out=sink).view_as(weight)
-    return linear_wgrad(g2, x2)
+        return sink
+    return None
+
+
+def _wgrad_to_sink(weight, g2, x2, f32: bool = False):
+    """``dW = g2^T x2``, written into the parameter's published gradient slot if that is still free."""
+    sink = _free_sink(weight, torch.float32 if f32 else g2.dtype)
+    dw = linear_wgrad(g2, x2, sink, f32)
+    return dw if sink is None else dw.view_as(weight)
 
 
 class _Linear(torch.autograd.Function):
@@ -385,6 +392,39 @@ class _Linear(torch.autograd.Function):
             db = (_raw().column_sum(g2) if g2.dtype == torch.bfloat16 and n >= 512 and n % 8 == 0 and g2.numel() and g2.data_ptr() % 16 == 0
                   else g2.float().sum(0).to(gy.dtype))
         return dx, dw, db, (gy if ctx.needs_input_grad[3] else None)
+
+
+class _MasterLinear(torch.autograd.Function):
+    """``y = x @ W^T + b`` of bf16 rows with fp32 parameters (training under bf16 autocast): the products take the parameters
+    rounded to bf16, and the parameters' gradients are the products' fp32 sums, not rounded on their way."""
+
+    @staticmethod
+    def forward(ctx, x, weight, bias):
+        from . import hip
+        xc = x if x.is_contiguous() else x.contiguous()
+        w = weight.detach().to(torch.bfloat16)
+        ctx.save_for_backward(xc.view(-1, x.shape[-1]), w)
+        ctx.parameter, ctx.has_bias = weight, bias is not None           # (the parameter: for its gradient slot)
+        return hip.linear(xc, w, None if bias is None else bias.detach().to(torch.bfloat16))
+
+    @staticmethod
+    def backward(ctx, gy):
+        x2, w = ctx.saved_tensors
+        n, k = w.shape
+        g2 = gy.reshape(-1, n)
+        g2 = g2 if g2.is_contiguous() else g2.contiguous()
+        dx = linear_dgrad(g2, w).view(*gy.shape[:-1], k) if ctx.needs_input_grad[0] else None
+        dw = _wgrad_to_sink(ctx.parameter, g2, x2, True) if ctx.needs_input_grad[1] else None
+        db = None
+        if ctx.has_bias and ctx.needs_input_grad[2]:
+            db = (_raw().column_sum(g2, True) if n >= 512 and n % 8 == 0 and g2.numel() and g2.data_ptr() % 16 == 0
+                  else g2.float().sum(0))
+        return dx, dw, db
+
+
+def linear_master(x, weight, bias=None):
+    """``linear`` of bf16 rows with fp32 parameters that take gradients (shapes as ``linear``'s kernels take them)."""
+    return _MasterLinear.apply(x, weight, bias)
 
 
 def _linear_fused_ok(x, weight, bias) -> bool:
@@ -649,7 +689,7 @@ class _LoRAProjection(torch.autograd.Function):
                 grads[2 * i] = _lowrank_wgrad(ab[2 * i], x2, dts[i], False, p, seeds[i])
             elif need:
                 for i in need:
-                    da = _free_sink(ab[2 * i], g2)
+                    da = _free_sink(ab[2 * i], g2.dtype)
                     grads[2 * i] = torch.empty_like(ab[2 * i]) if da is None else da.view_as(ab[2 * i])
                 raw.lowrank_wgrad_(x2, [dts[i] for i in need], [grads[2 * i] for i in need], False, p, [seeds[i] for i in need])
             if dx2 is not None and len(group) == 1:
@@ -660,19 +700,9 @@ class _LoRAProjection(torch.autograd.Function):
         return (dx, None, (gy if ctx.needs_input_grad[2] else None), None, None, None, *grads)
 
 
-def _free_sink(weight, g2):
-    """The parameter's published gradient slot if it is still free this step (marks it used), else None."""
-    sink = getattr(weight, "_grad_sink", None)
-    if (sink is not None and weight.grad is None and not getattr(weight, "_grad_sink_used", True)
-            and sink.dtype == g2.dtype and sink.shape == weight.shape and sink.is_contiguous()):
-        weight._grad_sink_used = True
-        return sink
-    return None
-
-
 def _lowrank_wgrad(weight, g, t, transposed, drop_p=0.0, seed=0):
     """``t^T (m (.) g)`` (or its transpose) in the parameter's published gradient slot if that is still free."""
-    sink = _free_sink(weight, t)
+    sink = _free_sink(weight, t.dtype)
     dw = _raw().lowrank_wgrad(g, t, transposed, drop_p, seed, sink)
     return dw if sink is None else dw.view_as(weight)
 

@@ -6,8 +6,9 @@ The hidden-state adapters (``align/adapters.py``) keep the reference's module st
 (pipeline/adapter_train/hidden_adapter.py:40-560) -- and train as fp32 parameters under bf16
 autocast.  Every ``F.linear`` of such a tree goes to the vendor GEMM library.  Inside
 ``InTreeLinear()`` the same calls run ``ops.differentiable.linear`` instead: operands are cast to
-bf16 exactly as autocast would (the casts are differentiable, so the weight gradient arrives at the
-fp32 parameter), forward / dgrad / wgrad are the MFMA GEMM of ``csrc/kernels/gemm.hip``.  Calls the
+bf16 exactly as autocast would (an fp32 parameter's gradient is the wgrad product's fp32 sums, which an
+optimizer's gradient slot takes from the kernel), forward / dgrad / wgrad are the MFMA GEMM of
+``csrc/kernels/gemm.hip``.  Calls the
 in-tree kernel does not take (CPU tensors, dimensions that are no multiple of 8, a handful of rows)
 fall through to the library untouched.
 
@@ -57,6 +58,9 @@ class InTreeLinear(TorchFunctionMode):
             if _eligible(x, w, b):
                 self.routed += 1
                 bf = torch.bfloat16
+                if (torch.is_grad_enabled() and w.dtype == torch.float32 and w.requires_grad and w.is_contiguous()
+                        and x.numel() and (b is None or b.dtype == torch.float32)):
+                    return diff.linear_master(x.to(bf), w, b)
                 return diff.linear(x.to(bf), w.to(bf), None if b is None else b.to(bf))
             self.passed += 1
         elif func is F.layer_norm:

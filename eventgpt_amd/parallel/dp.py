@@ -101,7 +101,7 @@ class ShardedAdamW:
         self.overlap = overlap and self.on_rccl
         self.comm_stream = torch.cuda.Stream() if self.on_rccl else None
         self._owner: Dict[int, _Bucket] = {}
-        # Direct gradients: a bf16 matrix on the GPU gets its slot of the flat buffer published as
+        # Direct gradients: a bf16 matrix or an fp32 parameter on the GPU gets its slot of the flat buffer published as
         # ``_grad_sink``.  The in-tree wgrad GEMM (``ops/differentiable.py``) writes a step's first
         # gradient straight into the slot and autograd adopts that view as ``.grad``: no zero fill of
         # the buffer and no read-modify-write accumulation into it (for a 7B decoder those are 13.6 GB
@@ -112,7 +112,7 @@ class ShardedAdamW:
         for b in self.buckets:
             for p, view in zip(b.params, b.grad_views):
                 self._owner[id(p)] = b
-                if direct_grads and p.is_cuda and p.dtype == torch.bfloat16 and p.dim() == 2:
+                if direct_grads and p.is_cuda and (p.dtype == torch.float32 or (p.dtype == torch.bfloat16 and p.dim() == 2)):
                     p._grad_sink = view
                     p._grad_sink_used = True   # until the first zero_grad hands the slot out
                     self._sink[id(p)] = view

@@ -330,3 +330,31 @@ def test_layernorm_parameter_gradients_of_few_columns(dev, rows, H):
     # float32 chains of at most the row count, and of the eight or fewer operations that make a row's term
     for got, term in ((dw, gd * xh), (db, gd)):
         assert bool(((got.double() - term.sum(0)).abs() <= (rows + H + 8) * 2.0 ** -23 * (term.abs().sum(0) + gd.abs().sum(0))).all())
+
+
+@pytest.mark.parametrize("rows,k,n,uses,passes", [(16, 8, 8, 1, 1), (65, 128, 520, 1, 2), (200, 512, 1024, 2, 1), (333, 1024, 512, 2, 2)])
+def test_fp32_parameters_get_the_sums_of_the_weight_gradient(dev, rows, k, n, uses, passes):
+    """Gradients of fp32 parameters of in-tree linears are fp32 sums of bf16 products, written into the optimizer's slot: used once or
+    twice in a graph, over one or two backward passes.  An fp32 sum of ``rows`` products in any order is within ``rows * 2^-24`` of the sum of
+    their absolute values; a second use or pass adds one rounding of the total."""
+    from eventgpt_amd.ops.intree_mode import InTreeLinear
+    from eventgpt_amd.parallel.dp import ShardedAdamW
+    g = torch.Generator().manual_seed(rows)
+    lin = torch.nn.Linear(k, n).to(dev)
+    xs = [torch.randn(rows, k, generator=g).to(dev) for _ in range(uses)]
+    gys = [torch.randn(rows, n, generator=g).to(dev).bfloat16() for _ in range(uses)]
+    opt = ShardedAdamW(lin.parameters(), lr=1e-3)
+    opt.zero_grad()
+    for _ in range(passes):
+        with torch.autocast("cuda", dtype=torch.bfloat16), InTreeLinear() as mode:
+            ys = [torch.nn.functional.linear(x, lin.weight, lin.bias) for x in xs]
+        assert mode.routed == uses
+        torch.autograd.backward(ys, gys)
+    opt.global_grad_norm()                                  # settles every gradient into its slot
+    want = passes * sum(gy.double().T @ x.bfloat16().double() for x, gy in zip(xs, gys))
+    size = passes * sum(gy.double().abs().T @ x.bfloat16().double().abs() for x, gy in zip(xs, gys))
+    flat = opt.buckets[0].flat_grad
+    for p, w, s in ((lin.weight, want, size), (lin.bias, passes * sum(gy.double().sum(0) for gy in gys),
+                                               passes * sum(gy.double().abs().sum(0) for gy in gys))):
+        assert p.grad.dtype == torch.float32 and flat.data_ptr() <= p.grad.data_ptr() < flat.data_ptr() + 4 * flat.numel()
+        assert bool(((p.grad.double() - w).abs() <= (rows + 4) * 2.0 ** -24 * s + 1e-30).all())
