@@ -35,7 +35,7 @@ SO_PATH = os.path.join(PKG_DIR, "_C.so")
 LAYERED_SO_PATH = os.path.join(PKG_DIR, "_D.so")
 # kernels of the layered decoders alone, and the ones they share with the rest
 LAYERED_KERNELS = ("attn_chunk", "conv1d", "decode_step", "gemm_f32", "latent", "linear_scan", "moe", "row_gemv", "rowops")
-LAYERED_SHARED = ("attn_decode", "attn_prefill", "gemm", "gemm_grouped", "gemm_quad", "sd")
+LAYERED_SHARED = ("attn_decode", "attn_prefill", "gemm", "gemm_grouped", "gemm_quad", "gemm_ring", "sd")
 ARCH = "gfx950"
 
 # -packed-fp32-ops is disabled on purpose: some packed-fp32 forms have produced

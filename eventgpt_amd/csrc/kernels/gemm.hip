@@ -39,8 +39,10 @@
 #include <type_traits>
 
 #include "gemm_common.h"
+#include "gemm_epilogue.h"
 #include "gemm_grouped.h"
 #include "gemm_quad.h"
+#include "gemm_ring.h"
 
 namespace evgpt {
 
@@ -72,132 +74,6 @@ __device__ __forceinline__ bf16x8_t frag_t(const unsigned char* tile, int cb, in
   const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4_t __attribute__((address_space(3)))*)a2);
   const s16x8_t v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
   return __builtin_bit_cast(bf16x8_t, v);
-}
-
-// Epilogue shared by the GEMM kernels: lane holds C[m][n .. n+3] of each 16x16 tile (m = row
-// lane & 15, n = 4 * (lane >> 4)); wave (wr, wc) owns the WM x WN sub-tile at (wr*WM, wc*WN).
-template <int TM, int TN, int WM, int WN, int WGN>
-__device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4_t (&acc)[TM][TN], int m0, int n0, int wr,
-                                              int wc, int tn, int tiles_n, int ksplit, int lane) {
-  const int frow = lane & 15, fq = lane >> 4;
-  if constexpr (TN % 2 == 0) {
-    if (p.glu_half) {
-      // tile columns j < TN/2 are gate, j + TN/2 the matching up columns; both factors are rounded to
-      // bf16 first (what a separate activation kernel would read back)
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const int m = m0 + wr * WM + i * 16 + frow;
-        if (m >= p.M) continue;
-#pragma unroll
-        for (int j = 0; j < TN / 2; ++j) {
-          const int n = n0 + wc * (WN / 2) + j * 16 + fq * 4;
-          if (n >= p.N) continue;
-          float v[4];
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            v[r] = glu_gate(bf16_to_f32(f32_to_bf16(acc[i][j][r])), p.glu_act) * bf16_to_f32(f32_to_bf16(acc[i][j + TN / 2][r]));
-          const size_t o = static_cast<size_t>(m) * p.ldc + n;
-          if (n + 3 < p.N && (p.ldc & 3) == 0) {
-            u32x2_t w = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-            *reinterpret_cast<u32x2_t*>(p.C + o) = w;
-          } else {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) if (n + r < p.N) p.C[o + r] = f32_to_bf16(v[r]);
-          }
-        }
-      }
-      return;
-    }
-  }
-  if (p.splitk > 1 || p.raw_partial) {
-    float* slab = p.partial + static_cast<size_t>(ksplit) * p.M * p.N;
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int m = m0 + wr * WM + i * 16 + frow;
-      if (m >= p.M) continue;
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int n = n0 + wc * WN + j * 16 + fq * 4;
-        float* dst = slab + static_cast<size_t>(m) * p.N + n;
-        if (n + 3 < p.N && (p.N & 3) == 0) {
-          *reinterpret_cast<f32x4_t*>(dst) = acc[i][j];
-        } else {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) if (n + r < p.N) dst[r] = acc[i][j][r];
-        }
-      }
-    }
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int m = m0 + wr * WM + i * 16 + frow;
-    if (p.amax_val) {
-      // row max over this wave's WN columns: in-lane over j and r, then across the
-      // 4 lanes (fq) that share the row
-      float bv = -INFINITY;
-      int bi = 0x7fffffff;
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int n = n0 + wc * WN + j * 16 + fq * 4 + r;
-          float v = acc[i][j][r];
-          if (p.bias && n < p.N) v += bf16_to_f32(p.bias[n]);
-          if (n < p.N && (v > bv || (v == bv && n < bi))) { bv = v; bi = n; }
-        }
-#pragma unroll
-      for (int off = 16; off < 64; off <<= 1) {
-        const float ov = __shfl_xor(bv, off, 64);
-        const int oi = __shfl_xor(bi, off, 64);
-        if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-      }
-      if (fq == 0 && m < p.M) {
-        const int n_part = tiles_n * WGN;
-        p.amax_val[static_cast<size_t>(m) * n_part + tn * WGN + wc] = bv;
-        p.amax_idx[static_cast<size_t>(m) * n_part + tn * WGN + wc] = bi;
-      }
-    }
-    if (m >= p.M || (!p.C && !p.Cf)) continue;
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int n = n0 + wc * WN + j * 16 + fq * 4;
-      if (n >= p.N) continue;
-      float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
-      const size_t o = static_cast<size_t>(m) * p.ldc + n;
-      const bool full = (n + 3 < p.N) && ((p.ldc & 3) == 0);
-      if (p.bias) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) if (n + r < p.N) v[r] += bf16_to_f32(p.bias[n + r]);
-      }
-      if (p.act != ACT_NONE) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = apply_act(v[r], p.act);
-      }
-      if (p.res) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (n + r < p.N) v[r] = bf16_to_f32(f32_to_bf16(v[r])) + bf16_to_f32(p.res[o + r]);
-      }
-      if (p.Cf) {
-        if (full) {
-          *reinterpret_cast<f32x4_t*>(p.Cf + o) = f32x4_t{v[0], v[1], v[2], v[3]};
-        } else {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) if (n + r < p.N) p.Cf[o + r] = v[r];
-        }
-      }
-      if (p.C) {
-        if (full) {
-          u32x2_t w = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-          *reinterpret_cast<u32x2_t*>(p.C + o) = w;
-        } else {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) if (n + r < p.N) p.C[o + r] = f32_to_bf16(v[r]);
-        }
-      }
-    }
-  }
 }
 
 // bf16 output of the 8-wave kernel through LDS.  The MFMA layout gives a lane 4 consecutive columns of 16
@@ -999,6 +875,12 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmParams p) {
   }
 }
 
+static void launch_splitk_reduce(const GemmParams& p, hipStream_t st) {
+  const long long quads = (static_cast<long long>(p.M) * p.N + 3) / 4;
+  const long long blocks = (quads + 255) / 256;
+  hipLaunchKernelGGL(splitk_reduce_kernel, dim3(static_cast<unsigned>(blocks > 2048 ? 2048 : blocks)), dim3(256), 0, st, p);
+}
+
 template <int BM, int BN, int WGM, int WGN, int STAGES, bool AT = false, bool BT = false, bool KT = false,
           bool ROPE = false>
 static void launch_cfg(const GemmParams& p, hipStream_t st) {
@@ -1268,13 +1150,16 @@ void launch_gemm_bf16(const bf16_t* A, const bf16_t* W, bf16_t* C, float* Cf, co
     // low-rank products and other short contractions; the tile choice matters little for them)
     if (M <= 32) launch_cfg<32, 64, 1, 4, 4, false, false, true>(p, st);
     else launch_cfg<64, 128, 2, 2, 3, false, false, true>(p, st);
-    if (p.splitk > 1) {
-      const long long quads = (static_cast<long long>(M) * N + 3) / 4;
-      int blocks = static_cast<int>((quads + 255) / 256);
-      if (blocks > 2048) blocks = 2048;
-      hipLaunchKernelGGL(splitk_reduce_kernel, dim3(blocks), dim3(256), 0, st, p);
-    }
+    if (p.splitk > 1) launch_splitk_reduce(p, st);
     return;
+  }
+  if (cfg != CFG_256x256 && g_forced_cfg < 0) {
+    const RingTile ring = gemm_ring_tile(p);
+    if (ring != RING_NONE) {
+      launch_gemm_ring(p, ring, st);
+      if (p.splitk > 1) launch_splitk_reduce(p, st);
+      return;
+    }
   }
   // One workgroup per CU means whole rounds of 256 tiles: a grid of 304 tiles takes as long as
   // one of 512.  When the last round would be under half full (and there are few rounds for it
@@ -1299,10 +1184,7 @@ void launch_gemm_bf16(const bf16_t* A, const bf16_t* W, bf16_t* C, float* Cf, co
         b.splitk = (K + b.k_per_split - 1) / b.k_per_split;
         b.partial = splitk_ws;
         launch_256<false, false>(b, st);
-        const long long quads = (static_cast<long long>(b.M) * b.N + 3) / 4;
-        int blocks = static_cast<int>((quads + 255) / 256);
-        if (blocks > 2048) blocks = 2048;
-        hipLaunchKernelGGL(splitk_reduce_kernel, dim3(blocks), dim3(256), 0, st, b);
+        launch_splitk_reduce(b, st);
       } else {
         launch_cfg<128, 128, 2, 2, 2>(b, st);
       }
@@ -1319,12 +1201,7 @@ void launch_gemm_bf16(const bf16_t* A, const bf16_t* W, bf16_t* C, float* Cf, co
     case CFG_128x256: launch_256<false, false, 128>(p, st); break;
     default: launch_cfg<32, 128, 1, 4, 4>(p, st); break;
   }
-  if (p.splitk > 1) {
-    const long long quads = (static_cast<long long>(M) * N + 3) / 4;
-    int blocks = static_cast<int>((quads + 255) / 256);
-    if (blocks > 2048) blocks = 2048;
-    hipLaunchKernelGGL(splitk_reduce_kernel, dim3(blocks), dim3(256), 0, st, p);
-  }
+  if (p.splitk > 1) launch_splitk_reduce(p, st);
 }
 
 // q | k | v projection of a prefill with RoPE and the cache append in the epilogue (head_dim 128): A [M][K],
@@ -1421,6 +1298,8 @@ void launch_gemm_glu(const bf16_t* A, const bf16_t* W, bf16_t* H, int M, int I, 
     }
   }
   if (g_forced_cfg == CFG_256x256 || (g_forced_cfg < 0 && use_256(M, 2 * I, K))) launch_256<false, false>(p, st);
+  else if (const RingTile ring = g_forced_cfg < 0 ? gemm_ring_tile(p) : RING_NONE; ring != RING_NONE)
+    launch_gemm_ring(p, ring, st);
   else if (g_forced_cfg == CFG_128x128 || (g_forced_cfg < 0 && tiles(128, 128) >= 384)) launch_cfg<128, 128, 2, 2, 2>(p, st);
   else if (g_forced_cfg == CFG_64x64) launch_cfg<64, 64, 2, 2, 4>(p, st);
   else launch_cfg<64, 128, 2, 2, 3>(p, st);
@@ -1469,12 +1348,7 @@ void launch_gemm_bf16_t(const bf16_t* A, const bf16_t* W, bf16_t* C, float* Cf, 
   else if (a_t) launch_t<true, false>(p, st);
   else if (w_t) launch_t<false, true>(p, st);
   else launch_t<false, false>(p, st);
-  if (p.splitk > 1) {
-    const long long quads = (static_cast<long long>(M) * N + 3) / 4;
-    int blocks = static_cast<int>((quads + 255) / 256);
-    if (blocks > 2048) blocks = 2048;
-    hipLaunchKernelGGL(splitk_reduce_kernel, dim3(blocks), dim3(256), 0, st, p);
-  }
+  if (p.splitk > 1) launch_splitk_reduce(p, st);
 }
 
 // Projection that stops at the fp32 split-K slabs partial[nslab][M][N]; returns
@@ -1514,6 +1388,13 @@ int launch_gemm_partial(const bf16_t* A, const bf16_t* W, float* partial, int M,
   g_for_slabs = true;
   const GemmCfg cfg = M > 32 ? pick_cfg(M, N, K) : pick_cfg(M, N);
   g_for_slabs = false;
+  if (cfg != CFG_256x256 && g_forced_cfg < 0) {
+    const RingTile ring = gemm_ring_tile(p);
+    if (ring != RING_NONE) {
+      launch_gemm_ring(p, ring, st);
+      return p.splitk;
+    }
+  }
   switch (cfg) {
     case CFG_128x128: launch_cfg<128, 128, 2, 2, 2>(p, st); break;
     case CFG_64x128: launch_cfg<64, 128, 2, 2, 3>(p, st); break;

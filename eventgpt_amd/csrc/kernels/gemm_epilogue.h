@@ -1,0 +1,133 @@
+// The epilogue that the GEMM kernels share.
+#pragma once
+#include "gemm_common.h"
+
+namespace evgpt {
+
+// Epilogue shared by the GEMM kernels: lane holds C[m][n .. n+3] of each 16x16 tile (m = row
+// lane & 15, n = 4 * (lane >> 4)); wave (wr, wc) owns the WM x WN sub-tile at (wr*WM, wc*WN).
+template <int TM, int TN, int WM, int WN, int WGN>
+__device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4_t (&acc)[TM][TN], int m0, int n0, int wr,
+                                              int wc, int tn, int tiles_n, int ksplit, int lane) {
+  const int frow = lane & 15, fq = lane >> 4;
+  if constexpr (TN % 2 == 0) {
+    if (p.glu_half) {
+      // tile columns j < TN/2 are gate, j + TN/2 the matching up columns; both factors are rounded to
+      // bf16 first (what a separate activation kernel would read back)
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int m = m0 + wr * WM + i * 16 + frow;
+        if (m >= p.M) continue;
+#pragma unroll
+        for (int j = 0; j < TN / 2; ++j) {
+          const int n = n0 + wc * (WN / 2) + j * 16 + fq * 4;
+          if (n >= p.N) continue;
+          float v[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            v[r] = glu_gate(bf16_to_f32(f32_to_bf16(acc[i][j][r])), p.glu_act) * bf16_to_f32(f32_to_bf16(acc[i][j + TN / 2][r]));
+          const size_t o = static_cast<size_t>(m) * p.ldc + n;
+          if (n + 3 < p.N && (p.ldc & 3) == 0) {
+            u32x2_t w = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+            *reinterpret_cast<u32x2_t*>(p.C + o) = w;
+          } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) if (n + r < p.N) p.C[o + r] = f32_to_bf16(v[r]);
+          }
+        }
+      }
+      return;
+    }
+  }
+  if (p.splitk > 1 || p.raw_partial) {
+    float* slab = p.partial + static_cast<size_t>(ksplit) * p.M * p.N;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int m = m0 + wr * WM + i * 16 + frow;
+      if (m >= p.M) continue;
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int n = n0 + wc * WN + j * 16 + fq * 4;
+        float* dst = slab + static_cast<size_t>(m) * p.N + n;
+        if (n + 3 < p.N && (p.N & 3) == 0) {
+          *reinterpret_cast<f32x4_t*>(dst) = acc[i][j];
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) if (n + r < p.N) dst[r] = acc[i][j][r];
+        }
+      }
+    }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int m = m0 + wr * WM + i * 16 + frow;
+    if (p.amax_val) {
+      // row max over this wave's WN columns: in-lane over j and r, then across the
+      // 4 lanes (fq) that share the row
+      float bv = -INFINITY;
+      int bi = 0x7fffffff;
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int n = n0 + wc * WN + j * 16 + fq * 4 + r;
+          float v = acc[i][j][r];
+          if (p.bias && n < p.N) v += bf16_to_f32(p.bias[n]);
+          if (n < p.N && (v > bv || (v == bv && n < bi))) { bv = v; bi = n; }
+        }
+#pragma unroll
+      for (int off = 16; off < 64; off <<= 1) {
+        const float ov = __shfl_xor(bv, off, 64);
+        const int oi = __shfl_xor(bi, off, 64);
+        if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
+      }
+      if (fq == 0 && m < p.M) {
+        const int n_part = tiles_n * WGN;
+        p.amax_val[static_cast<size_t>(m) * n_part + tn * WGN + wc] = bv;
+        p.amax_idx[static_cast<size_t>(m) * n_part + tn * WGN + wc] = bi;
+      }
+    }
+    if (m >= p.M || (!p.C && !p.Cf)) continue;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int n = n0 + wc * WN + j * 16 + fq * 4;
+      if (n >= p.N) continue;
+      float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+      const size_t o = static_cast<size_t>(m) * p.ldc + n;
+      const bool full = (n + 3 < p.N) && ((p.ldc & 3) == 0);
+      if (p.bias) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) if (n + r < p.N) v[r] += bf16_to_f32(p.bias[n + r]);
+      }
+      if (p.act != ACT_NONE) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = apply_act(v[r], p.act);
+      }
+      if (p.res) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (n + r < p.N) v[r] = bf16_to_f32(f32_to_bf16(v[r])) + bf16_to_f32(p.res[o + r]);
+      }
+      if (p.Cf) {
+        if (full) {
+          *reinterpret_cast<f32x4_t*>(p.Cf + o) = f32x4_t{v[0], v[1], v[2], v[3]};
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) if (n + r < p.N) p.Cf[o + r] = v[r];
+        }
+      }
+      if (p.C) {
+        if (full) {
+          u32x2_t w = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+          *reinterpret_cast<u32x2_t*>(p.C + o) = w;
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) if (n + r < p.N) p.C[o + r] = f32_to_bf16(v[r]);
+        }
+      }
+    }
+  }
+}
+
+}  // namespace evgpt

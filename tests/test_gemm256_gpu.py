@@ -331,8 +331,30 @@ def test_four_waves_on_the_256_tile(dev, force256, M, N, K, act):
         assert torch.equal(force256.linear(x, w, bias, res, act, False), first)
     if N % 16 == 0 or act:
         return
-    half = N // 2 // 8 * 8                                # gated: gate rows, then up rows
+    half = N // 2 // 32 * 32                              # gated: gate rows, then up rows
     gu = x.float() @ w[:2 * half].float().t()
     if half >= 16:
         g, u = gu[:, :half].to(torch.bfloat16).float(), gu[:, half:].to(torch.bfloat16).float()
         _check(force256.linear_swiglu(x, w[:2 * half].contiguous()), torch.nn.functional.silu(g) * u, K)
+
+
+@pytest.mark.parametrize("M,N,K,act", [(577, 3072, 1024, 0), (577, 4096, 1024, 2), (300, 4096, 4096, 0), (257, 2056, 64, 1), (2308, 1024, 1024, 0),
+                                       (1154, 3080, 192, 0), (1010, 1000, 256, 1), (160, 9288, 128, 0), (33, 9304, 576, 0)])
+def test_one_round_of_tiles_on_the_deep_ring(dev, M, N, K, act):
+    """``gemm_ring.hip`` by the rule that chooses it: all five tiles, ragged rows and columns, fewer K-tiles than its ring, bias, activation and
+    residual, gated and as fp32 slabs, against fp32 (``_check``'s bound); the same bits from run to run."""
+    from eventgpt_amd.ops import hip
+    x, w = _rand(M, K, dev=dev), _rand(N, K, dev=dev, seed=1, scale=0.05)
+    bias, res = _rand(N, dev=dev, seed=2), _rand(M, N, dev=dev, seed=3)
+    lin = x.float() @ w.float().t()
+    h = lin + bias.float()
+    want = (h, torch.nn.functional.gelu(h), h * torch.sigmoid(1.702 * h))[act].to(torch.bfloat16).float() + res.float()
+    first = hip.raw.linear(x, w, bias, res, act, False)
+    _check(first, want, K)
+    for _ in range(3):
+        assert torch.equal(hip.raw.linear(x, w, bias, res, act, False), first)
+    _check(hip.raw.linear(x, w, None, None, 0, True), lin, K)
+    _check(hip.raw.linear_partial(x, w).sum(0), lin, K)
+    half = N // 2 // 32 * 32
+    g, u = lin[:, :half].to(torch.bfloat16).float(), lin[:, half:2 * half].to(torch.bfloat16).float()
+    _check(hip.raw.linear_swiglu(x, w[:2 * half].contiguous()), torch.nn.functional.silu(g) * u, K)
