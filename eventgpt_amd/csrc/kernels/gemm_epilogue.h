@@ -6,7 +6,8 @@ namespace evgpt {
 
 // Epilogue shared by the GEMM kernels: lane holds C[m][n .. n+3] of each 16x16 tile (m = row
 // lane & 15, n = 4 * (lane >> 4)); wave (wr, wc) owns the WM x WN sub-tile at (wr*WM, wc*WN).
-template <int TM, int TN, int WM, int WN, int WGN>
+// ACT: the activation as a constant (-1: p.act, a choice among all of them unrolled for every element).
+template <int TM, int TN, int WM, int WN, int WGN, int ACT = -1>
 __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4_t (&acc)[TM][TN], int m0, int n0, int wr,
                                               int wc, int tn, int tiles_n, int ksplit, int lane) {
   const int frow = lane & 15, fq = lane >> 4;
@@ -100,9 +101,9 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4_t (&acc
 #pragma unroll
         for (int r = 0; r < 4; ++r) if (n + r < p.N) v[r] += bf16_to_f32(p.bias[n + r]);
       }
-      if (p.act != ACT_NONE) {
+      if (ACT < 0 ? p.act != ACT_NONE : ACT != ACT_NONE) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = apply_act(v[r], p.act);
+        for (int r = 0; r < 4; ++r) v[r] = apply_act(v[r], ACT < 0 ? p.act : ACT);
       }
       if (p.res) {
 #pragma unroll

@@ -24,7 +24,7 @@ __device__ __forceinline__ void load_to_lds16(const unsigned char* src, int byte
 }
 
 // WGM x WGN waves, each TM x TN tiles of 16 x 16; S K-tiles of 64 in the ring
-template <int TM, int TN, int WGM, int WGN, int S>
+template <int TM, int TN, int WGM, int WGN, int S, int ACT>
 __global__ __launch_bounds__(512) void gemm_ring_kernel(GemmParams p) {
   constexpr int NW = WGM * WGN, WM = TM * 16, WN = TN * 16, BM = WM * WGM, BN = WN * WGN, A_BYTES = BM * 128, STAGE = (BM + BN) * 128;
   constexpr int IA = BM / (8 * NW), IW = BN / (8 * NW), G = IA + IW;           // staging instructions per wave and K-tile
@@ -127,18 +127,25 @@ __global__ __launch_bounds__(512) void gemm_ring_kernel(GemmParams p) {
     __builtin_amdgcn_sched_barrier(0);
   }
   wait_loads<0>();
-  gemm_epilogue<TM, TN, WM, WN, WGN>(p, acc, m0, n0, wr, wc, tn, tiles_n, ksplit, lane);
+  gemm_epilogue<TM, TN, WM, WN, WGN, ACT>(p, acc, m0, n0, wr, wc, tn, tiles_n, ksplit, lane);
 }
 
-template <int TM, int TN, int WGM, int WGN, int S>
-void launch(const GemmParams& p, hipStream_t st) {
+template <int TM, int TN, int WGM, int WGN, int S, int ACT>
+void launch_act(const GemmParams& p, hipStream_t st) {
   constexpr int BM = TM * 16 * WGM, BN = TN * 16 * WGN, lds = S * (BM + BN) * 128;
-  static const bool attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_ring_kernel<TM, TN, WGM, WGN, S>),
+  static const bool attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_ring_kernel<TM, TN, WGM, WGN, S, ACT>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess;
   (void)attr;
   const int bn_out = p.glu_half ? BN / 2 : BN;
   const int tiles = (p.M + BM - 1) / BM * ((p.N + bn_out - 1) / bn_out) * p.splitk;
-  hipLaunchKernelGGL((gemm_ring_kernel<TM, TN, WGM, WGN, S>), dim3(tiles), dim3(512), lds, st, p);
+  hipLaunchKernelGGL((gemm_ring_kernel<TM, TN, WGM, WGN, S, ACT>), dim3(tiles), dim3(512), lds, st, p);
+}
+template <int TM, int TN, int WGM, int WGN, int S>
+void launch(const GemmParams& p, hipStream_t st) {
+  const int act = p.splitk > 1 || p.raw_partial ? ACT_NONE : p.act;       // (slabs: their consumer's)
+  if (act == ACT_GELU) launch_act<TM, TN, WGM, WGN, S, ACT_GELU>(p, st);
+  else if (act == ACT_QUICK_GELU) launch_act<TM, TN, WGM, WGN, S, ACT_QUICK_GELU>(p, st);
+  else launch_act<TM, TN, WGM, WGN, S, ACT_NONE>(p, st);
 }
 
 }  // namespace
@@ -156,6 +163,7 @@ void launch(const GemmParams& p, hipStream_t st) {
 //    160, 39.7 / 37.5; 400 x 5632 x 4096, 176, 35.4 / 48.1)
 RingTile gemm_ring_tile(const GemmParams& p) {
   const long long lim = 1ll << 31;
+  if (p.act != ACT_NONE && p.act != ACT_GELU && p.act != ACT_QUICK_GELU) return RING_NONE;
   if (p.M <= 32 || p.k_cols || p.amax_val || p.rope_cos || p.grp_start) return RING_NONE;
   if (2ll * 128 * p.lda >= lim || 2ll * (p.glu_half ? 2ll * p.glu_half : 192) * p.ldw >= lim) return RING_NONE;
   auto tiles = [&](int bm, int bn) {
