@@ -114,6 +114,13 @@ __global__ __launch_bounds__((WIDE ? 256 : 64) * KW) void head_linear_kernel(Hea
   const int wn = wid % WN, wk = wid / WN;
   const int n0 = blockIdx.x * (16 * WN) + wn * 16;
   const T* wp = static_cast<const T*>(a.w) + (static_cast<long long>(h) * a.N + min(n0 + fr, a.N - 1)) * K + g * 8;
+  // the gate and the first weights are on their way while inputs are staged (32 rows of 16 heads, 512 x 128: 4.8-5.0 -> 4.4-4.9 us; behind a
+  // merge the registers are not there for them, 9.4 -> 11.3)
+  constexpr int PF = MERGE ? 0 : 4;
+  Frag<T> wf[PF > 0 ? PF : 1];
+#pragma unroll
+  for (int i = 0; i < PF; ++i) wf[i] = load_frag(wp + min((wk + i * KW) * 32, K - 32));
+  const float gate = !MERGE && a.gate.p ? src1(a.gate, r0 + min(fr, nr - 1), a.gcol + h) : 0.f;
   if constexpr (MERGE) {
     // A wave takes a whole row (WIDE), or its share of the columns of every row with four groups of lanes on different
     // splits.  Maxima and sums (a lane per split, at most 64) are on their way together with the first partial rows.
@@ -175,8 +182,13 @@ __global__ __launch_bounds__((WIDE ? 256 : 64) * KW) void head_linear_kernel(Hea
   __syncthreads();
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
   const T* xp = xs + fr * ldx + g * 8;
+#pragma unroll
+  for (int i = 0; i < PF; ++i) {
+    const int k = (wk + i * KW) * 32;
+    if (k < K) acc = mma(wf[i], load_frag(xp + k), acc);
+  }
 #pragma unroll 4
-  for (int k = wk * 32; k < K; k += KW * 32) acc = mma(load_frag(wp + k), load_frag(xp + k), acc);
+  for (int k = (wk + PF * KW) * 32; k < K; k += KW * 32) acc = mma(load_frag(wp + k), load_frag(xp + k), acc);
   if constexpr (KW > 1) {
     if (wk > 0) *reinterpret_cast<f32x4_t*>(part[wk - 1][wn][lane]) = acc;
     __syncthreads();
@@ -187,7 +199,7 @@ __global__ __launch_bounds__((WIDE ? 256 : 64) * KW) void head_linear_kernel(Hea
   const int n = n0 + g * 4;                       // N % 16 == 0: all four or none
   if (fr >= nr || n >= a.N) return;
   const long long row = r0 + fr;
-  if (a.gate.p) acc *= sigmoid_f(src1(a.gate, row, a.gcol + h));
+  if (a.gate.p) acc *= sigmoid_f(MERGE ? src1(a.gate, row, a.gcol + h) : gate);
   store4(static_cast<T*>(a.y) + (row * a.H + h) * a.N + n, acc[0], acc[1], acc[2], acc[3]);
 }
 template <typename T, bool MERGE>

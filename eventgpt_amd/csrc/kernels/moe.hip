@@ -100,6 +100,55 @@ void launch_moe_group(const int* idx, int* perm, int* inv, int* start, int n, in
   hipLaunchKernelGGL(moe_group_kernel, dim3(E), dim3(1024), 0, st, idx, perm, inv, start, n, E);
 }
 
+// Routing and sorting of up to 1024 entries in one launch (32 rows of 8 experts: 7.3-8.1 us, two launches 4.7 + 5.1 and what lies between): a wave per row, then a wave per
+// expert counts and places its entries with ballots.
+constexpr int RG_ENTRIES = 1024, RG_EXPERTS = 256;
+__global__ __launch_bounds__(1024) void moe_route_group_kernel(MoeRoute a, float* __restrict__ w, int* __restrict__ perm, int* __restrict__ inv,
+                                                               int* __restrict__ start, int rows) {
+  extern __shared__ float z[];                     // [16][E]
+  __shared__ int sel[RG_ENTRIES], count[RG_EXPERTS];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, n = rows * a.top;
+  for (int row = wid; row < rows; row += 16) {
+    int e;
+    float f;
+    route_row(a, row, z + wid * a.E, lane, e, f);
+    if (lane < a.top) {
+      sel[row * a.top + lane] = e;
+      w[static_cast<long long>(row) * a.top + lane] = f;
+    }
+  }
+  __syncthreads();
+  for (int e = wid; e < a.E; e += 16) {
+    int c = 0;
+    for (int i = lane; i - lane < n; i += 64) c += __builtin_popcountll(__builtin_amdgcn_ballot_w64(i < n && sel[i] == e));
+    if (lane == 0) count[e] = c;
+  }
+  __syncthreads();
+  for (int e = wid; e < a.E; e += 16) {
+    int before = 0;
+    for (int j = lane; j < e; j += 64) before += count[j];
+    int at = wave_sum_int(before);
+    if (lane == 0) {
+      start[e] = at;
+      if (e == a.E - 1) start[a.E] = n;
+    }
+    for (int i = lane; i - lane < n; i += 64) {
+      const bool mine = i < n && sel[i] == e;
+      const unsigned long long all = __builtin_amdgcn_ballot_w64(mine);
+      if (mine) {
+        const int to = at + __builtin_popcountll(all & ((1ull << lane) - 1));
+        perm[to] = i;
+        inv[i] = to;
+      }
+      at += __builtin_popcountll(all);
+    }
+  }
+}
+bool moe_route_group_ok(int rows, int E, int top) { return static_cast<long long>(rows) * top <= RG_ENTRIES && E <= RG_EXPERTS; }
+void launch_moe_route_group(const MoeRoute& r, float* w, int* perm, int* inv, int* start, int rows, hipStream_t st) {
+  hipLaunchKernelGGL(moe_route_group_kernel, dim3(1), dim3(1024), 64 * r.E, st, r, w, perm, inv, start, rows);
+}
+
 __device__ __forceinline__ float dot_chunk(const u32x4_t& w, const u32x4_t& x, float acc, bf16_t) { return dot8_bf16(w, x, acc); }
 __device__ __forceinline__ float dot_chunk(const u32x4_t& w, const u32x4_t& x, float acc, float) {
 #pragma unroll

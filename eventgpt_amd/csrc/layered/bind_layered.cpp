@@ -879,6 +879,20 @@ std::tuple<Tensor, Tensor, Tensor> moe_group(const Tensor& idx, int64_t E) {
   evgpt::launch_moe_group(idx.data_ptr<int>(), perm.data_ptr<int>(), inv.data_ptr<int>(), start.data_ptr<int>(), (int)idx.numel(), (int)E, cur_stream());
   return {perm, inv, start};
 }
+// moe_route and moe_group: {weights [M, top], perm, inverse, start}; one launch where there are few entries
+std::tuple<Tensor, Tensor, Tensor, Tensor> moe_route_group(const Tensor& logits, const Tensor& bias, int64_t top) {
+  int64_t M;
+  const evgpt::MoeRoute r = route_of(logits, bias, top, &M);
+  if (M < 1 || !evgpt::moe_route_group_ok((int)std::min<int64_t>(M, 1 << 20), r.E, r.top)) {
+    auto [idx, w] = moe_route(logits, bias, top);
+    auto [perm, inv, start] = moe_group(idx, r.E);
+    return {w, perm, inv, start};
+  }
+  const auto ints = bias.options().dtype(at::kInt);
+  Tensor w = at::empty({M, top}, bias.options()), perm = at::empty({M * top}, ints), inv = at::empty({M, top}, ints), start = at::empty({r.E + 1}, ints);
+  evgpt::launch_moe_route_group(r, w.data_ptr<float>(), perm.data_ptr<int>(), inv.data_ptr<int>(), start.data_ptr<int>(), (int)M, cur_stream());
+  return {w, perm, inv, start};
+}
 // Rows sorted by expert times each expert's matrix w [E, N, K]: row i is x[perm[i] / top] (gather) or x[i].  act >= 0: w's
 // rows are [gate | up] and the result is act(gate) * up [rows, N / 2].
 Tensor moe_linear(const Tensor& x, const Tensor& w, const Tensor& start, const OptTensor& perm, int64_t top, int64_t act) {
@@ -1002,6 +1016,7 @@ TORCH_LIBRARY(evlay, m) {
   m.def("latent_max() -> int", []() { return (int64_t)evgpt::LATENT_MAX; });
   m.def("moe_route(Tensor logits, Tensor bias, int top) -> (Tensor, Tensor)", &moe_route);
   m.def("moe_group(Tensor idx, int E) -> (Tensor, Tensor, Tensor)", &moe_group);
+  m.def("moe_route_group(Tensor logits, Tensor bias, int top) -> (Tensor, Tensor, Tensor, Tensor)", &moe_route_group);
   m.def("moe_linear(Tensor x, Tensor w, Tensor start, Tensor? perm, int top, int act) -> Tensor", &moe_linear);
   m.def("moe_step(Tensor x, Tensor logits, Tensor bias, int top, Tensor w_gate_up, Tensor w_down, int act) -> Tensor", &moe_step);
   m.def("merge_norm_rows_(Tensor(a!) x, Tensor a, Tensor b, Tensor wa, Tensor wb, Tensor? w, int n, float eps, bool f32) -> Tensor", &merge_norm_rows_);

@@ -154,6 +154,9 @@ struct MoeRoute {
 void launch_moe_route(const MoeRoute& r, int* idx, float* w, int rows, hipStream_t st);      // idx, w [rows][top]
 // Entries (row * top + k) sorted by expert: perm [n], its inverse inv [n], start [E + 1]
 void launch_moe_group(const int* idx, int* perm, int* inv, int* start, int n, int E, hipStream_t st);
+// both in one launch
+bool moe_route_group_ok(int rows, int E, int top);
+void launch_moe_route_group(const MoeRoute& r, float* w, int* perm, int* inv, int* start, int rows, hipStream_t st);
 // Up to four rows, weights of the chosen experts streamed: h[b][k] = act(Wg x) * (Wu x), y[b] = sum_k w_k Wd h[b][k].
 // w_gate_up [E][2 F][K], w_down [E][N][F]
 struct MoeStep {

@@ -605,8 +605,7 @@ class MoE(Mixer):
             return
         xn = stream.normed(norm)
         logits = raw.linear_slabs(xn, self.w_router)
-        idx, weights = raw.moe_route(logits, self.bias, top)
-        perm, inv, start = raw.moe_group(idx, self.spec.experts)
+        weights, perm, inv, start = raw.moe_route_group(logits, self.bias, top)
         h = raw.moe_linear(xn, self.w_gate_up, start, perm, top, self.act)
         y = raw.moe_linear(h, self.w_down, start, None, 1, -1)
         stream.pending = ("mix", y, inv, weights, stream.post)

@@ -294,6 +294,20 @@ def test_routing(raw, dev, E, top):
     assert int(idx.min()) >= 0 and int(idx.max()) < E and all(len(set(r)) == top for r in idx.tolist())
 
 
+@pytest.mark.parametrize("M,E,top", [(1, 1, 1), (32, 8, 2), (17, 70, 3), (512, 256, 2), (513, 8, 2), (40, 300, 40), (100, 5, 5)])
+def test_routing_and_sorting_in_one_launch(raw, dev, M, E, top):
+    """What ``moe_route`` and ``moe_group`` give, bit for bit: around its bounds of entries and experts, slabs, ties and rows without a number."""
+    z, b = rnd(M, -(-E // 8) * 8).float(), rnd(E, seed=1).float().to(dev)
+    z[M // 2:M // 2 + 2] = 0.5
+    z[M // 3] = float("nan")
+    for logits in (z.to(dev), torch.stack([z, z]).to(dev)):
+        idx, want = raw.moe_route(logits, b, top)
+        w, perm, inv, start = raw.moe_route_group(logits, b, top)
+        assert torch.equal(w, want)
+        for got, ref in zip((perm, inv, start), raw.moe_group(idx, E)):
+            assert torch.equal(got, ref)
+
+
 @pytest.mark.parametrize("M,E,top", [(1, 1, 1), (5, 9, 2), (700, 6, 3), (3000, 70, 4), (64, 5, 5)])
 def test_sorting_by_expert(raw, dev, M, E, top):
     g = torch.Generator().manual_seed(M)
