@@ -518,8 +518,8 @@ static void launch_fewrow(const GemmParams& p, hipStream_t st) {
 
 // ---------------------------------------------------------------------------------------
 // 256 x 256 x 64 tile, 8 waves (2 x 4, each 128 x 64 of C), one workgroup per CU: the kernel
-// for GEMMs with thousands of rows whose operands are K-strided or whose output gemm_quad.hip does not store.  The 4-wave kernel above stops near 900 TFLOP/s however it
-// is pipelined, because one wave per SIMD has to alternate between feeding the LDS pipe and
+// for GEMMs with thousands of rows whose operands are K-strided or whose output gemm_quad.hip
+// does not store.  The 4-wave kernel above stops near 900 TFLOP/s however it is pipelined, because one wave per SIMD has to alternate between feeding the LDS pipe and
 // the MFMA pipe; here each SIMD holds two waves that run HALF A PHASE APART, so one issues
 // MFMAs while the other issues its LDS reads and the staging loads.
 //
@@ -938,7 +938,8 @@ static bool use_256(int M, int N, int K = 0) {
 // CU), or with three under 400 tiles (about three for every two CUs: 577 x 4096 x 1024 from memory 18.7 us, two stages
 // 22.2, four waves 20.5).  Behind where the tiles leave CUs idle (577 x 3072, 240 tiles: 13.6 vs 11.9), over longer
 // contractions (636 x 12288 x 4096: 116 vs 74; 600 x 9280 x 2048 39 vs 36) and for 1024 columns (2885 rows 15.5 vs 14.2).
-// Lines between, us with weights from memory, this tile vs the other choice:
+// (Under 400 tiles nearly all are gemm_ring.hip's: products of one round of its tiles.)  Lines between, us with weights from memory, this
+// tile vs the other choice:
 //  * one round of three workgroups a CU (768 tiles) is ahead: 750 tiles 1.09 to 1.47 times as fast
 //  * more than a round where the 128 x 128 tile takes one (512): ahead up to K = 320 (1.03 to 1.15; with 256 rows, whose few row
 //    tiles share a weight tile, 0.96), behind from there to 256 x 32000 x 1024 46.0 vs 33.0, 1000 x 8192 x 1024 40.0 vs 29.8, 2308 x
