@@ -294,9 +294,9 @@ def test_routing(raw, dev, E, top):
     assert int(idx.min()) >= 0 and int(idx.max()) < E and all(len(set(r)) == top for r in idx.tolist())
 
 
-@pytest.mark.parametrize("M,E,top", [(1, 1, 1), (32, 8, 2), (17, 70, 3), (512, 256, 2), (513, 8, 2), (40, 300, 40), (100, 5, 5)])
+@pytest.mark.parametrize("M,E,top", [(1, 1, 1), (32, 8, 2), (17, 70, 3), (48, 256, 21), (49, 8, 2), (40, 300, 40), (48, 64, 22), (300, 8, 2)])
 def test_routing_and_sorting_in_one_launch(raw, dev, M, E, top):
-    """What ``moe_route`` and ``moe_group`` give, bit for bit: around its bounds of entries and experts, slabs, ties and rows without a number."""
+    """What ``moe_route`` and ``moe_group`` give, bit for bit: around its bounds of rows, entries and experts, slabs, ties and rows without a number."""
     z, b = rnd(M, -(-E // 8) * 8).float(), rnd(E, seed=1).float().to(dev)
     z[M // 2:M // 2 + 2] = 0.5
     z[M // 3] = float("nan")
