@@ -334,13 +334,19 @@ def _transposed_for_dgrad(weight) -> Optional[torch.Tensor]:
 
 
 def _free_sink(weight, dtype):
-    """The parameter's published gradient slot, taken, if it is still free and of this type."""
+    """The parameter's published gradient slot, taken, if it is still free and of this type.  Free: no gradient yet, or
+    zeros in the slot that nobody has written to."""
     sink = getattr(weight, "_grad_sink", None)
-    if (sink is not None and weight.grad is None and not getattr(weight, "_grad_sink_used", True)
-            and sink.dtype == dtype and sink.shape == weight.shape and sink.is_contiguous()):
-        weight._grad_sink_used = True
-        return sink
-    return None
+    if (sink is None or getattr(weight, "_grad_sink_used", True) or sink.dtype != dtype or sink.shape != weight.shape
+            or not sink.is_contiguous()):
+        return None
+    grad = weight.grad
+    zeros = grad is sink and sink._version == getattr(weight, "_grad_sink_zeros", None)
+    if not (grad is None or zeros):
+        return None
+    weight._grad_sink_used = True
+    weight.grad = None                         # autograd adopts what the node returns
+    return sink
 
 
 def _wgrad_to_sink(weight, g2, x2, f32: bool = False):

@@ -45,7 +45,7 @@ class _Bucket:
             n = p.numel()
             self.flat_param[off:off + n].copy_(p.data.reshape(-1))
             p.data = self.flat_param[off:off + n].view_as(p)
-            p.grad = self.flat_grad[off:off + n].view_as(p)
+            p.grad = self.flat_grad[off:off + n].view_as(p).data     # (.data: a version counter of its own, see zero_grad)
             self.grad_views.append(p.grad)
             off += n
         lo = rank * self.shard_len
@@ -101,21 +101,22 @@ class ShardedAdamW:
         self.overlap = overlap and self.on_rccl
         self.comm_stream = torch.cuda.Stream() if self.on_rccl else None
         self._owner: Dict[int, _Bucket] = {}
-        # Direct gradients: a bf16 matrix or an fp32 parameter on the GPU gets its slot of the flat buffer published as
-        # ``_grad_sink``.  The in-tree wgrad GEMM (``ops/differentiable.py``) writes a step's first
-        # gradient straight into the slot and autograd adopts that view as ``.grad``: no zero fill of
-        # the buffer and no read-modify-write accumulation into it (for a 7B decoder those are 13.6 GB
-        # written plus 41 GB moved per step).  Whatever reaches ``.grad`` some other way is settled into
-        # the slot before the buffer is reduced, so correctness never depends on the shortcut.
+        # Direct gradients: a matrix on the GPU gets its slot of the flat buffer published as ``_grad_sink``.
+        # The in-tree wgrad GEMM (``ops/differentiable.py``) writes a step's first gradient straight into the
+        # slot and autograd adopts that view as ``.grad``: no read-modify-write accumulation into it and, for
+        # bf16, no zero fill of the buffer (for a 7B decoder those are 13.6 GB written plus 41 GB moved per
+        # step).  Whatever reaches ``.grad`` some other way is settled into the slot before the buffer is
+        # reduced, so correctness never depends on the shortcut.
         self._sink: Dict[int, torch.Tensor] = {}
         self._hooks = []
         for b in self.buckets:
             for p, view in zip(b.params, b.grad_views):
                 self._owner[id(p)] = b
                 if direct_grads and p.is_cuda and (p.dtype == torch.float32 or (p.dtype == torch.bfloat16 and p.dim() == 2)):
-                    p._grad_sink = view
-                    p._grad_sink_used = True   # until the first zero_grad hands the slot out
                     self._sink[id(p)] = view
+                    if p.dim() == 2:
+                        p._grad_sink = view
+                        p._grad_sink_used = True   # until the first zero_grad hands the slot out
                 if self.overlap:
                     self._hooks.append(p.register_post_accumulate_grad_hook(self._on_grad))
         self._arm()
@@ -129,9 +130,9 @@ class ShardedAdamW:
         for b in self.buckets:
             for p in b.params:
                 if id(p) in self._sink:
-                    del p._grad_sink
-                    if hasattr(p, "_grad_sink_used"):
-                        del p._grad_sink_used
+                    for name in ("_grad_sink", "_grad_sink_used", "_grad_sink_zeros"):
+                        if hasattr(p, name):
+                            delattr(p, name)
                 p.grad = None
         self._sink = {}
 
@@ -209,10 +210,21 @@ class ShardedAdamW:
 
     # -------------------------------------------------------------------- step
     def zero_grad(self, set_to_none: bool = False) -> None:
+        """Every gradient is zeros in its slot of the flat buffer afterwards; a bf16 matrix that takes its
+        gradient directly has none until the next one is written."""
         for b in self.buckets:
             direct = [id(p) in self._sink for p in b.params]
-            if not any(direct):
+            if b.flat_grad.dtype == torch.float32 or not any(direct):
                 b.flat_grad.zero_()
+                for p, view, d in zip(b.params, b.grad_views, direct):
+                    if d:
+                        p.grad = view
+                        if p.dim() == 2:
+                            # The slot may be overwritten while it holds these zeros: while the view's counter of
+                            # in-place writes stands where it stands now (``ops.differentiable._free_sink``; writes
+                            # through ``p.grad.data`` have a counter of their own).
+                            p._grad_sink_zeros = view._version
+                            p._grad_sink_used = False
                 continue
             for p, view, d in zip(b.params, b.grad_views, direct):
                 if d:

@@ -358,3 +358,41 @@ def test_fp32_parameters_get_the_sums_of_the_weight_gradient(dev, rows, k, n, us
                                                passes * sum(gy.double().abs().sum(0) for gy in gys))):
         assert p.grad.dtype == torch.float32 and flat.data_ptr() <= p.grad.data_ptr() < flat.data_ptr() + 4 * flat.numel()
         assert bool(((p.grad.double() - w).abs() <= (rows + 4) * 2.0 ** -24 * s + 1e-30).all())
+
+
+def _in_tree_loss(net, x):
+    """A loss of ``net`` with its linears on the in-tree products; their weight gradients are the same bits from call to call."""
+    from eventgpt_amd.ops.intree_mode import InTreeLinear
+    with torch.autocast("cuda", dtype=torch.bfloat16), InTreeLinear() as mode:
+        y = net(x)
+    assert mode.routed > 0
+    return y.float().square().mean()
+
+
+def test_gradients_after_zero_grad_are_zeros_that_count(dev):
+    """``zero_grad`` leaves every fp32 gradient as zeros in its slot: what a program adds to it before the backward counts, and a
+    parameter that takes no part has a gradient of zeros."""
+    from eventgpt_amd.parallel.dp import ShardedAdamW
+    torch.manual_seed(0)
+    net = torch.nn.Sequential(torch.nn.Linear(64, 128), torch.nn.LayerNorm(128), torch.nn.Linear(128, 64)).to(dev)
+    unused = torch.nn.Linear(64, 64).to(dev)
+    x = torch.randn(48, 64, generator=torch.Generator().manual_seed(1)).to(dev)
+    want = torch.autograd.grad(_in_tree_loss(net, x), list(net.parameters()))
+    opt = ShardedAdamW([*net.parameters(), *unused.parameters()], lr=1e-3)
+    flat = opt.buckets[0].flat_grad
+    for plus in (0.0, 0.5, 0.0):
+        flat.fill_(7.0)
+        opt.zero_grad()
+        for p in (*net.parameters(), *unused.parameters()):
+            assert p.grad is not None and flat.data_ptr() <= p.grad.data_ptr() < flat.data_ptr() + 4 * flat.numel()
+            assert not bool(p.grad.any())
+        if plus:
+            net[0].weight.grad.add_(plus)
+            net[1].weight.grad.add_(plus)
+        _in_tree_loss(net, x).backward()
+        for p, w in zip(net.parameters(), want):
+            assert torch.equal(p.grad, w + plus if plus and (p is net[0].weight or p is net[1].weight) else w)
+        assert all(not bool(p.grad.any()) for p in unused.parameters())
+        assert (net[2].weight.grad.data_ptr() == net[2].weight._grad_sink.data_ptr()) and net[2].weight._grad_sink_used
+        opt.global_grad_norm()
+        assert all(flat.data_ptr() <= p.grad.data_ptr() < flat.data_ptr() + 4 * flat.numel() for p in net.parameters())
