@@ -333,25 +333,39 @@ def _transposed_for_dgrad(weight) -> Optional[torch.Tensor]:
     return wt
 
 
-def _free_sink(weight, dtype):
-    """The parameter's published gradient slot, taken, if it is still free and of this type.  Free: no gradient yet, or
-    zeros in the slot that nobody has written to."""
+def _only_accumulated(ctx, weight) -> bool:
+    """Whether the gradient that the node ``ctx`` is about to return for its input ``weight`` goes into ``weight.grad`` and nowhere
+    else: ``torch.autograd.grad`` gives it to its caller, and a hook may keep it."""
+    if weight._backward_hooks:
+        return False
+    for node, _ in ctx.next_functions:
+        if getattr(node, "variable", None) is weight:
+            try:
+                return torch._C._will_engine_execute_node(node)
+            except RuntimeError:               # raised while ``torch.autograd.grad`` collects this leaf's gradient
+                return False
+    return False
+
+
+def _free_sink(ctx, weight, dtype):
+    """The parameter's published gradient slot, taken, if it is still free, of this type and nothing but ``.grad`` will refer
+    to it.  Free: no gradient yet, or zeros in the slot that nobody has written to."""
     sink = getattr(weight, "_grad_sink", None)
     if (sink is None or getattr(weight, "_grad_sink_used", True) or sink.dtype != dtype or sink.shape != weight.shape
             or not sink.is_contiguous()):
         return None
     grad = weight.grad
     zeros = grad is sink and sink._version == getattr(weight, "_grad_sink_zeros", None)
-    if not (grad is None or zeros):
+    if not (grad is None or zeros) or not _only_accumulated(ctx, weight):
         return None
     weight._grad_sink_used = True
     weight.grad = None                         # autograd adopts what the node returns
     return sink
 
 
-def _wgrad_to_sink(weight, g2, x2, f32: bool = False):
+def _wgrad_to_sink(ctx, weight, g2, x2, f32: bool = False):
     """``dW = g2^T x2``, written into the parameter's published gradient slot if that is still free."""
-    sink = _free_sink(weight, torch.float32 if f32 else g2.dtype)
+    sink = _free_sink(ctx, weight, torch.float32 if f32 else g2.dtype)
     dw = linear_wgrad(g2, x2, sink, f32)
     return dw if sink is None else dw.view_as(weight)
 
@@ -392,7 +406,7 @@ class _Linear(torch.autograd.Function):
             # A weight used several times in one graph gets all its gradients summed by autograd
             # BEFORE ``.grad`` is set, so "the slot is free" is tracked by the optimizer's own flag
             # (cleared by its ``zero_grad``), never inferred from ``.grad`` alone.
-            dw = _wgrad_to_sink(weight, g2, x2)
+            dw = _wgrad_to_sink(ctx, weight, g2, x2)
         if ctx.has_bias and ctx.needs_input_grad[2]:
             # (one read of the gradient; rows of under 512 columns, where half of a wave's lanes idle, by the library's reduction)
             db = (_raw().column_sum(g2) if g2.dtype == torch.bfloat16 and n >= 512 and n % 8 == 0 and g2.numel() and g2.data_ptr() % 16 == 0
@@ -420,7 +434,7 @@ class _MasterLinear(torch.autograd.Function):
         g2 = gy.reshape(-1, n)
         g2 = g2 if g2.is_contiguous() else g2.contiguous()
         dx = linear_dgrad(g2, w).view(*gy.shape[:-1], k) if ctx.needs_input_grad[0] else None
-        dw = _wgrad_to_sink(ctx.parameter, g2, x2, True) if ctx.needs_input_grad[1] else None
+        dw = _wgrad_to_sink(ctx, ctx.parameter, g2, x2, True) if ctx.needs_input_grad[1] else None
         db = None
         if ctx.has_bias and ctx.needs_input_grad[2]:
             db = (_raw().column_sum(g2, True) if n >= 512 and n % 8 == 0 and g2.numel() and g2.data_ptr() % 16 == 0
@@ -594,9 +608,9 @@ class _LowRank(torch.autograd.Function):
         dx = da = db = None
         dt = _raw().lowrank_out(g2, b.detach().t().contiguous(), ctx.scale)      # scale * dY B  [M, r]
         if ctx.needs_input_grad[2]:
-            db = _wgrad_to_sink(b, g2, t2)
+            db = _wgrad_to_sink(ctx, b, g2, t2)
         if ctx.needs_input_grad[1]:
-            da = _wgrad_to_sink(a, dt, x2)
+            da = _wgrad_to_sink(ctx, a, dt, x2)
         if ctx.needs_input_grad[0]:
             dx = linear_dgrad(dt, a.detach().contiguous()).view(*gy.shape[:-1], a.shape[1])
         return dx, da, db, None
@@ -687,15 +701,15 @@ class _LoRAProjection(torch.autograd.Function):
             if ctx.needs_input_grad[6 + 2 * i] or dx2 is not None:
                 dts[i] = raw.lowrank_out(gi, b.detach().t().contiguous(), s_eff, 0.0, 0)  # s / (1 - p) * dY_i B_i
             if ctx.needs_input_grad[7 + 2 * i]:
-                grads[2 * i + 1] = _lowrank_wgrad(b, gi, t, True)
+                grads[2 * i + 1] = _lowrank_wgrad(ctx, b, gi, t, True)
         for group in _adapter_groups(ab):
             need = [i for i in group if ctx.needs_input_grad[6 + 2 * i]]
             if len(need) == 1:
                 i = need[0]
-                grads[2 * i] = _lowrank_wgrad(ab[2 * i], x2, dts[i], False, p, seeds[i])
+                grads[2 * i] = _lowrank_wgrad(ctx, ab[2 * i], x2, dts[i], False, p, seeds[i])
             elif need:
                 for i in need:
-                    da = _free_sink(ab[2 * i], g2.dtype)
+                    da = _free_sink(ctx, ab[2 * i], g2.dtype)
                     grads[2 * i] = torch.empty_like(ab[2 * i]) if da is None else da.view_as(ab[2 * i])
                 raw.lowrank_wgrad_(x2, [dts[i] for i in need], [grads[2 * i] for i in need], False, p, [seeds[i] for i in need])
             if dx2 is not None and len(group) == 1:
@@ -706,9 +720,9 @@ class _LoRAProjection(torch.autograd.Function):
         return (dx, None, (gy if ctx.needs_input_grad[2] else None), None, None, None, *grads)
 
 
-def _lowrank_wgrad(weight, g, t, transposed, drop_p=0.0, seed=0):
+def _lowrank_wgrad(ctx, weight, g, t, transposed, drop_p=0.0, seed=0):
     """``t^T (m (.) g)`` (or its transpose) in the parameter's published gradient slot if that is still free."""
-    sink = _free_sink(weight, t.dtype)
+    sink = _free_sink(ctx, weight, t.dtype)
     dw = _raw().lowrank_wgrad(g, t, transposed, drop_p, seed, sink)
     return dw if sink is None else dw.view_as(weight)
 

@@ -396,3 +396,48 @@ def test_gradients_after_zero_grad_are_zeros_that_count(dev):
         assert (net[2].weight.grad.data_ptr() == net[2].weight._grad_sink.data_ptr()) and net[2].weight._grad_sink_used
         opt.global_grad_norm()
         assert all(flat.data_ptr() <= p.grad.data_ptr() < flat.data_ptr() + 4 * flat.numel() for p in net.parameters())
+
+
+@pytest.mark.parametrize("kind", ["fp32", "bf16", "lora"])
+def test_gradients_handed_out_are_not_the_optimizers_memory(dev, kind):
+    """What ``torch.autograd.grad`` returns and what a hook keeps is theirs: later passes, ``zero_grad`` and steps leave it alone, and
+    a backward after it still counts in full."""
+    from eventgpt_amd.ops import differentiable as diff
+    from eventgpt_amd.parallel.dp import ShardedAdamW
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(96, 128, generator=g).to(dev).bfloat16()
+    w0 = (torch.randn(64, 128, generator=g) / 8).to(dev)
+    a, b = (torch.nn.Parameter((torch.randn(*s, generator=g) / 8).to(dev).bfloat16()) for s in ((8, 128), (64, 8)))
+    w = torch.nn.Parameter(w0 if kind == "fp32" else w0.bfloat16())
+    frozen = w0.bfloat16()
+    params = [a, b] if kind == "lora" else [w]
+
+    def loss():
+        if kind == "lora":
+            return diff.lora_projection(x, frozen, [(0, a, b)], 2.0).float().square().mean()
+        if kind == "bf16":
+            return diff.linear(x, w).float().square().mean()
+        return _in_tree_loss(lambda t: F.linear(t, w), x)
+    want = [t.clone() for t in torch.autograd.grad(loss(), params)]
+    opt = ShardedAdamW(params, lr=1e-3)
+    flat = opt.buckets[0].flat_grad
+    inside = lambda t: flat.data_ptr() <= t.data_ptr() < flat.data_ptr() + flat.numel() * flat.element_size()
+    opt.zero_grad()
+    got = torch.autograd.grad(loss(), params)
+    loss().backward()                                    # the first gradient that is accumulated
+    assert all(inside(p.grad) and torch.equal(p.grad, t) for p, t in zip(params, want))
+    opt.zero_grad()
+    kept = []
+    hooks = [p.register_hook(kept.append) for p in params]
+    loss().backward()
+    for h in hooks:
+        h.remove()
+    assert len(kept) == len(params) and all(torch.equal(p.grad, t) for p, t in zip(params, want))
+    opt.global_grad_norm()
+    assert all(inside(p.grad) and torch.equal(p.grad, t) for p, t in zip(params, want))
+    opt.zero_grad()
+    opt.global_grad_norm()                               # settles gradients of zeros
+    flat.fill_(7.0)
+    kept.sort(key=lambda t: [p.shape for p in params].index(t.shape))
+    for t, k, w_ in zip(got, kept, want):
+        assert torch.equal(t, w_) and torch.equal(k, w_)
