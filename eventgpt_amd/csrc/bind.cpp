@@ -190,15 +190,16 @@ Tensor linear_t(const Tensor& a, const Tensor& w, bool a_t, bool w_t, const c10:
   if (bias.has_value()) { check_bf16(*bias, "bias"); TORCH_CHECK(bias->numel() == N); }
   if (res.has_value()) { check_bf16(*res, "residual"); TORCH_CHECK(res->numel() == M * N); }
   Tensor y;
+  bool copied = false;
   if (out.has_value()) {
     y = *out;
     TORCH_CHECK(y.is_cuda() && y.is_contiguous() && y.numel() == M * N &&
                 y.scalar_type() == (out_f32 ? at::kFloat : at::kBFloat16), "linear_t: out must be a contiguous [M, N] "
                 "tensor of the result's dtype");
-  } else {
-    y = at::empty({M, N}, a.options().dtype(out_f32 ? at::kFloat : at::kBFloat16));
+    copied = reinterpret_cast<uintptr_t>(y.data_ptr()) % 16 != 0;       // (the epilogues store four columns at once)
   }
-  if (M == 0 || N == 0) return y;
+  if (!out.has_value() || copied) y = at::empty({M, N}, a.options().dtype(out_f32 ? at::kFloat : at::kBFloat16));
+  if (M == 0 || N == 0) return copied ? *out : y;
   const int sk = evgpt::gemm_splitk_t((int)M, (int)N, (int)K);
   Tensor ws;
   if (sk > 1) ws = at::empty({sk * M * N}, a.options().dtype(at::kFloat));
@@ -206,7 +207,10 @@ Tensor linear_t(const Tensor& a, const Tensor& w, bool a_t, bool w_t, const c10:
                             bptr_opt(bias), bptr_opt(res), (int)M, (int)N, (int)K, (int)a.stride(0), (int)w.stride(0),
                             (int)N, (int)act, a_t, w_t, (int)ka_rows, (int)kw_rows, cur_stream(),
                             sk > 1 ? ws.data_ptr<float>() : nullptr, sk);
-  return y;
+  if (!copied) return y;
+  Tensor dst = *out;
+  dst.view({M, N}).copy_(y);
+  return dst;
 }
 
 // t [.., R] = alpha * x [.., K] · w [R, K]^T for a low-rank adapter's R <= 16 rows: one launch, no split-K pass.

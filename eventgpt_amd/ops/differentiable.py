@@ -348,11 +348,11 @@ def _only_accumulated(ctx, weight) -> bool:
 
 
 def _free_sink(ctx, weight, dtype):
-    """The parameter's published gradient slot, taken, if it is still free, of this type and nothing but ``.grad`` will refer
-    to it.  Free: no gradient yet, or zeros in the slot that nobody has written to."""
+    """The parameter's published gradient slot, taken, if it is still free, of this type, on 16 bytes as the kernels' stores want
+    it, and nothing but ``.grad`` will refer to it.  Free: no gradient yet, or zeros in the slot that nobody has written to."""
     sink = getattr(weight, "_grad_sink", None)
     if (sink is None or getattr(weight, "_grad_sink_used", True) or sink.dtype != dtype or sink.shape != weight.shape
-            or not sink.is_contiguous()):
+            or not sink.is_contiguous() or sink.data_ptr() % 16):
         return None
     grad = weight.grad
     zeros = grad is sink and sink._version == getattr(weight, "_grad_sink_zeros", None)

@@ -441,3 +441,50 @@ def test_gradients_handed_out_are_not_the_optimizers_memory(dev, kind):
     kept.sort(key=lambda t: [p.shape for p in params].index(t.shape))
     for t, k, w_ in zip(got, kept, want):
         assert torch.equal(t, w_) and torch.equal(k, w_)
+
+
+def _misaligned_slots(params):
+    return [p for p in params if p.dim() == 2 and p._grad_sink.data_ptr() % 16]
+
+
+@pytest.mark.parametrize("level", [2, 3])
+def test_fp32_gradients_behind_scalar_parameters(dev, level):
+    """Adapters whose scalars shift the slots of the matrices behind them off 16 bytes: the gradients are what the same products give
+    without an optimizer, and no kernel stores its four floats at once into such a slot."""
+    from eventgpt_amd.align.adapters import create_adapter
+    from eventgpt_amd.parallel.dp import ShardedAdamW
+    torch.manual_seed(level)
+    net = create_adapter(level, 64, bottleneck_dim=64, num_blocks=3, dropout=0.0).to(dev).train()
+    with torch.no_grad():
+        for p in net.parameters():
+            p.add_(torch.randn_like(p) * 0.05)           # (the up-projections start at zero)
+    x = torch.randn(40, 64, generator=torch.Generator().manual_seed(level)).to(dev)
+    names, params = zip(*net.named_parameters())
+    want = torch.autograd.grad(_in_tree_loss(net, x), params)
+    opt = ShardedAdamW(params, lr=1e-3)
+    odd = _misaligned_slots(params)
+    assert odd
+    opt.zero_grad()
+    _in_tree_loss(net, x).backward()
+    assert not any(p._grad_sink_used for p in odd)
+    for name, p, w in zip(names, params, want):
+        assert torch.equal(p.grad, w), name
+    opt.global_grad_norm()
+    for name, p, w in zip(names, params, want):
+        assert torch.equal(p.grad, w), name
+
+
+@pytest.mark.parametrize("f32", [True, False])
+@pytest.mark.parametrize("M,N,K", [(64, 64, 40), (264, 520, 96), (1032, 1304, 128)])
+def test_weight_gradients_into_memory_off_16_bytes(dev, f32, M, N, K):
+    """``linear_wgrad`` into an ``out`` at every element of a 16-byte line: the same bits as into a tensor of its own, and nothing beside it."""
+    from eventgpt_amd.ops import differentiable as diff
+    gy, x = _rand(K, M, dev=dev), _rand(K, N, dev=dev, seed=1)
+    want = diff.linear_wgrad(gy, x, None, f32)
+    for off in range(1, 16 // want.element_size()):
+        buf = torch.full((M * N + 32,), 3.0, device=dev, dtype=want.dtype)
+        out = buf[off:off + M * N].view(M, N)
+        assert out.data_ptr() % 16
+        got = diff.linear_wgrad(gy, x, out, f32)
+        assert got.data_ptr() == out.data_ptr() and torch.equal(out, want)
+        assert bool((buf[:off] == 3).all()) and bool((buf[off + M * N:] == 3).all())
