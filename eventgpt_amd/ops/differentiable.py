@@ -350,7 +350,7 @@ def _only_accumulated(ctx, weight) -> bool:
 def _free_sink(ctx, weight, dtype):
     """The parameter's published gradient slot, taken, if it is still free, of this type, on 16 bytes as the kernels' stores want
     it, and nothing but ``.grad`` will refer to it.  Free: no gradient yet, or zeros in the slot that nobody has written to."""
-    sink = getattr(weight, "_grad_sink", None)
+    sink = getattr(weight, "_grad_sink", None)                       # (weight None: nothing that has a slot)
     if (sink is None or getattr(weight, "_grad_sink_used", True) or sink.dtype != dtype or sink.shape != weight.shape
             or not sink.is_contiguous() or sink.data_ptr() % 16):
         return None
@@ -424,7 +424,8 @@ class _MasterLinear(torch.autograd.Function):
         xc = x if x.is_contiguous() else x.contiguous()
         w = weight.detach().to(torch.bfloat16)
         ctx.save_for_backward(xc.view(-1, x.shape[-1]), w)
-        ctx.parameter, ctx.has_bias = weight, bias is not None           # (the parameter: for its gradient slot)
+        # (the parameter for its gradient slot; a weight that was computed is not kept until the backward)
+        ctx.parameter, ctx.has_bias = weight if weight.is_leaf else None, bias is not None
         return hip.linear(xc, w, None if bias is None else bias.detach().to(torch.bfloat16))
 
     @staticmethod

@@ -488,3 +488,21 @@ def test_weight_gradients_into_memory_off_16_bytes(dev, f32, M, N, K):
         got = diff.linear_wgrad(gy, x, out, f32)
         assert got.data_ptr() == out.data_ptr() and torch.equal(out, want)
         assert bool((buf[:off] == 3).all()) and bool((buf[off + M * N:] == 3).all())
+
+
+def test_computed_fp32_weights_are_not_kept_for_the_backward(dev):
+    """A weight that is itself the result of an operation is freed with its last reference, as the backward needs its bf16 copy only."""
+    import weakref
+    from eventgpt_amd.ops.intree_mode import InTreeLinear
+    p, s = torch.nn.Parameter(torch.randn(64, 128, device=dev)), torch.nn.Parameter(torch.randn(64, 1, device=dev))
+    x = torch.randn(32, 128, device=dev)
+    w = p * s
+    with torch.autocast("cuda", dtype=torch.bfloat16), InTreeLinear() as mode:
+        y = F.linear(x, w)
+    assert mode.routed == 1
+    ref = weakref.ref(w)
+    want = y.detach().float().T @ x.bfloat16().float()            # dW of y^2 / 2, up to the products' roundings
+    del w
+    assert ref() is None
+    (y.float().square().sum() / 2).backward()
+    assert float((p.grad - want * s.detach()).norm() / p.grad.norm()) < 1e-4
