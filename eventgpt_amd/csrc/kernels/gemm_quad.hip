@@ -200,7 +200,8 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(GemmParams p) {
         });
         stage ^= STAGE;
       }
-      // the last two K-tiles: staged meanwhile are the next output tile's first two (or zeros that nobody uses)
+      // The last two K-tiles: staged meanwhile are the next output tile's first two, or what nobody uses: nearly all zeros, by a range
+      // that ends with the first row's two K-tiles.  (Not an empty range: less the scalar offset of 128 it need not be empty.)
       left = part ? 0 : 2;
       koff = part ? 128 : -128;
       if (part == 0) {
@@ -208,7 +209,7 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(GemmParams p) {
           locate(t + gridDim.x, nxt);
           la = nxt.a; lw = nxt.w; lba = nxt.bytes_a; lbw = nxt.bytes_w;
         } else {
-          lba = 0; lbw = 0;
+          lba = 256; lbw = 256;
         }
       }
     }

@@ -60,13 +60,15 @@ __global__ __launch_bounds__(512) void gemm_ring_kernel(GemmParams p) {
   const int bytes_a = (min(p.M - m0, BM) * p.lda - k_begin) * 2;
   const int bytes_w = ((p.glu_half ? 2 * p.glu_half - n0 : min(p.N - n0, BN)) * p.ldw - k_begin) * 2;
   int next = 0, into = 0;                     // K-tile staged next and the stage it goes to
-  auto stage = [&]() {                        // (past the last one: zero fills that nobody reads keep the counts uniform)
-    const int la = next < nk ? bytes_a : 0, lw = next < nk ? bytes_w : 0;
+  // Past the last one zero fills that nobody reads keep the counts uniform: an empty range, and with it no offset, so that range minus
+  // offset is empty too.
+  auto stage = [&]() {
+    const int la = next < nk ? bytes_a : 0, lw = next < nk ? bytes_w : 0, off = next < nk ? next * (BK * 2) : 0;
     unsigned char* d = smem + into;
 #pragma unroll
-    for (int i = 0; i < IW; ++i) load_to_lds16(W, lw, d + A_BYTES + (wid * IW + i) * 1024, vw[i], next * (BK * 2));
+    for (int i = 0; i < IW; ++i) load_to_lds16(W, lw, d + A_BYTES + (wid * IW + i) * 1024, vw[i], off);
 #pragma unroll
-    for (int i = 0; i < IA; ++i) load_to_lds16(A, la, d + (wid * IA + i) * 1024, va[i], next * (BK * 2));
+    for (int i = 0; i < IA; ++i) load_to_lds16(A, la, d + (wid * IA + i) * 1024, va[i], off);
     ++next;
     into = into == (S - 1) * STAGE ? 0 : into + STAGE;
   };
