@@ -340,7 +340,7 @@ def test_four_waves_on_the_256_tile(dev, force256, M, N, K, act):
 
 @pytest.mark.parametrize("M,N,K,act", [(577, 3072, 1024, 0), (577, 4096, 1024, 2), (300, 4096, 4096, 0), (257, 2056, 64, 1), (2308, 1024, 1024, 0),
                                        (1154, 3080, 192, 0), (1010, 1000, 256, 1), (160, 9288, 128, 0), (33, 9304, 576, 0),
-                                       (4039, 500, 1088, 0)])
+                                       (4039, 488, 1088, 0)])
 def test_one_round_of_tiles_on_the_deep_ring(dev, M, N, K, act):
     """``gemm_ring.hip`` by the rule that chooses it: all five tiles, ragged rows and columns, fewer K-tiles than its ring, bias, activation and
     residual, gated and as fp32 slabs, against fp32 (``_check``'s bound); the same bits from run to run."""
