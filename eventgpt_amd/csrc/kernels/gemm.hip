@@ -1161,7 +1161,7 @@ void launch_gemm_bf16(const bf16_t* A, const bf16_t* W, bf16_t* C, float* Cf, co
     return;
   }
   if (cfg != CFG_256x256 && g_forced_cfg < 0) {
-    const RingTile ring = gemm_ring_tile(p);
+    const RingTile ring = gemm_ring_tile(p, cfg == CFG_64x128_W8);
     if (ring != RING_NONE) {
       launch_gemm_ring(p, ring, st);
       if (p.splitk > 1) launch_splitk_reduce(p, st);
@@ -1305,7 +1305,7 @@ void launch_gemm_glu(const bf16_t* A, const bf16_t* W, bf16_t* H, int M, int I, 
     }
   }
   if (g_forced_cfg == CFG_256x256 || (g_forced_cfg < 0 && use_256(M, 2 * I, K))) launch_256<false, false>(p, st);
-  else if (const RingTile ring = g_forced_cfg < 0 ? gemm_ring_tile(p) : RING_NONE; ring != RING_NONE)
+  else if (const RingTile ring = g_forced_cfg < 0 ? gemm_ring_tile(p, false) : RING_NONE; ring != RING_NONE)
     launch_gemm_ring(p, ring, st);
   else if (g_forced_cfg == CFG_128x128 || (g_forced_cfg < 0 && tiles(128, 128) >= 384)) launch_cfg<128, 128, 2, 2, 2>(p, st);
   else if (g_forced_cfg == CFG_64x64) launch_cfg<64, 64, 2, 2, 4>(p, st);
@@ -1396,7 +1396,7 @@ int launch_gemm_partial(const bf16_t* A, const bf16_t* W, float* partial, int M,
   const GemmCfg cfg = M > 32 ? pick_cfg(M, N, K) : pick_cfg(M, N);
   g_for_slabs = false;
   if (cfg != CFG_256x256 && g_forced_cfg < 0) {
-    const RingTile ring = gemm_ring_tile(p);
+    const RingTile ring = gemm_ring_tile(p, cfg == CFG_64x128_W8);
     if (ring != RING_NONE) {
       launch_gemm_ring(p, ring, st);
       return p.splitk;

@@ -157,8 +157,8 @@ void launch(const GemmParams& p, hipStream_t st) {
 }  // namespace
 
 // The smallest tile that is one round: a CU's time goes with its tile's area (64 x 128 / 64 x 192 / 128 x 128 with 1024 k 10.7 / 13.7 /
-// 15 us), and 128 x 64 reads the weights half as often as 64 x 128.  Against the tiles of gemm.hip over 1 010 products of 40 to 4 039 rows,
-// 1 024 to 12 288 columns and 512 to 11 008 k, weights from memory: 10 to 25 % ahead at the mean of every tile and length, same bits.
+// 15 us), and 128 x 64 reads the weights half as often as 64 x 128.  Against the tiles of gemm.hip over 22 900 products of 33 to 4 200
+// rows, 64 to 16 384 columns and 64 to 12 288 k, each timed as both: 0.85 of their time at the mean where this rule takes them, same bits.
 // The lines, this / the other choice:
 //  * 64 x 64 from 128 tiles on; not with split K (64 x 1024 x 11008 in eight 12.4 / 10.3 us); under 256 rows up to 1024 k (160 x 3072 x
 //    2048 14.5 / 12.3, x 1024 7.0 / 7.5)
@@ -167,7 +167,15 @@ void launch(const GemmParams& p, hipStream_t st) {
 //  * 128 x 64 over 512 k: from 200 rows on (160 x 5632 6.8 / 6.3)
 //  * 128 x 128: up to 240 tiles (4039 x 1024, 256 of them, 25.8 / 24.8); gated with under 1024 rows from 170 tiles on (636 x 4096 x 4096,
 //    160, 39.7 / 37.5; 400 x 5632 x 4096, 176, 35.4 / 48.1)
-RingTile gemm_ring_tile(const GemmParams& p) {
+//  * short contractions, where filling the ring is what there is, by what the epilogue adds to both (this over the other at the mean):
+//    64 x 64 plain 1.04 at 64 k under 600 rows, 0.95 over 1000, 0.93 at 192; a bias 0.97 and 0.92; a residual 1.05 to 1.13 up to 192 k
+//    below 152 tiles, 0.96 above.  128 x 64 where the other choice is 64 x 64: plain 1.06 at 64, 0.96 at 320 (fp32 and slabs 1.0), a
+//    residual 1.05 and 0.98, with a bias or activation ahead at any length.  Where it is 32 x 64 (under 300 tiles of 64 x 64): a bias
+//    1.11 at 64, 1.0 at 512, quick-gelu 1.04 and 0.92, gelu 1.1 and 1.0, a residual 1.27, 1.09 and at 2048 0.96.
+//    128 x 128: 1.0 to 1.1 up to 320 k, gated 1.02 at 128 and 0.98 at 192
+//  * the eight waves of the 64 x 128 tile (`w8`), which share a CU with two other workgroups, take a bias or an activation sooner than
+//    128 x 128 here (1.08 to 1.14), quick-gelu up to 192 k than 64 x 192 (1.1)
+RingTile gemm_ring_tile(const GemmParams& p, bool w8) {
   const long long lim = 1ll << 31;
   if (p.act != ACT_NONE && p.act != ACT_GELU && p.act != ACT_QUICK_GELU) return RING_NONE;
   if (p.M <= 32 || p.k_cols || p.amax_val || p.rope_cos || p.grp_start) return RING_NONE;
@@ -176,17 +184,30 @@ RingTile gemm_ring_tile(const GemmParams& p) {
     const int out = p.glu_half ? bn / 2 : bn;
     return static_cast<long long>((p.M + bm - 1) / bm) * ((p.N + out - 1) / out) * p.splitk;
   };
-  const bool plain = p.glu_half == 0;
-  long long t = tiles(64, 64);
-  if (t <= 256 && plain) return t >= 128 && p.splitk == 1 && (p.M >= 256 || p.K <= 1024) ? RING_64x64 : RING_NONE;
-  for (const RingTile r : {RING_128x64, RING_64x128}) {
-    t = r == RING_128x64 ? tiles(128, 64) : tiles(64, 128);
-    if (t > 256) continue;
-    return t >= (p.K > 4096 && plain ? 170 : 32) && (p.K > 512 || p.M >= 200 || !plain) ? r : RING_NONE;
+  const bool gated = p.glu_half != 0, slabs = p.splitk > 1 || p.raw_partial;
+  const bool act = !slabs && p.act != ACT_NONE, bias = !slabs && p.bias, res = !slabs && p.res;
+  // longer than what the epilogue asks for
+  auto longer = [&](int residual, int activation, int with_bias, int plain) {
+    return p.k_per_split > (res ? residual : act ? activation : bias ? with_bias : plain);
+  };
+  const long long t64 = tiles(64, 64);
+  if (t64 <= 256 && !gated) {
+    if (t64 < 128 || p.splitk > 1 || (p.M < 256 && p.K > 1024)) return RING_NONE;
+    return longer(t64 < 152 ? 512 : 192, 0, 128, 128) || (p.M > 600 && !res) ? RING_64x64 : RING_NONE;
   }
-  if (plain && tiles(64, 192) <= 256) return p.K <= 4096 ? RING_64x192 : RING_NONE;
-  t = tiles(128, 128);
-  return t <= 240 && (plain || t >= 170 || p.M >= 1024) ? RING_128x128 : RING_NONE;
+  for (const RingTile r : {RING_128x64, RING_64x128}) {
+    const long long t = r == RING_128x64 ? tiles(128, 64) : tiles(64, 128);
+    if (t > 256) continue;
+    if (t < (p.K > 4096 && !gated ? 170 : 32) || (p.K <= 512 && p.M < 200 && !gated)) return RING_NONE;
+    if (gated) return r;
+    const int sums = p.Cf || slabs ? 320 : 192;
+    return (t64 < 300 ? longer(2048, p.act == ACT_GELU ? 1024 : 512, 512, 512) : longer(320, 0, 0, sums)) ? r : RING_NONE;
+  }
+  if (!gated && tiles(64, 192) <= 256)
+    return p.K <= 4096 && !(w8 && p.act == ACT_QUICK_GELU && p.K <= 192) ? RING_64x192 : RING_NONE;
+  const long long t = tiles(128, 128);
+  if (t > 240 || (gated && t < 170 && p.M < 1024) || (w8 && (act || bias))) return RING_NONE;
+  return p.k_per_split > (gated ? 128 : 320) ? RING_128x128 : RING_NONE;
 }
 
 void launch_gemm_ring(const GemmParams& p, RingTile tile, hipStream_t st) {

@@ -1,8 +1,9 @@
-"""The 256 x 256 8-wave GEMM (phase-staggered wave rows) forced onto shapes that exercise its edges:
-rows / columns that do not fill a tile, one K-tile, odd and even K-tile counts, every epilogue, the
-K-strided operand layouts of the backward products; each against an fp32 matmul.  Every case runs
-several times: its synchronisation is counted waits and barriers, so a race would show as a
-difference between repeats."""
+"""The 256 x 256 GEMMs forced onto shapes that exercise their edges: rows / columns that do not fill a tile, one K-tile, odd
+and even K-tile counts, every epilogue, the K-strided operand layouts of the backward products; each against an fp32 matmul.
+A forced product runs on the four waves of ``gemm_quad.hip`` where those take it (K-contiguous operands, two K-tiles or more in every
+split, bf16 output in whole 16-byte chunks or slabs) and on the eight phase-staggered ones of ``gemm256_kernel`` otherwise.  Then the
+tiles of ``gemm_ring.hip``.  Every case runs several times: the synchronisation is counted waits and barriers, so a race would show as
+a difference between repeats."""
 import math
 
 import pytest
@@ -316,7 +317,21 @@ def test_slabs_of_about_a_round_of_tiles(dev, M, N, K, slabs):
     _check(part.sum(0), x.float() @ w.float().t(), K)
 
 
-@pytest.mark.parametrize("M,N,K,act", [(1, 8, 128, 0), (257, 264, 128, 2), (300, 520, 192, 1), (5000, 4104, 128, 0), (5000, 4104, 192, 2),
+def _kernels(fn):
+    """What ``fn`` returns and the names of the kernels it launches."""
+    fn()
+    torch.cuda.synchronize()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        out = fn()
+        torch.cuda.synchronize()
+    return out, [e.key for e in prof.key_averages() if "evgpt" in e.key]
+
+
+def _act(h, act):
+    return (h, torch.nn.functional.gelu(h), h * torch.sigmoid(1.702 * h))[act]
+
+
+@pytest.mark.parametrize("M,N,K,act", [(33, 8, 128, 0), (257, 264, 128, 2), (300, 520, 192, 1), (5000, 4104, 128, 0), (5000, 4104, 192, 2),
                                        (9000, 2056, 320, 0)])
 def test_four_waves_on_the_256_tile(dev, force256, M, N, K, act):
     """``gemm_quad.hip``: two and odd numbers of K-tiles, one and several output tiles a workgroup, ragged rows and columns, every
@@ -324,8 +339,9 @@ def test_four_waves_on_the_256_tile(dev, force256, M, N, K, act):
     x, w = _rand(M, K, dev=dev), _rand(N, K, dev=dev, seed=1, scale=0.05)
     bias, res = _rand(N, dev=dev, seed=2), _rand(M, N, dev=dev, seed=3)
     lin = x.float() @ w.float().t() + bias.float()
-    want = (lin, torch.nn.functional.gelu(lin), lin * torch.sigmoid(1.702 * lin))[act].to(torch.bfloat16).float() + res.float()
-    first = force256.linear(x, w, bias, res, act, False)
+    want = _act(lin, act).to(torch.bfloat16).float() + res.float()
+    first, ran = _kernels(lambda: force256.linear(x, w, bias, res, act, False))
+    assert len(ran) == 1 and "gemm_quad_kernel" in ran[0], ran
     _check(first, want, K)
     for _ in range(3):
         assert torch.equal(force256.linear(x, w, bias, res, act, False), first)
@@ -335,27 +351,107 @@ def test_four_waves_on_the_256_tile(dev, force256, M, N, K, act):
     gu = x.float() @ w[:2 * half].float().t()
     if half >= 16:
         g, u = gu[:, :half].to(torch.bfloat16).float(), gu[:, half:].to(torch.bfloat16).float()
-        _check(force256.linear_swiglu(x, w[:2 * half].contiguous()), torch.nn.functional.silu(g) * u, K)
+        gated, ran = _kernels(lambda: force256.linear_swiglu(x, w[:2 * half].contiguous()))
+        assert len(ran) == 1 and "gemm_quad_kernel" in ran[0], ran
+        _check(gated, torch.nn.functional.silu(g) * u, K)
 
 
-@pytest.mark.parametrize("M,N,K,act", [(577, 3072, 1024, 0), (577, 4096, 1024, 2), (300, 4096, 4096, 0), (257, 2056, 64, 1), (2308, 1024, 1024, 0),
-                                       (1154, 3080, 192, 0), (1010, 1000, 256, 1), (160, 9288, 128, 0), (33, 9304, 576, 0),
-                                       (4039, 488, 1088, 0)])
-def test_one_round_of_tiles_on_the_deep_ring(dev, M, N, K, act):
-    """``gemm_ring.hip`` by the rule that chooses it: all five tiles, ragged rows and columns, fewer K-tiles than its ring, bias, activation and
-    residual, gated and as fp32 slabs, against fp32 (``_check``'s bound); the same bits from run to run."""
+RING = {"64x64": "<2, 1, 2, 4, 4,", "128x64": "<2, 2, 4, 2, 5,", "64x128": "<2, 2, 2, 4, 5,", "64x192": "<2, 3, 2, 4, 4,",
+        "128x128": "<4, 2, 2, 4, 4,"}
+
+
+def _ring_tile(ran):
+    """The tile of ``gemm_ring.hip`` that ran, None: another kernel's."""
+    assert len(ran) == 1, ran
+    return next((t for t, args in RING.items() if "gemm_ring_kernel" + args in ran[0]), None)
+
+
+@pytest.mark.parametrize("act", [0, 1, 2])
+@pytest.mark.parametrize("M,N,K,tile", [(577, 1000, 576, "64x64"), (577, 3080, 1024, "128x64"), (4039, 500, 1088, "128x64"), (576, 3400, 384, "64x128"),
+                                        (577, 4104, 64, "64x192"), (577, 4096, 1024, "64x192"), (1154, 3064, 1088, "128x128"), (257, 9800, 1088, "128x128")])
+def test_one_round_of_tiles_on_the_deep_ring(dev, M, N, K, act, tile):
+    """``gemm_ring.hip`` by the rule that chooses it: all five tiles with bias, every activation and a residual, ragged rows and columns, rows
+    walked along either side of the output, fewer K-tiles than the ring, bf16 and fp32 out, against fp32 (``_check``'s bound); the same bits from
+    run to run."""
     from eventgpt_amd.ops import hip
+    if (tile, K, act) == ("64x192", 64, 2):
+        pytest.skip("eight waves on 64 x 128 take quick-gelu over so short a contraction")
     x, w = _rand(M, K, dev=dev), _rand(N, K, dev=dev, seed=1, scale=0.05)
     bias, res = _rand(N, dev=dev, seed=2), _rand(M, N, dev=dev, seed=3)
     lin = x.float() @ w.float().t()
-    h = lin + bias.float()
-    want = (h, torch.nn.functional.gelu(h), h * torch.sigmoid(1.702 * h))[act].to(torch.bfloat16).float() + res.float()
-    first = hip.raw.linear(x, w, bias, res, act, False)
-    _check(first, want, K)
+    h = _act(lin + bias.float(), act).to(torch.bfloat16).float()
+    first, ran = _kernels(lambda: hip.raw.linear(x, w, bias, res, act, False))
+    assert _ring_tile(ran) == tile, ran
+    _check(first, h + res.float(), K)
     for _ in range(3):
         assert torch.equal(hip.raw.linear(x, w, bias, res, act, False), first)
-    _check(hip.raw.linear(x, w, None, None, 0, True), lin, K)
-    _check(hip.raw.linear_partial(x, w).sum(0), lin, K)
-    half = N // 2 // 32 * 32
-    g, u = lin[:, :half].to(torch.bfloat16).float(), lin[:, half:2 * half].to(torch.bfloat16).float()
-    _check(hip.raw.linear_swiglu(x, w[:2 * half].contiguous()), torch.nn.functional.silu(g) * u, K)
+    y, ran = _kernels(lambda: hip.raw.linear(x, w, bias, None, act, False))
+    assert _ring_tile(ran) == tile, ran
+    _check(y, h, K)
+    if act == 0:
+        y, ran = _kernels(lambda: hip.raw.linear(x, w, None, None, 0, True))
+        assert _ring_tile(ran) == tile, ran
+        _check(y, lin, K)
+
+
+@pytest.mark.parametrize("M,N,K,tile", [(577, 1000, 64, "64x64"), (577, 3080, 64, "128x64"), (576, 3400, 64, "64x128"), (300, 4096, 128, "128x64")])
+def test_activations_over_fewer_k_tiles_than_the_ring(dev, M, N, K, tile):
+    from eventgpt_amd.ops import hip
+    x, w, bias = _rand(M, K, dev=dev), _rand(N, K, dev=dev, seed=1, scale=0.05), _rand(N, dev=dev, seed=2)
+    for act in (1, 2):
+        y, ran = _kernels(lambda: hip.raw.linear(x, w, bias, None, act, False))
+        assert _ring_tile(ran) == tile, ran
+        _check(y, _act(x.float() @ w.float().t() + bias.float(), act), K)
+
+
+@pytest.mark.parametrize("M,N,K,tile", [(577, 1024, 4096, "128x64"), (1154, 1024, 4096, "128x128")])
+def test_split_contractions_on_the_deep_ring(dev, M, N, K, tile):
+    """K in splits, as fp32 slabs and (with the sum's launch) as a finished product."""
+    from eventgpt_amd.ops import hip
+    x, w, bias = _rand(M, K, dev=dev), _rand(N, K, dev=dev, seed=1, scale=0.05), _rand(N, dev=dev, seed=2)
+    lin = x.float() @ w.float().t()
+    slabs, ran = _kernels(lambda: hip.raw.linear_partial(x, w))
+    assert slabs.shape[0] > 1 and _ring_tile(ran) == tile, (slabs.shape, ran)
+    _check(slabs.sum(0), lin, K)
+    assert torch.equal(hip.raw.linear_partial(x, w), slabs)
+    _check(hip.raw.linear(x, w, bias, None, 2, False), _act(lin + bias.float(), 2), K)
+
+
+@pytest.mark.parametrize("M,half,K,tile", [(33, 4640, 576, "128x64"), (577, 1536, 64, "128x64"), (4039, 192, 128, "128x64"), (192, 4160, 1024, "64x128"),
+                                           (1154, 1536, 192, "128x128"), (3000, 480, 256, "128x128"), (300, 5056, 1024, "128x128")])
+def test_gated_products_on_the_deep_ring(dev, M, half, K, tile):
+    from eventgpt_amd.ops import hip
+    x, w = _rand(M, K, dev=dev), _rand(2 * half, K, dev=dev, seed=1, scale=0.05)
+    lin = x.float() @ w.float().t()
+    g, u = lin[:, :half].to(torch.bfloat16).float(), lin[:, half:].to(torch.bfloat16).float()
+    first, ran = _kernels(lambda: hip.raw.linear_swiglu(x, w))
+    assert _ring_tile(ran) == tile, ran
+    _check(first, torch.nn.functional.silu(g) * u, K)
+    for _ in range(3):
+        assert torch.equal(hip.raw.linear_swiglu(x, w), first)
+
+
+@pytest.mark.parametrize("M,N,K,kind,tile", [
+    (577, 3080, 192, "plain", None), (577, 3080, 256, "plain", "128x64"), (577, 3080, 320, "f32", None), (577, 3080, 384, "f32", "128x64"),
+    (577, 3080, 320, "residual", None), (577, 3080, 384, "residual", "128x64"), (577, 3080, 64, "bias", "128x64"),
+    (577, 1664, 512, "bias", None), (577, 1664, 576, "bias", "128x64"), (577, 1664, 2048, "residual", None), (577, 1664, 2112, "residual", "128x64"),
+    (577, 1664, 512, "quick-gelu", None), (577, 1664, 576, "quick-gelu", "128x64"), (577, 1664, 1024, "gelu", None), (577, 1664, 1088, "gelu", "128x64"),
+    (577, 1000, 128, "plain", None), (577, 1000, 192, "plain", "64x64"), (700, 1000, 64, "plain", "64x64"), (577, 1000, 192, "residual", None),
+    (577, 900, 512, "residual", None), (577, 900, 576, "residual", "64x64"), (1154, 3064, 320, "plain", None), (1154, 3064, 384, "plain", "128x128"),
+    (1154, 3064, 1024, "bias", None), (577, 4104, 192, "quick-gelu", None), (577, 4104, 256, "quick-gelu", "64x192")])
+def test_which_products_go_on_the_deep_ring(dev, M, N, K, kind, tile):
+    """Both sides of the lines of ``gemm_ring_tile``: the tile it names runs (None: a kernel of ``gemm.hip``), and the result is bit for bit what a
+    general tile makes of the product."""
+    from eventgpt_amd.ops import hip
+    x, w = _rand(M, K, dev=dev), _rand(N, K, dev=dev, seed=1, scale=0.05)
+    bias, res = _rand(N, dev=dev, seed=2), _rand(M, N, dev=dev, seed=3)
+    fn = dict(plain=lambda: hip.raw.linear(x, w, None, None, 0, False), f32=lambda: hip.raw.linear(x, w, None, None, 0, True),
+              residual=lambda: hip.raw.linear(x, w, None, res, 0, False), bias=lambda: hip.raw.linear(x, w, bias, None, 0, False),
+              gelu=lambda: hip.raw.linear(x, w, bias, None, 1, False))
+    fn["quick-gelu"] = lambda: hip.raw.linear(x, w, bias, None, 2, False)
+    got, ran = _kernels(fn[kind])
+    assert _ring_tile(ran) == tile, ran
+    hip.raw.gemm_force_config(1)
+    other, ran = _kernels(fn[kind])
+    hip.raw.gemm_force_config(-1)
+    assert "gemm_bf16_kernel" in ran[0] and torch.equal(got, other)
