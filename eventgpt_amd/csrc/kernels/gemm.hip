@@ -800,6 +800,11 @@ __global__ __launch_bounds__(512) void gemm256_kernel(GemmParams p) {
   }
 }
 
+enum GemmCfg { CFG_128x128 = 0, CFG_64x128 = 1, CFG_64x64 = 2, CFG_32x64 = 3, CFG_32x128 = 4, CFG_256x256 = 5,
+               CFG_128x256 = 6, CFG_64x128_W8 = 7 };
+
+static int g_forced_cfg = -1;
+void gemm_force_config(int cfg) { g_forced_cfg = cfg; }
 static bool g_use_256 = true;
 void gemm_enable_256(bool on) { g_use_256 = on; }
 static bool g_persist_256 = true;     // false: one workgroup per tile (A/B runs)
@@ -836,7 +841,7 @@ static void launch_256(const GemmParams& p, hipStream_t st, int grp_rows = 0) {
                     (reinterpret_cast<uintptr_t>(p.C) & 15) == 0 &&
                     (!p.res || (reinterpret_cast<uintptr_t>(p.res) & 15) == 0);
   if constexpr (!AT && !BT && BM == 256) {
-    if (gemm_quad_serves(q)) {
+    if (gemm_quad_serves(q) && (g_forced_cfg == CFG_256x256 || gemm_quad_ahead(q, tiles))) {
       launch_gemm_quad(q, grid, st);
       return;
     }
@@ -904,11 +909,6 @@ static void launch_cfg(const GemmParams& p, hipStream_t st) {
 // CUs; shapes that cannot (prefill of a few hundred rows against a 1024- or
 // 4096-wide matrix, verify batches) take smaller tiles with a deeper ring, since
 // a grid below one block per CU is bound by the latency of its own K loop.
-enum GemmCfg { CFG_128x128 = 0, CFG_64x128 = 1, CFG_64x64 = 2, CFG_32x64 = 3, CFG_32x128 = 4, CFG_256x256 = 5,
-               CFG_128x256 = 6, CFG_64x128_W8 = 7 };
-
-static int g_forced_cfg = -1;
-void gemm_force_config(int cfg) { g_forced_cfg = cfg; }
 
 // The 8-wave kernel pays once there are rows to fill 256-row tiles and about half a round of
 // tiles (measured on MI355X, TFLOP/s, 8-wave vs best 4-wave config: 2115 x 4096 x 11008, 144 tiles,

@@ -334,6 +334,21 @@ bool gemm_quad_serves(const GemmParams& p) {
   return (reinterpret_cast<uintptr_t>(p.bias) & 7) == 0 && (p.act == ACT_NONE || p.act == ACT_GELU || p.act == ACT_QUICK_GELU);
 }
 
+// Over short contractions its ends, longer than the 8-wave kernel's, are what there is; that kernel's own end is the longer one with a bias or
+// an activation (a choice among all of them).  Its time over the 8-wave kernel's at the mean of 13 200 products of 768 to 9 000 rows, up to 256
+// tiles and more, K = 128 / 448 / 768 / 1024 / 1536 / 2048:
+//  * plain 1.08 / 1.04 / 1.00 / 0.98 / 0.97 / 0.97 and 1.00 / 0.97 / 0.96 / 0.96 / 0.96 / 0.96
+//  * slabs 1.06 / 1.04 / 1.03 / 1.02 / 1.00 / 0.97 and 1.00 / 0.96 / 0.96 / 0.96 / 0.94 / 0.94
+//  * gated 1.08 / 1.05 / 1.04 / 1.03 / 1.00 / 0.98 and 1.06 / 1.02 / 1.01 / 0.99 / 0.98 / 0.97
+//  * a residual 1.00 to 0.96 and 0.96 to 0.94, a bias 0.80 to 0.86, gelu 0.88 to 0.94, quick-gelu 0.70 to 0.80
+bool gemm_quad_ahead(const GemmParams& p, int tiles) {
+  const int k = p.k_per_split;
+  const bool many = tiles > 256;
+  if (p.glu_half) return k > (many ? 768 : 1024);
+  if (p.splitk > 1 || p.raw_partial) return k > (many ? 192 : 1024);
+  return p.bias || p.res || p.act != ACT_NONE || k > (many ? 192 : 576);
+}
+
 void launch_gemm_quad(const GemmParams& p, int grid, hipStream_t st) {
   if (p.grp_start) launch<true>(p, grid, st);
   else if (p.splitk > 1 || p.raw_partial || p.act == ACT_NONE) launch<false>(p, grid, st);

@@ -356,6 +356,35 @@ def test_four_waves_on_the_256_tile(dev, force256, M, N, K, act):
         _check(gated, torch.nn.functional.silu(g) * u, K)
 
 
+@pytest.mark.parametrize("M,N,K,kind,quad", [
+    (2600, 5120, 576, "plain", False), (2600, 5120, 640, "plain", True), (2600, 9216, 192, "plain", False), (2600, 9216, 256, "plain", True),
+    (2600, 5120, 1024, "slabs", False), (2600, 5120, 1088, "slabs", True), (2600, 9216, 192, "slabs", False), (2600, 9216, 256, "slabs", True),
+    (2600, 5120, 1024, "gated", False), (2600, 5120, 1088, "gated", True), (2600, 9216, 768, "gated", False), (2600, 9216, 832, "gated", True),
+    (2600, 5120, 128, "residual", True), (2600, 5120, 128, "bias", True), (2600, 5120, 128, "gelu", True), (2600, 5120, 64, "bias", False)])
+def test_which_kernel_takes_256_tiles(dev, M, N, K, kind, quad):
+    """Both sides of every line of ``gemm_quad_ahead``: the kernel it names runs, and its result is right and what the tiles forced onto the
+    other kernel's shapes give (``_check``'s bound; plain, bias and residual bit for bit what the general tiles make of the product)."""
+    from eventgpt_amd.ops import hip
+    x, w = _rand(M, K, dev=dev), _rand(N, K, dev=dev, seed=1, scale=0.05)
+    bias, res = _rand(N, dev=dev, seed=2), _rand(M, N, dev=dev, seed=3)
+    fn = dict(plain=lambda: hip.raw.linear(x, w, None, None, 0, False), slabs=lambda: hip.raw.linear_partial(x, w),
+              gated=lambda: hip.raw.linear_swiglu(x, w), residual=lambda: hip.raw.linear(x, w, None, res, 0, False),
+              bias=lambda: hip.raw.linear(x, w, bias, None, 0, False), gelu=lambda: hip.raw.linear(x, w, bias, None, 1, False))[kind]
+    got, ran = _kernels(fn)
+    assert len(ran) == 1 and ("gemm_quad_kernel" if quad else "gemm256_kernel") in ran[0], ran
+    lin = x.float() @ w.float().t()
+    half = N // 2
+    want = dict(plain=lambda: lin, slabs=lambda: lin, residual=lambda: lin.to(torch.bfloat16).float() + res.float(),
+                bias=lambda: lin + bias.float(), gelu=lambda: _act(lin + bias.float(), 1),
+                gated=lambda: torch.nn.functional.silu(lin[:, :half].to(torch.bfloat16).float()) * lin[:, half:].to(torch.bfloat16).float())[kind]()
+    _check(got.sum(0) if kind == "slabs" else got, want, K)
+    if kind in ("plain", "bias", "residual"):
+        hip.raw.gemm_force_config(0)
+        other, ran = _kernels(fn)
+        hip.raw.gemm_force_config(-1)
+        assert "gemm_bf16_kernel" in ran[0] and torch.equal(got, other)
+
+
 RING = {"64x64": "<2, 1, 2, 4, 4,", "128x64": "<2, 2, 4, 2, 5,", "64x128": "<2, 2, 2, 4, 5,", "64x192": "<2, 3, 2, 4, 4,",
         "128x128": "<4, 2, 2, 4, 4,"}
 
