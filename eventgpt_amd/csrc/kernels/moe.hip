@@ -1,5 +1,5 @@
 // Mixture of experts: routing, sorting of a prompt's tokens by expert, and the two products of a decode step of a
-// few rows.  The grouped matrix products of a prompt are instances of gemm.hip (bf16) and gemm_f32.hip.
+// few rows.  The grouped products of more rows are gemm_grouped.hip's, gemm_quad.hip's and instances of gemm.hip (bf16) and gemm_f32.hip.
 //
 // Routing is fp32: the `top` largest of logits + bias, the lower index of equals first, softmax over the chosen.
 // A decode step reads only the chosen experts' weights: every workgroup routes its row again from the logits (a few
@@ -100,10 +100,10 @@ void launch_moe_group(const int* idx, int* perm, int* inv, int* start, int n, in
   hipLaunchKernelGGL(moe_group_kernel, dim3(E), dim3(1024), 0, st, idx, perm, inv, start, n, E);
 }
 
-// Routing and sorting of a decode step's rows in one launch (32 rows of 8 experts: 7.3-8.1 us, two launches 4.7 + 5.1 and what lies between): a wave
-// per row, then a wave per expert counts and places its entries with ballots.  One workgroup routes sixteen rows at a time, one after the other:
-// 300 rows take 60 us more than the two launches, which spread over the chip.
-constexpr int RG_ROWS = 48, RG_ENTRIES = 1024, RG_EXPERTS = 256;
+// Routing and sorting of a decode step's rows in one launch: a wave per row, then a wave per expert counts and places its entries with
+// ballots.  One workgroup routes sixteen rows at a time and sorts sixteen experts at a time, one after the other, where the two launches spread
+// over the chip: see moe_route_group_ok.
+constexpr int RG_ROWS = 32, RG_ENTRIES = 128, RG_EXPERTS = 32;
 __global__ __launch_bounds__(1024) void moe_route_group_kernel(MoeRoute a, float* __restrict__ w, int* __restrict__ perm, int* __restrict__ inv,
                                                                int* __restrict__ start, int rows) {
   extern __shared__ float z[];                     // [16][E]
@@ -145,7 +145,13 @@ __global__ __launch_bounds__(1024) void moe_route_group_kernel(MoeRoute a, float
     }
   }
 }
-bool moe_route_group_ok(int rows, int E, int top) { return rows <= RG_ROWS && rows * top <= RG_ENTRIES && E <= RG_EXPERTS; }
+// Two launches / this, us: 16 rows of 8 experts, one, two, four and eight chosen 5.8 / 3.7, 6.4 / 4.5, 7.6 / 6.0, 10.1 / 9.3; of 32 experts 5.7 / 4.5, 6.4 /
+// 5.3, 7.6 / 6.9, 10.0 / 10.4, six 8.8 / 8.8; of 64 5.8 / 5.7, 6.4 / 6.5, 7.5 / 8.1.  32 rows of 8 to 16: one or two chosen 5.8 / 5.1 and 6.5 / 6.6,
+// three 7.2 / 8.3; of 32: one 5.8 / 5.9, two 6.5 / 7.4.  36 rows of 8, two chosen: 6.5 / 7.8; 48 rows of 64, eight chosen: 10.2 / 28.9.
+bool moe_route_group_ok(int rows, int E, int top) {
+  if (rows > RG_ROWS || E > RG_EXPERTS) return false;
+  return top <= (rows <= 16 ? (E <= 16 ? 8 : 6) : (E <= 16 ? 2 : 1));
+}
 void launch_moe_route_group(const MoeRoute& r, float* w, int* perm, int* inv, int* start, int rows, hipStream_t st) {
   hipLaunchKernelGGL(moe_route_group_kernel, dim3(1), dim3(1024), 64 * r.E, st, r, w, perm, inv, start, rows);
 }

@@ -294,15 +294,27 @@ def test_routing(raw, dev, E, top):
     assert int(idx.min()) >= 0 and int(idx.max()) < E and all(len(set(r)) == top for r in idx.tolist())
 
 
-@pytest.mark.parametrize("M,E,top", [(1, 1, 1), (32, 8, 2), (17, 70, 3), (48, 256, 21), (49, 8, 2), (40, 300, 40), (48, 64, 22), (300, 8, 2)])
-def test_routing_and_sorting_in_one_launch(raw, dev, M, E, top):
-    """What ``moe_route`` and ``moe_group`` give, bit for bit: around its bounds of rows, entries and experts, slabs, ties and rows without a number."""
+def _kernels(fn):
+    """What ``fn`` returns and the names of the kernels it launches."""
+    fn()
+    torch.cuda.synchronize()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        out = fn()
+        torch.cuda.synchronize()
+    return out, [e.key for e in prof.key_averages() if "evgpt" in e.key]
+
+
+@pytest.mark.parametrize("M,E,top,launches", [(1, 1, 1, 1), (16, 16, 8, 1), (16, 16, 9, 2), (16, 32, 6, 1), (13, 32, 7, 2), (16, 33, 2, 2), (17, 8, 2, 1), (32, 16, 2, 1),
+                                              (32, 8, 3, 2), (32, 17, 2, 2), (32, 32, 1, 1), (33, 8, 1, 2), (17, 70, 3, 2), (48, 256, 21, 2), (40, 300, 40, 2), (300, 8, 2, 2)])
+def test_routing_and_sorting_in_one_launch(raw, dev, M, E, top, launches):
+    """What ``moe_route`` and ``moe_group`` give, bit for bit: around its bounds of rows, experts and chosen ones, slabs, ties and rows without a number."""
     z, b = rnd(M, -(-E // 8) * 8).float(), rnd(E, seed=1).float().to(dev)
     z[M // 2:M // 2 + 2] = 0.5
     z[M // 3] = float("nan")
     for logits in (z.to(dev), torch.stack([z, z]).to(dev)):
         idx, want = raw.moe_route(logits, b, top)
-        w, perm, inv, start = raw.moe_route_group(logits, b, top)
+        (w, perm, inv, start), ran = _kernels(lambda: raw.moe_route_group(logits, b, top))
+        assert len(ran) == launches, ran
         assert torch.equal(w, want)
         for got, ref in zip((perm, inv, start), raw.moe_group(idx, E)):
             assert torch.equal(got, ref)
