@@ -6,9 +6,8 @@
 // two pairs of waves (704 and 512 workgroups), in K-tiles of 128, 256 contiguous bytes of a weight row each; rows that a group
 // does not have are neither fetched nor, past the first 16, multiplied.
 //
-// us, general tile -> this, weights from memory, 8 experts of 4096 x 5504 (two a row): gate / up 16 rows 149 -> 133, 32 rows 144 -> 132 (721 MB:
-// 5.5 TB/s), down 98 -> 73 and 94 -> 75; of 2048 x 2816: down 22.3 -> 21.1 and 22.8 -> 21.9, gate / up see the rule below.
-// Two stages: gate / up 155, down 94; four: down level.
+// us, general tile -> this, weights from memory, 8 experts of 4096 x 5504 (two a row, 8 to 64 rows): gate / up 139 -> 128 (721 MB: 5.6 TB/s),
+// down 92 -> 75; of 2048 x 2816 42.7 -> 40.0 and 23.0 -> 18.1.  Two stages: gate / up 155, down 94 where three take 132 and 75; four: down level.
 #include <type_traits>
 
 #include "gemm_common.h"
@@ -17,7 +16,7 @@ namespace evgpt {
 
 namespace {
 
-constexpr int TK = 128, AM = 32, TN = 32, STAGES = 3;
+constexpr int TK = 128, AM = 32, TN = 32, STAGES = 3, RUN = 16;
 
 template <bool GLU>
 __global__ __launch_bounds__(256) void gemm_grouped_few_kernel(GemmParams p) {
@@ -26,7 +25,12 @@ __global__ __launch_bounds__(256) void gemm_grouped_few_kernel(GemmParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int tiles_n = p.N / TN;
-  int tile = xcd_remap(blockIdx.x, gridDim.x);
+  // The XCDs take turns in runs of sixteen tiles: the grid is for the most tiles there can be, and cut into eight ranges it left the last XCDs
+  // those that there are not (no more rows than experts: 0.66 of the general tile's time at the mean, in ranges 0.93; gated 0.69 and 0.98).
+  // Ranges of the tiles there are lie a power of two apart for many shapes and meet in the same channels (0.67, more rows than experts
+  // level), single tiles read 4096 k slower than runs do (0.85 against 0.79).
+  const int xcd = blockIdx.x & 7, turn = blockIdx.x >> 3;
+  int tile = ((turn / RUN) * 8 + xcd) * RUN + turn % RUN;
   const int e = group_of_tile(p.grp_start, p.grp_count, AM, tiles_n, tile);
   if (e < 0) return;
   const int first = p.grp_start[e], all = p.grp_start[e + 1] - first;
@@ -126,28 +130,31 @@ __global__ __launch_bounds__(256) void gemm_grouped_few_kernel(GemmParams p) {
 }
 
 template <bool GLU>
-void launch(const GemmParams& p, int tiles, hipStream_t st) {
+void launch(const GemmParams& p, int grid, hipStream_t st) {
   constexpr int smem = STAGES * (AM + (GLU ? 2 * TN : TN)) * TK * 2;
   static const bool attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_grouped_few_kernel<GLU>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, smem) == hipSuccess;
   (void)attr;
-  hipLaunchKernelGGL((gemm_grouped_few_kernel<GLU>), dim3(tiles), dim3(256), smem, st, p);
+  hipLaunchKernelGGL((gemm_grouped_few_kernel<GLU>), dim3(grid), dim3(256), smem, st, p);
 }
 
 }  // namespace
 
-// Up to 16 rows an average group: 24 (96 rows, two experts each) down 25.4 vs 30.6 us.  The gated tiles come two to a CU, 512 a round: 704 of them
-// (2048 x 2816) are level with the 32 x 128 tile or up to 4 % behind from 16 rows on, 1376 (4096 x 5504) ahead by 9 %; with fewer than four
-// rows a group some groups are empty and they are ahead anyway (8 rows 39.7 -> 36.5, 5 rows 36.0 -> 32.6).
+// Up to 16 rows an average group: 24 (96 rows, two experts each) down 25.4 vs 30.6 us.  Time over the general tile's at the mean of 11 600
+// products of 2 to 32 experts, 512 to 5 504 k, 512 to 9 000 columns, rows dealt at random, weights from memory: 0.78 and gated 0.84, 2 % of
+// them behind by more than 2.5 %.  Not the gated ones of 257 to 384 workgroups (groups x columns / 32: over a round of one a CU, most CUs with one)
+// and more rows than groups, 0.94 at the mean and a fifth of them behind; up to 256 are at 0.80, up to 512 at 0.84.
 bool gemm_grouped_few_serves(const GemmParams& p, int rows) {
   if (p.K % TK || p.N % TN || p.ldc % 4 || rows > 16 * p.grp_count) return false;
-  return !p.glu_half || rows < 4 * p.grp_count || p.grp_count * (p.N / TN) > 1024;
+  const int most = p.grp_count * (p.N / TN);
+  return !p.glu_half || rows <= p.grp_count || most <= 256 || most > 384;
 }
 
 void launch_gemm_grouped_few(const GemmParams& p, int rows, hipStream_t st) {
-  const int tiles = (rows / AM + p.grp_count) * (p.N / TN);       // at least as many as there can be
-  if (p.glu_half) launch<true>(p, tiles, st);
-  else launch<false>(p, tiles, st);
+  const int most = (rows / AM + p.grp_count) * (p.N / TN);        // at least as many as there can be
+  const int grid = (most + 8 * RUN - 1) / (8 * RUN) * (8 * RUN);  // every XCD's whole turns
+  if (p.glu_half) launch<true>(p, grid, st);
+  else launch<false>(p, grid, st);
 }
 
 }  // namespace evgpt

@@ -340,6 +340,11 @@ def test_sorting_by_expert(raw, dev, M, E, top):
 def test_grouped_products(raw, dev, dtype, counts, K, N):
     """Every tile size (by the average group), more tiles than workgroups, empty and uneven groups, gathered and consecutive
     rows, all activations."""
+    _grouped_products(raw, dev, dtype, counts, K, N)
+
+
+def _grouped_products(raw, dev, dtype, counts, K, N, plain=None, gated=None):
+    """``plain`` / ``gated``: the kernel that is meant to run."""
     E, top = len(counts), 2
     rows = sum(counts)
     M = -(-rows // top)
@@ -353,23 +358,42 @@ def test_grouped_products(raw, dev, dtype, counts, K, N):
 
     def grouped(a):
         return torch.cat([a[start[e]:start[e + 1]] @ wr[e].T for e in range(E)])
+
+    def run(name, *args):
+        got, ran = _kernels(lambda: raw.moe_linear(*args)) if name else (raw.moe_linear(*args), None)
+        assert not name or (len(ran) == 1 and name in ran[0]), ran
+        return got
     y = grouped(xr[perm // top])
     tol = 2e-6 if dtype == F32 else 8e-3
-    assert Z.rel_err(raw.moe_linear(x, w, st, pm, top, -1), y) < tol
+    assert Z.rel_err(run(plain, x, w, st, pm, top, -1), y) < tol
     g, u = y.chunk(2, -1)
-    assert Z.rel_err(raw.moe_linear(x, w, st, pm, top, SILU), oracle.silu(g) * u) < 2 * tol
+    assert Z.rel_err(run(gated, x, w, st, pm, top, SILU), oracle.silu(g) * u) < 2 * tol
     gelu = torch.nn.functional.gelu(g, approximate="tanh")
-    assert Z.rel_err(raw.moe_linear(x, w, st, pm, top, GELU), gelu * u) < 2 * tol
+    assert Z.rel_err(run(gated, x, w, st, pm, top, GELU), gelu * u) < 2 * tol
     full, fr = typed(rnd(rows, K, seed=2), dtype, dev)
-    assert Z.rel_err(raw.moe_linear(full, w, st, None, 1, -1), grouped(fr)) < tol
+    assert Z.rel_err(run(plain, full, w, st, None, 1, -1), grouped(fr)) < tol
 
 
-@pytest.mark.parametrize("counts,K,N", [([1, 0, 17, 33, 5, 0, 16, 32], 128, 64), ([3, 0, 1, 2], 384, 192), ([16] * 8, 2048, 8256),
-                                        ([0, 65, 0, 1], 256, 128), ([2], 640, 64)])
-def test_grouped_products_of_a_few_rows(raw, dev, counts, K, N):
-    """``gemm_grouped.hip``: groups of none, one, 16, 17, 32, 33 and 65 rows, one K-tile and more than its ring, both products.
+@pytest.mark.parametrize("counts,K,N,gated", [
+    ([1, 0, 17, 33, 5, 0, 16, 32], 128, 64, True), ([3, 0, 1, 2], 384, 192, True), ([16] * 8, 2048, 8256, True), ([0, 65, 0, 1, 14], 256, 128, True),
+    ([2], 640, 64, True), ([65, 0, 33, 17, 1, 0, 12, 0], 1152, 8256, True), ([17, 0, 33, 32] + [1] * 20, 512, 1088, True),
+    ([0, 1, 0, 0, 2, 0, 0, 0, 1, 0, 0, 0], 256, 2048, True), ([4] * 8, 256, 2688, False), ([4] * 8, 256, 3200, True), ([0] * 70 + [2], 128, 64, True)])
+def test_grouped_products_of_a_few_rows(raw, dev, counts, K, N, gated):
+    """``gemm_grouped.hip``: groups of none, one, 16, 17, 32, 33 and 65 rows, one K-tile and more than its ring, more tiles than a turn of the XCDs,
+    both products; gated ones of 257 to 384 workgroups are the general tile's.
     Sums of K products in bf16 operands: what is stored is rounded once (2^-9), the gate's two factors before that."""
-    test_grouped_products(raw, dev, BF16, list(counts), K, N)
+    _grouped_products(raw, dev, BF16, list(counts), K, N, "gemm_grouped_few_kernel", "gemm_grouped_few_kernel" if gated else "gemm_bf16_kernel")
+
+
+@pytest.mark.parametrize("counts,K,N,plain,gated", [
+    ([1800, 1500], 192, 4736, "gemm256_kernel", "gemm256_kernel"), ([1800, 1500], 320, 4736, "gemm_quad_kernel", "gemm256_kernel"),
+    ([2050, 0, 1270, 900], 832, 4736, "gemm_quad_kernel", "gemm_quad_kernel"), ([5, 3100], 896, 4736, "gemm_quad_kernel", "gemm_quad_kernel"),
+    ([900, 800], 1088, 1024, "gemm_quad_kernel", "gemm_quad_kernel")])
+def test_grouped_products_of_many_rows(raw, dev, counts, K, N, plain, gated):
+    """256-row tiles of groups on both kernels that have them: more tiles than workgroups, so that a workgroup's next tile belongs to another group
+    whose first K-tiles are staged under this one's last; odd and even numbers of K-tiles, an empty group, one of a few rows, gathered and consecutive
+    rows, gated."""
+    _grouped_products(raw, dev, BF16, list(counts), K, N, plain, gated)
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
