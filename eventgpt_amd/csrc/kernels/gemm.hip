@@ -518,10 +518,11 @@ static void launch_fewrow(const GemmParams& p, hipStream_t st) {
 
 // ---------------------------------------------------------------------------------------
 // 256 x 256 x 64 tile, 8 waves (2 x 4, each 128 x 64 of C), one workgroup per CU: the kernel
-// for GEMMs with thousands of rows whose operands are K-strided or whose output gemm_quad.hip
-// does not store.  The 4-wave kernel above stops near 900 TFLOP/s however it is pipelined, because one wave per SIMD has to alternate between feeding the LDS pipe and
-// the MFMA pipe; here each SIMD holds two waves that run HALF A PHASE APART, so one issues
-// MFMAs while the other issues its LDS reads and the staging loads.
+// for GEMMs with thousands of rows whose operands are K-strided, whose output gemm_quad.hip does
+// not store, or whose contraction is too short for it (gemm_quad_ahead).  The 4-wave kernel above
+// stops near 900 TFLOP/s however it is pipelined, because one wave per SIMD has to alternate
+// between feeding the LDS pipe and the MFMA pipe; here each SIMD holds two waves that run HALF A
+// PHASE APART, so one issues MFMAs while the other issues its LDS reads and the staging loads.
 //
 // A K-tile is four phases; a phase is  [LDS reads + staging loads] barrier [16 MFMAs] barrier.
 // The two wave rows (wr = 0 / 1) are offset by one barrier: wr = 1 passes one extra barrier
@@ -800,11 +801,16 @@ __global__ __launch_bounds__(512) void gemm256_kernel(GemmParams p) {
   }
 }
 
+// Tile choice: the largest tile that still puts >= ~1.5 blocks on each of the 256
+// CUs; shapes that cannot (prefill of a few hundred rows against a 1024- or
+// 4096-wide matrix, verify batches) take smaller tiles with a deeper ring, since
+// a grid below one block per CU is bound by the latency of its own K loop.
 enum GemmCfg { CFG_128x128 = 0, CFG_64x128 = 1, CFG_64x64 = 2, CFG_32x64 = 3, CFG_32x128 = 4, CFG_256x256 = 5,
                CFG_128x256 = 6, CFG_64x128_W8 = 7 };
 
 static int g_forced_cfg = -1;
 void gemm_force_config(int cfg) { g_forced_cfg = cfg; }
+
 static bool g_use_256 = true;
 void gemm_enable_256(bool on) { g_use_256 = on; }
 static bool g_persist_256 = true;     // false: one workgroup per tile (A/B runs)
@@ -905,15 +911,13 @@ static void launch_cfg(const GemmParams& p, hipStream_t st) {
                      smem, st, q);
 }
 
-// Tile choice: the largest tile that still puts >= ~1.5 blocks on each of the 256
-// CUs; shapes that cannot (prefill of a few hundred rows against a 1024- or
-// 4096-wide matrix, verify batches) take smaller tiles with a deeper ring, since
-// a grid below one block per CU is bound by the latency of its own K loop.
-
-// The 8-wave kernel pays once there are rows to fill 256-row tiles and about half a round of
-// tiles (measured on MI355X, TFLOP/s, 8-wave vs best 4-wave config: 2115 x 4096 x 11008, 144 tiles,
-// 913 vs 751; 4643 x 12288 x 4096 1190 vs 930; 20352 x 4096 x 4096 1230 vs 905; but 636 rows 717 vs
-// 948 and 2885 x 1024 x 4096, 48 tiles, 282 vs 567).
+// 256 x 256 tiles pay once there are rows to fill them and about half a round of tiles.  With the 8-wave kernel (measured on
+// MI355X, TFLOP/s, 8-wave vs best 4-wave config): 2115 x 4096 x 11008, 144 tiles, 913 vs 751; 4643 x 12288 x 4096 1190 vs 930;
+// 20352 x 4096 x 4096 1230 vs 905; but 636 rows 717 vs 948 and 2885 x 1024 x 4096, 48 tiles, 282 vs 567.
+// The lines are that kernel's.  Where gemm_quad.hip takes the tiles, us, 256 x 256 / the other choice: 2115 x 4096 x 4096, 144 tiles,
+// 76 / 107, x 2048 45 / 53; 1024 x 9216 x 1024 30 / 36; 836 x 10240 x 1024, 160, 29 / 37; behind at 128 tiles of 1024 x 8192 x 4096 81 /
+// 73.  Some that the lines leave out would gain: 768 x 12288 x 4096, 144 tiles, 127 where it would be 78; 768 x 11008 x 4096, 129, 108
+// and 78; with a residual 3840 x 2304 x 1024, 135, 45 and 32.
 // K (0 = not known to the caller): a 256 x 256 tile's prologue and epilogue are one workgroup's alone (one per
 // CU), so over a short contraction the 4-wave 128 x 128 tile -- two workgroups per CU, each hiding the other's
 // ends -- is ahead.  With the grouped tile walk, TFLOP/s 8-wave vs 128 x 128: 23080 x 3072 x 1024 782 vs 816,
@@ -944,9 +948,11 @@ static bool use_256(int M, int N, int K = 0) {
 //  * more than a round where the 128 x 128 tile takes one (512): ahead up to K = 320 (1.03 to 1.15; with 256 rows, whose few row
 //    tiles share a weight tile, 0.96), behind from there to 256 x 32000 x 1024 46.0 vs 33.0, 1000 x 8192 x 1024 40.0 vs 29.8, 2308 x
 //    3072 x 1024 32.0 vs 28.3; with an activation, whose epilogue more waves take, level at K = 640, behind from 768 (836 x 8192 0.87)
-//  * where that takes two: ahead (3300 x 2560 x 1024, 520 tiles of it, 1.33) unless the 8-wave kernel has more than 152 tiles
-//    of a round to itself: 140 to 152 of them 1.09 to 1.19, 172 to 192 0.84 to 1.0; with an activation 1.09 to 1.5 up to 199
-//  * a residual, which that kernel's epilogue reads in whole lines, keeps it ahead of this tile: 0.81 to 0.95
+//  * where that takes two: ahead (3300 x 2560 x 1024, 520 tiles of it, 1.33) unless the 256 x 256 tile has more than 152 tiles
+//    of a round to itself.  With the 8-wave kernel 140 to 152 of them 1.09 to 1.19, 172 to 192 0.84 to 1.0, with an activation 1.09 to
+//    1.5 up to 199; gemm_quad.hip brought that to 0.92 (2115 x 4096 x 1024, 144) and, with gelu, 1.09 at 144, 0.96 at 192 (2885 x 4096)
+//    and 0.85 at 172 (1024 x 11008)
+//  * a residual, which those tiles' epilogue reads in whole lines, keeps them ahead of this one: 0.81 to 0.95
 static bool use_64x128_w8(int M, int N, int K, bool act, bool res) {
   auto tiles = [&](int bm, int bn) {
     return static_cast<long long>((M + bm - 1) / bm) * ((N + bn - 1) / bn);
@@ -975,10 +981,11 @@ static thread_local bool g_for_slabs = false;
 
 // 768..1024 rows into a few thousand columns over a long contraction (one ~840-token sample against
 // the 4096-wide matrices with K = 11008 / 12288 / 22016): 48..128 tiles of 256x256 are a fraction of a
-// round, but with K split over the rest of the round the 8-wave kernel is ahead of every 4-wave
+// round, but with K split over the rest of the round 256 x 256 tiles are ahead of every 4-wave
 // choice (benchmarks/bench_gemm_splitk256.py, TFLOP/s, 4 splits vs the best 4-wave configuration:
 // 836x4096x11008 878 vs 811, x12288 926 vs 844, x22016 1038 vs 871; at 636 rows -- three row tiles,
-// a quarter of the last one used -- it is behind, 725 vs 807).  Returns the split count, or 0.
+// a quarter of the last one used -- it is behind, 725 vs 807).  With gemm_quad.hip, us, so / the other choice: 836 x 4096 x 11008 83 / 95,
+// x 22016 144 / 177, 1000 rows x 11008 88 / 136; behind at 128 tiles in two splits, 1024 x 8192 x 8192 152 / 136.  Returns the split count, or 0.
 static int narrow_256_splits(int M, int N, int K) {
   if (!g_use_256 || g_forced_cfg >= 0 || g_forced_splitk > 0 || M < 768 || M > 1024 || K < 8192) return 0;
   const long long t = static_cast<long long>((M + 255) / 256) * ((N + 255) / 256);
@@ -1042,9 +1049,10 @@ int gemm_splitk(int M, int N, int K) {
     if (M > 1024) {
       // A single partial round of 256 x 256 tiles over a long contraction: with K split s ways the tiles
       // make ceil(t s / 256) rounds of 1 / s the length.  Taken when that model promises a third off and
-      // s <= 3 (the fp32 slabs cost about one more pass over the output per split): 2115 x 4096 x 11008,
-      // 144 tiles, s = 3: 231-262 -> 209 us; 1500 rows, 96 tiles, s = 2: 152 -> 130 us; 2885 rows, 192
-      // tiles: every split count measures behind and the model agrees.
+      // s <= 3 (the fp32 slabs cost about one more pass over the output per split).  us, split / not: 1800 x 4096 x
+      // 11008, 128 tiles, s = 2, 145 / 190, slabs 129 / 192; 2115 rows, 144, s = 3, 198 / 197 (with the 8-wave kernel 209 /
+      // 231-262), slabs 176 / 189; 2600 x 3072, 132, s = 3, 206 / 183, slabs 187 / 185; 192 tiles: every split count measures
+      // behind and the model agrees.
       if (g_tail_splitk && K >= 8192 && use_256(M, N, K)) {
         const long long t = static_cast<long long>((M + 255) / 256) * ((N + 255) / 256);
         if (t < 256) {
@@ -1093,11 +1101,13 @@ int gemm_splitk(int M, int N, int K) {
   return sk < 2 ? 1 : sk;
 }
 
-// One workgroup per CU means whole rounds of 256 tiles.  When the 8-wave kernel's last round would be
+// One workgroup per CU means whole rounds of 256 tiles.  When the 256 x 256 kernels' last round would be
 // under half full (and there are only one or two full rounds for it to hide behind), the columns of the
-// whole rounds (n1) go first and the remaining ones are a second launch: on the 4-wave kernel, or --
-// *tail_s >= 2, contraction long enough -- on the 8-wave kernel again with K split tail_s ways so that
-// the few tiles spread over the idle CUs (4643 x 4096 x 11008: 304 tiles = 247 + 57 x 4 splits).
+// whole rounds (n1) go first and the remaining ones are a second launch: on the 128 x 128 tile, or --
+// *tail_s >= 2, contraction long enough -- on 256 x 256 again with K split tail_s ways so that the few
+// tiles spread over the idle CUs (4643 x 4096 x 11008: 304 tiles = 247 + 57 x 4 splits).  us, so / the 128 x 128 tile
+// for the rest / one launch: 304 tiles x 11008 328 / 388 / 412, x 4096 145 / 156 / 161; 266 tiles x 4096 131 / 156 / 159; two rounds and
+// 96 tiles 636 / 639 / 666; over 1024 k, on the 128 x 128 tile, 266 tiles 51 / 54, 304 56 / 56, 608 88 / 86.
 static bool last_round_split(int M, int N, int K, int* n1, int* tail_s) {
   const int tiles_m = (M + 255) / 256, tiles_n = (N + 255) / 256;
   const long long total = static_cast<long long>(tiles_m) * tiles_n;
@@ -1170,8 +1180,8 @@ void launch_gemm_bf16(const bf16_t* A, const bf16_t* W, bf16_t* C, float* Cf, co
   }
   // One workgroup per CU means whole rounds of 256 tiles: a grid of 304 tiles takes as long as
   // one of 512.  When the last round would be under half full (and there are few rounds for it
-  // to hide in), the 8-wave kernel takes the columns that make whole rounds and the 4-wave
-  // kernel, several blocks per CU, the remaining ones.
+  // to hide in), the 256 x 256 kernels take the columns that make whole rounds and the rest goes as
+  // last_round_split says.
   if (cfg == CFG_256x256 && g_forced_cfg < 0 && p.splitk == 1 && !amax_val) {
     int n1 = 0, tail_s = 0;
     if (last_round_split(M, N, K, &n1, &tail_s)) {
@@ -1185,7 +1195,7 @@ void launch_gemm_bf16(const bf16_t* A, const bf16_t* W, bf16_t* C, float* Cf, co
       if (res) b.res = res + n1;
       launch_256<false, false>(a, st);
       if (tail_s >= 2 && splitk_ws) {
-        // the few tiles of the last round stay on the 8-wave kernel, their K split over the idle CUs
+        // the few tiles of the last round stay on 256 x 256 tiles, their K split over the idle CUs
         const int ksteps = K / 64;
         b.k_per_split = ((ksteps + tail_s - 1) / tail_s) * 64;
         b.splitk = (K + b.k_per_split - 1) / b.k_per_split;
@@ -1268,7 +1278,10 @@ void launch_gemm_grouped(const bf16_t* A, const bf16_t* W, bf16_t* C, const int*
   p.glu_act = glu - 1;
   p.grp_start = start; p.grp_perm = perm; p.grp_top = top; p.grp_count = E;
   p.grp_wstride = static_cast<long long>(N) * K;
-  const int per = rows / E;             // rows of an average group
+  // Rows of an average group.  (The last line is the 8-wave kernel's; with gemm_quad.hip 256 x 256 tiles would be ahead sooner.  us, gate / up and
+  // down, 128 x 128 / 256 x 256: 8 experts of 4096 x 5504, 256 rows a group 356 / 218 and 216 / 140, 767 678 / 476 and 348 / 232; of 2048 x
+  // 2816, 256 rows 115 / 66 and 47 / 59, 384 120 / 110 and 50 / 61, 640 175 / 151 and 75 / 62.)
+  const int per = rows / E;
   if (gemm_grouped_few_serves(p, rows)) launch_gemm_grouped_few(p, rows, st);
   else if (per < 48) launch_grp<32, 128, 1, 4, 4>(p, rows, st);
   else if (per < 192) launch_grp<64, 128, 2, 2, 3>(p, rows, st);
@@ -1287,7 +1300,8 @@ void launch_gemm_glu(const bf16_t* A, const bf16_t* W, bf16_t* H, int M, int I, 
   auto tiles = [&](int bm, int bn) { return static_cast<long long>((M + bm - 1) / bm) * ((2 * I + bn - 1) / bn); };
   if (g_forced_cfg < 0 && use_256(M, 2 * I, K) && g_tail_splitk && I % 128 == 0) {
     // a handful of 256 x 128 output tiles past the last full round (2115 rows x 11008: 774 = 3 x 256 + 6)
-    // would cost a whole further round of the 8-wave kernel: their columns go to 64 x 64 tiles instead
+    // would cost a whole further round: their columns go to 64 x 64 tiles instead (us, so / one launch: that one 316 / 351; 1500 rows,
+    // 516 tiles, 214 / 257; 2304 x 3840 x 1024, 270, 45 / 58)
     const int tiles_m = (M + 255) / 256, tiles_n = I / 128;
     const long long total = static_cast<long long>(tiles_m) * tiles_n;
     const int rounds = static_cast<int>(total / 256), rem = static_cast<int>(total % 256);

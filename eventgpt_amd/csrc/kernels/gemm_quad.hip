@@ -11,7 +11,7 @@
 //    BAR1 + 1.. one staging load (direct to LDS) every LOAD_EVERY: the K-tile after next
 //    BAR2       the next K-tile has landed (counted vmcnt: the loads just issued stay out)
 //    BAR2 + 1.. one LDS read each: the first 32 k of the next K-tile
-// so a staging load has 100 to 190 MFMAs (0.8 to 1.5 us) to land and there are two barriers a K-tile.  Spreading the loads matters
+// so a staging load has 134 to 209 MFMAs (128 + BAR2 less the slot it is issued at: 1.5 to 2.3 us) to land and there are two barriers a K-tile.  Spreading the loads matters
 // most: one every two MFMAs 6688 x 22016 x 4096 944 us, every four or five 872 to 905, and reads at one every two MFMAs instead of
 // one each 5 % behind.  The staging runs on over the ends of output tiles: during a tile's last two K-tiles it fetches the next
 // one's first two, which land under the epilogue (32 KB of the LDS are the epilogue's own, so it needs no barrier).
