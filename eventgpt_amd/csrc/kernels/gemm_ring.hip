@@ -34,7 +34,11 @@ __global__ __launch_bounds__(512) void gemm_ring_kernel(GemmParams p) {
   const int wr = wid / WGN, wc = wid % WGN;
   const int bn_out = p.glu_half ? BN / 2 : BN;
   const int tiles_n = (p.N + bn_out - 1) / bn_out, tiles_m = (p.M + BM - 1) / BM, tiles = tiles_m * tiles_n;
-  const int bid = xcd_remap(blockIdx.x, tiles * p.splitk), tile = bid % tiles, ksplit = bid / tiles;    // (an XCD inside one K range)
+  int tile = xcd_remap(blockIdx.x, tiles * p.splitk), ksplit = 0;
+  if (p.splitk > 1) {                         // (an XCD inside one K range)
+    ksplit = tile / tiles;
+    tile -= ksplit * tiles;
+  }
   // An XCD's tiles are consecutive ones.  They share the panels of the larger operand, so that it is read once into some L2 and the smaller
   // one into each (4 052 x 464 x 4480 by columns of tiles 44.2 us, the general tiles 31.6; by rows 4 011 x 496 x 4352 26.2 and 32.6).
   const bool tall = (p.glu_half ? p.M / 2 : p.M) > p.N;
