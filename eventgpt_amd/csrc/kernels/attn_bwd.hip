@@ -97,10 +97,8 @@ __device__ __forceinline__ void mma_tr(f32x4_t (&acc)[D / 16], const unsigned ch
 #pragma unroll
     for (int dt = 0; dt < D / 16; ++dt) {
       const int ch = dt * 2 + (p4 >> 1);
-      const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-          (s16x4_t __attribute__((address_space(3)))*)(lds + tile_off<D>(r0, ch) + 8 * (p4 & 1)));
-      const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-          (s16x4_t __attribute__((address_space(3)))*)(lds + tile_off<D>(r1, ch) + 8 * (p4 & 1)));
+      const s16x4_t lo = read_tr16((lds_s16x4_t*)(lds + tile_off<D>(r0, ch) + 8 * (p4 & 1)));
+      const s16x4_t hi = read_tr16((lds_s16x4_t*)(lds + tile_off<D>(r1, ch) + 8 * (p4 & 1)));
       const s16x8_t vv = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
       acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, vv), pf, acc[dt], 0, 0, 0);
     }

@@ -244,10 +244,8 @@ __global__ __launch_bounds__(256 * GROUPS) void attn_prefill_kernel(AttnParams p
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
         const int ch = dt * 2 + (p4 >> 1);
-        const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (s16x4_t __attribute__((address_space(3)))*)(v_lds + tile_off<D>(r0, ch) + 8 * (p4 & 1)));
-        const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (s16x4_t __attribute__((address_space(3)))*)(v_lds + tile_off<D>(r1, ch) + 8 * (p4 & 1)));
+        const s16x4_t lo = read_tr16((lds_s16x4_t*)(v_lds + tile_off<D>(r0, ch) + 8 * (p4 & 1)));
+        const s16x4_t hi = read_tr16((lds_s16x4_t*)(v_lds + tile_off<D>(r1, ch) + 8 * (p4 & 1)));
         typedef __attribute__((ext_vector_type(8))) short s16x8_t;
         const s16x8_t vv = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
         if constexpr (WP)
@@ -519,10 +517,8 @@ __global__ __launch_bounds__(AW_WAVES * 64) void attn_prefill_wide_kernel(AttnPa
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
         const int ch = dt * 2 + (p4 >> 1);
-        const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (s16x4_t __attribute__((address_space(3)))*)(v_lds + tile_off<D>(r0, ch) + 8 * (p4 & 1)));
-        const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (s16x4_t __attribute__((address_space(3)))*)(v_lds + tile_off<D>(r1, ch) + 8 * (p4 & 1)));
+        const s16x4_t lo = read_tr16((lds_s16x4_t*)(v_lds + tile_off<D>(r0, ch) + 8 * (p4 & 1)));
+        const s16x4_t hi = read_tr16((lds_s16x4_t*)(v_lds + tile_off<D>(r1, ch) + 8 * (p4 & 1)));
         typedef __attribute__((ext_vector_type(8))) short s16x8_t;
         const s16x8_t vv = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
 #pragma unroll

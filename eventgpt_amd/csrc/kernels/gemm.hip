@@ -70,8 +70,8 @@ __device__ __forceinline__ bf16x8_t frag_t(const unsigned char* tile, int cb, in
   const int chunk = (cb >> 3) + (pp >> 1);
   const unsigned char* a1 = tile + row1 * (BX * 2) + ((chunk ^ swz_t<BX>(row1)) << 4) + 8 * (pp & 1);
   const unsigned char* a2 = tile + row2 * (BX * 2) + ((chunk ^ swz_t<BX>(row2)) << 4) + 8 * (pp & 1);
-  const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4_t __attribute__((address_space(3)))*)a1);
-  const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4_t __attribute__((address_space(3)))*)a2);
+  const s16x4_t lo = read_tr16((lds_s16x4_t*)a1);
+  const s16x4_t hi = read_tr16((lds_s16x4_t*)a2);
   const s16x8_t v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
   return __builtin_bit_cast(bf16x8_t, v);
 }

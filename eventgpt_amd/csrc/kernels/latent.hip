@@ -345,8 +345,8 @@ __global__ __launch_bounds__(256 * HT) void latent_attend_kernel(const bf16_t* _
 #pragma unroll
       for (int t = 0; t < CT; ++t) {
         const unsigned char* vp = tile + vaddr[t] + s * (32 * R * 2);
-        const s16x4_t va = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4_t __attribute__((address_space(3)))*)(vp));
-        const s16x4_t vb = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4_t __attribute__((address_space(3)))*)(vp + 16 * R * 2));
+        const s16x4_t va = read_tr16((lds_s16x4_t*)(vp));
+        const s16x4_t vb = read_tr16((lds_s16x4_t*)(vp + 16 * R * 2));
         typedef __attribute__((ext_vector_type(8))) short s16x8_t;
         const s16x8_t vv = {va[0], va[1], va[2], va[3], vb[0], vb[1], vb[2], vb[3]};
         vf[t] = __builtin_bit_cast(bf16x8_t, vv);
