@@ -29,6 +29,25 @@ __device__ __forceinline__ unsigned int bf16_rest(float a, float b, unsigned int
   return pack_bf16x2(a - bf16lo(packed), b - bf16hi(packed));
 }
 
+// The largest of a lane's sixteen scores, then of the four lanes (16 apart) that hold the query's other keys.  v_maximum3 takes
+// three scores as an MFMA leaves them (fmaxf quiets its operands first, two instructions more a pair); the lanes trade rows of
+// 16 and 32 in registers, where a shuffle waits for the LDS four times a key tile.
+__device__ __forceinline__ float maximum3(float a, float b, float c) {
+  return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c);
+}
+__device__ __forceinline__ float score_max(const f32x4_t (&st)[4]) {
+  float a = maximum3(st[0][0], st[0][1], st[0][2]), b = maximum3(st[0][3], st[1][0], st[1][1]);
+  a = maximum3(a, st[1][2], st[1][3]);
+  b = maximum3(b, st[2][0], st[2][1]);
+  a = maximum3(a, st[2][2], st[2][3]);
+  b = maximum3(b, st[3][0], st[3][1]);
+  a = maximum3(a, st[3][2], st[3][3]);
+  a = __builtin_elementwise_maximum(a, b);
+  const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(a), false, false);
+  a = __builtin_elementwise_maximum(__uint_as_float(x[0]), __uint_as_float(x[1]));
+  const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(a), false, false);
+  return __builtin_elementwise_maximum(__uint_as_float(y[0]), __uint_as_float(y[1]));
+}
 struct AttnParams {
   const bf16_t* q; const bf16_t* k; const bf16_t* v; bf16_t* o;
   long long q_sb, q_ss, q_sh;   // element strides: batch, sequence, head
@@ -197,11 +216,7 @@ __global__ __launch_bounds__(256 * GROUPS) void attn_prefill_kernel(AttnParams p
         for (int r = 0; r < 4; ++r)
           if (key0 + n * 16 + r > lim) st[n][r] = -INFINITY;
     }
-    float mt = fmaxf(fmaxf(st[0][0], st[0][1]), fmaxf(st[0][2], st[0][3]));
-#pragma unroll
-    for (int n = 1; n < 4; ++n) mt = fmaxf(mt, fmaxf(fmaxf(st[n][0], st[n][1]), fmaxf(st[n][2], st[n][3])));
-    mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
-    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+    const float mt = score_max(st);
     const float mn = fmaxf(m, mt);
     const float msafe = mn == -INFINITY ? 0.f : mn;
     if (__builtin_amdgcn_ballot_w64(mn != m) != 0) {
@@ -346,7 +361,7 @@ __device__ __forceinline__ void attn_buffer_to_lds16(const unsigned char* src, i
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (void __attribute__((address_space(3)))*)lds, 16, voff, 0, 0, 0);
 }
 
-constexpr int AW_STAGES = 4;   // K / V tiles in the LDS ring: three in flight while one is computed
+constexpr int AW_STAGES = 4;   // K / V tiles in the LDS ring: three are read between two barriers, one is on its way
 
 // AW_WAVES = 8: 256 query rows per block (long prompts); 4: 128 rows (a few hundred tokens, the ViT)
 // QT: 16-row query tiles per wave (2: every K / V fragment feeds two MFMAs; 1: twice the blocks)
@@ -425,9 +440,9 @@ __global__ __launch_bounds__(AW_WAVES * 64) void attn_prefill_wide_kernel(AttnPa
 
   // The loop is software-pipelined into two phases per key tile,
   //   S: softmax of tile t (VALU)            M: P·V of tile t, then K·Q^T of tile t+1 (MFMA)
-  // each closed by a barrier, and the two halves of the block (waves 0-3 / 4-7, one of each per
-  // SIMD) run ONE BARRIER APART: while one half is in its MFMA phase the other is in its softmax,
-  // so the SIMD's matrix and vector pipes work at the same time instead of taking turns.
+  // and the two halves of the block (waves 0-3 / 4-7, one of each per SIMD) meet at ONE barrier per tile, which the first
+  // half passes after M and the second after S: while one half is in its MFMA phase the other is in its
+  // softmax, so the SIMD's matrix and vector pipes work at the same time instead of taking turns.
   f32x4_t st[QT][4];
   unsigned int pk[QT][4][2], pl[QT][WP ? 4 : 1][2];
   auto qk = [&](const unsigned char* k_lds) {
@@ -467,12 +482,7 @@ __global__ __launch_bounds__(AW_WAVES * 64) void attn_prefill_wide_kernel(AttnPa
           for (int r = 0; r < 4; ++r)
             if (key0 + n * 16 + r > lim) st[qt][n][r] = -INFINITY;
       }
-      float mt = fmaxf(fmaxf(st[qt][0][0], st[qt][0][1]), fmaxf(st[qt][0][2], st[qt][0][3]));
-#pragma unroll
-      for (int n = 1; n < 4; ++n)
-        mt = fmaxf(mt, fmaxf(fmaxf(st[qt][n][0], st[qt][n][1]), fmaxf(st[qt][n][2], st[qt][n][3])));
-      mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
-      mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+      const float mt = score_max(st[qt]);
       const float mn = fmaxf(m[qt], mt);
       const float msafe = mn == -INFINITY ? 0.f : mn;
       if (__builtin_amdgcn_ballot_w64(mn != m[qt]) != 0) {   // some row's maximum moved
@@ -537,39 +547,60 @@ __global__ __launch_bounds__(AW_WAVES * 64) void attn_prefill_wide_kernel(AttnPa
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
   };
-  auto mine = [&](int t) { return wave_active && (!CAUSAL || t * TK <= q_hi + q_off); };
-  auto wait_tile = [&]() {   // all but the youngest tile's loads of this wave have landed
-    static_assert(2 * NIW == 2 || 2 * NIW == 4 || 2 * NIW == 8, "vmcnt literal");
-    if constexpr (2 * NIW == 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-    else if constexpr (2 * NIW == 4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+  // Ring of AW_STAGES tiles.  Between barriers k and k + 1 the early half is in S and M of tile k, the late half in M of tile
+  // k - 1 and S of tile k: tiles k - 1 to k + 1 are read, tile k + 2 is requested into the fourth stage, whose content, tile k - 2,
+  // was last read before barrier k (every wave waits for its LDS reads there).  A tile has landed one barrier after its request:
+  // every wave waits for its own part.  Tiles past the last one are requested too: zero fills of a stage nobody reads.
+  // (With a second barrier a tile, which closed S for one half and M for the other, 4643 tokens of 32 heads took 201 us instead
+  // of 196, eight sequences of 836 99 instead of 93: a wave that had a new maximum held up all of them.)
+  auto landed = [&]() {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    fence();
   };
-
-  // Ring of AW_STAGES tiles: while tile t is multiplied, t+1 is being scored, t+2 is landing and
-  // t+3 has just been requested.  Tiles past the last one are requested too: their out-of-range
-  // loads zero-fill a stage nobody reads and keep the count of loads in flight uniform.
-  //   * a stage is re-requested at the start of phase M of tile t for tile t+3: its previous
-  //     content, tile t-1, was last read in phase M of tile t-1, which the late half finishes
-  //     at the barrier the early half passes on entering phase M of tile t;
-  //   * tile t+2 is waited for at the end of phase M of tile t, by every wave before the
-  //     barrier that closes it, and first read in phase M of tile t+1.
   const bool late = wid >= AW_WAVES / 2;
-#pragma unroll
-  for (int i = 0; i < AW_STAGES - 1; ++i) stage(i, i);
-  wait_tile();                       // tiles 0 and 1
-  fence();
-  if (ntiles > 0 && mine(0)) qk(lds);
-  if (late) fence();
+  stage(0, 0);
+  stage(1, 1);
+  landed();
+  stage(2, 2);
+  const int n_mine = !wave_active ? 0 : CAUSAL ? min(ntiles, (q_hi + q_off + TK) / TK) : ntiles;
+  if (n_mine > 0) qk(lds);
   for (int t = 0; t < ntiles; ++t) {
-    if (mine(t)) softmax(t);
-    fence();
-    stage((t + AW_STAGES - 1) % AW_STAGES, t + AW_STAGES - 1);
-    if (mine(t)) pv(lds + (t % AW_STAGES) * 2 * TILE_BYTES + TILE_BYTES);
-    if (t + 1 < ntiles && mine(t + 1)) qk(lds + ((t + 1) % AW_STAGES) * 2 * TILE_BYTES);
-    wait_tile();                     // tile t+2
-    fence();
+    if (t < n_mine) softmax(t);
+    if (late) {
+      landed();
+      stage((t + 3) % AW_STAGES, t + 3);
+    }
+    const unsigned char* v_lds = lds + (t % AW_STAGES) * 2 * TILE_BYTES + TILE_BYTES;
+    const unsigned char* k_lds = lds + ((t + 1) % AW_STAGES) * 2 * TILE_BYTES;
+    __builtin_amdgcn_s_setprio(1);
+    if (!WP && t + 1 < n_mine) {
+      // one block of code: sixteen LDS reads ahead of the products, of which a V read feeds one and a K read two
+      __builtin_amdgcn_sched_barrier(0);
+      pv(v_lds);
+      qk(k_lds);
+      __builtin_amdgcn_sched_group_barrier(0x100, 16, 0);
+#pragma unroll
+      for (int i = 0; i < DT * QT - 8; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < KS * 4; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, 16, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    } else {                           // (both parts of the weights leave no registers to read ahead into)
+      if (t < n_mine) pv(v_lds);
+      if (WP && t + 1 < n_mine) qk(k_lds);
+    }
+    __builtin_amdgcn_s_setprio(0);
+    if (!late) {
+      landed();
+      stage((t + 3) % AW_STAGES, t + 3);
+    }
   }
-  if (!late) fence();
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // zero fills land before the LDS is handed on
 
 #pragma unroll

@@ -57,6 +57,30 @@ def test_wide_attention_packed_qkv_and_spike(dev, wide):
     assert torch.allclose(o.float(), want.float(), atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("mode", [0, 2])                      # 64-row blocks, ring-staged blocks
+@pytest.mark.parametrize("D,H,S,causal,step", [(128, 4, 700, True, 5.0), (64, 4, 577, False, 9.0), (128, 16, 2100, True, 0.5), (128, 4, 300, True, -5.0)])
+def test_attention_whose_maximum_creeps(dev, wide, mode, D, H, S, causal, step):
+    """Scores that rise (or fall) by ``step`` in base 2 from one tile of 64 keys to the next, the largest of a tile in every column of
+    its 16 x 4 in turn: the maximum over a lane's keys and over the lanes that share a query."""
+    g = torch.Generator(device=dev).manual_seed(S)
+    unit = torch.zeros(D, device=dev)
+    unit[0] = 1.0
+    at = torch.arange(S, device=dev)
+    level = ((at // 64).float() * step + 4.0 * (at % 64 == (at // 64 * 7) % 64)) * 0.6931472
+    q = (torch.randn(1, S, H, D, device=dev, generator=g) * 0.5 * (1 - unit) + 16.0 * unit).bfloat16()
+    k = (torch.randn(1, S, H, D, device=dev, generator=g) * (1 - unit) + (level * D ** 0.5 / 16.0)[None, :, None, None] * unit).bfloat16()
+    v = _rand(1, S, H, D, dev=dev)
+    wide.raw.attn_enable_wide(mode)
+    o, lse = wide.raw.attention_fwd_lse(q, k, v, causal, D ** -0.5, 0)
+    s = torch.matmul(q.double().transpose(1, 2), k.double().permute(0, 2, 3, 1).contiguous()) * D ** -0.5
+    if causal:
+        s = s.masked_fill(torch.ones(S, S, device=dev, dtype=torch.bool).triu(1), float("-inf"))
+    want = torch.matmul(torch.softmax(s, -1), v.double().transpose(1, 2).contiguous()).transpose(1, 2)
+    # weights and outputs are rounded to bf16 once each: 2^-9 of values up to 4, twice
+    assert torch.allclose(o.double(), want, atol=2e-2, rtol=2e-2), float((o.double() - want).abs().max())
+    assert torch.allclose(lse.double(), torch.logsumexp(s, -1) * 1.4426950408889634, atol=1e-3, rtol=1e-5)
+
+
 def test_wide_attention_against_cache_with_device_length(dev, wide):
     from eventgpt_amd.ops import hip, reference
     D, Hq, Hkv, Sq, kv, Lmax = 128, 4, 2, 300, 900, 1024
