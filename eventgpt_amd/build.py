@@ -42,7 +42,9 @@ ARCH = "gfx950"
 # wrong results on this hardware pool, so the compiler must not emit them.
 # No -ffast-math: the kernels use +/-inf as softmax / argmax sentinels, and
 # finite-math-only lets the compiler fold `x == -INFINITY` away (NaNs follow).
-HIP_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-fno-math-errno",
+# kernarg-preload: leading scalar arguments of a kernel are in scalar registers when its waves start (14 dwords of them; a structure and
+# what follows it are loads).
+HIP_FLAGS = ["-mllvm", "-amdgpu-kernarg-preload-count=16", "-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-fno-math-errno",
              "-ffp-contract=fast",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
              "-Wno-unused-result", "-Wno-unknown-warning-option", "-Wno-unused-command-line-argument",

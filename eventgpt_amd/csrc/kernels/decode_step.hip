@@ -95,7 +95,7 @@ __device__ void head_step(const AttnPrepArgs& a, int b, int head, int p, bool li
       src8(a.src, b, col + c, t);
       s += sumsq8(t);
     }
-    r = rsqrtf(block_sum(s, red) / static_cast<float>(is_q ? a.nq : a.nk) + a.eps);
+    r = rsqrtf(block_sum<4>(s, red) / static_cast<float>(is_q ? a.nq : a.nk) + a.eps);
   }
   if (!is_q && !live) return;
   const int half = a.rot >> 1, pt = min(max(p, 0), a.max_pos - 1);
@@ -166,7 +166,7 @@ __global__ __launch_bounds__(256) void parallel_step_kernel(StepHeads sh, StepMe
     if (v0 == 0) m.n[to * m.N + e] = n1;
     dot += n1 * qs[e];
   }
-  dot = block_sum(dot, red);            // (its barriers also publish avs)
+  dot = block_sum<4>(dot, red);            // (its barriers also publish avs)
   if (v0 == 0 && threadIdx.x == 0) m.m[to] = m1;
   const float inv = 1.f / (fmaxf(fabsf(dot), expf(-m1)) + 1e-6f);
   float* out = m.out + static_cast<long long>(gi) * m.V + v0;

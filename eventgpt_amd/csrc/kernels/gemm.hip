@@ -202,7 +202,8 @@ __device__ __forceinline__ void gemm_rope_epilogue(const GemmParams& p, f32x4_t 
 
 template <int BM, int BN, int WGM, int WGN, int STAGES, bool AT = false, bool BT = false, bool KT = false,
           bool ROPE = false, bool GRP = false, int ACT = -1>
-__global__ __launch_bounds__(WGM * WGN * 64) void gemm_bf16_kernel(GemmParams p) {
+__global__ __launch_bounds__(WGM * WGN * 64) void gemm_bf16_kernel(EVGPT_GEMM_ARGS) {
+  EVGPT_GEMM_TAKE;
   static_assert(!GRP || (!AT && !BT && !KT && !ROPE), "grouped products are plain ones");
   static_assert(!AT || BM == 64 || BM == 128, "K-strided A needs a 64- or 128-row tile");
   static_assert(!BT || BN == 64 || BN == 128, "K-strided W needs a 64- or 128-column tile");
@@ -417,7 +418,8 @@ constexpr int FR_BK = 128, FR_W_BYTES = 64 * FR_BK * 2;
 
 // (a 16-row x image for up to 16 rows and four stages instead of three measure within 2 % of this; four stages
 // with the 32-row image, one workgroup per CU, 10 % behind)
-__global__ __launch_bounds__(256) void gemm_fewrow_kernel(GemmParams p) {
+__global__ __launch_bounds__(256) void gemm_fewrow_kernel(EVGPT_GEMM_ARGS) {
+  EVGPT_GEMM_TAKE;
   constexpr int AM = 32, STAGES = 3;   // rows of the x image, K-tiles in the ring
   constexpr int A_BYTES = AM * FR_BK * 2, STAGE = A_BYTES + FR_W_BYTES;
   constexpr int TM = AM / 16;      // 16-row blocks of x
@@ -513,7 +515,7 @@ static void launch_fewrow(const GemmParams& p, hipStream_t st) {
   }();
   (void)attr;
   const int tiles_n = (p.N + 63) / 64;
-  hipLaunchKernelGGL(gemm_fewrow_kernel, dim3(tiles_n * p.splitk), dim3(256), smem, st, p);
+  hipLaunchKernelGGL(gemm_fewrow_kernel, dim3(tiles_n * p.splitk), dim3(256), smem, st, EVGPT_GEMM_PASS(p));
 }
 
 // ---------------------------------------------------------------------------------------
@@ -908,7 +910,7 @@ static void launch_cfg(const GemmParams& p, hipStream_t st) {
   q.group_m = g_group_m;
   q.split_major = (g_split_major && p.splitk > 1 && p.M > 32) ? 1 : 0;
   hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, WGM, WGN, STAGES, AT, BT, KT, ROPE, false, ACT>), dim3(tiles), dim3(WGM * WGN * 64),
-                     smem, st, q);
+                     smem, st, EVGPT_GEMM_PASS(q));
 }
 
 // 256 x 256 tiles pay once there are rows to fill them and about half a round of tiles.  With the 8-wave kernel (measured on
@@ -1268,7 +1270,7 @@ static void launch_grp(GemmParams p, int rows, hipStream_t st) {
   }();
   (void)attr;
   p.group_m = g_group_m;
-  hipLaunchKernelGGL(kern, dim3(tiles), dim3(256), smem, st, p);
+  hipLaunchKernelGGL(kern, dim3(tiles), dim3(256), smem, st, EVGPT_GEMM_PASS(p));
 }
 void launch_gemm_grouped(const bf16_t* A, const bf16_t* W, bf16_t* C, const int* start, const int* perm, int top, int E,
                          int a_rows, int rows, int N, int K, int glu, hipStream_t st) {

@@ -19,7 +19,8 @@ namespace {
 constexpr int TK = 128, AM = 32, TN = 32, STAGES = 3, RUN = 16;
 
 template <bool GLU>
-__global__ __launch_bounds__(256) void gemm_grouped_few_kernel(GemmParams p) {
+__global__ __launch_bounds__(256) void gemm_grouped_few_kernel(EVGPT_GEMM_ARGS) {
+  EVGPT_GEMM_TAKE;
   constexpr int W_ROWS = GLU ? 2 * TN : TN, WI = W_ROWS / 16;      // staging instructions per wave: 4 rows x 256 bytes each
   constexpr int A_BYTES = AM * TK * 2, STAGE = A_BYTES + W_ROWS * TK * 2;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -135,7 +136,7 @@ void launch(const GemmParams& p, int grid, hipStream_t st) {
   static const bool attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_grouped_few_kernel<GLU>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, smem) == hipSuccess;
   (void)attr;
-  hipLaunchKernelGGL((gemm_grouped_few_kernel<GLU>), dim3(grid), dim3(256), smem, st, p);
+  hipLaunchKernelGGL((gemm_grouped_few_kernel<GLU>), dim3(grid), dim3(256), smem, st, EVGPT_GEMM_PASS(p));
 }
 
 }  // namespace

@@ -25,7 +25,8 @@ __device__ __forceinline__ void load_to_lds16(const unsigned char* src, int byte
 
 // WGM x WGN waves, each TM x TN tiles of 16 x 16; S K-tiles of 64 in the ring
 template <int TM, int TN, int WGM, int WGN, int S, int ACT>
-__global__ __launch_bounds__(512) void gemm_ring_kernel(GemmParams p) {
+__global__ __launch_bounds__(512) void gemm_ring_kernel(EVGPT_GEMM_ARGS) {
+  EVGPT_GEMM_TAKE;
   constexpr int NW = WGM * WGN, WM = TM * 16, WN = TN * 16, BM = WM * WGM, BN = WN * WGN, A_BYTES = BM * 128, STAGE = (BM + BN) * 128;
   constexpr int IA = BM / (8 * NW), IW = BN / (8 * NW), G = IA + IW;           // staging instructions per wave and K-tile
   static_assert(NW == 8 && IA * 64 == BM && IW * 64 == BN && S >= 3, "eight waves stage whole groups of eight rows");
@@ -148,7 +149,7 @@ void launch_act(const GemmParams& p, hipStream_t st) {
   (void)attr;
   const int bn_out = p.glu_half ? BN / 2 : BN;
   const int tiles = (p.M + BM - 1) / BM * ((p.N + bn_out - 1) / bn_out) * p.splitk;
-  hipLaunchKernelGGL((gemm_ring_kernel<TM, TN, WGM, WGN, S, ACT>), dim3(tiles), dim3(512), lds, st, p);
+  hipLaunchKernelGGL((gemm_ring_kernel<TM, TN, WGM, WGN, S, ACT>), dim3(tiles), dim3(512), lds, st, EVGPT_GEMM_PASS(p));
 }
 template <int TM, int TN, int WGM, int WGN, int S>
 void launch(const GemmParams& p, hipStream_t st) {

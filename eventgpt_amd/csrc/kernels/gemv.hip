@@ -75,6 +75,17 @@ struct GemvParams {
   W4Code code;           // byte planes of the 16 bf16 codebook entries
 };
 
+// What the first loads need, ahead of the other parameters: with kernel argument preload (build.py) it is in scalar registers when
+// a wave starts.  aux: the residual, or the positions.  (A chat of 636 + 32 tokens 95.7 -> 95.3 ms; 4-bit level.)
+#define EVGPT_GEMV_ARGS \
+  const bf16_t *w_, const bf16_t *x_, const bf16_t *norm_, const float *absmax_, const void *aux_, int n_, int k_, float eps_, GemvParams p
+#define EVGPT_GEMV_TAKE(E)                                                          \
+  p.W = w_, p.x = x_, p.norm_w = norm_, p.absmax = absmax_, p.N = n_, p.K = k_, p.eps = eps_; \
+  if constexpr (E == E_RESIDUAL) p.res = static_cast<const bf16_t*>(aux_);          \
+  else if constexpr (E == E_QKV_ROPE) p.pos = static_cast<const int*>(aux_)
+#define EVGPT_GEMV_PASS(p, E) \
+  (p).W, (p).x, (p).norm_w, (p).absmax, E == E_RESIDUAL ? static_cast<const void*>((p).res) : static_cast<const void*>((p).pos), (p).N, (p).K, (p).eps, p
+
 // Measured on the 7B decode step (ms per token, same box): PRE/UNROLL/OCC = 1/4/4: 2.72,
 // 2/4/4: 3.13 (spills), 4/6/1: 2.90, 4/8/1: 2.94, 4/6/3: 4.39 (spills) -- prefetching more of
 // the first unit ahead of the norm, or issuing more than four iterations at once, costs
@@ -257,7 +268,7 @@ __global__ __launch_bounds__(GEMV_WAVES * 64, Q ? (B <= 2 ? 4 : 3) : (B == 1 ? E
             const float lo = bf16lo(xr[i][j]), hi = bf16hi(xr[i][j]);
             ss += lo * lo + hi * hi;
           }
-        ss = block_sum(ss, red);
+        ss = block_sum<GEMV_WAVES>(ss, red);
         const float rstd = rsqrtf(ss / static_cast<float>(p.K) + p.eps);
 #pragma unroll
         for (int i = 0; i < XC; ++i) {
@@ -285,7 +296,7 @@ __global__ __launch_bounds__(GEMV_WAVES * 64, Q ? (B <= 2 ? 4 : 3) : (B == 1 ? E
             ss += lo * lo + hi * hi;
           }
         }
-        ss = block_sum(ss, red);
+        ss = block_sum<GEMV_WAVES>(ss, red);
         const float rstd = rsqrtf(ss / static_cast<float>(p.K) + p.eps);
         for (int c = tid; c < nchunk; c += blockDim.x) {
           u32x4_t v = load16(p.x + (static_cast<size_t>(b) * p.K + c * 8));
@@ -667,7 +678,8 @@ __global__ __launch_bounds__(GEMV_WAVES * 64, Q ? (B <= 2 ? 4 : 3) : (B == 1 ? E
 // rows per unit -- all resident at once, every block's reduce / store tail exposed at the end of the launch;
 // two rows per unit (plain row order only) make 2048 blocks of half the work.
 template <int P, int E, int KS, int RR = 4>
-__global__ __launch_bounds__(GEMV_WAVES * 64, EVGPT_ROW1_OCC) void gemv_row1_kernel(GemvParams p) {
+__global__ __launch_bounds__(GEMV_WAVES * 64, EVGPT_ROW1_OCC) void gemv_row1_kernel(EVGPT_GEMV_ARGS) {
+  EVGPT_GEMV_TAKE(E);
   static_assert(RR == 4 || RR == 2 || ((E == E_RESIDUAL || E == E_STORE) && RR == 1), "rows per unit");
   constexpr int R = RR;          // shadows the family's constant inside this kernel
   constexpr int NP = RR / 2;     // rotate-half / gate-up pairs per unit
@@ -721,6 +733,8 @@ __global__ __launch_bounds__(GEMV_WAVES * 64, EVGPT_ROW1_OCC) void gemv_row1_ker
       }
     }
   }
+  if constexpr (E == E_QKV_ROPE) have_now(p.q_out, p.k_cache, p.v_cache, p.n_q_heads, p.n_kv_heads, p.head_dim, p.l_max, p.cos_tab, p.sin_tab);
+  else if constexpr (E != E_LOGITS) have_now(p.y);
   if constexpr (P == P_RMSNORM) {
     constexpr int XC = 2;  // x chunks a thread keeps in registers between the two passes
     if (nchunk <= XC * GEMV_WAVES * 64) {
@@ -745,7 +759,7 @@ __global__ __launch_bounds__(GEMV_WAVES * 64, EVGPT_ROW1_OCC) void gemv_row1_ker
             ss += lo * lo + hi * hi;
           }
         }
-        ss = block_sum(ss, red);
+        ss = block_sum<GEMV_WAVES>(ss, red);
         const float rstd = rsqrtf(ss / static_cast<float>(p.K) + p.eps);
 #pragma unroll
         for (int i = 0; i < XC; ++i) {
@@ -773,7 +787,7 @@ __global__ __launch_bounds__(GEMV_WAVES * 64, EVGPT_ROW1_OCC) void gemv_row1_ker
             ss += lo * lo + hi * hi;
           }
         }
-        ss = block_sum(ss, red);
+        ss = block_sum<GEMV_WAVES>(ss, red);
         const float rstd = rsqrtf(ss / static_cast<float>(p.K) + p.eps);
         for (int c = tid; c < nchunk; c += blockDim.x) {
           u32x4_t v = load16(p.x + (static_cast<size_t>(b) * p.K + c * 8));
@@ -1132,7 +1146,8 @@ struct RowsStep {
 // Q = 0 streams bf16 weights through the same pipeline (no table, plain x images, one 16-byte x chunk
 // per 16 bytes of weights and x row).
 template <int P, int E, int B, int Q>
-__global__ __launch_bounds__(W4R_WAVES * 64, (B == 1 && Q) ? 2 : 1) void gemv_rows_kernel(GemvParams p) {
+__global__ __launch_bounds__(W4R_WAVES * 64, (B == 1 && Q) ? 2 : 1) void gemv_rows_kernel(EVGPT_GEMV_ARGS) {
+  EVGPT_GEMV_TAKE(E);
   static_assert(E != E_LOGITS, "the LM head has a kernel of its own");
   static_assert(B >= 1 && B <= 4 && (Q == 0 || B <= 3), "x rows");
   constexpr bool W4 = Q != 0;
@@ -1249,6 +1264,9 @@ __global__ __launch_bounds__(W4R_WAVES * 64, (B == 1 && Q) ? 2 : 1) void gemv_ro
   issue_aux(b1, g1);
   __builtin_amdgcn_sched_barrier(0);
 
+  if constexpr (E == E_QKV_ROPE) have_now(p.q_out, p.k_cache, p.v_cache, p.n_q_heads, p.n_kv_heads, p.head_dim, p.l_max);
+  else have_now(p.y);
+
   // ---- table: entry t = (value[t & 15], value[t >> 4]), 32 copies 4 bytes apart
   if (W4 && tid < 256) {
     unsigned int e[4];
@@ -1275,7 +1293,7 @@ __global__ __launch_bounds__(W4R_WAVES * 64, (B == 1 && Q) ? 2 : 1) void gemv_ro
           }
         }
       }
-      ss = block_sum(ss, red);
+      ss = block_sum<W4R_WAVES>(ss, red);
       const float rstd = rsqrtf(ss / static_cast<float>(p.K) + p.eps);
 #pragma unroll
       for (int i = 0; i < XC; ++i) {
@@ -1575,7 +1593,7 @@ static void launch_rows_b(const GemvParams& p, hipStream_t st) {
     const int per_wave = (groups + cap * W4R_WAVES - 1) / (cap * W4R_WAVES);
     blocks = (groups + per_wave * W4R_WAVES - 1) / (per_wave * W4R_WAVES);
   }
-  hipLaunchKernelGGL((gemv_rows_kernel<P, E, B, Q>), dim3(blocks), dim3(W4R_WAVES * 64), smem, st, p);
+  hipLaunchKernelGGL((gemv_rows_kernel<P, E, B, Q>), dim3(blocks), dim3(W4R_WAVES * 64), smem, st, EVGPT_GEMV_PASS(p, E));
 }
 
 template <int P, int E>
@@ -1675,17 +1693,17 @@ static void launch_bk(const GemvParams& p, int B, hipStream_t st) {
           const int rr = plain ? rr_res : rr_pair;
           const bool fits = p.N % 4 == 0 && (E != E_QKV_ROPE || p.head_dim % 4 == 0);
           if (fits && rr == 2) {
-            hipLaunchKernelGGL((gemv_row1_kernel<P, E, KS, 2>), dim3(((p.N + 1) / 2 + upb - 1) / upb), b, smem, st, p);
+            hipLaunchKernelGGL((gemv_row1_kernel<P, E, KS, 2>), dim3(((p.N + 1) / 2 + upb - 1) / upb), b, smem, st, EVGPT_GEMV_PASS(p, E));
             break;
           }
           if constexpr (plain) {
             if (fits && rr == 1) {
-              hipLaunchKernelGGL((gemv_row1_kernel<P, E, KS, 1>), dim3((p.N + upb - 1) / upb), b, smem, st, p);
+              hipLaunchKernelGGL((gemv_row1_kernel<P, E, KS, 1>), dim3((p.N + upb - 1) / upb), b, smem, st, EVGPT_GEMV_PASS(p, E));
               break;
             }
           }
         }
-        hipLaunchKernelGGL((gemv_row1_kernel<P, E, KS>), g, b, smem, st, p);
+        hipLaunchKernelGGL((gemv_row1_kernel<P, E, KS>), g, b, smem, st, EVGPT_GEMV_PASS(p, E));
       } else {
         hipLaunchKernelGGL((gemv_kernel<1, P, E, KS, Q>), g, b, smem, st, p);
       }

@@ -173,7 +173,7 @@ __device__ void prepare_merge(const GemvInput& in, int b, int K, T* xs, float* r
     ss += sumsq8(v);
     if (lead) store8(in.x_out + o + c, v);
   }
-  const float r = rsqrtf(block_sum(ss, red) * inv_n + in.eps);
+  const float r = rsqrtf(block_sum<4>(ss, red) * inv_n + in.eps);
   auto put = [&](int c, const float (&v)[8], float (&w)[8]) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) w[i] *= v[i] * r;
@@ -276,23 +276,34 @@ __device__ void prepare_group(const GemvInput& in, int b, int K, T* xs, float* i
 // the RMS norm of the stream, branches and group norms, PREP_ALL for either norm of the stream, the norm after a
 // sublayer and columns of a projection, with the latent store and the finished rows.
 enum { PREP_NONE = 0, PREP_RMS = 1, PREP_ALL = 2 };
+// Ahead of the call, in scalar registers when a wave starts (build.py): the first problem's weights, row and norm weights; q0, q1 its
+// branch outputs, or q0 the second problem's weights.  (A chat of one stream, width 2048: 22.67 -> 22.35 ms.)
 template <typename T, int B, int EPI, int PREP>
-__global__ __launch_bounds__(256) void row_gemv_kernel(GemvCall call, int blocks0) {
+__global__ __launch_bounds__(256) void row_gemv_kernel(const void* w0_, const void* x0_, const float* norm0_, const void* q0_, const void* q1_, int n0_,
+                                                       int k0_, int blocks0, GemvCall call) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   constexpr int CE = 16 / sizeof(T);                      // elements per 16-byte chunk
   __shared__ float part[2][4][GV_R * B];
   __shared__ float red[16];
   constexpr bool PLAIN = PREP == PREP_NONE;
   if constexpr (PREP == PREP_ALL) {
-    if (call.latent.cache && blockIdx.x + 1 == gridDim.x) {
+    if (static_cast<int>(blockIdx.x) >= blocks0) {           // (the one block more there is)
       store_latents<T>(call.latent, B);
       return;
     }
   }
-  const bool second = call.count == 2 && static_cast<int>(blockIdx.x) >= blocks0;
-  const GemvProblem& p = call.p[second ? 1 : 0];
+  const bool second = PREP == PREP_RMS && static_cast<int>(blockIdx.x) >= blocks0;     // (blocks0: the grid, if there is one problem)
+  GemvProblem p = call.p[second ? 1 : 0];
+  if (second) {
+    p.W = q0_;
+  } else {
+    p.W = w0_, p.N = n0_, p.K = k0_, p.in.x = x0_, p.in.w = norm0_;
+    if constexpr (PREP == PREP_RMS) {
+      if (call.count == 1) p.in.a = static_cast<const float*>(q0_), p.in.b = static_cast<const float*>(q1_);
+    }
+  }
   const int blk = second ? blockIdx.x - blocks0 : blockIdx.x;
-  const int nblk = call.count == 2 ? (second ? gridDim.x - blocks0 : blocks0) : blocks0;
+  const int nblk = second ? gridDim.x - blocks0 : blocks0;
   const int K = p.K, nchunk = K / CE, nit = (nchunk + 255) / 256;
   const int units = p.N / GV_R;
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
@@ -420,16 +431,20 @@ static void launch_b(const GemvCall& c, size_t lds, hipStream_t st) {
   const dim3 grid(b0 + b1 + (c.latent.cache ? 1 : 0)), block(256);
   const bool plain = c.count == 1 && kind == GV_PLAIN;
   const bool all = c.count == 1 && (kind == GV_POST || kind == GV_ROWS || (kind == GV_NORM && (c.p[0].in.layer || c.p[0].in.xn_out || c.finish)));
+  const GemvProblem& p0 = c.p[0];
+  const void* q0 = c.count == 2 ? c.p[1].W : p0.in.a;
+#define EVGPT_GEMV_PASS p0.W, p0.in.x, p0.in.w, q0, p0.in.b, p0.N, p0.K, b0, c
 #define EVGPT_GEMV(E)                                                                                    \
-  if (plain) hipLaunchKernelGGL((row_gemv_kernel<T, B, E, PREP_NONE>), grid, block, 0, st, c, b0);       \
-  else hipLaunchKernelGGL((row_gemv_kernel<T, B, E, PREP_RMS>), grid, block, lds, st, c, b0)
+  if (plain) hipLaunchKernelGGL((row_gemv_kernel<T, B, E, PREP_NONE>), grid, block, 0, st, EVGPT_GEMV_PASS);       \
+  else hipLaunchKernelGGL((row_gemv_kernel<T, B, E, PREP_RMS>), grid, block, lds, st, EVGPT_GEMV_PASS)
   // (nothing is added to the stream behind a PREP_ALL input)
-  if (all && c.epilogue == GV_GLU) hipLaunchKernelGGL((row_gemv_kernel<T, B, GV_GLU, PREP_ALL>), grid, block, lds, st, c, b0);
-  else if (all) hipLaunchKernelGGL((row_gemv_kernel<T, B, GV_STORE, PREP_ALL>), grid, block, lds, st, c, b0);
+  if (all && c.epilogue == GV_GLU) hipLaunchKernelGGL((row_gemv_kernel<T, B, GV_GLU, PREP_ALL>), grid, block, lds, st, EVGPT_GEMV_PASS);
+  else if (all) hipLaunchKernelGGL((row_gemv_kernel<T, B, GV_STORE, PREP_ALL>), grid, block, lds, st, EVGPT_GEMV_PASS);
   else if (c.epilogue == GV_STORE) { EVGPT_GEMV(GV_STORE); }
   else if (c.epilogue == GV_ADD) { EVGPT_GEMV(GV_ADD); }
   else { EVGPT_GEMV(GV_GLU); }
 #undef EVGPT_GEMV
+#undef EVGPT_GEMV_PASS
 }
 void launch_row_gemv(const GemvCall& c, bool f32, int B, hipStream_t st) {
   const size_t lds = row_gemv_lds(c, f32, B);

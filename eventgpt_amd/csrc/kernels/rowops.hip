@@ -75,8 +75,8 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(float* __restrict__ 
       src8(b, row, c, t);
       sb += sumsq8(t);
     }
-    ra = 0.5f * rsqrtf(block_sum(sa, red) * inv_n + eps);
-    rb = 0.5f * rsqrtf(block_sum(sb, red) * inv_n + eps);
+    ra = 0.5f * rsqrtf(block_sum<4>(sa, red) * inv_n + eps);
+    rb = 0.5f * rsqrtf(block_sum<4>(sb, red) * inv_n + eps);
   }
   if constexpr (MODE >= 3) {
 #pragma unroll

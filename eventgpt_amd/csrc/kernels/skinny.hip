@@ -86,7 +86,7 @@ __global__ __launch_bounds__(256) void reduce_residual_norm_kernel(
     }
   }
   if (!norm_w) return;  // block-uniform
-  ss = block_sum(ss, red);
+  ss = block_sum<4>(ss, red);
   const float rstd = rsqrtf(ss / static_cast<float>(N) + eps);
   for (int c = threadIdx.x; c < nchunk; c += 256) {
     const u32x4_t v = load16(x_out + base + c * 8);  // this thread's own stores

@@ -113,7 +113,7 @@ __device__ __forceinline__ RowStat row_stat(const float (&keep)[NC][8], int n, i
   if (!layer) {
     float ss = 0.f;
     each([&](int, const float (&v)[8]) { ss += sumsq8(v); });
-    return {0.f, rsqrtf(block_sum(ss, red) / static_cast<float>(n) + eps)};
+    return {0.f, rsqrtf(block_sum<4>(ss, red) / static_cast<float>(n) + eps)};
   }
   float s = 0.f, cnt = 0.f;
   each([&](int c, const float (&v)[8]) {
