@@ -43,10 +43,7 @@ __device__ __forceinline__ float score_max(const f32x4_t (&st)[4]) {
   b = maximum3(b, st[3][0], st[3][1]);
   a = maximum3(a, st[3][2], st[3][3]);
   a = __builtin_elementwise_maximum(a, b);
-  const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(a), false, false);
-  a = __builtin_elementwise_maximum(__uint_as_float(x[0]), __uint_as_float(x[1]));
-  const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(a), false, false);
-  return __builtin_elementwise_maximum(__uint_as_float(y[0]), __uint_as_float(y[1]));
+  return max_of_quads(a);
 }
 struct AttnParams {
   const bf16_t* q; const bf16_t* k; const bf16_t* v; bf16_t* o;

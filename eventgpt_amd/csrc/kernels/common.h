@@ -99,6 +99,14 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// the largest of the four lanes 16 apart (v_permlane16 / 32_swap: a shuffle is a round trip through the LDS)
+__device__ __forceinline__ float max_of_quads(float a) {
+  const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(a), false, false);
+  a = __builtin_elementwise_maximum(__uint_as_float(x[0]), __uint_as_float(x[1]));
+  const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(a), false, false);
+  return __builtin_elementwise_maximum(__uint_as_float(y[0]), __uint_as_float(y[1]));
+}
+
 // Block-wide sum for blocks of up to 1024 threads; `scratch` holds >= 16 floats.  NW: the block's waves where the kernel is launched
 // with that many only (the block's size is a load otherwise, and the partial sums a loop of LDS reads).
 template <int NW = 0>

@@ -6,6 +6,8 @@
 // A recurrent state is streamed once: sixteen lanes per state row read it, decay it, add the token, dot it with
 // the query and write it back.  A block owns some rows of one head; it prepares the head's small vectors
 // (query, key, convolution outputs, gates) itself in LDS rather than waiting for another launch.
+#include <type_traits>
+
 #include "src_rows.h"
 
 namespace evgpt {
@@ -81,140 +83,154 @@ __device__ __forceinline__ void stream_state(float* __restrict__ S, int N, int v
   }
 }
 
-template <typename T>
+// (every operand of a thread's first element is requested before the sum of squares)
+template <typename T, int M>
 __device__ void head_step(const AttnPrepArgs& a, int b, int head, int p, bool live, float* red) {
   const bool is_q = head < a.Hq;
   const int h = is_q ? head : head - a.Hq;
   const int col = is_q ? a.q_col : a.k_col, width = (is_q ? a.Hq : a.Hkv) * a.D;
   const float* w = is_q ? a.qw : a.kw;
+  const int half = a.rot >> 1;
+  auto partner = [&](int d) { return h * a.D + (d < half ? d + half : d - half); };
+  const int d0 = min(static_cast<int>(threadIdx.x), a.D - 1), c0 = h * a.D + d0, p0 = d0 < a.rot ? partner(d0) : c0;
+  const float u0 = src1<M>(a.src, b, col + c0), o0 = src1<M>(a.src, b, col + p0);
+  const float wu0 = w ? w[c0] : 1.f, wo0 = w ? w[p0] : 1.f;
+  const float vv0 = is_q ? 0.f : src1<M>(a.src, b, a.v_col + c0);
+  const int pt = min(max(p, 0), a.max_pos - 1);
+  const float* cs = a.cos_tab + static_cast<long long>(pt) * half;
+  const float* sn = a.sin_tab + static_cast<long long>(pt) * half;
+  const int i0 = min(d0 < half ? d0 : d0 - half, half - 1);
+  const float cs0 = half > 0 ? cs[i0] : 1.f, sn0 = half > 0 ? sn[i0] : 0.f;
   float r = 1.f;
   if (w) {
     float s = 0.f;
     for (int c = threadIdx.x * 8; c < width; c += 2048) {
       float t[8];
-      src8(a.src, b, col + c, t);
+      src8<M>(a.src, b, col + c, t);
       s += sumsq8(t);
     }
     r = rsqrtf(block_sum<4>(s, red) / static_cast<float>(is_q ? a.nq : a.nk) + a.eps);
   }
   if (!is_q && !live) return;
-  const int half = a.rot >> 1, pt = min(max(p, 0), a.max_pos - 1);
-  const float* cs = a.cos_tab + static_cast<long long>(pt) * half;
-  const float* sn = a.sin_tab + static_cast<long long>(pt) * half;
   for (int d = threadIdx.x; d < a.D; d += 256) {
+    const bool first = d < 256;
     const int c = h * a.D + d;
-    float u = src1(a.src, b, col + c) * r;
-    if (w) u *= w[c];
+    float u = (first ? u0 : src1<M>(a.src, b, col + c)) * r;
+    if (w) u *= first ? wu0 : w[c];
     if (d < a.rot) {
-      const int i = d < half ? d : d - half, c2 = d < half ? c + half : c - half;
-      float o = src1(a.src, b, col + c2) * r;
-      if (w) o *= w[c2];
-      u = d < half ? u * cs[i] - o * sn[i] : u * cs[i] + o * sn[i];
+      const int i = d < half ? d : d - half, c2 = partner(d);
+      float o = (first ? o0 : src1<M>(a.src, b, col + c2)) * r;
+      if (w) o *= first ? wo0 : w[c2];
+      const float ci = first ? cs0 : cs[i], si = first ? sn0 : sn[i];
+      u = d < half ? u * ci - o * si : u * ci + o * si;
     }
     if (is_q) {
       static_cast<T*>(a.q_out)[static_cast<long long>(b) * width + c] = from_f32<T>(u);
     } else {
       const long long o = ((static_cast<long long>(b) * a.Hkv + h) * a.cap + max(p, 0) % a.cap) * a.D + d;
       static_cast<T*>(a.k_cache)[o] = from_f32<T>(u);
-      static_cast<T*>(a.v_cache)[o] = from_f32<T>(src1(a.src, b, a.v_col + c));
+      static_cast<T*>(a.v_cache)[o] = from_f32<T>(first ? vv0 : src1<M>(a.src, b, a.v_col + c));
     }
   }
 }
 
-template <typename T, bool AHEAD>
+// Whatever a block combines with its state rows is requested with them, in both images where the position says which one is read: the
+// kernel is the slowest of these loads, one barrier for the small vectors and one for the sum, instead of eight round trips one behind
+// the other.  A chat of one stream, width 2048: 21.9 -> 21.35 ms with the state-space step below (6.3 and 5.4 us a launch before).
+template <typename T, bool AHEAD, int M>
 __global__ __launch_bounds__(256) void parallel_step_kernel(StepHeads sh, StepMemory m, const int* __restrict__ pos,
                                                             const int* __restrict__ live, int vb) {
   extern __shared__ __attribute__((aligned(16))) float lds[];      // [N] query, [N] key, [vb] weighted values
-  __shared__ float red[16], gates[2];
+  __shared__ float red[16];
   const int b = blockIdx.y, p = pos[b];
   const bool alive = live == nullptr || live[b] != 0;
   const int n_heads = sh.on ? sh.a.Hq + sh.a.Hkv : 0;
   if (static_cast<int>(blockIdx.x) < n_heads) {
-    head_step<T>(sh.a, b, blockIdx.x, p, alive, red);
+    head_step<T, M>(sh.a, b, blockIdx.x, p, alive, red);
     return;
   }
-  const int per = m.V / vb, i0 = blockIdx.x - n_heads, h = i0 / per, v0 = (i0 % per) * vb;
+  const int per = m.V / vb, i0 = blockIdx.x - n_heads, h = i0 / per, v0 = (i0 % per) * vb, tid = threadIdx.x;
   const int gi = b * m.H + h;
-  if (!alive) {                         // a parked sequence keeps its state
-    for (int i = threadIdx.x; i < vb; i += 256) m.out[static_cast<long long>(gi) * m.V + v0 + i] = 0.f;
-    return;
-  }
+  float* out = m.out + static_cast<long long>(gi) * m.V + v0;
   float* S = m.S + static_cast<long long>(gi) * m.V * m.N;
   const StateRows rows = request_state(S, m.N, v0, vb);
+  const int e0 = min(tid, m.N - 1);
+  const long long image = static_cast<long long>(m.slots) * m.H;
+  const float m_img[2] = {m.m[gi], m.m[image + gi]};
+  const float n_img[2] = {m.n[static_cast<long long>(gi) * m.N + e0], m.n[(image + gi) * m.N + e0]};
+  const float gi0 = src1<M>(m.src, b, m.i_col + h), gf0 = src1<M>(m.src, b, m.f_col + h), ib = m.ib[h], fb = m.fb[h];
+  const float q0 = src1<M>(m.src, b, m.q_col + h * m.N + e0), k0 = src1<M>(m.src, b, m.k_col + h * m.N + e0);
+  const float vr = src1<M>(m.src, b, m.v_col + h * m.V + v0 + min(tid, vb - 1));
+  if (!alive) {                         // a parked sequence keeps its state
+    for (int i = tid; i < vb; i += 256) out[i] = 0.f;
+    return;
+  }
   const bool fresh = p <= 0;
   float *qs = lds, *ks = lds + m.N, *avs = ks + m.N;
   const long long from = (static_cast<long long>(p & 1) * m.slots + b) * m.H + h;
   const long long to = (static_cast<long long>((p + 1) & 1) * m.slots + b) * m.H + h;
-  const float m_old = m.m[from];
-  const float n_old = m.n[from * m.N + min(static_cast<int>(threadIdx.x), m.N - 1)];
-  if (threadIdx.x == 255) {
-    gates[0] = m.cap * tanhf((src1(m.src, b, m.i_col + h) + m.ib[h]) / m.cap);
-    gates[1] = -softplus_f(-m.cap * tanhf((src1(m.src, b, m.f_col + h) + m.fb[h]) / m.cap));
-  }
-  for (int e = threadIdx.x; e < m.N; e += 256) {
-    qs[e] = src_t<T>(m.src, b, m.q_col + h * m.N + e) * m.qscale;
-    ks[e] = src_t<T>(m.src, b, m.k_col + h * m.N + e);
-  }
-  __syncthreads();
-  const float m0 = fresh ? 0.f : m_old;
-  const float li = gates[0], lf = gates[1], m1 = fmaxf(lf + m0, li);
-  const float decay = expf(lf + m0 - m1), add = expf(li - m1);
-  for (int i = threadIdx.x; i < vb; i += 256) avs[i] = add * src_t<T>(m.src, b, m.v_col + h * m.V + v0 + i);
+  const float li = m.cap * tanhf((gi0 + ib) / m.cap), lf = -softplus_f(-m.cap * tanhf((gf0 + fb) / m.cap));
+  const float mt = fresh ? 0.f : m_img[p & 1], m1 = fmaxf(lf + mt, li);
+  const float decay = expf(lf + mt - m1), add = expf(li - m1);
+  for (int i = tid; i < vb; i += 256) avs[i] = add * (i < 256 ? to_f32(from_f32<T>(vr)) : src_t<T, M>(m.src, b, m.v_col + h * m.V + v0 + i));
   float dot = 0.f;
-  for (int e = threadIdx.x; e < m.N; e += 256) {
-    const float n1 = (fresh ? 0.f : (e < 256 ? n_old : m.n[from * m.N + e]) * decay) + add * ks[e];
+  for (int e = tid; e < m.N; e += 256) {
+    const bool first = e < 256;
+    const float q = (first ? to_f32(from_f32<T>(q0)) : src_t<T, M>(m.src, b, m.q_col + h * m.N + e)) * m.qscale;
+    const float k = first ? to_f32(from_f32<T>(k0)) : src_t<T, M>(m.src, b, m.k_col + h * m.N + e);
+    qs[e] = q;
+    ks[e] = k;
+    const float n1 = (fresh ? 0.f : (first ? n_img[p & 1] : m.n[from * m.N + e]) * decay) + add * k;
     if (v0 == 0) m.n[to * m.N + e] = n1;
-    dot += n1 * qs[e];
+    dot += n1 * q;
   }
-  dot = block_sum<4>(dot, red);            // (its barriers also publish avs)
-  if (v0 == 0 && threadIdx.x == 0) m.m[to] = m1;
+  dot = block_sum<4>(dot, red);         // (its barriers also publish the vectors)
+  if (v0 == 0 && tid == 0) m.m[to] = m1;
   const float inv = 1.f / (fmaxf(fabsf(dot), expf(-m1)) + 1e-6f);
-  float* out = m.out + static_cast<long long>(gi) * m.V + v0;
   stream_state<AHEAD>(S, m.N, v0, vb, fresh, decay, qs, ks, avs, rows, [&](int i, float y) { out[i] = y * inv; });
 }
 
-// threads: one per convolution channel of the block where that is at most 512 (the state takes four waves)
-template <typename T, bool AHEAD>
+// threads: one per convolution channel of the block where that is at most 512 (the state takes four waves).  As above, with all
+// slots of the convolution's ring requested: the position picks among them.
+template <typename T, bool AHEAD, int M>
 __global__ __launch_bounds__(512) void ssd_step_kernel(StepSsd a, const int* __restrict__ pos, const int* __restrict__ live,
                                                        int vb) {
   extern __shared__ __attribute__((aligned(16))) float lds[];      // [N] C, [N] B, [vb] weighted x, [vb] x, [vb] silu(z)
-  __shared__ float gates[2];
   const int b = blockIdx.z, h = blockIdx.y, v0 = blockIdx.x * vb, p = pos[b];
   const int gi = b * a.H + h, per_group = a.H / a.G, g = h / per_group, nt = blockDim.x;
   float* out = a.out + static_cast<long long>(gi) * a.V + v0;
-  if (live && !live[b]) {
-    for (int i = threadIdx.x; i < vb; i += nt) out[i] = 0.f;
-    return;
-  }
   float* S = a.S + static_cast<long long>(gi) * a.V * a.N;
   const StateRows rows = request_state(S, a.N, v0, vb);
-  const bool fresh = p <= 0;
+  const float dt0 = src1<M>(a.src, b, a.dt_col + h), dt_bias = a.dt_bias[h], a_log = a.a_log[h], skip = a.skip[h];
+  const bool parked = live && !live[b];
   float *cs = lds, *bs = lds + a.N, *avs = bs + a.N, *xs = avs + vb, *zs = xs + vb;
   const int C = a.H * a.V + 2 * a.G * a.N;
-  if (static_cast<int>(threadIdx.x) == nt - 1) {
-    const float dt = softplus_f(src1(a.src, b, a.dt_col + h) + a.dt_bias[h]);
-    gates[0] = expf(-expf(a.a_log[h]) * dt);
-    gates[1] = dt;
-  }
   T* ring = static_cast<T*>(a.ring) + static_cast<long long>(b) * a.taps * C;
+  float dt = 0.f;
   for (int i = threadIdx.x; i < 2 * a.N + vb; i += nt) {
-    const bool is_x = i >= 2 * a.N;
+    const bool is_x = i >= 2 * a.N, first = i == static_cast<int>(threadIdx.x);
     const int c = is_x ? h * a.V + v0 + i - 2 * a.N
                        : a.H * a.V + (i < a.N ? g * a.N + i : (a.G + g) * a.N + i - a.N);     // B, then C
     const float* w = a.conv_w + static_cast<long long>(c) * a.taps;
     float acc = a.conv_b[c];
-    T cur;
+    const float now = src1<M>(a.src, b, a.x_col + c);
+    const float z0 = is_x ? src1<M>(a.src, b, a.z_col + c) : 0.f;
+    const T cur = from_f32<T>(now);
     if (a.taps == 4) {                  // (all operands on their way before the first product)
       const f32x4_t w4 = load4(w);
-      T old[3];
+      T old[4];
 #pragma unroll
-      for (int j = 0; j < 3; ++j) old[j] = ring[static_cast<long long>(max(p + j - 3, 0) & 3) * C + c];
-      cur = from_f32<T>(src1(a.src, b, a.x_col + c));
+      for (int j = 0; j < 4; ++j) old[j] = ring[static_cast<long long>(j) * C + c];
+      if (parked) break;
 #pragma unroll
-      for (int j = 0; j < 3; ++j) acc = fmaf(w4[j], p + j - 3 < 0 ? 0.f : to_f32(old[j]), acc);
+      for (int j = 0; j < 3; ++j) {
+        const int at = max(p + j - 3, 0) & 3;
+        const T o = at & 2 ? (at & 1 ? old[3] : old[2]) : (at & 1 ? old[1] : old[0]);
+        acc = fmaf(w4[j], p + j - 3 < 0 ? 0.f : to_f32(o), acc);
+      }
       acc = fmaf(w4[3], p < 0 ? 0.f : to_f32(cur), acc);
     } else {
-      cur = from_f32<T>(src1(a.src, b, a.x_col + c));
+      if (parked) break;
       for (int j = 0; j < a.taps; ++j) {
         const int d = a.taps - 1 - j;
         if (p - d < 0) continue;
@@ -222,22 +238,28 @@ __global__ __launch_bounds__(512) void ssd_step_kernel(StepSsd a, const int* __r
       }
     }
     const float v = to_f32(from_f32<T>(acc * sigmoid_f(acc)));
-    if (is_x) xs[i - 2 * a.N] = v;
-    else if (i < a.N) bs[i] = v;
-    else cs[i - a.N] = v;
-    // the current input's slot is read by nobody in this step; one block per channel stores it
+    if (first) dt = softplus_f(dt0 + dt_bias);
+    if (is_x) {
+      const float z = to_f32(from_f32<T>(z0));
+      xs[i - 2 * a.N] = v;
+      avs[i - 2 * a.N] = dt * v;
+      zs[i - 2 * a.N] = z * sigmoid_f(z);
+    } else if (i < a.N) {
+      bs[i] = v;
+    } else {
+      cs[i - a.N] = v;
+    }
+    // what is in the current input's slot is used by nobody in this step (requested with the others and dropped); one block per
+    // channel stores it
     if (is_x || (v0 == 0 && h % per_group == 0)) ring[static_cast<long long>(max(p, 0) % a.taps) * C + c] = cur;
   }
-  __syncthreads();
-  const float decay = gates[0], dt = gates[1];
-  for (int i = threadIdx.x; i < vb; i += nt) {
-    avs[i] = dt * xs[i];
-    const float z = src_t<T>(a.src, b, a.z_col + h * a.V + v0 + i);
-    zs[i] = z * sigmoid_f(z);
+  if (parked) {
+    for (int i = threadIdx.x; i < vb; i += nt) out[i] = 0.f;
+    return;
   }
+  const float decay = expf(-expf(a_log) * softplus_f(dt0 + dt_bias));
   __syncthreads();
-  const float skip = a.skip[h];
-  stream_state<AHEAD>(S, a.N, v0, vb, fresh, decay, cs, bs, avs, rows, [&](int i, float y) { out[i] = (y + skip * xs[i]) * zs[i]; });
+  stream_state<AHEAD>(S, a.N, v0, vb, p <= 0, decay, cs, bs, avs, rows, [&](int i, float y) { out[i] = (y + skip * xs[i]) * zs[i]; });
 }
 
 // state rows per block: sixteen keep a single stream's launch wide, more amortise the head's small vectors
@@ -252,18 +274,30 @@ void launch_parallel_step(const StepHeads& h, const StepMemory& m, const int* po
   const int vb = rows_per_block(m.H, m.V, B);
   const dim3 grid((h.on ? h.a.Hq + h.a.Hkv : 0) + m.H * (m.V / vb), B);
   const size_t lds = (2 * m.N + vb) * 4;
-  const auto kernel = vb > 16 ? (f32 ? &parallel_step_kernel<float, true> : &parallel_step_kernel<bf16_t, true>)
-                              : (f32 ? &parallel_step_kernel<float, false> : &parallel_step_kernel<bf16_t, false>);
-  hipLaunchKernelGGL(kernel, grid, dim3(256), lds, st, h, m, pos, live, vb);
+  // (both halves read the same projection; fp32 storage has one instance)
+  const bool same = !h.on || (h.a.src.p == m.src.p && src_mode(h.a.src) == src_mode(m.src));
+  const int mode = f32 || !same ? SRC_ANY : src_mode(m.src);
+  auto kernel = [&](auto ahead) {
+    constexpr bool A = decltype(ahead)::value;
+    if (f32) return &parallel_step_kernel<float, A, SRC_ANY>;
+    return mode == SRC_ONE ? &parallel_step_kernel<bf16_t, A, SRC_ONE>
+                           : mode == SRC_FOUR ? &parallel_step_kernel<bf16_t, A, SRC_FOUR> : &parallel_step_kernel<bf16_t, A, SRC_ANY>;
+  };
+  hipLaunchKernelGGL((vb > 16 ? kernel(std::true_type{}) : kernel(std::false_type{})), grid, dim3(256), lds, st, h, m, pos, live, vb);
 }
 void launch_ssd_step(const StepSsd& a, const int* pos, const int* live, bool f32, int B, hipStream_t st) {
   const int vb = rows_per_block(a.H, a.V, B);
   const dim3 grid(a.V / vb, a.H, B);
   const size_t lds = (2 * a.N + 3 * vb) * 4;
   const int threads = min(512, max(256, (2 * a.N + vb + 63) / 64 * 64));
-  const auto kernel = vb > 16 ? (f32 ? &ssd_step_kernel<float, true> : &ssd_step_kernel<bf16_t, true>)
-                              : (f32 ? &ssd_step_kernel<float, false> : &ssd_step_kernel<bf16_t, false>);
-  hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, st, a, pos, live, vb);
+  const int mode = f32 ? SRC_ANY : src_mode(a.src);
+  auto kernel = [&](auto ahead) {
+    constexpr bool A = decltype(ahead)::value;
+    if (f32) return &ssd_step_kernel<float, A, SRC_ANY>;
+    return mode == SRC_ONE ? &ssd_step_kernel<bf16_t, A, SRC_ONE>
+                           : mode == SRC_FOUR ? &ssd_step_kernel<bf16_t, A, SRC_FOUR> : &ssd_step_kernel<bf16_t, A, SRC_ANY>;
+  };
+  hipLaunchKernelGGL((vb > 16 ? kernel(std::true_type{}) : kernel(std::false_type{})), grid, dim3(threads), lds, st, a, pos, live, vb);
 }
 
 }  // namespace evgpt

@@ -20,17 +20,19 @@ namespace evgpt {
 
 // ---------------------------------------------------------------- prep
 // A block per row.  The first chunk of either section stays in registers, further ones are read again.
-template <typename T>
+template <typename T, int M>
 __global__ __launch_bounds__(256) void latent_prep_kernel(LatentPrepArgs a) {
   __shared__ float red[8];
   const long long row = blockIdx.x;
-  const int tid = threadIdx.x, Q = a.q_out ? a.Q : 0, R = a.cache && !(a.live && !a.live[row]) ? a.R : 0;
-  float vq[8], vc[8], sq = 0.f, sc = 0.f;
+  const int tid = threadIdx.x, Q = a.q_out ? a.Q : 0, R = a.cache ? a.R : 0;
+  float vq[8], vc[8], gq[8], gc[8], sq = 0.f, sc = 0.f;
   // the latents' chunks go to the last threads first: they are free where the query section is short of a full pass
   const int tc = 255 - tid;
+  if (tid * 8 < Q) load8(a.qw + tid * 8, gq);
+  if (tc * 8 < R) load8(a.cw + tc * 8, gc);
   for (int c = tid * 8; c < Q; c += 2048) {
     float v[8];
-    section8(a.src, row, a.q_col, a.nq, c, v);
+    section8<M>(a.src, row, a.q_col, a.nq, c, v);
     sq += sumsq8(v);
     if (c == tid * 8)
 #pragma unroll
@@ -38,41 +40,45 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(LatentPrepArgs a) {
   }
   for (int c = tc * 8; c < R; c += 2048) {
     float v[8];
-    section8(a.src, row, a.c_col, a.nc, c, v);
+    section8<M>(a.src, row, a.c_col, a.nc, c, v);
     sc += sumsq8(v);
     if (c == tc * 8)
 #pragma unroll
       for (int i = 0; i < 8; ++i) vc[i] = v[i];
   }
+  const bool alive = R > 0 && (!a.live || a.live[row]);
+  const long long slot = R > 0 && a.row_slot ? a.row_slot[row] : row;
+  const int p = R > 0 ? min(max(a.row_pos[row], 0), a.cap - 1) : 0;
   sq = wave_sum(sq);
   sc = wave_sum(sc);
   if ((tid & 63) == 0) { red[tid >> 6] = sq; red[4 + (tid >> 6)] = sc; }
   __syncthreads();
   const float rq = rsqrtf((red[0] + red[1] + red[2] + red[3]) / static_cast<float>(a.nq) + a.eps);
   const float rc = rsqrtf((red[4] + red[5] + red[6] + red[7]) / static_cast<float>(a.nc) + a.eps);
-  auto put = [&](int c, int first, const float (&kept)[8], int col, int n, const float* w, float r, T* out) {
+  auto put = [&](int c, int first, const float (&kept)[8], const float (&weight)[8], int col, int n, const float* w, float r, T* out) {
     float v[8], g[8];
     if (c == first) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = kept[i];
+      for (int i = 0; i < 8; ++i) { v[i] = kept[i]; g[i] = weight[i]; }
     } else {
-      section8(a.src, row, col, n, c, v);
+      section8<M>(a.src, row, col, n, c, v);
+      load8(w + c, g);
     }
-    load8(w + c, g);
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] *= r * g[i];
     store8(out + c, v);
   };
-  for (int c = tid * 8; c < Q; c += 2048) put(c, tid * 8, vq, a.q_col, a.nq, a.qw, rq, static_cast<T*>(a.q_out) + row * a.Q);
-  if (R == 0) return;
-  const long long slot = a.row_slot ? a.row_slot[row] : row;
-  const int p = min(max(a.row_pos[row], 0), a.cap - 1);
+  for (int c = tid * 8; c < Q; c += 2048) put(c, tid * 8, vq, gq, a.q_col, a.nq, a.qw, rq, static_cast<T*>(a.q_out) + row * a.Q);
+  if (!alive) return;
   T* out = static_cast<T*>(a.cache) + (slot * a.cap + p) * a.R;
-  for (int c = tc * 8; c < R; c += 2048) put(c, tc * 8, vc, a.c_col, a.nc, a.cw, rc, out);
+  for (int c = tc * 8; c < R; c += 2048) put(c, tc * 8, vc, gc, a.c_col, a.nc, a.cw, rc, out);
 }
 void launch_latent_prep(const LatentPrepArgs& a, bool f32, int rows, hipStream_t st) {
-  if (f32) hipLaunchKernelGGL(latent_prep_kernel<float>, dim3(rows), dim3(256), 0, st, a);
-  else hipLaunchKernelGGL(latent_prep_kernel<bf16_t>, dim3(rows), dim3(256), 0, st, a);
+  const int mode = f32 ? SRC_ANY : src_mode(a.src);
+  if (f32) hipLaunchKernelGGL((latent_prep_kernel<float, SRC_ANY>), dim3(rows), dim3(256), 0, st, a);
+  else if (mode == SRC_ONE) hipLaunchKernelGGL((latent_prep_kernel<bf16_t, SRC_ONE>), dim3(rows), dim3(256), 0, st, a);
+  else if (mode == SRC_FOUR) hipLaunchKernelGGL((latent_prep_kernel<bf16_t, SRC_FOUR>), dim3(rows), dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((latent_prep_kernel<bf16_t, SRC_ANY>), dim3(rows), dim3(256), 0, st, a);
 }
 
 // copies [n][4] of {slot, first position, first buffer row, count}; rows are vec 16-byte chunks
@@ -102,7 +108,7 @@ __device__ __forceinline__ int latent_len(const int* pos, int row, int cap) { re
 // Block: sixteen rows and one head.  WIDE: 64 outputs, 16 of them per wave column; otherwise 16.  The contraction is shared
 // by KW waves per column.  The rows' inputs are staged in LDS: columns of SrcRows, or the merge of attend's splits (a wave
 // per row).
-template <typename T, bool MERGE, bool WIDE, int KW>
+template <typename T, bool MERGE, bool WIDE, int KW, int XM, int GM>
 __global__ __launch_bounds__((WIDE ? 256 : 64) * KW) void head_linear_kernel(HeadLinearArgs a, int rows) {
   constexpr int WN = WIDE ? 4 : 1, NT = 64 * WN * KW;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -116,15 +122,18 @@ __global__ __launch_bounds__((WIDE ? 256 : 64) * KW) void head_linear_kernel(Hea
   const T* wp = static_cast<const T*>(a.w) + (static_cast<long long>(h) * a.N + min(n0 + fr, a.N - 1)) * K + g * 8;
   // the gate and the first weights are on their way while inputs are staged (32 rows of 16 heads, 512 x 128: 4.8-5.0 -> 4.4-4.9 us; behind a
   // merge the registers are not there for them, 9.4 -> 11.3)
-  constexpr int PF = MERGE ? 0 : 4;
-  Frag<T> wf[PF > 0 ? PF : 1];
+  constexpr int PF = 4;
+  Frag<T> wf[PF];
+  auto first_weights = [&]() {
 #pragma unroll
-  for (int i = 0; i < PF; ++i) wf[i] = load_frag(wp + min((wk + i * KW) * 32, K - 32));
-  const float gate = !MERGE && a.gate.p ? src1(a.gate, r0 + min(fr, nr - 1), a.gcol + h) : 0.f;
+    for (int i = 0; i < PF; ++i) wf[i] = load_frag(wp + min((wk + i * KW) * 32, K - 32));
+  };
+  if constexpr (!MERGE) first_weights();
+  const float gate = a.gate.p ? src1<GM>(a.gate, r0 + min(fr, nr - 1), a.gcol + h) : 0.f;
   if constexpr (MERGE) {
     // A wave takes a whole row (WIDE), or its share of the columns of every row with four groups of lanes on different
     // splits.  Maxima and sums (a lane per split, at most 64) are on their way together with the first partial rows.
-    constexpr int LG = WIDE ? 1 : 4, CL = 64 / LG, U = WIDE ? 8 : 4, STEP = WIDE ? 512 : CL * 8 * KW;
+    constexpr int LG = WIDE ? 1 : 4, CL = 64 / LG, U = 4, STEP = WIDE ? 512 : CL * 8 * KW;
     const int sg = lane / CL, c_lane = ((WIDE ? 0 : wk * CL) + lane % CL) * 8;
     for (int r = WIDE ? wid : 0; r < 16; r += WIDE ? NT / 64 : 1) {
       if (r >= nr) {
@@ -154,7 +163,10 @@ __global__ __launch_bounds__((WIDE ? 256 : 64) * KW) void head_linear_kernel(Hea
 #pragma unroll
           for (int u = 0; u < U; ++u) {
             const int s = s0 + u * LG + sg;
-            const float t = __shfl(f, s & 63, 64), fu = s < used ? t : 0.f;
+            float t;
+            if constexpr (WIDE) t = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), s & 63));
+            else t = __shfl(f, s & 63, 64);
+            const float fu = s < used ? t : 0.f;
 #pragma unroll
             for (int i = 0; i < 8; ++i) o[i] += fu * v[u][i];
           }
@@ -170,12 +182,13 @@ __global__ __launch_bounds__((WIDE ? 256 : 64) * KW) void head_linear_kernel(Hea
         if (sg == 0 && c0 + c_lane < K) store8(xs + r * ldx + c, o);
       }
     }
+    first_weights();
   } else {
     const int per = K >> 3;
     for (int i = tid; i < 16 * per; i += NT) {
       const int r = i / per, c = i % per * 8;
       float v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-      if (r < nr) src8(a.x, r0 + r, a.x_col + h * K + c, v);
+      if (r < nr) src8<XM>(a.x, r0 + r, a.x_col + h * K + c, v);
       store8(xs + r * ldx + c, v);
     }
   }
@@ -199,25 +212,36 @@ __global__ __launch_bounds__((WIDE ? 256 : 64) * KW) void head_linear_kernel(Hea
   const int n = n0 + g * 4;                       // N % 16 == 0: all four or none
   if (fr >= nr || n >= a.N) return;
   const long long row = r0 + fr;
-  if (a.gate.p) acc *= sigmoid_f(MERGE ? src1(a.gate, row, a.gcol + h) : gate);
+  if (a.gate.p) acc *= sigmoid_f(gate);
   store4(static_cast<T*>(a.y) + (row * a.H + h) * a.N + n, acc[0], acc[1], acc[2], acc[3]);
 }
-template <typename T, bool MERGE>
+template <typename T, bool MERGE, int XM, int GM>
 static void launch_heads(const HeadLinearArgs& a, int rows, hipStream_t st) {
   const int tiles = (rows + 15) / 16, wide = (a.N + 63) / 64;
   const size_t lds = 16ull * (a.K * sizeof(T) + 16);
   // the 64-wide tiles where they are enough blocks, or where inputs are merged (the narrow ones merge four times as often)
   if (MERGE && rows > 2)
-    hipLaunchKernelGGL((head_linear_kernel<T, MERGE, true, 4>), dim3(wide, a.H, tiles), dim3(1024), lds, st, a, rows);
+    hipLaunchKernelGGL((head_linear_kernel<T, MERGE, true, 4, XM, GM>), dim3(wide, a.H, tiles), dim3(1024), lds, st, a, rows);
   else if (static_cast<long long>(wide) * a.H * tiles >= 192)
-    hipLaunchKernelGGL((head_linear_kernel<T, MERGE, true, 1>), dim3(wide, a.H, tiles), dim3(256), lds, st, a, rows);
+    hipLaunchKernelGGL((head_linear_kernel<T, MERGE, true, 1, XM, GM>), dim3(wide, a.H, tiles), dim3(256), lds, st, a, rows);
   else
-    hipLaunchKernelGGL((head_linear_kernel<T, MERGE, false, 4>), dim3(a.N / 16, a.H, tiles), dim3(256), lds, st, a, rows);
+    hipLaunchKernelGGL((head_linear_kernel<T, MERGE, false, 4, XM, GM>), dim3(a.N / 16, a.H, tiles), dim3(256), lds, st, a, rows);
 }
 void launch_head_linear(const HeadLinearArgs& a, bool f32, int rows, hipStream_t st) {
-  if (a.part_o) launch_heads<bf16_t, true>(a, rows, st);
-  else if (f32) launch_heads<float, false>(a, rows, st);
-  else launch_heads<bf16_t, false>(a, rows, st);
+  const int x = a.part_o ? SRC_ANY : src_mode(a.x), gate = a.gate.p ? src_mode(a.gate) : SRC_ANY;
+  if (a.part_o) {
+    if (gate == SRC_ONE) launch_heads<bf16_t, true, SRC_ANY, SRC_ONE>(a, rows, st);
+    else if (gate == SRC_FOUR) launch_heads<bf16_t, true, SRC_ANY, SRC_FOUR>(a, rows, st);
+    else launch_heads<bf16_t, true, SRC_ANY, SRC_ANY>(a, rows, st);
+  } else if (f32) {
+    launch_heads<float, false, SRC_ANY, SRC_ANY>(a, rows, st);
+  } else if (!a.gate.p && x == SRC_ONE) {           // (only merged inputs are gated today)
+    launch_heads<bf16_t, false, SRC_ONE, SRC_ANY>(a, rows, st);
+  } else if (!a.gate.p && x == SRC_FOUR) {
+    launch_heads<bf16_t, false, SRC_FOUR, SRC_ANY>(a, rows, st);
+  } else {
+    launch_heads<bf16_t, false, SRC_ANY, SRC_ANY>(a, rows, st);
+  }
 }
 
 // ---------------------------------------------------------------- attend
@@ -310,8 +334,7 @@ __global__ __launch_bounds__(256 * HT) void latent_attend_kernel(const bf16_t* _
       if (k0 + w4 * 16 + g * 4 + r >= k_end) s0[r] = -INFINITY;
       mt = fmaxf(mt, s0[r]);
     }
-    mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
-    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+    mt = max_of_quads(mt);
     if (g == 0) s_max[ht][w4][fr] = mt;
     lds_barrier();
     mt = m;                                       // the tile's first key is there: finite

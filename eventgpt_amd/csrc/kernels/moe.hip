@@ -9,8 +9,9 @@
 namespace evgpt {
 
 // One wave: z [E] in LDS is used up (a lane touches its own entries only); lane k < top returns its expert and weight.
+template <int M = SRC_ANY>
 __device__ __forceinline__ void route_row(const MoeRoute& a, long long row, float* z, int lane, int& expert, float& weight) {
-  for (int e = lane; e < a.E; e += 64) z[e] = fmaxf(src1(a.z, row, e) + a.bias[e], -3.4e38f);   // (NaN: last)
+  for (int e = lane; e < a.E; e += 64) z[e] = fmaxf(src1<M>(a.z, row, e) + a.bias[e], -3.4e38f);   // (NaN: last)
   float best0 = 0.f, mine = -INFINITY;
   expert = 0;
   for (int k = 0; k < a.top; ++k) {
@@ -104,6 +105,7 @@ void launch_moe_group(const int* idx, int* perm, int* inv, int* start, int n, in
 // ballots.  One workgroup routes sixteen rows at a time and sorts sixteen experts at a time, one after the other, where the two launches spread
 // over the chip: see moe_route_group_ok.
 constexpr int RG_ROWS = 32, RG_ENTRIES = 128, RG_EXPERTS = 32;
+template <int M>
 __global__ __launch_bounds__(1024) void moe_route_group_kernel(MoeRoute a, float* __restrict__ w, int* __restrict__ perm, int* __restrict__ inv,
                                                                int* __restrict__ start, int rows) {
   extern __shared__ float z[];                     // [16][E]
@@ -112,7 +114,7 @@ __global__ __launch_bounds__(1024) void moe_route_group_kernel(MoeRoute a, float
   for (int row = wid; row < rows; row += 16) {
     int e;
     float f;
-    route_row(a, row, z + wid * a.E, lane, e, f);
+    route_row<M>(a, row, z + wid * a.E, lane, e, f);
     if (lane < a.top) {
       sel[row * a.top + lane] = e;
       w[static_cast<long long>(row) * a.top + lane] = f;
@@ -153,7 +155,10 @@ bool moe_route_group_ok(int rows, int E, int top) {
   return top <= (rows <= 16 ? (E <= 16 ? 8 : 6) : (E <= 16 ? 2 : 1));
 }
 void launch_moe_route_group(const MoeRoute& r, float* w, int* perm, int* inv, int* start, int rows, hipStream_t st) {
-  hipLaunchKernelGGL(moe_route_group_kernel, dim3(1), dim3(1024), 64 * r.E, st, r, w, perm, inv, start, rows);
+  const int mode = src_mode(r.z);
+  const auto kernel = mode == SRC_ONE ? &moe_route_group_kernel<SRC_ONE>
+                                      : mode == SRC_FOUR ? &moe_route_group_kernel<SRC_FOUR> : &moe_route_group_kernel<SRC_ANY>;
+  hipLaunchKernelGGL(kernel, dim3(1), dim3(1024), 64 * r.E, st, r, w, perm, inv, start, rows);
 }
 
 __device__ __forceinline__ float dot_chunk(const u32x4_t& w, const u32x4_t& x, float acc, bf16_t) { return dot8_bf16(w, x, acc); }

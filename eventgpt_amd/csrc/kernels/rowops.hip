@@ -36,7 +36,7 @@ void launch_embed_rows(const int* tok, const void* embed, bool f32, float scale,
 // first.  MODE 3: x += norm(a) wa first.  MODE 4: the same (or x += y without wa) with y the weighted sum of a few
 // rows of another matrix.  norm: RMS, or layer norm (LN).  A thread keeps its first NC chunks of eight in registers
 // between the passes; MODE 3 and 4 request the stream and the branch's weights with the branch.
-template <typename T, int MODE, bool LN, int NC>
+template <typename T, int MODE, bool LN, int NC, int M>
 __global__ __launch_bounds__(256) void residual_norm_kernel(float* __restrict__ x, const int* __restrict__ sel,
                                                             SrcRows a, SrcRows b, MixRows mix, const float* __restrict__ wa,
                                                             const float* __restrict__ wb, const float* __restrict__ w,
@@ -47,10 +47,16 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(float* __restrict__ 
   float keep[NC][8];
   constexpr int NX = MODE >= 3 ? NC : 1;
   float xk[NX][8], ak[NX][8];
+  // (the last norm's weights are on their way with everything else)
+  float wk[NC][8];
+  if (w != nullptr)
+#pragma unroll
+    for (int k = 0; k < NC; ++k)
+      if (const int c = (threadIdx.x + k * 256) * 8; c < ld) load8(w + c, wk[k]);
   float ra = 0.f, rb = 0.f;
   RowStat sy{0.f, 1.f};
   auto branch = [&](int c, float (&v)[8]) {          // MODE 3 and 4: the sublayer's output
-    if constexpr (MODE == 3) src8(a, row, c, v);
+    if constexpr (MODE == 3) src8<M>(a, row, c, v);
     if constexpr (MODE == 4) {
       const int* pick = mix.pick + row * mix.top;
       const float* pw = mix.w + row * mix.top;
@@ -70,9 +76,9 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(float* __restrict__ 
     float sa = 0.f, sb = 0.f;
     for (int c = threadIdx.x * 8; c < ld; c += 2048) {
       float t[8];
-      src8(a, row, c, t);
+      src8<M>(a, row, c, t);
       sa += sumsq8(t);
-      src8(b, row, c, t);
+      src8<M>(b, row, c, t);
       sb += sumsq8(t);
     }
     ra = 0.5f * rsqrtf(block_sum<4>(sa, red) * inv_n + eps);
@@ -98,14 +104,14 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(float* __restrict__ 
     load8(xr + c, v);
     if constexpr (MODE == 1) {
       float t[8];
-      src8(a, row, c, t);
+      src8<M>(a, row, c, t);
 #pragma unroll
       for (int i = 0; i < 8; ++i) v[i] += t[i];
     }
     if constexpr (MODE == 2) {
       float t[8], u[8], p[8], q[8];
-      src8(a, row, c, t);
-      src8(b, row, c, u);
+      src8<M>(a, row, c, t);
+      src8<M>(b, row, c, u);
       load8(wa + c, p);
       load8(wb + c, q);
 #pragma unroll
@@ -142,9 +148,7 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(float* __restrict__ 
   // each thread re-reads what it wrote
   const RowStat st = row_stat<NC>(keep, n, ld, eps, LN, red, [&](int c, float (&v)[8]) { load8(xr + c, v); });
   T* o = xn + row * ld;
-  auto put = [&](int c, const float (&v)[8]) {
-    float g[8];
-    load8(w + c, g);
+  auto put = [&](int c, const float (&v)[8], float (&g)[8]) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) g[i] *= (v[i] - st.mean) * st.r;
     store8(o + c, g);
@@ -152,26 +156,32 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(float* __restrict__ 
 #pragma unroll
   for (int k = 0; k < NC; ++k) {
     const int c = (threadIdx.x + k * 256) * 8;
-    if (c < ld) put(c, keep[k]);
+    if (c < ld) put(c, keep[k], wk[k]);
   }
   for (int c = (threadIdx.x + NC * 256) * 8; c < ld; c += 2048) {
-    float v[8];
+    float v[8], g[8];
     load8(xr + c, v);
-    put(c, v);
+    load8(w + c, g);
+    put(c, v, g);
   }
 }
 template <int MODE>
 static void launch_residual(float* x, const int* sel, const SrcRows& a, const SrcRows& b, const MixRows& mix, const float* wa,
                             const float* wb, const float* w, void* xn, bool f32, int rows, int n, int ld, float eps,
                             bool layer, hipStream_t st) {
+#define EVGPT_RES_M(T, LN, NC, M) hipLaunchKernelGGL((residual_norm_kernel<T, MODE, LN, NC, M>), dim3(rows), dim3(256), 0, st, x, sel, a, b, mix, \
+                                                     wa, wb, w, static_cast<T*>(xn), n, ld, eps)
 #define EVGPT_RES(T, LN) \
-  if (ld <= 4096) hipLaunchKernelGGL((residual_norm_kernel<T, MODE, LN, 2>), dim3(rows), dim3(256), 0, st, x, sel, a, b, mix, wa, wb, w, \
-                                     static_cast<T*>(xn), n, ld, eps); \
-  else hipLaunchKernelGGL((residual_norm_kernel<T, MODE, LN, 4>), dim3(rows), dim3(256), 0, st, x, sel, a, b, mix, wa, wb, w, \
-                          static_cast<T*>(xn), n, ld, eps)
+  if (ld > 4096) EVGPT_RES_M(T, LN, 4, SRC_ANY); \
+  else if (mode == SRC_ONE) EVGPT_RES_M(T, LN, 2, (MODE == 0 || MODE == 4 ? SRC_ANY : SRC_ONE)); \
+  else if (mode == SRC_FOUR) EVGPT_RES_M(T, LN, 2, (MODE == 0 || MODE == 4 ? SRC_ANY : SRC_FOUR)); \
+  else if (mode == SRC_EIGHT) EVGPT_RES_M(T, LN, 2, (MODE == 0 || MODE == 4 ? SRC_ANY : SRC_EIGHT)); \
+  else EVGPT_RES_M(T, LN, 2, SRC_ANY)
+  const int mode = MODE == 0 || MODE == 4 || (MODE == 2 && (!b.f32 || a.nslab != b.nslab)) || !a.f32 ? SRC_ANY : a.nslab;
   if (layer) { if (f32) { EVGPT_RES(float, true); } else { EVGPT_RES(bf16_t, true); } }
   else { if (f32) { EVGPT_RES(float, false); } else { EVGPT_RES(bf16_t, false); } }
 #undef EVGPT_RES
+#undef EVGPT_RES_M
 }
 void launch_norm_rows(const float* x, const int* sel, const float* w, void* xn, bool f32, int rows, int n, int ld,
                       float eps, bool layer, hipStream_t st) {
@@ -208,15 +218,15 @@ void launch_cap_logits(float* x, long long n, float scale, float cap, hipStream_
   hipLaunchKernelGGL(cap_logits_kernel, dim3(static_cast<unsigned>(want < 4096 ? want : 4096)), dim3(256), 0, st, x, n, scale, cap);
 }
 
-template <typename T, int ACT>
+template <typename T, int ACT, int M>
 __global__ __launch_bounds__(256) void glu_rows_kernel(SrcRows src, T* __restrict__ h, long long total, int ip) {
   const int per = ip >> 3;
   for (long long i = blockIdx.x * 256ll + threadIdx.x; i < total; i += gridDim.x * 256ll) {
     const long long row = i / per;
     const int c = static_cast<int>(i % per) * 8;
     float a[8], b[8];
-    src8(src, row, c, a);
-    src8(src, row, ip + c, b);
+    src8<M>(src, row, c, a);
+    src8<M>(src, row, ip + c, b);
 #pragma unroll
     for (int j = 0; j < 8; ++j) a[j] = (ACT == GLU_SILU ? a[j] * sigmoid_f(a[j]) : gelu_tanh_f(a[j])) * b[j];
     store8(h + row * ip + c, a);
@@ -226,13 +236,17 @@ void launch_glu_rows(const SrcRows& src, void* h, bool f32, int rows, int ip, in
   const long long total = static_cast<long long>(rows) * (ip / 8);
   const long long want = (total + 255) / 256;
   const dim3 grid(static_cast<unsigned>(want < 4096 ? want : 4096)), block(256);
-  if (f32) {
-    if (act == GLU_SILU) hipLaunchKernelGGL((glu_rows_kernel<float, GLU_SILU>), grid, block, 0, st, src, static_cast<float*>(h), total, ip);
-    else hipLaunchKernelGGL((glu_rows_kernel<float, GLU_GELU_TANH>), grid, block, 0, st, src, static_cast<float*>(h), total, ip);
-  } else {
-    if (act == GLU_SILU) hipLaunchKernelGGL((glu_rows_kernel<bf16_t, GLU_SILU>), grid, block, 0, st, src, static_cast<bf16_t*>(h), total, ip);
-    else hipLaunchKernelGGL((glu_rows_kernel<bf16_t, GLU_GELU_TANH>), grid, block, 0, st, src, static_cast<bf16_t*>(h), total, ip);
-  }
+  const int mode = f32 ? SRC_ANY : src_mode(src);
+#define EVGPT_GLU(T, ACT, M) hipLaunchKernelGGL((glu_rows_kernel<T, ACT, M>), grid, block, 0, st, src, static_cast<T*>(h), total, ip)
+#define EVGPT_GLU_ACT(ACT) \
+  if (f32) EVGPT_GLU(float, ACT, SRC_ANY); \
+  else if (mode == SRC_ONE) EVGPT_GLU(bf16_t, ACT, SRC_ONE); \
+  else if (mode == SRC_FOUR) EVGPT_GLU(bf16_t, ACT, SRC_FOUR); \
+  else EVGPT_GLU(bf16_t, ACT, SRC_ANY)
+  if (act == GLU_SILU) { EVGPT_GLU_ACT(GLU_SILU); }
+  else { EVGPT_GLU_ACT(GLU_GELU_TANH); }
+#undef EVGPT_GLU_ACT
+#undef EVGPT_GLU
 }
 
 // Group norm with a gate.  The row is staged in LDS (gated first when the gate comes before the norm), every

@@ -17,8 +17,18 @@ template <int S> __device__ __forceinline__ void sum_slabs8(const float* p, long
     for (int k = 1; k < S; ++k) o[i] += t[k][i];
   }
 }
+// What a kernel knows of its source when it is compiled: nothing, one matrix of fp32 rows, or four (eight: the residual kernel) fp32 slabs.  A source that is looked at
+// for every value puts its loads behind branches, where each waits for the one before it; the decode kernels, which are a handful of
+// such round trips long, have instances for the two that a decode step makes (`src_mode`).
+enum { SRC_ANY = 0, SRC_ONE = 1, SRC_FOUR = 4, SRC_EIGHT = 8 };
+__host__ inline int src_mode(const SrcRows& s) { return !s.f32 ? SRC_ANY : s.nslab == 1 ? SRC_ONE : s.nslab == 4 ? SRC_FOUR : SRC_ANY; }
+
 // eight consecutive values of a projection row
-__device__ __forceinline__ void src8(const SrcRows& s, long long row, int col, float (&o)[8]) {
+template <int M = SRC_ANY> __device__ __forceinline__ void src8(const SrcRows& s, long long row, int col, float (&o)[8]) {
+  if constexpr (M != SRC_ANY) {
+    sum_slabs8<M>(static_cast<const float*>(s.p) + row * s.ld + col, s.slab, o);
+    return;
+  }
   if (!s.f32) {
     load8(static_cast<const bf16_t*>(s.p) + row * s.ld + col, o);
     return;
@@ -37,7 +47,12 @@ __device__ __forceinline__ void src8(const SrcRows& s, long long row, int col, f
     }
   }
 }
-__device__ __forceinline__ float src1(const SrcRows& s, long long row, int col) {
+template <int M = SRC_ANY> __device__ __forceinline__ float src1(const SrcRows& s, long long row, int col) {
+  if constexpr (M != SRC_ANY) {
+    const float* p = static_cast<const float*>(s.p) + row * s.ld + col;
+    if constexpr (M == SRC_ONE) return p[0];
+    else return p[0] + p[s.slab] + p[2 * s.slab] + p[3 * s.slab];
+  }
   if (!s.f32) return bf16_to_f32(static_cast<const bf16_t*>(s.p)[row * s.ld + col]);
   const float* p = static_cast<const float*>(s.p) + row * s.ld + col;
   if (s.nslab == 4) return p[0] + p[s.slab] + p[2 * s.slab] + p[3 * s.slab];
@@ -46,8 +61,8 @@ __device__ __forceinline__ float src1(const SrcRows& s, long long row, int col) 
   return v;
 }
 // a projected value as a matrix stored in T would hold it
-template <typename T> __device__ __forceinline__ float src_t(const SrcRows& s, long long row, int col) {
-  return to_f32(from_f32<T>(src1(s, row, col)));
+template <typename T, int M = SRC_ANY> __device__ __forceinline__ float src_t(const SrcRows& s, long long row, int col) {
+  return to_f32(from_f32<T>(src1<M>(s, row, col)));
 }
 __device__ __forceinline__ float sumsq8(const float (&v)[8]) {
   float s = 0.f;
@@ -57,10 +72,10 @@ __device__ __forceinline__ float sumsq8(const float (&v)[8]) {
 }
 
 // eight columns of a section of `n` true columns; zeros past them
-__device__ __forceinline__ void section8(const SrcRows& s, long long row, int col, int n, int c, float (&v)[8]) {
-  if (c + 8 <= n) { src8(s, row, col + c, v); return; }
+template <int M = SRC_ANY> __device__ __forceinline__ void section8(const SrcRows& s, long long row, int col, int n, int c, float (&v)[8]) {
+  if (c + 8 <= n) { src8<M>(s, row, col + c, v); return; }
 #pragma unroll
-  for (int i = 0; i < 8; ++i) v[i] = c + i < n ? src1(s, row, col + c + i) : 0.f;
+  for (int i = 0; i < 8; ++i) v[i] = c + i < n ? src1<M>(s, row, col + c + i) : 0.f;
 }
 // RMS norm of `n` columns of a projection row by one wave, stored with zeros up to `ld` columns
 template <typename T>

@@ -938,3 +938,72 @@ def test_limits_are_refused(small):
     bad["layers"][0]["mixer"]["left"]["dim"] = 600
     with pytest.raises(ValueError):
         LayeredDecoder.from_config(LayeredConfig(bad), torch.bfloat16, small.device).engine(max_len=64)
+
+
+@pytest.mark.parametrize("slabs", [1, 2, 4, 8])
+def test_sources_of_the_step_kernels(raw, dev, slabs):
+    """A projection as one matrix, four (and eight) slabs, which have instances of their own, and two, which does not: every kernel of a
+    decode step gives the bits of the one matrix that holds the slabs' sum, taken in their order."""
+    f, B, W = dict(dtype=torch.float32, device=dev), 3, 512
+    g = torch.Generator().manual_seed(slabs)
+
+    def source(n):
+        t = torch.randn(slabs, B, n, generator=g).to(dev)
+        one = t[0].clone()
+        for i in range(1, slabs):
+            one += t[i]
+        return (t if slabs > 1 else t[0]), one
+    weight = [rnd(W, seed=i).float().to(dev) for i in range(2)]
+    y, y1 = source(W)
+    for op in (raw.post_norm_rows_, raw.add_norm_rows_):
+        out = []
+        for src in (y, y1):
+            x = torch.ones(B, W, **f)
+            extra = weight[:1] if op is raw.post_norm_rows_ else []
+            out += [op(x, src, *extra, weight[1], W - 3, 1e-5, False, False), x]
+        assert torch.equal(out[0], out[2]) and torch.equal(out[1], out[3])
+    a, b = source(W), source(W)
+    out = []
+    for i in range(2):
+        x = torch.ones(B, W, **f)
+        out += [raw.merge_norm_rows_(x, a[i], b[i], *weight, weight[0], W, 1e-5, False), x]
+    assert torch.equal(out[0], out[2]) and torch.equal(out[1], out[3])
+    assert torch.equal(*(raw.glu_rows(src, 1, False) for src in (y, y1)))
+    # matrix memory beside attention heads, and the state-space step
+    H, Nn, V, D = 2, 64, 64, 64
+    at = 3 * D
+    m_dims = [at, at + H * Nn, at + 2 * H * Nn, at + 2 * H * Nn + H * V, at + 2 * H * Nn + H * V + H, H, Nn, V]
+    src = source(m_dims[4] + H + (-(m_dims[4] + H)) % 8)
+    state = [torch.randn(*s, generator=g).to(dev) for s in ((B, H, V, Nn), (2, B, H, Nn), (2, B, H))]
+    ones, trig, ib = torch.ones(D, **f), torch.rand(16, 8, generator=g).to(dev), rnd(H, seed=6).float().to(dev)
+    pos, live = torch.tensor([0, 3, 6], dtype=torch.int32, device=dev), torch.tensor([1, 1, 0], dtype=torch.int32, device=dev)
+    got = []
+    for rows in src:
+        S, n, m = (t.clone() for t in state)
+        cache = torch.zeros(2, B, 1, 8, D, dtype=torch.bfloat16, device=dev)
+        q, o = raw.parallel_step_(rows, [0, D, 2 * D, 1, 1, D, D, D], ones, ones, 1e-3, trig, trig, cache[0], cache[1], m_dims, ib, ib, 5.0, 0.4, S, n, m,
+                                  pos, live)
+        got.append([q, o, S, n, m, cache])
+    assert all(torch.equal(x, y) for x, y in zip(*got))
+    G = 1
+    C, inner = H * V + 2 * G * Nn, H * V
+    conv, bias, dt_bias, a_log, skip = (rnd(*s, seed=i).float().to(dev) for i, s in enumerate([(C, 4), (C,), (H,), (H,), (H,)]))
+    src, ring0 = source(inner + C + H + (-H) % 8), torch.randn(B, 4, C, generator=g).to(torch.bfloat16).to(dev)
+    got = []
+    for rows in src:
+        S, ring = state[0].clone(), ring0.clone()
+        got.append([raw.ssd_step_(rows, [0, inner, inner + C, H, G, Nn, V], conv, bias, ring, dt_bias, a_log, skip, S, pos, live), S, ring])
+    assert all(torch.equal(x, y) for x, y in zip(*got))
+
+
+@pytest.mark.parametrize("rows,inner,K", [(1, 32, 128), (5, 96, 256), (16, 5632, 2048), (17, 160, 384), (32, 544, 640), (32, 32, 64), (33, 96, 256)])
+@pytest.mark.parametrize("act", [0, 1])
+def test_gated_products_of_few_rows(raw, dev, rows, inner, K, act):
+    """Up to 32 rows over whole K-tiles of 128 are one launch; other lengths and more rows are not."""
+    x, w = (typed(rnd(*s, seed=i, scale=0.3), torch.bfloat16, dev)[0] for i, s in enumerate([(rows, K), (2 * inner, K)]))
+    g, u = (x.double() @ t.double().t() for t in (w[:inner], w[inner:]))
+    f = torch.nn.functional.silu(g) if act == 1 else torch.nn.functional.gelu(g, approximate="tanh")
+    got = raw.linear_glu(x, w, act)
+    # one rounding to bf16 (the general product rounds its factors too); sums of K float32 products
+    bound = (f * u).abs() * 2.0 ** (-8 if rows <= 32 else -6) + K * 2.0 ** -22 * (f * u).abs().max()
+    assert bool(((got.double() - f * u).abs() <= bound).all())
