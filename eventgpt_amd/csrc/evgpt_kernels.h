@@ -110,6 +110,9 @@ void launch_gemm_glu(const bf16_t* A, const bf16_t* W, bf16_t* H, int M, int I, 
 // grouped product of experts; glu: 0 plain, otherwise 1 + the GLU activation of launch_gemm_glu
 void launch_gemm_grouped(const bf16_t* A, const bf16_t* W, bf16_t* C, const int* start, const int* perm, int top, int E,
                          int a_rows, int rows, int N, int K, int glu, hipStream_t st);
+// gated product of up to 32 rows, act(A Wgate^T) * (A Wup^T): a launch whose workgroups stream 32 gate and 32 up rows; whether it takes the sizes
+bool gemm_few_glu_serves(int rows, int I, int K);
+void launch_gemm_few_glu(const bf16_t* A, const bf16_t* W, bf16_t* C, int rows, int I, int K, int glu_act, hipStream_t st);
 bool launch_gemm_qkv_rope(const bf16_t* A, const bf16_t* W, int M, int K, bf16_t* q_out, bf16_t* k_cache,
                           bf16_t* v_cache, const float* cos_tab, const float* sin_tab, const int* pos0, int Hq,
                           int Hkv, int l_max, hipStream_t st);

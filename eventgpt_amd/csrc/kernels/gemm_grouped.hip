@@ -18,7 +18,8 @@ namespace {
 
 constexpr int TK = 128, AM = 32, TN = 32, STAGES = 3, RUN = 16;
 
-template <bool GLU>
+// ONE: all rows are one group (a dense gated product of a decode step); its gate and up sums are not rounded on the way
+template <bool GLU, bool ONE>
 __global__ __launch_bounds__(256) void gemm_grouped_few_kernel(EVGPT_GEMM_ARGS) {
   EVGPT_GEMM_TAKE;
   constexpr int W_ROWS = GLU ? 2 * TN : TN, WI = W_ROWS / 16;      // staging instructions per wave: 4 rows x 256 bytes each
@@ -32,9 +33,14 @@ __global__ __launch_bounds__(256) void gemm_grouped_few_kernel(EVGPT_GEMM_ARGS) 
   // level), single tiles read 4096 k slower than runs do (0.85 against 0.79).
   const int xcd = blockIdx.x & 7, turn = blockIdx.x >> 3;
   int tile = ((turn / RUN) * 8 + xcd) * RUN + turn % RUN;
-  const int e = group_of_tile(p.grp_start, p.grp_count, AM, tiles_n, tile);
-  if (e < 0) return;
-  const int first = p.grp_start[e], all = p.grp_start[e + 1] - first;
+  int e = 0, first = 0, all = p.M;
+  if constexpr (ONE) {
+    if (tile >= (p.M + AM - 1) / AM * tiles_n) return;
+  } else {
+    e = group_of_tile(p.grp_start, p.grp_count, AM, tiles_n, tile);
+    if (e < 0) return;
+    first = p.grp_start[e], all = p.grp_start[e + 1] - first;
+  }
   const int tiles_m = (all + AM - 1) / AM;
   const int m0 = tile % tiles_m * AM, n0 = tile / tiles_m * TN, rows = min(all - m0, AM);
   const int nk = p.K / TK;
@@ -46,7 +52,7 @@ __global__ __launch_bounds__(256) void gemm_grouped_few_kernel(EVGPT_GEMM_ARGS) 
 #pragma unroll
     for (int i = 0; i < AI; ++i) {
       const int row = (wid * AI + i) * 4 + r4, at = first + m0 + min(row, rows - 1);
-      const int src = p.grp_perm ? p.grp_perm[at] / p.grp_top : at;
+      const int src = !ONE && p.grp_perm ? p.grp_perm[at] / p.grp_top : at;
       voff_a[i] = row < rows ? (src * p.lda + ((slot ^ (row & 15)) * 8)) * 2 : 0x7fffff00;     // (past the range: zeros)
     }
 #pragma unroll
@@ -55,7 +61,7 @@ __global__ __launch_bounds__(256) void gemm_grouped_few_kernel(EVGPT_GEMM_ARGS) 
       voff_w[i] = ((n0 + (row & (TN - 1)) + (row / TN) * p.glu_half) * p.ldw + ((slot ^ (row & 15)) * 8)) * 2;
     }
     const unsigned char* A = reinterpret_cast<const unsigned char*>(p.A);
-    const unsigned char* W = reinterpret_cast<const unsigned char*>(p.W + e * p.grp_wstride);
+    const unsigned char* W = reinterpret_cast<const unsigned char*>(p.W + (ONE ? 0 : e * p.grp_wstride));
     const int bytes_a = 2 * p.M * p.lda, bytes_w = 2 * (GLU ? 2 * p.glu_half : p.N) * p.ldw;
     auto stage_w = [&](int buf, int kt) {
 #pragma unroll
@@ -119,7 +125,8 @@ __global__ __launch_bounds__(256) void gemm_grouped_few_kernel(EVGPT_GEMM_ARGS) 
       float v[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        v[r] = GLU ? glu_gate(bf16_to_f32(f32_to_bf16(acc[i][r])), p.glu_act) * bf16_to_f32(f32_to_bf16(o[r])) : acc[i][r] + o[r];
+        v[r] = !GLU ? acc[i][r] + o[r] : ONE ? glu_gate(acc[i][r], p.glu_act) * o[r]
+                                             : glu_gate(bf16_to_f32(f32_to_bf16(acc[i][r])), p.glu_act) * bf16_to_f32(f32_to_bf16(o[r]));
       if (i * 16 + frow < rows) {
         const u32x2_t w = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
         *reinterpret_cast<u32x2_t*>(p.C + static_cast<size_t>(first + m0 + i * 16 + frow) * p.ldc + n0 + col * 16 + fq * 4) = w;
@@ -130,13 +137,13 @@ __global__ __launch_bounds__(256) void gemm_grouped_few_kernel(EVGPT_GEMM_ARGS) 
   else run(std::integral_constant<int, 2>{});
 }
 
-template <bool GLU>
+template <bool GLU, bool ONE>
 void launch(const GemmParams& p, int grid, hipStream_t st) {
   constexpr int smem = STAGES * (AM + (GLU ? 2 * TN : TN)) * TK * 2;
-  static const bool attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_grouped_few_kernel<GLU>),
+  static const bool attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_grouped_few_kernel<GLU, ONE>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, smem) == hipSuccess;
   (void)attr;
-  hipLaunchKernelGGL((gemm_grouped_few_kernel<GLU>), dim3(grid), dim3(256), smem, st, EVGPT_GEMM_PASS(p));
+  hipLaunchKernelGGL((gemm_grouped_few_kernel<GLU, ONE>), dim3(grid), dim3(256), smem, st, EVGPT_GEMM_PASS(p));
 }
 
 }  // namespace
@@ -154,8 +161,19 @@ bool gemm_grouped_few_serves(const GemmParams& p, int rows) {
 void launch_gemm_grouped_few(const GemmParams& p, int rows, hipStream_t st) {
   const int most = (rows / AM + p.grp_count) * (p.N / TN);        // at least as many as there can be
   const int grid = (most + 8 * RUN - 1) / (8 * RUN) * (8 * RUN);  // every XCD's whole turns
-  if (p.glu_half) launch<true>(p, grid, st);
-  else launch<false>(p, grid, st);
+  if (p.glu_half) launch<true, false>(p, grid, st);
+  else launch<false, false>(p, grid, st);
+}
+
+// A dense gated product of a decode step.  us against the slabs of gemm_fewrow_kernel and the launch that sums and gates them, 5 / 32 rows:
+// 2 x 2816 columns over 1024 k 6.0 / 6.5 against 8.0 / 8.8, 2 x 5632 over 2048 11.5 / 13.3 and 14.5 / 15.9, 2 x 11008 over 4096 39.2 / 42.8 and 38.6 /
+// 42.8 (344 workgroups: a round and a third of one a CU), 2 x 13824 over 5120 51.6 / 57.7 and 56.8 / 66.0; the error against 64 bits is the same.
+bool gemm_few_glu_serves(int rows, int I, int K) { return rows <= AM && K % TK == 0 && I % TN == 0; }
+void launch_gemm_few_glu(const bf16_t* A, const bf16_t* W, bf16_t* C, int rows, int I, int K, int glu_act, hipStream_t st) {
+  GemmParams p{};
+  p.A = A, p.W = W, p.C = C, p.M = rows, p.N = I, p.K = p.lda = p.ldw = K, p.ldc = I, p.splitk = 1, p.k_per_split = K;
+  p.glu_half = I, p.glu_act = glu_act;
+  launch<true, true>(p, (I / TN + 8 * RUN - 1) / (8 * RUN) * (8 * RUN), st);
 }
 
 }  // namespace evgpt

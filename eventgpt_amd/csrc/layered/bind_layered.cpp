@@ -95,6 +95,15 @@ Tensor linear_glu(const Tensor& x, const Tensor& w, int64_t act) {
   TORCH_CHECK(act == evgpt::GLU_GELU_TANH || act == evgpt::GLU_SILU, "linear_glu: act 0 or 1");
   TORCH_CHECK(w.dim() == 2 && w.size(0) % 64 == 0, "linear_glu: w_gate_up [2 I, K], I % 32 == 0");
   const int64_t I = w.size(0) / 2;
+  if (!is_f32(x) && x.dim() == 2 && evgpt::gemm_few_glu_serves((int)x.size(0), (int)I, (int)x.size(1))) {
+    check_t(x, "x"); check_t(w, "w");
+    const int64_t M = x.size(0), K = x.size(1);
+    TORCH_CHECK(M >= 1 && !is_f32(w) && w.size(1) == K, "linear_glu: x [M, K], w [2 I, K] of one type");
+    TORCH_CHECK(2 * I * K < (1ll << 30), "linear_glu: operands are addressed with 32-bit offsets");
+    Tensor h = at::empty({M, I}, x.options());
+    evgpt::launch_gemm_few_glu(bptr(x), bptr(w), bptr_mut(h), (int)M, (int)I, (int)K, act == evgpt::GLU_SILU ? 0 : 1, cur_stream());
+    return h;
+  }
   if (is_f32(x) || x.size(0) <= 32) {
     const Tensor y = is_f32(x) ? linear(x, w, true) : linear_slabs(x, w);
     Tensor h = at::empty({x.size(0), I}, x.options());
