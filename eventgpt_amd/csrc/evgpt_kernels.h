@@ -300,6 +300,8 @@ void launch_argmax_pair_local(const float* part_val, const int* part_idx, int B,
 void launch_argmax_pair_select(const unsigned* pairs, int W, int B, int* token, hipStream_t st);
 
 // ---- attn_decode.hip
+// out [B][Hq][D] from the splits' partial results (at most 16)
+void launch_attn_decode_merge(const float* part_o, const float* part_ml, bf16_t* out, int B, int Hq, int D, int nsplit, hipStream_t st);
 void launch_attn_decode(const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_cache,
                         bf16_t* out, float* part_o, float* part_ml, const int* pos, int B, int Hq,
                         int Hkv, int D, int l_max, int nsplit, float scale, hipStream_t st, int ring = 0);

@@ -156,6 +156,12 @@ __global__ __launch_bounds__(D) void attn_decode_combine_kernel(const float* __r
   out[(static_cast<size_t>(b) * Hq + h) * D + d] = f32_to_bf16(oo / ll);
 }
 
+void launch_attn_decode_merge(const float* part_o, const float* part_ml, bf16_t* out, int B, int Hq, int D, int nsplit, hipStream_t st) {
+  if (D == 128)
+    hipLaunchKernelGGL(attn_decode_combine_kernel<128>, dim3(Hq, B), dim3(128), 0, st, part_o, part_ml, out, Hq, nsplit);
+  else
+    hipLaunchKernelGGL(attn_decode_combine_kernel<64>, dim3(Hq, B), dim3(64), 0, st, part_o, part_ml, out, Hq, nsplit);
+}
 void launch_attn_decode(const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_cache,
                         bf16_t* out, float* part_o, float* part_ml, const int* pos, int B, int Hq,
                         int Hkv, int D, int l_max, int nsplit, float scale, hipStream_t st,
@@ -173,14 +179,11 @@ void launch_attn_decode(const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_
   if (D == 128) {
     hipLaunchKernelGGL((attn_decode_split_kernel<128, false>), grid, block, 0, st, q, k_cache, v_cache,
                        part_o, part_ml, pos, Hq, Hkv, l_max, scale, out, ring);
-    hipLaunchKernelGGL(attn_decode_combine_kernel<128>, dim3(Hq, B), dim3(128), 0, st, part_o,
-                       part_ml, out, Hq, nsplit);
   } else {
     hipLaunchKernelGGL((attn_decode_split_kernel<64, false>), grid, block, 0, st, q, k_cache, v_cache,
                        part_o, part_ml, pos, Hq, Hkv, l_max, scale, out, ring);
-    hipLaunchKernelGGL(attn_decode_combine_kernel<64>, dim3(Hq, B), dim3(64), 0, st, part_o,
-                       part_ml, out, Hq, nsplit);
   }
+  launch_attn_decode_merge(part_o, part_ml, out, B, Hq, D, nsplit, st);
 }
 
 }  // namespace evgpt

@@ -138,18 +138,8 @@ __device__ void head_step(const AttnPrepArgs& a, int b, int head, int p, bool li
 // kernel is the slowest of these loads, one barrier for the small vectors and one for the sum, instead of eight round trips one behind
 // the other.  A chat of one stream, width 2048: 21.9 -> 21.35 ms with the state-space step below (6.3 and 5.4 us a launch before).
 template <typename T, bool AHEAD, int M>
-__global__ __launch_bounds__(256) void parallel_step_kernel(StepHeads sh, StepMemory m, const int* __restrict__ pos,
-                                                            const int* __restrict__ live, int vb) {
-  extern __shared__ __attribute__((aligned(16))) float lds[];      // [N] query, [N] key, [vb] weighted values
-  __shared__ float red[16];
-  const int b = blockIdx.y, p = pos[b];
-  const bool alive = live == nullptr || live[b] != 0;
-  const int n_heads = sh.on ? sh.a.Hq + sh.a.Hkv : 0;
-  if (static_cast<int>(blockIdx.x) < n_heads) {
-    head_step<T, M>(sh.a, b, blockIdx.x, p, alive, red);
-    return;
-  }
-  const int per = m.V / vb, i0 = blockIdx.x - n_heads, h = i0 / per, v0 = (i0 % per) * vb, tid = threadIdx.x;
+__device__ __forceinline__ void memory_step(const StepMemory& m, int b, int i0, int vb, int p, bool alive, float* lds, float* red) {
+  const int per = m.V / vb, h = i0 / per, v0 = (i0 % per) * vb, tid = threadIdx.x;
   const int gi = b * m.H + h;
   float* out = m.out + static_cast<long long>(gi) * m.V + v0;
   float* S = m.S + static_cast<long long>(gi) * m.V * m.N;
@@ -188,6 +178,160 @@ __global__ __launch_bounds__(256) void parallel_step_kernel(StepHeads sh, StepMe
   if (v0 == 0 && tid == 0) m.m[to] = m1;
   const float inv = 1.f / (fmaxf(fabsf(dot), expf(-m1)) + 1e-6f);
   stream_state<AHEAD>(S, m.N, v0, vb, fresh, decay, qs, ks, avs, rows, [&](int i, float y) { out[i] = y * inv; });
+}
+template <typename T, bool AHEAD, int M>
+__global__ __launch_bounds__(256) void parallel_step_kernel(StepHeads sh, StepMemory m, const int* __restrict__ pos,
+                                                            const int* __restrict__ live, int vb) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];      // [N] query, [N] key, [vb] weighted values
+  __shared__ float red[16];
+  const int b = blockIdx.y, p = pos[b];
+  const bool alive = live == nullptr || live[b] != 0;
+  const int n_heads = sh.on ? sh.a.Hq + sh.a.Hkv : 0;
+  if (static_cast<int>(blockIdx.x) < n_heads) head_step<T, M>(sh.a, b, blockIdx.x, p, alive, red);
+  else memory_step<T, AHEAD, M>(m, b, blockIdx.x - n_heads, vb, p, alive, lds, red);
+}
+
+// The same step with the attention over the cached keys in it, for a few sequences: a block takes a head's query (norm, rotation) and one
+// of the splits of its keys, which are on their way meanwhile; the new key and value, which the cache will only hold afterwards,
+// are made by the blocks of the first split and join there.  What is left of the attention is the merge of the splits.
+// Partial results as attn_decode_split_kernel leaves them.
+// A chat of one stream, width 2048, 100 + 64 tokens: 21.35 -> 20.9 ms (a launch of 4.1 us and its gap less in every second layer).
+template <int D, int M>
+__device__ __forceinline__ void attend_split(const AttnPrepArgs& a, const StepSplits& sp, int b, int h, int split, int p, bool live) {
+  constexpr int LPK = D / 8, KPW = 64 / LPK, U = 4, NP = 4 * KPW;
+  __shared__ __attribute__((aligned(16))) float s_o[NP][D];
+  __shared__ float s_m[NP], s_l[NP], sums[8];
+  __shared__ __attribute__((aligned(16))) bf16_t vec[3][D];        // query, new key, new value
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, sub = lane / LPK, dl = lane % LPK;
+  const int hk = h / (a.Hq / a.Hkv), slot = max(p, 0) % a.cap;      // keys 0 .. slot - 1 are cached
+  const int ngroups = (slot + KPW - 1) / KPW, gper = (ngroups + sp.nsplit - 1) / sp.nsplit;
+  const int g0 = split * gper, g1 = min(g0 + gper, ngroups);
+  const bf16_t* kb = static_cast<const bf16_t*>(a.k_cache) + (static_cast<long long>(b) * a.Hkv + hk) * a.cap * D + dl * 8;
+  const bf16_t* vb = static_cast<const bf16_t*>(a.v_cache) + (static_cast<long long>(b) * a.Hkv + hk) * a.cap * D + dl * 8;
+  u32x4_t kv[U], vv[U];
+  int key[U];
+  auto request = [&](int g) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      key[u] = (g + u) * KPW + sub;
+      const bool ok = g + u < g1 && key[u] < slot;
+      const int kk = ok ? key[u] : 0;
+      kv[u] = load16(kb + static_cast<long long>(kk) * D);
+      vv[u] = load16(vb + static_cast<long long>(kk) * D);
+      if (!ok) key[u] = -1;
+    }
+  };
+  request(g0 + wid * U);
+  // a thread's element: of the query (first D threads), of the new key and value (next D)
+  const bool is_q = tid < D;
+  const int d = tid & (D - 1), half = a.rot >> 1;
+  const int col = is_q ? a.q_col + h * D : a.k_col + hk * D, wrow = is_q ? h * D : hk * D;
+  const float* w = is_q ? a.qw : a.kw;
+  const int d2 = d < a.rot ? (d < half ? d + half : d - half) : d;
+  const float u0 = src1<M>(a.src, b, col + d), o0 = src1<M>(a.src, b, col + d2);
+  const float v0 = src1<M>(a.src, b, a.v_col + hk * D + d);
+  const float wu = w ? w[wrow + d] : 1.f, wo = w ? w[wrow + d2] : 1.f;
+  const int pt = min(max(p, 0), a.max_pos - 1), i = min(d < half ? d : d - half, half - 1);
+  const float cs = half > 0 ? a.cos_tab[static_cast<long long>(pt) * half + max(i, 0)] : 1.f;
+  const float sn = half > 0 ? a.sin_tab[static_cast<long long>(pt) * half + max(i, 0)] : 0.f;
+  auto total = [&](const float* norm, int c0, int width) {
+    float s = 0.f;
+    if (norm)
+      for (int c = tid * 8; c < width; c += 2048) {
+        float t[8];
+        src8<M>(a.src, b, c0 + c, t);
+        s += sumsq8(t);
+      }
+    return wave_sum(s);
+  };
+  const float sq = total(a.qw, a.q_col, a.Hq * D), sk = total(a.kw, a.k_col, a.Hkv * D);
+  if (lane == 0) { sums[wid] = sq; sums[4 + wid] = sk; }
+  __syncthreads();
+  const int at = is_q ? 0 : 4;
+  const float r = w ? rsqrtf((sums[at] + sums[at + 1] + sums[at + 2] + sums[at + 3]) / static_cast<float>(is_q ? a.nq : a.nk) + a.eps) : 1.f;
+  float u = u0 * r * wu;
+  if (d < a.rot) {
+    const float o = o0 * r * wo;
+    u = d < half ? u * cs - o * sn : u * cs + o * sn;
+  }
+  if (tid < 2 * D) vec[is_q ? 0 : 1][d] = f32_to_bf16(u);
+  if (tid >= D && tid < 2 * D) vec[2][d] = f32_to_bf16(v0);
+  __syncthreads();
+  if (split == 0 && live && h % (a.Hq / a.Hkv) == 0 && tid >= D && tid < 2 * D) {
+    const long long o = ((static_cast<long long>(b) * a.Hkv + hk) * a.cap + slot) * D + d;
+    static_cast<bf16_t*>(a.k_cache)[o] = vec[1][d];
+    static_cast<bf16_t*>(a.v_cache)[o] = vec[2][d];
+  }
+  const u32x4_t qv = *reinterpret_cast<const u32x4_t*>(&vec[0][dl * 8]);
+  float mx = -INFINITY, l = 0.f, o[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  for (int g = g0 + wid * U; g < g1; g += 4 * U) {
+    if (g != g0 + wid * U) request(g);
+    float sc[U], mn = mx;
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      sc[k] = group_sum<LPK>(dot8_bf16(qv, kv[k], 0.f)) * sp.scale;
+      if (key[k] >= 0) mn = fmaxf(mn, sc[k]);
+    }
+    const float al = mn == -INFINITY ? 1.f : __expf(mx - mn);
+    l *= al;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] *= al;
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      const float pr = key[k] >= 0 ? __expf(sc[k] - mn) : 0.f;
+      l += pr;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        o[2 * e] += pr * bf16lo(vv[k][e]);
+        o[2 * e + 1] += pr * bf16hi(vv[k][e]);
+      }
+    }
+    mx = mn;
+  }
+  if (split == 0 && wid == 0) {                       // the new key: the first group of lanes
+    const float sc = group_sum<LPK>(dot8_bf16(qv, *reinterpret_cast<const u32x4_t*>(&vec[1][dl * 8]), 0.f)) * sp.scale;
+    const u32x4_t nv = *reinterpret_cast<const u32x4_t*>(&vec[2][dl * 8]);
+    if (sub == 0) {
+      const float mn = fmaxf(mx, sc), al = __expf(mx - mn), pr = __expf(sc - mn);     // (mx = -inf: al = 0)
+      l = l * al + pr;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        o[2 * e] = o[2 * e] * al + pr * bf16lo(nv[e]);
+        o[2 * e + 1] = o[2 * e + 1] * al + pr * bf16hi(nv[e]);
+      }
+      mx = mn;
+    }
+  }
+  const int pidx = wid * KPW + sub;
+  *reinterpret_cast<f32x4_t*>(&s_o[pidx][dl * 8]) = f32x4_t{o[0], o[1], o[2], o[3]};
+  *reinterpret_cast<f32x4_t*>(&s_o[pidx][dl * 8 + 4]) = f32x4_t{o[4], o[5], o[6], o[7]};
+  if (dl == 0) { s_m[pidx] = mx; s_l[pidx] = l; }
+  __syncthreads();
+  if (tid < D) {
+    float mm = s_m[0];
+#pragma unroll
+    for (int k = 1; k < NP; ++k) mm = fmaxf(mm, s_m[k]);
+    float ll = 0.f, oo = 0.f;
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+      const float c = s_m[k] == -INFINITY ? 0.f : __expf(s_m[k] - mm);
+      ll += s_l[k] * c;
+      oo += s_o[k][tid] * c;
+    }
+    const long long at_split = (static_cast<long long>(b) * a.Hq + h) * sp.nsplit + split;
+    sp.part_o[at_split * D + tid] = oo;
+    if (tid == 0) { sp.part_ml[at_split * 2] = mm; sp.part_ml[at_split * 2 + 1] = ll; }
+  }
+}
+template <int D, bool AHEAD, int M>
+__global__ __launch_bounds__(256) void attend_step_kernel(const int* __restrict__ pos, const int* __restrict__ live, int vb, StepHeads sh,
+                                                          StepSplits sp, StepMemory m) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  __shared__ float red[16];
+  const int b = blockIdx.y, p = pos[b], i = blockIdx.x, n_attend = sh.a.Hq * sp.nsplit;
+  const bool alive = live == nullptr || live[b] != 0;
+  if (i < n_attend) attend_split<D, M>(sh.a, sp, b, i % sh.a.Hq, i / sh.a.Hq, p, alive);
+  else memory_step<bf16_t, AHEAD, M>(m, b, i - n_attend, vb, p, alive, lds, red);
 }
 
 // threads: one per convolution channel of the block where that is at most 512 (the state takes four waves).  As above, with all
@@ -284,6 +428,19 @@ void launch_parallel_step(const StepHeads& h, const StepMemory& m, const int* po
                            : mode == SRC_FOUR ? &parallel_step_kernel<bf16_t, A, SRC_FOUR> : &parallel_step_kernel<bf16_t, A, SRC_ANY>;
   };
   hipLaunchKernelGGL((vb > 16 ? kernel(std::true_type{}) : kernel(std::false_type{})), grid, dim3(256), lds, st, h, m, pos, live, vb);
+}
+bool attend_step_ok(const StepHeads& h, const StepMemory& m, int B, int nsplit) {
+  return B <= GEMV_ROWS_MAX && nsplit > 1 && nsplit <= 16 && (h.a.D == 64 || h.a.D == 128) && src_mode(m.src) == SRC_ONE && h.a.src.p == m.src.p;
+}
+void launch_attend_step(const StepHeads& h, const StepMemory& m, const StepSplits& sp, const int* pos, const int* live, int B, hipStream_t st) {
+  const int vb = rows_per_block(m.H, m.V, B);
+  const dim3 grid(h.a.Hq * sp.nsplit + m.H * (m.V / vb), B);
+  const size_t lds = (2 * m.N + vb) * 4;
+  const bool ahead = vb > 16;
+#define EVGPT_ATTEND_STEP(D, A) hipLaunchKernelGGL((attend_step_kernel<D, A, SRC_ONE>), grid, dim3(256), lds, st, pos, live, vb, h, sp, m)
+  if (h.a.D == 128) { if (ahead) EVGPT_ATTEND_STEP(128, true); else EVGPT_ATTEND_STEP(128, false); }
+  else { if (ahead) EVGPT_ATTEND_STEP(64, true); else EVGPT_ATTEND_STEP(64, false); }
+#undef EVGPT_ATTEND_STEP
 }
 void launch_ssd_step(const StepSsd& a, const int* pos, const int* live, bool f32, int B, hipStream_t st) {
   const int vb = rows_per_block(a.H, a.V, B);

@@ -508,7 +508,7 @@ Tensor scan_prefill_(const Tensor& q, const Tensor& k, const Tensor& v, int64_t 
 // ---------------------------------------------------------------- decode steps
 // One token per sequence from the projection rows `src`: the attention heads (norm, rotation, cache append; q is
 // returned) and the matrix memory (its output is returned, fp32).  Rows whose `live` is 0 change no state.
-std::tuple<Tensor, Tensor> parallel_step_(const Tensor& src, at::IntArrayRef attn, const OptTensor& qw, const OptTensor& kw,
+std::tuple<Tensor, Tensor> step_heads(bool attend, double scale, int64_t nsplit, const Tensor& src, at::IntArrayRef attn, const OptTensor& qw, const OptTensor& kw,
                                           double eps, const Tensor& cos, const Tensor& sin, const Tensor& k_cache, const Tensor& v_cache,
                                           at::IntArrayRef mem, const Tensor& ib, const Tensor& fb, double cap, double qscale,
                                           const Tensor& S, const Tensor& n, const Tensor& m, const Tensor& pos, const OptTensor& live) {
@@ -536,8 +536,34 @@ std::tuple<Tensor, Tensor> parallel_step_(const Tensor& src, at::IntArrayRef att
   evgpt::StepMemory sm{rows, (int)mem[0], (int)mem[1], (int)mem[2], (int)mem[3], (int)mem[4], ib.data_ptr<float>(), fb.data_ptr<float>(),
                        (float)cap, (float)qscale, (int)H, (int)Nq, (int)V, S.data_ptr<float>(), n.data_ptr<float>(),
                        m.data_ptr<float>(), (int)S.size(0), o.data_ptr<float>()};
+  if (!attend) {
+    if (B > 0) evgpt::launch_parallel_step(sh, sm, pos.data_ptr<int>(), iptr(live), f32, (int)B, cur_stream());
+    return {q, o};
+  }
+  nsplit = std::min<int64_t>(std::max<int64_t>(nsplit, 1), 16);
+  if (B > 0 && !f32 && evgpt::attend_step_ok(sh, sm, (int)B, (int)nsplit)) {
+    const int64_t Hq = attn[3], D = attn[5];
+    Tensor po = at::empty({B * Hq * nsplit * D}, S.options()), pm = at::empty({B * Hq * nsplit * 2}, S.options());
+    const evgpt::StepSplits sp{po.data_ptr<float>(), pm.data_ptr<float>(), (int)nsplit, (float)scale};
+    evgpt::launch_attend_step(sh, sm, sp, pos.data_ptr<int>(), iptr(live), (int)B, cur_stream());
+    evgpt::launch_attn_decode_merge(sp.part_o, sp.part_ml, bptr_mut(q), (int)B, (int)Hq, (int)D, (int)nsplit, cur_stream());
+    return {q, o};
+  }
   if (B > 0) evgpt::launch_parallel_step(sh, sm, pos.data_ptr<int>(), iptr(live), f32, (int)B, cur_stream());
-  return {q, o};
+  return {attn_chunk_decode(q, k_cache, v_cache, pos, scale, nsplit), o};
+}
+std::tuple<Tensor, Tensor> parallel_step_(const Tensor& src, at::IntArrayRef attn, const OptTensor& qw, const OptTensor& kw,
+                                          double eps, const Tensor& cos, const Tensor& sin, const Tensor& k_cache, const Tensor& v_cache,
+                                          at::IntArrayRef mem, const Tensor& ib, const Tensor& fb, double cap, double qscale,
+                                          const Tensor& S, const Tensor& n, const Tensor& m, const Tensor& pos, const OptTensor& live) {
+  return step_heads(false, 0.0, 1, src, attn, qw, kw, eps, cos, sin, k_cache, v_cache, mem, ib, fb, cap, qscale, S, n, m, pos, live);
+}
+// the step, and the attention of the new queries over the chunk's cached keys: ([B, Hq, D] outputs, memory [B, H * V])
+std::tuple<Tensor, Tensor> attend_step_(const Tensor& src, at::IntArrayRef attn, const OptTensor& qw, const OptTensor& kw,
+                                        double eps, const Tensor& cos, const Tensor& sin, const Tensor& k_cache, const Tensor& v_cache,
+                                        at::IntArrayRef mem, const Tensor& ib, const Tensor& fb, double cap, double qscale, const Tensor& S,
+                                        const Tensor& n, const Tensor& m, const Tensor& pos, const OptTensor& live, double scale, int64_t nsplit) {
+  return step_heads(true, scale, nsplit, src, attn, qw, kw, eps, cos, sin, k_cache, v_cache, mem, ib, fb, cap, qscale, S, n, m, pos, live);
 }
 // the state-space recurrence with its convolution and silu(z) gate: [B, H * V] fp32
 Tensor ssd_step_(const Tensor& src, at::IntArrayRef dims, const Tensor& conv_w, const Tensor& conv_b, const Tensor& ring,
@@ -1042,6 +1068,7 @@ TORCH_LIBRARY(evlay, m) {
   m.def("attn_chunk_decode(Tensor q, Tensor k_cache, Tensor v_cache, Tensor pos, float scale, int nsplit) -> Tensor", &attn_chunk_decode);
   m.def("scan_prefill_(Tensor q, Tensor k, Tensor v, int H, int per_group, int N, int V, float qscale, Tensor log_decay, Tensor? log_in, Tensor? scale_in, Tensor? skip, Tensor(a!) S, Tensor(b!)? n, Tensor(c!)? m, Tensor chunks, Tensor seqs) -> Tensor", &scan_prefill_);
   m.def("parallel_step_(Tensor src, int[] attn, Tensor? qw, Tensor? kw, float eps, Tensor cos, Tensor sin, Tensor(a!) k_cache, Tensor(b!) v_cache, int[] mem, Tensor ib, Tensor fb, float cap, float qscale, Tensor(c!) S, Tensor(d!) n, Tensor(e!) m, Tensor pos, Tensor? live) -> (Tensor, Tensor)", &parallel_step_);
+  m.def("attend_step_(Tensor src, int[] attn, Tensor? qw, Tensor? kw, float eps, Tensor cos, Tensor sin, Tensor(a!) k_cache, Tensor(b!) v_cache, int[] mem, Tensor ib, Tensor fb, float cap, float qscale, Tensor(c!) S, Tensor(d!) n, Tensor(e!) m, Tensor pos, Tensor? live, float scale, int nsplit) -> (Tensor, Tensor)", &attend_step_);
   m.def("ssd_step_(Tensor src, int[] dims, Tensor conv_w, Tensor conv_b, Tensor(a!) ring, Tensor dt_bias, Tensor a_log, Tensor skip, Tensor(b!) S, Tensor pos, Tensor? live) -> Tensor", &ssd_step_);
   m.def("gemv_norm(Tensor x, Tensor norm, int n, float eps, Tensor w, int act, Tensor? a, Tensor? b, Tensor? wa, Tensor? wb, Tensor(a!)? x_out, bool layer=False, Tensor(b!)? xn_out=None, float? scale=None, float cap=0.0) -> Tensor", &gemv_norm);
   m.def("gemv_add_(Tensor(a!) x, Tensor w, Tensor h) -> ()", &gemv_add_);

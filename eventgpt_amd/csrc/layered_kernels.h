@@ -228,6 +228,15 @@ struct StepMemory {                // matrix memory half
 };
 void launch_parallel_step(const StepHeads& h, const StepMemory& m, const int* pos, const int* live, bool f32, int B,
                           hipStream_t st);
+// the step and the attention of each row's query over the ring of cached keys and the new one, as partial results for
+// launch_attn_decode_merge; whether it takes the call (bf16 storage)
+struct StepSplits {
+  float* part_o; float* part_ml;   // [B][Hq][nsplit][D], [B][Hq][nsplit][2]
+  int nsplit;
+  float scale;
+};
+bool attend_step_ok(const StepHeads& h, const StepMemory& m, int B, int nsplit);
+void launch_attend_step(const StepHeads& h, const StepMemory& m, const StepSplits& sp, const int* pos, const int* live, int B, hipStream_t st);
 struct StepSsd {
   SrcRows src;
   int z_col, x_col, dt_col;        // x, B and C are consecutive

@@ -343,10 +343,6 @@ class AttentionBranch(Mixer):
         s = self.spec
         return [col["lq"], col["lk"], col["lv"], s.heads, s.kv_heads, self.D, s.heads * s.dim, s.kv_heads * s.dim]
 
-    def step(self, rows: RowBatch, q: torch.Tensor) -> torch.Tensor:
-        o = self.raw.attn_chunk_decode(q, self.k_cache, self.v_cache, rows.pos, self.spec.scale, self.nsplit)
-        return o.view(o.shape[0], -1)
-
     def prompt(self, rows: RowBatch, src: torch.Tensor, col: Dict[str, int]) -> torch.Tensor:
         s, raw = self.spec, self.raw
         runs, items, row_kv, keep, copies, kv_rows = rows.chunk_tables(self.size, s.heads, self.D)
@@ -414,10 +410,10 @@ class ParallelMixer(Mixer):
         raw, left, right, col = self.raw, self.left, self.right, self.proj.col
         if rows.decode:
             src = self.proj.step(stream, norm)
-            q, mem = raw.parallel_step_(src, left.dims(col), left.qw, left.kw, self.eps, left.cos, left.sin, left.k_cache,
-                                        left.v_cache, right.dims(col), right.ib, right.fb, right.spec.gate_cap, right.qscale,
-                                        right.S, right.n, right.m, rows.pos, rows.live)
-            o = left.step(rows, q)
+            o, mem = raw.attend_step_(src, left.dims(col), left.qw, left.kw, self.eps, left.cos, left.sin, left.k_cache,
+                                      left.v_cache, right.dims(col), right.ib, right.fb, right.spec.gate_cap, right.qscale,
+                                      right.S, right.n, right.m, rows.pos, rows.live, left.spec.scale, left.nsplit)
+            o = o.view(o.shape[0], -1)
             if self.few(stream, max(left.w_o.shape[1], right.kp)):
                 a, b = raw.gemv_branches(left.w_o, o, right.w_o, mem, src, col["rg"], right.norm, right.spec.heads,
                                          right.spec.vdim, right.V, self.eps).unbind(0)

@@ -1007,3 +1007,42 @@ def test_gated_products_of_few_rows(raw, dev, rows, inner, K, act):
     # one rounding to bf16 (the general product rounds its factors too); sums of K float32 products
     bound = (f * u).abs() * 2.0 ** (-8 if rows <= 32 else -6) + K * 2.0 ** -22 * (f * u).abs().max()
     assert bool(((got.double() - f * u).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("H,G,D,rot,normed,B,nsplit,slabs", [(4, 2, 128, 128, True, 1, 16, 1), (6, 2, 64, 32, True, 4, 5, 1), (2, 2, 128, 0, False, 3, 2, 1),
+                                                            (4, 1, 64, 64, False, 2, 16, 1), (4, 2, 128, 64, True, 5, 4, 1), (4, 2, 128, 64, True, 2, 4, 2),
+                                                            (4, 2, 128, 64, True, 2, 1, 1)])
+def test_attention_inside_the_step_is_the_one_behind_it(raw, dev, H, G, D, rot, normed, B, nsplit, slabs):
+    """One launch for the step and the attention over the splits of the cached keys (up to four rows of one matrix) against the two: from
+    the first position, through rings that wrap, with parked sequences, without norms or rotations; the last three cases are the two
+    launches themselves."""
+    f, cap, Hr, Nn, V = dict(dtype=torch.float32, device=dev), 150, 2, 64, 64
+    g = torch.Generator().manual_seed(D + B)
+    at = (H + 2 * G) * D
+    a_dims = [0, H * D, (H + G) * D, H, G, D, H * D, G * D]
+    m_dims = [at, at + Hr * Nn, at + 2 * Hr * Nn, at + 2 * Hr * Nn + Hr * V, at + 2 * Hr * Nn + Hr * V + Hr, Hr, Nn, V]
+    width = m_dims[4] + Hr + (-(m_dims[4] + Hr)) % 8
+    qw, kw = ((1 + 0.2 * torch.randn(n * D, generator=g)).to(dev) for n in (H, G)) if normed else (None, None)
+    ang = torch.arange(1024)[:, None] * 0.9 ** torch.arange(max(rot // 2, 1))
+    cos, sin = (t[:, :rot // 2].contiguous().to(dev) for t in (ang.cos(), ang.sin()))
+    cache = torch.randn(2, B, G, cap, D, generator=g).to(torch.bfloat16).to(dev)
+    state = [torch.randn(*s, generator=g).to(dev) for s in ((B, Hr, V, Nn), (2, B, Hr, Nn), (2, B, Hr))]
+    ib = rnd(Hr, seed=6).float().to(dev)
+    for start in (0, 1, 63, cap - 1, cap, 3 * cap + 77):
+        pos = torch.tensor([start + 5 * b for b in range(B)], dtype=torch.int32, device=dev)
+        live = torch.tensor([int(b != 1) for b in range(B)], dtype=torch.int32, device=dev)
+        src = torch.randn(slabs, B, width, generator=g).to(dev)
+        src = src if slabs > 1 else src[0]
+        got = []
+        for fused in (False, True):
+            c, (S, n, m) = cache.clone(), (t.clone() for t in state)
+            args = (src, a_dims, qw, kw, 1e-5, cos, sin, c[0], c[1], m_dims, ib, ib, 5.0, 0.4, S, n, m, pos, live)
+            if fused:
+                o, mem = raw.attend_step_(*args, D ** -0.5, nsplit)
+            else:
+                q, mem = raw.parallel_step_(*args)
+                o = raw.attn_chunk_decode(q, c[0], c[1], pos, D ** -0.5, nsplit)
+            got.append((o.view(B, H, D)[live.bool()].double(), mem, c, S, n, m))
+        assert all(torch.equal(x, y) for x, y in zip(got[0][1:], got[1][1:])), start
+        # fp32 partial sums in another order, rounded to bf16 once
+        assert bool(((got[0][0] - got[1][0]).abs() <= 2.0 ** -8 * got[0][0].abs() + 1e-5).all()), start
