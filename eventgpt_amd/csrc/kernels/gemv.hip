@@ -1084,8 +1084,12 @@ __global__ __launch_bounds__(GEMV_WAVES * 64, EVGPT_ROW1_OCC) void gemv_row1_ker
 // streaming.  This kernel therefore
 //   * looks codes up instead of permuting bytes: one code byte (weights j and 4+j of a word)
 //     indexes an LDS table of 256 bf16 pairs, kept once per bank so that the 32 lanes of an
-//     access group never meet in a bank (2 address instructions + 1 lookup + 1 v_dot2c per
-//     two weights, against ~7 instructions by v_perm_b32); the x image in LDS holds the
+//     access group never meet in a bank; entries are 256 bytes apart (the second half of each is not
+//     used), so that one v_perm_b32 that puts the code byte above the lane's bank is the address, and the
+//     table is static, so that nothing is added to it (1 address instruction + 1 lookup + 1 v_dot2c
+//     per two weights; a dynamic table 128 bytes apart took a shift, an and-or and an addition of the
+//     symbol's zero: gate / up 14.1 -> 12.9 us, down 8.9 -> 8.05, o 5.2 -> 5.1; of these 10.9, 6.6 and 4.2
+//     are left with the products left out; 64 copies cost 0.6 us to fill); the x image in LDS holds the
 //     matching pairs (x_j, x_4+j);
 //   * gives each wave whole rows (no cross-wave sums, no barrier after the prologue) two at
 //     a time -- a gate / up pair, a rotate-half pair or two plain rows -- in steps of
@@ -1094,7 +1098,7 @@ __global__ __launch_bounds__(GEMV_WAVES * 64, EVGPT_ROW1_OCC) void gemv_row1_ker
 //     steps before it is used.
 constexpr int W4R_WAVES = 8;                // waves per block (they share the table and the x image)
 constexpr int W4R_NI = 2;                   // 64-lane chunk-iterations per step
-constexpr int W4_TAB_BYTES = 256 * 32 * 4;  // 256 code bytes x 32 bank copies of one bf16 pair
+constexpr int W4_TAB_BYTES = 256 * 256;     // 256 code bytes x 32 bank copies of one bf16 pair, and as much unused
 
 // The x image the table path multiplies against: a chunk (x0..x7) is stored as the pairs
 // (x0,x4) (x1,x5) (x2,x6) (x3,x7), the two weights one code byte carries.
@@ -1103,9 +1107,9 @@ __device__ __forceinline__ u32x4_t w4_x_image(u32x4_t o) {
                  perm_b32(o[3], o[1], 0x05040100u), perm_b32(o[3], o[1], 0x07060302u)};
 }
 
-// bf16 pair of code byte i of w; tab_lane points at this lane's bank copy of entry 0
-__device__ __forceinline__ unsigned int w4_lookup(const unsigned char* tab_lane, unsigned int w, int i) {
-  return *reinterpret_cast<const unsigned int*>(tab_lane + ((w >> (8 * i)) & 0xFFu) * 128u);
+// bf16 pair of code byte i of w; bank: the lane's copy, in bytes
+__device__ __forceinline__ unsigned int w4_lookup(const unsigned char* tab, unsigned int bank, unsigned int w, int i) {
+  return *reinterpret_cast<const unsigned int*>(tab + perm_b32(w, bank, 0x0c0c0400u + (static_cast<unsigned int>(i) << 8)));
 }
 
 // the row pair ("group") g of a projection
@@ -1155,10 +1159,10 @@ __global__ __launch_bounds__(W4R_WAVES * 64, (B == 1 && Q) ? 2 : 1) void gemv_ro
   constexpr int IT_SHIFT = W4 ? 5 : 3;             // weights per 16-byte chunk: 32 / 8
   using Step = RowsStep<B, NI>;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  // LDS carve: [block-sum scratch 64 B][table 32 KB (4-bit)][B x images of K * 2 B]
+  __shared__ __attribute__((aligned(256))) unsigned char tab[W4 ? W4_TAB_BYTES : 16];
+  // LDS carve: [block-sum scratch 64 B][B x images of K * 2 B]
   float* red = reinterpret_cast<float*>(smem);
-  const unsigned char* tab = smem + 64;
-  unsigned char* xs_bytes = smem + 64 + (W4 ? W4_TAB_BYTES : 0);
+  unsigned char* xs_bytes = smem + 64;
   const unsigned int x_bytes = static_cast<unsigned int>(p.K) * 2u;   // one image
   // the wave index as a scalar: everything derived from it (this wave's rows, its step count,
   // the loop below) is then uniform to the compiler, which branches instead of masking lanes
@@ -1267,12 +1271,12 @@ __global__ __launch_bounds__(W4R_WAVES * 64, (B == 1 && Q) ? 2 : 1) void gemv_ro
   if constexpr (E == E_QKV_ROPE) have_now(p.q_out, p.k_cache, p.v_cache, p.n_q_heads, p.n_kv_heads, p.head_dim, p.l_max);
   else have_now(p.y);
 
-  // ---- table: entry t = (value[t & 15], value[t >> 4]), 32 copies 4 bytes apart
+  // ---- table: entry t = (value[t & 15], value[t >> 4]), 32 copies 4 bytes apart in its first 128 bytes
   if (W4 && tid < 256) {
     unsigned int e[4];
     w4_expand8(static_cast<unsigned int>(tid), p.code, e);   // weight 0 = code t & 15, weight 4 = code t >> 4
     const unsigned int v = (e[0] & 0xFFFFu) | (e[2] << 16);
-    u32x4_t* dst = reinterpret_cast<u32x4_t*>(smem + 64 + tid * 128);
+    u32x4_t* dst = reinterpret_cast<u32x4_t*>(tab + tid * 256);
 #pragma unroll
     for (int i = 0; i < 8; ++i) dst[i] = u32x4_t{v, v, v, v};
   }
@@ -1317,7 +1321,7 @@ __global__ __launch_bounds__(W4R_WAVES * 64, (B == 1 && Q) ? 2 : 1) void gemv_ro
   }
   __syncthreads();   // the last barrier: no wave waits for another below
 
-  const unsigned char* tab_lane = tab + (lane & 31) * 4;
+  const unsigned int bank = (lane & 31) * 4;
   float acc[2][B];
 #pragma unroll
   for (int r = 0; r < 2; ++r)
@@ -1342,7 +1346,7 @@ __global__ __launch_bounds__(W4R_WAVES * 64, (B == 1 && Q) ? 2 : 1) void gemv_ro
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int k = 0; k < 4; ++k) e[4 * j + k] = w4_lookup(tab_lane, w[j], k);
+      for (int k = 0; k < 4; ++k) e[4 * j + k] = w4_lookup(tab, bank, w[j], k);
   };
   auto xread = [&](u32x4_t (&xv)[B][4], unsigned int xit) {
 #pragma unroll
@@ -1542,6 +1546,7 @@ __global__ __launch_bounds__(W4R_WAVES * 64, (B == 1 && Q) ? 2 : 1) void gemv_ro
 
 // shapes the rows kernel takes: 1..3 x rows of 4-bit weights or (EVGPT_ROWS_BF16: the x rows it takes)
 // bf16 weights, row pairs, whole scale blocks, the table and the x images inside a CU's LDS
+constexpr int rows_lds(bool w4) { return w4 ? 160 * 1024 - W4_TAB_BYTES : 128 * 1024; }      // for the x images, beside the table
 static bool rows_kernel_ok(const GemvParams& p, int B, int E) {
   static const bool on = [] { const char* e = getenv("EVGPT_W4_ROW1"); return !e || atoi(e) != 0; }();
   static const int max_b = [] { const char* e = getenv("EVGPT_W4_ROWS_MAX"); return e ? atoi(e) : 3; }();
@@ -1566,19 +1571,19 @@ static bool rows_kernel_ok(const GemvParams& p, int B, int E) {
   if (p.bias || p.act != ACT_NONE) return false;   // no load may sit in this kernel's epilogue
   if (p.N % 2 != 0) return false;
   if (E == E_QKV_ROPE && p.head_dim % 2 != 0) return false;
-  if (64 + (p.absmax ? W4_TAB_BYTES : 0) + static_cast<size_t>(B) * p.K * 2 > 128 * 1024) return false;
+  if (64 + static_cast<size_t>(B) * p.K * 2 > static_cast<size_t>(rows_lds(p.absmax != nullptr))) return false;
   return p.K <= 3 * W4R_WAVES * 64 * 8;   // the x chunks a block keeps in registers through the norm
 }
 
 template <int P, int E, int B, int Q>
 static void launch_rows_b(const GemvParams& p, hipStream_t st) {
-  const size_t smem = 64 + (Q ? W4_TAB_BYTES : 0) + static_cast<size_t>(B) * p.K * 2;
+  const size_t smem = 64 + static_cast<size_t>(B) * p.K * 2;
   // one block per CU (two would hold their tables and x images at once; 256 measured ahead of 512);
   // fewer blocks when there are fewer row pairs than waves
   static const int cap = [] { const char* e = getenv("EVGPT_W4_ROW1_BLOCKS"); return e && atoi(e) > 0 ? atoi(e) : 256; }();
   static const bool attr = [] {   // more than the 64 KB a launch may ask for without opting in (several long x rows)
     return hipFuncSetAttribute(reinterpret_cast<const void*>(gemv_rows_kernel<P, E, B, Q>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024) == hipSuccess;
+                               hipFuncAttributeMaxDynamicSharedMemorySize, rows_lds(Q != 0)) == hipSuccess;
   }();
   (void)attr;
   const int groups = p.N >> 1;
