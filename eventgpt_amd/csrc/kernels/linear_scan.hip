@@ -49,29 +49,101 @@ __device__ __forceinline__ double wave_max_f64(double v) {
   return v;
 }
 
-// rows [row0, row0 + len) x 64 columns from col (nc of them exist) of a T matrix, transposed into
-// lds[column][row] with rows past len as zeros
-template <typename T, int SL>
-__device__ __forceinline__ void load_transposed(const T* __restrict__ p, long long ld, long long row0, int len, int col,
-                                                int nc, T* lds) {
-#pragma unroll
-  for (int i = 0; i < SL / 32; ++i) {
-    const int idx = threadIdx.x + i * 256, s = idx % SL, c8 = (idx / SL) * 8;
-    T t[8];
-    if (s < len && c8 < nc) {
-      const T* g = p + (row0 + s) * ld + col + c8;
-      if constexpr (sizeof(T) == 2) *reinterpret_cast<u32x4_t*>(t) = load16(g);
-      else {
-        *reinterpret_cast<f32x4_t*>(t) = load4(g);
-        *reinterpret_cast<f32x4_t*>(t + 4) = load4(g + 4);
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) t[j] = T(0);
-    }
-#pragma unroll
-    for (int j = 0; j < 8; ++j) lds[(c8 + j) * (SL + 8) + s] = t[j];
+// Rows [row0, row0 + len) x 64 columns from col (nc of them exist) of a T matrix, zeros past them, as MFMA operands whose contraction
+// runs down the rows.  bf16: rows as they are, 16 bytes a store, read with the transposing read (chunks swizzled so that the eight rows of a
+// half-wave's read lie on different banks); one element a store into a transposed tile took a third of the kernels' instructions.
+template <typename T, int SL> struct Columns;
+template <int SL> struct Columns<bf16_t, SL> {
+  static constexpr int LOADS = SL * 8 / 256;
+  unsigned char bytes[SL * 128];
+  struct Regs { u32x4_t v[LOADS]; };
+  static __device__ __forceinline__ int at(int row, int chunk) {
+    return row * 128 + ((chunk ^ ((((row >> 1) & 1) | (((row >> 3) & 1) << 1)) << 1)) << 4);
   }
+  static __device__ __forceinline__ Regs request(const bf16_t* __restrict__ p, long long ld, long long row0, int len, int col, int nc) {
+    Regs r;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int idx = threadIdx.x + i * 256, row = idx >> 3, c = (idx & 7) * 8;
+      r.v[i] = row < len && c < nc ? load16(p + (row0 + row) * ld + col + c) : u32x4_t{0, 0, 0, 0};
+    }
+    return r;
+  }
+  __device__ __forceinline__ void put(const Regs& r) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int idx = threadIdx.x + i * 256;
+      *reinterpret_cast<u32x4_t*>(bytes + at(idx >> 3, idx & 7)) = r.v[i];
+    }
+  }
+  // columns c0 + (lane & 15), rows 32 kb + 8 (lane >> 4) .. + 7
+  __device__ __forceinline__ Frag<bf16_t> frag(int c0, int kb) const {
+    typedef __attribute__((ext_vector_type(8))) short s16x8_t;
+    const int lane = threadIdx.x & 63, fr = lane & 15, g = lane >> 4, row = kb * 32 + g * 8 + (fr >> 2), chunk = (c0 >> 3) + ((fr & 3) >> 1);
+    const s16x4_t a = read_tr16((lds_s16x4_t*)(bytes + at(row, chunk) + 8 * (fr & 1)));
+    const s16x4_t b = read_tr16((lds_s16x4_t*)(bytes + at(row + 4, chunk) + 8 * (fr & 1)));
+    const s16x8_t v = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+    return {__builtin_bit_cast(bf16x8_t, v)};
+  }
+  __device__ __forceinline__ f32x4_t four(int row, int c) const {            // c % 4 == 0
+    return load4(reinterpret_cast<const bf16_t*>(bytes + at(row, c >> 3) + (c & 4) * 2));
+  }
+  __device__ __forceinline__ float one(int row, int c) const {
+    return bf16_to_f32(*reinterpret_cast<const bf16_t*>(bytes + at(row, c >> 3) + (c & 7) * 2));
+  }
+};
+template <int SL> struct Columns<float, SL> {
+  static constexpr int LOADS = SL / 32, TS = SL + 8;
+  float t[64 * TS];                       // [column][row]
+  struct Regs { f32x4_t v[LOADS][2]; };
+  static __device__ __forceinline__ Regs request(const float* __restrict__ p, long long ld, long long row0, int len, int col, int nc) {
+    Regs r;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int idx = threadIdx.x + i * 256, s = idx % SL, c8 = (idx / SL) * 8;
+      const bool in = s < len && c8 < nc;
+      const float* g = p + (row0 + s) * ld + col + c8;
+      r.v[i][0] = in ? load4(g) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+      r.v[i][1] = in ? load4(g + 4) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    return r;
+  }
+  __device__ __forceinline__ void put(const Regs& r) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int idx = threadIdx.x + i * 256, s = idx % SL, c8 = (idx / SL) * 8;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) t[(c8 + j) * TS + s] = r.v[i][j >> 2][j & 3];
+    }
+  }
+  __device__ __forceinline__ Frag<float> frag(int c0, int kb) const {
+    const int lane = threadIdx.x & 63;
+    return load_frag(t + (c0 + (lane & 15)) * TS + kb * 32 + (lane >> 4) * 8);
+  }
+  __device__ __forceinline__ f32x4_t four(int row, int c) const {
+    return f32x4_t{t[c * TS + row], t[(c + 1) * TS + row], t[(c + 2) * TS + row], t[(c + 3) * TS + row]};
+  }
+  __device__ __forceinline__ float one(int row, int c) const { return t[c * TS + row]; }
+};
+__device__ __forceinline__ void unpack(const Frag<bf16_t>& f, float (&x)[8]) {
+  const u32x4_t w = __builtin_bit_cast(u32x4_t, f.v);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) { x[2 * i] = bf16lo(w[i]); x[2 * i + 1] = bf16hi(w[i]); }
+}
+__device__ __forceinline__ void unpack(const Frag<float>& f, float (&x)[8]) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) x[i] = f.v[i];
+}
+
+// A double in units of log2 as two floats: sums of two of these, high parts first, keep the float rounding of the sum's exponent.
+struct Log2Pair { float hi, lo; };
+__device__ __forceinline__ Log2Pair log2_pair(double natural) {
+  const double v = natural * 1.4426950408889634074;
+  const float hi = static_cast<float>(v);
+  return {hi, fabsf(hi) < INFINITY ? static_cast<float>(v - static_cast<double>(hi)) : 0.f};
+}
+__device__ __forceinline__ float exp_sum(const Log2Pair& a, const Log2Pair& b) {
+  return __builtin_amdgcn_exp2f((a.hi + b.hi) + (a.lo + b.lo));
 }
 
 // One wave: decay sums F of a chunk's tokens (lane l: tokens l NH .. l NH + NH - 1), and with STAB the running maxima
@@ -107,19 +179,35 @@ __device__ __forceinline__ void chunk_gates(const ScanArgs& a, int row0, int len
   }
 }
 
+// A block's 64 value rows of a head and chunk.  The blocks of one head and chunk read the same queries and keys: one XCD takes them.  Heads of
+// one block go by the grid: neighbours' value rows then meet in memory while the eight XCDs read them (head 64 wide: 103 us, by XCD 113).
+struct ScanTile {
+  int v0, h, chunk;
+  __device__ __forceinline__ explicit ScanTile(int heads) : v0(0), h(blockIdx.y), chunk(blockIdx.z) {
+    const int nx = gridDim.x;
+    if (nx == 1) return;
+    const int id = xcd_remap(blockIdx.x + nx * (blockIdx.y + heads * blockIdx.z), nx * heads * gridDim.z);
+    v0 = id % nx * 64;
+    h = id / nx % heads;
+    chunk = id / nx / heads;
+  }
+};
+
 // Block: 64 value rows of one head and chunk, all of N in runs of 64.
 template <typename T, bool STAB, int SL>
 __global__ __launch_bounds__(256) void scan_chunk_state_kernel(ScanArgs a, ScanChunks c) {
-  constexpr int TS = SL + 8, NH = SL / 64;
-  __shared__ __attribute__((aligned(16))) T kt[64 * TS];
-  __shared__ __attribute__((aligned(16))) T vt[64 * TS];
+  constexpr int NH = SL / 64;
+  using Tile = Columns<T, SL>;
+  __shared__ __attribute__((aligned(16))) Tile kt, vt;
   __shared__ __attribute__((aligned(16))) float wgt[SL];
-  const int v0 = blockIdx.x * 64, h = blockIdx.y, ci = blockIdx.z;
+  __shared__ float dn_s[4][64];
+  const ScanTile tile(a.H);
+  const int v0 = tile.v0, h = tile.h, ci = tile.chunk;
   const int row0 = c.chunks[ci * 4], len = min(c.chunks[ci * 4 + 1], SL);
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, fr = lane & 15, g = lane >> 4;
   const int nv = min(64, a.V - v0), k_col = (h / a.per_group) * a.N;
-  load_transposed<T, SL>(static_cast<const T*>(a.v), a.ldv, row0, len, h * a.V + v0, nv, vt);
-  load_transposed<T, SL>(static_cast<const T*>(a.k), a.ldk, row0, len, k_col, min(64, a.N), kt);
+  const auto vr = Tile::request(static_cast<const T*>(a.v), a.ldv, row0, len, h * a.V + v0, nv);
+  auto kr = Tile::request(static_cast<const T*>(a.k), a.ldk, row0, len, k_col, min(64, a.N));
   if (wid == 0) {
     double F[NH], m[NH];
     float li[NH];
@@ -132,18 +220,20 @@ __global__ __launch_bounds__(256) void scan_chunk_state_kernel(ScanArgs a, ScanC
       const float e = static_cast<float>(FL - F[i] + (STAB ? static_cast<double>(li[i]) - top : 0.0));
       wgt[lane * NH + i] = lane * NH + i < len ? expf(e) * (STAB ? 1.f : li[i]) : 0.f;
     }
-    if (blockIdx.x == 0 && lane == 0) {
+    if (v0 == 0 && lane == 0) {
       const long long o = static_cast<long long>(ci) * a.H + h;
       c.am[o] = top;
       c.fl[o] = FL;
     }
   }
+  vt.put(vr);
+  kt.put(kr);
   __syncthreads();
   WideFrag<T> vf[SL / 32];          // a wave owns 16 value rows, weighted
 #pragma unroll
   for (int ks = 0; ks < SL / 32; ++ks) {
     float x[8], w[8];
-    load8(vt + (wid * 16 + fr) * TS + ks * 32 + g * 8, x);
+    unpack(vt.frag(wid * 16, ks), x);
     load8(wgt + ks * 32 + g * 8, w);
 #pragma unroll
     for (int j = 0; j < 8; ++j) x[j] *= w[j];
@@ -152,18 +242,14 @@ __global__ __launch_bounds__(256) void scan_chunk_state_kernel(ScanArgs a, ScanC
   float* dS = c.dS + ((static_cast<long long>(ci) * a.H + h) * a.V + v0) * a.N;
   for (int n0 = 0; n0 < a.N; n0 += 64) {
     const int nn = min(64, a.N - n0);
-    if (n0 > 0) {
-      __syncthreads();
-      load_transposed<T, SL>(static_cast<const T*>(a.k), a.ldk, row0, len, k_col + n0, nn, kt);
-      __syncthreads();
-    }
+    if (n0 + 64 < a.N) kr = Tile::request(static_cast<const T*>(a.k), a.ldk, row0, len, k_col + n0 + 64, min(64, a.N - n0 - 64));
     f32x4_t acc[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < SL / 32; ++ks)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] = mma(load_frag(kt + (i * 16 + fr) * TS + ks * 32 + g * 8), vf[ks], acc[i]);
+      for (int i = 0; i < 4; ++i) acc[i] = mma(kt.frag(i * 16, ks), vf[ks], acc[i]);
     // D[n][v]: a lane holds four consecutive n of value row fr
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -171,11 +257,20 @@ __global__ __launch_bounds__(256) void scan_chunk_state_kernel(ScanArgs a, ScanC
       if (v < nv && n < nn) *reinterpret_cast<f32x4_t*>(dS + static_cast<long long>(v) * a.N + n0 + n) = acc[i];
     }
     if constexpr (STAB) {
-      if (v0 == 0 && tid < nn) {
+      if (v0 == 0) {                  // (block-uniform) a wave per quarter of the tokens
         float s = 0.f;
-        for (int t = 0; t < SL; ++t) s += wgt[t] * to_f32(kt[tid * TS + t]);
-        c.dn[(static_cast<long long>(ci) * a.H + h) * a.N + n0 + tid] = s;
+#pragma unroll 8
+        for (int t = 0; t < SL / 4; ++t) s += wgt[wid * (SL / 4) + t] * kt.one(wid * (SL / 4) + t, lane);
+        dn_s[wid][lane] = s;
+        __syncthreads();
+        if (tid < nn)
+          c.dn[(static_cast<long long>(ci) * a.H + h) * a.N + n0 + tid] = dn_s[0][tid] + dn_s[1][tid] + dn_s[2][tid] + dn_s[3][tid];
       }
+    }
+    if (n0 + 64 < a.N) {
+      __syncthreads();
+      kt.put(kr);
+      __syncthreads();
     }
   }
 }
@@ -232,44 +327,58 @@ __global__ __launch_bounds__(256) void scan_chunk_pass_kernel(ScanArgs a, ScanCh
   }
 }
 
+// Weighted scores of 64 tokens as operands: [token][key].  bf16: both parts of `WideFrag`, made once where the four waves would each make them.
+template <typename T, int SL> struct Weights;
+template <int SL> struct Weights<bf16_t, SL> {
+  static constexpr int BYTES = 2 * 64 * SL * 2, CH = SL / 8;
+  static __device__ __forceinline__ int at(int t, int s) { return t * (SL * 2) + (((s >> 3) ^ (t & (CH - 1))) << 4) + (s & 7) * 2; }
+  static __device__ __forceinline__ void put(unsigned char* p, int t, int s, const f32x4_t& w) {          // s % 4 == 0
+    const u32x2_t hi = {pack_bf16x2(w[0], w[1]), pack_bf16x2(w[2], w[3])};
+    const u32x2_t lo = {pack_bf16x2(w[0] - bf16lo(hi[0]), w[1] - bf16hi(hi[0])), pack_bf16x2(w[2] - bf16lo(hi[1]), w[3] - bf16hi(hi[1]))};
+    *reinterpret_cast<u32x2_t*>(p + at(t, s)) = hi;
+    *reinterpret_cast<u32x2_t*>(p + 64 * SL * 2 + at(t, s)) = lo;
+  }
+  static __device__ __forceinline__ WideFrag<bf16_t> frag(const unsigned char* p, int t, int s) {         // s % 8 == 0
+    return {__builtin_bit_cast(bf16x8_t, load16(p + at(t, s))), __builtin_bit_cast(bf16x8_t, load16(p + 64 * SL * 2 + at(t, s)))};
+  }
+};
+template <int SL> struct Weights<float, SL> {
+  static constexpr int PS = SL + 4, BYTES = 64 * PS * 4;
+  static __device__ __forceinline__ void put(unsigned char* p, int t, int s, const f32x4_t& w) {
+    *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(p) + t * PS + s) = w;
+  }
+  static __device__ __forceinline__ WideFrag<float> frag(const unsigned char* p, int t, int s) {
+    float x[8];
+    load8(reinterpret_cast<const float*>(p) + t * PS + s, x);
+    return wide_frag<float>(x);
+  }
+};
+
 // Block: 64 value columns of one head and chunk.  Scores are computed transposed, a wave per sixteen keys of every
 // 64, and meet in LDS (in the query tile's place); then a wave owns sixteen value rows for all tokens, so that the
-// chunk's start state -- most of the bytes this kernel reads -- is read once.
+// chunk's start state -- most of the bytes this kernel reads -- is read once.  Everything a step of 32 state columns reads
+// is requested a step ahead, the first of them with the values; what is left is latency, so three blocks to a CU (168 registers a lane,
+// under 54 KB of LDS).  A weight's exponent is the sum of two numbers kept as pairs of floats in units of log2 (`Log2Pair`): three
+// additions and one instruction where the double difference and expf took most of the vector instructions.  4096 tokens, 134 MB of
+// states: 8 heads of 512 x 256 with a maximum 105 us, 128 heads of 64 x 128 106, were both 174 (state 52 and 58, were 74).
 template <typename T, bool STAB, int SL>
-__global__ __launch_bounds__(256) void scan_chunk_out_kernel(ScanArgs a, ScanChunks c) {
-  constexpr int TS = SL + 8, NH = SL / 64, PS = SL + 4, QS = 64 + 8;
-  constexpr int Q_BYTES = SL * QS * sizeof(T), P_BYTES = 64 * PS * 4;
-  __shared__ __attribute__((aligned(16))) T vt[64 * TS];              // [value][key]
-  __shared__ __attribute__((aligned(16))) unsigned char qp_lds[Q_BYTES > P_BYTES ? Q_BYTES : P_BYTES];
+__global__ __launch_bounds__(256, 3) void scan_chunk_out_kernel(ScanArgs a, ScanChunks c) {
+  constexpr int NH = SL / 64, QS = 64 + 8, QV = sizeof(T) == 4 ? 2 : 1;
+  using Tile = Columns<T, SL>;
+  using Wgt = Weights<T, SL>;
+  constexpr int Q_BYTES = SL * QS * sizeof(T);
+  __shared__ __attribute__((aligned(16))) Tile vt;                                // values of the chunk's tokens
+  __shared__ __attribute__((aligned(16))) unsigned char qp_lds[Q_BYTES > Wgt::BYTES ? Q_BYTES : Wgt::BYTES];
   T* qs = reinterpret_cast<T*>(qp_lds);                               // [token][64 of N]
-  float* ps = reinterpret_cast<float*>(qp_lds);                       // [token of a half][key] weighted scores
-  __shared__ double F_s[SL];
-  __shared__ float in_s[SL], m_s[SL], inv_s[64];
-  const int v0 = blockIdx.x * 64, h = blockIdx.y, ci = blockIdx.z;
+  __shared__ Log2Pair tok_s[SL], key_s[SL];                           // F - m and log_in - F (F and -F)
+  __shared__ float in_s[SL], m_s[SL], inv_s[64], den_s[4][64];
+  __shared__ __attribute__((aligned(16))) float nrm_s[64];            // the start state's normaliser, of the columns at hand
+  const ScanTile tile(a.H);
+  const int v0 = tile.v0, h = tile.h, ci = tile.chunk;
   const int row0 = c.chunks[ci * 4], len = min(c.chunks[ci * 4 + 1], SL);
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, fr = lane & 15, g = lane >> 4;
   const int nv = min(64, a.V - v0), hk = h / a.per_group;
   const long long ho = static_cast<long long>(ci) * a.H + h;
-  const float m0 = STAB ? c.m0[ho] : 0.f;
-  load_transposed<T, SL>(static_cast<const T*>(a.v), a.ldv, row0, len, h * a.V + v0, nv, vt);
-  if (wid == 0) {
-    double F[NH], top[NH];
-    float li[NH];
-    chunk_gates<NH, STAB>(a, row0, len, h, F, li, top);
-#pragma unroll
-    for (int i = 0; i < NH; ++i) {
-      const int t = lane * NH + i;
-      F_s[t] = F[i];
-      in_s[t] = li[i];
-      m_s[t] = STAB ? static_cast<float>(F[i] + fmax(static_cast<double>(m0), top[i])) : 0.f;
-    }
-    if constexpr (STAB) {
-      const int last = c.chunks[ci * 4 + 3];
-      if (blockIdx.x == 0 && lane == 0 && (last & 1))
-        a.m[(static_cast<long long>(last >> 1 & 1) * a.slots + c.chunks[ci * 4 + 2]) * a.H + h] =
-            static_cast<float>(fmax(c.fl[ho] + m0, c.am[ho]));
-    }
-  }
   const T* qp = static_cast<const T*>(a.q) + static_cast<long long>(hk) * a.N;
   const T* kp[NH];
 #pragma unroll
@@ -278,6 +387,56 @@ __global__ __launch_bounds__(256) void scan_chunk_out_kernel(ScanArgs a, ScanChu
   const float* S0 = c.dS + (ho * a.V + v0 + wid * 16 + fr) * a.N;
   const float* nrm = STAB ? c.dn + ho * a.N : nullptr;
   const bool rows_v = wid * 16 < nv;              // this wave has value rows
+  const auto vr = Tile::request(static_cast<const T*>(a.v), a.ldv, row0, len, h * a.V + v0, nv);
+  u32x4_t qr[2 * NH][QV];
+  float nr = 0.f;
+  auto request_q = [&](int n0) {
+    if (STAB && tid < 64 && n0 + tid < a.N) nr = nrm[n0 + tid];
+#pragma unroll
+    for (int i = 0; i < 2 * NH; ++i) {
+      const int idx = tid + i * 256, t = idx >> 3, c8 = (idx & 7) * 8;
+      if (n0 + c8 < a.N) {
+        const T* p = qp + (row0 + min(t, len - 1)) * a.ldq + n0 + c8;
+#pragma unroll
+        for (int v = 0; v < QV; ++v) qr[i][v] = load16(p + v * 4);
+      }
+    }
+  };
+  Frag<T> kn[NH];
+  float xn[8];
+  auto request_step = [&](int n) {
+#pragma unroll
+    for (int k = 0; k < NH; ++k) kn[k] = load_frag(kp[k] + n + g * 8);
+    if (rows_v) load8(S0 + n + g * 8, xn);
+    else
+#pragma unroll
+      for (int j = 0; j < 8; ++j) xn[j] = 0.f;
+  };
+  request_q(0);
+  request_step(0);
+  const float m0 = STAB ? c.m0[ho] : 0.f;
+  if (wid == 0) {
+    double F[NH], top[NH];
+    float li[NH];
+    chunk_gates<NH, STAB>(a, row0, len, h, F, li, top);
+#pragma unroll
+    for (int i = 0; i < NH; ++i) {
+      const int t = lane * NH + i;
+      const float mt = STAB ? static_cast<float>(F[i] + fmax(static_cast<double>(m0), top[i])) : 0.f;
+      in_s[t] = li[i];
+      m_s[t] = mt;
+      tok_s[t] = log2_pair(F[i] - static_cast<double>(mt));
+      key_s[t] = log2_pair((STAB ? static_cast<double>(li[i]) : 0.0) - F[i]);
+    }
+    if constexpr (STAB) {
+      const int last = c.chunks[ci * 4 + 3];
+      if (v0 == 0 && lane == 0 && (last & 1))
+        a.m[(static_cast<long long>(last >> 1 & 1) * a.slots + c.chunks[ci * 4 + 2]) * a.H + h] =
+            static_cast<float>(fmax(c.fl[ho] + m0, c.am[ho]));
+    }
+  }
+  const Log2Pair start = log2_pair(static_cast<double>(m0));
+  vt.put(vr);
   f32x4_t st[NH][NH][4], inter[NH][4];            // [key half][token half][token tile]
   float nq[NH];
 #pragma unroll
@@ -296,24 +455,19 @@ __global__ __launch_bounds__(256) void scan_chunk_out_kernel(ScanArgs a, ScanChu
 #pragma unroll
     for (int i = 0; i < 2 * NH; ++i) {
       const int idx = tid + i * 256, t = idx >> 3, c8 = (idx & 7) * 8;
-      if (c8 < nn) {
-        const T* p = qp + (row0 + min(t, len - 1)) * a.ldq + n0 + c8;
-        T* d = qs + t * QS + c8;
-        *reinterpret_cast<u32x4_t*>(d) = load16(p);
-        if constexpr (sizeof(T) == 4) *reinterpret_cast<u32x4_t*>(d + 4) = load16(p + 4);
-      }
+      if (c8 < nn)
+#pragma unroll
+        for (int v = 0; v < QV; ++v) *reinterpret_cast<u32x4_t*>(qs + t * QS + c8 + v * 4) = qr[i][v];
     }
+    if (STAB && tid < 64) nrm_s[tid] = nr;
+    if (n0 + 64 < a.N) request_q(n0 + 64);
     __syncthreads();
     for (int n = 0; n < nn; n += 32) {
       Frag<T> kf[NH];
 #pragma unroll
-      for (int k = 0; k < NH; ++k) kf[k] = load_frag(kp[k] + n0 + n + g * 8);
-      float x[8];
-      if (rows_v) load8(S0 + n0 + n + g * 8, x);
-      else
-#pragma unroll
-        for (int j = 0; j < 8; ++j) x[j] = 0.f;
-      const WideFrag<T> sf = wide_frag<T>(x);
+      for (int k = 0; k < NH; ++k) kf[k] = kn[k];
+      const WideFrag<T> sf = wide_frag<T>(xn);
+      if (n0 + n + 32 < a.N) request_step(n0 + n + 32);
 #pragma unroll
       for (int th = 0; th < NH; ++th)
 #pragma unroll
@@ -326,55 +480,65 @@ __global__ __launch_bounds__(256) void scan_chunk_out_kernel(ScanArgs a, ScanChu
         }
     }
     if constexpr (STAB) {
-      const int part = (tid & 3) * 16;
 #pragma unroll
-      for (int th = 0; th < NH; ++th)
-        for (int n = part; n < min(part + 16, nn); ++n) nq[th] += nrm[n0 + n] * to_f32(qs[(th * 64 + (tid >> 2)) * QS + n]);
+      for (int half = 0; half < 2; ++half) {
+        const int n = (tid & 3) * 16 + half * 8;
+        if (n >= nn) break;
+        float w[8], x[8];
+        load8(nrm_s + n, w);
+#pragma unroll
+        for (int th = 0; th < NH; ++th) {
+          load8(qs + (th * 64 + (tid >> 2)) * QS + n, x);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) nq[th] += w[j] * x[j];
+        }
+      }
     }
   }
   Frag<T> vf[SL / 32];
 #pragma unroll
-  for (int kb = 0; kb < SL / 32; ++kb) vf[kb] = load_frag(vt + (wid * 16 + fr) * TS + kb * 32 + g * 8);
+  for (int kb = 0; kb < SL / 32; ++kb) vf[kb] = vt.frag(wid * 16, kb);
   const float skip = a.skip ? a.skip[h] : 0.f;
 #pragma unroll
   for (int th = 0; th < NH; ++th) {
     if (th * 64 >= len) break;                    // block-uniform
     __syncthreads();                              // the query tile, or the scores of the half before, are no longer read
+    float den[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int k = 0; k <= th; ++k)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         // weighted scores of keys 64 k + 16 wid + 4 g + r and token 64 th + 16 j + fr
-        const int t = th * 64 + j * 16 + fr;
-        const double Ft = F_s[t];
+        const int t = th * 64 + j * 16 + fr, s0 = k * 64 + wid * 16 + g * 4;
+        const Log2Pair Ft = tok_s[t];
         f32x4_t w = st[k][th][j];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int s = k * 64 + wid * 16 + g * 4 + r;
-          float e = 0.f;
-          if (s <= t && t < len) {
-            if constexpr (STAB) e = expf(static_cast<float>(Ft - F_s[s] + static_cast<double>(in_s[s] - m_s[t])));
-            else e = expf(static_cast<float>(Ft - F_s[s])) * in_s[s];
-          }
-          w[r] *= e * a.qscale;
+          const int s = s0 + r;
+          float e = exp_sum(Ft, key_s[s]);
+          if constexpr (!STAB) e *= in_s[s];
+          w[r] = s <= t && t < len ? w[r] * (e * a.qscale) : 0.f;
+          den[j] += w[r];
         }
-        *reinterpret_cast<f32x4_t*>(ps + (j * 16 + fr) * PS + k * 64 + wid * 16 + g * 4) = w;
+        Wgt::put(qp_lds, j * 16 + fr, s0, w);
       }
+    if constexpr (STAB) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float d = den[j];
+        d += __shfl_xor(d, 16, 64);
+        d += __shfl_xor(d, 32, 64);
+        if (g == 0) den_s[wid][j * 16 + fr] = d;
+      }
+    }
     __syncthreads();
     if constexpr (STAB) {
       const int tl = tid >> 2, t = th * 64 + tl;
-      float den = 0.f;
-#pragma unroll
-      for (int k = 0; k <= th; ++k)
-#pragma unroll
-        for (int i = 0; i < 16; i += 4) {
-          const f32x4_t x = *reinterpret_cast<const f32x4_t*>(ps + tl * PS + k * 64 + (tid & 3) * 16 + i);
-          den += x[0] + x[1] + x[2] + x[3];
-        }
-      den += nq[th] * expf(static_cast<float>(F_s[t] + static_cast<double>(m0 - m_s[t]))) * a.qscale;
-      den += __shfl_xor(den, 1, 64);
-      den += __shfl_xor(den, 2, 64);
-      if ((tid & 3) == 0) inv_s[tl] = 1.f / (fmaxf(fabsf(den), expf(-m_s[t])) + 1e-6f);
+      float d = nq[th];
+      d += __shfl_xor(d, 1, 64);
+      d += __shfl_xor(d, 2, 64);
+      d = d * exp_sum(tok_s[t], start) * a.qscale + (den_s[0][tl] + den_s[1][tl] + den_s[2][tl] + den_s[3][tl]);
+      if ((tid & 3) == 0) inv_s[tl] = 1.f / (fmaxf(fabsf(d), expf(-m_s[t])) + 1e-6f);
       __syncthreads();
     }
     if (!rows_v) continue;
@@ -384,19 +548,12 @@ __global__ __launch_bounds__(256) void scan_chunk_out_kernel(ScanArgs a, ScanChu
       f32x4_t y = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kb = 0; kb < SL / 32; ++kb)
-        if (kb < 2 * th || (kb < 2 * th + 2 && (kb - 2 * th) * 2 <= j)) {
-          float x[8];
-          load8(ps + tl * PS + kb * 32 + g * 8, x);
-          y = mma(vf[kb], wide_frag<T>(x), y);
-        }
+        if (kb < 2 * th || (kb < 2 * th + 2 && (kb - 2 * th) * 2 <= j)) y = mma(vf[kb], Wgt::frag(qp_lds, tl, kb * 32 + g * 8), y);
       if (t >= len) continue;
-      y += inter[th][j] * (expf(static_cast<float>(F_s[t] + static_cast<double>(m0 - m_s[t]))) * a.qscale);
+      y += inter[th][j] * (exp_sum(tok_s[t], start) * a.qscale);
       if constexpr (STAB) y *= inv_s[tl];
       const int v = wid * 16 + g * 4;
-      if (a.skip) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) y[r] += skip * to_f32(vt[(v + r) * TS + t]);
-      }
+      if (a.skip) y += skip * vt.four(t, v);
       store4(static_cast<T*>(a.out) + (static_cast<long long>(row0 + t) * a.H + h) * a.V + v0 + v, y[0], y[1], y[2], y[3]);
     }
   }

@@ -1046,3 +1046,36 @@ def test_attention_inside_the_step_is_the_one_behind_it(raw, dev, H, G, D, rot, 
         assert all(torch.equal(x, y) for x, y in zip(got[0][1:], got[1][1:])), start
         # fp32 partial sums in another order, rounded to bf16 once
         assert bool(((got[0][0] - got[1][0]).abs() <= 2.0 ** -8 * got[0][0].abs() + 1e-5).all()), start
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("kind,H,V", [("ssd", 3, 64), ("mlstm", 3, 64), ("mlstm", 2, 320)])
+def test_recurrence_of_strong_decays(raw, dev, dtype, kind, H, V):
+    """Sums of decays in the hundreds: a weight is the exponential of a small
+    difference of long sums, for one and for several blocks of value rows."""
+    T, Nn = 200, 64
+    q, qr = typed(rnd(T, H, Nn) + 0.8, dtype, dev)
+    k, kr = typed(rnd(T, H, Nn, seed=1) + 0.8, dtype, dev)
+    v, vr = typed(rnd(T, H, V, seed=2), dtype, dev)
+    ld = -(20 * rnd(T, H, seed=3).abs()).float()
+    f = dict(device=dev, dtype=torch.float32)
+    li = (2 * rnd(T, H, seed=4)).float() if kind == "mlstm" else None
+    dt = None if li is not None else torch.nn.functional.softplus(rnd(T, H, seed=4)).float()
+    if li is not None:
+        want = oracle.mlstm_scan(qr, kr, vr, li.double(), ld.double())
+        st = (torch.zeros(1, H, V, Nn, **f), torch.zeros(2, 1, H, Nn, **f), torch.zeros(2, 1, H, **f))
+    else:
+        S, want = torch.zeros(H, V, Nn, dtype=torch.float64), []
+        for t in range(T):
+            S = S * ld[t].double().exp()[:, None, None] + dt[t].double()[:, None, None] * vr[t][:, :, None] * kr[t][:, None, :]
+            want.append((S * qr[t][:, None, :]).sum(-1))
+        want = torch.stack(want)
+        st = (torch.zeros(1, H, V, Nn, **f), None, None)
+    rb = RowBatch(dev, False, seqs=pack([T]), scan_chunk=raw.scan_chunk(dtype == torch.float32))
+    o = raw.scan_prefill_(q.view(T, -1), k.view(T, -1), v.view(T, -1), H, 1, Nn, V, 1.0, ld.to(dev), None if li is None else li.to(dev),
+                          None if dt is None else dt.to(dev), None, *st, rb.chunks, rb.scan_seqs)
+    # sums of up to 264 products of weights good to 2^-17 (two bf16 parts; an exponent of up to 100 at 2^-24 costs 2^-17 too): 2e-5 of the
+    # largest output at most; bf16 has 8 significant bits, so the result itself is rounded by up to 2^-8 of each element
+    want = want.reshape(T, -1)
+    bound = 2e-5 * want.abs().max() + (0.0 if dtype == torch.float32 else 2.0 ** -8 * 1.01) * want.abs()
+    assert bool(((o.cpu().double() - want).abs() <= bound).all())
