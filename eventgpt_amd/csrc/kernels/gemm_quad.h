@@ -5,7 +5,7 @@
 namespace evgpt {
 
 // What it takes: at least two K-tiles in every split, byte offsets of a tile's rows within 31 bits, and an output it stores in whole
-// 16-byte chunks (bf16, plain or gated) or fp32 slabs.
+// 16-byte chunks (bf16, plain or gated; fp32 sums as they are) or fp32 slabs.
 bool gemm_quad_serves(const GemmParams& p);
 // Whether it is ahead of the 8-wave kernel there; tiles: of the output, times the splits
 bool gemm_quad_ahead(const GemmParams& p, int tiles);

@@ -219,15 +219,17 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(GemmParams p) {
     const int M = cur.rows;
     bf16_t* C = p.C + (GRP ? static_cast<size_t>(cur.first) * p.ldc : 0);
     unsigned char* rows = smem + 2 * STAGE + wid * SCRATCH;
-    if (!GRP && (p.splitk > 1 || p.raw_partial)) {
-      float* slab = p.partial + static_cast<size_t>(cur.ksplit) * p.M * p.N;
+    if (!GRP && (p.splitk > 1 || p.raw_partial || p.Cf)) {
+      const bool whole = p.splitk == 1 && !p.raw_partial;              // the fp32 output itself
+      float* slab = whole ? p.Cf : p.partial + static_cast<size_t>(cur.ksplit) * p.M * p.N;
+      const size_t ld = whole ? p.ldc : p.N;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const int m = cur.m0 + wr * 128 + i * 16 + frow;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           const int n = cur.n0 + wc * 128 + j * 16 + fq * 4;
-          if (m < M && n < p.N) *reinterpret_cast<f32x4_t*>(slab + static_cast<size_t>(m) * p.N + n) = take(acc[i][j]);
+          if (m < M && n < p.N) *reinterpret_cast<f32x4_t*>(slab + m * ld + n) = take(acc[i][j]);
         }
       }
     } else if (ACT == ACT_NONE && p.glu_half) {
@@ -325,10 +327,13 @@ bool gemm_quad_serves(const GemmParams& p) {
   const long long lim = 1ll << 31;
   const int tail = p.K % p.k_per_split;
   if (p.k_per_split < 2 * BK || (tail && tail < 2 * BK)) return false;
-  if (p.k_cols || p.Cf || p.amax_val || p.rope_cos) return false;
+  if (p.k_cols || p.amax_val || p.rope_cos) return false;
   if (2ll * 256 * p.lda >= lim || 2ll * (p.glu_half ? 2ll * p.glu_half : 256) * p.ldw >= lim) return false;
   if (p.grp_start && (2ll * p.M * p.lda >= lim || p.res || p.bias || p.act != ACT_NONE)) return false;
   if (p.splitk > 1 || p.raw_partial) return !p.glu_half && p.partial && p.N % 4 == 0;
+  if (p.Cf)
+    return !p.C && !p.grp_start && !p.glu_half && !p.bias && !p.res && p.act == ACT_NONE && p.N % 4 == 0 && p.ldc % 4 == 0 &&
+           (reinterpret_cast<uintptr_t>(p.Cf) & 15) == 0;
   if (p.N % 8 || p.ldc % 8 || !p.C || (reinterpret_cast<uintptr_t>(p.C) & 15) || (reinterpret_cast<uintptr_t>(p.res) & 15)) return false;
   if (p.glu_half) return !p.bias && !p.res && p.act == ACT_NONE;
   return (reinterpret_cast<uintptr_t>(p.bias) & 7) == 0 && (p.act == ACT_NONE || p.act == ACT_GELU || p.act == ACT_QUICK_GELU);
@@ -340,18 +345,20 @@ bool gemm_quad_serves(const GemmParams& p) {
 //  * plain 1.08 / 1.04 / 1.00 / 0.98 / 0.97 / 0.97 and 1.00 / 0.97 / 0.96 / 0.96 / 0.96 / 0.96
 //  * slabs 1.06 / 1.04 / 1.03 / 1.02 / 1.00 / 0.97 and 1.00 / 0.96 / 0.96 / 0.96 / 0.94 / 0.94
 //  * gated 1.08 / 1.05 / 1.04 / 1.03 / 1.00 / 0.98 and 1.06 / 1.02 / 1.01 / 0.99 / 0.98 / 0.97
+//  * an fp32 output, us before (the 8-wave kernel with its general epilogue) / now: 4096 x 4096 x 4096 104 / 96, x 2048 63 / 56, 6688 x 4096 x
+//    1024 71 / 58, 4096 x 11008 x 320 67 / 52; the line is the slabs'
 //  * a residual 1.00 to 0.96 and 0.96 to 0.94, a bias 0.80 to 0.86, gelu 0.88 to 0.94, quick-gelu 0.70 to 0.80
 bool gemm_quad_ahead(const GemmParams& p, int tiles) {
   const int k = p.k_per_split;
   const bool many = tiles > 256;
   if (p.glu_half) return k > (many ? 768 : 1024);
-  if (p.splitk > 1 || p.raw_partial) return k > (many ? 192 : 1024);
+  if (p.splitk > 1 || p.raw_partial || p.Cf) return k > (many ? 192 : 1024);
   return p.bias || p.res || p.act != ACT_NONE || k > (many ? 192 : 576);
 }
 
 void launch_gemm_quad(const GemmParams& p, int grid, hipStream_t st) {
   if (p.grp_start) launch<true>(p, grid, st);
-  else if (p.splitk > 1 || p.raw_partial || p.act == ACT_NONE) launch<false>(p, grid, st);
+  else if (p.splitk > 1 || p.raw_partial || p.Cf || p.act == ACT_NONE) launch<false>(p, grid, st);
   else if (p.act == ACT_GELU) launch<false, ACT_GELU>(p, grid, st);
   else launch<false, ACT_QUICK_GELU>(p, grid, st);
 }

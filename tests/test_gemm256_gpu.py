@@ -484,3 +484,36 @@ def test_which_products_go_on_the_deep_ring(dev, M, N, K, kind, tile):
     other, ran = _kernels(fn[kind])
     hip.raw.gemm_force_config(-1)
     assert "gemm_bf16_kernel" in ran[0] and torch.equal(got, other)
+
+
+@pytest.mark.parametrize("m,n,k", [(1027, 8192, 1088), (1027, 8196, 1088), (1027, 8195, 1088), (2060, 4096, 1024), (1100, 14336, 1152),
+                                   (1100, 14340, 4096), (200, 1028, 640), (70, 131, 192)])
+def test_fp32_outputs(m, n, k):
+    """Sums stored as they are: whole and ragged columns, contractions on both sides of the lines between the kernels, columns in two launches
+    (280 tiles), and the same product with an addend, which the general epilogue keeps."""
+    from eventgpt_amd.ops import hip
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a, w, bias = (torch.randn(s, generator=g, device="cuda").bfloat16() for s in ((m, k), (n, k), (n,)))
+    want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    # an element is K / 32 additions to a register and the sums of 32 inside the matrix instruction, 2^-24 of the sum so far each
+    bound = (k / 32 + 32) * 2.0 ** -24 * size
+    assert bool(((hip.raw.linear(a, w, None, None, 0, True).double() - want).abs() <= bound).all())
+    y = hip.raw.linear(a, w, bias, None, 0, True).double() - bias.double()
+    assert bool(((y - want).abs() <= bound + 2.0 ** -23 * (want + bias.double()).abs()).all())
+
+
+@pytest.mark.parametrize("m,n,t", [(1032, 8192, 1100), (1032, 8192, 70), (264, 1032, 130), (72, 8, 64)])
+def test_fp32_weight_gradients(m, n, t):
+    """dY^T X into a new tensor and into a slice of a flat buffer whose neighbours stay."""
+    from eventgpt_amd.ops import hip
+    g = torch.Generator(device="cuda").manual_seed(m + n + t)
+    a, w = (torch.randn(s, generator=g, device="cuda").bfloat16() for s in ((t, m), (t, n)))
+    want, size = a.double().T @ w.double(), a.double().abs().T @ w.double().abs()
+    bound = (t / 32 + 32) * 2.0 ** -24 * size
+    kk = (t + 63) // 64 * 64
+    assert bool(((hip.raw.linear_t(a, w, True, True, None, None, 0, True, kk).double() - want).abs() <= bound).all())
+    for at in (4, 3):                                 # aligned and not
+        flat = torch.full((m * n + 8,), 7.0, device="cuda")
+        hip.raw.linear_t(a, w, True, True, None, None, 0, True, kk, flat[at:at + m * n].view(m, n))
+        assert bool(((flat[at:at + m * n].view(m, n).double() - want).abs() <= bound).all())
+        assert bool((flat[:at] == 7).all()) and bool((flat[at + m * n:] == 7).all())
