@@ -60,6 +60,44 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4_t (&acc
     }
     return;
   }
+  // A bf16 output in whole quads of columns (ACT < 0: without an activation): the bias is read once, a row's residual together.  (The general
+  // way below asks for bias, activation, residual and edges at every quad and waits for each load of its own.  us, so / now, with a bias, a
+  // residual, both: 577 x 4096 x 1024 13.0 / 11.2, 16.0 / 12.7, 18.1 / 12.7; 836 x 4096 x 4096 36.7 / 34.5, 40.9 / 36.3, 44.1 / 36.3; 40 x 4096 x
+  // 1024 7.7 / 7.2, 8.0 / 7.3, 8.5 / 7.4.  Without either it was as fast.)
+  if (p.C && !p.Cf && !p.amax_val && (ACT >= 0 || p.act == ACT_NONE) && ((p.N | p.ldc) & 3) == 0 &&
+      ((reinterpret_cast<uintptr_t>(p.C) | reinterpret_cast<uintptr_t>(p.bias) | reinterpret_cast<uintptr_t>(p.res)) & 7) == 0) {
+    const int n = n0 + wc * WN + fq * 4;
+    u32x2_t bw[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      bw[j] = p.bias && n + j * 16 < p.N ? *reinterpret_cast<const u32x2_t*>(p.bias + n + j * 16) : u32x2_t{0, 0};
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int m = m0 + wr * WM + i * 16 + frow;
+      if (m >= p.M) continue;
+      const size_t o = static_cast<size_t>(m) * p.ldc + n;
+      u32x2_t rw[TN];
+      if (p.res)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          if (n + j * 16 < p.N) rw[j] = *reinterpret_cast<const u32x2_t*>(p.res + o + j * 16);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        if (n + j * 16 >= p.N) continue;
+        float v[4] = {acc[i][j][0] + bf16lo(bw[j][0]), acc[i][j][1] + bf16hi(bw[j][0]), acc[i][j][2] + bf16lo(bw[j][1]), acc[i][j][3] + bf16hi(bw[j][1])};
+        if constexpr (ACT > 0) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = apply_act(v[r], ACT);
+        }
+        u32x2_t w = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+        if (p.res)
+          w = u32x2_t{pack_bf16x2(bf16lo(w[0]) + bf16lo(rw[j][0]), bf16hi(w[0]) + bf16hi(rw[j][0])),
+                      pack_bf16x2(bf16lo(w[1]) + bf16lo(rw[j][1]), bf16hi(w[1]) + bf16hi(rw[j][1]))};
+        *reinterpret_cast<u32x2_t*>(p.C + o + j * 16) = w;
+      }
+    }
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     const int m = m0 + wr * WM + i * 16 + frow;

@@ -517,3 +517,21 @@ def test_fp32_weight_gradients(m, n, t):
         hip.raw.linear_t(a, w, True, True, None, None, 0, True, kk, flat[at:at + m * n].view(m, n))
         assert bool(((flat[at:at + m * n].view(m, n).double() - want).abs() <= bound).all())
         assert bool((flat[:at] == 7).all()) and bool((flat[at + m * n:] == 7).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(40, 516, 320), (40, 514, 320), (300, 260, 192), (577, 1024, 1024), (577, 1028, 256), (1154, 3076, 128),
+                                   (130, 4100, 640), (836, 4096, 576)])
+def test_bias_and_residual(m, n, k):
+    """Whole and broken quads of columns, edges of tiles, with a bias, a residual and both."""
+    from eventgpt_amd.ops import hip
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a, w, b, r = (torch.randn(s, generator=g, device="cuda").bfloat16() for s in ((m, k), (n, k), (n,), (m, n)))
+    sums, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    exact = (k / 32 + 32) * 2.0 ** -24 * size                # (as in test_fp32_outputs)
+    for bias, res in ((b, None), (None, r), (b, r)):
+        mid = sums + (bias.double() if bias is not None else 0)
+        want = mid + (res.double() if res is not None else 0)
+        y = hip.raw.linear(a, w, bias, res, 0, False).double()
+        # bf16 rounds by up to 2^-8 of the value (8 significant bits): the sum with the bias, then the total with the residual
+        bound = exact + 2.0 ** -8 * 1.01 * (want.abs() + (mid.abs() + exact if res is not None else 0)) + 1e-30
+        assert bool(((y - want).abs() <= bound).all()), (bias is None, res is None)
