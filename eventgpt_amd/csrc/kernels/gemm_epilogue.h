@@ -69,8 +69,11 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4_t (&acc
     const int n = n0 + wc * WN + fq * 4;
     u32x2_t bw[TN];
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
-      bw[j] = p.bias && n + j * 16 < p.N ? *reinterpret_cast<const u32x2_t*>(p.bias + n + j * 16) : u32x2_t{0, 0};
+    for (int j = 0; j < TN; ++j) bw[j] = u32x2_t{0, 0};
+    if (p.bias)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        if (n + j * 16 < p.N) bw[j] = *reinterpret_cast<const u32x2_t*>(p.bias + n + j * 16);
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const int m = m0 + wr * WM + i * 16 + frow;

@@ -535,3 +535,25 @@ def test_bias_and_residual(m, n, k):
         # bf16 rounds by up to 2^-8 of the value (8 significant bits): the sum with the bias, then the total with the residual
         bound = exact + 2.0 ** -8 * 1.01 * (want.abs() + (mid.abs() + exact if res is not None else 0)) + 1e-30
         assert bool(((y - want).abs() <= bound).all()), (bias is None, res is None)
+
+
+@pytest.mark.parametrize("m,n,k", [(33, 16, 4096), (300, 22, 4096), (40, 4100, 2048), (577, 1024, 4096), (836, 4096, 8192), (1800, 4096, 8192)])
+def test_sums_of_split_products(m, n, k):
+    """Two to sixteen slabs, whole and broken quads of columns: bias, activation, residual and fp32 outputs of the pass that adds them."""
+    from eventgpt_amd.ops import hip
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a, w, b, r = (torch.randn(s, generator=g, device="cuda").bfloat16() for s in ((m, k), (n, k), (n,), (m, n)))
+    w = (w * 0.03125).contiguous()
+    sums, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    exact = (k / 32 + 32) * 2.0 ** -24 * size                # (as in test_fp32_outputs; the slabs' sum is a few additions of these)
+    for bias, res, act in ((None, None, 0), (b, None, 0), (None, r, 0), (b, r, 0), (b, r, 1)):
+        mid = sums + (bias.double() if bias is not None else 0)
+        if act:
+            mid = torch.nn.functional.gelu(mid)              # (slope at most 1.13; its value in fp32 to 2^-20)
+        want = mid + (res.double() if res is not None else 0)
+        near = 1.13 * exact + 2.0 ** -20 * (mid.abs() + 1)
+        for f32 in (False, True):
+            y = hip.raw.linear(a, w, bias, res, act, f32).double()
+            # 2^-8 of the value where bf16 holds it: the sum before a residual is added, and a bf16 result
+            bound = near + 2.0 ** -8 * 1.01 * ((mid.abs() + near if res is not None else 0) + (0 if f32 else want.abs() + near))
+            assert bool(((y - want).abs() <= bound).all()), (bias is None, res is None, act, f32)
