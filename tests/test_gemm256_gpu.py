@@ -1,7 +1,7 @@
 """The 256 x 256 GEMMs forced onto shapes that exercise their edges: rows / columns that do not fill a tile, one K-tile, odd
 and even K-tile counts, every epilogue, the K-strided operand layouts of the backward products; each against an fp32 matmul.
 A forced product runs on the four waves of ``gemm_quad.hip`` where those take it (K-contiguous operands, two K-tiles or more in every
-split, bf16 output in whole 16-byte chunks or slabs) and on the eight phase-staggered ones of ``gemm256_kernel`` otherwise.  Then the
+split, bf16 output in whole 16-byte chunks, fp32 sums or slabs) and on the eight phase-staggered ones of ``gemm256_kernel`` otherwise.  Then the
 tiles of ``gemm_ring.hip``.  Every case runs several times: the synchronisation is counted waits and barriers, so a race would show as
 a difference between repeats."""
 import math
