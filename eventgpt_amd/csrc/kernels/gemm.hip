@@ -1240,7 +1240,9 @@ void launch_gemm_bf16(const bf16_t* A, const bf16_t* W, bf16_t* C, float* Cf, co
   if (cfg != CFG_256x256 && g_forced_cfg < 0) {
     const RingTile ring = gemm_ring_tile(p, cfg == CFG_64x128_W8);
     if (ring != RING_NONE) {
-      launch_gemm_ring(p, ring, st);
+      GemmParams q = p;
+      output_as_slab(q);
+      launch_gemm_ring(q, ring, st);
       if (p.splitk > 1) launch_splitk_reduce(p, st);
       return;
     }
