@@ -135,16 +135,8 @@ __device__ __forceinline__ void unpack(const Frag<float>& f, float (&x)[8]) {
   for (int i = 0; i < 8; ++i) x[i] = f.v[i];
 }
 
-// A double in units of log2 as two floats: sums of two of these, high parts first, keep the float rounding of the sum's exponent.
-struct Log2Pair { float hi, lo; };
-__device__ __forceinline__ Log2Pair log2_pair(double natural) {
-  const double v = natural * 1.4426950408889634074;
-  const float hi = static_cast<float>(v);
-  return {hi, fabsf(hi) < INFINITY ? static_cast<float>(v - static_cast<double>(hi)) : 0.f};
-}
-__device__ __forceinline__ float exp_sum(const Log2Pair& a, const Log2Pair& b) {
-  return __builtin_amdgcn_exp2f((a.hi + b.hi) + (a.lo + b.lo));
-}
+// exp of an exponent put together in double: v_exp_f32 on its float in units of log2 (0 below 2^-126)
+__device__ __forceinline__ float exp_of(double v) { return __builtin_amdgcn_exp2f(static_cast<float>(v * 1.4426950408889634074)); }
 
 // One wave: decay sums F of a chunk's tokens (lane l: tokens l NH .. l NH + NH - 1), and with STAB the running maxima
 // of log_in - F.
@@ -358,9 +350,10 @@ template <int SL> struct Weights<float, SL> {
 // 64, and meet in LDS (in the query tile's place); then a wave owns sixteen value rows for all tokens, so that the
 // chunk's start state -- most of the bytes this kernel reads -- is read once.  Everything a step of 32 state columns reads
 // is requested a step ahead, the first of them with the values; what is left is latency, so three blocks to a CU (168 registers a lane,
-// under 54 KB of LDS).  A weight's exponent is the sum of two numbers kept as pairs of floats in units of log2 (`Log2Pair`): three
-// additions and one instruction where the double difference and expf took most of the vector instructions.  4096 tokens, 134 MB of
-// states: 8 heads of 512 x 256 with a maximum 105 us, 128 heads of 64 x 128 106, were both 174 (state 52 and 58, were 74).
+// under 54 KB of LDS).  A weight's exponent is put together in double, as the sums it is the difference of are, and goes to v_exp_f32 in
+// units of log2; expf of it, with the library's range checks, took most of the vector instructions.  (Sums kept as pairs of floats are as
+// fast and lose bits from 2^30 on.)  4096 tokens, 134 MB of states: 8 heads of 512 x 256 with a maximum 105 us, 128 heads of 64 x 128 106,
+// were both 174 (state 52 and 58, were 74).
 template <typename T, bool STAB, int SL>
 __global__ __launch_bounds__(256, 3) void scan_chunk_out_kernel(ScanArgs a, ScanChunks c) {
   constexpr int NH = SL / 64, QS = 64 + 8, QV = sizeof(T) == 4 ? 2 : 1;
@@ -370,8 +363,9 @@ __global__ __launch_bounds__(256, 3) void scan_chunk_out_kernel(ScanArgs a, Scan
   __shared__ __attribute__((aligned(16))) Tile vt;                                // values of the chunk's tokens
   __shared__ __attribute__((aligned(16))) unsigned char qp_lds[Q_BYTES > Wgt::BYTES ? Q_BYTES : Wgt::BYTES];
   T* qs = reinterpret_cast<T*>(qp_lds);                               // [token][64 of N]
-  __shared__ Log2Pair tok_s[SL], key_s[SL];                           // F - m and log_in - F (F and -F)
-  __shared__ float in_s[SL], m_s[SL], inv_s[64], den_s[4][64];
+  __shared__ __attribute__((aligned(16))) double F_s[SL];
+  __shared__ __attribute__((aligned(16))) float in_s[SL];
+  __shared__ float m_s[SL], inv_s[64], den_s[4][64];
   __shared__ __attribute__((aligned(16))) float nrm_s[64];            // the start state's normaliser, of the columns at hand
   const ScanTile tile(a.H);
   const int v0 = tile.v0, h = tile.h, ci = tile.chunk;
@@ -422,11 +416,9 @@ __global__ __launch_bounds__(256, 3) void scan_chunk_out_kernel(ScanArgs a, Scan
 #pragma unroll
     for (int i = 0; i < NH; ++i) {
       const int t = lane * NH + i;
-      const float mt = STAB ? static_cast<float>(F[i] + fmax(static_cast<double>(m0), top[i])) : 0.f;
+      F_s[t] = F[i];
       in_s[t] = li[i];
-      m_s[t] = mt;
-      tok_s[t] = log2_pair(F[i] - static_cast<double>(mt));
-      key_s[t] = log2_pair((STAB ? static_cast<double>(li[i]) : 0.0) - F[i]);
+      m_s[t] = STAB ? static_cast<float>(F[i] + fmax(static_cast<double>(m0), top[i])) : 0.f;
     }
     if constexpr (STAB) {
       const int last = c.chunks[ci * 4 + 3];
@@ -435,7 +427,6 @@ __global__ __launch_bounds__(256, 3) void scan_chunk_out_kernel(ScanArgs a, Scan
             static_cast<float>(fmax(c.fl[ho] + m0, c.am[ho]));
     }
   }
-  const Log2Pair start = log2_pair(static_cast<double>(m0));
   vt.put(vr);
   f32x4_t st[NH][NH][4], inter[NH][4];            // [key half][token half][token tile]
   float nq[NH];
@@ -505,23 +496,28 @@ __global__ __launch_bounds__(256, 3) void scan_chunk_out_kernel(ScanArgs a, Scan
     __syncthreads();                              // the query tile, or the scores of the half before, are no longer read
     float den[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int k = 0; k <= th; ++k)
+    for (int k = 0; k <= th; ++k) {
+      // weighted scores of keys 64 k + 16 wid + 4 g + r and token 64 th + 16 j + fr
+      const int s0 = k * 64 + wid * 16 + g * 4;
+      const f32x4_t in = load4(in_s + s0);
+      double Fs[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) Fs[r] = F_s[s0 + r];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        // weighted scores of keys 64 k + 16 wid + 4 g + r and token 64 th + 16 j + fr
-        const int t = th * 64 + j * 16 + fr, s0 = k * 64 + wid * 16 + g * 4;
-        const Log2Pair Ft = tok_s[t];
+        const int t = th * 64 + j * 16 + fr;
+        const double Ft = F_s[t];
+        const float mt = m_s[t];
         f32x4_t w = st[k][th][j];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int s = s0 + r;
-          float e = exp_sum(Ft, key_s[s]);
-          if constexpr (!STAB) e *= in_s[s];
-          w[r] = s <= t && t < len ? w[r] * (e * a.qscale) : 0.f;
+          const float e = STAB ? exp_of(Ft - Fs[r] + static_cast<double>(in[r] - mt)) : exp_of(Ft - Fs[r]) * in[r];
+          w[r] = s0 + r <= t && t < len ? w[r] * (e * a.qscale) : 0.f;
           den[j] += w[r];
         }
         Wgt::put(qp_lds, j * 16 + fr, s0, w);
       }
+    }
     if constexpr (STAB) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -537,7 +533,7 @@ __global__ __launch_bounds__(256, 3) void scan_chunk_out_kernel(ScanArgs a, Scan
       float d = nq[th];
       d += __shfl_xor(d, 1, 64);
       d += __shfl_xor(d, 2, 64);
-      d = d * exp_sum(tok_s[t], start) * a.qscale + (den_s[0][tl] + den_s[1][tl] + den_s[2][tl] + den_s[3][tl]);
+      d = d * exp_of(F_s[t] + static_cast<double>(m0 - m_s[t])) * a.qscale + (den_s[0][tl] + den_s[1][tl] + den_s[2][tl] + den_s[3][tl]);
       if ((tid & 3) == 0) inv_s[tl] = 1.f / (fmaxf(fabsf(d), expf(-m_s[t])) + 1e-6f);
       __syncthreads();
     }
@@ -550,7 +546,7 @@ __global__ __launch_bounds__(256, 3) void scan_chunk_out_kernel(ScanArgs a, Scan
       for (int kb = 0; kb < SL / 32; ++kb)
         if (kb < 2 * th || (kb < 2 * th + 2 && (kb - 2 * th) * 2 <= j)) y = mma(vf[kb], Wgt::frag(qp_lds, tl, kb * 32 + g * 8), y);
       if (t >= len) continue;
-      y += inter[th][j] * (exp_sum(tok_s[t], start) * a.qscale);
+      y += inter[th][j] * (exp_of(F_s[t] + static_cast<double>(m0 - m_s[t])) * a.qscale);
       if constexpr (STAB) y *= inv_s[tl];
       const int v = wid * 16 + g * 4;
       if (a.skip) y += skip * vt.four(t, v);

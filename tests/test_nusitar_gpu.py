@@ -1079,3 +1079,43 @@ def test_recurrence_of_strong_decays(raw, dev, dtype, kind, H, V):
     want = want.reshape(T, -1)
     bound = 2e-5 * want.abs().max() + (0.0 if dtype == torch.float32 else 2.0 ** -8 * 1.01) * want.abs()
     assert bool(((o.cpu().double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("kind,H,V", [("ssd", 3, 64), ("mlstm", 2, 128)])
+@pytest.mark.parametrize("reset", [-2.0 ** 40, torch.finfo(torch.float32).min])
+def test_recurrence_through_a_reset(raw, dev, dtype, kind, H, V, reset):
+    """A decay that empties the state inside a chunk (the lowest float: at the last token) and ordinary ones
+    behind it.  Decays and gates are multiples of 1 / 256, so sums of them are exact in double and a weight is as good as without the reset."""
+    T, Nn = 199, 64
+    q, qr = typed(rnd(T, H, Nn) + 0.8, dtype, dev)
+    k, kr = typed(rnd(T, H, Nn, seed=1) + 0.8, dtype, dev)
+    v, vr = typed(rnd(T, H, V, seed=2), dtype, dev)
+    ld = -((rnd(T, H, seed=3).abs() * 64).round() / 256).float()
+    for t in (20, 75, 150) if reset > -1e30 else (T - 1,):
+        ld[t] = reset
+    f = dict(device=dev, dtype=torch.float32)
+    F = ld.double().cumsum(0)
+    w = F[:, None] - F[None]                                          # [t, s, H]
+    w[~torch.ones(T, T, dtype=torch.bool).tril()] = -torch.inf
+    if kind == "mlstm":
+        li = ((256 * rnd(T, H, seed=4)).round() / 256).float()
+        li[-1] = 0                                                    # (a sum with the lowest float drops it)
+        gates, st = (li.to(dev), None), (torch.zeros(1, H, V, Nn, **f), torch.zeros(2, 1, H, Nn, **f), torch.zeros(2, 1, H, **f))
+        w = w + li.double()[None]
+        m = torch.maximum(w.amax(1), F)
+        w = (w - m[:, None]).exp()
+    else:
+        dt = torch.nn.functional.softplus(rnd(T, H, seed=4)).float()
+        gates, st = (None, dt.to(dev)), (torch.zeros(1, H, V, Nn, **f), None, None)
+        w = w.exp() * dt.double()[None]
+    w, size = w * torch.einsum("thn,shn->tsh", qr, kr), w * torch.einsum("thn,shn->tsh", qr.abs(), kr.abs())
+    want, size_of_y = torch.einsum("tsh,shv->thv", w, vr), torch.einsum("tsh,shv->thv", size, vr.abs())
+    if kind == "mlstm":
+        den = (torch.maximum(w.sum(1).abs(), (-m).exp()) + 1e-6)[..., None]
+        want, size_of_y = want / den, (size_of_y + (want / den).abs() * size.sum(1)[..., None]) / den
+    rb = RowBatch(dev, False, seqs=pack([T]), scan_chunk=raw.scan_chunk(dtype == torch.float32))
+    o = raw.scan_prefill_(q.view(T, -1), k.view(T, -1), v.view(T, -1), H, 1, Nn, V, 1.0, ld.to(dev), *gates, None, *st, rb.chunks, rb.scan_seqs)
+    # weights and states in two bf16 parts, 2^-17 of a product each, an exponent of up to 64 as a float 2^-18, and fp32 sums; bf16 rounds the result
+    bound = 2.0 ** -15 * size_of_y + (0.0 if dtype == torch.float32 else 2.0 ** -8 * 1.01) * want.abs()
+    assert bool(((o.cpu().double().view(T, H, V) - want).abs() <= bound).all())
