@@ -154,7 +154,7 @@ __device__ __forceinline__ void chunk_gates(const ScanArgs& a, int row0, int len
     if constexpr (STAB) li[i] = t < len ? a.log_in[gi] : -INFINITY;
     else li[i] = t < len ? a.scale_in[gi] : 0.f;
   }
-  const double before = wave_scan_add(sum) - sum;
+  const double upto = __shfl_up(wave_scan_add(sum), 1, 64), before = lane > 0 ? upto : 0.0;     // (less `sum`, a long one would take it away)
 #pragma unroll
   for (int i = 0; i < NH; ++i) F[i] += before;
   if constexpr (STAB) {

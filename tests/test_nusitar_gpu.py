@@ -1084,10 +1084,11 @@ def test_recurrence_of_strong_decays(raw, dev, dtype, kind, H, V):
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("kind,H,V", [("ssd", 3, 64), ("mlstm", 2, 128)])
 @pytest.mark.parametrize("reset", [-2.0 ** 40, torch.finfo(torch.float32).min])
-def test_recurrence_through_a_reset(raw, dev, dtype, kind, H, V, reset):
+@pytest.mark.parametrize("T", [199, 200])          # (bf16: the last token has a lane of the prefix sums to itself, or shares it)
+def test_recurrence_through_a_reset(raw, dev, dtype, kind, H, V, reset, T):
     """A decay that empties the state inside a chunk (the lowest float: at the last token) and ordinary ones
     behind it.  Decays and gates are multiples of 1 / 256, so sums of them are exact in double and a weight is as good as without the reset."""
-    T, Nn = 199, 64
+    Nn = 64
     q, qr = typed(rnd(T, H, Nn) + 0.8, dtype, dev)
     k, kr = typed(rnd(T, H, Nn, seed=1) + 0.8, dtype, dev)
     v, vr = typed(rnd(T, H, V, seed=2), dtype, dev)
