@@ -146,8 +146,9 @@ __device__ __forceinline__ void memory_step(const StepMemory& m, int b, int i0, 
   const StateRows rows = request_state(S, m.N, v0, vb);
   const int e0 = min(tid, m.N - 1);
   const long long image = static_cast<long long>(m.slots) * m.H;
-  const float m_img[2] = {m.m[gi], m.m[image + gi]};
-  const float n_img[2] = {m.n[static_cast<long long>(gi) * m.N + e0], m.n[(image + gi) * m.N + e0]};
+  // (picked by a select below: an array indexed with the position is scratch memory)
+  const float m_even = m.m[gi], m_odd = m.m[image + gi];
+  const float n_even = m.n[static_cast<long long>(gi) * m.N + e0], n_odd = m.n[(image + gi) * m.N + e0];
   const float gi0 = src1<M>(m.src, b, m.i_col + h), gf0 = src1<M>(m.src, b, m.f_col + h), ib = m.ib[h], fb = m.fb[h];
   const float q0 = src1<M>(m.src, b, m.q_col + h * m.N + e0), k0 = src1<M>(m.src, b, m.k_col + h * m.N + e0);
   const float vr = src1<M>(m.src, b, m.v_col + h * m.V + v0 + min(tid, vb - 1));
@@ -160,7 +161,7 @@ __device__ __forceinline__ void memory_step(const StepMemory& m, int b, int i0, 
   const long long from = (static_cast<long long>(p & 1) * m.slots + b) * m.H + h;
   const long long to = (static_cast<long long>((p + 1) & 1) * m.slots + b) * m.H + h;
   const float li = m.cap * tanhf((gi0 + ib) / m.cap), lf = -softplus_f(-m.cap * tanhf((gf0 + fb) / m.cap));
-  const float mt = fresh ? 0.f : m_img[p & 1], m1 = fmaxf(lf + mt, li);
+  const float mt = fresh ? 0.f : p & 1 ? m_odd : m_even, m1 = fmaxf(lf + mt, li);
   const float decay = expf(lf + mt - m1), add = expf(li - m1);
   for (int i = tid; i < vb; i += 256) avs[i] = add * (i < 256 ? to_f32(from_f32<T>(vr)) : src_t<T, M>(m.src, b, m.v_col + h * m.V + v0 + i));
   float dot = 0.f;
@@ -170,7 +171,7 @@ __device__ __forceinline__ void memory_step(const StepMemory& m, int b, int i0, 
     const float k = first ? to_f32(from_f32<T>(k0)) : src_t<T, M>(m.src, b, m.k_col + h * m.N + e);
     qs[e] = q;
     ks[e] = k;
-    const float n1 = (fresh ? 0.f : (first ? n_img[p & 1] : m.n[from * m.N + e]) * decay) + add * k;
+    const float n1 = (fresh ? 0.f : (first ? (p & 1 ? n_odd : n_even) : m.n[from * m.N + e]) * decay) + add * k;
     if (v0 == 0) m.n[to * m.N + e] = n1;
     dot += n1 * q;
   }
