@@ -19,6 +19,8 @@
 //
 // n and m are stored twice, indexed by the parity of the position they are read at, so that a decode step
 // (decode_step.hip) can write the next ones while other blocks still read the old ones.
+#include <algorithm>
+
 #include "elem.h"
 #include "../layered_kernels.h"
 
@@ -350,11 +352,14 @@ template <int SL> struct Weights<float, SL> {
 // 64, and meet in LDS (in the query tile's place); then a wave owns sixteen value rows for all tokens, so that the
 // chunk's start state -- most of the bytes this kernel reads -- is read once.  Everything a step of 32 state columns reads
 // is requested a step ahead, the first of them with the values; what is left is latency, so three blocks to a CU (168 registers a lane,
-// under 54 KB of LDS).  A weight's exponent is put together in double, as the sums it is the difference of are, and goes to v_exp_f32 in
-// units of log2; expf of it, with the library's range checks, took most of the vector instructions.  (Sums kept as pairs of floats are as
-// fast and lose bits from 2^30 on.)  4096 tokens, 134 MB of states: 8 heads of 512 x 256 with a maximum 105 us, 128 heads of 64 x 128 106,
-// were both 174 (state 52 and 58, were 74).
-template <typename T, bool STAB, int SL>
+// under 54 KB of LDS).  To stay within those registers rows are offsets from a uniform base, 32 bits wide but for strides that need `Off`
+// to be 64, and the values' operands are read behind the scores: with a pointer a lane and those operands early 13 registers of the
+// instance with a maximum lay in scratch memory.  A weight's exponent is put together in double, as the sums it is the difference of are,
+// and goes to v_exp_f32 in units of log2; expf of it, with the library's range checks, took most of the vector instructions.  (Sums kept as
+// pairs of floats are as fast and lose bits from 2^30 on.)  4096 tokens, 134 MB of states: 8 heads of 512 x 256 with a maximum 87 us (105 out
+// of scratch memory), 128 heads of 64 x 128 89, were both 174 with neither (state 48 and 53, were 74); the three launches 147 and 184, 100
+// tokens of 4 heads 30.9 (163.6, 185.2 and 32.8 out of scratch memory).
+template <typename T, bool STAB, int SL, typename Off>
 __global__ __launch_bounds__(256, 3) void scan_chunk_out_kernel(ScanArgs a, ScanChunks c) {
   constexpr int NH = SL / 64, QS = 64 + 8, QV = sizeof(T) == 4 ? 2 : 1;
   using Tile = Columns<T, SL>;
@@ -370,27 +375,26 @@ __global__ __launch_bounds__(256, 3) void scan_chunk_out_kernel(ScanArgs a, Scan
   const ScanTile tile(a.H);
   const int v0 = tile.v0, h = tile.h, ci = tile.chunk;
   const int row0 = c.chunks[ci * 4], len = min(c.chunks[ci * 4 + 1], SL);
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, fr = lane & 15, g = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6), fr = lane & 15, g = lane >> 4;
   const int nv = min(64, a.V - v0), hk = h / a.per_group;
   const long long ho = static_cast<long long>(ci) * a.H + h;
-  const T* qp = static_cast<const T*>(a.q) + static_cast<long long>(hk) * a.N;
-  const T* kp[NH];
-#pragma unroll
-  for (int k = 0; k < NH; ++k)
-    kp[k] = static_cast<const T*>(a.k) + (row0 + min(k * 64 + wid * 16 + fr, len - 1)) * a.ldk + static_cast<long long>(hk) * a.N;
-  const float* S0 = c.dS + (ho * a.V + v0 + wid * 16 + fr) * a.N;
+  const T* qp = static_cast<const T*>(a.q) + row0 * a.ldq + static_cast<long long>(hk) * a.N;
+  const T* kp = static_cast<const T*>(a.k) + row0 * a.ldk + static_cast<long long>(hk) * a.N;
+  const Off ldq = static_cast<Off>(a.ldq), ldk = static_cast<Off>(a.ldk);
+  const float* S0 = c.dS + (ho * a.V + v0 + wid * 16) * a.N;
+  const unsigned S_lane = fr * a.N + g * 8;
   const float* nrm = STAB ? c.dn + ho * a.N : nullptr;
   const bool rows_v = wid * 16 < nv;              // this wave has value rows
   const auto vr = Tile::request(static_cast<const T*>(a.v), a.ldv, row0, len, h * a.V + v0, nv);
   u32x4_t qr[2 * NH][QV];
   float nr = 0.f;
   auto request_q = [&](int n0) {
-    if (STAB && tid < 64 && n0 + tid < a.N) nr = nrm[n0 + tid];
+    if constexpr (STAB) nr = nrm[min(n0 + lane, a.N - 1)];
 #pragma unroll
     for (int i = 0; i < 2 * NH; ++i) {
       const int idx = tid + i * 256, t = idx >> 3, c8 = (idx & 7) * 8;
       if (n0 + c8 < a.N) {
-        const T* p = qp + (row0 + min(t, len - 1)) * a.ldq + n0 + c8;
+        const T* p = qp + (min(t, len - 1) * ldq + (n0 + c8));
 #pragma unroll
         for (int v = 0; v < QV; ++v) qr[i][v] = load16(p + v * 4);
       }
@@ -400,8 +404,8 @@ __global__ __launch_bounds__(256, 3) void scan_chunk_out_kernel(ScanArgs a, Scan
   float xn[8];
   auto request_step = [&](int n) {
 #pragma unroll
-    for (int k = 0; k < NH; ++k) kn[k] = load_frag(kp[k] + n + g * 8);
-    if (rows_v) load8(S0 + n + g * 8, xn);
+    for (int k = 0; k < NH; ++k) kn[k] = load_frag(kp + (min(k * 64 + wid * 16 + fr, len - 1) * ldk + (n + g * 8)));
+    if (rows_v) load8(S0 + (S_lane + n), xn);
     else
 #pragma unroll
       for (int j = 0; j < 8; ++j) xn[j] = 0.f;
@@ -450,7 +454,7 @@ __global__ __launch_bounds__(256, 3) void scan_chunk_out_kernel(ScanArgs a, Scan
 #pragma unroll
         for (int v = 0; v < QV; ++v) *reinterpret_cast<u32x4_t*>(qs + t * QS + c8 + v * 4) = qr[i][v];
     }
-    if (STAB && tid < 64) nrm_s[tid] = nr;
+    if (STAB && wid == 0) nrm_s[lane] = nr;
     if (n0 + 64 < a.N) request_q(n0 + 64);
     __syncthreads();
     for (int n = 0; n < nn; n += 32) {
@@ -486,9 +490,6 @@ __global__ __launch_bounds__(256, 3) void scan_chunk_out_kernel(ScanArgs a, Scan
       }
     }
   }
-  Frag<T> vf[SL / 32];
-#pragma unroll
-  for (int kb = 0; kb < SL / 32; ++kb) vf[kb] = vt.frag(wid * 16, kb);
   const float skip = a.skip ? a.skip[h] : 0.f;
 #pragma unroll
   for (int th = 0; th < NH; ++th) {
@@ -538,6 +539,9 @@ __global__ __launch_bounds__(256, 3) void scan_chunk_out_kernel(ScanArgs a, Scan
       __syncthreads();
     }
     if (!rows_v) continue;
+    Frag<T> vf[SL / 32];                          // (here and not ahead of the scores, where there are no registers left)
+#pragma unroll
+    for (int kb = 0; kb < 2 * (th + 1); ++kb) vf[kb] = vt.frag(wid * 16, kb);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int tl = j * 16 + fr, t = th * 64 + tl;
@@ -563,7 +567,10 @@ static void launch_scan(const ScanArgs& a, const ScanChunks& c, hipStream_t st) 
   const dim3 g2(static_cast<unsigned>((quads + 255) / 256) + (STAB ? 1 : 0), a.H, c.nseq);
   hipLaunchKernelGGL((scan_chunk_state_kernel<T, STAB, SL>), g1, block, 0, st, a, c);
   hipLaunchKernelGGL(scan_chunk_pass_kernel<STAB>, g2, block, 0, st, a, c);
-  hipLaunchKernelGGL((scan_chunk_out_kernel<T, STAB, SL>), g1, block, 0, st, a, c);
+  if (std::max(a.ldq, a.ldk) < (1ll << 31) / SL - a.N)
+    hipLaunchKernelGGL((scan_chunk_out_kernel<T, STAB, SL, unsigned>), g1, block, 0, st, a, c);
+  else
+    hipLaunchKernelGGL((scan_chunk_out_kernel<T, STAB, SL, long long>), g1, block, 0, st, a, c);
 }
 void launch_scan_prefill(const ScanArgs& a, const ScanChunks& c, bool f32, hipStream_t st) {
   const bool stab = a.log_in != nullptr;

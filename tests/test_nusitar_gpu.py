@@ -1120,3 +1120,21 @@ def test_recurrence_through_a_reset(raw, dev, dtype, kind, H, V, reset, T):
     # weights and states in two bf16 parts, 2^-17 of a product each, an exponent of up to 64 as a float 2^-18, and fp32 sums; bf16 rounds the result
     bound = 2.0 ** -15 * size_of_y + (0.0 if dtype == torch.float32 else 2.0 ** -8 * 1.01) * want.abs()
     assert bool(((o.cpu().double().view(T, H, V) - want).abs() <= bound).all())
+
+
+def test_recurrence_over_rows_far_apart(raw, dev):
+    """Queries and keys of row strides on both sides of what 32-bit offsets reach within a chunk: the bits of close ones."""
+    T, H, Nn, V = 130, 2, 64, 64
+    f = dict(device=dev, dtype=torch.float32)
+    q, k = (typed(rnd(T, H * Nn, seed=i), torch.bfloat16, dev)[0] for i in range(2))
+    v, _ = typed(rnd(T, H * V, seed=2), torch.bfloat16, dev)
+    ld, li = -rnd(T, H, seed=3).abs().float().to(dev), rnd(T, H, seed=4).float().to(dev)
+    rb = RowBatch(dev, False, seqs=pack([T]), scan_chunk=raw.scan_chunk(False))
+    outs = []
+    for stride in (H * Nn, 2 ** 24 - 256, 2 ** 24 + 256):
+        buf = torch.empty((T - 1) * stride + 2 * H * Nn, dtype=torch.bfloat16, device=dev) if stride > H * Nn else None
+        a, b = (q, k) if buf is None else (torch.as_strided(buf, (T, H * Nn), (stride, 1), o * H * Nn).copy_(t) for o, t in enumerate((q, k)))
+        st = (torch.zeros(1, H, V, Nn, **f), torch.zeros(2, 1, H, Nn, **f), torch.zeros(2, 1, H, **f))
+        outs.append([raw.scan_prefill_(a, b, v, H, 1, Nn, V, 1.0, ld, li, None, None, *st, rb.chunks, rb.scan_seqs), *st])
+        del buf, a, b
+    assert all(torch.equal(x, y) for o in outs[1:] for x, y in zip(outs[0], o))
