@@ -168,7 +168,7 @@ void launch_gemm_grouped_few(const GemmParams& p, int rows, hipStream_t st) {
 // A dense gated product of a decode step.  us against the slabs of gemm_fewrow_kernel and the launch that sums and gates them, 5 / 32 rows:
 // 2 x 2816 columns over 1024 k 6.0 / 6.5 against 8.0 / 8.8, 2 x 5632 over 2048 11.5 / 13.3 and 14.5 / 15.9, 2 x 11008 over 4096 39.2 / 42.8 and 38.6 /
 // 42.8 (344 workgroups: a round and a third of one a CU), 2 x 13824 over 5120 51.6 / 57.7 and 56.8 / 66.0; the error against 64 bits is the same.
-bool gemm_few_glu_serves(int rows, int I, int K) { return rows <= AM && K % TK == 0 && I % TN == 0; }
+bool gemm_few_glu_serves(int rows, int I, int K) { return rows <= AM && K > 0 && K % TK == 0 && I % TN == 0; }
 void launch_gemm_few_glu(const bf16_t* A, const bf16_t* W, bf16_t* C, int rows, int I, int K, int glu_act, hipStream_t st) {
   GemmParams p{};
   p.A = A, p.W = W, p.C = C, p.M = rows, p.N = I, p.K = p.lda = p.ldw = K, p.ldc = I, p.splitk = 1, p.k_per_split = K;

@@ -1138,3 +1138,10 @@ def test_recurrence_over_rows_far_apart(raw, dev):
         outs.append([raw.scan_prefill_(a, b, v, H, 1, Nn, V, 1.0, ld, li, None, None, *st, rb.chunks, rb.scan_seqs), *st])
         del buf, a, b
     assert all(torch.equal(x, y) for o in outs[1:] for x, y in zip(outs[0], o))
+
+
+@pytest.mark.parametrize("rows", [4, 40])
+def test_gated_products_without_a_contraction_are_refused(raw, dev, rows):
+    x, w = (torch.empty(n, 0, dtype=torch.bfloat16, device=dev) for n in (rows, 64))
+    with pytest.raises(RuntimeError):
+        raw.linear_glu(x, w, 1)
