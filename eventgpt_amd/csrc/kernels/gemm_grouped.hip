@@ -165,10 +165,29 @@ void launch_gemm_grouped_few(const GemmParams& p, int rows, hipStream_t st) {
   else launch<false, false>(p, grid, st);
 }
 
-// A dense gated product of a decode step.  us against the slabs of gemm_fewrow_kernel and the launch that sums and gates them, 5 / 32 rows:
-// 2 x 2816 columns over 1024 k 6.0 / 6.5 against 8.0 / 8.8, 2 x 5632 over 2048 11.5 / 13.3 and 14.5 / 15.9, 2 x 11008 over 4096 39.2 / 42.8 and 38.6 /
-// 42.8 (344 workgroups: a round and a third of one a CU), 2 x 13824 over 5120 51.6 / 57.7 and 56.8 / 66.0; the error against 64 bits is the same.
-bool gemm_few_glu_serves(int rows, int I, int K) { return rows <= AM && K > 0 && K % TK == 0 && I % TN == 0; }
+// A dense gated product of a decode step, against the slabs of gemm_fewrow_kernel and the launch that sums and gates them; the error against 64
+// bits is the same.  What it saves is the slabs; what it gives up is K divided over more workgroups than there are tiles, and whole rounds.
+// Time with it / without, weights from memory, 5 / 16 / 32 rows:
+//  * K below 2048, 4 to 1024 tiles: 0.5 to 0.99 (1920 and 64 tiles 1.03 at 32 rows)
+//  * K 2048, tiles 48 / 64 / 72 / 88 / 128 / 176 / 256: 1.17 1.17 1.20 / 1.11 1.07 1.14 / 0.97 0.94 0.94 / 0.98 0.94 0.93 / 0.92 0.89 0.92 / 0.79 0.78
+//    0.80 / 0.86 0.84 0.78 (2 x 5632 columns 13.9 -> 10.9 us, 14.2 -> 11.1, 14.9 -> 12.0)
+//  * K 2560 to 4608 below 136 tiles: 0.9 to 1.6; 144: 0.88 to 0.99, 176: 0.90 to 0.98, 256: 0.78 to 0.98.  K 5120: 144 between 0.94 and 1.11 from run to
+//    run, 176 0.89 0.89 0.93, 256 0.85 0.84 0.80
+//  * a round and a part, 257 / 288 / 320 / 352 / 400 tiles: K 2048 1.01 1.03 1.02 / 1.01 1.02 1.02 / 0.96 0.92 0.95 / 0.93 0.90 0.87 / 0.93 0.87 0.85; 4096
+//    1.14 1.14 1.12 / 1.18 1.18 1.18 / 1.08 1.02 1.06 / 1.04 0.98 0.98 / 0.96 0.93 0.91; 5120 1.10 1.09 1.12 / 1.12 1.10 1.14 / 1.09 1.07 1.08 / 1.05 1.00
+//    0.99 / 0.94 0.92 0.89; 512: 0.87 to 1.02, 0.80 to 0.96, 0.73 to 0.86
+//  * more rounds, 576 / 640 / 768 / 1024 tiles: K 2048 1.10 1.00 0.92 / 1.05 0.93 0.84 / 1.04 0.92 0.80 / 0.97 0.95 0.91; 4096 1.15 1.03 0.99 / 1.02 0.91 0.85 /
+//    0.97 0.84 0.80 / 0.97 0.94 0.94
+//  * K 6144: 1.0 to 1.3 below 400 tiles; 8192: 0.9 to 1.2
+bool gemm_few_glu_serves(int rows, int I, int K) {
+  if (rows > AM || K <= 0 || K % TK || I % TN) return false;
+  const int tiles = I / TN;
+  if (K < 2048) return true;
+  if (K > 5120) return false;
+  if (tiles <= 256) return tiles >= (K < 2304 ? 72 : 160);
+  if (tiles <= 512) return tiles >= (K < 2304 ? 320 : 400);
+  return rows > 8 && tiles >= 640;
+}
 void launch_gemm_few_glu(const bf16_t* A, const bf16_t* W, bf16_t* C, int rows, int I, int K, int glu_act, hipStream_t st) {
   GemmParams p{};
   p.A = A, p.W = W, p.C = C, p.M = rows, p.N = I, p.K = p.lda = p.ldw = K, p.ldc = I, p.splitk = 1, p.k_per_split = K;

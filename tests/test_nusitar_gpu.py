@@ -1145,3 +1145,25 @@ def test_gated_products_without_a_contraction_are_refused(raw, dev, rows):
     x, w = (torch.empty(n, 0, dtype=torch.bfloat16, device=dev) for n in (rows, 64))
     with pytest.raises(RuntimeError):
         raw.linear_glu(x, w, 1)
+
+
+@pytest.mark.parametrize("rows,inner,K", [(5, 71 * 32, 2048), (5, 159 * 32, 2560), (5, 159 * 32, 4096), (32, 257 * 32, 4096), (5, 399 * 32, 4096), (8, 640 * 32, 2048),
+                                          (32, 639 * 32, 2048), (4, 96, 5248)])
+def test_gated_products_that_divide_their_contraction(raw, dev, rows, inner, K):
+    """Few tiles over a long contraction, a round and a part of one: the slabs and the launch behind them, to the bit."""
+    x, w = (torch.randn(n, K, dtype=torch.bfloat16, device=dev) * 0.1 for n in (rows, 2 * inner))
+    assert torch.equal(raw.linear_glu(x, w, 1), raw.glu_rows(raw.linear_slabs(x, w), 1, False))
+
+
+@pytest.mark.parametrize("rows,inner,K", [(3, 32, 1920), (16, 72 * 32, 2048), (9, 160 * 32, 2304), (32, 256 * 32, 2304), (17, 320 * 32, 2048), (2, 400 * 32, 2304),
+                                          (9, 640 * 32, 2048)])
+def test_gated_products_of_whole_contractions(raw, dev, rows, inner, K):
+    """On the other side of the lines: one launch, against 64 bits."""
+    x, w = (torch.randn(n, K, dtype=torch.bfloat16, device=dev) * 0.1 for n in (rows, 2 * inner))
+    y = x.double() @ w.double().t()
+    g, u = y[:, :inner], y[:, inner:]
+    want = torch.nn.functional.silu(g) * u
+    # a bf16 result, and factors that are sums of K products, 2^-24 of the sum so far each (silu's slope is at most 1.1)
+    size = x.double().abs() @ w.double().abs().t()
+    off = (K / 32 + 32) * 2.0 ** -24 * (1.1 * size[:, :inner] * u.abs() + size[:, inner:] * g.abs()) + 2.0 ** -20 * want.abs()
+    assert bool(((raw.linear_glu(x, w, 1).double() - want).abs() <= off + 2.0 ** -8 * 1.01 * want.abs()).all())
