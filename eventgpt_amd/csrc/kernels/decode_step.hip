@@ -430,8 +430,15 @@ void launch_parallel_step(const StepHeads& h, const StepMemory& m, const int* po
   };
   hipLaunchKernelGGL((vb > 16 ? kernel(std::true_type{}) : kernel(std::false_type{})), grid, dim3(256), lds, st, h, m, pos, live, vb);
 }
+// Where one launch is ahead of two.  us, two / one, 600 cached keys, 16 splits: 16 heads 10.3 / 7.9 for one stream, 12.1 / 9.3 for two, four splits
+// 13.7 / 10.9 and 15.1 / 12.8 for three and four; 32 heads (the same order, four splits from three on) 11.7 / 9.2, 14.4 / 12.7, 17.6 / 14.5, 21.1 /
+// 17.9.  Every block makes the norms of all heads anew, which is level around a thousand blocks and lost with more: 64 heads, 16 splits, one
+// stream 14.9 / 13.6, two (2048 blocks) 20.2 / 20.6, four 32.7 / 34.0 (100 keys 25.0 / 27.9); 128 heads, one stream 17.8 / 19.5, but with two splits
+// 17.9 / 16.5, four streams of those (1024 blocks) 24.8 / 22.0.  And it has fewer waves a CU to stream long caches with: 64 key heads of 2000 keys, two
+// streams (131 MB) 35.6 / 34.2, three 50.4 / 54.0, four 62.7 / 69.4.
 bool attend_step_ok(const StepHeads& h, const StepMemory& m, int B, int nsplit) {
-  return B <= GEMV_ROWS_MAX && nsplit > 1 && nsplit <= 16 && (h.a.D == 64 || h.a.D == 128) && src_mode(m.src) == SRC_ONE && h.a.src.p == m.src.p;
+  return B <= GEMV_ROWS_MAX && nsplit > 1 && nsplit <= 16 && (h.a.D == 64 || h.a.D == 128) && src_mode(m.src) == SRC_ONE && h.a.src.p == m.src.p &&
+         static_cast<long long>(B) * h.a.Hq * nsplit <= 1024 && static_cast<long long>(B) * h.a.Hkv * h.a.cap * h.a.D <= 1ll << 25;
 }
 void launch_attend_step(const StepHeads& h, const StepMemory& m, const StepSplits& sp, const int* pos, const int* live, int B, hipStream_t st) {
   const int vb = rows_per_block(m.H, m.V, B);

@@ -1011,11 +1011,12 @@ def test_gated_products_of_few_rows(raw, dev, rows, inner, K, act):
 
 @pytest.mark.parametrize("H,G,D,rot,normed,B,nsplit,slabs", [(4, 2, 128, 128, True, 1, 16, 1), (6, 2, 64, 32, True, 4, 5, 1), (2, 2, 128, 0, False, 3, 2, 1),
                                                             (4, 1, 64, 64, False, 2, 16, 1), (4, 2, 128, 64, True, 5, 4, 1), (4, 2, 128, 64, True, 2, 4, 2),
-                                                            (4, 2, 128, 64, True, 2, 1, 1)])
+                                                            (32, 8, 128, 128, True, 2, 16, 1), (40, 40, 64, 64, True, 1, 16, 1),
+                                                            (33, 33, 64, 0, True, 2, 16, 1), (4, 2, 128, 64, True, 2, 1, 1)])
 def test_attention_inside_the_step_is_the_one_behind_it(raw, dev, H, G, D, rot, normed, B, nsplit, slabs):
     """One launch for the step and the attention over the splits of the cached keys (up to four rows of one matrix) against the two: from
-    the first position, through rings that wrap, with parked sequences, without norms or rotations; the last three cases are the two
-    launches themselves."""
+    the first position, through rings that wrap, with parked sequences, without norms or rotations, norms of more columns than a block has
+    in one pass; more rows, two slabs, over a thousand blocks and one split are the two launches themselves."""
     f, cap, Hr, Nn, V = dict(dtype=torch.float32, device=dev), 150, 2, 64, 64
     g = torch.Generator().manual_seed(D + B)
     at = (H + 2 * G) * D
