@@ -823,10 +823,10 @@ void gemm_group_m(int g) { g_group_m = g; }
 // grp_rows > 0: grouped, that many rows in all groups
 // An fp32 output without bias, activation or residual is the one slab of an unsplit product: the kernels store a slab without the
 // choices of the general epilogue, which they make anew for each of a lane's elements.  us before / now: dY^T X 12288 x 4096 x 3200 282 / 250,
-// 4096 x 4096 x 640 37 / 33, 1000 x 72 x 320 4.9 / 4.3; x W^T 4096 x 4096 x 640 35 / 30, 1024 x 2048 x 256 6.2 / 5.9.
+// 4096 x 4096 x 640 37 / 33, 1000 x 72 x 320 4.9 / 4.3; x W^T 4096 x 4096 x 640 35 / 30, 1024 x 2048 x 256 6.2 / 5.9.  (A slab lies on 16 bytes.)
 static void output_as_slab(GemmParams& q) {
   if (!q.Cf || q.C || q.splitk > 1 || q.raw_partial || q.amax_val || q.glu_half || q.rope_cos || q.grp_start || q.bias || q.res ||
-      q.act != ACT_NONE || q.ldc != q.N)
+      q.act != ACT_NONE || q.ldc != q.N || (reinterpret_cast<uintptr_t>(q.Cf) & 15))
     return;
   q.partial = q.Cf;
   q.raw_partial = 1;
