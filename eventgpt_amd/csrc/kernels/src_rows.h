@@ -50,8 +50,13 @@ template <int M = SRC_ANY> __device__ __forceinline__ void src8(const SrcRows& s
 template <int M = SRC_ANY> __device__ __forceinline__ float src1(const SrcRows& s, long long row, int col) {
   if constexpr (M != SRC_ANY) {
     const float* p = static_cast<const float*>(s.p) + row * s.ld + col;
-    if constexpr (M == SRC_ONE) return p[0];
-    else return p[0] + p[s.slab] + p[2 * s.slab] + p[3 * s.slab];
+    float t[M], v;
+#pragma unroll
+    for (int k = 0; k < M; ++k) t[k] = p[k * s.slab];
+    v = t[0];
+#pragma unroll
+    for (int k = 1; k < M; ++k) v += t[k];
+    return v;
   }
   if (!s.f32) return bf16_to_f32(static_cast<const bf16_t*>(s.p)[row * s.ld + col]);
   const float* p = static_cast<const float*>(s.p) + row * s.ld + col;
