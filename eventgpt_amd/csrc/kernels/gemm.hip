@@ -204,7 +204,7 @@ template <int BM, int BN, int WGM, int WGN, int STAGES, bool AT = false, bool BT
           bool ROPE = false, bool GRP = false, int ACT = -1>
 __global__ __launch_bounds__(WGM * WGN * 64) void gemm_bf16_kernel(EVGPT_GEMM_ARGS) {
   EVGPT_GEMM_TAKE;
-  if constexpr (KT) p.k_cols = glu_half_, p.glu_half = 0;      // (launch_cfg: what the first loads need comes in registers)
+  if constexpr (KT) p.k_cols = cols_, p.glu_half = 0;          // (the first loads look at it)
   static_assert(!GRP || (!AT && !BT && !KT && !ROPE), "grouped products are plain ones");
   static_assert(!AT || BM == 64 || BM == 128, "K-strided A needs a 64- or 128-row tile");
   static_assert(!BT || BN == 64 || BN == 128, "K-strided W needs a 64- or 128-column tile");
@@ -972,10 +972,9 @@ static void launch_cfg(const GemmParams& p, hipStream_t st) {
   GemmParams q = p;
   q.group_m = g_group_m;
   output_as_slab(q);
-  if constexpr (KT) q.glu_half = q.k_cols;                     // (a gated product never takes these instances)
   q.split_major = (g_split_major && p.splitk > 1 && p.M > 32) ? 1 : 0;
   hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, WGM, WGN, STAGES, AT, BT, KT, ROPE, false, ACT>), dim3(tiles), dim3(WGM * WGN * 64),
-                     smem, st, EVGPT_GEMM_PASS(q));
+                     smem, st, EVGPT_GEMM_PASS_COLS(q, KT ? q.k_cols : q.glu_half));
 }
 
 // 256 x 256 tiles pay once there are rows to fill them and about half a round of tiles.  With the 8-wave kernel (measured on

@@ -64,12 +64,14 @@ struct GemmParams {
 
 // What a kernel needs for its first loads, as arguments of their own ahead of the other parameters: with kernel argument preload
 // (build.py) they are in scalar registers when a wave starts; a structure is fetched.  Vision tower, one frame, 1867 us without preload, 1830
-// with it where arguments were scalars already (norms, slab sums), 1800 with these.
+// with it where arguments were scalars already (norms, slab sums), 1800 with these.  cols_: the gated half, or -- instances with a short last K-tile, which
+// no gated product takes -- the rows' true columns.
 #define EVGPT_GEMM_ARGS                                                                                                              \
-  const bf16_t *a_, const bf16_t *w_, int m_, int n_, int k_, int lda_, int ldw_, int splitk_, int k_per_split_, int glu_half_, GemmParams p
+  const bf16_t *a_, const bf16_t *w_, int m_, int n_, int k_, int lda_, int ldw_, int splitk_, int k_per_split_, int cols_, GemmParams p
 #define EVGPT_GEMM_TAKE \
-  p.A = a_, p.W = w_, p.M = m_, p.N = n_, p.K = k_, p.lda = lda_, p.ldw = ldw_, p.splitk = splitk_, p.k_per_split = k_per_split_, p.glu_half = glu_half_
-#define EVGPT_GEMM_PASS(p) (p).A, (p).W, (p).M, (p).N, (p).K, (p).lda, (p).ldw, (p).splitk, (p).k_per_split, (p).glu_half, p
+  p.A = a_, p.W = w_, p.M = m_, p.N = n_, p.K = k_, p.lda = lda_, p.ldw = ldw_, p.splitk = splitk_, p.k_per_split = k_per_split_, p.glu_half = cols_
+#define EVGPT_GEMM_PASS_COLS(p, cols) (p).A, (p).W, (p).M, (p).N, (p).K, (p).lda, (p).ldw, (p).splitk, (p).k_per_split, cols, p
+#define EVGPT_GEMM_PASS(p) EVGPT_GEMM_PASS_COLS(p, (p).glu_half)
 
 // wait until at most `n` of this wave's direct-to-LDS loads are still in flight
 template <int N> __device__ __forceinline__ void wait_vm() {
