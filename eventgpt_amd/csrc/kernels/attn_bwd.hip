@@ -107,7 +107,8 @@ __device__ __forceinline__ void mma_tr(f32x4_t (&acc)[D / 16], const unsigned ch
 
 // st[n] = rows n*16.. of the LDS tile (A operand, ds_read_b128) times the register fragments; the k-step outermost, so that four
 // independent products follow each other (with it innermost every one waits for the one before: eight sequences of 836, 32
-// heads of 128, both kernels 475 us, now 446 with keys masked only in tiles that cross the diagonal or an end)
+// heads of 128, both kernels 475 us, now 446 with keys masked only in tiles that cross the diagonal or an end, and the
+// weights by v_exp_f32 as it is, which is 0 below 2^-126)
 template <int D>
 __device__ __forceinline__ void mma_rows(f32x4_t (&st)[4], const unsigned char* lds,
                                          const bf16x8_t (&bfrag)[D / 32], int fr, int g) {

@@ -9,7 +9,7 @@
 //     S^T[key][q] = K · Q^T        (K rows = MFMA A operand, Q^T = B operand)
 // so that the query index lives on the lane (lane & 15) and a lane's 16
 // accumulator values are 16 different keys of ONE query.  Consequences:
-//   * softmax row statistics are in-lane reductions + 2 cross-lane shuffles;
+//   * softmax row statistics are in-lane reductions + 2 lane swaps (maxima) or shuffles (sums);
 //   * the exponentiated tile, converted to bf16, already *is* the B operand of
 //     the second product  O^T[d][q] = V^T · P^T  — no LDS round trip for P
 //     (the contraction index is permuted consistently on both operands);
@@ -351,8 +351,8 @@ __global__ __launch_bounds__(256 * GROUPS) void attn_prefill_kernel(AttnParams p
 // feeds two MFMAs instead of one -- with 16 rows per wave the kernel above reads 32 KB of LDS
 // per wave and key tile for 32 MFMAs and is bound by the LDS pipe.  K / V tiles are staged
 // straight into LDS (buffer_load ... lds, swizzle applied to the per-lane source offset; keys past
-// the end come back as zeros from the descriptor's range check) into a two-tile ring: the loads
-// of tile t+1 are in flight while tile t is computed, and no staging registers are held.
+// the end come back as zeros from the descriptor's range check) into a ring of AW_STAGES tiles:
+// loads are in flight while other tiles are computed, and no staging registers are held.
 __device__ __forceinline__ void attn_buffer_to_lds16(const unsigned char* src, int bytes, unsigned char* lds, int voff) {
   const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(src), 0, bytes, 0x00020000);
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (void __attribute__((address_space(3)))*)lds, 16, voff, 0, 0, 0);
@@ -548,8 +548,9 @@ __global__ __launch_bounds__(AW_WAVES * 64) void attn_prefill_wide_kernel(AttnPa
   // k - 1 and S of tile k: tiles k - 1 to k + 1 are read, tile k + 2 is requested into the fourth stage, whose content, tile k - 2,
   // was last read before barrier k (every wave waits for its LDS reads there).  A tile has landed one barrier after its request:
   // every wave waits for its own part.  Tiles past the last one are requested too: zero fills of a stage nobody reads.
-  // (With a second barrier a tile, which closed S for one half and M for the other, 4643 tokens of 32 heads took 201 us instead
-  // of 196, eight sequences of 836 99 instead of 93: a wave that had a new maximum held up all of them.)
+  // (With a second barrier a tile, which closed S for one half and M for the other, 4643 tokens of 32 heads took 2 to 3 % longer, eight
+  // sequences of 836 6 %: a wave that had a new maximum held up all of them.  One call after another they take 201 and 99 us, were 233 and
+  // 116; inside a prompt 231.)
   auto landed = [&]() {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     fence();

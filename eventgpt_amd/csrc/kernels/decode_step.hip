@@ -196,7 +196,8 @@ __global__ __launch_bounds__(256) void parallel_step_kernel(StepHeads sh, StepMe
 // of the splits of its keys, which are on their way meanwhile; the new key and value, which the cache will only hold afterwards,
 // are made by the blocks of the first split and join there.  What is left of the attention is the merge of the splits.
 // Partial results as attn_decode_split_kernel leaves them.
-// A chat of one stream, width 2048, 100 + 64 tokens: 21.35 -> 20.9 ms (a launch of 4.1 us and its gap less in every second layer).
+// A chat of one stream, width 2048, 100 + 64 tokens: 21.35 -> 20.9 ms (a launch of 4.1 us and its gap less in every second layer); 20.6 with
+// the state's image picked by a select, 5.5 us a launch.
 template <int D, int M>
 __device__ __forceinline__ void attend_split(const AttnPrepArgs& a, const StepSplits& sp, int b, int h, int split, int p, bool live) {
   constexpr int LPK = D / 8, KPW = 64 / LPK, U = 4, NP = 4 * KPW;

@@ -820,7 +820,6 @@ static bool g_persist_256 = true;     // false: one workgroup per tile (A/B runs
 void gemm_persist_256(bool on) { g_persist_256 = on; }
 void gemm_group_m(int g) { g_group_m = g; }
 
-// grp_rows > 0: grouped, that many rows in all groups
 // An fp32 output without bias, activation or residual is the one slab of an unsplit product: the kernels store a slab without the
 // choices of the general epilogue, which they make anew for each of a lane's elements.  us before / now: dY^T X 12288 x 4096 x 3200 282 / 250,
 // 4096 x 4096 x 640 37 / 33, 1000 x 72 x 320 4.9 / 4.3; x W^T 4096 x 4096 x 640 35 / 30, 1024 x 2048 x 256 6.2 / 5.9.  (A slab lies on 16 bytes.)
@@ -832,6 +831,7 @@ static void output_as_slab(GemmParams& q) {
   q.raw_partial = 1;
 }
 
+// grp_rows > 0: grouped, that many rows in all groups
 template <bool AT, bool BT, int BM = 256, bool GRP = false>
 static void launch_256(const GemmParams& p, hipStream_t st, int grp_rows = 0) {
   const int bn_out = p.glu_half ? 128 : 256;

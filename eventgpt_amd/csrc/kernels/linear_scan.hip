@@ -45,11 +45,6 @@ __device__ __forceinline__ double wave_scan_max(double v) {
   }
   return v;
 }
-__device__ __forceinline__ double wave_max_f64(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
-  return v;
-}
 
 // Rows [row0, row0 + len) x 64 columns from col (nc of them exist) of a T matrix, zeros past them, as MFMA operands whose contraction
 // runs down the rows.  bf16: rows as they are, 16 bytes a store, read with the transposing read (chunks swizzled so that the eight rows of a

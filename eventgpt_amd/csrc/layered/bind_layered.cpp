@@ -552,6 +552,8 @@ std::tuple<Tensor, Tensor> step_heads(bool attend, double scale, int64_t nsplit,
   if (B > 0) evgpt::launch_parallel_step(sh, sm, pos.data_ptr<int>(), iptr(live), f32, (int)B, cur_stream());
   return {attn_chunk_decode(q, k_cache, v_cache, pos, scale, nsplit), o};
 }
+// the first of the two launches that attend_step_ makes where one does not take the call: ([B, Hq, D] queries, memory [B, H * V]); the decoders
+// go through attend_step_, this is for comparing with it
 std::tuple<Tensor, Tensor> parallel_step_(const Tensor& src, at::IntArrayRef attn, const OptTensor& qw, const OptTensor& kw,
                                           double eps, const Tensor& cos, const Tensor& sin, const Tensor& k_cache, const Tensor& v_cache,
                                           at::IntArrayRef mem, const Tensor& ib, const Tensor& fb, double cap, double qscale,
