@@ -258,11 +258,10 @@ void launch_event_voxel_ranges(const int* x, const int* y, const int* p, const i
 //   count  a block owns one (bin, band): it adds the runs of all chunks in LDS counters and writes both outputs whole
 // The chunk of a sorted stream lies in one or two bins, so the sort reads t at its two ends only; the unsorted one
 // reads it for every event.  Bound by memory: 12 B in, 2 B out, 2 B in per event (and 8 B for the span) plus 12 B out per
-// pixel and bin.  1e7 clustered events, 480 x 640, 5 bins by time on a sorted stream: span 16 us, sort 34, count 24; the
-// whole call 86 us (218 MB it cannot do without: 2.5 TB/s), 766 with voxel_lds_kernel below, which scans y once a band
+// pixel and bin.  1e7 clustered events, 480 x 640, 5 bins by time on a sorted stream: span 17 us, sort 31, count 19; the
+// whole call 79 us (218 MB it cannot do without: 2.8 TB/s), 766 with voxel_lds_kernel above, which scans y once a band
 // (506 us) behind host round trips for the extent and the order of t.
 constexpr int VS_THREADS = 512, VS_PER = 16, VS_CHUNK = VS_THREADS * VS_PER, VS_KEYS = 4096, VS_SPANS = 256;
-constexpr int VC_THREADS = 1024;
 
 struct VoxelSpan { long long lo, hi; long long unsorted; };
 
@@ -325,6 +324,14 @@ __global__ __launch_bounds__(VS_THREADS) void voxel_sort_kernel(VoxelArgs a) {
   __shared__ int unsorted_s;
   const int c0 = blockIdx.x * VS_CHUNK, tid = threadIdx.x;
   const int in_chunk = min(VS_CHUNK, a.n - c0);
+  // what the chunk's bins come from is requested ahead of the events: behind them it arrives behind them (34 -> 31 us)
+  VoxelSpan ext{};
+  long long t_end = 0;
+  if (!a.by_count) {
+    ext = a.span[tid & (VS_SPANS - 1)];
+    t_end = a.t[c0 + ((tid & 63) == 0 ? 0 : in_chunk - 1)];
+  }
+  asm volatile("" ::: "memory");
   int xv[VS_PER], yv[VS_PER], pv[VS_PER];
 #pragma unroll
   for (int e = 0; e < VS_PER; ++e) {
@@ -333,19 +340,18 @@ __global__ __launch_bounds__(VS_THREADS) void voxel_sort_kernel(VoxelArgs a) {
   }
   long long t0 = 0;
   double span = 1.0;
-  const auto bin_of = [&](int i) {
-    const int b = a.by_count ? static_cast<int>(static_cast<long long>(i) * a.bins / a.n)
-                             : static_cast<int>(static_cast<double>(a.t[i] - t0) / span * a.bins);
+  const auto bin_at = [&](long long t) {
+    const int b = static_cast<int>(static_cast<double>(t - t0) / span * a.bins);
     return b < 0 ? 0 : (b >= a.bins ? a.bins - 1 : b);
   };
+  const auto bin_of = [&](int i) { return a.by_count ? static_cast<int>(static_cast<long long>(i) * a.bins / a.n) : bin_at(a.t[i]); };
   bool unsorted = false;
   if (!a.by_count) {
     if (tid == 0) unsorted_s = 0;
     __syncthreads();
     if (tid < VS_SPANS) {
-      const VoxelSpan s = a.span[tid];
-      long long lo = s.lo, hi = s.hi;
-      if (s.unsorted) unsorted_s = 1;
+      long long lo = ext.lo, hi = ext.hi;
+      if (ext.unsorted) unsorted_s = 1;
 #pragma unroll
       for (int off = 32; off > 0; off >>= 1) {
         lo = min(lo, static_cast<long long>(__shfl_xor(lo, off, 64)));
@@ -360,7 +366,15 @@ __global__ __launch_bounds__(VS_THREADS) void voxel_sort_kernel(VoxelArgs a) {
     span = static_cast<double>(t1 > t0 ? t1 - t0 : 1);
     unsorted = unsorted_s != 0;
   }
-  const int b0 = unsorted ? 0 : bin_of(c0), b1 = unsorted ? a.bins - 1 : bin_of(c0 + in_chunk - 1);
+  int b0 = 0, b1 = a.bins - 1;
+  if (a.by_count) {
+    b0 = bin_of(c0);
+    b1 = bin_of(c0 + in_chunk - 1);
+  } else if (!unsorted) {
+    const int b = bin_at(t_end);
+    b0 = __builtin_amdgcn_readlane(b, 0);
+    b1 = __builtin_amdgcn_readlane(b, 63);
+  }
   const int keys = (b1 - b0 + 1) * a.bands, rows = 1 << a.log_rows;
   for (int k = tid; k < keys; k += VS_THREADS) cnt[k] = 0;
   __syncthreads();
@@ -419,48 +433,102 @@ __global__ __launch_bounds__(VS_THREADS) void voxel_sort_kernel(VoxelArgs a) {
   for (int i = tid; i * 8 < total; i += VS_THREADS) dst[i] = src[i];      // (the tail past `total` is never read)
 }
 
-__global__ __launch_bounds__(VC_THREADS) void voxel_count_kernel(VoxelArgs a, int* __restrict__ out_hist, float* __restrict__ out_vox,
-                                                                 int signed_mode) {
-  extern __shared__ int cnt[];                     // [2][rows][W]
-  __shared__ int2 runs[VC_THREADS];                // first record and length
-  __shared__ int n_runs;
-  const int band = blockIdx.x, b = blockIdx.y, rows = 1 << a.log_rows, tid = threadIdx.x;
+// Every wave takes its own share of the chunks, a lane a chunk and neighbouring chunks in different waves (a bin of a sorted stream is a
+// range of chunks), and has eight runs on their way, two records a load, before it counts the first: a run is some 70 records, and one
+// after another they were as many round trips (24 -> 19 us; 5e6 events, one bin of 203 x 301: 34 -> 32).  What is left is the LDS adds, half of their lanes empty; runs filled up to 16 bytes, a
+// lane a piece of one, took 2 us less here and cost the sort more.
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void voxel_count_kernel(VoxelArgs a, int* __restrict__ out_hist, float* __restrict__ out_vox,
+                                                              int signed_mode) {
+  constexpr int WAVES = THREADS / 64, PASSES = 4, RUNS = 8;
+  extern __shared__ __attribute__((aligned(16))) int cnt[];                     // [2][rows][W]
+  const int band = blockIdx.x, b = blockIdx.y, rows = 1 << a.log_rows, tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = rows * a.W;
-  for (int i = tid; i < 2 * half; i += VC_THREADS) cnt[i] = 0;
-  const int lane = tid & 63;
-  for (int base = 0; base < a.chunks; base += VC_THREADS) {
-    if (tid == 0) n_runs = 0;
-    __syncthreads();
-    const int c = base + tid;
-    if (c < a.chunks) {
-      const int2 r = a.range[c];
-      if (r.x <= b && b <= r.y) {
-        const unsigned short* off = a.off + static_cast<size_t>(c) * (a.keys + 1) + (b - r.x) * a.bands + band;
-        const int s = off[0], len = off[1] - s;
-        if (len > 0) runs[atomicAdd(&n_runs, 1)] = make_int2(c * VS_CHUNK + s, len);
+  for (int i = tid; i < 2 * half; i += THREADS) cnt[i] = 0;
+  __syncthreads();
+  const auto count = [&](unsigned int two, int at, int from, int to) {          // records `at`, `at` + 1 of a run that is from .. to
+    if (at >= from && at < to) atomicAdd(&cnt[two & 0xffff], 1);
+    if (at + 1 < to) atomicAdd(&cnt[two >> 16], 1);
+  };
+  const unsigned int* words = reinterpret_cast<const unsigned int*>(a.rec);
+  for (int base = 0; base < a.chunks; base += THREADS * PASSES) {
+    int start[PASSES], len[PASSES];
+    int2 r[PASSES];
+#pragma unroll
+    for (int s = 0; s < PASSES; ++s) {
+      const int c = base + s * THREADS + lane * WAVES + wid;
+      r[s] = c < a.chunks ? a.range[c] : make_int2(1, 0);
+    }
+#pragma unroll
+    for (int s = 0; s < PASSES; ++s) {
+      const int c = base + s * THREADS + lane * WAVES + wid;
+      start[s] = len[s] = 0;
+      if (r[s].x <= b && b <= r[s].y) {
+        const unsigned short* off = a.off + static_cast<size_t>(c) * (a.keys + 1) + (b - r[s].x) * a.bands + band;
+        start[s] = off[0];
+        len[s] = off[1];
       }
     }
-    __syncthreads();
-    const int n = n_runs;
-    for (int j = tid >> 6; j < n; j += VC_THREADS / 64) {
-      const int2 r = runs[j];
-      const unsigned short* rec = a.rec + r.x;
-      for (int i = lane; i < r.y; i += 256) {      // four loads of a run in flight
-        int v[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = i + u * 64 < r.y ? rec[i + u * 64] : -1;
+    for (int s = 0; s < PASSES; ++s) {
+      len[s] -= start[s];
+      start[s] = len[s] > 0 ? start[s] + (base + s * THREADS + lane * WAVES + wid) * VS_CHUNK : 0;      // (below 2^31: the events are)
+    }
+#pragma unroll 1
+    for (int s = 0; s < PASSES; ++s) {
+      const int at_s = s == 0 ? start[0] : s == 1 ? start[1] : s == 2 ? start[2] : start[3];
+      const int len_s = s == 0 ? len[0] : s == 1 ? len[1] : s == 2 ? len[2] : len[3];
+      unsigned long long todo = __builtin_amdgcn_ballot_w64(len_s > 0);
+      while (todo) {
+        int first[RUNS], odd[RUNS], end[RUNS];                                  // first word; the run among the words' records
+        unsigned int v[RUNS][2];
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-          if (v[u] >= 0) atomicAdd(&cnt[v[u]], 1);
+        for (int u = 0; u < RUNS; ++u) {                                        // (lanes past the run, and runs past the last, read a word twice)
+          const int l = __builtin_ctzll(todo | 1ull << 63);
+          const int at = __builtin_amdgcn_readlane(at_s, l), n = todo ? __builtin_amdgcn_readlane(len_s, l) : 0;
+          todo &= todo - 1;
+          first[u] = at >> 1;
+          odd[u] = at & 1;
+          end[u] = odd[u] + n;
+          const int last = max(end[u] - 1, 0) >> 1;
+          v[u][0] = words[first[u] + min(lane, last)];
+          v[u][1] = words[first[u] + min(64 + lane, last)];
+        }
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int u = 0; u < RUNS; ++u) {
+          count(v[u][0], lane * 2, odd[u], end[u]);
+          if (end[u] > 128) count(v[u][1], 128 + lane * 2, odd[u], end[u]);
+          for (int i = 256 + lane * 2; i < end[u]; i += 512) {                  // four loads of a long run in flight
+            unsigned int w[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) w[q] = words[first[u] + (min(i + q * 128, end[u] - 1) >> 1)];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) count(w[q], i + q * 128, odd[u], end[u]);
+          }
+        }
       }
     }
-    __syncthreads();
   }
+  __syncthreads();
   const int y0 = band << a.log_rows, cells = min(rows, a.H - y0) * a.W;
   const size_t plane = static_cast<size_t>(a.H) * a.W, at = static_cast<size_t>(y0) * a.W;
   int* hist = out_hist + static_cast<size_t>(b) * 2 * plane + at;
   float* vox = out_vox + static_cast<size_t>(b) * plane + at;
-  for (int i = tid; i < cells; i += VC_THREADS) {
+  if ((a.W & 3) == 0) {                            // (the outputs start on 16 bytes: they are allocated with the call)
+    for (int i = tid * 4; i < cells; i += THREADS * 4) {
+      const i32x4_t neg = *reinterpret_cast<const i32x4_t*>(cnt + i), pos = *reinterpret_cast<const i32x4_t*>(cnt + half + i);
+      *reinterpret_cast<i32x4_t*>(hist + i) = neg;
+      *reinterpret_cast<i32x4_t*>(hist + plane + i) = pos;
+      f32x4_t v;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = static_cast<float>(signed_mode ? pos[k] - neg[k] : pos[k] + neg[k]);
+      *reinterpret_cast<f32x4_t*>(vox + i) = v;
+    }
+    return;
+  }
+  for (int i = tid; i < cells; i += THREADS) {
     const int neg = cnt[i], pos = cnt[half + i];
     hist[i] = neg;
     hist[plane + i] = pos;
@@ -508,12 +576,19 @@ void launch_event_voxel_sorted(const int* x, const int* y, const int* p, const l
   if (!by_count) hipLaunchKernelGGL(voxel_span_kernel, dim3(VS_SPANS), dim3(1024), 0, st, t, n, span);
   hipLaunchKernelGGL(voxel_sort_kernel, dim3(plan.chunks), dim3(VS_THREADS), 0, st, a);
   const size_t smem = static_cast<size_t>(2) * (1 << plan.log_rows) * W * sizeof(int);
-  static bool attr_set = false;
-  if (!attr_set) {
-    hipFuncSetAttribute(reinterpret_cast<const void*>(&voxel_count_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024);  // (W = 19 200; the runs take 8 KB)
-    attr_set = true;
-  }
-  hipLaunchKernelGGL(voxel_count_kernel, dim3(plan.bands, bins), dim3(VC_THREADS), smem, st, a, out_hist, out_vox, signed_mode);
+  const auto count = [&](auto kernel, int threads) {
+    static bool attr_set = false;                       // (one a kernel)
+    if (!attr_set) {
+      hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024);  // (W = 19 200)
+      attr_set = true;
+    }
+    hipLaunchKernelGGL(kernel, dim3(plan.bands, bins), dim3(threads), smem, st, a, out_hist, out_vox, signed_mode);
+  };
+  // two blocks a CU and more of few events each: half as many threads, so that all are resident at once (600 blocks, 1e6 events 31.4 ->
+  // 28.6 us, 2.4e6 40.2 -> 38.8); with more the block of the busiest band is
+  // waited for, and its waves count (1e7 77.7 with 512 threads, 75.6 with 1 024; 4.3e6 0.98 to 1.03 of the time with 512)
+  if (plan.bands * bins >= 512 && n / (plan.bands * bins) < 5000) count(&voxel_count_kernel<512>, 512);
+  else count(&voxel_count_kernel<1024>, 1024);
 }
 
 // --------------------------------------------------------- CLIP preprocessing

@@ -108,6 +108,20 @@ def test_voxel_counts_over_more_chunks_than_one_pass_lists(dev, order):
     assert int(h.sum()) == n and torch.equal(h, h_at) and torch.equal(v, v_at)
 
 
+# events per chunk of the busiest band from under one load of a wave to a whole chunk; blocks of 1 024 threads (fewer than 512 blocks, or 5 000
+# events each) and of 512; one pass over the chunks (4 096 and 2 048 of them) and a second one
+@pytest.mark.parametrize("bins,n,spread", [(3, 20_000, 97), (3, 300_000, 40), (3, 300_000, 1), (6, 300_000, 12), (6, 300_000, 1),
+                                           (6, 3_000_000, 97), (900, 2048 * 8192 + 3, 97), (3, 4096 * 8192 + 3, 97)])
+def test_voxel_counts_runs_of_any_length(dev, bins, n, spread):
+    from eventgpt_amd.ops import event_ops as eo
+    hw, g = (97, 130), torch.Generator(device=dev).manual_seed(n + spread)
+    def ints(hi):
+        return torch.randint(0, hi, (n,), generator=g, device=dev, dtype=torch.int32)
+    d = {"x": ints(hw[1]), "y": ints(spread) + (hw[0] - spread) // 2, "p": ints(2), "t": torch.arange(n, device=dev)}
+    (h, v), (h_at, v_at) = (eo.voxel_grid_gpu(d, bins, hw, privatised=private) for private in (True, False))
+    assert int(h.sum()) == n and torch.equal(h, h_at) and torch.equal(v, v_at)
+
+
 @pytest.mark.parametrize("hw", [(480, 640), (120, 160), (336, 336), (400, 300)])
 def test_clip_preprocess_matches_host(dev, hw):
     from eventgpt_amd.ops import event_ops as eo
