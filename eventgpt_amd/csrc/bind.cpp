@@ -1174,9 +1174,13 @@ bool linear_qkv_rope(const Tensor& x, const Tensor& w_qkv, const Tensor& q_out, 
   TORCH_CHECK(q_out.numel() == S * Hq * 128 && k_cache.size(1) == Hkv && v_cache.sizes() == k_cache.sizes() &&
               pos0.numel() >= 1 && cos.size(-1) == 64 && sin.size(-1) == 64 && cos.size(0) >= k_cache.size(2) &&
               sin.size(0) >= k_cache.size(2), "linear_qkv_rope: shapes");
+  const int64_t ws = evgpt::gemm_tail_ws_floats((int)S, (int)w_qkv.size(0), (int)K);
+  Tensor slabs;
+  if (ws > 0) slabs = at::empty({ws}, cos.options());
   return evgpt::launch_gemm_qkv_rope(bptr(x), bptr(w_qkv), (int)S, (int)K, bptr_mut(q_out), bptr_mut(k_cache),
                                      bptr_mut(v_cache), cos.data_ptr<float>(), sin.data_ptr<float>(),
-                                     pos0.data_ptr<int>(), (int)Hq, (int)Hkv, (int)k_cache.size(2), cur_stream());
+                                     pos0.data_ptr<int>(), (int)Hq, (int)Hkv, (int)k_cache.size(2),
+                                     ws > 0 ? slabs.data_ptr<float>() : nullptr, cur_stream());
 }
 
 // Row argmax of (x @ w^T + bias) without materialising the product: the GEMM

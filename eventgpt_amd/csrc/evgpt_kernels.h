@@ -115,7 +115,7 @@ bool gemm_few_glu_serves(int rows, int I, int K);
 void launch_gemm_few_glu(const bf16_t* A, const bf16_t* W, bf16_t* C, int rows, int I, int K, int glu_act, hipStream_t st);
 bool launch_gemm_qkv_rope(const bf16_t* A, const bf16_t* W, int M, int K, bf16_t* q_out, bf16_t* k_cache,
                           bf16_t* v_cache, const float* cos_tab, const float* sin_tab, const int* pos0, int Hq,
-                          int Hkv, int l_max, hipStream_t st);
+                          int Hkv, int l_max, float* splitk_ws, hipStream_t st);
 int gemm_splitk_slabs(int M, int N, int K);   // K splits of launch_gemm_partial (slabs summed by the caller)
 int gemm_splitk_t(int M, int N, int K);   // K splits for launch_gemm_bf16_t (1 = none)
 void launch_gemm_bf16_t(const bf16_t* A, const bf16_t* W, bf16_t* C, float* Cf, const bf16_t* bias,

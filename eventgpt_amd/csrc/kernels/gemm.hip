@@ -150,7 +150,7 @@ __device__ __forceinline__ void gemm_rope_epilogue(const GemmParams& p, f32x4_t 
                                                    int m0, int n0, int wid, int lane) {
   static_assert(TM == 4 && TN == 4, "128 x 128 tile, 2 x 2 waves");
   const int wr = wid >> 1, wc = wid & 1, frow = lane & 15, fq = lane >> 4;
-  const int head = n0 >> 7;
+  const int head = (n0 >> 7) + p.rope_head0;
   const bool is_v = head >= p.rope_hq + p.rope_hkv;
   float* xch = reinterpret_cast<float*>(smem);        // [4 waves][64 values][64 lanes]
   __syncthreads();                                    // every wave is done with the operand tiles
@@ -899,7 +899,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmParams p) {
 // division and one store.  (Element by element the four 64-bit divisions and the loads one after another were the time: 4643 x 768 and x 1024 columns
 // of four slabs -- 60 MB -- 15.6 us, now 12.7; with the product in front, 577 x 1024 x 4096
 // in three 16.8 / 15.4, 300 x 16 x 4096 10.8 / 7.6, 20 x 4096 x 4096 11.9 / 10.1.)  S: the slabs, 0: any number, four at a time.
-template <int S>
+// V: the columns are v heads of a q | k | v projection, stored in the cache.
+template <int S, bool V = false>
 __global__ __launch_bounds__(256) void splitk_reduce_quads_kernel(GemmParams p) {
   const unsigned cols = static_cast<unsigned>(p.N) >> 2, quads = static_cast<unsigned>(p.M) * cols;
   const size_t slab = static_cast<size_t>(p.M) * p.N;
@@ -936,6 +937,13 @@ __global__ __launch_bounds__(256) void splitk_reduce_quads_kernel(GemmParams p) 
     if (p.res) {
       const u32x2_t w = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
       v = f32x4_t{bf16lo(w[0]) + bf16lo(rw[0]), bf16hi(w[0]) + bf16hi(rw[0]), bf16lo(w[1]) + bf16lo(rw[1]), bf16hi(w[1]) + bf16hi(rw[1])};
+    }
+    if constexpr (V) {
+      const int pos = (p.rope_pos0 ? p.rope_pos0[0] : 0) + static_cast<int>(m);
+      if (pos >= 0 && pos < p.rope_lmax)
+        *reinterpret_cast<u32x2_t*>(p.rope_v + ((static_cast<size_t>(n >> 7) + p.rope_head0 - p.rope_hq - p.rope_hkv) * p.rope_lmax + pos) * 128 + (n & 127)) =
+            u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+      continue;
     }
     if (p.Cf) *reinterpret_cast<f32x4_t*>(p.Cf + o) = v;
     if (p.C) *reinterpret_cast<u32x2_t*>(p.C + o) = u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
@@ -1294,13 +1302,41 @@ void launch_gemm_bf16(const bf16_t* A, const bf16_t* W, bf16_t* C, float* Cf, co
 // pos0[0] + row.  Returns false (nothing launched) for shapes the fused tile does not take.
 bool launch_gemm_qkv_rope(const bf16_t* A, const bf16_t* W, int M, int K, bf16_t* q_out, bf16_t* k_cache,
                           bf16_t* v_cache, const float* cos_tab, const float* sin_tab, const int* pos0, int Hq,
-                          int Hkv, int l_max, hipStream_t st) {
+                          int Hkv, int l_max, float* splitk_ws, hipStream_t st) {
   const int N = (Hq + 2 * Hkv) * 128;
   if (K % 64 || M < 1 || g_forced_cfg >= 0) return false;
   GemmParams p{A, W, nullptr, nullptr, nullptr, nullptr, M, N, K, K, K, N, ACT_NONE, nullptr, nullptr, 1, K,
                nullptr, 0, K, K};
   p.rope_q = q_out; p.rope_k = k_cache; p.rope_v = v_cache; p.rope_cos = cos_tab; p.rope_sin = sin_tab;
   p.rope_pos0 = pos0; p.rope_hq = Hq; p.rope_hkv = Hkv; p.rope_lmax = l_max;
+  // 256 x 256 tiles where the plain product takes them (of the four-wave kernel; the other one has no such epilogue).  7B prompt of 800 /
+  // 900 / 1024 tokens on 128 x 128 tiles 14.30 / 14.82 / 15.53 ms, so 12.71 / 13.26 / 13.82; longer ones had a pass of their own for the rotation
+  GemmParams tail = p;
+  int n1 = 0, tail_s = 0;
+  const bool two = last_round_split(M, N, K, &n1, &tail_s);
+  if (use_256(M, N, K) && gemm_quad_serves(p) && gemm_quad_ahead(p, static_cast<int>(cfg_tiles(CFG_256x256, M, two ? n1 : N))) &&
+      (!two || (n1 >> 7) >= Hq + Hkv)) {
+    if (two) {                  // the columns past the whole rounds, v heads all of them: as launch_gemm_bf16
+      p.N = n1;
+      tail.N = N - n1;
+      tail.W = W + static_cast<size_t>(n1) * K;
+      tail.rope_head0 = n1 >> 7;
+    }
+    launch_256<false, false>(p, st);
+    if (two && tail_s >= 2 && splitk_ws) {
+      tail.k_per_split = ((K / 64 + tail_s - 1) / tail_s) * 64;
+      tail.splitk = (K + tail.k_per_split - 1) / tail.k_per_split;
+      tail.partial = splitk_ws;
+      launch_256<false, false>(tail, st);
+      const long long blocks = (static_cast<long long>(M) * (tail.N / 4) + 255) / 256;
+      const dim3 grid(static_cast<unsigned>(blocks > 2048 ? 2048 : blocks));
+      if (tail.splitk == 3) hipLaunchKernelGGL((splitk_reduce_quads_kernel<3, true>), grid, dim3(256), 0, st, tail);
+      else hipLaunchKernelGGL((splitk_reduce_quads_kernel<0, true>), grid, dim3(256), 0, st, tail);
+    } else if (two) {
+      launch_cfg<128, 128, 2, 2, 2, false, false, false, true>(tail, st);
+    }
+    return true;
+  }
   launch_cfg<128, 128, 2, 2, 2, false, false, false, true>(p, st);
   return true;
 }

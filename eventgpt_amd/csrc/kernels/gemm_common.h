@@ -49,6 +49,7 @@ struct GemmParams {
   const float* rope_cos; const float* rope_sin;     // [l_max][64]
   const int* rope_pos0;
   int rope_hq, rope_hkv, rope_lmax;
+  int rope_head0;      // the head of the output's first column (the last heads of a projection are a launch of their own)
   // row tiles per group of the tile walk (0: whole columns); set by the launchers
   int group_m;
   int rows_epilogue;   // 8-wave kernel: bf16 output stored as whole lines through LDS (set by launch_256)

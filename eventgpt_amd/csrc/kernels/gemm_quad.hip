@@ -58,7 +58,12 @@ __device__ __forceinline__ f32x4_t take(const f32x4_t& a) {
   return f32x4_t{x, y, z, w};
 }
 
-// ACT: activation of a plain output (a constant: 256 run-time choices among the functions are 300 KB of instructions)
+// ACT: activation of a plain output (a constant: 256 run-time choices among the functions are 300 KB of instructions), or ROPE: a q | k | v
+// projection whose heads of 128 columns are rotated and go to their places in q and the cache (gemm_rope_epilogue's rules and rounding).
+// A wave's columns are one head and both halves of a pair are its own lane's, so the rotation costs the tables' values, from L2 and 16 rows
+// ahead, and no exchange.  As a pass of its own over the packed rows it took 40 us a layer at 4643 rows (228 MB).  7B prompt, ms, so / now:
+// 4643 tokens 57.9 / 57.1 (the card's power limit takes back half of it), 3000 36.1 / 35.2, 2115 27.8 / 27.4, 1300 20.96 / 20.57.
+constexpr int ROPE = -2;
 template <bool GRP, int ACT>
 __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(GemmParams p) {
   constexpr int BM = 256, BN = 256;
@@ -219,7 +224,7 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(GemmParams p) {
     const int M = cur.rows;
     bf16_t* C = p.C + (GRP ? static_cast<size_t>(cur.first) * p.ldc : 0);
     unsigned char* rows = smem + 2 * STAGE + wid * SCRATCH;
-    if (!GRP && (p.splitk > 1 || p.raw_partial || p.Cf)) {
+    if (!GRP && ACT != ROPE && (p.splitk > 1 || p.raw_partial || p.Cf)) {
       const bool whole = p.splitk == 1 && !p.raw_partial;              // the fp32 output itself
       float* slab = whole ? p.Cf : p.partial + static_cast<size_t>(cur.ksplit) * p.M * p.N;
       const size_t ld = whole ? p.ldc : p.N;
@@ -232,6 +237,64 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(GemmParams p) {
           if (m < M && n < p.N) *reinterpret_cast<f32x4_t*>(slab + m * ld + n) = take(acc[i][j]);
         }
       }
+    } else if constexpr (ACT == ROPE) {
+      const int head = (cur.n0 >> 7) + wc + p.rope_head0, pos0 = p.rope_pos0 ? p.rope_pos0[0] : 0;
+      const bool to_cache = head >= p.rope_hq, is_v = head >= p.rope_hq + p.rope_hkv, inside = cur.n0 + wc * 128 < p.N;
+      // the head's rows: of q, one after another by token; of k and v by position
+      bf16_t* dst = !to_cache ? p.rope_q + head * 128
+                              : (is_v ? p.rope_v : p.rope_k) + static_cast<size_t>(head - p.rope_hq - (is_v ? p.rope_hkv : 0)) * p.rope_lmax * 128;
+      const int ld = to_cache ? 128 : p.rope_hq * 128, most = to_cache ? p.rope_lmax : M;
+      const auto heads = [&](auto rotated) {      // (one head a wave)
+        constexpr bool TURN = decltype(rotated)::value;
+        f32x4_t cs[2][4], sn[2][4];        // the tables of 16 rows, and of the next 16 on their way
+        const auto request = [&](int i) {
+          const int pos = min(max(pos0 + min(cur.m0 + wr * 128 + i * 16 + frow, M - 1), 0), p.rope_lmax - 1);
+          const unsigned int at = static_cast<unsigned int>(pos) * 256 + fq * 16;      // (rope_lmax * 256 is below 2^32: gemm_quad_serves)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            cs[i & 1][j] = *reinterpret_cast<const f32x4_t*>(reinterpret_cast<const char*>(p.rope_cos) + at + j * 64);
+            sn[i & 1][j] = *reinterpret_cast<const f32x4_t*>(reinterpret_cast<const char*>(p.rope_sin) + at + j * 64);
+          }
+        };
+        if constexpr (TURN) request(0);
+        each<4>([&](auto pc) {
+          constexpr int pass = decltype(pc)::value;
+          each<2>([&](auto ic) {
+            constexpr int il = decltype(ic)::value, i = pass * 2 + il;
+            if constexpr (TURN && i < 7) request(i + 1);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              f32x4_t a = take(acc[i][j]), b = take(acc[i][j + 4]);
+              if constexpr (TURN) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {          // (sums rounded as rope_kv_prefill_kernel's)
+                  const float x = bf16_to_f32(f32_to_bf16(a[r])), y = bf16_to_f32(f32_to_bf16(b[r])), c = cs[i & 1][j][r], t = sn[i & 1][j][r];
+                  a[r] = fmaf(c, x, -(t * y));
+                  b[r] = fmaf(c, y, t * x);
+                }
+              }
+#pragma unroll
+              for (int h = 0; h < 2; ++h) {
+                const f32x4_t v = h ? b : a;
+                const u32x2_t w = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+                const int chunk = ((j + h * 4) * 2 + (fq >> 1)) ^ frow;
+                *reinterpret_cast<u32x2_t*>(rows + (il * 16 + frow) * 256 + chunk * 16 + (fq & 1) * 8) = w;
+              }
+            }
+          });
+          asm volatile("" ::: "memory");
+#pragma unroll
+          for (int q = 0; q < 8; ++q) {
+            const int r = q * 4 + (lane >> 4), c = lane & 15;
+            const u32x4_t d = *reinterpret_cast<const u32x4_t*>(rows + r * 256 + ((c ^ (r & 15)) << 4));
+            const int m = cur.m0 + wr * 128 + pass * 32 + r, row = to_cache ? pos0 + m : m;
+            if (m < M && inside && row >= 0 && row < most) *reinterpret_cast<u32x4_t*>(dst + static_cast<long long>(row) * ld + c * 8) = d;
+          }
+          asm volatile("" ::: "memory");
+        });
+      };
+      if (is_v) heads(std::false_type{});
+      else heads(std::true_type{});
     } else if (ACT == ACT_NONE && p.glu_half) {
       each<4>([&](auto pc) {
         constexpr int pass = decltype(pc)::value;
@@ -282,7 +345,7 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(GemmParams p) {
             const f32x4_t o = take(acc[pass * 2 + il][j]);
             float v[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] = ACT == ACT_NONE ? o[r] + b[r] : apply_act(o[r] + b[r], ACT);
+            for (int r = 0; r < 4; ++r) v[r] = ACT <= ACT_NONE ? o[r] + b[r] : apply_act(o[r] + b[r], ACT);
             const u32x2_t w = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
             const int chunk = (j * 2 + (fq >> 1)) ^ frow;
             *reinterpret_cast<u32x2_t*>(rows + (il * 16 + frow) * 256 + chunk * 16 + (fq & 1) * 8) = w;
@@ -327,10 +390,13 @@ bool gemm_quad_serves(const GemmParams& p) {
   const long long lim = 1ll << 31;
   const int tail = p.K % p.k_per_split;
   if (p.k_per_split < 2 * BK || (tail && tail < 2 * BK)) return false;
-  if (p.k_cols || p.amax_val || p.rope_cos) return false;
+  if (p.k_cols || p.amax_val) return false;
   if (2ll * 256 * p.lda >= lim || 2ll * (p.glu_half ? 2ll * p.glu_half : 256) * p.ldw >= lim) return false;
   if (p.grp_start && (2ll * p.M * p.lda >= lim || p.res || p.bias || p.act != ACT_NONE)) return false;
   if (p.splitk > 1 || p.raw_partial) return !p.glu_half && p.partial && p.N % 4 == 0;
+  if (p.rope_cos)
+    return !p.grp_start && p.rope_lmax < (1 << 24) && ((reinterpret_cast<uintptr_t>(p.rope_q) | reinterpret_cast<uintptr_t>(p.rope_k) | reinterpret_cast<uintptr_t>(p.rope_v) |
+                             reinterpret_cast<uintptr_t>(p.rope_cos) | reinterpret_cast<uintptr_t>(p.rope_sin)) & 15) == 0;
   if (p.Cf)
     return !p.C && !p.grp_start && !p.glu_half && !p.bias && !p.res && p.act == ACT_NONE && p.N % 4 == 0 && p.ldc % 4 == 0 &&
            (reinterpret_cast<uintptr_t>(p.Cf) & 15) == 0;
@@ -357,7 +423,8 @@ bool gemm_quad_ahead(const GemmParams& p, int tiles) {
 }
 
 void launch_gemm_quad(const GemmParams& p, int grid, hipStream_t st) {
-  if (p.grp_start) launch<true>(p, grid, st);
+  if (p.rope_cos && p.splitk == 1) launch<false, ROPE>(p, grid, st);
+  else if (p.grp_start) launch<true>(p, grid, st);
   else if (p.splitk > 1 || p.raw_partial || p.Cf || p.act == ACT_NONE) launch<false>(p, grid, st);
   else if (p.act == ACT_GELU) launch<false, ACT_GELU>(p, grid, st);
   else launch<false, ACT_QUICK_GELU>(p, grid, st);

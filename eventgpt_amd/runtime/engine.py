@@ -702,11 +702,16 @@ class GenerationEngine(DecodeEngine):
         kv_len = pos0 + S
         q = torch.empty(1, S, self.Hq, self.D, dtype=torch.bfloat16, device=self.device)
         o = torch.empty_like(q)
+        # rotation and cache append in the projection's epilogue, as in _forward_rows_prompt
+        rope_gemm = self.D == 128 and S > self.prompt_fused_rows
         for l in self.layers:
             kc, vc = l.k_cache[batch:batch + 1], l.v_cache[batch:batch + 1]
             xn = raw.rmsnorm(x, l.norm1, self.eps)
-            qkv = raw.linear(xn, self._w(l, "w_qkv"), None, None, 0, False)
-            raw.prefill_rope_kv(qkv, q, kc, vc, self.cos, self.sin, pos0, self.Hq, self.Hkv, self.D)
+            if not (rope_gemm and raw.linear_qkv_rope(xn, self._w(l, "w_qkv"), q, kc, vc, self.cos, self.sin, pos0,
+                                                      self.Hq, self.Hkv)):
+                rope_gemm = False
+                qkv = raw.linear(xn, self._w(l, "w_qkv"), None, None, 0, False)
+                raw.prefill_rope_kv(qkv, q, kc, vc, self.cos, self.sin, pos0, self.Hq, self.Hkv, self.D)
             raw.attention_cache(q, kc, vc, o, kv_len, self.scale)
             x = raw.linear(o.view(1, S, self.Hq * self.D), self._w(l, "w_o"), None, x, 0, False)
             xn = raw.rmsnorm(x, l.norm2, self.eps)

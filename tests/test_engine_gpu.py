@@ -470,8 +470,13 @@ def test_long_prompt_prefill_and_decode(dev):
         eng.prefill(torch.zeros(3073, 256, dtype=torch.bfloat16, device=dev), start=0)
 
 
+# the last seven on 256 x 256 tiles: one round, a column tile that is half there, rows past the cache, the columns past the whole rounds on
+# 128 x 128 tiles, in four and in three splits, and (one k head: not all of them v) back on 128 x 128 tiles
 @pytest.mark.parametrize("S,Hq,Hkv,K,p0,l_max", [(636, 32, 32, 4096, 0, 1024), (77, 4, 4, 512, 5, 80),
-                                                  (300, 8, 2, 1024, 17, 512), (129, 4, 1, 512, 40, 160)])
+                                                  (300, 8, 2, 1024, 17, 512), (129, 4, 1, 512, 40, 160),
+                                                  (1100, 32, 32, 640, 0, 1200), (2000, 33, 1, 1024, 9, 2400), (1025, 32, 32, 1024, 40, 1040),
+                                                  (1301, 32, 32, 1024, 3, 1400), (1300, 32, 32, 4096, 0, 1400), (1601, 32, 32, 4096, 50, 1640),
+                                                  (4000, 32, 1, 1024, 0, 4000)])
 def test_qkv_gemm_with_rope_epilogue_equals_gemm_then_rope(dev, S, Hq, Hkv, K, p0, l_max):
     """The q | k | v GEMM whose epilogue rotates and appends to the cache writes exactly what the plain
     GEMM followed by the RoPE / append kernel writes (same bf16 rounding points), including rows that
