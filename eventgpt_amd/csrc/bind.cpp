@@ -459,7 +459,7 @@ Tensor row_stats(const Tensor& a, const Tensor& b) {
               a.sizes() == b.sizes() && a.scalar_type() == b.scalar_type(),
               "row_stats: two contiguous GPU tensors of one shape and dtype");
   const int64_t H = a.size(-1), rows = H ? a.numel() / H : 0;
-  Tensor s = at::zeros({rows, 4}, a.options().dtype(at::kFloat));
+  Tensor s = at::empty({rows, 4}, a.options().dtype(at::kFloat));
   if (rows == 0) return s;
   if (a.scalar_type() == at::kFloat) {
     TORCH_CHECK(H % 4 == 0, "row_stats: row length must be a multiple of 4 (fp32)");
@@ -475,18 +475,39 @@ Tensor row_stats(const Tensor& a, const Tensor& b) {
   return s;
 }
 
-// grad[r] = A_r (p_r - t_r) + B_r t_r + C_r p_r with coef [rows, 3] fp32
-Tensor row_affine_grad(const Tensor& p, const Tensor& t, const Tensor& coef) {
-  check_f32(coef, "coef");
+// (masked MSE, masked mean cosine, weight of the valid rows) from row_stats' sums; mask fp32 [rows]
+std::tuple<Tensor, Tensor, Tensor> row_pair_loss(const Tensor& stats, const c10::optional<Tensor>& mask, int64_t H) {
+  check_f32(stats, "stats");
+  const int64_t rows = stats.size(0);
+  TORCH_CHECK(stats.dim() == 2 && stats.size(1) == 4 && H >= 1, "row_pair_loss: stats [rows, 4]");
+  if (mask.has_value()) { check_f32(*mask, "mask"); TORCH_CHECK(mask->numel() == rows, "row_pair_loss: a weight a row"); }
+  auto one = [&] { return at::empty({}, stats.options()); };
+  Tensor mse = one(), cos = one(), n = one();
+  evgpt::launch_row_pair_loss(stats.data_ptr<float>(), mask.has_value() ? mask->data_ptr<float>() : nullptr, rows, (int)H,
+                              mse.data_ptr<float>(), cos.data_ptr<float>(), n.data_ptr<float>(), cur_stream());
+  return {mse, cos, n};
+}
+
+// d (g_mse mse + g_cos cos) / d p of row_pair_loss; g_mse, g_cos: fp32 scalars on the device, absent for zero
+Tensor row_pair_grad(const Tensor& p, const Tensor& t, const Tensor& stats, const c10::optional<Tensor>& mask, const Tensor& n_valid,
+                     const c10::optional<Tensor>& g_mse, const c10::optional<Tensor>& g_cos) {
+  check_f32(stats, "stats"); check_f32(n_valid, "n_valid");
   TORCH_CHECK(p.is_cuda() && t.is_cuda() && p.is_contiguous() && t.is_contiguous() && p.sizes() == t.sizes() &&
-              p.scalar_type() == t.scalar_type(), "row_affine_grad: two contiguous GPU tensors of one shape and dtype");
+              p.scalar_type() == t.scalar_type(), "row_pair_grad: two contiguous GPU tensors of one shape and dtype");
   const int64_t H = p.size(-1), rows = H ? p.numel() / H : 0;
   const bool bf = p.scalar_type() == at::kBFloat16;
-  TORCH_CHECK(bf || p.scalar_type() == at::kFloat, "row_affine_grad: float32 or bfloat16 only");
-  TORCH_CHECK(H % (bf ? 8 : 4) == 0 && coef.numel() == rows * 3, "row_affine_grad: row length / coefficient count");
+  TORCH_CHECK(bf || p.scalar_type() == at::kFloat, "row_pair_grad: float32 or bfloat16 only");
+  TORCH_CHECK(H % (bf ? 8 : 4) == 0 && stats.numel() == rows * 4 && n_valid.numel() == 1, "row_pair_grad: row length, sums");
+  auto scalar = [](const c10::optional<Tensor>& s, int64_t n, const char* what) -> const float* {
+    if (!s.has_value()) return nullptr;
+    check_f32(*s, what);
+    TORCH_CHECK(s->numel() == n, "row_pair_grad: ", what);
+    return s->data_ptr<float>();
+  };
   Tensor g = at::empty_like(p);
-  if (rows) evgpt::launch_row_affine_grad(p.data_ptr(), t.data_ptr(), coef.data_ptr<float>(), g.data_ptr(), rows, (int)H, bf,
-                                          cur_stream());
+  if (rows)
+    evgpt::launch_row_pair_grad(p.data_ptr(), t.data_ptr(), stats.data_ptr<float>(), scalar(mask, rows, "mask"), n_valid.data_ptr<float>(),
+                                scalar(g_mse, 1, "g_mse"), scalar(g_cos, 1, "g_cos"), g.data_ptr(), rows, (int)H, bf, cur_stream());
   return g;
 }
 
@@ -897,17 +918,8 @@ Tensor swiglu_bwd(const Tensor& gate_up, const Tensor& gh) {
   return dgu;
 }
 
-// One optimizer shard: grad/param_out in the parameters' storage type (bf16 or fp32), fp32
-// master weights and moments, all of the same length; updates master, moments and param_out.
-void fused_adamw(const Tensor& grad, const Tensor& master, const Tensor& exp_avg, const Tensor& exp_avg_sq,
-                 const Tensor& param_out, double lr, double beta1, double beta2, double eps,
-                 double weight_decay, int64_t step, double clip, const c10::optional<Tensor>& clip_dev) {
-  check_f32(master, "master"); check_f32(exp_avg, "exp_avg"); check_f32(exp_avg_sq, "exp_avg_sq");
-  const int64_t n = master.numel();
-  TORCH_CHECK(grad.is_cuda() && grad.is_contiguous() && param_out.is_cuda() && param_out.is_contiguous() &&
-              grad.numel() == n && param_out.numel() == n && exp_avg.numel() == n && exp_avg_sq.numel() == n,
-              "fused_adamw: all tensors are contiguous device tensors of one length");
-  TORCH_CHECK(grad.scalar_type() == param_out.scalar_type() && step >= 1, "fused_adamw: dtype/step");
+static evgpt::AdamWArgs adamw_args(double lr, double beta1, double beta2, double eps, double weight_decay, int64_t step, double clip,
+                                   const c10::optional<Tensor>& clip_dev) {
   evgpt::AdamWArgs a;
   a.clip_dev = nullptr;
   if (clip_dev.has_value()) {
@@ -919,6 +931,26 @@ void fused_adamw(const Tensor& grad, const Tensor& master, const Tensor& exp_avg
   a.decay = (float)(1.0 - lr * weight_decay);
   a.step_size = (float)(lr / (1.0 - std::pow(beta1, (double)step)));
   a.inv_sqrt_bc2 = (float)(1.0 / std::sqrt(1.0 - std::pow(beta2, (double)step)));
+  return a;
+}
+static void check_adamw(const Tensor& grad, const Tensor& master, const Tensor& exp_avg, const Tensor& exp_avg_sq, const Tensor& param_out) {
+  check_f32(master, "master"); check_f32(exp_avg, "exp_avg"); check_f32(exp_avg_sq, "exp_avg_sq");
+  const int64_t n = master.numel();
+  TORCH_CHECK(grad.is_cuda() && grad.is_contiguous() && param_out.is_cuda() && param_out.is_contiguous() &&
+              grad.numel() == n && param_out.numel() == n && exp_avg.numel() == n && exp_avg_sq.numel() == n,
+              "fused_adamw: all tensors are contiguous device tensors of one length");
+  TORCH_CHECK(grad.scalar_type() == param_out.scalar_type(), "fused_adamw: dtype");
+}
+
+// One optimizer shard: grad/param_out in the parameters' storage type (bf16 or fp32), fp32
+// master weights and moments, all of the same length; updates master, moments and param_out.
+void fused_adamw(const Tensor& grad, const Tensor& master, const Tensor& exp_avg, const Tensor& exp_avg_sq,
+                 const Tensor& param_out, double lr, double beta1, double beta2, double eps,
+                 double weight_decay, int64_t step, double clip, const c10::optional<Tensor>& clip_dev) {
+  check_adamw(grad, master, exp_avg, exp_avg_sq, param_out);
+  TORCH_CHECK(step >= 1, "fused_adamw: step");
+  const int64_t n = master.numel();
+  const evgpt::AdamWArgs a = adamw_args(lr, beta1, beta2, eps, weight_decay, step, clip, clip_dev);
   if (grad.scalar_type() == at::kBFloat16)
     evgpt::launch_fused_adamw_bf16(bptr(grad), master.data_ptr<float>(), exp_avg.data_ptr<float>(),
                                    exp_avg_sq.data_ptr<float>(), bptr_mut(param_out), n, a, cur_stream());
@@ -927,6 +959,54 @@ void fused_adamw(const Tensor& grad, const Tensor& master, const Tensor& exp_avg
                                   exp_avg_sq.data_ptr<float>(), param_out.data_ptr<float>(), n, a, cur_stream());
   else
     TORCH_CHECK(false, "fused_adamw: bfloat16 or float32 parameters");
+}
+
+// Several shards (of one type) in one launch; every tensor starts on 16 bytes.
+void fused_adamw_many(at::TensorList grads, at::TensorList masters, at::TensorList exp_avgs, at::TensorList exp_avg_sqs,
+                      at::TensorList params_out, double lr, double beta1, double beta2, double eps, double weight_decay, int64_t step,
+                      const c10::optional<Tensor>& clip_dev) {
+  const size_t n = grads.size();
+  TORCH_CHECK(n >= 1 && masters.size() == n && exp_avgs.size() == n && exp_avg_sqs.size() == n && params_out.size() == n && step >= 1,
+              "fused_adamw_many: lists of one length");
+  evgpt::AdamWArgs a = adamw_args(lr, beta1, beta2, eps, weight_decay, step, 1.0, clip_dev);
+  const auto type = grads[0].scalar_type();
+  TORCH_CHECK(type == at::kBFloat16 || type == at::kFloat, "fused_adamw_many: bfloat16 or float32 parameters");
+  std::vector<evgpt::AdamWShard> shards(n);
+  for (size_t i = 0; i < n; ++i) {
+    check_adamw(grads[i], masters[i], exp_avgs[i], exp_avg_sqs[i], params_out[i]);
+    TORCH_CHECK(grads[i].scalar_type() == type, "fused_adamw_many: shards of one type");
+    shards[i] = {grads[i].data_ptr(), masters[i].data_ptr<float>(), exp_avgs[i].data_ptr<float>(), exp_avg_sqs[i].data_ptr<float>(),
+                 params_out[i].data_ptr(), (long long)masters[i].numel()};
+    const uintptr_t all = reinterpret_cast<uintptr_t>(shards[i].grad) | reinterpret_cast<uintptr_t>(shards[i].master) |
+                          reinterpret_cast<uintptr_t>(shards[i].m) | reinterpret_cast<uintptr_t>(shards[i].v) | reinterpret_cast<uintptr_t>(shards[i].out);
+    TORCH_CHECK(all % 16 == 0, "fused_adamw_many: 16-byte aligned shards");
+  }
+  evgpt::launch_fused_adamw_many(shards.data(), (int)n, type == at::kBFloat16, a, cur_stream());
+}
+
+// sum of squares of all of the tensors together (bf16 or fp32, on 16 bytes), [1], deterministic
+Tensor sumsq_many(at::TensorList xs) {
+  TORCH_CHECK(xs.size() >= 1, "sumsq_many: at least one tensor");
+  std::vector<evgpt::SumsqShard> shards;
+  for (const Tensor& x : xs) {
+    TORCH_CHECK(x.is_cuda() && x.is_contiguous() && (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kFloat) &&
+                    reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0,
+                "sumsq_many: contiguous bf16 / fp32 device tensors on 16 bytes");
+    shards.push_back({x.data_ptr(), (long long)x.numel(), x.scalar_type() == at::kBFloat16});
+  }
+  const auto f32 = xs[0].options().dtype(at::kFloat);
+  Tensor part = at::empty({evgpt::sumsq_many_blocks(shards.data(), (int)shards.size())}, f32), out = at::empty({1}, f32);
+  evgpt::launch_sumsq_many(shards.data(), (int)shards.size(), part.data_ptr<float>(), out.data_ptr<float>(), cur_stream());
+  return out;
+}
+
+// (norm, clip factor [1]) of a squared gradient norm on the device: min(1, max_norm / (norm + 1e-6))
+std::tuple<Tensor, Tensor> clip_factor(const Tensor& sq, double max_norm) {
+  check_f32(sq, "sq");
+  TORCH_CHECK(sq.numel() == 1, "clip_factor: one value");
+  Tensor norm = at::empty({}, sq.options()), clip = at::empty({1}, sq.options());
+  evgpt::launch_clip_factor(sq.data_ptr<float>(), (float)max_norm, norm.data_ptr<float>(), clip.data_ptr<float>(), cur_stream());
+  return {norm, clip};
 }
 
 // acc[0] += sum(x^2) over a contiguous bf16 / fp32 device tensor (16-byte aligned), deterministic
@@ -1565,7 +1645,8 @@ TORCH_LIBRARY(evgpt, m) {
   m.def("argmax_rows(Tensor x) -> Tensor", &argmax_rows);
   m.def("row_metrics(Tensor a, Tensor b, float eps) -> (Tensor, Tensor)", &row_metrics);
   m.def("row_stats(Tensor a, Tensor b) -> Tensor", &row_stats);
-  m.def("row_affine_grad(Tensor p, Tensor t, Tensor coef) -> Tensor", &row_affine_grad);
+  m.def("row_pair_loss(Tensor stats, Tensor? mask, int H) -> (Tensor, Tensor, Tensor)", &row_pair_loss);
+  m.def("row_pair_grad(Tensor p, Tensor t, Tensor stats, Tensor? mask, Tensor n_valid, Tensor? g_mse, Tensor? g_cos) -> Tensor", &row_pair_grad);
   m.def("decode_qkv(Tensor x, Tensor norm_w, Tensor w_qkv, Tensor(a!) q_out, Tensor(b!) k_cache, Tensor(c!) v_cache, Tensor cos, Tensor sin, Tensor pos, float eps, int Hq, int Hkv, int D, bool one_seq=False) -> ()", &decode_qkv);
   m.def("decode_attn(Tensor q, Tensor k_cache, Tensor v_cache, Tensor(a!) out, Tensor(b!) part_o, Tensor(c!) part_ml, Tensor pos, int nsplit, float scale) -> ()", &decode_attn);
   m.def("decode_gemv_residual(Tensor w, Tensor xin, Tensor(a!) y) -> ()", &decode_gemv_residual);
@@ -1584,6 +1665,9 @@ TORCH_LIBRARY(evgpt, m) {
   m.def("layernorm_bwd(Tensor x, Tensor weight, Tensor grad, float eps, bool want_params=True) -> (Tensor, Tensor, Tensor)", &layernorm_bwd);
   m.def("column_sum(Tensor g, bool out_f32=False) -> Tensor", &column_sum);
   m.def("sumsq_accumulate(Tensor x, Tensor(a!) acc) -> ()", &sumsq_accumulate);
+  m.def("sumsq_many(Tensor[] xs) -> Tensor", &sumsq_many);
+  m.def("clip_factor(Tensor sq, float max_norm) -> (Tensor, Tensor)", &clip_factor);
+  m.def("fused_adamw_many(Tensor[] grads, Tensor(a!)[] masters, Tensor(b!)[] exp_avgs, Tensor(c!)[] exp_avg_sqs, Tensor(d!)[] params_out, float lr, float beta1, float beta2, float eps, float weight_decay, int step, Tensor? clip_dev=None) -> ()", &fused_adamw_many);
   m.def("fused_adamw(Tensor grad, Tensor(a!) master, Tensor(b!) exp_avg, Tensor(c!) exp_avg_sq, Tensor(d!) param_out, float lr, float beta1, float beta2, float eps, float weight_decay, int step, float clip, Tensor? clip_dev=None) -> ()", &fused_adamw);
   m.def("w4_dequant(Tensor packed, Tensor absmax, Tensor code, Tensor(a!)? out=None) -> Tensor", &w4_dequant);
   m.def("gemv_w4_max_batch() -> int", []() { return (int64_t)evgpt::gemv_w4_max_batch(); });

@@ -88,6 +88,12 @@ void launch_fused_adamw_bf16(const bf16_t* grad, float* master, float* m, float*
 void launch_fused_adamw_f32(const float* grad, float* master, float* m, float* v, float* out, long long n,
                             const AdamWArgs& a, hipStream_t st);
 
+struct AdamWShard { const void* grad; float* master; float* m; float* v; void* out; long long n; };
+void launch_fused_adamw_many(const AdamWShard* shards, int count, bool bf16, const AdamWArgs& a, hipStream_t st);
+struct SumsqShard { const void* x; long long n; bool bf16; };
+long long sumsq_many_blocks(const SumsqShard* shards, int count);      // floats of `part`
+void launch_sumsq_many(const SumsqShard* shards, int count, float* part, float* out, hipStream_t st);
+void launch_clip_factor(const float* sq, float max_norm, float* norm, float* clip, hipStream_t st);
 int sumsq_blocks(long long n);
 void launch_sumsq(const void* x, bool bf16, long long n, float* part, float* acc, hipStream_t st);
 
@@ -226,8 +232,9 @@ void launch_row_metrics_f32(const float* a, const float* b, float* cos_out, floa
                             long long rows, int H, float eps, hipStream_t st, float* stats = nullptr);
 void launch_row_metrics_bf16(const bf16_t* a, const bf16_t* b, float* cos_out, float* mse_out,
                              long long rows, int H, float eps, hipStream_t st, float* stats = nullptr);
-void launch_row_affine_grad(const void* p, const void* t, const float* coef, void* grad, long long rows, int H,
-                            bool bf16, hipStream_t st);
+void launch_row_pair_loss(const float* stats, const float* mask, long long rows, int H, float* mse, float* cos, float* n_valid, hipStream_t st);
+void launch_row_pair_grad(const void* p, const void* t, const float* stats, const float* mask, const float* n_valid, const float* g_mse,
+                          const float* g_cos, void* grad, long long rows, int H, bool bf16, hipStream_t st);
 bool launch_reduce_residual_layernorm(const float* partial, int nslab, int M, int N, const bf16_t* bias,
                                       const bf16_t* res, bf16_t* x_out, const bf16_t* ln_w, const bf16_t* ln_b,
                                       bf16_t* y_out, float eps, hipStream_t st);

@@ -44,14 +44,13 @@ __global__ __launch_bounds__(256) void fused_adamw_kernel(const T* __restrict__ 
   }
 }
 
-// 8 elements per thread with 16-byte accesses (all pointers 16-byte aligned, n % 8 == 0)
+// 8 elements per thread with 16-byte accesses (all pointers 16-byte aligned); block `block` of the shard's `blocks`
 template <typename T>
-__global__ __launch_bounds__(256) void fused_adamw_vec_kernel(const T* __restrict__ grad, float* __restrict__ master,
-                                                              float* __restrict__ m, float* __restrict__ v,
-                                                              T* __restrict__ param_out, long long n8, AdamWArgs a) {
-  if (a.clip_dev) a.clip *= *a.clip_dev;
-  const long long stride = static_cast<long long>(gridDim.x) * blockDim.x;
-  for (long long c = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; c < n8; c += stride) {
+__device__ __forceinline__ void adamw_vec(const T* __restrict__ grad, float* __restrict__ master, float* __restrict__ m,
+                                          float* __restrict__ v, T* __restrict__ param_out, long long n8, const AdamWArgs& a, int block,
+                                          int blocks) {
+  const long long stride = static_cast<long long>(blocks) * 256;
+  for (long long c = static_cast<long long>(block) * 256 + threadIdx.x; c < n8; c += stride) {
     float g[8], mm[8], vv[8], w[8];
     if constexpr (sizeof(T) == 2) {
       const u32x4_t gv = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(grad) + c);
@@ -94,6 +93,37 @@ __global__ __launch_bounds__(256) void fused_adamw_vec_kernel(const T* __restric
   }
 }
 
+template <typename T>
+__global__ __launch_bounds__(256) void fused_adamw_vec_kernel(const T* __restrict__ grad, float* __restrict__ master,
+                                                              float* __restrict__ m, float* __restrict__ v,
+                                                              T* __restrict__ param_out, long long n8, AdamWArgs a) {
+  if (a.clip_dev) a.clip *= *a.clip_dev;
+  adamw_vec(grad, master, m, v, param_out, n8, a, blockIdx.x, gridDim.x);
+}
+
+// All shards of a step: a small one (biases, a scalar) is a launch of 4 to 5 us by itself and a few blocks here.
+constexpr int MANY = 32;
+struct AdamWTable { AdamWShard s[MANY]; int first[MANY + 1]; };      // a shard's blocks: first[i] .. first[i + 1]
+
+template <typename T>
+__global__ __launch_bounds__(256) void fused_adamw_many_kernel(AdamWTable t, AdamWArgs a) {
+  if (a.clip_dev) a.clip *= *a.clip_dev;
+  int i = 0;
+  while (static_cast<int>(blockIdx.x) >= t.first[i + 1]) ++i;
+  const AdamWShard& s = t.s[i];
+  const int block = blockIdx.x - t.first[i];
+  const T* grad = static_cast<const T*>(s.grad);
+  T* out = static_cast<T*>(s.out);
+  adamw_vec(grad, s.master, s.m, s.v, out, s.n / 8, a, block, t.first[i + 1] - t.first[i]);
+  const long long e = s.n / 8 * 8 + threadIdx.x;
+  if (block == 0 && e < s.n) {
+    float mi = s.m[e], vi = s.v[e];
+    const float w = adamw_one(ld_as_f32(grad + e), mi, vi, s.master[e], a);
+    s.m[e] = mi; s.v[e] = vi; s.master[e] = w;
+    st_from_f32(out + e, w);
+  }
+}
+
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 template <typename T>
@@ -123,14 +153,28 @@ void launch_fused_adamw_f32(const float* grad, float* master, float* m, float* v
   launch_t<float>(grad, master, m, v, out, n, a, st);
 }
 
+void launch_fused_adamw_many(const AdamWShard* shards, int count, bool bf16, const AdamWArgs& a, hipStream_t st) {
+  for (int at = 0; at < count; at += MANY) {
+    AdamWTable t{};
+    const int n = count - at < MANY ? count - at : MANY;
+    for (int i = 0; i < n; ++i) {
+      t.s[i] = shards[at + i];
+      const long long want = (t.s[i].n / 8 + 255) / 256;
+      t.first[i + 1] = t.first[i] + static_cast<int>(want > 8192 ? 8192 : (want < 1 && t.s[i].n > 0 ? 1 : want));
+    }
+    if (t.first[n] == 0) continue;
+    if (bf16) hipLaunchKernelGGL(fused_adamw_many_kernel<bf16_t>, dim3(t.first[n]), dim3(256), 0, st, t, a);
+    else hipLaunchKernelGGL(fused_adamw_many_kernel<float>, dim3(t.first[n]), dim3(256), 0, st, t, a);
+  }
+}
+
 // ---- sum of squares of a gradient shard (global-norm clipping), two deterministic stages:
 // `blocks` partial sums, then one block adds them to acc[0] (fp32; accumulates across buckets).
 template <typename T>
-__global__ __launch_bounds__(256) void sumsq_partial_kernel(const T* __restrict__ x, long long n, float* __restrict__ part) {
-  __shared__ float red[4];
+__device__ __forceinline__ float sumsq_block(const T* __restrict__ x, long long n, int block, int blocks, float* red) {
   float s = 0.f;
-  const long long stride = static_cast<long long>(gridDim.x) * 256 * 8;
-  for (long long i0 = (static_cast<long long>(blockIdx.x) * 256 + threadIdx.x) * 8; i0 < n; i0 += stride) {
+  const long long stride = static_cast<long long>(blocks) * 256 * 8;
+  for (long long i0 = (static_cast<long long>(block) * 256 + threadIdx.x) * 8; i0 < n; i0 += stride) {
     if (i0 + 8 <= n) {
       if constexpr (sizeof(T) == 2) {
         const u32x4_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(x + i0));
@@ -147,8 +191,37 @@ __global__ __launch_bounds__(256) void sumsq_partial_kernel(const T* __restrict_
       for (long long i = i0; i < n; ++i) { const float a = ld_as_f32(x + i); s += a * a; }
     }
   }
-  s = block_sum(s, red);
+  return block_sum(s, red);
+}
+template <typename T>
+__global__ __launch_bounds__(256) void sumsq_partial_kernel(const T* __restrict__ x, long long n, float* __restrict__ part) {
+  __shared__ float red[4];
+  const float s = sumsq_block(x, n, blockIdx.x, gridDim.x, red);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
+}
+
+// Every shard of a gradient: two launches in all instead of two a shard, each 4 to 5 us at the least.
+struct SumsqTable { const void* x[MANY]; long long n[MANY]; int first[MANY + 1]; unsigned int bf16; };
+__global__ __launch_bounds__(256) void sumsq_many_kernel(SumsqTable t, float* __restrict__ part) {
+  __shared__ float red[4];
+  int i = 0;
+  while (static_cast<int>(blockIdx.x) >= t.first[i + 1]) ++i;
+  const int block = blockIdx.x - t.first[i], blocks = t.first[i + 1] - t.first[i];
+  const float s = t.bf16 >> i & 1 ? sumsq_block(static_cast<const bf16_t*>(t.x[i]), t.n[i], block, blocks, red)
+                                  : sumsq_block(static_cast<const float*>(t.x[i]), t.n[i], block, blocks, red);
+  if (threadIdx.x == 0) part[blockIdx.x] = s;
+}
+__global__ __launch_bounds__(1024) void sumsq_many_final_kernel(const float* __restrict__ part, long long n, float* __restrict__ out) {
+  __shared__ float red[16];
+  float s = 0.f;
+  for (long long i = threadIdx.x; i < n; i += 1024) s += part[i];
+  s = block_sum<16>(s, red);
+  if (threadIdx.x == 0) out[0] = s;
+}
+__global__ void clip_factor_kernel(const float* __restrict__ sq, float max_norm, float* __restrict__ norm, float* __restrict__ clip) {
+  const float n = sqrtf(*sq), c = max_norm / (n + 1e-6f);
+  *norm = n;
+  *clip = c > 1.f ? 1.f : c;             // (not a number stays that)
 }
 
 __global__ __launch_bounds__(256) void sumsq_final_kernel(const float* __restrict__ part, int n, float* __restrict__ acc) {
@@ -169,6 +242,30 @@ void launch_sumsq(const void* x, bool bf16, long long n, float* part, float* acc
   if (bf16) hipLaunchKernelGGL(sumsq_partial_kernel<bf16_t>, dim3(blocks), dim3(256), 0, st, static_cast<const bf16_t*>(x), n, part);
   else hipLaunchKernelGGL(sumsq_partial_kernel<float>, dim3(blocks), dim3(256), 0, st, static_cast<const float*>(x), n, part);
   hipLaunchKernelGGL(sumsq_final_kernel, dim3(1), dim3(256), 0, st, part, blocks, acc);
+}
+
+long long sumsq_many_blocks(const SumsqShard* shards, int count) {
+  long long n = 0;
+  for (int i = 0; i < count; ++i) n += sumsq_blocks(shards[i].n);
+  return n;
+}
+void launch_sumsq_many(const SumsqShard* shards, int count, float* part, float* out, hipStream_t st) {
+  long long done = 0;
+  for (int at = 0; at < count; at += MANY) {
+    SumsqTable t{};
+    const int n = count - at < MANY ? count - at : MANY;
+    for (int i = 0; i < n; ++i) {
+      t.x[i] = shards[at + i].x; t.n[i] = shards[at + i].n;
+      t.bf16 |= static_cast<unsigned int>(shards[at + i].bf16) << i;
+      t.first[i + 1] = t.first[i] + sumsq_blocks(t.n[i]);
+    }
+    hipLaunchKernelGGL(sumsq_many_kernel, dim3(t.first[n]), dim3(256), 0, st, t, part + done);
+    done += t.first[n];
+  }
+  hipLaunchKernelGGL(sumsq_many_final_kernel, dim3(1), dim3(1024), 0, st, part, done, out);
+}
+void launch_clip_factor(const float* sq, float max_norm, float* norm, float* clip, hipStream_t st) {
+  hipLaunchKernelGGL(clip_factor_kernel, dim3(1), dim3(1), 0, st, sq, max_norm, norm, clip);
 }
 
 }  // namespace evgpt

@@ -306,20 +306,51 @@ __global__ __launch_bounds__(256) void row_metrics_kernel(const T* __restrict__ 
   }
 }
 
-// Gradient of a loss that is a function of the per-row sums above (masked MSE + cosine):
-//   grad[r][i] = A_r (p_i - t_i) + B_r t_i + C_r p_i,   coef[r] = {A_r, B_r, C_r}
-// in one pass over the pair (autograd through normalise / multiply / reduce writes and re-reads
-// a dozen full-size temporaries).
+// The alignment loss from those sums, rows by their weight m (1 without a mask): out = {sum se m / (n H), sum cos m / n, n}, n = sum m, at
+// least 1.  One block: a row is 16 bytes, and as tensor expressions the same was 17 launches, and 17 for the coefficients below.
+constexpr float ROW_PAIR_EPS = 1e-12f;      // F.normalize's clamp on the norms (a NaN stays one)
+__device__ __forceinline__ float at_least(float x, float low) { return x < low ? low : x; }
+
+__global__ __launch_bounds__(1024) void row_pair_loss_kernel(const float* __restrict__ stats, const float* __restrict__ mask,
+                                                             long long rows, int H, float* __restrict__ mse, float* __restrict__ cos,
+                                                             float* __restrict__ n_valid) {
+  __shared__ float scratch[16];
+  float se = 0.f, co = 0.f, n = 0.f;
+  for (long long r = threadIdx.x; r < rows; r += 1024) {
+    const f32x4_t s = *reinterpret_cast<const f32x4_t*>(stats + r * 4);
+    const float m = mask ? mask[r] : 1.f;
+    se += s[3] * m;
+    co += s[0] / (at_least(sqrtf(s[1]), ROW_PAIR_EPS) * at_least(sqrtf(s[2]), ROW_PAIR_EPS)) * m;
+    n += m;
+  }
+  se = block_sum<16>(se, scratch);
+  co = block_sum<16>(co, scratch);
+  n = at_least(block_sum<16>(n, scratch), 1.f);
+  if (threadIdx.x == 0) {
+    *mse = se / (n * static_cast<float>(H));
+    *cos = co / n;
+    *n_valid = n;
+  }
+}
+
+// Its gradient: grad[r][i] = A (p_i - t_i) + B t_i + C p_i with A, B, C of the row's sums and weight, in one pass over the pair (autograd
+// through normalise / multiply / reduce writes and re-reads a dozen full-size temporaries).  g_mse, g_cos: null for zero.
 template <typename T>
-__global__ __launch_bounds__(256) void row_affine_grad_kernel(const T* __restrict__ p, const T* __restrict__ t,
-                                                              const float* __restrict__ coef, T* __restrict__ grad,
-                                                              long long rows, int H) {
+__global__ __launch_bounds__(256) void row_pair_grad_kernel(const T* __restrict__ p, const T* __restrict__ t, const float* __restrict__ stats,
+                                                            const float* __restrict__ mask, const float* __restrict__ n_valid,
+                                                            const float* __restrict__ g_mse, const float* __restrict__ g_cos,
+                                                            T* __restrict__ grad, long long rows, int H) {
   constexpr int EPV = 16 / sizeof(T);
   const int cpr = H / EPV;
   const long long total = rows * cpr;
+  const float gm = g_mse ? *g_mse * 2.f : 0.f, gc = g_cos ? *g_cos : 0.f, inv_n = 1.f / *n_valid;
   for (long long idx = blockIdx.x * 256ll + threadIdx.x; idx < total; idx += gridDim.x * 256ll) {
     const long long r = idx / cpr;
-    const float A = coef[r * 3], B = coef[r * 3 + 1], C = coef[r * 3 + 2];
+    const f32x4_t s = *reinterpret_cast<const f32x4_t*>(stats + r * 4);
+    const float w = (mask ? mask[r] : 1.f) * inv_n;
+    const float pn = at_least(sqrtf(s[1]), ROW_PAIR_EPS), both = pn * at_least(sqrtf(s[2]), ROW_PAIR_EPS);
+    // d mse / d p = 2 (p - t) m / (n H),  d cos / d p = t / (|p||t|) - cos p / |p|^2
+    const float A = gm * w / static_cast<float>(H), B = gc * w / both, C = -gc * w * (s[0] / both) / (pn * pn);
     if constexpr (sizeof(T) == 4) {
       const f32x4_t vp = reinterpret_cast<const f32x4_t*>(p)[idx], vt = reinterpret_cast<const f32x4_t*>(t)[idx];
       f32x4_t g;
@@ -339,18 +370,20 @@ __global__ __launch_bounds__(256) void row_affine_grad_kernel(const T* __restric
   }
 }
 
-void launch_row_affine_grad(const void* p, const void* t, const float* coef, void* grad, long long rows, int H,
-                            bool bf16, hipStream_t st) {
+void launch_row_pair_loss(const float* stats, const float* mask, long long rows, int H, float* mse, float* cos, float* n_valid, hipStream_t st) {
+  hipLaunchKernelGGL(row_pair_loss_kernel, dim3(1), dim3(1024), 0, st, stats, mask, rows, H, mse, cos, n_valid);
+}
+void launch_row_pair_grad(const void* p, const void* t, const float* stats, const float* mask, const float* n_valid, const float* g_mse,
+                          const float* g_cos, void* grad, long long rows, int H, bool bf16, hipStream_t st) {
   const long long total = rows * (H / (bf16 ? 8 : 4));
-  int blocks = static_cast<int>((total + 255) / 256);
-  if (blocks > 4096) blocks = 4096;
+  int blocks = static_cast<int>((total + 255) / 256 > 4096 ? 4096 : (total + 255) / 256);
   if (blocks < 1) return;
   if (bf16)
-    hipLaunchKernelGGL(row_affine_grad_kernel<bf16_t>, dim3(blocks), dim3(256), 0, st, static_cast<const bf16_t*>(p),
-                       static_cast<const bf16_t*>(t), coef, static_cast<bf16_t*>(grad), rows, H);
+    hipLaunchKernelGGL(row_pair_grad_kernel<bf16_t>, dim3(blocks), dim3(256), 0, st, static_cast<const bf16_t*>(p),
+                       static_cast<const bf16_t*>(t), stats, mask, n_valid, g_mse, g_cos, static_cast<bf16_t*>(grad), rows, H);
   else
-    hipLaunchKernelGGL(row_affine_grad_kernel<float>, dim3(blocks), dim3(256), 0, st, static_cast<const float*>(p),
-                       static_cast<const float*>(t), coef, static_cast<float*>(grad), rows, H);
+    hipLaunchKernelGGL(row_pair_grad_kernel<float>, dim3(blocks), dim3(256), 0, st, static_cast<const float*>(p),
+                       static_cast<const float*>(t), stats, mask, n_valid, g_mse, g_cos, static_cast<float*>(grad), rows, H);
 }
 
 void launch_row_metrics_f32(const float* a, const float* b, float* cos_out, float* mse_out,

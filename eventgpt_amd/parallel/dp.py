@@ -239,16 +239,15 @@ class ShardedAdamW:
         ranks).  Stays on the device with RCCL; a gloo group gets host tensors only."""
         dev = self.buckets[0].grad_shard.device
         if dev.type == "cuda":
-            # one streaming pass per bucket (csrc/kernels/optim.hip), accumulated on the device
+            # one streaming pass over all buckets (csrc/kernels/optim.hip)
             from ..ops import hip
-            acc = torch.zeros(1, dtype=torch.float32, device=dev)
-            for b in self.buckets:
-                g = b.grad_shard
-                if g.dtype in (torch.bfloat16, torch.float32) and g.data_ptr() % 16 == 0:
-                    hip.raw.sumsq_accumulate(g, acc)
-                else:
-                    acc += torch.linalg.vector_norm(g, dtype=torch.float32).square()
-            sq = acc[0]
+            shards = [b.grad_shard for b in self.buckets]
+            taken = [g for g in shards if g.dtype in (torch.bfloat16, torch.float32) and g.data_ptr() % 16 == 0]
+            sq = hip.raw.sumsq_many(taken)[0] if taken else torch.zeros((), dtype=torch.float32, device=dev)
+            if len(taken) < len(shards):
+                for g in shards:
+                    if not any(g is t for t in taken):
+                        sq = sq + torch.linalg.vector_norm(g, dtype=torch.float32).square()
         else:
             sq = torch.zeros((), dtype=torch.float32, device=dev)
             for b in self.buckets:
@@ -289,18 +288,25 @@ class ShardedAdamW:
         computed and consumed on the device (the fused AdamW kernel reads it), so a step on
         RCCL makes no host round trip unless the caller converts the norm (``float(norm)``)."""
         self._finish_reduces()
-        norm = self._global_sq_norm().sqrt()
-        clip_t = None
-        if max_grad_norm is not None:
-            clip_t = (max_grad_norm / (norm + 1e-6)).clamp(max=1.0).reshape(1)
+        sq, clip_t = self._global_sq_norm(), None
+        if max_grad_norm is not None and sq.is_cuda:
+            from ..ops import hip
+            norm, clip_t = hip.raw.clip_factor(sq, float(max_grad_norm))
+        else:
+            norm = sq.sqrt()
+            if max_grad_norm is not None:
+                clip_t = (max_grad_norm / (norm + 1e-6)).clamp(max=1.0).reshape(1)
         self.step_count += 1
         lr = self.param_groups[0]["lr"]
         b1, b2 = self.betas
         bc1 = 1 - b1 ** self.step_count
         bc2 = 1 - b2 ** self.step_count
         gather = self.distributed and self.world > 1
-        for b in self.buckets:
+        done = self._adamw_together(lr, clip_t) if not gather else ()
+        for i, b in enumerate(self.buckets):
             b.work = None
+            if i in done:
+                continue
             if b.master.is_cuda and b.flat_param.dtype in (torch.bfloat16, torch.float32):
                 # one pass over the shard (csrc/kernels/optim.hip) instead of ten launches
                 from ..ops import hip
@@ -330,6 +336,23 @@ class ShardedAdamW:
         if self.comm_stream is not None and gather:
             torch.cuda.current_stream().wait_stream(self.comm_stream)
         return norm
+
+    def _adamw_together(self, lr: float, clip_t: Optional[torch.Tensor]) -> set:
+        """The update of every bucket whose shard is refreshed in place, one launch a type.  Returns their indices."""
+        done = set()
+        for dtype in (torch.float32, torch.bfloat16):
+            new = {i: b.flat_param[b.shard_slice] for i, b in enumerate(self.buckets)
+                   if b.master.is_cuda and b.flat_param.dtype == dtype}
+            new = {i: t for i, t in new.items() if t.data_ptr() % 16 == 0 and self.buckets[i].grad_shard.data_ptr() % 16 == 0}
+            if not new:
+                continue
+            from ..ops import hip
+            some = [self.buckets[i] for i in new]
+            hip.raw.fused_adamw_many([b.grad_shard for b in some], [b.master for b in some], [b.exp_avg for b in some],
+                                     [b.exp_avg_sq for b in some], list(new.values()), lr, *self.betas, self.eps,
+                                     self.weight_decay, self.step_count, clip_t)
+            done.update(new)
+        return done
 
     # ------------------------------------------------------------- checkpointing
     def state_dict(self) -> dict:

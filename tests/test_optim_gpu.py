@@ -117,6 +117,64 @@ def test_sumsq_accumulate(dtype, n):
     assert abs(float(acc) - want) < 1e-4 * want
 
 
+# lengths about the 8 elements of a thread and the 2 048 of a block, and more shards than a launch's table holds
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("lengths", [[1], [7, 8, 9, 2047, 2048, 2049], [4099, 0, 70_000], list(range(1, 71))])
+def test_shards_of_a_step_in_one_launch(dtype, lengths):
+    """The update of every shard is the one a launch of its own makes: bit for bit in whole vectors; shards with a remainder have a
+    launch whose sums are contracted in another order, a rounding or two of the largest value.  The sum of squares is their sum."""
+    from eventgpt_amd.ops import hip
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(len(lengths))
+    def rows(scale, kind=torch.float32):
+        return [(torch.randn(n, device=dev, generator=g) * scale).to(kind) for n in lengths]
+    grads, master, m, v = rows(0.01, dtype), rows(0.05), rows(1e-3), [t.abs() for t in rows(1e-5)]
+    out, clip = rows(0.0, dtype), torch.tensor([0.7], device=dev)
+    alone = [[t.clone() for t in ts] for ts in (master, m, v, out)]
+    for gr, *state in zip(grads, *alone):
+        hip.raw.fused_adamw(gr, *state, 1e-2, 0.9, 0.999, 1e-8, 0.1, 3, 1.0, clip)
+    hip.raw.fused_adamw_many(grads, master, m, v, out, 1e-2, 0.9, 0.999, 1e-8, 0.1, 3, clip)
+    for ours, theirs, digits in zip((master, m, v, out), alone, (22, 22, 22, 22 if dtype == torch.float32 else 7)):
+        for a, b in zip(ours, theirs):
+            if a.numel() % 8 == 0:
+                assert torch.equal(a, b)
+            else:
+                assert float((a - b).abs().max()) <= 2.0 ** -digits * float(b.abs().max())
+    want = float(sum(t.double().pow(2).sum() for t in grads))
+    assert abs(float(hip.raw.sumsq_many(grads)) - want) <= 1e-4 * want
+
+
+@pytest.mark.parametrize("sq,top", [(4.0, 1.0), (0.25, 1.0), (0.0, 0.5), (float("inf"), 1.0), (float("nan"), 1.0)])
+def test_clip_factor_is_the_tensor_expression(sq, top):
+    from eventgpt_amd.ops import hip
+    t = torch.tensor(sq, device="cuda:0")
+    norm, clip = hip.raw.clip_factor(t, top)
+    assert torch.equal(norm.nan_to_num(-1), t.sqrt().nan_to_num(-1)) and norm.dim() == 0 and clip.shape == (1,)
+    assert torch.allclose(clip, (top / (t.sqrt() + 1e-6)).clamp(max=1.0).reshape(1), rtol=2.0 ** -22, atol=0, equal_nan=True)     # two roundings
+
+
+@pytest.mark.parametrize("kind", ["mse", "cos", "both"])
+@pytest.mark.parametrize("rows", [1, 1023, 1025])
+def test_pair_loss_of_each_term_and_of_rows_that_are_nothing(kind, rows):
+    """Gradients of either term alone, rows of zeros (the norms' clamp), no valid row, and a mask of another type."""
+    from eventgpt_amd.align import losses as L
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(rows)
+    pred = torch.randn(rows, 1, 64, device=dev, generator=g)
+    pred[::3] = 0
+    target = torch.randn(rows, 1, 64, device=dev, generator=g)
+    for mask in (None, torch.rand(rows, 1, device=dev, generator=g) > 0.5, torch.zeros(rows, 1, device=dev)):
+        got, want = [], []
+        for into, fused in ((got, True), (want, False)):
+            p = pred.clone().requires_grad_()
+            mse, cos = L._RowPairLoss.apply(p, target, mask) if fused else (
+                L.masked_mse(p, target, mask), L.masked_mean(L.cosine_per_position(p, target), mask))
+            ({"mse": mse, "cos": cos, "both": 3 * mse - cos}[kind]).backward()
+            into += [mse.detach(), cos.detach(), p.grad[1::3]]        # (at a row of zeros the cosine has no derivative)
+        for a, b in zip(got, want):
+            assert torch.allclose(a, b, rtol=1e-5, atol=1e-5 * float(b.abs().max()) if b.numel() else 0)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("masked", [False, True])
 def test_fused_alignment_loss_matches_tensor_expressions(dtype, masked):
