@@ -28,6 +28,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
+from ..ops.intree_mode import add_norm, toward, without_hooks
 from .losses import alignment_losses
 
 
@@ -194,11 +195,17 @@ def _blocks(hidden_dim, num_heads, ffn_dim, num_layers, dropout) -> nn.ModuleLis
 
 
 def _run_blocks(layers, x, causal, attention_mask):
-    kpm = None if attention_mask is None else (attention_mask == 0)
+    """``(x, last)``: the rows ahead of the last sublayer's addition, and what it adds (``None`` without a layer)."""
+    kpm, d = None if attention_mask is None else (attention_mask == 0), None
     for layer in layers:
-        x = x + layer["attn"](layer["attn_norm"](x), causal=causal, key_padding_mask=kpm)
-        x = x + layer["ffn"](layer["ffn_norm"](x))
-    return x
+        x, h = (x, layer["attn_norm"](x)) if d is None else add_norm(x, d, layer["attn_norm"])
+        x, h = add_norm(x, layer["attn"](h, causal=causal, key_padding_mask=kpm), layer["ffn_norm"])
+        d = layer["ffn"](h)
+    return x, d
+
+
+def _normed(x, d, norm):
+    return norm(x) if d is None else add_norm(x, d, norm)[1]
 
 
 # ------------------------------------------------------------------------ levels
@@ -291,8 +298,12 @@ class AttentionAdapter(HiddenAdapterBase):
         nn.init.zeros_(self.output_proj[1].bias)
 
     def forward(self, hidden_states, attention_mask=None):
-        x = _run_blocks(self.layers, hidden_states, False, attention_mask)
-        return hidden_states + self.alpha * (self.output_proj(x) - hidden_states)
+        x, d = _run_blocks(self.layers, hidden_states, False, attention_mask)
+        if without_hooks(self.output_proj):
+            y = self.output_proj[1](_normed(x, d, self.output_proj[0]))
+        else:
+            y = self.output_proj(x if d is None else x + d)
+        return toward(hidden_states, y, self.alpha)
 
     def align(self, source, target=None, attention_mask=None):
         return self.forward(source, attention_mask)
@@ -333,9 +344,8 @@ class EAGLEStyleAdapter(HiddenAdapterBase):
         if self.use_token_embed and prev_tokens is not None:
             x = self.token_fusion(torch.cat([x, self.token_embed(prev_tokens)], dim=-1))
         x = self.input_norm(x) + self.pos_embed[:, :x.shape[1]]
-        x = _run_blocks(self.layers, x, True, attention_mask)
-        out = self.output_proj(self.output_norm(x))
-        return hidden_states + self.alpha * (out - hidden_states)
+        x, d = _run_blocks(self.layers, x, True, attention_mask)
+        return toward(hidden_states, self.output_proj(_normed(x, d, self.output_norm)), self.alpha)
 
     def align(self, source, target=None, attention_mask=None):
         return self.forward(source, attention_mask=attention_mask)
@@ -387,9 +397,8 @@ class FusedEAGLEAdapter(HiddenAdapterBase):
         g = self.gate(both)
         x = self.fusion_norm(g * egpt_hidden + (1 - g) * vl_hidden + self.fusion_proj(both))
         x = x + self.pos_embed[:, :x.shape[1]]
-        x = _run_blocks(self.layers, x, True, attention_mask)
-        out = self.output_proj(self.output_norm(x))
-        return vl_hidden + self.alpha * (out - vl_hidden)
+        x, d = _run_blocks(self.layers, x, True, attention_mask)
+        return toward(vl_hidden, self.output_proj(_normed(x, d, self.output_norm)), self.alpha)
 
     def align(self, source, target=None, attention_mask=None):
         if target is None:

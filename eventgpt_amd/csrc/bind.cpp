@@ -818,9 +818,80 @@ Tensor dropout_fwd(const Tensor& x, double p, int64_t seed) {
   return y;
 }
 
-// (dx, dw, db): fp32 parameter gradients when want_params, else empty tensors
+static Tensor param_out(const c10::optional<Tensor>& out, int64_t n, const at::TensorOptions& f32) {
+  if (!out.has_value()) return at::empty({n}, f32);
+  check_f32(*out, "out");
+  TORCH_CHECK(out->numel() == n, "out: one value a column");
+  return *out;
+}
+static void check_add_layernorm(const Tensor& s, const Tensor& d, const Tensor& w, const char* what) {
+  check_f32(s, what); check_bf16(d, what); check_bf16(w, what);
+  const int64_t H = s.dim() ? s.size(-1) : 0;
+  TORCH_CHECK(H >= 8 && H % 8 == 0 && H <= 8192 && w.numel() == H && d.sizes() == s.sizes() && s.numel() / H < (1ll << 31),
+              what, ": two tensors of one shape, rows of a multiple of 8 up to 8192");
+  TORCH_CHECK((reinterpret_cast<uintptr_t>(s.data_ptr()) | reinterpret_cast<uintptr_t>(d.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr())) % 16 == 0,
+              what, ": on 16 bytes");
+}
+
+// (x + d, LayerNorm of that rounded to bf16)
+std::tuple<Tensor, Tensor> add_layernorm(const Tensor& x, const Tensor& d, const Tensor& w, const c10::optional<Tensor>& b, double eps) {
+  check_add_layernorm(x, d, w, "add_layernorm");
+  if (b.has_value()) { check_bf16(*b, "bias"); TORCH_CHECK(b->numel() == w.numel() && reinterpret_cast<uintptr_t>(b->data_ptr()) % 16 == 0); }
+  Tensor s = at::empty_like(x), h = at::empty_like(d);
+  evgpt::launch_add_layernorm(x.data_ptr<float>(), bptr(d), bptr(w), bptr_opt(b), s.data_ptr<float>(), bptr_mut(h), (int)(x.numel() / x.size(-1)),
+                              (int)x.size(-1), (float)eps, cur_stream());
+  return {s, h};
+}
+
+// Its backward by s: (gradient of s in fp32 when want_sum, the same in bf16, dw, db); gs: what reaches s beside the norm
+std::tuple<Tensor, Tensor, Tensor, Tensor> add_layernorm_bwd(const Tensor& s, const Tensor& w, const Tensor& g, const c10::optional<Tensor>& gs,
+                                                             double eps, bool want_sum, bool want_params, const c10::optional<Tensor>& dw_out,
+                                                             const c10::optional<Tensor>& db_out) {
+  check_add_layernorm(s, g, w, "add_layernorm_bwd");
+  if (gs.has_value()) { check_f32(*gs, "gs"); TORCH_CHECK(gs->numel() == s.numel() && reinterpret_cast<uintptr_t>(gs->data_ptr()) % 16 == 0, "add_layernorm_bwd: gs"); }
+  const int64_t H = s.size(-1), rows = s.numel() / H;
+  auto f32 = s.options();
+  Tensor dx = at::empty_like(g), dsum, pw, pb;
+  if (want_sum) dsum = at::empty_like(s);
+  else dsum = at::empty({0}, f32);
+  const int64_t nb = want_params && rows > 0 ? evgpt::layernorm_bwd_blocks((int)rows) : 0;
+  if (nb) { pw = at::empty({nb, H}, f32); pb = at::empty({nb, H}, f32); }
+  evgpt::launch_add_layernorm_bwd(s.data_ptr<float>(), bptr(w), bptr(g), gs.has_value() ? gs->data_ptr<float>() : nullptr,
+                                  want_sum ? dsum.data_ptr<float>() : nullptr, bptr_mut(dx), nb ? pw.data_ptr<float>() : nullptr,
+                                  nb ? pb.data_ptr<float>() : nullptr, (int)rows, (int)H, (float)eps, cur_stream());
+  if (!nb) return {dsum, dx, at::zeros({want_params ? H : 0}, f32), at::zeros({want_params ? H : 0}, f32)};
+  Tensor dw = param_out(dw_out, H, f32), db = param_out(db_out, H, f32);
+  evgpt::launch_column_sum_pair(pw.data_ptr<float>(), pb.data_ptr<float>(), dw.data_ptr<float>(), db.data_ptr<float>(), (int)nb, (int)H, cur_stream());
+  return {dsum, dx, dw, db};
+}
+
+static void check_toward(const Tensor& base, const Tensor& y, const Tensor& alpha) {
+  check_f32(base, "base"); check_bf16(y, "y"); check_f32(alpha, "alpha");
+  TORCH_CHECK(base.sizes() == y.sizes() && base.numel() % 8 == 0 && base.numel() > 0 && alpha.numel() == 1 &&
+                  (reinterpret_cast<uintptr_t>(base.data_ptr()) | reinterpret_cast<uintptr_t>(y.data_ptr())) % 16 == 0,
+              "toward: two tensors of one shape and whole 16-byte pieces, one alpha");
+}
+// base + alpha (y - base)
+Tensor toward(const Tensor& base, const Tensor& y, const Tensor& alpha) {
+  check_toward(base, y, alpha);
+  Tensor out = at::empty_like(base);
+  evgpt::launch_toward(base.data_ptr<float>(), bptr(y), alpha.data_ptr<float>(), out.data_ptr<float>(), base.numel(), cur_stream());
+  return out;
+}
+// gradients of y and alpha
+std::tuple<Tensor, Tensor> toward_bwd(const Tensor& g, const Tensor& base, const Tensor& y, const Tensor& alpha) {
+  check_toward(base, y, alpha);
+  check_f32(g, "g");
+  TORCH_CHECK(g.numel() == base.numel() && reinterpret_cast<uintptr_t>(g.data_ptr()) % 16 == 0, "toward_bwd: g");
+  Tensor gy = at::empty_like(y), part = at::empty({evgpt::toward_blocks(g.numel())}, g.options()), ga = at::empty(alpha.sizes(), alpha.options());
+  evgpt::launch_toward_bwd(g.data_ptr<float>(), base.data_ptr<float>(), bptr(y), alpha.data_ptr<float>(), bptr_mut(gy), part.data_ptr<float>(),
+                           ga.data_ptr<float>(), g.numel(), cur_stream());
+  return {gy, ga};
+}
+
+// (dx, dw, db): fp32 parameter gradients when want_params, else empty tensors; dw_out, db_out: where they go
 std::tuple<Tensor, Tensor, Tensor> layernorm_bwd(const Tensor& x, const Tensor& w, const Tensor& g, double eps,
-                                                 bool want_params) {
+                                                 bool want_params, const c10::optional<Tensor>& dw_out, const c10::optional<Tensor>& db_out) {
   check_bf16(x, "x"); check_bf16(w, "weight"); check_bf16(g, "grad");
   const int64_t H = x.size(-1), rows = x.numel() / H;
   TORCH_CHECK(H % 8 == 0 && H <= 8192 && w.numel() == H && g.numel() == x.numel(),
@@ -839,20 +910,22 @@ std::tuple<Tensor, Tensor, Tensor> layernorm_bwd(const Tensor& x, const Tensor& 
     auto none = [&] { return at::zeros({want_params ? H : 0}, f32); };
     return std::make_tuple(dx, none(), none());
   }
-  Tensor dw = at::empty({H}, f32), db = at::empty({H}, f32);
+  Tensor dw = param_out(dw_out, H, f32), db = param_out(db_out, H, f32);
   evgpt::launch_column_sum_pair(pw.data_ptr<float>(), pb.data_ptr<float>(), dw.data_ptr<float>(), db.data_ptr<float>(), (int)pw.size(0),
                                 (int)H, cur_stream());
   return std::make_tuple(dx, dw, db);
 }
 
 // sum over the rows of bf16 [M, N] in float32, rounded once (bias gradients)
-Tensor column_sum(const Tensor& g, bool out_f32) {
+Tensor column_sum(const Tensor& g, bool out_f32, const c10::optional<Tensor>& into) {
   check_bf16(g, "g");
   TORCH_CHECK(g.dim() == 2 && g.size(0) >= 1 && g.size(0) < (1ll << 30) && g.size(1) >= 8 && g.size(1) < (1ll << 30) &&
                   g.size(1) % 8 == 0 && reinterpret_cast<uintptr_t>(g.data_ptr()) % 16 == 0,
               "column_sum: contiguous [M, N], N a multiple of 8, on 16 bytes");
   const int M = (int)g.size(0), N = (int)g.size(1);
-  Tensor part = at::empty({evgpt::column_sum_slabs(M, N), N}, g.options().dtype(at::kFloat)), out = at::empty({N}, g.options().dtype(out_f32 ? at::kFloat : at::kBFloat16));
+  TORCH_CHECK(!into.has_value() || out_f32, "column_sum: written into a float32 tensor");
+  const auto f32 = g.options().dtype(at::kFloat);
+  Tensor part = at::empty({evgpt::column_sum_slabs(M, N), N}, f32), out = out_f32 ? param_out(into, N, f32) : at::empty({N}, g.options());
   evgpt::launch_column_sum(bptr(g), part.data_ptr<float>(), out.data_ptr(), out_f32, M, N, cur_stream());
   return out;
 }
@@ -1662,8 +1735,12 @@ TORCH_LIBRARY(evgpt, m) {
   m.def("gelu_fwd(Tensor x) -> Tensor", &gelu_fwd);
   m.def("gelu_bwd(Tensor x, Tensor grad) -> Tensor", &gelu_bwd);
   m.def("dropout_fwd(Tensor x, float p, int seed) -> Tensor", &dropout_fwd);
-  m.def("layernorm_bwd(Tensor x, Tensor weight, Tensor grad, float eps, bool want_params=True) -> (Tensor, Tensor, Tensor)", &layernorm_bwd);
-  m.def("column_sum(Tensor g, bool out_f32=False) -> Tensor", &column_sum);
+  m.def("layernorm_bwd(Tensor x, Tensor weight, Tensor grad, float eps, bool want_params=True, Tensor(a!)? dw_out=None, Tensor(b!)? db_out=None) -> (Tensor, Tensor, Tensor)", &layernorm_bwd);
+  m.def("column_sum(Tensor g, bool out_f32=False, Tensor(a!)? into=None) -> Tensor", &column_sum);
+  m.def("add_layernorm(Tensor x, Tensor d, Tensor weight, Tensor? bias, float eps) -> (Tensor, Tensor)", &add_layernorm);
+  m.def("add_layernorm_bwd(Tensor s, Tensor weight, Tensor grad, Tensor? gs, float eps, bool want_sum, bool want_params, Tensor(a!)? dw_out=None, Tensor(b!)? db_out=None) -> (Tensor, Tensor, Tensor, Tensor)", &add_layernorm_bwd);
+  m.def("toward(Tensor base, Tensor y, Tensor alpha) -> Tensor", &toward);
+  m.def("toward_bwd(Tensor g, Tensor base, Tensor y, Tensor alpha) -> (Tensor, Tensor)", &toward_bwd);
   m.def("sumsq_accumulate(Tensor x, Tensor(a!) acc) -> ()", &sumsq_accumulate);
   m.def("sumsq_many(Tensor[] xs) -> Tensor", &sumsq_many);
   m.def("clip_factor(Tensor sq, float max_norm) -> (Tensor, Tensor)", &clip_factor);

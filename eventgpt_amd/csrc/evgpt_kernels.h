@@ -59,6 +59,14 @@ int column_sum_slabs(int M, int N);
 // out [N]: bf16 or fp32
 void launch_column_sum(const bf16_t* G, float* part, void* out, bool out_f32, int M, int N, hipStream_t st);
 void launch_column_sum_pair(const float* p0, const float* p1, float* out0, float* out1, int slabs, int N, hipStream_t st);
+void launch_add_layernorm(const float* x, const bf16_t* d, const bf16_t* w, const bf16_t* b, float* s, bf16_t* h, int rows, int H, float eps,
+                          hipStream_t st);
+void launch_add_layernorm_bwd(const float* s, const bf16_t* w, const bf16_t* g, const float* gs, float* dsum, bf16_t* dx, float* dw, float* db,
+                              int rows, int H, float eps, hipStream_t st);
+int toward_blocks(long long n);        // floats of `part`
+void launch_toward(const float* base, const bf16_t* y, const float* alpha, float* out, long long n, hipStream_t st);
+void launch_toward_bwd(const float* g, const float* base, const bf16_t* y, const float* alpha, bf16_t* gy, float* part, float* galpha, long long n,
+                       hipStream_t st);
 int layernorm_bwd_blocks(int rows);    // rows of the [blocks][H] fp32 dw / db partial buffers
 void launch_layernorm_bwd(const bf16_t* x, const bf16_t* w, const bf16_t* g, bf16_t* dx, float* dw, float* db,
                           int rows, int H, float eps, hipStream_t st);

@@ -423,51 +423,86 @@ __device__ __forceinline__ void ln_block_sum2(float& a, float& b, float* scratch
   a = scratch[0] + scratch[1] + scratch[2] + scratch[3];
   b = scratch[8] + scratch[9] + scratch[10] + scratch[11];
 }
-__global__ __launch_bounds__(256) void layernorm_bwd_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+// eight float32 values as bf16
+__device__ __forceinline__ u32x4_t rounded8(const float* p) {
+  const f32x4_t a = *reinterpret_cast<const f32x4_t*>(p), b = *reinterpret_cast<const f32x4_t*>(p + 4);
+  return u32x4_t{pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3]), pack_bf16x2(b[0], b[1]), pack_bf16x2(b[2], b[3])};
+}
+// SUM: the backward of s = x + d, h = LayerNorm(s rounded to bf16) by s: x is the float32 s, gs (or null) the gradient that reaches s beside the
+// norm, their sum goes out in float32 (sum_out, or null) and bf16 (dx).
+// NC: 16-byte chunks a thread has of a row (rows of up to 2 048 NC), so that a row of 4 096 leaves registers for the next one, which is
+// requested ahead of this one's three block sums.  3 200 x 4 096: 26 us plain (93 MB; four chunks and none ahead 26 too), 32 with the sum (197 MB).
+template <bool SUM, int NC>
+__global__ __launch_bounds__(256) void layernorm_bwd_kernel(const void* __restrict__ x_, const bf16_t* __restrict__ w,
                                                             const bf16_t* __restrict__ g, bf16_t* __restrict__ dx,
                                                             float* __restrict__ dw, float* __restrict__ db, int rows,
-                                                            int H, float eps, int rows_per_block) {
+                                                            int H, float eps, int rows_per_block, const float* __restrict__ gs,
+                                                            float* __restrict__ sum_out) {
   __shared__ float scratch[16];
   const int tid = threadIdx.x, nchunk = H >> 3;
-  float dwacc[LN_MAX_CHUNKS][8], dbacc[LN_MAX_CHUNKS][8];
+  float dwacc[NC][8], dbacc[NC][8], wv[NC][8];
 #pragma unroll
-  for (int i = 0; i < LN_MAX_CHUNKS; ++i)
-#pragma unroll
-    for (int k = 0; k < 8; ++k) { dwacc[i][k] = 0.f; dbacc[i][k] = 0.f; }
-  float wv[LN_MAX_CHUNKS][8];
-#pragma unroll
-  for (int i = 0; i < LN_MAX_CHUNKS; ++i) {
+  for (int i = 0; i < NC; ++i) {
     const int c = tid + i * 256;
     const u32x4_t t = c < nchunk ? load16(w + c * 8) : u32x4_t{0, 0, 0, 0};
 #pragma unroll
     for (int j = 0; j < 4; ++j) { wv[i][2 * j] = bf16lo(t[j]); wv[i][2 * j + 1] = bf16hi(t[j]); }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) { dwacc[i][k] = 0.f; dbacc[i][k] = 0.f; }
   }
   const float inv_h = 1.f / static_cast<float>(H);
   const int r0 = blockIdx.x * rows_per_block, r1 = min(r0 + rows_per_block, rows);
-  for (int r = r0; r < r1; ++r) {
-    const bf16_t* xr = x + static_cast<size_t>(r) * H;
-    const bf16_t* gr = g + static_cast<size_t>(r) * H;
-    float xe[LN_MAX_CHUNKS][8], ge[LN_MAX_CHUNKS][8];
-    float s1 = 0.f, zero = 0.f;
+  u32x4_t xn[NC], gn[NC];              // the row that is requested (SUM: its float32 halves in xn and xh)
+  u32x4_t xh[SUM ? NC : 1], sn[SUM ? NC : 1][2];
+  const u32x4_t none = {0, 0, 0, 0};
+  const auto request = [&](int r) {
 #pragma unroll
-    for (int i = 0; i < LN_MAX_CHUNKS; ++i) {
+    for (int i = 0; i < NC; ++i) {
       const int c = tid + i * 256;
       const bool ok = c < nchunk;
-      const u32x4_t xv = ok ? load16(xr + c * 8) : u32x4_t{0, 0, 0, 0};
-      const u32x4_t gv = ok ? load16(gr + c * 8) : u32x4_t{0, 0, 0, 0};
+      const size_t at = static_cast<size_t>(r) * H + (ok ? c : 0) * 8;
+      gn[i] = ok ? load16(g + at) : none;
+      if constexpr (SUM) {
+        const float* xs = static_cast<const float*>(x_) + at;
+        xn[i] = ok ? load16(xs) : none;
+        xh[i] = ok ? load16(xs + 4) : none;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) sn[i][h] = ok && gs ? load16(gs + at + h * 4) : none;
+      } else {
+        xn[i] = ok ? load16(static_cast<const bf16_t*>(x_) + at) : none;
+      }
+    }
+  };
+  if (r0 < r1) request(r0);
+  for (int r = r0; r < r1; ++r) {
+    float xe[NC][8], ge[NC][8], se[SUM ? NC : 1][8];
+    float s1 = 0.f, zero = 0.f;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      u32x4_t xv = xn[i];
+      if constexpr (SUM) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          xv[j] = pack_bf16x2(__uint_as_float(xn[i][2 * j]), __uint_as_float(xn[i][2 * j + 1]));
+          xv[2 + j] = pack_bf16x2(__uint_as_float(xh[i][2 * j]), __uint_as_float(xh[i][2 * j + 1]));
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) se[i][j] = __uint_as_float(sn[i][j >> 2][j & 3]);
+      }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         xe[i][2 * j] = bf16lo(xv[j]); xe[i][2 * j + 1] = bf16hi(xv[j]);
-        ge[i][2 * j] = bf16lo(gv[j]); ge[i][2 * j + 1] = bf16hi(gv[j]);
+        ge[i][2 * j] = bf16lo(gn[i][j]); ge[i][2 * j + 1] = bf16hi(gn[i][j]);
         s1 += xe[i][2 * j] + xe[i][2 * j + 1];
       }
     }
+    if (r + 1 < r1) request(r + 1);
     ln_block_sum2(s1, zero, scratch);
     const float mu = s1 * inv_h;
     float s2 = 0.f;
     zero = 0.f;
 #pragma unroll
-    for (int i = 0; i < LN_MAX_CHUNKS; ++i) {
+    for (int i = 0; i < NC; ++i) {
       const bool ok = tid + i * 256 < nchunk;
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
@@ -479,7 +514,7 @@ __global__ __launch_bounds__(256) void layernorm_bwd_kernel(const bf16_t* __rest
     const float rstd = rsqrtf(s2 * inv_h + eps);
     float a = 0.f, bsum = 0.f;      // sum(g w), sum(g w xh)
 #pragma unroll
-    for (int i = 0; i < LN_MAX_CHUNKS; ++i)
+    for (int i = 0; i < NC; ++i)
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         xe[i][k] *= rstd;                       // xh
@@ -492,26 +527,37 @@ __global__ __launch_bounds__(256) void layernorm_bwd_kernel(const bf16_t* __rest
     ln_block_sum2(a, bsum, scratch);
     const float ma = a * inv_h, mb = bsum * inv_h;
 #pragma unroll
-    for (int i = 0; i < LN_MAX_CHUNKS; ++i) {
+    for (int i = 0; i < NC; ++i) {
       const int c = tid + i * 256;
       if (c >= nchunk) continue;
+      const size_t at = static_cast<size_t>(r) * H + c * 8;
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        v[j] = rstd * (ge[i][j] * wv[i][j] - ma - xe[i][j] * mb);
+        if constexpr (SUM) v[j] += se[i][j];
+      }
+      if (SUM && sum_out) {
+        *reinterpret_cast<f32x4_t*>(sum_out + at) = f32x4_t{v[0], v[1], v[2], v[3]};
+        *reinterpret_cast<f32x4_t*>(sum_out + at + 4) = f32x4_t{v[4], v[5], v[6], v[7]};
+      }
       u32x4_t o;
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        o[j] = pack_bf16x2(rstd * (ge[i][2 * j] * wv[i][2 * j] - ma - xe[i][2 * j] * mb),
-                           rstd * (ge[i][2 * j + 1] * wv[i][2 * j + 1] - ma - xe[i][2 * j + 1] * mb));
-      *reinterpret_cast<u32x4_t*>(dx + static_cast<size_t>(r) * H + c * 8) = o;
+      for (int j = 0; j < 4; ++j) o[j] = pack_bf16x2(v[2 * j], v[2 * j + 1]);
+      *reinterpret_cast<u32x4_t*>(dx + at) = o;
     }
   }
   if (dw) {
 #pragma unroll
-    for (int i = 0; i < LN_MAX_CHUNKS; ++i) {
+    for (int i = 0; i < NC; ++i) {
       const int c = tid + i * 256;
       if (c >= nchunk) continue;
+      float* dst[2] = {dw + static_cast<size_t>(blockIdx.x) * H + c * 8, db + static_cast<size_t>(blockIdx.x) * H + c * 8};
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        dw[static_cast<size_t>(blockIdx.x) * H + c * 8 + k] = dwacc[i][k];
-        db[static_cast<size_t>(blockIdx.x) * H + c * 8 + k] = dbacc[i][k];
+      for (int h = 0; h < 2; ++h) {
+        const float* v = h ? dbacc[i] : dwacc[i];
+        *reinterpret_cast<f32x4_t*>(dst[h]) = f32x4_t{v[0], v[1], v[2], v[3]};
+        *reinterpret_cast<f32x4_t*>(dst[h] + 4) = f32x4_t{v[4], v[5], v[6], v[7]};
       }
     }
   }
@@ -527,7 +573,133 @@ void launch_layernorm_bwd(const bf16_t* x, const bf16_t* w, const bf16_t* g, bf1
   if (rows <= 0) return;
   const int blocks = layernorm_bwd_blocks(rows);
   const int rpb = (rows + blocks - 1) / blocks;
-  hipLaunchKernelGGL(layernorm_bwd_kernel, dim3(blocks), dim3(256), 0, st, x, w, g, dx, dw, db, rows, H, eps, rpb);
+  if (H <= 4096) hipLaunchKernelGGL((layernorm_bwd_kernel<false, 2>), dim3(blocks), dim3(256), 0, st, x, w, g, dx, dw, db, rows, H, eps, rpb, nullptr, nullptr);
+  else hipLaunchKernelGGL((layernorm_bwd_kernel<false, LN_MAX_CHUNKS>), dim3(blocks), dim3(256), 0, st, x, w, g, dx, dw, db, rows, H, eps, rpb, nullptr, nullptr);
+}
+void launch_add_layernorm_bwd(const float* s, const bf16_t* w, const bf16_t* g, const float* gs, float* dsum, bf16_t* dx, float* dw, float* db,
+                              int rows, int H, float eps, hipStream_t st) {
+  if (rows <= 0) return;
+  const int blocks = layernorm_bwd_blocks(rows);
+  const int rpb = (rows + blocks - 1) / blocks;
+  if (H <= 4096) hipLaunchKernelGGL((layernorm_bwd_kernel<true, 2>), dim3(blocks), dim3(256), 0, st, s, w, g, dx, dw, db, rows, H, eps, rpb, gs, dsum);
+  else hipLaunchKernelGGL((layernorm_bwd_kernel<true, LN_MAX_CHUNKS>), dim3(blocks), dim3(256), 0, st, s, w, g, dx, dw, db, rows, H, eps, rpb, gs, dsum);
+}
+
+// s = x + d (float32 residual rows, bf16 sublayer output) and h = LayerNorm(s rounded to bf16).  Bound by memory: one pass, the row in
+// registers, where an addition, a cast and the norm read and wrote it three times.  3 200 x 4 096: 49 us in three launches, 28 so; the
+// backward, which adds the norm's gradient to the residual's and rounds the sum for the products ahead of it, 74 and 34.
+__global__ __launch_bounds__(256) void add_layernorm_kernel(const float* __restrict__ x, const bf16_t* __restrict__ d,
+                                                            const bf16_t* __restrict__ w, const bf16_t* __restrict__ b,
+                                                            float* __restrict__ s, bf16_t* __restrict__ h, int H, float eps) {
+  __shared__ float red[4];
+  const int tid = threadIdx.x, nchunk = H >> 3;
+  const size_t base = static_cast<size_t>(blockIdx.x) * H;
+  float e[LN_MAX_CHUNKS][8];
+  float sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < LN_MAX_CHUNKS; ++i) {
+    const int c = tid + i * 256;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) e[i][j] = 0.f;
+    if (c >= nchunk) continue;
+    const size_t at = base + c * 8;
+    f32x4_t lo = *reinterpret_cast<const f32x4_t*>(x + at), hi = *reinterpret_cast<const f32x4_t*>(x + at + 4);
+    const u32x4_t dv = load16(d + at);
+    lo += f32x4_t{bf16lo(dv[0]), bf16hi(dv[0]), bf16lo(dv[1]), bf16hi(dv[1])};
+    hi += f32x4_t{bf16lo(dv[2]), bf16hi(dv[2]), bf16lo(dv[3]), bf16hi(dv[3])};
+    *reinterpret_cast<f32x4_t*>(s + at) = lo;
+    *reinterpret_cast<f32x4_t*>(s + at + 4) = hi;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      e[i][j] = bf16_to_f32(f32_to_bf16(lo[j]));
+      e[i][4 + j] = bf16_to_f32(f32_to_bf16(hi[j]));
+      sum += e[i][j] + e[i][4 + j];
+    }
+  }
+  const float mean = block_sum<4>(sum, red) / static_cast<float>(H);
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < LN_MAX_CHUNKS; ++i)
+    if (tid + i * 256 < nchunk)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) { const float t = e[i][j] - mean; ss += t * t; }
+  const float rstd = rsqrtf(block_sum<4>(ss, red) / static_cast<float>(H) + eps);
+#pragma unroll
+  for (int i = 0; i < LN_MAX_CHUNKS; ++i) {
+    const int c = tid + i * 256;
+    if (c >= nchunk) continue;
+    const u32x4_t g = load16(w + c * 8), bb = b ? load16(b + c * 8) : u32x4_t{0, 0, 0, 0};
+    u32x4_t o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      o[j] = pack_bf16x2((e[i][2 * j] - mean) * rstd * bf16lo(g[j]) + bf16lo(bb[j]), (e[i][2 * j + 1] - mean) * rstd * bf16hi(g[j]) + bf16hi(bb[j]));
+    *reinterpret_cast<u32x4_t*>(h + base + c * 8) = o;
+  }
+}
+void launch_add_layernorm(const float* x, const bf16_t* d, const bf16_t* w, const bf16_t* b, float* s, bf16_t* h, int rows, int H, float eps,
+                          hipStream_t st) {
+  if (rows > 0) hipLaunchKernelGGL(add_layernorm_kernel, dim3(rows), dim3(256), 0, st, x, d, w, b, s, h, H, eps);
+}
+
+// ------------------------------------------------------------------- out = base + alpha (y - base)
+// Base rows in float32, y bf16, alpha a float32 scalar on the device: the adapters' last step.  Bound by memory; as tensor expressions forward and
+// backward were three passes each (3 200 x 4 096: 66 and 77 us, so 22 and 24).  The backward gives y's gradient and alpha's, block sums in a
+// second launch.
+constexpr int TOWARD_BLOCKS = 2048;
+__global__ __launch_bounds__(256) void toward_kernel(const float* __restrict__ base, const bf16_t* __restrict__ y, const float* __restrict__ alpha,
+                                                     float* __restrict__ out, long long n8) {
+  const float a = *alpha;
+  for (long long i = blockIdx.x * 256ll + threadIdx.x; i < n8; i += gridDim.x * 256ll) {
+    const u32x4_t yv = load16(y + i * 8);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const f32x4_t bv = *reinterpret_cast<const f32x4_t*>(base + i * 8 + h * 4);
+      const f32x4_t t = {bf16lo(yv[2 * h]), bf16hi(yv[2 * h]), bf16lo(yv[2 * h + 1]), bf16hi(yv[2 * h + 1])};
+      *reinterpret_cast<f32x4_t*>(out + i * 8 + h * 4) = bv + a * (t - bv);
+    }
+  }
+}
+__global__ __launch_bounds__(256) void toward_bwd_kernel(const float* __restrict__ g, const float* __restrict__ base, const bf16_t* __restrict__ y,
+                                                         const float* __restrict__ alpha, bf16_t* __restrict__ gy, float* __restrict__ part,
+                                                         long long n8) {
+  __shared__ float red[4];
+  const float a = *alpha;
+  float s = 0.f;
+  for (long long i = blockIdx.x * 256ll + threadIdx.x; i < n8; i += gridDim.x * 256ll) {
+    const u32x4_t yv = load16(y + i * 8);
+    u32x4_t o;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const f32x4_t gv = *reinterpret_cast<const f32x4_t*>(g + i * 8 + h * 4), bv = *reinterpret_cast<const f32x4_t*>(base + i * 8 + h * 4);
+      const f32x4_t t = {bf16lo(yv[2 * h]), bf16hi(yv[2 * h]), bf16lo(yv[2 * h + 1]), bf16hi(yv[2 * h + 1])};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s += gv[j] * (t[j] - bv[j]);
+      o[2 * h] = pack_bf16x2(gv[0] * a, gv[1] * a);
+      o[2 * h + 1] = pack_bf16x2(gv[2] * a, gv[3] * a);
+    }
+    *reinterpret_cast<u32x4_t*>(gy + i * 8) = o;
+  }
+  s = block_sum<4>(s, red);
+  if (threadIdx.x == 0) part[blockIdx.x] = s;
+}
+__global__ __launch_bounds__(256) void toward_alpha_kernel(const float* __restrict__ part, int n, float* __restrict__ out) {
+  __shared__ float red[4];
+  float s = 0.f;
+  for (int i = threadIdx.x; i < n; i += 256) s += part[i];
+  s = block_sum<4>(s, red);
+  if (threadIdx.x == 0) *out = s;
+}
+int toward_blocks(long long n) {
+  const long long b = (n / 8 + 255) / 256;
+  return static_cast<int>(b > TOWARD_BLOCKS ? TOWARD_BLOCKS : (b < 1 ? 1 : b));
+}
+void launch_toward(const float* base, const bf16_t* y, const float* alpha, float* out, long long n, hipStream_t st) {
+  hipLaunchKernelGGL(toward_kernel, dim3(toward_blocks(n)), dim3(256), 0, st, base, y, alpha, out, n / 8);
+}
+void launch_toward_bwd(const float* g, const float* base, const bf16_t* y, const float* alpha, bf16_t* gy, float* part, float* galpha, long long n,
+                       hipStream_t st) {
+  hipLaunchKernelGGL(toward_bwd_kernel, dim3(toward_blocks(n)), dim3(256), 0, st, g, base, y, alpha, gy, part, n / 8);
+  hipLaunchKernelGGL(toward_alpha_kernel, dim3(1), dim3(256), 0, st, part, toward_blocks(n), galpha);
 }
 
 // ----------------------------------------------------------------------------- column sums (bias gradients)

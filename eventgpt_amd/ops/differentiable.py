@@ -120,17 +120,100 @@ class _LayerNorm(torch.autograd.Function):
         wb = weight.detach().to(torch.bfloat16).contiguous()
         bb = None if bias is None else bias.detach().to(torch.bfloat16).contiguous()
         ctx.save_for_backward(xc, wb)
-        ctx.eps, ctx.has_bias = eps, bias is not None
-        ctx.pdtype = (weight.dtype, None if bias is None else bias.dtype)
+        ctx.eps = eps
+        _keep_norm_parameters(ctx, weight, bias)
         return _raw().layernorm(xc, wb, bb, eps, 0)
 
     @staticmethod
     def backward(ctx, g):
         x, wb = ctx.saved_tensors
-        want = bool(ctx.needs_input_grad[1] or (ctx.has_bias and ctx.needs_input_grad[2]))
-        dx, dw, db = _raw().layernorm_bwd(x, wb, g.contiguous(), ctx.eps, want)
-        return (dx, dw.to(ctx.pdtype[0]).view_as(wb) if ctx.needs_input_grad[1] else None,
-                db.to(ctx.pdtype[1]).view_as(wb) if (ctx.has_bias and ctx.needs_input_grad[2]) else None, None)
+        sinks, want = _norm_sinks(ctx, *ctx.needs_input_grad[1:3])
+        dx, dw, db = _raw().layernorm_bwd(x, wb, g.contiguous(), ctx.eps, want, *sinks)
+        return (dx, *_norm_grads(ctx, wb, sinks, dw, db, *ctx.needs_input_grad[1:3]), None)
+
+
+def _keep_norm_parameters(ctx, weight, bias):
+    # (the parameters for their gradient slots; computed ones are not kept until the backward)
+    ctx.parameters = tuple(t if t is not None and t.is_leaf else None for t in (weight, bias))
+    ctx.pdtype = (weight.dtype, None if bias is None else bias.dtype)
+
+
+def _norm_sinks(ctx, want_w: bool, want_b: bool):
+    """The gradient slots of a norm's parameters that are free, and whether their gradients are wanted at all."""
+    want = (want_w, want_b and ctx.pdtype[1] is not None)
+    return tuple(_free_sink(ctx, p, torch.float32) if w and p is not None and p.dtype == torch.float32 else None
+                 for p, w in zip(ctx.parameters, want)), any(want)
+
+
+def _norm_grads(ctx, wb, sinks, dw, db, want_w: bool, want_b: bool):
+    return (dw.to(ctx.pdtype[0]).view_as(wb) if want_w else None,
+            db.to(ctx.pdtype[1]).view_as(wb) if want_b and ctx.pdtype[1] is not None else None)
+
+
+class _AddLayerNorm(torch.autograd.Function):
+    """``s = x + d`` and ``LayerNorm(s rounded to bf16)`` of fp32 residual rows and a bf16 sublayer output, in one pass each way
+    (``csrc/kernels/adapter_train.hip``)."""
+
+    @staticmethod
+    def forward(ctx, x, d, weight, bias, eps):
+        ctx.set_materialize_grads(False)
+        wb = weight.detach().to(torch.bfloat16).contiguous()
+        bb = None if bias is None else bias.detach().to(torch.bfloat16).contiguous()
+        s, h = _raw().add_layernorm(x, d, wb, bb, eps)
+        ctx.save_for_backward(s, wb)
+        ctx.eps = eps
+        _keep_norm_parameters(ctx, weight, bias)
+        return s, h
+
+    @staticmethod
+    def backward(ctx, gs, gh):
+        s, wb = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        if gh is None:
+            return (gs if need[0] else None, gs.to(torch.bfloat16) if gs is not None and need[1] else None, None, None, None)
+        sinks, want = _norm_sinks(ctx, *need[2:4])
+        aligned = None if gs is None else gs.contiguous() if gs.data_ptr() % 16 == 0 else gs.clone(memory_format=torch.contiguous_format)
+        dsum, dd, dw, db = _raw().add_layernorm_bwd(s, wb, gh.contiguous(), aligned, ctx.eps, need[0], want, *sinks)
+        return (dsum if need[0] else None, dd if need[1] else None, *_norm_grads(ctx, wb, sinks, dw, db, *need[2:4]), None)
+
+
+def add_layernorm_ok(x, d, weight, bias) -> bool:
+    h = x.shape[-1]
+    return (x.is_cuda and x.dtype == torch.float32 and _fused(d) and d.shape == x.shape and x.is_contiguous() and d.is_contiguous()
+            and x.data_ptr() % 16 == 0 and d.data_ptr() % 16 == 0 and h % 8 == 0 and 8 <= h <= 8192 and x.numel() > 0
+            and weight is not None and weight.is_cuda and weight.numel() == h and (bias is None or (bias.is_cuda and bias.numel() == h)))
+
+
+def add_layernorm(x, d, weight, bias, eps: float = 1e-5):
+    """``(x + d, layer_norm(x + d))`` where ``add_layernorm_ok``."""
+    return _AddLayerNorm.apply(x, d, weight, bias, eps)
+
+
+class _Toward(torch.autograd.Function):
+    """``base + alpha (y - base)`` of fp32 rows that need no gradient, bf16 ``y`` and an fp32 scalar."""
+
+    @staticmethod
+    def forward(ctx, base, y, alpha):
+        ctx.save_for_backward(base, y, alpha)
+        return _raw().toward(base, y, alpha.detach())
+
+    @staticmethod
+    def backward(ctx, g):
+        base, y, alpha = ctx.saved_tensors
+        g = g.contiguous() if g.data_ptr() % 16 == 0 else g.clone(memory_format=torch.contiguous_format)
+        gy, ga = _raw().toward_bwd(g, base, y, alpha.detach())
+        return None, gy if ctx.needs_input_grad[1] else None, ga if ctx.needs_input_grad[2] else None
+
+
+def toward_ok(base, y, alpha) -> bool:
+    return (base.is_cuda and base.dtype == torch.float32 and not base.requires_grad and _ew_ok(y) and y.shape == base.shape
+            and base.is_contiguous() and y.is_contiguous() and base.data_ptr() % 16 == 0 and y.data_ptr() % 16 == 0
+            and isinstance(alpha, torch.Tensor) and alpha.is_cuda and alpha.dtype == torch.float32 and alpha.numel() == 1 and alpha.dim() == 0)
+
+
+def toward(base, y, alpha):
+    """``base + alpha * (y - base)`` where ``toward_ok``."""
+    return _Toward.apply(base, y, alpha)
 
 
 class _Gelu(torch.autograd.Function):
@@ -424,8 +507,9 @@ class _MasterLinear(torch.autograd.Function):
         xc = x if x.is_contiguous() else x.contiguous()
         w = weight.detach().to(torch.bfloat16)
         ctx.save_for_backward(xc.view(-1, x.shape[-1]), w)
-        # (the parameter for its gradient slot; a weight that was computed is not kept until the backward)
+        # (the parameters for their gradient slots; one that was computed is not kept until the backward)
         ctx.parameter, ctx.has_bias = weight if weight.is_leaf else None, bias is not None
+        ctx.bias = bias if bias is not None and bias.is_leaf else None
         return hip.linear(xc, w, None if bias is None else bias.detach().to(torch.bfloat16))
 
     @staticmethod
@@ -438,8 +522,12 @@ class _MasterLinear(torch.autograd.Function):
         dw = _wgrad_to_sink(ctx, ctx.parameter, g2, x2, True) if ctx.needs_input_grad[1] else None
         db = None
         if ctx.has_bias and ctx.needs_input_grad[2]:
-            db = (_raw().column_sum(g2, True) if n >= 512 and n % 8 == 0 and g2.numel() and g2.data_ptr() % 16 == 0
-                  else g2.float().sum(0))
+            if n >= 512 and n % 8 == 0 and g2.numel() and g2.data_ptr() % 16 == 0:
+                sink = _free_sink(ctx, ctx.bias, torch.float32)
+                db = _raw().column_sum(g2, True, sink)
+                db = db if sink is None else db.view_as(sink)
+            else:
+                db = g2.float().sum(0)
         return dx, dw, db
 
 

@@ -22,7 +22,7 @@ from __future__ import annotations
 
 import torch
 import torch.nn.functional as F
-from torch.overrides import TorchFunctionMode
+from torch.overrides import TorchFunctionMode, handle_torch_function, has_torch_function
 
 from . import differentiable as diff
 
@@ -42,6 +42,28 @@ def _eligible(x, w, b) -> bool:
     return x.numel() // k >= 16 and diff._raw() is not None
 
 
+def without_hooks(module) -> bool:
+    """Whether a call of ``module`` may be left out for its parts: nobody is told of calls of it, or of all modules'."""
+    m = torch.nn.modules.module
+    return not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+                or m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks or m._global_backward_pre_hooks)
+
+
+def add_norm(x, d, norm):
+    """``(x + d, norm(x + d))``, ``norm`` an ``nn.LayerNorm``: a step of the residual stream, one launch inside ``InTreeLinear``."""
+    if has_torch_function((x, d)):
+        return handle_torch_function(add_norm, (x, d), x, d, norm)
+    s = x + d
+    return s, norm(s)
+
+
+def toward(base, y, alpha):
+    """``base + alpha * (y - base)``, one launch inside ``InTreeLinear``."""
+    if has_torch_function((base, y, alpha)):
+        return handle_torch_function(toward, (base, y, alpha), base, y, alpha)
+    return base + alpha * (y - base)
+
+
 class InTreeLinear(TorchFunctionMode):
     """``with InTreeLinear(): loss = model(...)`` -- see the module docstring."""
 
@@ -52,6 +74,20 @@ class InTreeLinear(TorchFunctionMode):
 
     def __torch_function__(self, func, types, args=(), kwargs=None):
         kwargs = kwargs or {}
+        if func is add_norm:
+            x, d, norm = args
+            if (type(norm) is torch.nn.LayerNorm and without_hooks(norm) and len(norm.normalized_shape) == 1
+                    and x.numel() // x.shape[-1] >= 16 and diff.add_layernorm_ok(x, d, norm.weight, norm.bias)):
+                self.routed += 1
+                return diff.add_layernorm(x, d, norm.weight, norm.bias, norm.eps)
+            s = x + d
+            with self:                                 # (a mode is off while it handles a call)
+                return s, norm(s)
+        if func is toward:
+            if diff.toward_ok(*args):
+                self.routed += 1
+                return diff.toward(*args)
+            return func(*args)
         if func is F.linear:
             x, w = args[0], args[1]
             b = args[2] if len(args) > 2 else kwargs.get("bias")

@@ -114,7 +114,7 @@ class ShardedAdamW:
                 self._owner[id(p)] = b
                 if direct_grads and p.is_cuda and (p.dtype == torch.float32 or (p.dtype == torch.bfloat16 and p.dim() == 2)):
                     self._sink[id(p)] = view
-                    if p.dim() == 2:
+                    if p.dim() == 2 or p.dtype == torch.float32:
                         p._grad_sink = view
                         p._grad_sink_used = True   # until the first zero_grad hands the slot out
                 if self.overlap:
@@ -219,7 +219,7 @@ class ShardedAdamW:
                 for p, view, d in zip(b.params, b.grad_views, direct):
                     if d:
                         p.grad = view
-                        if p.dim() == 2:
+                        if hasattr(p, "_grad_sink"):
                             # The slot may be overwritten while it holds these zeros: while the view's counter of
                             # in-place writes stands where it stands now (``ops.differentiable._free_sink``; writes
                             # through ``p.grad.data`` have a counter of their own).

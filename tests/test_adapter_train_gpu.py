@@ -506,3 +506,74 @@ def test_computed_fp32_weights_are_not_kept_for_the_backward(dev):
     assert ref() is None
     (y.float().square().sum() / 2).backward()
     assert float((p.grad - want * s.detach()).norm() / p.grad.norm()) < 1e-4
+
+
+# columns about a thread's chunks (2 048 a chunk, two or four of them), rows about a block's share
+@pytest.mark.parametrize("rows,H", [(16, 8), (17, 520), (33, 2048), (2049, 2056), (65, 4096), (40, 4104), (19, 8192)])
+@pytest.mark.parametrize("residual", [True, False])
+def test_residual_step_and_norm_in_one_launch(dev, rows, H, residual):
+    """``add_norm`` inside the mode against float64 of the same expression (the norm of the sum rounded to bf16): values and all gradients, with
+    and without a gradient that reaches the sum beside the norm.  bf16 results are off by 2^-8 of their row's largest term, the parameters' sums by
+    that of every row's."""
+    from eventgpt_amd.ops.intree_mode import InTreeLinear, add_norm
+    g = torch.Generator(device=dev).manual_seed(rows + H)
+    def rnd(*shape):
+        return torch.randn(*shape, device=dev, generator=g)
+    norm = torch.nn.LayerNorm(H).to(dev)
+    with torch.no_grad():
+        norm.weight.copy_(1 + 0.1 * rnd(H)), norm.bias.copy_(0.1 * rnd(H))
+    x, d = rnd(1, rows, H).requires_grad_(), rnd(1, rows, H).bfloat16().requires_grad_()
+    gs, gh = rnd(1, rows, H), rnd(1, rows, H).bfloat16()
+    with InTreeLinear() as mode:
+        s, h = add_norm(x, d, norm)
+    assert mode.routed == 1 and type(h.grad_fn).__name__ == "_AddLayerNormBackward"
+    torch.autograd.backward([s, h] if residual else [h], [gs, gh] if residual else [gh])
+    assert torch.equal(s, x + d)
+    x64, w, b = s.detach().bfloat16().double().requires_grad_(), norm.weight.detach().bfloat16().double(), norm.bias.detach().bfloat16().double()
+    w.requires_grad_(), b.requires_grad_()
+    want = F.layer_norm(x64, (H,), w, b, norm.eps)
+    want.backward(gh.double())
+    def close(got, ref, size):
+        assert bool(((got.double() - ref).abs() <= 2.0 ** -8 * size + 1e-6).all()), float(((got.double() - ref).abs() / (size + 1e-9)).max())
+    close(h, want.detach(), want.detach().abs())
+    ref = x64.grad + (gs.double() if residual else 0)
+    close(x.grad, ref, x64.grad.abs().amax(-1, keepdim=True) * 2.0 ** -8)
+    close(d.grad, ref, ref.abs() + x64.grad.abs().amax(-1, keepdim=True) * 2.0 ** -8)
+    close(norm.weight.grad, w.grad, 2.0 ** -8 * (gh.double().abs() * 5).sum((0, 1)))
+    close(norm.bias.grad, b.grad, 2.0 ** -8 * gh.double().abs().sum((0, 1)))
+
+
+@pytest.mark.parametrize("n", [8, 2048, 2056, 2048 * 2048 + 8])
+def test_step_toward_the_output_in_one_launch(dev, n):
+    from eventgpt_amd.ops.intree_mode import InTreeLinear, toward
+    g = torch.Generator(device=dev).manual_seed(n)
+    base, y = torch.randn(n, device=dev, generator=g), torch.randn(n, device=dev, generator=g).bfloat16().requires_grad_()
+    alpha = torch.nn.Parameter(torch.tensor(0.3, device=dev))
+    with InTreeLinear() as mode:
+        out = toward(base, y, alpha)
+        plain = toward(base.requires_grad_(), y, alpha)              # rows that need a gradient stay with the expression
+    assert mode.routed == 1 and type(out.grad_fn).__name__ == "_TowardBackward" and type(plain.grad_fn).__name__ == "AddBackward0"
+    gy = torch.randn(n, device=dev, generator=g)
+    out.backward(gy)
+    b, t = base.detach().double(), y.detach().double()
+    want, terms = b + alpha.detach().double() * (t - b), gy.double() * (t - b)
+    assert bool(((out.double() - want).abs() <= 2.0 ** -22 * (b.abs() + t.abs())).all())
+    assert torch.equal(y.grad, (gy * alpha.detach()).bfloat16())
+    assert abs(float(alpha.grad) - float(terms.sum())) <= 64 * 2.0 ** -24 * float(terms.abs().sum()) + 1e-6      # (sums of up to 64 in a row)
+
+
+def test_parts_of_a_block_that_is_listened_to_are_called_whole(dev):
+    """Hooks on a norm or on the output projection see their calls inside the mode; the loss is the same but for roundings."""
+    from eventgpt_amd.align.adapters import create_adapter
+    from eventgpt_amd.ops.intree_mode import InTreeLinear
+    torch.manual_seed(3)
+    m, h = create_adapter(4, 512, num_heads=1, ffn_dim=256).to(dev).eval(), torch.randn(4, 16, 512, device=dev)
+    def loss():
+        with torch.autocast("cuda", dtype=torch.bfloat16), InTreeLinear():
+            return float(m.compute_loss(h, h + 0.1 * h.roll(1, 0))["total_loss"].detach())
+    seen, quiet = [], loss()
+    hooks = [part.register_forward_hook(lambda part, *a: seen.append(type(part).__name__)) for part in (m.output_proj, m.layers[0]["ffn_norm"])]
+    assert abs(loss() - quiet) < 1e-2 * quiet and seen == ["LayerNorm", "Sequential"]
+    for hook in hooks:
+        hook.remove()
+    assert loss() == quiet and len(seen) == 2
