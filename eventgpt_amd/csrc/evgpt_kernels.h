@@ -149,6 +149,7 @@ void launch_event_raster(const int* x, const int* y, const int* p, int n_events,
                          int H, int W, int* keys, unsigned char* img, int mode, hipStream_t st);
 // how an event stream is counted by sorting (log_rows < 0: not), and the bytes of its scratch memory
 struct EventVoxelPlan { int log_rows, bands, chunks; size_t rec_bytes, span_bytes, range_bytes, off_bytes; };
+void launch_copy_words(const int* src, int* dst, long long n, hipStream_t st);      // (src may be pinned host memory; both on 16 bytes)
 EventVoxelPlan event_voxel_plan(int n, int bins, int H, int W);
 void launch_event_voxel_sorted(const int* x, const int* y, const int* p, const long long* t, int n, int bins, int H, int W,
                                const EventVoxelPlan& plan, unsigned char* work, int* out_hist, float* out_vox, int signed_mode,

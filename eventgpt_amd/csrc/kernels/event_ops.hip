@@ -60,6 +60,19 @@ void launch_event_raster(const int* x, const int* y, const int* p, int n_events,
   hipLaunchKernelGGL(raster_colorize_kernel, dim3(cb), dim3(256), 0, st, keys, img, n_pix, mode);
 }
 
+// Words out of pinned host memory, a 16-byte read a lane so that the bus has many of them at once.  (A copy command for them takes 11 us at 80 KB.)
+__global__ __launch_bounds__(256) void copy_words_kernel(const int* __restrict__ src, int* __restrict__ dst, long long n) {
+  const long long quads = n / 4;
+  for (long long i = blockIdx.x * 256ll + threadIdx.x; i < quads; i += gridDim.x * 256ll)
+    reinterpret_cast<i32x4_t*>(dst)[i] = reinterpret_cast<const i32x4_t*>(src)[i];
+  if (blockIdx.x == 0 && threadIdx.x < (n & 3)) dst[quads * 4 + threadIdx.x] = src[quads * 4 + threadIdx.x];
+}
+void launch_copy_words(const int* src, int* dst, long long n, hipStream_t st) {
+  if (n <= 0) return;
+  const long long blocks = (n / 4 + 255) / 256;
+  hipLaunchKernelGGL(copy_words_kernel, dim3(static_cast<unsigned>(blocks > 512 ? 512 : (blocks < 1 ? 1 : blocks))), dim3(256), 0, st, src, dst, n);
+}
+
 // Frames of a packed stream (x | y << 15 | positive << 30, one word an event) as one code a pixel: 0 untouched, 1 positive, 2
 // negative.  A block owns some rows of one slice in LDS and scans the slice's events, so nothing is filled beforehand, no
 // atomic leaves the CU and what the preprocessing reads is a third of an RGB frame.  Bound by the passes over LDS and the scan's

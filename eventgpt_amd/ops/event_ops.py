@@ -199,7 +199,7 @@ def _packed(events: dict):
     if any(c.ndim != 1 or c.size != t.size or c.dtype.kind not in "iub" for c in cols) or t.ndim != 1 or t.dtype.kind not in "iuf":
         return None
     try:
-        out = hip.raw.pack_events(*(torch.from_numpy(np.require(c, requirements="CAW")) for c in cols))
+        out = hip.raw.pack_events(*(torch.from_numpy(np.require(c, requirements="CAW")) for c in cols), True)
     except (TypeError, ValueError):   # a dtype or byte order torch does not have
         return None
     return (out[0], tuple(out[1].tolist())) if out else None
@@ -209,8 +209,8 @@ def event_frames_gpu(events: dict, device, n_frames: int = 5, size: int = CLIP_I
                      conflict: str = "last") -> Tuple[list, torch.Tensor]:
     """Host event dict -> ``([H, W], bf16 [T,3,size,size])`` on the GPU.  Integer streams go up as one word an event
     (polarity and coordinates; timestamps play no part in equal-count slices); other streams, images and sizes, and a
-    stream under capture, take the general ops.  The copy is a plain blocking one: from pinned blocks a call is 31 us
-    instead of 43 in a fresh process, but 107 after other work in it, since a pool of them grows with the calls in flight."""
+    stream under capture, take the general ops.  The words are packed into pinned memory of this thread and read from there by
+    the device, so a call does not wait for its copy."""
     dev = torch.device(device)
     packed = None
     if dev.type == "cuda" and not torch.cuda.is_current_stream_capturing() and _may_pack(events, n_frames, size):
@@ -221,7 +221,7 @@ def event_frames_gpu(events: dict, device, n_frames: int = 5, size: int = CLIP_I
         rh, rw = cp.resized_shape(h, w, size)
         ksv = cp.resample_table(h, rh).weight.shape[1] if rh != h else 1
         if rh >= size and rw >= size and hip.raw.event_codes_ok(words.numel(), n_frames, h, w, rh, ksv):
-            words = words.to(dev)
+            words = hip.raw.upload_words(words, torch.cuda.current_device() if dev.index is None else dev.index)
             return [h, w], hip.raw.event_clip_frames(words, n_frames, h, w, {"last": 0, "negative": 1}[conflict],
                                                      *_with_crop(h, w, size, words.device))
     ev = events_to_device(events, device)

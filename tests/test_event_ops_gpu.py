@@ -256,3 +256,29 @@ def test_streams_that_do_not_pack_stay_on_the_general_ops(dev):
     for v in locked.values():
         v.flags.writeable = False
     assert torch.equal(eo._packed(locked)[0], eo._packed(good)[0])
+
+
+def test_words_in_flight_and_words_that_are_held_are_not_written_over(dev):
+    """Clips one after another without a wait, of growing and shrinking length, on two streams and from two threads: each is what its
+    events give.  Packed words that a caller still holds stay as they are while others are packed."""
+    import threading
+    from eventgpt_amd.ops import event_ops as eo
+    clips = [_host_stream(n, 97 + i, 130, np.int32, np.int8, seed=i) for i, n in enumerate((20_000, 70_000, 5_000, 200_000, 20_001, 7))]
+    want = [eo.clip_preprocess_gpu(eo.rasterize_gpu(eo.events_to_device(ev, dev), 5, (97 + i, 130))) for i, ev in enumerate(clips)]
+    torch.cuda.synchronize()
+    bad = []
+    def go():
+        streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+        got = []
+        for turn in range(3):
+            for i, ev in enumerate(clips):
+                with torch.cuda.stream(streams[(i + turn) % 2]):
+                    got.append((i, eo.event_frames_gpu(ev, dev)[1]))
+        torch.cuda.synchronize()
+        bad.extend(i for i, px in got if not torch.equal(px, want[i]))
+    threads = [threading.Thread(target=go) for _ in range(2)]
+    [t.start() for t in threads], [t.join() for t in threads], go()
+    assert not bad
+    held = [eo._packed(ev)[0] for ev in clips]
+    for words, ev in zip(held, clips):
+        assert np.array_equal(words.numpy(), ev["x"] | ev["y"] << 15 | (ev["p"] != 0).astype(np.int32) << 30)
