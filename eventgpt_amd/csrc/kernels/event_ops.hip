@@ -589,19 +589,20 @@ void launch_event_voxel_sorted(const int* x, const int* y, const int* p, const l
   if (!by_count) hipLaunchKernelGGL(voxel_span_kernel, dim3(VS_SPANS), dim3(1024), 0, st, t, n, span);
   hipLaunchKernelGGL(voxel_sort_kernel, dim3(plan.chunks), dim3(VS_THREADS), 0, st, a);
   const size_t smem = static_cast<size_t>(2) * (1 << plan.log_rows) * W * sizeof(int);
-  const auto count = [&](auto kernel, int threads) {
-    static bool attr_set = false;                       // (one a kernel)
+  const auto count = [&](auto threads) {
+    constexpr int T = decltype(threads)::value;
+    static bool attr_set = false;                       // (one a number of threads: the kernels' types are the same)
     if (!attr_set) {
-      hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024);  // (W = 19 200)
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&voxel_count_kernel<T>), hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024);  // (W = 19 200)
       attr_set = true;
     }
-    hipLaunchKernelGGL(kernel, dim3(plan.bands, bins), dim3(threads), smem, st, a, out_hist, out_vox, signed_mode);
+    hipLaunchKernelGGL(voxel_count_kernel<T>, dim3(plan.bands, bins), dim3(T), smem, st, a, out_hist, out_vox, signed_mode);
   };
   // two blocks a CU and more of few events each: half as many threads, so that all are resident at once (600 blocks, 1e6 events 31.4 ->
   // 28.6 us, 2.4e6 40.2 -> 38.8); with more the block of the busiest band is
   // waited for, and its waves count (1e7 77.7 with 512 threads, 75.6 with 1 024; 4.3e6 0.98 to 1.03 of the time with 512)
-  if (plan.bands * bins >= 512 && n / (plan.bands * bins) < 5000) count(&voxel_count_kernel<512>, 512);
-  else count(&voxel_count_kernel<1024>, 1024);
+  if (plan.bands * bins >= 512 && n / (plan.bands * bins) < 5000) count(std::integral_constant<int, 512>{});
+  else count(std::integral_constant<int, 1024>{});
 }
 
 // --------------------------------------------------------- CLIP preprocessing
