@@ -371,6 +371,22 @@ def test_attention_backward(dev, D, H, Hkv, Sq, Sk, causal):
     _close(v.grad, dv, 3e-2, 3e-2)
 
 
+# edges of the streamed tiles (32 rows of 128 values, 64 of 64) and of the blocks (64), more keys than queries, shared key heads
+@pytest.mark.parametrize("D,H,Hkv,Sq,Sk,causal", [
+    (128, 2, 2, 1, 1, True), (128, 2, 2, 31, 31, True), (128, 2, 1, 32, 32, True), (128, 4, 2, 33, 65, True), (128, 2, 2, 97, 97, False),
+    (128, 2, 2, 64, 161, True), (128, 3, 1, 129, 129, True), (64, 2, 2, 63, 63, True), (64, 4, 2, 65, 129, True), (64, 2, 2, 128, 1, False)])
+def test_attention_backward_tile_edges(dev, D, H, Hkv, Sq, Sk, causal):
+    from eventgpt_amd.ops import hip
+    q, go = _rand(2, Sq, H, D, dev=dev), _rand(2, Sq, H, D, dev=dev, seed=3)
+    k, v = _rand(2, Sk, Hkv, D, dev=dev, seed=1), _rand(2, Sk, Hkv, D, dev=dev, seed=2)
+    q_offset = Sk - Sq if causal else 0
+    o, lse = hip.raw.attention_fwd_lse(q, k, v, causal, D ** -0.5, q_offset)
+    got = hip.raw.attention_bwd(q, k, v, o, go, lse, causal, D ** -0.5, q_offset)
+    _, *want = _attn_ref_grads(q, k, v, go, causal, q_offset)
+    for g, w in zip(got, want):
+        _close(g, w, 3e-2, 3e-2)
+
+
 def test_attention_lse(dev):
     from eventgpt_amd.ops import hip
     q, k, v = _rand(1, 100, 2, 128, dev=dev), _rand(1, 100, 2, 128, dev=dev, seed=1), _rand(1, 100, 2, 128, dev=dev, seed=2)
