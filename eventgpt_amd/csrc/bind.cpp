@@ -586,11 +586,17 @@ void fill_strides_bshd(const Tensor& t, long long* s) {
 }
 
 // q [B,Sq,Hq,D], k/v [B,Sk,Hkv,D] (any strides with contiguous D)
-Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, bool causal, double scale,
+Tensor attention(const Tensor& q, const Tensor& k_in, const Tensor& v_in, bool causal, double scale,
                  int64_t q_offset) {
-  TORCH_CHECK(q.is_cuda() && q.scalar_type() == at::kBFloat16 && k.scalar_type() == at::kBFloat16 &&
-              v.scalar_type() == at::kBFloat16, "attention: bf16 GPU tensors required");
-  TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && v.dim() == 4);
+  TORCH_CHECK(q.is_cuda() && q.scalar_type() == at::kBFloat16 && k_in.scalar_type() == at::kBFloat16 &&
+              v_in.scalar_type() == at::kBFloat16, "attention: bf16 GPU tensors required");
+  TORCH_CHECK(q.dim() == 4 && k_in.dim() == 4 && v_in.dim() == 4);
+  // (key tiles go to LDS 16 bytes at a time, rows of a tile within 31 bits of each other)
+  const auto rows16 = [](const Tensor& t) {
+    return t.stride(3) == 1 && ((t.size(0) > 1 && t.stride(0) % 8) || t.stride(1) >= (1ll << 24) || reinterpret_cast<uintptr_t>(t.data_ptr()) % 16)
+               ? t.clone(at::MemoryFormat::Contiguous) : t;
+  };
+  const Tensor k = rows16(k_in), v = rows16(v_in);
   const int64_t B = q.size(0), Sq = q.size(1), Hq = q.size(2), D = q.size(3);
   const int64_t Sk = k.size(1), Hkv = k.size(2);
   TORCH_CHECK(D == 64 || D == 128, "attention: head_dim must be 64 or 128");
@@ -1365,7 +1371,6 @@ void gemm_split_major(int64_t on) { evgpt::gemm_split_major((int)on); }
 void attn_force_groups(int64_t g) { evgpt::attn_force_groups((int)g); }
 void gemm_enable_tail_splitk(bool on) { evgpt::gemm_enable_tail_splitk(on); }
 void attn_enable_wide(int64_t mode) { evgpt::attn_enable_wide((int)mode); }
-void attn_wide4_min_rows(int64_t rows) { evgpt::attn_wide4_min_rows((int)rows); }
 void gemm_force_splitk(int64_t sk) { evgpt::gemm_force_splitk((int)sk); }
 void gemv_force_ks(int64_t ks) { evgpt::gemv_force_ks((int)ks); }
 
@@ -1872,7 +1877,6 @@ TORCH_LIBRARY(evgpt, m) {
   m.def("attn_force_groups(int groups) -> ()", &attn_force_groups);
   m.def("gemm_enable_tail_splitk(bool on) -> ()", &gemm_enable_tail_splitk);
   m.def("attn_enable_wide(int mode) -> ()", &attn_enable_wide);
-  m.def("attn_wide4_min_rows(int rows) -> ()", &attn_wide4_min_rows);
   m.def("gemm_force_splitk(int sk) -> ()", &gemm_force_splitk);
   m.def("gemv_force_ks(int ks) -> ()", &gemv_force_ks);
   m.def("decode_gemv_partial(Tensor w, Tensor xin, Tensor(a!) out_f32) -> ()", &decode_gemv_partial);

@@ -109,8 +109,7 @@ void launch_sumsq(const void* x, bool bf16, long long n, float* part, float* acc
 int gemm_argmax_partials(int M, int N);
 void gemm_force_config(int cfg);  // -1 = automatic; for tuning runs
 void attn_force_groups(int g);      // key-tile groups per 64-row attention block: 0 by shape (default), 1, 2
-void attn_wide4_min_rows(int rows); // fewest query rows that take the 128-row wide blocks
-void attn_enable_wide(int mode);   // 128-query-row prefill attention: 0 never, 1 by shape (default), 2 always
+void attn_enable_wide(int mode);   // 256-query-row prefill attention: 0 never, 1 by shape (default), 2 always; 3: 128 rows always
 void gemm_group_m(int g);          // row tiles per group of the kernels' tile walk (0: whole columns)
 void gemm_split_major(int on);     // split-K workgroups of the 4-wave kernel ordered split by split
 void gemm_persist_256(bool on);   // the 256 x 256 kernels walk several tiles per workgroup (default on)

@@ -2,10 +2,9 @@
 // head_dim 128), speculative-verify batches (causal with an offset into a long
 // cache) and the ViT encoder (non-causal, head_dim 64, 577 tokens).
 //
-// One block = 4 waves = 64 query rows of one (batch, head); each wave owns 16
-// rows.  K/V tiles of 64 keys are staged through LDS (register-staged: the
-// global loads of tile t+1 are issued before the MFMAs of tile t and written to
-// LDS after the barrier).  The score tile is computed TRANSPOSED,
+// One block = 4 or 8 waves = 64 or 128 query rows of one (batch, head); each wave owns 16
+// rows.  K/V tiles of 64 keys go straight into LDS, the next one while a tile is
+// multiplied.  The score tile is computed TRANSPOSED,
 //     S^T[key][q] = K · Q^T        (K rows = MFMA A operand, Q^T = B operand)
 // so that the query index lives on the lane (lane & 15) and a lane's 16
 // accumulator values are 16 different keys of ONE query.  Consequences:
@@ -18,6 +17,8 @@
 //   * rescaling O by exp(m_old - m_new) is a per-lane scalar multiply.
 // LDS images are XOR-swizzled at 16-byte-chunk granularity so both the row
 // reads (ds_read_b128) and the transposed reads spread over the banks.
+#include <type_traits>
+
 #include "common.h"
 #include "attn_common.h"
 #include "../evgpt_kernels.h"
@@ -44,6 +45,12 @@ __device__ __forceinline__ float score_max(const f32x4_t (&st)[4]) {
   a = maximum3(a, st[3][2], st[3][3]);
   a = __builtin_elementwise_maximum(a, b);
   return max_of_quads(a);
+}
+__device__ __forceinline__ float score_max(const f32x4_t (&st)[2]) {
+  float a = maximum3(st[0][0], st[0][1], st[0][2]);
+  const float b = maximum3(st[0][3], st[1][0], st[1][1]);
+  a = maximum3(a, st[1][2], st[1][3]);
+  return max_of_quads(__builtin_elementwise_maximum(a, b));
 }
 struct AttnParams {
   const bf16_t* q; const bf16_t* k; const bf16_t* v; bf16_t* o;
@@ -83,30 +90,43 @@ __device__ __forceinline__ float head_gate(const AttnParams& p, long long row, i
   return 1.f / (1.f + __expf(-bf16_to_f32(p.gate[row * p.gate_ld + h])));
 }
 
+__device__ __forceinline__ void attn_buffer_to_lds16(const unsigned char* src, int bytes, unsigned char* lds, int voff) {
+  const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(src), 0, bytes, 0x00020000);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (void __attribute__((address_space(3)))*)lds, 16, voff, 0, 0, 0);
+}
+
 // GROUPS = 2: the block is two such groups of 4 waves over the SAME 64 query rows; group 0 takes the
 // even key tiles of the block's range and group 1 the odd ones, each through its own K / V tile
 // buffers, and group 1's running (max, sum, O) is merged into group 0's at the end through LDS.  A
 // few hundred query rows of a few heads are fewer blocks than CUs, each a serial chain over its key
 // tiles; two groups halve the chain and double the waves (used for the ViT, see launch_attn_prefill).
+// WAVES = 8: 128 query rows share the tiles, so that a CU has twice the waves in the same LDS.
+// Bound by the chain of a tile (scores, maxima, exponentials, weights times values) and by LDS reads of twice the matrix time, which
+// other waves fill.  Tiles through registers behind two barriers / straight into LDS behind one, us: 636 causal rows, 32 heads of 128
+// 22.8 / 17.8; 300 10.6 / 8.3; 1 024 39.3 / 28.4; 100 rows over 300 keys, 8 key heads 10.8 / 8.0; one frame of 577 tokens, 16 heads of
+// 64 9.2 / 8.3, two 15.9 / 13.5; ITEMS, eight prompts of 342 to 685, 32 heads 77 / 67.  With D = 128 tiles of 32 keys, five blocks a CU instead
+// of two, 23 where these take 18, in 170 registers instead of 150 20; ITEMS of 200 and fewer rows 2 to 10 % ahead with them, longer
+// ones as much behind.
 // WP: the softmax weights enter the second product as two bf16 parts (16 mantissa bits) instead of one.
 // ITEMS: block x takes the query rows, keys and position of an entry of `items`, so runs of any lengths and sequences share
 // a launch.  Eight prompts of 342 to 682 tokens, 32 heads of 128: one launch a prompt 170 us a layer, one for all 80; 32 prompts of
 // 200, 16 heads: 52 (148 with the 64-column blocks of attn_chunk.hip).
-template <int D, bool CAUSAL, bool SPLIT = false, int GROUPS = 1, bool WP = false, bool ITEMS = false>
-__global__ __launch_bounds__(256 * GROUPS) void attn_prefill_kernel(AttnParams p) {
+template <int D, bool CAUSAL, bool SPLIT = false, int GROUPS = 1, bool WP = false, bool ITEMS = false, int WAVES = 4>
+__global__ __launch_bounds__(64 * WAVES * GROUPS, WAVES == 8 || GROUPS == 2 ? 4 : 2) void attn_prefill_kernel(AttnParams p) {
+  constexpr int TR = D == 128 && GROUPS == 2 ? 32 : 64;       // keys of a tile
   constexpr int CPR = D / 8;                  // 16-byte chunks per row
-  constexpr int TILE_BYTES = TK * D * 2;
-  constexpr int LD_PER_THREAD = TK * CPR / 256;  // chunks each thread stages per tile
+  constexpr int TILE_BYTES = TR * D * 2;
+  constexpr int NIW = TILE_BYTES / 1024 / WAVES;  // 1 KB staging instructions per wave and tile
   constexpr int KS = D / 32;                  // k-steps of the QK^T product
   constexpr int DT = D / 16;                  // 16-wide output column tiles
+  constexpr int NT = TR / 16;                 // 16-key sub-tiles
   static_assert(GROUPS == 1 || GROUPS == 2, "one or two groups of four waves");
-  static_assert(GROUPS == 1 || (DT * 4 + 2) * 256 * 4 <= GROUPS * 2 * TILE_BYTES, "merge buffer fits the tile buffers");
-  __shared__ __attribute__((aligned(16))) unsigned char lds[GROUPS * 2 * TILE_BYTES];
-  const int grp = GROUPS == 1 ? 0 : static_cast<int>(threadIdx.x >> 8);
-  unsigned char* k_lds = lds + grp * 2 * TILE_BYTES;
-  unsigned char* v_lds = k_lds + TILE_BYTES;
+  static_assert(GROUPS == 1 || (DT * 4 + 2) * 256 * 4 <= GROUPS * 4 * TILE_BYTES, "merge buffer fits the tile buffers");
+  __shared__ __attribute__((aligned(16))) unsigned char lds[GROUPS * 4 * TILE_BYTES];
+  const int grp = GROUPS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * WAVES));
+  unsigned char* ring = lds + grp * 4 * TILE_BYTES;       // [2][K | V]
 
-  const int tid = threadIdx.x & 255, lane = tid & 63, wid = tid >> 6;   // within the group
+  const int tid = threadIdx.x % (64 * WAVES), lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);   // within the group
   const int fr = lane & 15, g = lane >> 4;
   const int b = blockIdx.z, h = blockIdx.y;
   const int hk = h / (p.Hq / p.Hkv);
@@ -124,7 +144,7 @@ __global__ __launch_bounds__(256 * GROUPS) void attn_prefill_kernel(AttnParams p
     p.q += row0 * p.q_ss; p.o += row0 * p.o_ss;
     p.k += static_cast<long long>(it[2]) * p.k_ss; p.v += static_cast<long long>(it[2]) * p.v_ss;
   }
-  const int qb0 = SPLIT || ITEMS ? 0 : blockIdx.x * 64;  // first query row of the block
+  const int qb0 = SPLIT || ITEMS ? 0 : (CAUSAL && WAVES == 8 ? gridDim.x - 1 - blockIdx.x : blockIdx.x) * (16 * WAVES);  // first query row of the block
   const int qi = qb0 + wid * 16 + fr;        // this lane's query row
   const int qi_c = qi < p.Sq ? qi : p.Sq - 1;
 
@@ -137,16 +157,16 @@ __global__ __launch_bounds__(256 * GROUPS) void attn_prefill_kernel(AttnParams p
       qf[ks] = load_q(p, qp + ks * 32 + g * 8);
   }
 
-  const bf16_t* kbase = p.k + b * p.k_sb + hk * p.k_sh;
-  const bf16_t* vbase = p.v + b * p.v_sb + hk * p.v_sh;
+  const unsigned char* kbase = reinterpret_cast<const unsigned char*>(p.k + b * p.k_sb + hk * p.k_sh);
+  const unsigned char* vbase = reinterpret_cast<const unsigned char*>(p.v + b * p.v_sb + hk * p.v_sh);
 
   // keys this block needs: all of them, or up to its last query's diagonal
   int k_end = Sk;
   if (CAUSAL) {
-    const int last_q = min(qb0 + 63, p.Sq - 1);
+    const int last_q = min(qb0 + 16 * WAVES - 1, p.Sq - 1);
     k_end = min(Sk, last_q + q_off + 1);
   }
-  int ntiles = (k_end + TK - 1) / TK;
+  int ntiles = (k_end + TR - 1) / TR;
   int t_begin = 0;
   if (SPLIT) {
     const int per = (ntiles + p.nsplit - 1) / p.nsplit;
@@ -156,28 +176,27 @@ __global__ __launch_bounds__(256 * GROUPS) void attn_prefill_kernel(AttnParams p
   // waves whose 16 query rows are all padding only help staging the tiles
   const bool wave_active = qb0 + wid * 16 < p.Sq;
 
-  // Two register sets: the loads of tile t+2 are issued while tile t is computed, so a tile has
-  // two compute phases to arrive before it is written to LDS (with one set the write at the top
-  // of every iteration waited out most of an L2 round trip: 2.5 us per 64-key tile).
-  u32x4_t kreg[2][LD_PER_THREAD], vreg[2][LD_PER_THREAD];
-  auto prefetch = [&](u32x4_t (&kr)[LD_PER_THREAD], u32x4_t (&vr)[LD_PER_THREAD], int t) {
+  const int q_hi = min(qb0 + wid * 16 + 15, p.Sq - 1);       // last query row of this wave
+
+  // Tiles go straight into LDS (the swizzle applied to the source; rows past the last key are zeros from the descriptor's range
+  // check), the next one while a tile is multiplied, one barrier a tile.
+  const long long k_bytes = Sk > 0 ? 2ll * ((Sk - 1) * p.k_ss + D) : 0;
+  const long long v_bytes = Sk > 0 ? 2ll * ((Sk - 1) * p.v_ss + D) : 0;
+  int voff_k[NIW], voff_v[NIW];
 #pragma unroll
-    for (int i = 0; i < LD_PER_THREAD; ++i) {
-      const int idx = tid + i * 256;
-      const int row = idx / CPR, ch = idx % CPR;
-      int key = t * TK + row; key = key < Sk ? key : Sk - 1;
-      kr[i] = load16(kbase + static_cast<long long>(key) * p.k_ss + ch * 8);
-      vr[i] = load16(vbase + static_cast<long long>(key) * p.v_ss + ch * 8);
-    }
-  };
-  auto commit = [&](const u32x4_t (&kr)[LD_PER_THREAD], const u32x4_t (&vr)[LD_PER_THREAD]) {
+  for (int j = 0; j < NIW; ++j) {
+    const int idx = (wid * NIW + j) * 64 + lane, row = idx / CPR, ch = (idx % CPR) ^ swz<D>(row);
+    voff_k[j] = static_cast<int>((row * p.k_ss + ch * 8) * 2);
+    voff_v[j] = static_cast<int>((row * p.v_ss + ch * 8) * 2);
+  }
+  auto range = [](long long left) { return static_cast<int>(left < 0 ? 0 : (left > 0x7fffffff ? 0x7fffffff : left)); };
+  auto stage = [&](int buf, int t) {
+    unsigned char* kd = ring + buf * 2 * TILE_BYTES + wid * NIW * 1024;
+    const long long ka = 2ll * t * TR * p.k_ss, va = 2ll * t * TR * p.v_ss;
 #pragma unroll
-    for (int i = 0; i < LD_PER_THREAD; ++i) {
-      const int idx = tid + i * 256;
-      const int row = idx / CPR, ch = idx % CPR;
-      *reinterpret_cast<u32x4_t*>(k_lds + tile_off<D>(row, ch)) = kr[i];
-      *reinterpret_cast<u32x4_t*>(v_lds + tile_off<D>(row, ch)) = vr[i];
-    }
+    for (int j = 0; j < NIW; ++j) attn_buffer_to_lds16(kbase + ka, range(k_bytes - ka), kd + j * 1024, voff_k[j]);
+#pragma unroll
+    for (int j = 0; j < NIW; ++j) attn_buffer_to_lds16(vbase + va, range(v_bytes - va), kd + TILE_BYTES + j * 1024, voff_v[j]);
   };
 
   f32x4_t o[DT];
@@ -185,15 +204,17 @@ __global__ __launch_bounds__(256 * GROUPS) void attn_prefill_kernel(AttnParams p
   for (int i = 0; i < DT; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
 
-  auto compute = [&](int t) {
-    // ---- S^T tile: 4 sub-tiles of 16 keys
-    f32x4_t st[4];
+  auto compute = [&](int buf, int t) {
+    const unsigned char* k_lds = ring + buf * 2 * TILE_BYTES;
+    const unsigned char* v_lds = k_lds + TILE_BYTES;
+    // ---- S^T tile: sub-tiles of 16 keys
+    f32x4_t st[NT];
 #pragma unroll
-    for (int n = 0; n < 4; ++n) st[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int n = 0; n < NT; ++n) st[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)      // k-step outermost: four independent accumulators in turn
+    for (int ks = 0; ks < KS; ++ks)      // k-step outermost: independent accumulators in turn
 #pragma unroll
-      for (int n = 0; n < 4; ++n) {
+      for (int n = 0; n < NT; ++n) {
         const bf16x8_t kf = *reinterpret_cast<const bf16x8_t*>(
             k_lds + tile_off<D>(n * 16 + fr, ks * 4 + g));
         st[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[ks], st[n], 0, 0, 0);
@@ -203,12 +224,12 @@ __global__ __launch_bounds__(256 * GROUPS) void attn_prefill_kernel(AttnParams p
     // is positive, so the maximum commutes with it and exp2(s * scale - m * scale) is one fma and
     // one v_exp_f32 per score; keys are masked only in tiles that cross the diagonal or the end
     // of the keys; the accumulators (AGPRs) are rescaled only when some row's maximum moved.
-    const int key0 = t * TK + g * 4;
-    const int last_key = t * TK + TK - 1;
+    const int key0 = t * TR + g * 4;
+    const int last_key = t * TR + TR - 1;
     if (last_key > Sk - 1 || (CAUSAL && last_key > qb0 + wid * 16 + q_off)) {
       const int lim = CAUSAL ? min(Sk - 1, qi + q_off) : Sk - 1;  // last visible key
 #pragma unroll
-      for (int n = 0; n < 4; ++n)
+      for (int n = 0; n < NT; ++n)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           if (key0 + n * 16 + r > lim) st[n][r] = -INFINITY;
@@ -225,9 +246,9 @@ __global__ __launch_bounds__(256 * GROUPS) void attn_prefill_kernel(AttnParams p
     }
     const float ms = msafe * p.scale_log2e;
     float psum = 0.f;
-    unsigned int pk[4][2], pl[4][2];
+    unsigned int pk[NT][2], pl[NT][2];
 #pragma unroll
-    for (int n = 0; n < 4; ++n) {
+    for (int n = 0; n < NT; ++n) {
       float e[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) { e[r] = __builtin_amdgcn_exp2f(fmaf(st[n][r], p.scale_log2e, -ms)); psum += e[r]; }
@@ -243,7 +264,7 @@ __global__ __launch_bounds__(256 * GROUPS) void attn_prefill_kernel(AttnParams p
     // ---- O^T += V^T · P^T, two k-steps of 32 keys; slot (g, j) <-> key
     //      32s + 4g + j (j < 4) or 32s + 16 + 4g + (j - 4)
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
+    for (int s = 0; s < TR / 32; ++s) {
       u32x4_t pw = {pk[2 * s][0], pk[2 * s][1], pk[2 * s + 1][0], pk[2 * s + 1][1]};
       const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, pw);
       bf16x8_t pf_lo = pf;
@@ -273,20 +294,13 @@ __global__ __launch_bounds__(256 * GROUPS) void attn_prefill_kernel(AttnParams p
   const int first = t_begin + grp;
   const int n_mine = first < ntiles ? (ntiles - first + GROUPS - 1) / GROUPS : 0;
   const int n_iter = t_begin < ntiles ? (ntiles - t_begin + GROUPS - 1) / GROUPS : 0;
-  if (0 < n_mine) prefetch(kreg[0], vreg[0], first);
-  if (1 < n_mine) prefetch(kreg[1], vreg[1], first + GROUPS);
-  for (int k = 0; k < n_iter; k += 2) {
-    __syncthreads();
-    if (k < n_mine) commit(kreg[0], vreg[0]);
-    __syncthreads();
-    if (k + 2 < n_mine) prefetch(kreg[0], vreg[0], first + GROUPS * (k + 2));
-    if (wave_active && k < n_mine) compute(first + GROUPS * k);
-    if (k + 1 >= n_iter) break;
-    __syncthreads();
-    if (k + 1 < n_mine) commit(kreg[1], vreg[1]);
-    __syncthreads();
-    if (k + 3 < n_mine) prefetch(kreg[1], vreg[1], first + GROUPS * (k + 3));
-    if (wave_active && k + 1 < n_mine) compute(first + GROUPS * (k + 1));
+  if (0 < n_mine) stage(0, first);
+  for (int k = 0; k < n_iter; ++k) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();                             // the tile is there, and every wave is done with the one before it
+    if (k + 1 < n_mine) stage((k + 1) & 1, first + GROUPS * (k + 1));
+    const int t = first + GROUPS * k;
+    if (wave_active && k < n_mine && !(CAUSAL && t * TR > q_hi + q_off)) compute(k & 1, t);      // (else nothing of it is visible)
   }
 
   // ---- finalise: l is a per-lane partial over this lane's key slots
@@ -346,23 +360,18 @@ __global__ __launch_bounds__(256 * GROUPS) void attn_prefill_kernel(AttnParams p
   }
 }
 
-// Same computation for long query ranges: one block = 128 query rows, each wave owns TWO 16-row
+// Same computation for long query ranges: one block = 256 query rows, each wave owns TWO 16-row
 // query tiles, so every K fragment (ds_read_b128) and every V^T fragment (two transposing reads)
 // feeds two MFMAs instead of one -- with 16 rows per wave the kernel above reads 32 KB of LDS
 // per wave and key tile for 32 MFMAs and is bound by the LDS pipe.  K / V tiles are staged
 // straight into LDS (buffer_load ... lds, swizzle applied to the per-lane source offset; keys past
 // the end come back as zeros from the descriptor's range check) into a ring of AW_STAGES tiles:
 // loads are in flight while other tiles are computed, and no staging registers are held.
-__device__ __forceinline__ void attn_buffer_to_lds16(const unsigned char* src, int bytes, unsigned char* lds, int voff) {
-  const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(src), 0, bytes, 0x00020000);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (void __attribute__((address_space(3)))*)lds, 16, voff, 0, 0, 0);
-}
-
 constexpr int AW_STAGES = 4;   // K / V tiles in the LDS ring: three are read between two barriers, one is on its way
 
-// AW_WAVES = 8: 256 query rows per block (long prompts); 4: 128 rows (a few hundred tokens, the ViT)
-// QT: 16-row query tiles per wave (2: every K / V fragment feeds two MFMAs; 1: twice the blocks)
-template <int D, bool CAUSAL, int AW_WAVES, int QT = 2, bool WP = false>
+// QT: 16-row query tiles per wave (2: every K / V fragment feeds two MFMAs); 256 query rows per block
+constexpr int AW_WAVES = 8, QT = 2;
+template <int D, bool CAUSAL, bool WP = false>
 __global__ __launch_bounds__(AW_WAVES * 64) void attn_prefill_wide_kernel(AttnParams p) {
   constexpr int CPR = D / 8;
   constexpr int TILE_BYTES = TK * D * 2;
@@ -671,10 +680,8 @@ void launch_attn_items(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf16_t
 
 static int g_attn_groups = 0;  // key-tile groups per 64-row block: 0 = by shape, 1 / 2 = forced (tests, tuning)
 void attn_force_groups(int g) { g_attn_groups = g; }
-static int g_attn_wide = 1;   // 0 = never, 1 = by shape, 2 = whenever the strides allow (tests, tuning)
-static int g_attn_wide4_min_rows = 1400;  // fewest query rows that take the 128-row blocks (mode 1): measured crossover 1300-1500 (1024 rows 18.3 vs 18.0 ms per 7B prefill, 1500 rows 25.9 vs 26.2; 636 rows 12.6 vs 12.3, ViT frame 2.50 vs 2.24)
+static int g_attn_wide = 1;   // the ring-staged blocks: 0 never, 1 by shape, 2 whenever the strides allow; 3: 128-row blocks of one tile a wave (tests, tuning)
 void attn_enable_wide(int mode) { g_attn_wide = mode; }
-void attn_wide4_min_rows(int rows) { g_attn_wide4_min_rows = rows; }
 
 void launch_attn_prefill(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf16_t* o,
                          const long long* strides /*12: q,k,v,o x (b,s,h)*/, const int* kv_len,
@@ -705,38 +712,61 @@ void launch_attn_prefill(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf16
     return;
   }
   dim3 block(256);
-  // Wide blocks (two query tiles per wave, K / V ring in LDS): 256 rows once those fill the chip,
-  // 128 rows for anything from two such blocks up; K / V must allow 16-byte row chunks
+  // Three block shapes: 64 rows (four waves), 128 rows (eight), and the ring-staged 256 rows of two tiles a wave, whose K / V must allow
+  // 16-byte row chunks.  us of 64 / 128 / 256 rows, causal heads of 128 unless noted; with D = 128 there are 512, 512 and 256 blocks at a time:
+  //  * 256 rows where they are one round, nearly full: 2 x 836, 32 heads 40 / 32 / 32; 1850 64 / 61 / 59; 4096, 16 heads 152 / 129 / 118;
+  //    4 x 836, 16 heads of 64, no mask 31 / 27 / 25
+  //  * 64 rows up to 640 blocks of them: 636, 32 heads 18 / 20 / 23; 1200 35 / 39 / 40; 2048, 16 heads 43 / 64 / 65; 4096, 8 heads 82 / 95 /
+  //    118.  Heads of 64 without a mask to 1056: 4 x 577, 16 heads 18 / 20 / 20; 4 x 1200 45 / 46 / 61
+  //  * beyond, 128 rows where they are one round (1400, 32 heads 45 / 43 / 44; 3 x 577 33 / 26 / 32; 1500, 2 x 16 heads 53 / 44 / 51) or
+  //    256 pad a tenth more rows (8 x 577 78 / 58 / 66; 8 x 836 116 / 93 / 99; 16 heads, 8 x 1200, which they don't, 96 / 88 / 88; 32
+  //    184 / 164 / 155), and for heads of 64 without a mask (40 x 577, 16 heads 123 / 107 / 135; 8 x 1600 133 / 129 / 151)
+  //  * 256 rows for the rest: 3000, 32 heads 129 / 139 / 93; 4643 265 / 256 / 203
   const bool strides_ok = strides[4] % 8 == 0 && strides[7] % 8 == 0 && strides[4] * 2ll * Sk < (1ll << 31) &&
                           strides[7] * 2ll * Sk < (1ll << 31);
-  const long long blocks256 = static_cast<long long>((Sq + 255) / 256) * Hq * B;
-  int wide = 0;             // waves per block of the ring-staged kernel (0: not used)
-  constexpr int qt = 2;     // query tiles per wave
-  if (strides_ok && g_attn_wide >= 1) {
-    if (Sq >= 512 && blocks256 >= 256) wide = 8;
-    else if (Sq >= g_attn_wide4_min_rows || g_attn_wide == 2) wide = 4;
-  }
-  if (wide) {
-    const int rows = wide * 16 * qt;
-    dim3 wgrid(Hq, (Sq + rows - 1) / rows, B), wblock(wide * 64);
-    auto go = [&](auto kern, int d) {
-      const int smem = AW_STAGES * 2 * TK * d * 2;
-      static bool attr_set = false;     // one flag per kernel: the lambda is instantiated per kernel type
-      if (!attr_set) {
-        hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-        attr_set = true;
-      }
-      hipLaunchKernelGGL(kern, wgrid, wblock, smem, st, p);
+  const long long heads = static_cast<long long>(Hq) * B, n64 = (Sq + 63) / 64 * heads, n128 = (Sq + 127) / 128 * heads,
+                  n256 = (Sq + 255) / 256 * heads;
+  const bool vit = D == 64 && !causal;
+  int rows = 64;
+  if (g_attn_wide == 2 || (g_attn_wide == 1 && n256 > 224 && n256 <= 256)) rows = 256;
+  else if (g_attn_wide == 3) rows = 128;
+  else if (n64 > (vit ? 1056 : 640))
+    rows = vit || (n128 <= 512 && Sq <= 1792) || n256 * 20 >= n128 * 11 || g_attn_wide == 0 ? 128 : 256;
+  if (rows == 256 && !strides_ok) rows = 128;
+  if (rows == 256) {
+    auto go = [&](auto d, auto masked, auto parts) {
+      constexpr auto kern = &attn_prefill_wide_kernel<decltype(d)::value, decltype(masked)::value, decltype(parts)::value>;
+      constexpr int smem = AW_STAGES * 2 * TK * decltype(d)::value * 2;
+      static const bool attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem) == hipSuccess;
+      (void)attr;
+      hipLaunchKernelGGL(kern, dim3(Hq, (Sq + 255) / 256, B), dim3(AW_WAVES * 64), smem, st, p);
     };
-    if (wide_p && causal) {
-      if (wide == 8) { if (D == 128) go(attn_prefill_wide_kernel<128, true, 8, qt, true>, 128); else go(attn_prefill_wide_kernel<64, true, 8, qt, true>, 64); }
-      else { if (D == 128) go(attn_prefill_wide_kernel<128, true, 4, qt, true>, 128); else go(attn_prefill_wide_kernel<64, true, 4, qt, true>, 64); }
-    } else if (wide == 8) {
-      if (D == 128) { if (causal) go(attn_prefill_wide_kernel<128, true, 8>, 128); else go(attn_prefill_wide_kernel<128, false, 8>, 128); }
-      else { if (causal) go(attn_prefill_wide_kernel<64, true, 8>, 64); else go(attn_prefill_wide_kernel<64, false, 8>, 64); }
+    using T = std::true_type;
+    using F = std::false_type;
+    if (D == 128) {
+      const std::integral_constant<int, 128> d;
+      if (wide_p && causal) go(d, T{}, T{});
+      else if (causal) go(d, T{}, F{});
+      else go(d, F{}, F{});
     } else {
-      if (D == 128) { if (causal) go(attn_prefill_wide_kernel<128, true, 4>, 128); else go(attn_prefill_wide_kernel<128, false, 4>, 128); }
-      else { if (causal) go(attn_prefill_wide_kernel<64, true, 4>, 64); else go(attn_prefill_wide_kernel<64, false, 4>, 64); }
+      const std::integral_constant<int, 64> d;
+      if (wide_p && causal) go(d, T{}, T{});
+      else if (causal) go(d, T{}, F{});
+      else go(d, F{}, F{});
+    }
+    return;
+  }
+  if (rows == 128) {
+    const dim3 grid128((Sq + 127) / 128, Hq, B), block8(512);
+    if (wide_p && causal) {
+      if (D == 128) hipLaunchKernelGGL((attn_prefill_kernel<128, true, false, 1, true, false, 8>), grid128, block8, 0, st, p);
+      else hipLaunchKernelGGL((attn_prefill_kernel<64, true, false, 1, true, false, 8>), grid128, block8, 0, st, p);
+    } else if (D == 128) {
+      if (causal) hipLaunchKernelGGL((attn_prefill_kernel<128, true, false, 1, false, false, 8>), grid128, block8, 0, st, p);
+      else hipLaunchKernelGGL((attn_prefill_kernel<128, false, false, 1, false, false, 8>), grid128, block8, 0, st, p);
+    } else {
+      if (causal) hipLaunchKernelGGL((attn_prefill_kernel<64, true, false, 1, false, false, 8>), grid128, block8, 0, st, p);
+      else hipLaunchKernelGGL((attn_prefill_kernel<64, false, false, 1, false, false, 8>), grid128, block8, 0, st, p);
     }
     return;
   }
@@ -746,14 +776,11 @@ void launch_attn_prefill(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf16
     else hipLaunchKernelGGL((attn_prefill_kernel<64, true, false, 1, true>), grid, block, 0, st, p);
     return;
   }
-  // Two key-tile groups per block for the ViT's shape class -- head_dim 64, non-causal, so few blocks
-  // that half the chip idles (577 tokens x 16 heads: 160) -- while all blocks are resident at once:
-  // 12.3 -> 9.9 us per layer.  Causal head_dim-128 blocks do not gain (636 tokens x 32 heads: 23.9 ->
-  // 25.1 us, 836: 30.4 -> 33.7): they are bound by the LDS pipe, not by the chain over their key
-  // tiles, and the diagonal splits unevenly (benchmarks/bench_attn_groups.py).
-  const long long nblocks = static_cast<long long>(grid.x) * Hq * B;
-  const bool two = g_attn_groups == 2 ||
-                   (g_attn_groups == 0 && D == 64 && !causal && nblocks <= 512 && Sk >= 4 * TK);
+  // Two key-tile groups per block for the ViT's shape class -- head_dim 64, non-causal, so few blocks that much of the chip idles
+  // (577 tokens x 16 heads: 160).  us, one group / two: 160 blocks 9.3 / 8.3, 224 7.6 / 7.5, 256 14.0 / 12.6, 320 13.8 / 13.5, 384 9.6 / 10.5, 480
+  // 13.8 / 15.1.  Causal head_dim-128 blocks do not gain (636 tokens x 32 heads: 23.9 -> 25.1, 836: 30.4 -> 33.7 when tiles went through
+  // registers): the diagonal splits unevenly (benchmarks/bench_attn_groups.py).
+  const bool two = g_attn_groups == 2 || (g_attn_groups == 0 && vit && n64 <= 320 && Sk >= 4 * TK);
   if (two) {
     dim3 block2(512);
     if (D == 128) {

@@ -30,11 +30,11 @@ ATTN_TILE = 64           # query rows per work item of the chunk attention
 
 
 def long_run(rows: int, reps: int, heads: int = 1, dim: int = 64, alone: bool = False) -> bool:
-    """Runs of query rows that get a launch of their own; the others of a pack share one launch of 64-row blocks.  The flash
-    kernel takes 256-row blocks of 1 400 rows, of several runs of 512, and from 512 rows on where the heads make 256 blocks
-    (``attn_prefill.hip``).  The last are worth it for a run that is ``alone``, from 1 024 rows, or that fills its blocks of 128-wide
-    heads; us of own launches / the shared one: 1 x 1024 rows, 64 heads of 128, 54 / 73; 4 x 1024 216 / 269; 8 x 512, 128 heads, 276 / 304;
-    behind with 520 + 60 + 60 rows, 96 heads (45 / 37), and 4 x 768, 96 heads of 64 (129 / 101)."""
+    """Runs of query rows that get a launch of their own; the others of a pack share one launch of 64-row blocks.  A launch of its
+    own takes blocks of 64, 128 or 256 rows (``attn_prefill.hip``).  It is worth it from 1 400 rows, for several runs of 512, and from 512
+    rows where the heads make 256 blocks of 256 rows: for a run that is ``alone``, from 1 024 rows, or that fills its blocks of 128-wide
+    heads; us of own launches / the shared one: 1 x 1024 rows, 64 heads of 128, 51 / 61; 4 x 1024 133 / 211; 8 x 512, 128 heads, 189 / 307;
+    level with 1 x 1024, 32 heads (33 / 33) and 4 x 768, 96 heads of 64 (86 / 84)."""
     if rows >= 1400 or (reps > 1 and rows >= 512):
         return True
     wide = rows >= 512 and -(-rows // 256) * heads >= 256

@@ -84,3 +84,41 @@ def test_two_group_forward_feeds_backward(dev, two):
     ref.attention(qf, kf, vf, True).backward(go.float())
     for got, want in ((q.grad, qf.grad), (k.grad, kf.grad), (v.grad, vf.grad)):
         assert torch.allclose(got.float(), want, atol=3e-2, rtol=3e-2), float((got.float() - want).abs().max())
+
+
+@pytest.fixture()
+def eight():
+    from eventgpt_amd.ops import hip
+    hip.raw.attn_enable_wide(3)
+    yield hip
+    hip.raw.attn_enable_wide(1)
+
+
+# edges of the 128-row blocks and of the key tiles, against the 64-row blocks: the same sums in the same order
+@pytest.mark.parametrize("D,H,Hkv,Sq,Sk,causal", [
+    (128, 4, 4, 1, 1, True), (128, 4, 2, 127, 127, True), (128, 2, 2, 128, 129, True), (128, 2, 1, 129, 700, True), (128, 4, 4, 836, 836, True),
+    (128, 2, 2, 257, 1000, False), (64, 4, 4, 577, 577, False), (64, 4, 2, 130, 259, True), (64, 2, 2, 70, 65, False), (64, 2, 2, 640, 63, False)])
+def test_eight_wave_attention_is_the_four_wave_one(dev, eight, D, H, Hkv, Sq, Sk, causal):
+    B = 2
+    q, k, v = _rand(B, Sq, H, D, dev=dev), _rand(B, Sk, Hkv, D, dev=dev, seed=1), _rand(B, Sk, Hkv, D, dev=dev, seed=2)
+    o, lse = eight.raw.attention_fwd_lse(q, k, v, causal, D ** -0.5, Sk - Sq if causal else 0)
+    rep = H // Hkv
+    want = ref.attention(q, k.repeat_interleave(rep, 2), v.repeat_interleave(rep, 2), causal, q_offset=Sk - Sq if causal else 0)
+    assert torch.allclose(o.float(), want.float(), atol=2e-2, rtol=2e-2)
+    eight.raw.attn_enable_wide(0)
+    eight.raw.attn_force_groups(1)
+    o4, lse4 = eight.raw.attention_fwd_lse(q, k, v, causal, D ** -0.5, Sk - Sq if causal else 0)
+    eight.raw.attn_force_groups(0)
+    assert torch.equal(o, o4) and torch.equal(lse, lse4)
+
+
+def test_attention_of_rows_off_their_alignment(dev):
+    """Keys and values two bytes off 16-byte alignment, and batches whose distance is not a multiple of eight."""
+    from eventgpt_amd.ops import hip
+    B, S, H, D = 2, 150, 2, 128
+    q = _rand(B, S, H, D, dev=dev)
+    flat = _rand(B * (S * H * D + 4) + 8, dev=dev, seed=1)
+    for k in (flat[1:1 + B * S * H * D].view(B, S, H, D), flat.as_strided((B, S, H, D), (S * H * D + 4, H * D, D, 1))):
+        o = hip.raw.attention(q, k, k, True, D ** -0.5, 0)
+        want = ref.attention(q, k.contiguous(), k.contiguous(), True)
+        assert torch.allclose(o.float(), want.float(), atol=2e-2, rtol=2e-2)
