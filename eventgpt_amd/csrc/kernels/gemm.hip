@@ -985,19 +985,21 @@ static void launch_cfg(const GemmParams& p, hipStream_t st) {
                      smem, st, EVGPT_GEMM_PASS_COLS(q, KT ? q.k_cols : q.glu_half));
 }
 
+// set while gemm_splitk_slabs / launch_gemm_partial plan a product whose caller sums the slabs itself
+static thread_local bool g_for_slabs = false;
+
 // 256 x 256 tiles pay once there are rows to fill them and about half a round of tiles.  With the 8-wave kernel (measured on
 // MI355X, TFLOP/s, 8-wave vs best 4-wave config): 2115 x 4096 x 11008, 144 tiles, 913 vs 751; 4643 x 12288 x 4096 1190 vs 930;
 // 20352 x 4096 x 4096 1230 vs 905; but 636 rows 717 vs 948 and 2885 x 1024 x 4096, 48 tiles, 282 vs 567.
 // The lines are that kernel's.  Where gemm_quad.hip takes the tiles, us, 256 x 256 / the other choice: 2115 x 4096 x 4096, 144 tiles,
 // 76 / 107, x 2048 45 / 53; 1024 x 9216 x 1024 30 / 36; 836 x 10240 x 1024, 160, 29 / 37; behind at 128 tiles of 1024 x 8192 x 4096 81 /
-// 73.  Some that the lines leave out would gain: 768 x 12288 x 4096, 144 tiles, 127 where it would be 78; 768 x 11008 x 4096, 129, 108
-// and 78; with a residual 3840 x 2304 x 1024, 135, 45 and 32.
+// 73.  What these lines leave out below 1 024 rows is use_256_few's; with a residual 3840 x 2304 x 1024, 135 tiles, 45 where it would be 32.
 // K (0 = not known to the caller): a 256 x 256 tile's prologue and epilogue are one workgroup's alone (one per
 // CU), so over a short contraction the 4-wave 128 x 128 tile -- two workgroups per CU, each hiding the other's
 // ends -- is ahead.  With the grouped tile walk, TFLOP/s 8-wave vs 128 x 128: 23080 x 3072 x 1024 782 vs 816,
 // 11540 x 3072 x 1024 674 vs 771, 4616 x 4096 x 1024 547 vs 707, 4616 x 4096 x 2048 717 vs 882, but
 // 6688 x 4096 x 2048 980 vs 945, 23080 x 4096 x 2048 1102 vs 1003 and 4643 x 12288 x 4096 1253 vs 1070.
-static bool use_256(int M, int N, int K = 0) {
+static bool use_256_base(int M, int N, int K = 0) {
   const long long t = static_cast<long long>((M + 255) / 256) * ((N + 255) / 256);
   // (Those were measured with the direct epilogue.  With whole-line stores through LDS -- gemm_epilogue_rows --
   // the 8-wave kernel is ahead over short contractions too once its tiles make more than half a round: 8-wave vs
@@ -1010,6 +1012,19 @@ static bool use_256(int M, int N, int K = 0) {
   // 836 x 11008 x 4096: 686 vs 582), behind for 64 tiles (836 x 4096: 338 vs 700)
   return g_use_256 && ((M >= 1024 && t >= 128) || (M >= 768 && t >= 160));
 }
+
+// Two to four row tiles, where only the four-wave kernel is ahead: once the 128 x 128 tiles are more than a round (512 workgroups) and
+// these are not, or those more than two rounds.  us, plain / gated / with a residual / slabs, so / as before: 700 x 12288 x 4096, 144 and 576 tiles,
+// 84 / 125, gated --, 84 / 127, 84 / 122; 400 x 22016 x 4096, 172 and 688, 88 / 131, 91 / 128, 87 / 134, 85 / 129; 636 x 20480 x 2048,
+// 240 and 800, 56 / 76, 52 / 71; 300 x 32000 x 4096, 250 and 750, 98 / 137; 636 rows, 375 and 1250, 164 / 198.  Under a round of the others
+// behind, 636 x 12288 x 4096, 144 and 480, 82 / 72.  More than 256 against two rounds: ahead where a few are left for last_round_split
+// (636 x 22016 x 4096, 258 and 860, 123 / 136, gated 116 / 132; slabs are not split so, 154 / 136), level at 288.  Four row tiles: 900 x 9216 x 4096, 144
+// and 576, 84 / 124, gated 85 / 123; 850 x 9728 x 2048, 152 and 532, 47 / 58.
+static bool use_256_few(int M, int N, int K) {
+  const long long t = static_cast<long long>((M + 255) / 256) * ((N + 255) / 256), t128 = static_cast<long long>((M + 127) / 128) * ((N + 127) / 128);
+  return g_use_256 && M > 256 && M < 1024 && K >= 2048 && t128 > 512 && (t <= 256 || t128 > 1024 || (t <= 264 && M > 512 && !g_for_slabs));
+}
+static bool use_256(int M, int N, int K = 0) { return use_256_base(M, N, K) || use_256_few(M, N, K); }
 
 // Short contractions (the ViT's 1024-wide layers: 16 K-tiles) are bound by the round trip of each K-tile, which waves of
 // other workgroups have to cover: eight waves on the 64 x 128 tile with two stages (48 KB: three workgroups, 24 waves a
@@ -1050,8 +1065,6 @@ static void launch_64x128_w8(const GemmParams& p, hipStream_t st) {
 
 static int g_forced_splitk = 0;
 static bool g_tail_splitk = true;
-// set while gemm_splitk_slabs / launch_gemm_partial plan a product whose caller sums the slabs itself
-static thread_local bool g_for_slabs = false;
 
 // 768..1024 rows into a few thousand columns over a long contraction (one ~840-token sample against
 // the 4096-wide matrices with K = 11008 / 12288 / 22016): 48..128 tiles of 256x256 are a fraction of a
@@ -1059,9 +1072,13 @@ static thread_local bool g_for_slabs = false;
 // choice (benchmarks/bench_gemm_splitk256.py, TFLOP/s, 4 splits vs the best 4-wave configuration:
 // 836x4096x11008 878 vs 811, x12288 926 vs 844, x22016 1038 vs 871; at 636 rows -- three row tiles,
 // a quarter of the last one used -- it is behind, 725 vs 807).  With gemm_quad.hip, us, so / the other choice: 836 x 4096 x 11008 83 / 95,
-// x 22016 144 / 177, 1000 rows x 11008 88 / 136; behind at 128 tiles in two splits, 1024 x 8192 x 8192 152 / 136.  Returns the split count, or 0.
-static int narrow_256_splits(int M, int N, int K) {
-  if (!g_use_256 || g_forced_cfg >= 0 || g_forced_splitk > 0 || M < 768 || M > 1024 || K < 8192) return 0;
+// x 22016 144 / 177, 1000 rows x 11008 88 / 136; behind at 128 tiles in two splits, 1024 x 8192 x 8192 152 / 136.  Three row tiles (513 to
+// 767 rows), the sum of the slabs included: ahead where the 128 x 128 tiles are more than 170 and leave room for two splits, 700 x 4096
+// x 11008 80 / 95, 767 x 4096 x 8192 65 / 74, 520 x 5120 x 13824 90 / 121; with three of them behind, 636 x 4096 x 11008 79 / 76.  strided: an
+// operand that only the 8-wave kernel takes.  Returns the split count, or 0.
+static int narrow_256_splits(int M, int N, int K, bool strided = false) {
+  if (!g_use_256 || g_forced_cfg >= 0 || g_forced_splitk > 0 || M < (strided ? 768 : 513) || M > 1024 || K < 8192) return 0;
+  if (M < 768 && static_cast<long long>((M + 127) / 128) * ((N + 127) / 128) <= 170) return 0;
   const long long t = static_cast<long long>((M + 255) / 256) * ((N + 255) / 256);
   if (t < 48 || t > 128) return 0;
   const int s = static_cast<int>(256 / t);
@@ -1347,7 +1364,7 @@ int gemm_splitk_t(int M, int N, int K) {
   if (g_forced_splitk > 0) return (K / 64) >= g_forced_splitk ? g_forced_splitk : 1;
   const long long t = static_cast<long long>((M + 127) / 128) * ((N + 127) / 128);
   if (g_forced_cfg >= 0 || M > 1024) return 1;
-  if (!use_256(M, N, K) && narrow_256_splits(M, N, K) >= 2) return narrow_256_splits(M, N, K);
+  if (!use_256_base(M, N, K) && narrow_256_splits(M, N, K, true) >= 2) return narrow_256_splits(M, N, K, true);
   if (t <= 32 && K >= 2048) {   // narrow output, long contraction (input gradient of a low-rank B): as in gemm_splitk
     const long long want = 256 / t, most = K / 256;
     const int s = static_cast<int>(want < most ? want : most);
@@ -1382,15 +1399,18 @@ void launch_gemm_grouped(const bf16_t* A, const bf16_t* W, bf16_t* C, const int*
   p.glu_act = glu - 1;
   p.grp_start = start; p.grp_perm = perm; p.grp_top = top; p.grp_count = E;
   p.grp_wstride = static_cast<long long>(N) * K;
-  // Rows of an average group.  (The last line is the 8-wave kernel's; with gemm_quad.hip 256 x 256 tiles would be ahead sooner.  us, gate / up and
-  // down, 128 x 128 / 256 x 256: 8 experts of 4096 x 5504, 256 rows a group 356 / 218 and 216 / 140, 767 678 / 476 and 348 / 232; of 2048 x
-  // 2816, 256 rows 115 / 66 and 47 / 59, 384 120 / 110 and 50 / 61, 640 175 / 151 and 75 / 62.)
+  // Rows of an average group.  256 x 256 tiles, which are gemm_quad.hip's, from 128 rows where the others are more than a round, plain, or these
+  // 170, gated.  us of 128 x 128 (from 192 rows; below 64 x 128) / 256 x 256 tiles, gate / up and down, tokens routed at random: 8 experts of 4096 x
+  // 5504, 96 rows 206 / 215 and 125 / 117, 160 268 / 218 and 151 / 125, 256 344 / 295 and 210 / 140, 512 488 / 383 and 287 / 233, 767 655 / 506 and 343 /
+  // 251; of 2048 x 2816, 128 rows 79 / 62 and 32 / 53, 256 111 / 108 and 44 / 57, 384 114 / 105 and 49 / 61, 448 139 / 107 and 71 / 60; 4 of 4096 x 8192,
+  // 224 227 / 157 and 136 / 149, 448 329 / 209 and 241 / 156.
   const int per = rows / E;
+  const long long t128 = static_cast<long long>(E) * ((per + 127) / 128) * ((N + 127) / 128), t256 = static_cast<long long>(E) * ((per + 255) / 256) * ((N + 255) / 256);
   if (gemm_grouped_few_serves(p, rows)) launch_gemm_grouped_few(p, rows, st);
+  else if (per >= 768 || (per >= 128 && K >= 2048 && g_use_256 && (glu ? t256 >= 170 : t128 >= 512))) launch_256<false, false, 256, true>(p, st, rows);
   else if (per < 48) launch_grp<32, 128, 1, 4, 4>(p, rows, st);
   else if (per < 192) launch_grp<64, 128, 2, 2, 3>(p, rows, st);
-  else if (per < 768) launch_grp<128, 128, 2, 2, 2>(p, rows, st);
-  else launch_256<false, false, 256, true>(p, st, rows);
+  else launch_grp<128, 128, 2, 2, 2>(p, rows, st);
 }
 
 // H[M, I] = act(A · Wgate^T) * (A · Wup^T), act = silu or (glu_act) gelu, with W = [gate rows | up rows] ([2I, K]): the gate/up
@@ -1447,9 +1467,9 @@ static void launch_t(const GemmParams& p, hipStream_t st) {
       return;
     }
   }
-  if (p.splitk > 1 && cols_ok && !use_256(p.M, p.N, p.K) && narrow_256_splits(p.M, p.N, p.K) >= 2) launch_256<AT, BT>(p, st);
+  if (p.splitk > 1 && cols_ok && !use_256_base(p.M, p.N, p.K) && narrow_256_splits(p.M, p.N, p.K, true) >= 2) launch_256<AT, BT>(p, st);
   else if (p.splitk > 1) launch_cfg<128, 128, 2, 2, 2, AT, BT>(p, st);
-  else if ((g_forced_cfg == CFG_256x256 || (g_forced_cfg < 0 && use_256(p.M, p.N, p.K))) && cols_ok) launch_256<AT, BT>(p, st);
+  else if ((g_forced_cfg == CFG_256x256 || (g_forced_cfg < 0 && use_256_base(p.M, p.N, p.K))) && cols_ok) launch_256<AT, BT>(p, st);
   else if (tiles(128, 128) >= 384) launch_cfg<128, 128, 2, 2, 2, AT, BT>(p, st);
   else if (tiles(64, 128) >= 300) launch_cfg<64, 128, 2, 2, 3, AT, BT>(p, st);
   else launch_cfg<64, 64, 2, 2, 4, AT, BT>(p, st);

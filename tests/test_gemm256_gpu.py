@@ -169,6 +169,31 @@ def test_last_round_tiles_with_k_split(dev, M, N, K):
     _check(yf, x.float() @ w.float().t(), K)
 
 
+# two to four row tiles: the fewest and most rows, one round, a few tiles past it, two rounds of them against three of the others
+@pytest.mark.parametrize("M,N,K", [(257, 22016, 2048), (400, 16640, 2112), (767, 11008, 2048), (636, 22016, 2048), (520, 28672, 2048), (700, 12288, 4096), (900, 9216, 2048)])
+def test_two_to_four_row_tiles(dev, M, N, K):
+    from eventgpt_amd.ops import hip
+    raw = hip.raw
+    x, w = _rand(M, K, dev=dev), _rand(N, K, dev=dev, seed=1, scale=0.05)
+    bias, res = _rand(N, dev=dev, seed=2), _rand(M, N, dev=dev, seed=3)
+    y = x.float() @ w.float().t()
+    _check(raw.linear(x, w, None, None, 0, False), y, K)
+    _check(raw.linear(x, w, bias, res, 1, False), torch.nn.functional.gelu(y + bias.float()).to(torch.bfloat16).float() + res.float(), K)
+    _check(raw.linear_partial(x, w).sum(0), y, K)
+    _check(raw.linear_swiglu(x, w), torch.nn.functional.silu(y[:, :N // 2]) * y[:, N // 2:], K)
+
+
+# slabs of three row tiles in K splits: the lines at 513 rows and at 170 tiles of 128 x 128
+@pytest.mark.parametrize("M,N,K", [(513, 4480, 8192), (641, 4096, 8192), (640, 4096, 8192), (767, 5120, 8256)])
+def test_slabs_of_three_row_tiles(dev, M, N, K):
+    from eventgpt_amd.ops import hip
+    raw = hip.raw
+    x, w = _rand(M, K, dev=dev), _rand(N, K, dev=dev, seed=1, scale=0.05)
+    res, want = _rand(M, N, dev=dev, seed=3), x.float() @ w.float().t()
+    _check(raw.linear_partial(x, w).sum(0), want, K)
+    _check(raw.linear(x, w, None, res, 0, False), want.to(torch.bfloat16).float() + res.float(), K)
+
+
 @pytest.mark.parametrize("M,I,K", [(2115, 4096, 1024), (1500, 11008, 512), (2115, 11008, 4096)])
 def test_swiglu_gemm_last_tiles_on_small_tiles(dev, M, I, K):
     """The gate/up GEMM with the SwiGLU epilogue when its 256 x 128 output tiles are whole rounds plus a

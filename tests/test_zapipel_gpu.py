@@ -388,7 +388,10 @@ def test_grouped_products_of_a_few_rows(raw, dev, counts, K, N, gated):
 @pytest.mark.parametrize("counts,K,N,plain,gated", [
     ([1800, 1500], 192, 4736, "gemm256_kernel", "gemm256_kernel"), ([1800, 1500], 320, 4736, "gemm_quad_kernel", "gemm256_kernel"),
     ([2050, 0, 1270, 900], 832, 4736, "gemm_quad_kernel", "gemm_quad_kernel"), ([5, 3100], 896, 4736, "gemm_quad_kernel", "gemm_quad_kernel"),
-    ([900, 800], 1088, 1024, "gemm_quad_kernel", "gemm_quad_kernel")])
+    ([900, 800], 1088, 1024, "gemm_quad_kernel", "gemm_quad_kernel"),
+    ([300, 0, 257, 129, 90, 1, 150, 105], 2048, 5632, "gemm_quad_kernel", "gemm_quad_kernel"),      # 129 rows a group
+    ([300, 0, 257, 129, 90, 1, 150, 94], 2048, 5632, "gemm_bf16_kernel", "gemm_bf16_kernel"),
+    ([260, 200, 180, 250], 2048, 10816, "gemm_quad_kernel", "gemm_quad_kernel"), ([260, 200, 180, 250], 2048, 8128, "gemm_quad_kernel", "gemm_bf16_kernel")])
 def test_grouped_products_of_many_rows(raw, dev, counts, K, N, plain, gated):
     """256-row tiles of groups on both kernels that have them: more tiles than workgroups, so that a workgroup's next tile belongs to another group
     whose first K-tiles are staged under this one's last; odd and even numbers of K-tiles, an empty group, one of a few rows, gathered and consecutive
