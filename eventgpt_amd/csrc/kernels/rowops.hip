@@ -333,6 +333,67 @@ __global__ __launch_bounds__(256) void group_norm_kernel(SrcRows y, SrcRows gate
     store8(out + row * ld_out + c, a);
   }
 }
+// The same for bf16 rows of NC * 2048 channels without padding whose parts are runs of whole 512 (a wave's): the row stays in registers, all of
+// it requested at once, and only the sums of 512 go through LDS (the kernel above stages the row there and reads it twice, its loads behind
+// the choice of their type).  4096 rows: 8192 channels, silu gate before, 61 -> 45 us (201 MB: 4.5 TB/s); 4096, sigmoid gate after, 31 -> 24.5.
+template <int GATE, int NC>
+__global__ __launch_bounds__(256) void group_norm_wide_kernel(const bf16_t* __restrict__ y, long long ldy, const bf16_t* __restrict__ gate,
+                                                              long long ldg, const float* __restrict__ w, bf16_t* __restrict__ out, int plen,
+                                                              float eps) {
+  __shared__ float sums[NC * 4];
+  const long long row = blockIdx.x;
+  const int c = threadIdx.x * 8, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  float a[NC][8], g[NC][8];
+#pragma unroll
+  for (int i = 0; i < NC; ++i) load8(y + row * ldy + c + i * 2048, a[i]);
+  if constexpr (GATE != GATE_NONE)
+#pragma unroll
+    for (int i = 0; i < NC; ++i) load8(gate + row * ldg + c + i * 2048, g[i]);
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    if constexpr (GATE == GATE_SILU_BEFORE)
+#pragma unroll
+      for (int k = 0; k < 8; ++k) a[i][k] *= g[i][k] * sigmoid_f(g[i][k]);
+    const float s = wave_sum(sumsq8(a[i]));
+    if ((threadIdx.x & 63) == 0) sums[i * 4 + wid] = s;
+  }
+  __syncthreads();
+  const int runs = plen >> 9;
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    const int first = (i * 4 + wid) / runs * runs;
+    float s = 0.f, wt[8];
+    for (int k = 0; k < runs; ++k) s += sums[first + k];
+    const float inv = rsqrtf(s / static_cast<float>(plen) + eps);
+    load8(w + c + i * 2048, wt);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      a[i][k] *= inv * wt[k];
+      if constexpr (GATE == GATE_SIGMOID_AFTER) a[i][k] *= sigmoid_f(g[i][k]);
+    }
+    store8(out + row * (NC * 2048) + c + i * 2048, a[i]);
+  }
+}
+static bool launch_group_norm_wide(const SrcRows& y, const SrcRows& gate, int gcol, int mode, const float* w, void* out, int rows, int slots,
+                                   int parts, float eps, hipStream_t st) {
+  const int plen = slots / parts, nc = slots / 2048;
+  if (slots % 2048 || plen % 512 || plen * parts != slots || (nc != 1 && nc != 2 && nc != 4) || y.f32 || (mode != GATE_NONE && gate.f32)) return false;
+  const bf16_t* yp = static_cast<const bf16_t*>(y.p);
+  const bf16_t* gp = mode == GATE_NONE ? nullptr : static_cast<const bf16_t*>(gate.p) + gcol;
+#define EVGPT_GN(GATE, NC) hipLaunchKernelGGL((group_norm_wide_kernel<GATE, NC>), dim3(rows), dim3(256), 0, st, yp, y.ld, gp, gate.ld, w, \
+                                              static_cast<bf16_t*>(out), plen, eps)
+#define EVGPT_GN_NC(GATE)         \
+  if (nc == 1) EVGPT_GN(GATE, 1); \
+  else if (nc == 2) EVGPT_GN(GATE, 2); \
+  else EVGPT_GN(GATE, 4)
+  if (mode == GATE_SILU_BEFORE) { EVGPT_GN_NC(GATE_SILU_BEFORE); }
+  else if (mode == GATE_SIGMOID_AFTER) { EVGPT_GN_NC(GATE_SIGMOID_AFTER); }
+  else { EVGPT_GN_NC(GATE_NONE); }
+#undef EVGPT_GN_NC
+#undef EVGPT_GN
+  return true;
+}
+
 template <typename T>
 static void launch_group_norm(const SrcRows& y, const SrcRows& gate, int gcol, int mode, const float* w, void* out, int rows,
                               int heads, int v, int vp, int parts, int ld_out, float eps, hipStream_t st) {
@@ -354,6 +415,7 @@ static void launch_group_norm(const SrcRows& y, const SrcRows& gate, int gcol, i
 void launch_group_norm_rows(const SrcRows& y, const SrcRows& gate, int gcol, int mode, const float* w, void* out, bool f32,
                             int rows, int heads, int v, int vp, int parts, int ld_out, float eps, hipStream_t st) {
   if (f32) launch_group_norm<float>(y, gate, gcol, mode, w, out, rows, heads, v, vp, parts, ld_out, eps, st);
+  else if (v == vp && ld_out == heads * vp && launch_group_norm_wide(y, gate, gcol, mode, w, out, rows, heads * vp, parts, eps, st)) return;
   else launch_group_norm<bf16_t>(y, gate, gcol, mode, w, out, rows, heads, v, vp, parts, ld_out, eps, st);
 }
 

@@ -131,6 +131,19 @@ def test_group_norm_with_gate(raw, dev, dtype, heads, v, vp, parts, before):
                      oracle.rms(y[..., :v].reshape(rows, -1).double(), eps, wr, parts)) < 2e-6
 
 
+# rows of whole 2048 channels in parts of whole 512 (kept in registers), and two forms next to them
+@pytest.mark.parametrize("heads,v,parts", [(4, 512, 4), (32, 64, 1), (64, 64, 4), (8, 512, 8), (128, 64, 8), (128, 64, 1), (96, 64, 3), (32, 64, 8)])
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_group_norm_of_wide_rows(raw, dev, heads, v, parts, mode):
+    rows, slots, eps = 3, heads * v, 1e-3
+    w = 1 + 0.2 * rnd(heads, v, seed=2).float()
+    (yd, yr), (gd, gr) = typed(rnd(rows, slots), torch.bfloat16, dev), typed(rnd(rows, 8 + slots, seed=1), torch.bfloat16, dev)
+    o = raw.group_norm_rows(yd, gd if mode else None, 8 if mode else 0, mode, w.to(dev), heads, v, v, parts, slots, eps, False)
+    g, wr = gr[:, 8:], w.reshape(-1).double()
+    want = oracle.rms(yr * oracle.silu(g) if mode == 1 else yr, eps, wr, parts) * (torch.sigmoid(g) if mode == 2 else 1.0)
+    assert N.rel_err(o, want) < 6e-3
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_glu(raw, dev, dtype):
     src, sr = typed(rnd(7, 2 * 72, scale=2), dtype, dev)
