@@ -18,7 +18,7 @@ if os.environ.get("EVGPT_GROUP_M"):        # row tiles per group of the GEMM til
     hip.raw.gemm_group_m(int(os.environ["EVGPT_GROUP_M"]))
 if os.environ.get("EVGPT_GEMM_SPLITK"):    # 1: never split K in GEMMs of more than 32 rows
     hip.raw.gemm_force_splitk(int(os.environ["EVGPT_GEMM_SPLITK"]))
-if os.environ.get("EVGPT_ATTN_WIDE"):      # 0: 64-row attention blocks only, 2: 128-row blocks for every shape
+if os.environ.get("EVGPT_ATTN_WIDE"):      # 0: no 256-row attention blocks, 2: they for every shape, 3: 128-row blocks
     hip.raw.attn_enable_wide(int(os.environ["EVGPT_ATTN_WIDE"]))
 dev = torch.device("cuda")
 cfg = EventChatConfig.eventgpt_7b()
