@@ -1117,7 +1117,9 @@ static GemmCfg pick_cfg(int M, int N, int K = 0, int k_real = 0, bool act = fals
   // 600 x 9280 x 2048, 365 tiles: 35.6 us, 64 x 128 tiles 42.5; 300 x 12288 x 4096, 288 tiles: 63.5 vs 53.8.  Not where the 64 x 128
   // tiles (72 KB: two workgroups a CU) are one round, rows that leave half of the larger ones empty: 156 x 21504 x 2048, 504 of
   // them, 35.1 us, 128 x 128 tiles 44.9
-  if (tiles(128, 128) >= 384 || (tiles(128, 128) >= 336 && tiles(64, 128) > 512)) return CFG_128x128;
+  // (more than a round of 64 x 128 tiles, so / 128 x 128: 512 x 9216 x 4096, 576 and 288, 80 / 72, with a residual 83 / 76; 600 x 8448 x 4096, 660 and 330, 77
+  // / 63; 390 x 10112 x 2048 38 / 35; gated 450 x 11264 x 2048 38 / 35, 600 x 9216 x 4096 75 / 62; a round of them, 448 x 9216 x 4096, 504, 54 / 68)
+  if (tiles(128, 128) >= 384 || tiles(64, 128) > 512) return CFG_128x128;
   if (tiles(64, 128) >= 300) return CFG_64x128;
   if (tiles(64, 64) >= 300) return CFG_64x64;
   return CFG_32x64;
@@ -1445,7 +1447,7 @@ void launch_gemm_glu(const bf16_t* A, const bf16_t* W, bf16_t* H, int M, int I, 
   if (g_forced_cfg == CFG_256x256 || (g_forced_cfg < 0 && use_256(M, 2 * I, K))) launch_256<false, false>(p, st);
   else if (const RingTile ring = g_forced_cfg < 0 ? gemm_ring_tile(p, false) : RING_NONE; ring != RING_NONE)
     launch_gemm_ring(p, ring, st);
-  else if (g_forced_cfg == CFG_128x128 || (g_forced_cfg < 0 && tiles(128, 128) >= 384)) launch_cfg<128, 128, 2, 2, 2>(p, st);
+  else if (g_forced_cfg == CFG_128x128 || (g_forced_cfg < 0 && (tiles(128, 128) >= 384 || tiles(64, 128) > 512))) launch_cfg<128, 128, 2, 2, 2>(p, st);
   else if (g_forced_cfg == CFG_64x64) launch_cfg<64, 64, 2, 2, 4>(p, st);
   else launch_cfg<64, 128, 2, 2, 3>(p, st);
 }
