@@ -334,15 +334,17 @@ __global__ __launch_bounds__(256) void group_norm_kernel(SrcRows y, SrcRows gate
   }
 }
 // The same for bf16 rows of NC * 2048 channels without padding whose parts are runs of whole 512 (a wave's): the row stays in registers, all of
-// it requested at once, and only the sums of 512 go through LDS (the kernel above stages the row there and reads it twice, its loads behind
-// the choice of their type).  4096 rows: 8192 channels, silu gate before, 61 -> 45 us (201 MB: 4.5 TB/s); 4096, sigmoid gate after, 31 -> 24.5.
+// it requested at once, and only the sums of eight channels go through LDS (the kernel above stages the row there and reads it twice, its loads
+// behind the choice of their type).  A lane adds its squares over the runs of a part ahead of the wave's sum, the order of the kernel above
+// for four parts and more: the same bits.  4096 rows: 8192 channels, silu gate before, 61 -> 45 us (201 MB: 4.5 TB/s); 4096, sigmoid gate after,
+// 31 -> 24.5.
 template <int GATE, int NC>
 __global__ __launch_bounds__(256) void group_norm_wide_kernel(const bf16_t* __restrict__ y, long long ldy, const bf16_t* __restrict__ gate,
                                                               long long ldg, const float* __restrict__ w, bf16_t* __restrict__ out, int plen,
                                                               float eps) {
-  __shared__ float sums[NC * 4];
+  __shared__ float sums[NC * 256];                 // [run of 512][lane]
   const long long row = blockIdx.x;
-  const int c = threadIdx.x * 8, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = threadIdx.x * 8, lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   float a[NC][8], g[NC][8];
 #pragma unroll
   for (int i = 0; i < NC; ++i) load8(y + row * ldy + c + i * 2048, a[i]);
@@ -354,17 +356,22 @@ __global__ __launch_bounds__(256) void group_norm_wide_kernel(const bf16_t* __re
     if constexpr (GATE == GATE_SILU_BEFORE)
 #pragma unroll
       for (int k = 0; k < 8; ++k) a[i][k] *= g[i][k] * sigmoid_f(g[i][k]);
-    const float s = wave_sum(sumsq8(a[i]));
-    if ((threadIdx.x & 63) == 0) sums[i * 4 + wid] = s;
+    sums[i * 256 + threadIdx.x] = sumsq8(a[i]);
   }
   __syncthreads();
   const int runs = plen >> 9;
+  int at = -1;
+  float inv = 0.f;
 #pragma unroll
   for (int i = 0; i < NC; ++i) {
     const int first = (i * 4 + wid) / runs * runs;
-    float s = 0.f, wt[8];
-    for (int k = 0; k < runs; ++k) s += sums[first + k];
-    const float inv = rsqrtf(s / static_cast<float>(plen) + eps);
+    if (first != at) {                             // (one wave's runs may be of one part)
+      float s = 0.f;
+      for (int k = 0; k < runs; ++k) s += sums[(first + k) * 64 + lane];
+      inv = rsqrtf(wave_sum(s) / static_cast<float>(plen) + eps);
+      at = first;
+    }
+    float wt[8];
     load8(w + c + i * 2048, wt);
 #pragma unroll
     for (int k = 0; k < 8; ++k) {

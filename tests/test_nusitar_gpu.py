@@ -144,6 +144,17 @@ def test_group_norm_of_wide_rows(raw, dev, heads, v, parts, mode):
     assert N.rel_err(o, want) < 6e-3
 
 
+@pytest.mark.parametrize("heads,v,parts", [(4, 512, 4), (64, 64, 4), (8, 512, 4), (8, 512, 8), (128, 64, 8), (128, 64, 4)])
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_group_norm_of_wide_rows_is_the_general_one(raw, dev, heads, v, parts, mode):
+    """Rows with room behind them take the general kernel: the squares of a part are added in the same order, so the same bits."""
+    rows, slots = 257, heads * v
+    w, y = (1 + 0.2 * rnd(heads, v, seed=2).float()).to(dev), rnd(rows, slots).bfloat16().to(dev)
+    gate = rnd(rows, slots, seed=1).bfloat16().to(dev) if mode else None
+    wide, general = (raw.group_norm_rows(y, gate, 0, mode, w, heads, v, v, parts, ld, 1e-3, False) for ld in (slots, slots + 64))
+    assert torch.equal(wide, general[:, :slots])
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_glu(raw, dev, dtype):
     src, sr = typed(rnd(7, 2 * 72, scale=2), dtype, dev)
