@@ -1013,7 +1013,7 @@ static bool use_256_base(int M, int N, int K = 0) {
   return g_use_256 && ((M >= 1024 && t >= 128) || (M >= 768 && t >= 160));
 }
 
-// Two to four row tiles, where only the four-wave kernel is ahead: once the 128 x 128 tiles are more than a round (512 workgroups) and
+// Two to four row tiles, where the four-wave kernel is ahead: once the 128 x 128 tiles are more than a round (512 workgroups) and
 // these are not, or those more than two rounds.  us, plain / gated / with a residual / slabs, so / as before: 700 x 12288 x 4096, 144 and 576 tiles,
 // 84 / 125, gated --, 84 / 127, 84 / 122; 400 x 22016 x 4096, 172 and 688, 88 / 131, 91 / 128, 87 / 134, 85 / 129; 636 x 20480 x 2048,
 // 240 and 800, 56 / 76, 52 / 71; 300 x 32000 x 4096, 250 and 750, 98 / 137; 636 rows, 375 and 1250, 164 / 198.  Under a round of the others
@@ -1025,6 +1025,17 @@ static bool use_256_few(int M, int N, int K) {
   return g_use_256 && M > 256 && M < 1024 && K >= 2048 && t128 > 512 && (t <= 256 || t128 > 1024 || (t <= 264 && M > 512 && !g_for_slabs));
 }
 static bool use_256(int M, int N, int K = 0) { return use_256_base(M, N, K) || use_256_few(M, N, K); }
+// Columns or an epilogue that the four-wave kernel does not take (rows off 16 bytes, an fp32 output with a bias) go to the eight-wave one on that
+// line.  us, so / 128 x 128 tiles: 300 x 32003 x 4096 119 / 153, 636 rows 190 / 222, 767 197 / 231; 60 products with odd columns, K from 4 096 on, plain
+// 1.04 to 1.53 times as fast, gelu 1.01 to 1.46, a residual 1.01 to 1.50, fp32 0.99 to 1.45.  Below 4 096 only plain and activated ones
+// whose larger tiles are full, 1.00 to 1.40; with a residual (944 x 9193 x 2048 89 / 84) or a fifth of their rows empty (548 x 13159 x 2048
+// 60 / 57, residual 87 / 71, 578 x 28606 x 2048 104 / 95) behind.
+static bool few_ahead(const GemmParams& p) {
+  GemmParams q = p;
+  output_as_slab(q);
+  const long long t = static_cast<long long>((p.M + 255) / 256) * ((p.N + 255) / 256), t128 = static_cast<long long>((p.M + 127) / 128) * ((p.N + 127) / 128);
+  return p.K >= 4096 || (gemm_quad_serves(q) && gemm_quad_ahead(q, static_cast<int>(t))) || (!p.res && t128 * 10 >= t * 39);
+}
 
 // Short contractions (the ViT's 1024-wide layers: 16 K-tiles) are bound by the round trip of each K-tile, which waves of
 // other workgroups have to cover: eight waves on the 64 x 128 tile with two stages (48 KB: three workgroups, 24 waves a
@@ -1073,12 +1084,12 @@ static bool g_tail_splitk = true;
 // 836x4096x11008 878 vs 811, x12288 926 vs 844, x22016 1038 vs 871; at 636 rows -- three row tiles,
 // a quarter of the last one used -- it is behind, 725 vs 807).  With gemm_quad.hip, us, so / the other choice: 836 x 4096 x 11008 83 / 95,
 // x 22016 144 / 177, 1000 rows x 11008 88 / 136; behind at 128 tiles in two splits, 1024 x 8192 x 8192 152 / 136.  Three row tiles (513 to
-// 767 rows), the sum of the slabs included: ahead where the 128 x 128 tiles are more than 170 and leave room for two splits, 700 x 4096
+// 767 rows; that kernel only, whose slabs are quads of columns: 640 x 5002 x 8192 on the eight-wave one 94, before 82), the sum of the slabs included: ahead where the 128 x 128 tiles are more than 170 and leave room for two splits, 700 x 4096
 // x 11008 80 / 95, 767 x 4096 x 8192 65 / 74, 520 x 5120 x 13824 90 / 121; with three of them behind, 636 x 4096 x 11008 79 / 76.  strided: an
 // operand that only the 8-wave kernel takes.  Returns the split count, or 0.
 static int narrow_256_splits(int M, int N, int K, bool strided = false) {
   if (!g_use_256 || g_forced_cfg >= 0 || g_forced_splitk > 0 || M < (strided ? 768 : 513) || M > 1024 || K < 8192) return 0;
-  if (M < 768 && static_cast<long long>((M + 127) / 128) * ((N + 127) / 128) <= 170) return 0;
+  if (M < 768 && (N % 4 || K % 64 || static_cast<long long>((M + 127) / 128) * ((N + 127) / 128) <= 170)) return 0;
   const long long t = static_cast<long long>((M + 255) / 256) * ((N + 255) / 256);
   if (t < 48 || t > 128) return 0;
   const int s = static_cast<int>(256 / t);
@@ -1087,8 +1098,8 @@ static int narrow_256_splits(int M, int N, int K, bool strided = false) {
 
 // K = 0: the caller cannot split K (argmax partials, K-strided operands)
 // k_real: the contraction length when the caller knows it (the tile choice depends on it), also where K = 0; act, res: the
-// epilogue applies an activation, adds a residual
-static GemmCfg pick_cfg(int M, int N, int K = 0, int k_real = 0, bool act = false, bool res = false) {
+// epilogue applies an activation, adds a residual; few: use_256_few's line is open to the product
+static GemmCfg pick_cfg(int M, int N, int K = 0, int k_real = 0, bool act = false, bool res = false, bool few = true) {
   if (k_real == 0) k_real = K;
   if (g_forced_cfg >= 0) return static_cast<GemmCfg>(g_forced_cfg);
   auto tiles = [&](int bm, int bn) {
@@ -1097,7 +1108,7 @@ static GemmCfg pick_cfg(int M, int N, int K = 0, int k_real = 0, bool act = fals
   // thresholds from benchmarks/bench_gemm.py on MI355X
   if (M <= 32) return tiles(32, 128) >= 256 ? CFG_32x128 : CFG_32x64;
   if (use_64x128_w8(M, N, k_real, act, res)) return CFG_64x128_W8;
-  if (use_256(M, N, k_real)) return CFG_256x256;
+  if (use_256_base(M, N, k_real) || (few && use_256_few(M, N, k_real))) return CFG_256x256;
   if (K && narrow_256_splits(M, N, K) >= 2) return CFG_256x256;
   // Narrow outputs over a long contraction (a few hundred rows into 4096 columns over 11008, the
   // ViT's 4096 -> 1024 projection): the larger tile, its grid filled by splitting K (gemm_splitk)
@@ -1254,7 +1265,7 @@ void launch_gemm_bf16(const bf16_t* A, const bf16_t* W, bf16_t* C, float* Cf, co
     p.splitk = (K + p.k_per_split - 1) / p.k_per_split;  // drop empty trailing splits
     p.partial = splitk_ws;
   }
-  GemmCfg cfg = pick_cfg(M, N, (splitk_ws && !amax_val) ? K : 0, amax_val ? 0 : K, act != ACT_NONE, res != nullptr);
+  GemmCfg cfg = pick_cfg(M, N, (splitk_ws && !amax_val) ? K : 0, amax_val ? 0 : K, act != ACT_NONE, res != nullptr, few_ahead(p));
   if (p.k_cols) {
     // short last K-tile: the two instances compiled with the masked staging path (these are the
     // low-rank products and other short contractions; the tile choice matters little for them)

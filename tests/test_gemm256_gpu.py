@@ -183,6 +183,28 @@ def test_two_to_four_row_tiles(dev, M, N, K):
     _check(raw.linear_swiglu(x, w), torch.nn.functional.silu(y[:, :N // 2]) * y[:, N // 2:], K)
 
 
+# columns and epilogues that the four-wave kernel does not take: (plain, with a residual, an fp32 output with a bias) on the eight-wave kernel
+@pytest.mark.parametrize("M,N,K,eight", [(300, 32003, 4096, (1, 1, 1)), (636, 32003, 4096, (1, 1, 1)), (500, 20483, 2048, (1, 0, 1)),
+                                         (548, 13159, 2048, (0, 0, 0)), (548, 13160, 2048, (0, 0, 0)), (640, 5002, 8192, (0, 0, 0))])
+def test_two_to_four_row_tiles_of_other_columns(dev, M, N, K, eight):
+    from eventgpt_amd.ops import hip
+    from torch.profiler import ProfilerActivity, profile
+    raw = hip.raw
+    x, w = _rand(M, K, dev=dev), _rand(N, K, dev=dev, seed=1, scale=0.05)
+    bias, res = _rand(N, dev=dev, seed=2), _rand(M, N, dev=dev, seed=3)
+    y = x.float() @ w.float().t()
+    calls = [(lambda: raw.linear(x, w, None, None, 0, False), y), (lambda: raw.linear(x, w, None, res, 0, False), y.to(torch.bfloat16).float() + res.float()),
+             (lambda: raw.linear(x, w, bias, None, 0, True), y + bias.float())]
+    for (call, want), on in zip(calls, eight):
+        with profile(activities=[ProfilerActivity.CUDA]) as p:
+            got = call()
+            torch.cuda.synchronize()
+        _check(got, want, K)
+        ran = [e.key for e in p.key_averages() if "gemm" in e.key]
+        served = N % 8 == 0 and got.dtype == torch.bfloat16
+        assert any(("gemm_quad_kernel" if served else "gemm256_kernel" if on else "gemm_bf16_kernel") in k for k in ran), ran
+
+
 # slabs of three row tiles in K splits: the lines at 513 rows and at 170 tiles of 128 x 128
 @pytest.mark.parametrize("M,N,K", [(513, 4480, 8192), (641, 4096, 8192), (640, 4096, 8192), (767, 5120, 8256)])
 def test_slabs_of_three_row_tiles(dev, M, N, K):
