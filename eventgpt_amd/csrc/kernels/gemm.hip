@@ -1367,6 +1367,11 @@ bool launch_gemm_qkv_rope(const bf16_t* A, const bf16_t* W, int M, int K, bf16_t
     }
     return true;
   }
+  // Otherwise 128 x 128 tiles; not for more rows than a prompt in one piece has (1024) where the plain product's own choice and a rotation pass are
+  // ahead: 256 x 256 tiles whose whole rounds end among the q or k heads (us, so / plain: 32 q and 8 k heads x 4096, 3400 rows 206 / 172, 64 and
+  // 8, 1900 rows 203 / 159, 40 and 8 x 5120, 2600 rows 241 / 184), and fewer than a tile a CU (8 and 2 x 1024, 1500 rows, 144 tiles, 21 / 18,
+  // 2600 rows, 252, 23.3 / 21.5; 3100 rows, 300, 27.2 / 27.8; 16 and 4 x 2048, 1200 rows, 240, 31 / 27, 1500 rows, 288, 36.6 / 38.2)
+  if (M > 1024 && (use_256(M, N, K) || cfg_tiles(CFG_128x128, M, N) <= 256)) return false;
   launch_cfg<128, 128, 2, 2, 2, false, false, false, true>(p, st);
   return true;
 }

@@ -470,13 +470,13 @@ def test_long_prompt_prefill_and_decode(dev):
         eng.prefill(torch.zeros(3073, 256, dtype=torch.bfloat16, device=dev), start=0)
 
 
-# the last seven on 256 x 256 tiles: one round, a column tile that is half there, rows past the cache, the columns past the whole rounds on
-# 128 x 128 tiles, in four and in three splits, and (one k head: not all of them v) back on 128 x 128 tiles
+# the last eight: 256 x 256 tiles in one round, a column tile that is half there, rows past the cache, the columns past the whole rounds on
+# 128 x 128 tiles, in four and in three splits; many rows on 128 x 128 tiles, little over a tile a CU, and of too few tiles for the larger ones
 @pytest.mark.parametrize("S,Hq,Hkv,K,p0,l_max", [(636, 32, 32, 4096, 0, 1024), (77, 4, 4, 512, 5, 80),
                                                   (300, 8, 2, 1024, 17, 512), (129, 4, 1, 512, 40, 160),
                                                   (1100, 32, 32, 640, 0, 1200), (2000, 33, 1, 1024, 9, 2400), (1025, 32, 32, 1024, 40, 1040),
                                                   (1301, 32, 32, 1024, 3, 1400), (1300, 32, 32, 4096, 0, 1400), (1601, 32, 32, 4096, 50, 1640),
-                                                  (4000, 32, 1, 1024, 0, 4000)])
+                                                  (1700, 8, 6, 1024, 2, 1750), (1200, 32, 8, 4096, 0, 1200)])
 def test_qkv_gemm_with_rope_epilogue_equals_gemm_then_rope(dev, S, Hq, Hkv, K, p0, l_max):
     """The q | k | v GEMM whose epilogue rotates and appends to the cache writes exactly what the plain
     GEMM followed by the RoPE / append kernel writes (same bf16 rounding points), including rows that
@@ -513,6 +513,19 @@ def test_qkv_gemm_with_rope_epilogue_equals_gemm_then_rope(dev, S, Hq, Hkv, K, p
     kk = rot[:n_in, Hq:Hq + Hkv].transpose(0, 1)
     assert (k2[0, :, p0:p0 + n_in].float() - kk).abs().max().item() < 0.02 * float(kk.abs().max()) + 1e-3
     assert torch.all(k2[0, :, :p0] == 7.0) and torch.all(v2[0, :, p0 + n_in:] == -7.0)
+
+
+# whole rounds of 256 x 256 tiles that end among the k heads and among the q heads; a tile a CU
+@pytest.mark.parametrize("S,Hq,Hkv,K", [(4000, 32, 1, 1024), (3400, 32, 8, 4096), (1900, 64, 8, 512), (2600, 8, 2, 1024)])
+def test_qkv_gemm_leaves_products_of_many_rows_to_the_plain_one(dev, S, Hq, Hkv, K):
+    """Nothing is written where the plain product and a rotation pass are ahead of 128 x 128 tiles, and the engine takes those."""
+    from eventgpt_amd import ops
+    raw = torch.ops.evgpt
+    cos, sin = (t.contiguous() for t in ops.rope_tables(S, 128, 10000.0, dev))
+    x, w = torch.randn(S, K, device=dev).bfloat16(), torch.randn((Hq + 2 * Hkv) * 128, K, device=dev).bfloat16()
+    q, k, v = (torch.full((1, h, S, 128), 7.0, dtype=torch.bfloat16, device=dev) for h in (Hq, Hkv, Hkv))
+    assert not raw.linear_qkv_rope(x, w, q, k, v, cos, sin, torch.zeros(1, dtype=torch.int32, device=dev), Hq, Hkv)
+    assert all(bool((t == 7.0).all()) for t in (q, k, v))
 
 
 def test_prompt_path_equals_plain_path(model, dev):
