@@ -1336,6 +1336,7 @@ bool linear_qkv_rope(const Tensor& x, const Tensor& w_qkv, const Tensor& q_out, 
   TORCH_CHECK(q_out.numel() == S * Hq * 128 && k_cache.size(1) == Hkv && v_cache.sizes() == k_cache.sizes() &&
               pos0.numel() >= 1 && cos.size(-1) == 64 && sin.size(-1) == 64 && cos.size(0) >= k_cache.size(2) &&
               sin.size(0) >= k_cache.size(2), "linear_qkv_rope: shapes");
+  if (S * K >= (1ll << 30) || w_qkv.numel() >= (1ll << 30)) return false;      // (operands are addressed with 32-bit byte offsets: `linear` says so)
   const int64_t ws = evgpt::gemm_tail_ws_floats((int)S, (int)w_qkv.size(0), (int)K);
   Tensor slabs;
   if (ws > 0) slabs = at::empty({ws}, cos.options());

@@ -520,12 +520,26 @@ def test_qkv_gemm_with_rope_epilogue_equals_gemm_then_rope(dev, S, Hq, Hkv, K, p
 def test_qkv_gemm_leaves_products_of_many_rows_to_the_plain_one(dev, S, Hq, Hkv, K):
     """Nothing is written where the plain product and a rotation pass are ahead of 128 x 128 tiles, and the engine takes those."""
     from eventgpt_amd import ops
-    raw = torch.ops.evgpt
+    from eventgpt_amd.ops import hip
+    raw = hip.raw
     cos, sin = (t.contiguous() for t in ops.rope_tables(S, 128, 10000.0, dev))
     x, w = torch.randn(S, K, device=dev).bfloat16(), torch.randn((Hq + 2 * Hkv) * 128, K, device=dev).bfloat16()
     q, k, v = (torch.full((1, h, S, 128), 7.0, dtype=torch.bfloat16, device=dev) for h in (Hq, Hkv, Hkv))
     assert not raw.linear_qkv_rope(x, w, q, k, v, cos, sin, torch.zeros(1, dtype=torch.int32, device=dev), Hq, Hkv)
     assert all(bool((t == 7.0).all()) for t in (q, k, v))
+
+
+def test_qkv_gemm_leaves_operands_of_2_gib_to_the_plain_one(dev):
+    """Byte offsets have 32 bits: nothing is launched, and the plain product refuses the rows."""
+    from eventgpt_amd import ops
+    from eventgpt_amd.ops import hip
+    raw, S, K = hip.raw, 1 << 18, 4096
+    cos, sin = (t.contiguous() for t in ops.rope_tables(64, 128, 10000.0, dev))
+    x, w = torch.empty(S, K, dtype=torch.bfloat16, device=dev), torch.zeros(4 * 128, K, dtype=torch.bfloat16, device=dev)
+    q, k, v = (torch.zeros(1, h, n, 128, dtype=torch.bfloat16, device=dev) for h, n in ((2, S), (1, 64), (1, 64)))
+    assert not raw.linear_qkv_rope(x, w, q, k, v, cos, sin, torch.zeros(1, dtype=torch.int32, device=dev), 2, 1)
+    with pytest.raises(RuntimeError, match="2 GiB"):
+        raw.linear(x, w, None, None, 0, False)
 
 
 def test_prompt_path_equals_plain_path(model, dev):
