@@ -299,10 +299,11 @@ class AttentionAdapter(HiddenAdapterBase):
 
     def forward(self, hidden_states, attention_mask=None):
         x, d = _run_blocks(self.layers, hidden_states, False, attention_mask)
-        if without_hooks(self.output_proj):
-            y = self.output_proj[1](_normed(x, d, self.output_proj[0]))
-        else:
-            y = self.output_proj(x if d is None else x + d)
+        proj = self.output_proj
+        if type(proj) is nn.Sequential and len(proj) == 2 and without_hooks(proj):
+            y = proj[1](_normed(x, d, proj[0]))
+        else:                                    # (somebody's own module, or one that is listened to)
+            y = proj(x if d is None else x + d)
         return toward(hidden_states, y, self.alpha)
 
     def align(self, source, target=None, attention_mask=None):

@@ -179,3 +179,29 @@ def test_adapter_self_test_table():
     assert [r["level"].split("_")[0] for r in rows] == ["L1", "L2", "L3", "L4", "L5", "L5F"]
     assert all(r["parameters"] > 0 and r["forward_ms"] >= 0 for r in rows)
     assert rows[3]["parameters"] > rows[0]["parameters"]          # attention adapter > bottleneck
+
+
+def _own_projection(kind):
+    class Doubled(torch.nn.Sequential):
+        def forward(self, x):
+            return 2 * super().forward(x)
+
+    class Alone(torch.nn.Module):
+        def forward(self, x):
+            return x.flip(-1)
+    parts = lambda: (torch.nn.LayerNorm(64), torch.nn.Linear(64, 64))
+    return {"three": lambda: torch.nn.Sequential(*parts(), torch.nn.Tanh()), "one": lambda: torch.nn.Sequential(torch.nn.Linear(64, 64)),
+            "subclass": lambda: Doubled(*parts()), "alone": Alone, "plain": lambda: torch.nn.Sequential(*parts())}[kind]()
+
+
+@pytest.mark.parametrize("kind", ["three", "one", "subclass", "alone", "plain"])
+def test_attention_adapter_calls_whatever_its_output_projection_is(kind):
+    """The norm of a plain pair is taken with the residual addition; any other module is called whole."""
+    torch.manual_seed(0)
+    m, h = create_adapter(4, 64, num_heads=2, ffn_dim=32, num_layers=2).eval(), torch.randn(2, 5, 64)
+    m.output_proj = _own_projection(kind)
+    x = h
+    for layer in m.layers:
+        x = x + layer["attn"](layer["attn_norm"](x), causal=False, key_padding_mask=None)
+        x = x + layer["ffn"](layer["ffn_norm"](x))
+    assert torch.equal(m(h), h + m.alpha * (m.output_proj(x) - h))
