@@ -22,7 +22,7 @@ from __future__ import annotations
 
 import torch
 import torch.nn.functional as F
-from torch.overrides import TorchFunctionMode, handle_torch_function, has_torch_function
+from torch.overrides import TorchFunctionMode, _get_current_function_mode, handle_torch_function, has_torch_function
 
 from . import differentiable as diff
 
@@ -49,9 +49,15 @@ def without_hooks(module) -> bool:
                 or m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks or m._global_backward_pre_hooks)
 
 
+def _routed(*tensors) -> bool:
+    """Whether ``InTreeLinear`` would be the first to see the call: other modes, and tensors of other types, see the expression's own."""
+    return (has_torch_function(tensors) and isinstance(_get_current_function_mode(), InTreeLinear)
+            and all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors))
+
+
 def add_norm(x, d, norm):
     """``(x + d, norm(x + d))``, ``norm`` an ``nn.LayerNorm``: a step of the residual stream, one launch inside ``InTreeLinear``."""
-    if has_torch_function((x, d)):
+    if _routed(x, d):
         return handle_torch_function(add_norm, (x, d), x, d, norm)
     s = x + d
     return s, norm(s)
@@ -59,7 +65,7 @@ def add_norm(x, d, norm):
 
 def toward(base, y, alpha):
     """``base + alpha * (y - base)``, one launch inside ``InTreeLinear``."""
-    if has_torch_function((base, y, alpha)):
+    if _routed(base, y, alpha):
         return handle_torch_function(toward, (base, y, alpha), base, y, alpha)
     return base + alpha * (y - base)
 

@@ -205,3 +205,35 @@ def test_attention_adapter_calls_whatever_its_output_projection_is(kind):
         x = x + layer["attn"](layer["attn_norm"](x), causal=False, key_padding_mask=None)
         x = x + layer["ffn"](layer["ffn_norm"](x))
     assert torch.equal(m(h), h + m.alpha * (m.output_proj(x) - h))
+
+
+def test_other_modes_and_tensor_types_see_the_steps_of_a_block():
+    """The residual additions, the norms and the step toward the output are calls of their own for whoever watches them."""
+    from collections import Counter
+    from torch.overrides import TorchFunctionMode
+
+    class Watch(TorchFunctionMode):
+        def __init__(self):
+            super().__init__()
+            self.seen = Counter()
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.seen[func.__name__] += 1
+            return func(*args, **(kwargs or {}))
+
+    class Own(torch.Tensor):
+        seen = Counter()
+
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            cls.seen[func.__name__] += 1
+            return super().__torch_function__(func, types, args, kwargs or {})
+    torch.manual_seed(0)
+    m, h = create_adapter(4, 64, num_heads=2, ffn_dim=32, num_layers=2).eval(), torch.randn(2, 5, 64)
+    want = m(h)
+    with Watch() as mode:
+        assert torch.equal(m(h), want)
+    got = m(h.as_subclass(Own))
+    assert type(got) is Own and torch.equal(got.as_subclass(torch.Tensor), want)
+    for seen in (mode.seen, Own.seen):
+        assert {n: seen[n] for n in ("layer_norm", "add", "sub", "mul")} == {"layer_norm": 5, "add": 5, "sub": 1, "mul": 1}, seen
