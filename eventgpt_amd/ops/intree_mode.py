@@ -43,9 +43,9 @@ def _eligible(x, w, b) -> bool:
 
 
 def without_hooks(module) -> bool:
-    """Whether a call of ``module`` may be left out for its parts: nobody is told of calls of it, or of all modules'."""
+    """Whether a call of ``module`` may be left out for its parts: its ``forward`` is its type's and nobody is told of calls of it, or of all modules'."""
     m = torch.nn.modules.module
-    return not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+    return not ("forward" in module.__dict__ or module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
                 or m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks or m._global_backward_pre_hooks)
 
 

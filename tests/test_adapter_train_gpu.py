@@ -577,3 +577,6 @@ def test_parts_of_a_block_that_is_listened_to_are_called_whole(dev):
     for hook in hooks:
         hook.remove()
     assert loss() == quiet and len(seen) == 2
+    norm = m.layers[0]["ffn_norm"]
+    norm.forward = lambda x: seen.append("own") or torch.nn.LayerNorm.forward(norm, x)      # a forward put on the module itself
+    assert abs(loss() - quiet) < 1e-2 * quiet and seen[2:] == ["own"]

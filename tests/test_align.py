@@ -190,11 +190,13 @@ def _own_projection(kind):
         def forward(self, x):
             return x.flip(-1)
     parts = lambda: (torch.nn.LayerNorm(64), torch.nn.Linear(64, 64))
-    return {"three": lambda: torch.nn.Sequential(*parts(), torch.nn.Tanh()), "one": lambda: torch.nn.Sequential(torch.nn.Linear(64, 64)),
+    patched = torch.nn.Sequential(*parts())
+    patched.forward = lambda x: 3 * torch.nn.Sequential.forward(patched, x)       # (as offloading libraries wrap a module in place)
+    return {"patched": lambda: patched, "three": lambda: torch.nn.Sequential(*parts(), torch.nn.Tanh()), "one": lambda: torch.nn.Sequential(torch.nn.Linear(64, 64)),
             "subclass": lambda: Doubled(*parts()), "alone": Alone, "plain": lambda: torch.nn.Sequential(*parts())}[kind]()
 
 
-@pytest.mark.parametrize("kind", ["three", "one", "subclass", "alone", "plain"])
+@pytest.mark.parametrize("kind", ["three", "one", "subclass", "alone", "patched", "plain"])
 def test_attention_adapter_calls_whatever_its_output_projection_is(kind):
     """The norm of a plain pair is taken with the residual addition; any other module is called whole."""
     torch.manual_seed(0)
