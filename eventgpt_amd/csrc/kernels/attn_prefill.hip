@@ -715,7 +715,10 @@ void launch_attn_prefill(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf16
   // Three block shapes: 64 rows (four waves), 128 rows (eight), and the ring-staged 256 rows of two tiles a wave, whose K / V must allow
   // 16-byte row chunks.  us of 64 / 128 / 256 rows, causal heads of 128 unless noted; with D = 128 there are 512, 512 and 256 blocks at a time:
   //  * 256 rows where they are one round, nearly full: 2 x 836, 32 heads 40 / 32 / 32; 1850 64 / 61 / 59; 4096, 16 heads 152 / 129 / 118;
-  //    4 x 836, 16 heads of 64, no mask 31 / 27 / 25
+  //    4 x 836, 16 heads of 64, no mask 31 / 27 / 25; and their rows are, without a mask more than half of them (8 x 100, 32 heads of 128 8.5 / 7.5 / 9.5,
+  //    8 x 128 of 64 5.8 / 6.2 / 7.0; 8 x 200 27.5 / 20.1 / 19.4 and 16.2 / 11.7 / 11.7; 8 x 280, 16 heads 23.5 / 20.5 / 19.5; 5 x 577, 16 heads of 64 23 / 20 / 20), with
+  //    one seven tenths and more than a block of them (8 x 20, 32 heads 4.2 / 4.8 / 6.1; 8 x 100 7.7 / 7.5 / 9.8; 8 x 200 23 / 16 / 19, of 64 12.6 / 9.7 / 11.2;
+  //    8 x 256 25 / 19 / 21; 4 x 260 17.5 / 15.3 / 17.1; 4 x 384 25 / 20 / 18.5; 5 x 520, 16 heads 25 / 22 / 24; 5 x 600 30 / 25 / 25)
   //  * 64 rows up to 640 blocks of them: 636, 32 heads 18 / 20 / 23; 1200 35 / 39 / 40; 2048, 16 heads 43 / 64 / 65; 4096, 8 heads 82 / 95 /
   //    118.  Heads of 64 without a mask to 1056: 4 x 577, 16 heads 18 / 20 / 20; 4 x 1200 45 / 46 / 61
   //  * beyond, 128 rows where they are one round (1400, 32 heads 45 / 43 / 44; 3 x 577 33 / 26 / 32; 1500, 2 x 16 heads 53 / 44 / 51) or
@@ -727,8 +730,10 @@ void launch_attn_prefill(const bf16_t* q, const bf16_t* k, const bf16_t* v, bf16
   const long long heads = static_cast<long long>(Hq) * B, n64 = (Sq + 63) / 64 * heads, n128 = (Sq + 127) / 128 * heads,
                   n256 = (Sq + 255) / 256 * heads;
   const bool vit = D == 64 && !causal;
+  const long long padded = (Sq + 255) / 256 * 256;
+  const bool filled = causal ? Sq > 256 && Sq * 10ll >= padded * 7 : Sq * 2ll > padded;
   int rows = 64;
-  if (g_attn_wide == 2 || (g_attn_wide == 1 && n256 > 224 && n256 <= 256)) rows = 256;
+  if (g_attn_wide == 2 || (g_attn_wide == 1 && n256 > 224 && n256 <= 256 && filled)) rows = 256;
   else if (g_attn_wide == 3) rows = 128;
   else if (n64 > (vit ? 1056 : 640))
     rows = vit || (n128 <= 512 && Sq <= 1792) || n256 * 20 >= n128 * 11 || g_attn_wide == 0 ? 128 : 256;

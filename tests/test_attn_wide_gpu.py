@@ -110,3 +110,19 @@ def test_wide_forward_feeds_backward(dev, wide):
     for got, want in ((q.grad, qf.grad), (k.grad, kf.grad), (v.grad, vf.grad)):
         assert torch.allclose(got.float(), want, atol=3e-2, rtol=3e-2), float((got.float() - want).abs().max())
 
+
+# a round of 256-row blocks whose rows are mostly padding, and next to the lines (seven tenths with a mask and more than one block, half without)
+@pytest.mark.parametrize("B,S,H,D,causal,wide", [
+    (8, 20, 32, 128, True, False), (8, 100, 32, 128, True, False), (8, 256, 32, 128, True, False), (4, 358, 32, 128, True, False), (4, 359, 32, 128, True, True),
+    (5, 520, 16, 128, True, False), (2, 836, 32, 128, True, True), (8, 128, 32, 128, False, False), (8, 129, 32, 128, False, True),
+    (8, 64, 32, 64, False, False), (5, 577, 16, 64, False, True), (8, 200, 32, 64, True, False)])
+def test_blocks_of_256_rows_where_they_are_filled(dev, B, S, H, D, causal, wide):
+    from eventgpt_amd.ops import hip
+    q, k, v = (torch.randn(B, S, H, D, device=dev).bfloat16() for _ in range(3))
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as p:
+        o, _ = hip.raw.attention_fwd_lse(q, k, v, causal, D ** -0.5, 0)
+        torch.cuda.synchronize()
+    names = [e.key for e in p.key_averages() if "attn_prefill" in e.key]
+    assert len(names) == 1 and ("attn_prefill_wide_kernel" in names[0]) == wide, names
+    want = torch.nn.functional.scaled_dot_product_attention(*(t.transpose(1, 2).float() for t in (q, k, v)), is_causal=causal).transpose(1, 2)
+    assert torch.allclose(o.float(), want, atol=2e-2, rtol=2e-2)
