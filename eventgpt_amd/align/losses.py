@@ -68,9 +68,7 @@ class _RowPairLoss(torch.autograd.Function):
         return hip.raw.row_pair_grad(pred, target, st, m, n_valid, g_mse, g_cos), None, None
 
 
-def _fused_pair_ok(pred: torch.Tensor, target: torch.Tensor, mask: Optional[torch.Tensor] = None) -> bool:
-    if mask is not None and not (mask.device == pred.device and mask.numel() * pred.shape[-1] == pred.numel()):
-        return False
+def _fused_pair_ok(pred: torch.Tensor, target: torch.Tensor) -> bool:
     return (pred.is_cuda and target.is_cuda and pred.dtype == target.dtype and pred.shape == target.shape
             and pred.dtype in (torch.float32, torch.bfloat16) and pred.shape[-1] % 8 == 0
             and pred.is_contiguous() and target.is_contiguous() and not target.requires_grad)
@@ -79,7 +77,7 @@ def _fused_pair_ok(pred: torch.Tensor, target: torch.Tensor, mask: Optional[torc
 def alignment_losses(pred: torch.Tensor, target: torch.Tensor,
                      mask: Optional[torch.Tensor] = None,
                      prediction_weight: float = 0.0) -> Dict[str, torch.Tensor]:
-    if _fused_pair_ok(pred, target, mask):
+    if _fused_pair_ok(pred, target):         # (a mask that is not one weight a row, there, is refused)
         mse, cos_sim = _RowPairLoss.apply(pred, target, mask)
     else:
         mse = masked_mse(pred, target, mask)

@@ -175,6 +175,15 @@ def test_pair_loss_of_each_term_and_of_rows_that_are_nothing(kind, rows):
             assert torch.allclose(a, b, rtol=1e-5, atol=1e-5 * float(b.abs().max()) if b.numel() else 0)
 
 
+@pytest.mark.parametrize("shape", [(1, 6), (4, 1), (6,), (4, 5)])
+def test_a_mask_of_another_size_is_refused(shape):
+    """Broadcast, it would be counted once and used for every sequence: a loss that many times too large."""
+    from eventgpt_amd.align.losses import alignment_losses
+    pred = torch.randn(4, 6, 64, device="cuda:0")
+    with pytest.raises(RuntimeError):
+        alignment_losses(pred, pred + 1, torch.ones(shape, device="cuda:0"))
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("masked", [False, True])
 def test_fused_alignment_loss_matches_tensor_expressions(dtype, masked):
