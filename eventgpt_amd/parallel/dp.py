@@ -289,7 +289,7 @@ class ShardedAdamW:
         RCCL makes no host round trip unless the caller converts the norm (``float(norm)``)."""
         self._finish_reduces()
         sq, clip_t = self._global_sq_norm(), None
-        if max_grad_norm is not None and sq.is_cuda:
+        if max_grad_norm is not None and sq.is_cuda and not isinstance(max_grad_norm, torch.Tensor):
             from ..ops import hip
             norm, clip_t = hip.raw.clip_factor(sq, float(max_grad_norm))
         else:

@@ -153,6 +153,25 @@ def test_clip_factor_is_the_tensor_expression(sq, top):
     assert torch.allclose(clip, (top / (t.sqrt() + 1e-6)).clamp(max=1.0).reshape(1), rtol=2.0 ** -22, atol=0, equal_nan=True)     # two roundings
 
 
+def test_a_largest_norm_on_the_device_is_not_waited_for():
+    from eventgpt_amd.parallel.dp import ShardedAdamW
+    dev, results = torch.device("cuda", 0), []
+    for top in (0.5, torch.tensor(0.5, device=dev)):
+        torch.manual_seed(0)
+        layer = torch.nn.Linear(64, 64).to(dev)
+        opt, x = ShardedAdamW(layer.parameters(), lr=1e-2), torch.randn(32, 64, device=dev)
+        opt.zero_grad()
+        layer(x).square().sum().backward()
+        torch.cuda.set_sync_debug_mode("error")
+        try:
+            norm = opt.step(max_grad_norm=top)
+        finally:
+            torch.cuda.set_sync_debug_mode("default")
+        results.append((norm, layer.weight.detach()))
+    for a, b in zip(*results):
+        assert torch.allclose(a, b, rtol=1e-6, atol=0)
+
+
 @pytest.mark.parametrize("kind", ["mse", "cos", "both"])
 @pytest.mark.parametrize("rows", [1, 1023, 1025])
 def test_pair_loss_of_each_term_and_of_rows_that_are_nothing(kind, rows):
