@@ -1091,19 +1091,6 @@ std::tuple<Tensor, Tensor> clip_factor(const Tensor& sq, double max_norm) {
   return {norm, clip};
 }
 
-// acc[0] += sum(x^2) over a contiguous bf16 / fp32 device tensor (16-byte aligned), deterministic
-void sumsq_accumulate(const Tensor& x, const Tensor& acc) {
-  check_f32(acc, "acc");
-  TORCH_CHECK(x.is_cuda() && x.is_contiguous() && (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kFloat),
-              "sumsq_accumulate: contiguous bf16 / fp32 device tensor");
-  TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0, "sumsq_accumulate: 16-byte aligned input");
-  const int64_t n = x.numel();
-  if (n == 0) return;
-  Tensor part = at::empty({evgpt::sumsq_blocks(n)}, acc.options());
-  evgpt::launch_sumsq(x.data_ptr(), x.scalar_type() == at::kBFloat16, n, part.data_ptr<float>(), acc.data_ptr<float>(),
-                      cur_stream());
-}
-
 // ---- 4-bit codebook weights: `packed` uint8 [N, K/2], `absmax` fp32 [N, K/64], `code` a
 // host bf16 tensor with the 16 codebook entries (read here on the host, so it must not
 // live on the device: these ops run inside graph captures)
@@ -1844,7 +1831,6 @@ TORCH_LIBRARY(evgpt, m) {
   m.def("add_layernorm_bwd(Tensor s, Tensor weight, Tensor grad, Tensor? gs, float eps, bool want_sum, bool want_params, Tensor(a!)? dw_out=None, Tensor(b!)? db_out=None) -> (Tensor, Tensor, Tensor, Tensor)", &add_layernorm_bwd);
   m.def("toward(Tensor base, Tensor y, Tensor alpha) -> Tensor", &toward);
   m.def("toward_bwd(Tensor g, Tensor base, Tensor y, Tensor alpha) -> (Tensor, Tensor)", &toward_bwd);
-  m.def("sumsq_accumulate(Tensor x, Tensor(a!) acc) -> ()", &sumsq_accumulate);
   m.def("sumsq_many(Tensor[] xs) -> Tensor", &sumsq_many);
   m.def("clip_factor(Tensor sq, float max_norm) -> (Tensor, Tensor)", &clip_factor);
   m.def("fused_adamw_many(Tensor[] grads, Tensor(a!)[] masters, Tensor(b!)[] exp_avgs, Tensor(c!)[] exp_avg_sqs, Tensor(d!)[] params_out, float lr, float beta1, float beta2, float eps, float weight_decay, int step, Tensor? clip_dev=None) -> ()", &fused_adamw_many);

@@ -102,8 +102,6 @@ struct SumsqShard { const void* x; long long n; bool bf16; };
 long long sumsq_many_blocks(const SumsqShard* shards, int count);      // floats of `part`
 void launch_sumsq_many(const SumsqShard* shards, int count, float* part, float* out, hipStream_t st);
 void launch_clip_factor(const float* sq, float max_norm, float* norm, float* clip, hipStream_t st);
-int sumsq_blocks(long long n);
-void launch_sumsq(const void* x, bool bf16, long long n, float* part, float* acc, hipStream_t st);
 
 // ---- gemm.hip
 int gemm_argmax_partials(int M, int N);

@@ -168,8 +168,8 @@ void launch_fused_adamw_many(const AdamWShard* shards, int count, bool bf16, con
   }
 }
 
-// ---- sum of squares of a gradient shard (global-norm clipping), two deterministic stages:
-// `blocks` partial sums, then one block adds them to acc[0] (fp32; accumulates across buckets).
+// ---- sum of squares of a gradient's shards (global-norm clipping), two deterministic stages: partial sums of blocks, then one block
+// adds them.  Two launches in all instead of two a shard, each 4 to 5 us at the least.
 template <typename T>
 __device__ __forceinline__ float sumsq_block(const T* __restrict__ x, long long n, int block, int blocks, float* red) {
   float s = 0.f;
@@ -193,14 +193,6 @@ __device__ __forceinline__ float sumsq_block(const T* __restrict__ x, long long 
   }
   return block_sum(s, red);
 }
-template <typename T>
-__global__ __launch_bounds__(256) void sumsq_partial_kernel(const T* __restrict__ x, long long n, float* __restrict__ part) {
-  __shared__ float red[4];
-  const float s = sumsq_block(x, n, blockIdx.x, gridDim.x, red);
-  if (threadIdx.x == 0) part[blockIdx.x] = s;
-}
-
-// Every shard of a gradient: two launches in all instead of two a shard, each 4 to 5 us at the least.
 struct SumsqTable { const void* x[MANY]; long long n[MANY]; int first[MANY + 1]; unsigned int bf16; };
 __global__ __launch_bounds__(256) void sumsq_many_kernel(SumsqTable t, float* __restrict__ part) {
   __shared__ float red[4];
@@ -224,24 +216,9 @@ __global__ void clip_factor_kernel(const float* __restrict__ sq, float max_norm,
   *clip = c > 1.f ? 1.f : c;             // (not a number stays that)
 }
 
-__global__ __launch_bounds__(256) void sumsq_final_kernel(const float* __restrict__ part, int n, float* __restrict__ acc) {
-  __shared__ float red[4];
-  float s = 0.f;
-  for (int i = threadIdx.x; i < n; i += 256) s += part[i];
-  s = block_sum(s, red);
-  if (threadIdx.x == 0) acc[0] += s;
-}
-
-int sumsq_blocks(long long n) {
+static int sumsq_blocks(long long n) {
   long long b = (n + 256 * 8 * 4 - 1) / (256 * 8 * 4);   // at least four 16-byte loads per thread
   return static_cast<int>(b < 1 ? 1 : (b > 2048 ? 2048 : b));
-}
-
-void launch_sumsq(const void* x, bool bf16, long long n, float* part, float* acc, hipStream_t st) {
-  const int blocks = sumsq_blocks(n);
-  if (bf16) hipLaunchKernelGGL(sumsq_partial_kernel<bf16_t>, dim3(blocks), dim3(256), 0, st, static_cast<const bf16_t*>(x), n, part);
-  else hipLaunchKernelGGL(sumsq_partial_kernel<float>, dim3(blocks), dim3(256), 0, st, static_cast<const float*>(x), n, part);
-  hipLaunchKernelGGL(sumsq_final_kernel, dim3(1), dim3(256), 0, st, part, blocks, acc);
 }
 
 long long sumsq_many_blocks(const SumsqShard* shards, int count) {

@@ -105,16 +105,14 @@ def test_device_resident_loaders_yield_the_host_loaders_batches(tmp_path):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n", [1, 7, 8, 4099, 1 << 20, (1 << 22) + 5])
-def test_sumsq_accumulate(dtype, n):
+def test_sumsq_of_one_shard(dtype, n):
     from eventgpt_amd.ops import hip
     dev = torch.device("cuda", 0)
     g = torch.Generator(device=dev).manual_seed(n)
     x = (torch.randn(n, device=dev, generator=g) * 3).to(dtype)
-    acc = torch.full((1,), 2.5, device=dev)
-    hip.raw.sumsq_accumulate(x, acc)
-    hip.raw.sumsq_accumulate(x, acc)                       # accumulates; same bits both times
-    want = 2.5 + 2 * float(x.double().pow(2).sum())
-    assert abs(float(acc) - want) < 1e-4 * want
+    got, want = hip.raw.sumsq_many([x]), float(x.double().pow(2).sum())
+    assert got.shape == (1,) and torch.equal(got, hip.raw.sumsq_many([x]))       # same bits both times
+    assert abs(float(got) - want) < 1e-4 * want
 
 
 # lengths about the 8 elements of a thread and the 2 048 of a block, and more shards than a launch's table holds
