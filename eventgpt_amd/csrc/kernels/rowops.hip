@@ -336,8 +336,8 @@ __global__ __launch_bounds__(256) void group_norm_kernel(SrcRows y, SrcRows gate
 // The same for bf16 rows of NC * 2048 channels without padding whose parts are runs of whole 512 (a wave's): the row stays in registers, all of
 // it requested at once, and only the sums of eight channels go through LDS (the kernel above stages the row there and reads it twice, its loads
 // behind the choice of their type).  A lane adds its squares over the runs of a part ahead of the wave's sum, the order of the kernel above
-// for four parts and more: the same bits.  4096 rows: 8192 channels, silu gate before, 61 -> 45 us (201 MB: 4.5 TB/s); 4096, sigmoid gate after,
-// 31 -> 24.5.
+// for four parts and more: the same bits.  4096 rows, us: 8192 channels, eight parts, silu gate before, 58 -> 42
+// (201 MB: 4.8 TB/s); 6144, twelve, sigmoid gate after, 43 -> 33; 4096, eight 29 -> 24; 2048, four 16.4 -> 13.6; one row 7.5 -> 5.5, 6.3 -> 4.3, 5.0 -> 3.6, 3.8 -> 3.0.
 template <int GATE, int NC>
 __global__ __launch_bounds__(256) void group_norm_wide_kernel(const bf16_t* __restrict__ y, long long ldy, const bf16_t* __restrict__ gate,
                                                               long long ldg, const float* __restrict__ w, bf16_t* __restrict__ out, int plen,
@@ -384,7 +384,7 @@ __global__ __launch_bounds__(256) void group_norm_wide_kernel(const bf16_t* __re
 static bool launch_group_norm_wide(const SrcRows& y, const SrcRows& gate, int gcol, int mode, const float* w, void* out, int rows, int slots,
                                    int parts, float eps, hipStream_t st) {
   const int plen = slots / parts, nc = slots / 2048;
-  if (slots % 2048 || plen % 512 || plen * parts != slots || (nc != 1 && nc != 2 && nc != 4) || y.f32 || (mode != GATE_NONE && gate.f32)) return false;
+  if (slots % 2048 || plen % 512 || plen * parts != slots || nc < 1 || nc > 4 || y.f32 || (mode != GATE_NONE && gate.f32)) return false;
   const bf16_t* yp = static_cast<const bf16_t*>(y.p);
   const bf16_t* gp = mode == GATE_NONE ? nullptr : static_cast<const bf16_t*>(gate.p) + gcol;
 #define EVGPT_GN(GATE, NC) hipLaunchKernelGGL((group_norm_wide_kernel<GATE, NC>), dim3(rows), dim3(256), 0, st, yp, y.ld, gp, gate.ld, w, \
@@ -392,6 +392,7 @@ static bool launch_group_norm_wide(const SrcRows& y, const SrcRows& gate, int gc
 #define EVGPT_GN_NC(GATE)         \
   if (nc == 1) EVGPT_GN(GATE, 1); \
   else if (nc == 2) EVGPT_GN(GATE, 2); \
+  else if (nc == 3) EVGPT_GN(GATE, 3); \
   else EVGPT_GN(GATE, 4)
   if (mode == GATE_SILU_BEFORE) { EVGPT_GN_NC(GATE_SILU_BEFORE); }
   else if (mode == GATE_SIGMOID_AFTER) { EVGPT_GN_NC(GATE_SIGMOID_AFTER); }

@@ -131,7 +131,7 @@ def test_group_norm_with_gate(raw, dev, dtype, heads, v, vp, parts, before):
                      oracle.rms(y[..., :v].reshape(rows, -1).double(), eps, wr, parts)) < 2e-6
 
 
-# rows of whole 2048 channels in parts of whole 512 (kept in registers), and two forms next to them
+# rows of whole 2048 channels in parts of whole 512 (kept in registers), and a form next to them
 @pytest.mark.parametrize("heads,v,parts", [(4, 512, 4), (32, 64, 1), (64, 64, 4), (8, 512, 8), (128, 64, 8), (128, 64, 1), (96, 64, 3), (32, 64, 8)])
 @pytest.mark.parametrize("mode", [0, 1, 2])
 def test_group_norm_of_wide_rows(raw, dev, heads, v, parts, mode):
@@ -144,7 +144,7 @@ def test_group_norm_of_wide_rows(raw, dev, heads, v, parts, mode):
     assert N.rel_err(o, want) < 6e-3
 
 
-@pytest.mark.parametrize("heads,v,parts", [(4, 512, 4), (64, 64, 4), (8, 512, 4), (8, 512, 8), (128, 64, 8), (128, 64, 4)])
+@pytest.mark.parametrize("heads,v,parts", [(4, 512, 4), (64, 64, 4), (8, 512, 4), (8, 512, 8), (128, 64, 8), (128, 64, 4), (96, 64, 4), (12, 512, 12), (24, 256, 6)])
 @pytest.mark.parametrize("mode", [0, 1, 2])
 def test_group_norm_of_wide_rows_is_the_general_one(raw, dev, heads, v, parts, mode):
     """Rows with room behind them take the general kernel: the squares of a part are added in the same order, so the same bits."""
