@@ -1506,8 +1506,8 @@ static bool pack_words(const X* x, const X* y, const P* p, int64_t n, int* out, 
 
 // Pinned memory for the words of this thread's calls, two blocks of up to 4 MB that go back with the thread.  A block is written again when
 // nobody holds its words and the copy out of it is done, so a call does not wait for its own copy (a pageable one blocks: 13 us of 48 for
-// 20 000 events, 37 of 118 for 200 000; with this and the loop above 31 and 66).  torch's own pool has a block for every call in flight and
-// was slower than the pageable copy.
+// 20 000 events, 37 of 118 for 200 000; with this and the loop above 31 and 66; recordings that are new each time 52 -> 34; after other models'
+// work in the process 44 to 49 -> 31 to 35).  torch's own pool has a block for every call in flight: 107 after such work.
 struct WordStaging {
   static constexpr int64_t MOST = 1 << 20;
   Tensor host;

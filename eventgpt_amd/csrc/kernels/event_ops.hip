@@ -271,8 +271,9 @@ void launch_event_voxel_ranges(const int* x, const int* y, const int* p, const i
 //   count  a block owns one (bin, band): it adds the runs of all chunks in LDS counters and writes both outputs whole
 // The chunk of a sorted stream lies in one or two bins, so the sort reads t at its two ends only; the unsorted one
 // reads it for every event.  Bound by memory: 12 B in, 2 B out, 2 B in per event (and 8 B for the span) plus 12 B out per
-// pixel and bin.  1e7 clustered events, 480 x 640, 5 bins by time on a sorted stream: span 17 us, sort 31, count 19; the
-// whole call 79 us (218 MB it cannot do without: 2.8 TB/s), 766 with voxel_lds_kernel above, which scans y once a band
+// pixel and bin.  1e7 clustered events, 480 x 640, 5 bins by time on a sorted stream, four recordings: span 15 to 18 us, sort 31,
+// count 20 to 25 (by how the events cluster); the whole call 68 to 72 us in a row on one stream, 82 on another one each time (218 MB it cannot do
+// without: 2.7 to 3.2 TB/s), 766 with voxel_lds_kernel above, which scans y once a band
 // (506 us) behind host round trips for the extent and the order of t.
 constexpr int VS_THREADS = 512, VS_PER = 16, VS_CHUNK = VS_THREADS * VS_PER, VS_KEYS = 4096, VS_SPANS = 256;
 
@@ -337,7 +338,7 @@ __global__ __launch_bounds__(VS_THREADS) void voxel_sort_kernel(VoxelArgs a) {
   __shared__ int unsorted_s;
   const int c0 = blockIdx.x * VS_CHUNK, tid = threadIdx.x;
   const int in_chunk = min(VS_CHUNK, a.n - c0);
-  // what the chunk's bins come from is requested ahead of the events: behind them it arrives behind them (34 -> 31 us)
+  // what the chunk's bins come from is requested ahead of the events: behind them it arrives behind them (1e7 events 34 -> 31 us)
   VoxelSpan ext{};
   long long t_end = 0;
   if (!a.by_count) {
@@ -448,8 +449,8 @@ __global__ __launch_bounds__(VS_THREADS) void voxel_sort_kernel(VoxelArgs a) {
 
 // Every wave takes its own share of the chunks, a lane a chunk and neighbouring chunks in different waves (a bin of a sorted stream is a
 // range of chunks), and has eight runs on their way, two records a load, before it counts the first: a run is some 70 records, and one
-// after another they were as many round trips (24 -> 19 us; 5e6 events, one bin of 203 x 301: 34 -> 32).  What is left is the LDS adds, half of their lanes empty; runs filled up to 16 bytes, a
-// lane a piece of one, took 2 us less here and cost the sort more.
+// after another they were as many round trips (1e7 events, four recordings: 28.7, 23.5, 28.5, 24.8 -> 25.1, 20.5, 24.0, 21.5 us; 5e6 events, one bin of 203 x 301: 34 -> 32).  What is left is the LDS adds, half
+// of their lanes empty; runs filled up to 16 bytes, a lane a piece of one, took 2 us less here and cost the sort more.
 template <int THREADS>
 __global__ __launch_bounds__(THREADS) void voxel_count_kernel(VoxelArgs a, int* __restrict__ out_hist, float* __restrict__ out_vox,
                                                               int signed_mode) {

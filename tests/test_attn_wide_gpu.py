@@ -1,4 +1,4 @@
-"""The 128-query-row prefill attention (two query tiles per wave, direct-to-LDS K / V ring) forced onto
+"""The 256-query-row prefill attention (eight waves of two query tiles, direct-to-LDS K / V ring) forced onto
 every shape class: causal with and without an offset into a longer key range, non-causal, grouped KV
 heads, ragged tails, a device-side key count, strided (packed-QKV) inputs; against the fp32 reference,
 repeated (its ring is ordered by counted waits and barriers), and its log-sum-exp feeding the backward."""
@@ -27,7 +27,7 @@ def wide():
     (128, 4, 4, 641, 641, True), (128, 8, 2, 300, 300, True), (128, 2, 2, 129, 700, True), (128, 2, 2, 128, 128, True),
     (64, 16, 16, 577, 577, False), (64, 4, 4, 250, 250, False), (128, 2, 2, 1, 130, True), (64, 2, 2, 130, 259, True),
     (128, 4, 4, 1500, 1500, True), (128, 2, 1, 257, 1000, False), (128, 2, 2, 700, 2300, True),
-    (128, 16, 4, 2100, 2100, True), (64, 32, 32, 1100, 1100, False)])    # enough 256-row blocks for the 8-wave variant
+    (128, 16, 4, 2100, 2100, True), (64, 32, 32, 1100, 1100, False)])    # several blocks a sequence
 def test_wide_attention_matches_reference(dev, wide, D, H, Hkv, Sq, Sk, causal):
     B = 2
     q, k, v = _rand(B, Sq, H, D, dev=dev), _rand(B, Sk, Hkv, D, dev=dev, seed=1), _rand(B, Sk, Hkv, D, dev=dev, seed=2)
